@@ -124,6 +124,34 @@ def test_linear_scan_in_pieces_side_by_side_equals_the_scan_in_order(heads, shar
         close(after[k], want[k][at:at + 1], 5e-5)
 
 
+def test_linear_scan_in_pieces_whose_last_ones_are_short():
+    """A segment's last piece of a few rows is walked long before the others: the state it stores must not be what the
+    first piece starts from.  Many heads, so that the launch is many times what the GPU holds at once."""
+    from runtime.kernels import ops
+    rng = np.random.default_rng(5)
+    heads, R, C, piece, lengths = 32, 128, 64, 128, [387, 259, 770, 515, 386]
+    T = sum(lengths)
+    starts = np.concatenate(([0], np.cumsum(lengths)))
+    q, k, v = (rng.standard_normal((T, n, d)) / d ** 0.5 for n, d in ((1, R), (1, R), (heads, C)))
+    a, begun = rng.uniform(0.9, 1.0, (T, heads)), rng.standard_normal((len(lengths), heads, R, C))
+    carry = [torch.empty(n, device=DEV) for n in ops.scan_carry(T, piece, heads, R, C, False)]
+    outs = []
+    for _ in range(3):
+        state, out = dev(begun.reshape(len(lengths), -1)), torch.empty(T, heads * C, device=DEV)
+        ops.linear_scan(dev(q[:, 0]), dev(k[:, 0]), dev(v.reshape(T, -1)), dev(a), out, state, ints(starts), ints(range(len(lengths))), heads, R, C,
+                        share=heads, piece=piece, carry=carry)
+        outs.append((out.cpu().numpy().reshape(T, heads, C), state.cpu().numpy().reshape(begun.shape)))
+    for h in (0, heads - 1):
+        for s, (lo, hi) in enumerate(zip(starts, starts[1:])):
+            S = begun[s, h]
+            for t in range(lo, hi):
+                S = a[t, h] * S + np.outer(k[t, 0], v[t, h])
+                if t in (lo, lo + piece - 1, lo + piece, hi - 1):
+                    close(outs[0][0][t, h], S.T @ q[t, 0], 5e-5)
+            close(outs[0][1][s, h], S, 5e-5)
+    assert all(np.array_equal(o, outs[0][0]) and np.array_equal(st, outs[0][1]) for o, st in outs[1:])
+
+
 @pytest.mark.parametrize("channels, taps, heads", [(10, 4, 3), (7, 2, 1), (300, 3, 2), (5, 1, 2), (6, 16, 0)])
 def test_short_convolution_carries_its_last_inputs_across_portions_of_any_size(channels, taps, heads):
     from runtime.kernels import ops
