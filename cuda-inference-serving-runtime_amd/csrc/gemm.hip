@@ -2,81 +2,11 @@
 // weights are stored [out, in] (reference: runtime/blas.py:41-56 does the same
 // product through a vendor library).
 //
-//  * gemm_f32: true 32-bit path.  float operands, FMA accumulation in float in
-//    ascending k order, no matrix-core instruction and no reduced-precision mode.
 //  * gemm_bf16: bf16 operands on the matrix cores (v_mfma_f32_16x16x32_bf16),
-//    float accumulation; output float or bf16.
-// Both take any M, N, K >= 1.  R (float, may be null, may alias a float C) is a
+//    float accumulation; output float or bf16.  (Float operands: gemm_f32.hip.)
+// Any M, N, K >= 1.  R (float, may be null, may alias a float C) is a
 // residual added in the epilogue from the float accumulator.
 #include "common.h"
-
-// ------------------------------------------------------------------ float
-#define F_BM 64
-#define F_BN 64
-#define F_BK 16
-
-__global__ void __launch_bounds__(256)
-gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-                float* C, int ldc, const float* R, int ldr, int M, int N, int K) {
-    __shared__ float As[F_BK][F_BM + 4];
-    __shared__ float Ws[F_BK][F_BN + 4];
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.y * F_BM, n0 = blockIdx.x * F_BN;
-    const int ty = tid / 16, tx = tid % 16;
-    const int lr = tid / 4, lk = (tid % 4) * 4;
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-    for (int k0 = 0; k0 < K; k0 += F_BK) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int k = k0 + lk + e;
-            const int am = m0 + lr, wn = n0 + lr;
-            As[lk + e][lr] = (am < M && k < K) ? A[(size_t)am * lda + k] : 0.f;
-            Ws[lk + e][lr] = (wn < N && k < K) ? W[(size_t)wn * ldw + k] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < F_BK; ++kk) {
-            float a[4], w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n >= N) continue;
-            float v = acc[i][j];
-            if (R) v += R[(size_t)m * ldr + n];
-            C[(size_t)m * ldc + n] = v;
-        }
-    }
-}
-
-extern "C" int cisr_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
-                             const float* R, int ldr, int M, int N, int K, hipStream_t stream) {
-    if (M <= 0 || N <= 0) return 0;
-    if (K <= 0) return (int)hipErrorInvalidValue;
-    dim3 grid((N + F_BN - 1) / F_BN, (M + F_BM - 1) / F_BM);
-    if (grid.y > 65535) return (int)hipErrorInvalidValue;
-    gemm_f32_kernel<<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, R, ldr, M, N, K);
-    return CISR_LAUNCH_CHECK();
-}
 
 // ------------------------------------------------------------------- bf16
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;

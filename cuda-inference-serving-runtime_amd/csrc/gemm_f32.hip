@@ -1,0 +1,198 @@
+// The 32-bit product  C[M,N] = A[M,K] . W[N,K]^T (+ R): float operands, float multiply-adds on the matrix cores
+// (v_mfma_f32_16x16x4_f32, whose inputs and sums are whole floats: no reduced-precision mode).
+//
+// With few rows the product is a stream of W, with many it is bound by the matrix instruction; in between (the layer
+// products of small models) it is a chain of trips to memory.  All three want K cut over the waves of a block: a tile of
+// TM x TN sixteens of C is made by WK waves, each with a contiguous run of K's sixteens, DEPTH of them in flight; a wave
+// hands its operands through LDS to the lanes that want them (loaded in the instruction's own layout, sixteen rows side by
+// side in neighbouring lanes, a load costs the cache four times the lines: 2 rows 4.5 -> 3.9 us, 16 rows 5.9 -> 4.6 at
+// 576 x 576), without a barrier; the waves' tiles meet in LDS once.
+//
+// The order of the sum of an element of C is fixed by K alone (WK by K, runs by WK, four interleaved chains a sixteen, a
+// tree over the waves), whatever M, N and the tile are: a row's result does not depend on the other rows of a step.
+//
+// Measured on an MI355X beside what stood here before (vector multiply-adds in tiles of 64 x 64 x 16 staged through LDS: 9
+// to 48 blocks at these sizes, one trip to memory a sixteen of K), 2 / 16 / 130 rows: 576 x 576 61 / 58 / 65 us -> 3.9 /
+// 4.6 / 7.8, 3072 x 576 60 / 58 / 61 -> 4.2 / 5.1 / 13.4, 576 x 1536 158 / 152 / 170 -> 5.7 / 7.1 / 14.7; the head of two
+// rows, 49152 x 576, 94 -> 28 (4.0 TB/s); 2,048 rows against 8192 x 2048 1,797 -> 786 (87 of 157 TFLOP/s).  Relative error
+// against 64 bits 4.3e-7 -> 1.6e-7 (K = 576), 8.1e-7 -> 2.1e-7 (K = 2,048): K's runs are sums of their own.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
+
+struct GemmF32Args {
+    const float* A; int lda;
+    const float* W; int ldw;
+    float* C; int ldc;
+    const float* R; int ldr;         // residual added at the end, or null; may be C
+    int M, N, K;
+    int m_tiles;
+};
+
+// Four floats of row `row` at k; VEC: one 16-byte load, rows 16-byte aligned and K a multiple of 4.  Addresses are
+// clamped, never branched around; what lies past K is cleared by `clear_tail`.
+template <bool VEC>
+__device__ __forceinline__ gf_f32x4 gf_load(const float* row, int k, int K) {
+    if (VEC) return *(const gf_f32x4*)(row + min(k, K - 4));
+    gf_f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = row[min(k + e, K - 1)];
+    return v;
+}
+
+__device__ __forceinline__ gf_f32x4 gf_clear_tail(gf_f32x4 v, int k, int K) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? v[e] : 0.f;
+    return v;
+}
+
+// What a wave wrote to LDS before is there for its own lanes after (a wave's LDS accesses are served in order: only the
+// compiler must not move them).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int TM, int TN, int WK, int DEPTH, bool VEC>
+__global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
+    extern __shared__ __attribute__((aligned(16))) char gf_lds[];
+    gf_f32x4* meet = (gf_f32x4*)gf_lds;                              // [WK][TM * TN][64], after the waves are through
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, r = lane % 16, g = lane / 16;
+    const int m0 = (blockIdx.x % p.m_tiles) * TM * 16, n0 = (blockIdx.x / p.m_tiles) * TN * 16;   // (neighbours share rows of W)
+    const int K = p.K, sixteens = (K + 15) / 16;
+    const int first = (int)((long long)sixteens * wave / WK), last = (int)((long long)sixteens * (wave + 1) / WK);
+    // Neighbouring lanes load neighbouring words of a row (lane: row lane / 4, four k from 4 (lane % 4)); the instruction wants
+    // row lane % 16, four k from 4 (lane / 16).  They change places in LDS, in slots of the wave's own: 16 bytes at row * 4 +
+    // (fourth ^ row / 2), so that neither way has two lanes on a bank.
+    const int lrow = lane / 4, lk = 4 * (lane % 4);
+    gf_f32x4* put = (gf_f32x4*)gf_lds + wave * (TM + TN) * WAVE + lrow * 4 + ((lane % 4) ^ (lrow / 2 % 4));
+    const gf_f32x4* get = (const gf_f32x4*)gf_lds + wave * (TM + TN) * WAVE + r * 4 + (g ^ (r / 2 % 4));
+    const float* a_row[TM];
+    const float* w_row[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a_row[i] = p.A + (size_t)min(m0 + i * 16 + lrow, p.M - 1) * p.lda;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) w_row[j] = p.W + (size_t)min(n0 + j * 16 + lrow, p.N - 1) * p.ldw;
+    gf_f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = (gf_f32x4){0.f, 0.f, 0.f, 0.f};
+    gf_f32x4 fa[DEPTH][TM], fw[DEPTH][TN];
+    auto ask = [&](int d, int s) {
+        const int k = min(s, sixteens - 1) * 16 + lk;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fw[d][j] = gf_load<VEC>(w_row[j], k, K);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[d][i] = gf_load<VEC>(a_row[i], k, K);
+    };
+    auto use = [&](int d, int s) {
+        if (s * 16 + 16 > K) {                                       // (uniform: K's last, partly filled sixteen)
+            const int k = s * 16 + lk;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fw[d][j] = gf_clear_tail(fw[d][j], k, K);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[d][i] = gf_clear_tail(fa[d][i], k, K);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) put[j * WAVE] = fw[d][j];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) put[(TN + i) * WAVE] = fa[d][i];
+        wave_order();
+        gf_f32x4 xa[TM], xw[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) xw[j] = get[j * WAVE];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) xa[i] = get[(TN + i) * WAVE];
+        wave_order();
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[i][e], xw[j][e], acc[i][j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        ask(d, first + d);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // whole turns ask for the turn behind them (past the last sixteen: that one again, so that every wait counts the same
+    // loads); the last turn asks for nothing: a wave with up to DEPTH sixteens is one trip to memory
+    int turn = first;
+    for (; turn + DEPTH < last; turn += DEPTH)
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            use(d, turn + d);
+            __builtin_amdgcn_sched_barrier(0);
+            ask(d, turn + d + DEPTH);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+        if (turn + d < last) use(d, turn + d);                       // (uniform over the wave)
+    // element 4 g + e of a lane's four is row 4 g + e, column r of its sixteen by sixteen
+    constexpr int ITEMS = TM * TN * WAVE;
+    const int t = tid / WAVE, i = t / TN, j = t % TN;                // (the first TM TN waves finish a sixteen by sixteen each)
+    static_assert(TM * TN <= WK, "a wave finishes at most one sixteen by sixteen");
+    const bool finishes = t < TM * TN;
+    const int n = n0 + j * 16 + r, m = m0 + i * 16 + 4 * g;
+    float resid[4] = {0.f, 0.f, 0.f, 0.f};
+    if (finishes && p.R && n < p.N)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) resid[e] = p.R[(size_t)min(m + e, p.M - 1) * p.ldr + n];
+    __syncthreads();                                                 // (the slots above are free)
+#pragma unroll
+    for (int ii = 0; ii < TM; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < TN; ++jj) meet[(wave * TM * TN + ii * TN + jj) * WAVE + lane] = acc[ii][jj];
+    __syncthreads();
+    if (!finishes || n >= p.N) return;
+    gf_f32x4 part[WK];
+#pragma unroll
+    for (int w = 0; w < WK; ++w) part[w] = meet[w * ITEMS + tid];
+#pragma unroll
+    for (int half = WK / 2; half > 0; half /= 2)
+#pragma unroll
+        for (int w = 0; w < half; ++w) part[w] += part[w + half];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (m + e < p.M) p.C[(size_t)(m + e) * p.ldc + n] = part[0][e] + resid[e];
+}
+
+template <int TM, int TN, int WK, int DEPTH, bool VEC>
+static int launch_f32(GemmF32Args p, hipStream_t stream) {
+    p.m_tiles = (p.M + 16 * TM - 1) / (16 * TM);
+    const long long blocks = (long long)p.m_tiles * ((p.N + 16 * TN - 1) / (16 * TN));
+    if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
+    constexpr int lds = WK * (TM * TN > TM + TN ? TM * TN : TM + TN) * WAVE * (int)sizeof(gf_f32x4);
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_kernel<TM, TN, WK, DEPTH, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    gemm_f32_kernel<TM, TN, WK, DEPTH, VEC><<<(unsigned)blocks, WK * WAVE, lds, stream>>>(p);
+    return CISR_LAUNCH_CHECK();
+}
+
+// The tile: 32 x 64 where that leaves two blocks a compute unit, 32 x 32 where it leaves a quarter of them a block, else 16 x 16
+// (up to 16 rows always: the other rows of a tile would be padding).
+template <int WK, bool VEC>
+static int launch_f32_tile(const GemmF32Args& p, hipStream_t stream) {
+    const long long m32 = (p.M + 31) / 32, n32 = (p.N + 31) / 32, n64 = (p.N + 63) / 64;
+    if (p.M > 16 && m32 * n64 >= 512) return launch_f32<2, 4, WK, 2, VEC>(p, stream);
+    if (p.M > 16 && m32 * n32 >= 64) return launch_f32<2, 2, WK, 4, VEC>(p, stream);
+    return launch_f32<1, 1, WK, 8, VEC>(p, stream);
+}
+
+// Waves a tile: sixteen from an inner size of 1,024 on, else eight (so that a wave has at least two sixteens at the small
+// models' 576).
+extern "C" int cisr_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
+                             const float* R, int ldr, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0) return (int)hipErrorInvalidValue;
+    const GemmF32Args p{A, lda, W, ldw, C, ldc, R, ldr, M, N, K, 0};
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+    if (K >= 1024) return vec ? launch_f32_tile<16, true>(p, stream) : launch_f32_tile<16, false>(p, stream);
+    return vec ? launch_f32_tile<8, true>(p, stream) : launch_f32_tile<8, false>(p, stream);
+}

@@ -1143,6 +1143,18 @@ def test_gemm_f32(ops, M, N, K):
     np.testing.assert_allclose(f64(out), want + f64(r), rtol=2e-5, atol=atol)
 
 
+@pytest.mark.parametrize("M, N, K, pad", [(16, 16, 1024, 0), (17, 577, 1536, 0), (40, 2100, 1028, 0), (700, 1500, 1023, 3), (600, 2049, 576, 4), (2, 33, 2060, 1)])
+def test_gemm_f32_at_the_edges_of_its_tiles(ops, M, N, K, pad):
+    """Every tile with rows, columns and sixteens of K off its size, rows of wider buffers with and without 16-byte
+    alignment.  The order of an element's sum is fixed by K: rows alone give the same bits.  Error: the bound of the test above."""
+    a, w = rnd(M, K + pad, seed=4)[:, :K], rnd(N, K + pad, seed=5)[:, :K]
+    got = ops.gemm(a, w, torch.full((M, N + 3), 5.0, device=DEV)[:, :N])
+    np.testing.assert_allclose(f64(got), f64(a) @ f64(w).T, rtol=2e-5, atol=3e-7 * K + 2e-6)
+    for rows in (slice(0, 1), slice(M - 2, M), slice(M // 3, M // 3 + 30)):
+        part = a[rows]
+        assert torch.equal(ops.gemm(part, w, torch.empty(len(part), N, device=DEV)), got[rows])
+
+
 @pytest.mark.parametrize("M, N, K", GEMM_SHAPES)
 def test_gemm_bf16(ops, M, N, K):
     a, w, r = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2), rnd(M, N, seed=3)
