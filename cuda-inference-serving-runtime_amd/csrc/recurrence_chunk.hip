@@ -1,18 +1,27 @@
-// The gated delta rule with a decay a key channel over prompt portions, chunk by chunk on the matrix cores (float operands,
-// v_mfma_f32_16x16x4_f32).  A segment's rows in chunks of 16; with D(t, i) the product of a chunk's decays g_(i+1) .. g_t,
-// channel by channel, D(t) that of g_0 .. g_t, and S0 the state at the chunk's start:
+// Recurrences over prompt portions, chunk by chunk on the matrix cores (float operands, v_mfma_f32_16x16x4_f32): the gated
+// delta rule (DELTA) and the linear scan S <- diag(g) S + k v^T, o = S^T q, each with a decay a key channel (VEC) or one a
+// head.  A segment's rows in chunks of 16; with D(t, i) the product of a chunk's decays g_(i+1) .. g_t, channel by channel,
+// D(t) that of g_0 .. g_t, and S0 the state at the chunk's start:
 //
-//   A[t, i] = beta_t sum_r k_t k_i D(t, i), i < t          P[t, i] = sum_r q_t k_i D(t, i), i <= t
-//   M = (I + A)^-1 diag(beta)
-//   U = M (V - Kg S0),   Kg_t = D(t) k_t                      (the rows' writes u_t)
+//   DELTA:  A[t, i] = beta_t sum_r k_t k_i D(t, i), i < t,  M = (I + A)^-1 diag(beta),  Kg_t = D(t) k_t
+//           U = M (V - Kg S0)                                 (the rows' writes u_t)
+//   else:   U = V, times the rows' step sizes if there are any
+//   P[t, i] = sum_r q_t k_i D(t, i), i <= t
 //   o_t = (D(t) q_t)^T S0 + sum_i P[t, i] u_i
 //   S  <- D(15) S0 + sum_i (D(15, i) k_i) u_i^T
 //
 // Every product of decays is made by multiplying decays along the rows: no quotients and no differences of logarithms, so a
 // channel whose decays vanish within a chunk costs neither range nor precision.  A first kernel makes, chunk by chunk and
 // all side by side, what does not need the state: M V, M Kg, D q, P, D(15, i) k and D(15); a second walks a segment's chunks
-// in order, a block a (head, 16 columns of S): its waves own the rows of S in turn, two products with S0, one meeting through
-// LDS, one product into S.  Rows behind a segment's end count as k = q = v = 0 with decays of one.
+// in order, a block a (head, 16 columns of S): its waves own the rows of S in turn, two products with S0 (one without DELTA),
+// one meeting through LDS, one product into S.  Rows behind a segment's end count as k = q = v = 0 with decays of one.
+// The operands lie in memory as the walk's lanes want them, 16 bytes a lane side by side: read in rows of the chunk instead,
+// each load of the walk touches four times the lines.
+// Measured on an MI355X, us of both kernels (in brackets the scans that walk row by row): 2,048 rows of one request, the delta
+// rule with 32 heads of 128 x 128 and a decay a channel 213 with the operands in rows of the chunk, 180 so (840); gated
+// linear attention, 8 heads of 128 x 256, 108 (290), three requests of 782 rows 94 (361); state-space duality, 64 heads of
+// 128 x 64, 193 (495) and 241 (477).  The walk's bound is its chain a chunk (0.7 to 1 us), with many heads what the two
+// kernels write and read in between (30 KB a chunk and head at 128 x 64).
 #include "common.h"
 
 #define CHUNK 16
@@ -23,8 +32,8 @@ struct ChunkArgs {
     const float* q; int ldq;          // q[t * ldq + (head / share) * R + r]
     const float* k; int ldk;
     const float* v; int ldv;          // v[t * ldv + head * C + c]
-    const float* g; int ldg;          // g[t * ldg + head * R + r]
-    const float* b; int ldb;          // b[t * ldb + head], beta = sigmoid(b)
+    const float* g; int ldg;          // VEC: g[t * ldg + head * R + r]; else g[t * ldg + head]
+    const float* b; int ldb;          // DELTA: b[t * ldb + head], beta = sigmoid(b); else null or the step size b[t * ldb + head] that multiplies v
     float* out; int ldo;
     float* state; long long slot_stride;
     const int* seg_start; const int* state_slots;
@@ -35,8 +44,21 @@ struct ChunkArgs {
     float* work;                      // [slots][heads][chunk_floats]
 };
 
-// Floats of a (chunk, head): M Kg and D q as [16][Rp], D(15, i) k as [Rp][16], M V as [Cp][16], P as [16][16], D(15) [Rp].
-__host__ __device__ __forceinline__ int chunk_floats(int Rp, int Cp) { return 3 * CHUNK * Rp + CHUNK * Cp + CHUNK * CHUNK + Rp; }
+// A (chunk, head) in `work`, in floats: M Kg (DELTA only) and D q as [Rp / 16] tiles of 16 rows x 16 channels, D(15, i) k as
+// tiles of 16 channels x 16 rows, M V as [Cp / 16] tiles of 16 columns x 16 rows, P as one tile, D(15) [Rp].  In a tile, float
+// ((b / 4) * 16 + a) * 4 + b % 4 is element (a, b): what lane 16 (b / 4) + a of the walk takes as its 16 bytes.
+template <bool DELTA>
+struct ChunkLayout {
+    int q, kd, u, pr, g, floats;
+    __host__ __device__ __forceinline__ ChunkLayout(int Rp, int Cp) {
+        q = DELTA ? CHUNK * Rp : 0;
+        kd = q + CHUNK * Rp;
+        u = kd + CHUNK * Rp;
+        pr = u + CHUNK * Cp;
+        g = pr + CHUNK * CHUNK;
+        floats = g + Rp;
+    }
+};
 
 // The segment whose chunk slots hold `slot` (segments without rows own a slot without a chunk).
 __device__ __forceinline__ int segment_of_slot(const int* seg_start, int segments, int slot) {
@@ -62,6 +84,7 @@ __device__ __forceinline__ float row_sum(float x) {
     return x;
 }
 
+template <bool DELTA, bool VEC>
 __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ float sA[CHUNK][CHUNK + 1], sBeta[CHUNK];
@@ -76,19 +99,21 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
     float* sg = sq + CHUNK * RS;
     const float* kh = p.k + (size_t)t0 * p.ldk + (size_t)(head / p.share) * R;
     const float* qh = p.q + (size_t)t0 * p.ldq + (size_t)(head / p.share) * R;
-    const float* gh = p.g + (size_t)t0 * p.ldg + (size_t)head * R;
+    const float* gh = p.g + (size_t)t0 * p.ldg + (VEC ? (size_t)head * R : (size_t)head);
     for (int idx = tid; idx < CHUNK * Rp; idx += 256) {
         const int i = idx / Rp, r = idx % Rp, tt = min(i, n - 1), rr = min(r, R - 1);
         const bool in = r < R && i < n;
-        const float k = kh[tt * p.ldk + rr], q = qh[tt * p.ldq + rr], g = gh[tt * p.ldg + rr];
+        const float k = kh[tt * p.ldk + rr], q = qh[tt * p.ldq + rr], g = gh[tt * p.ldg + (VEC ? rr : 0)];
         sk[i * RS + r] = in ? k : 0.f;
         sq[i * RS + r] = in ? q * p.q_scale : 0.f;
         sg[i * RS + r] = in ? g : 1.f;
     }
-    if (tid < CHUNK) sBeta[tid] = tid < n ? 1.0f / (1.0f + expf(-p.b[(size_t)(t0 + tid) * p.ldb + head])) : 0.f;
+    if (DELTA && tid < CHUNK) sBeta[tid] = tid < n ? 1.0f / (1.0f + expf(-p.b[(size_t)(t0 + tid) * p.ldb + head])) : 0.f;
+    if (!DELTA && tid < CHUNK) sBeta[tid] = tid < n && p.b ? p.b[(size_t)(t0 + tid) * p.ldb + head] : 1.f;     // (the step sizes)
     __syncthreads();
-    float* work = p.work + ((size_t)blockIdx.y * p.heads + head) * chunk_floats(Rp, p.Cp);
-    float* wP = work + 3 * CHUNK * Rp + CHUNK * p.Cp;
+    const ChunkLayout<DELTA> at(Rp, p.Cp);
+    float* work = p.work + ((size_t)blockIdx.y * p.heads + head) * at.floats;
+    float* wP = work + at.pr;
     // column i of A and P: sixteen neighbouring threads, each with every sixteenth run of four channels, carry k_i down the
     // rows behind i (times their decays) and meet
     {
@@ -105,20 +130,20 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
                 if (r >= Rp || t < i) continue;
                 const f32x4_t k = *(const f32x4_t*)(sk + t * RS + r), q = *(const f32x4_t*)(sq + t * RS + r);
                 if (t > i) x[j] *= *(const f32x4_t*)(sg + t * RS + r);
-                a += (x[j][0] * k[0] + x[j][1] * k[1]) + (x[j][2] * k[2] + x[j][3] * k[3]);
+                if (DELTA) a += (x[j][0] * k[0] + x[j][1] * k[1]) + (x[j][2] * k[2] + x[j][3] * k[3]);
                 b += (x[j][0] * q[0] + x[j][1] * q[1]) + (x[j][2] * q[2] + x[j][3] * q[3]);
             }
-            a = row_sum(a);
+            if (DELTA) a = row_sum(a);
             b = row_sum(b);
             if (part == t) {
-                sA[t][i] = sBeta[t] * a;                           // (only i < t is read)
-                wP[t * CHUNK + i] = b;                             // (0 for i > t)
+                if (DELTA) sA[t][i] = sBeta[t] * a;                // (only i < t is read)
+                wP[(i / 4 * 16 + t) * 4 + i % 4] = b;              // (0 for i > t)
             }
         }
     }
     __syncthreads();
     // column j of the inverse of the unit triangle I + A by forward substitution, times beta_j
-    if (tid < CHUNK) {
+    if (DELTA && tid < CHUNK) {
         float x[CHUNK];
 #pragma unroll
         for (int t = 0; t < CHUNK; ++t) {
@@ -132,51 +157,61 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
         for (int t = 0; t < CHUNK; ++t) sM[t][tid] = x[t] * sBeta[tid];
     }
     __syncthreads();
-    // a thread a channel (M Kg and the other operands over the state's rows) or a column of v (M V)
+    // a thread a channel (M Kg and the other operands over the state's rows, which take the place of k, q and the decays) or a
+    // column of v (M V)
     for (int idx = tid; idx < Rp + p.Cp; idx += 256) {
         const bool key = idx < Rp;
         const int c = key ? idx : idx - Rp;
-        float x[CHUNK];
+        float x[CHUNK], kd[CHUNK];
         if (key) {
-            float* wq = work + CHUNK * Rp + c;
-            float* wk = work + 2 * CHUNK * Rp + (size_t)c * CHUNK;
-            float d = 1.f, kd[CHUNK];
-#pragma unroll
-            for (int i = 0; i < CHUNK; ++i) {
-                d *= sg[i * RS + c];
-                x[i] = sk[i * RS + c] * d;
-                wq[(size_t)i * Rp] = sq[i * RS + c] * d;
-            }
-            work[3 * CHUNK * Rp + CHUNK * p.Cp + CHUNK * CHUNK + c] = d;
-            d = 1.f;
+            float d = 1.f;
 #pragma unroll
             for (int i = CHUNK - 1; i >= 0; --i) {
                 kd[i] = sk[i * RS + c] * d;
                 d *= sg[i * RS + c];
             }
+            d = 1.f;
 #pragma unroll
-            for (int i = 0; i < CHUNK; i += 4) *(f32x4_t*)(wk + i) = (f32x4_t){kd[i], kd[i + 1], kd[i + 2], kd[i + 3]};
+            for (int i = 0; i < CHUNK; ++i) {
+                d *= sg[i * RS + c];
+                if (DELTA) x[i] = sk[i * RS + c] * d;
+                sq[i * RS + c] *= d;
+            }
+            work[at.g + c] = d;
+#pragma unroll
+            for (int i = 0; i < CHUNK; ++i) sg[i * RS + c] = kd[i];
         } else {
 #pragma unroll
             for (int i = 0; i < CHUNK; ++i) x[i] = i < n && c < C ? p.v[(size_t)(t0 + min(i, n - 1)) * p.ldv + (size_t)head * C + min(c, C - 1)] : 0.f;
         }
+        if (!DELTA && key) continue;
         float y[CHUNK];
 #pragma unroll
         for (int t = 0; t < CHUNK; ++t) {
-            float s = 0.f;
+            float s = DELTA ? 0.f : x[t] * sBeta[t];
+            if (DELTA) {
 #pragma unroll
-            for (int i = 0; i <= t; ++i) s += sM[t][i] * x[i];
+                for (int i = 0; i <= t; ++i) s += sM[t][i] * x[i];
+            }
             y[t] = s;
-            __builtin_amdgcn_sched_barrier(0);
+            if (DELTA) __builtin_amdgcn_sched_barrier(0);
         }
         if (key) {
 #pragma unroll
-            for (int t = 0; t < CHUNK; ++t) work[(size_t)t * Rp + c] = y[t];
+            for (int t = 0; t < CHUNK; ++t) sk[t * RS + c] = y[t];
         } else {
-            float* wv = work + 3 * CHUNK * Rp + (size_t)c * CHUNK;
+            f32x4_t* wv = (f32x4_t*)(work + at.u) + c / 16 * WAVE + c % 16;
 #pragma unroll
-            for (int t = 0; t < CHUNK; t += 4) *(f32x4_t*)(wv + t) = (f32x4_t){y[t], y[t + 1], y[t + 2], y[t + 3]};
+            for (int t = 0; t < CHUNK; t += 4) wv[t * 4] = (f32x4_t){y[t], y[t + 1], y[t + 2], y[t + 3]};
         }
+    }
+    __syncthreads();
+    for (int unit = tid; unit < Rp * 4; unit += 256) {             // (CHUNK * Rp floats in 16 bytes each)
+        const int tile = unit / WAVE, a = unit % 16, b = unit % WAVE / 16 * 4;
+        ((f32x4_t*)(work + at.q))[unit] = *(const f32x4_t*)(sq + a * RS + tile * 16 + b);
+        if (DELTA) ((f32x4_t*)work)[unit] = *(const f32x4_t*)(sk + a * RS + tile * 16 + b);
+        const float* kd = sg + b * RS + tile * 16 + a;
+        ((f32x4_t*)(work + at.kd))[unit] = (f32x4_t){kd[0], kd[RS], kd[2 * RS], kd[3 * RS]};
     }
 }
 
@@ -187,9 +222,9 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
 // and the new S; the fifth wave adds the shares of (D q) S0 and P U, one chunk behind, and writes the results.
 // AHEAD chunks' operands are in flight (an even number).  The loads of a chunk are kept together in program order: they
 // return in order, so a chunk's wait then leaves those of the chunks behind it in flight.
-template <int NT, int AHEAD>
+template <int NT, int AHEAD, bool DELTA>
 __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))) channel_walk_kernel(ChunkArgs p) {
-    __shared__ f32x4_t share_w[2][4][WAVE], share_o[2][4][WAVE];         // [chunk parity][wave][lane]
+    __shared__ f32x4_t share_w[DELTA ? 2 : 1][4][DELTA ? WAVE : 1], share_o[2][4][WAVE];         // [chunk parity][wave][lane]
     const int head = blockIdx.x, seg = blockIdx.z, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     const int t0 = p.seg_start[seg], t1 = p.seg_start[seg + 1];
     if (t1 <= t0) return;
@@ -198,15 +233,17 @@ __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))
     if (first >= last) return;
     const int m = lane % 16, kg = lane / 16, R = p.R, C = p.C, Rp = p.Rp;
     const int c = blockIdx.y * 16 + m;
-    const size_t per = (size_t)chunk_floats(Rp, p.Cp);
+    const ChunkLayout<DELTA> at(Rp, p.Cp);
+    const size_t per = (size_t)at.floats;
     auto operands = [&](int slot) { return (const char*)(p.work + ((size_t)(min(slot, last - 1) - p.slot0) * p.heads + head) * per); };
     // byte offsets of this lane's words from a chunk's operands (a uniform address): 32 bits
-    const unsigned at_u = (3u * CHUNK * Rp + c * CHUNK + 4 * kg) * 4u;
+    const unsigned at_u = (at.u + (blockIdx.y * WAVE + lane) * 4) * 4u;
     auto writes = [&](f32x4_t u, int par) {          // the rows' writes: M V - M Kg S0
+        if (!DELTA) return u;
         return u - ((share_w[par][0][lane] + share_w[par][1][lane]) + (share_w[par][2][lane] + share_w[par][3][lane]));
     };
     if (wave == 4) {
-        const unsigned at_p = (3u * CHUNK * Rp + CHUNK * p.Cp + m * CHUNK + 4 * kg) * 4u;
+        const unsigned at_p = (at.pr + lane * 4) * 4u;
         struct Result { f32x4_t u, pr; } ring[AHEAD];
         auto fetch = [&](Result& r, int slot) {
             const char* w = operands(slot);
@@ -249,38 +286,41 @@ __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int r = (wave * NT + j) * 16 + 4 * kg + i;
             S[j][i] = r < R && c < C ? state[(size_t)r * C + c] : 0.f;
         }
-    struct Operands { f32x4_t kg[NT], qg[NT], kd[NT], g[NT], u; } ring[AHEAD];
-    unsigned at_k[NT], at_d[NT], at_g[NT];
+    struct Operands { f32x4_t kg[DELTA ? NT : 1], qg[NT], kd[NT], g[NT], u; } ring[AHEAD];
+    unsigned at_k[NT], at_g[NT];
     float mine[NT];
-    const unsigned q_words = CHUNK * Rp * 4u;
+    const unsigned q_words = at.q * 4u, d_words = at.kd * 4u;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const unsigned r = min((wave * NT + j) * 16, Rp - 16);          // (a wave without this tile reads another: its S stays zero)
         mine[j] = (wave * NT + j) * 16 < Rp ? 1.f : 0.f;
-        at_k[j] = (m * Rp + r + 4 * kg) * 4u;
-        at_d[j] = (2u * CHUNK * Rp + (r + m) * CHUNK + 4 * kg) * 4u;
-        at_g[j] = (3u * CHUNK * Rp + CHUNK * p.Cp + CHUNK * CHUNK + r + 4 * kg) * 4u;
+        at_k[j] = (r * 4 + lane) * 16u;
+        at_g[j] = (at.g + r + 4 * kg) * 4u;
     }
     auto fetch = [&](Operands& o, int slot) {
         const char* w = operands(slot);
+        if (DELTA) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j) o.kg[j] = *(const f32x4_t*)(w + at_k[j]);
+            for (int j = 0; j < NT; ++j) o.kg[j] = *(const f32x4_t*)(w + at_k[j]);
+        }
 #pragma unroll
         for (int j = 0; j < NT; ++j) o.qg[j] = *(const f32x4_t*)(w + q_words + at_k[j]);
         o.u = *(const f32x4_t*)(w + at_u);
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             o.g[j] = *(const f32x4_t*)(w + at_g[j]);
-            o.kd[j] = *(const f32x4_t*)(w + at_d[j]);
+            o.kd[j] = *(const f32x4_t*)(w + d_words + at_k[j]);
         }
     };
     auto walk = [&](Operands& now, int par) {
         f32x4_t w = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f};
+        if (DELTA) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kg[j][i], S[j][i], w, 0, 0, 0);
-        share_w[par][wave][lane] = w;
+                for (int i = 0; i < 4; ++i) w = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kg[j][i], S[j][i], w, 0, 0, 0);
+            share_w[par][wave][lane] = w;
+        }
         __syncthreads();           // (the other parity's shares were read before the barrier before this one's writes)
         const f32x4_t u = writes(now.u, par);
 #pragma unroll
@@ -322,35 +362,44 @@ __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // Chunk slots of a step, and floats of `work` a slot takes.
 extern "C" int cisr_channel_chunk_slots(int rows, int segments) { return rows / CHUNK + segments; }
-extern "C" long long cisr_channel_chunk_floats(int heads, int R, int C) {
-    return (long long)heads * chunk_floats((R + 15) / 16 * 16, (C + 15) / 16 * 16);
+extern "C" long long cisr_channel_chunk_floats(int heads, int R, int C, int delta) {
+    const int Rp = (R + 15) / 16 * 16, Cp = (C + 15) / 16 * 16;
+    return (long long)heads * (delta ? ChunkLayout<true>(Rp, Cp).floats : ChunkLayout<false>(Rp, Cp).floats);
 }
 
-// The step's rows in launches of `slab` chunk slots each (two kernels a slab); work: slab * cisr_channel_chunk_floats floats.
-extern "C" int cisr_channel_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* g, int ldg,
-                                   const float* b, int ldb, float* out, int ldo, float* state, long long slot_stride,
-                                   const int* seg_start, const int* state_slots, int rows, int segments, int heads, int R, int C,
-                                   int share, float q_scale, float* work, int slab, hipStream_t stream) {
-    if (rows <= 0 || segments <= 0 || heads <= 0) return 0;
-    if (R <= 0 || R > 256 || C <= 0 || share <= 0 || heads % share || segments > 65535 || (C + 15) / 16 > 65535 || slab <= 0 || slab > 65535 ||
-        (uintptr_t)work % 16)
-        return (int)hipErrorInvalidValue;
-    ChunkArgs p{q, ldq, k, ldk, v, ldv, g, ldg, b, ldb, out, ldo, state, slot_stride, seg_start, state_slots, R, C, share, heads, segments,
-                q_scale, (R + 15) / 16 * 16, (C + 15) / 16 * 16, 0, 0, work};
-    const int total = rows / CHUNK + segments, nt = (p.Rp / 16 + 3) / 4;
+template <bool DELTA, bool VEC>
+static int launch_chunks(ChunkArgs p, int rows, int slab, hipStream_t stream) {
+    const int total = rows / CHUNK + p.segments, nt = (p.Rp / 16 + 3) / 4;
     const size_t lds = (size_t)3 * CHUNK * (p.Rp + 4) * sizeof(float);
     for (p.slot0 = 0; p.slot0 < total; p.slot0 += slab) {
         p.slots = min(slab, total - p.slot0);
-        channel_chunk_kernel<<<dim3(heads, p.slots), 256, lds, stream>>>(p);
+        channel_chunk_kernel<DELTA, VEC><<<dim3(p.heads, p.slots), 256, lds, stream>>>(p);
         int err = CISR_LAUNCH_CHECK();
         if (err) return err;
-        const dim3 grid(heads, p.Cp / 16, segments);
-        if (nt == 1) channel_walk_kernel<1, 4><<<grid, 320, 0, stream>>>(p);
-        else if (nt == 2) channel_walk_kernel<2, 4><<<grid, 320, 0, stream>>>(p);
-        else if (nt == 3) channel_walk_kernel<3, 2><<<grid, 320, 0, stream>>>(p);
-        else channel_walk_kernel<4, 2><<<grid, 320, 0, stream>>>(p);
+        const dim3 grid(p.heads, p.Cp / 16, p.segments);
+        if (nt == 1) channel_walk_kernel<1, 4, DELTA><<<grid, 320, 0, stream>>>(p);
+        else if (nt == 2) channel_walk_kernel<2, 4, DELTA><<<grid, 320, 0, stream>>>(p);
+        else if (nt == 3) channel_walk_kernel<3, 2, DELTA><<<grid, 320, 0, stream>>>(p);
+        else channel_walk_kernel<4, 2, DELTA><<<grid, 320, 0, stream>>>(p);
         err = CISR_LAUNCH_CHECK();
         if (err) return err;
     }
     return 0;
+}
+
+// The step's rows in launches of `slab` chunk slots each (two kernels a slab); work: slab * cisr_channel_chunk_floats floats.
+// `delta`: the delta rule (b: its write strengths before the sigmoid); else the linear scan (b: null or its step sizes).
+// `vec`: a decay a head and key channel; else one a head.
+extern "C" int cisr_channel_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* g, int ldg,
+                                   const float* b, int ldb, float* out, int ldo, float* state, long long slot_stride,
+                                   const int* seg_start, const int* state_slots, int rows, int segments, int heads, int R, int C,
+                                   int share, float q_scale, int delta, int vec, float* work, int slab, hipStream_t stream) {
+    if (rows <= 0 || segments <= 0 || heads <= 0) return 0;
+    if (R <= 0 || R > 256 || C <= 0 || share <= 0 || heads % share || segments > 65535 || (C + 15) / 16 > 65535 || slab <= 0 || slab > 65535 ||
+        (delta && !b) || (uintptr_t)work % 16)
+        return (int)hipErrorInvalidValue;
+    const ChunkArgs p{q, ldq, k, ldk, v, ldv, g, ldg, b, ldb, out, ldo, state, slot_stride, seg_start, state_slots, R, C, share, heads, segments,
+                      q_scale, (R + 15) / 16 * 16, (C + 15) / 16 * 16, 0, 0, work};
+    if (delta) return vec ? launch_chunks<true, true>(p, rows, slab, stream) : launch_chunks<true, false>(p, rows, slab, stream);
+    return vec ? launch_chunks<false, true>(p, rows, slab, stream) : launch_chunks<false, false>(p, rows, slab, stream);
 }

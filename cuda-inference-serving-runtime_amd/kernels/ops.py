@@ -1348,7 +1348,7 @@ def _rec():
             "cisr_channel_inputs": [p, i, p, i, p, ll, p, p, p, p, i, i, i, i, i, i, f, i, i, p, i, p, p, p, i, i, p, i, p, i, i, p],
             "cisr_channel_step": [p, i, p, i, p, i, p, i, p, i, p, ll, p, p, i, i, i, i, i, f, p, i, p, f, p, i, i, p],
             "cisr_channel_step_ok": [i, i, ll],
-            "cisr_channel_chunks": [p, i, p, i, p, i, p, i, p, i, p, i, p, ll, p, p, i, i, i, i, i, i, f, p, i, p],
+            "cisr_channel_chunks": [p, i, p, i, p, i, p, i, p, i, p, i, p, ll, p, p, i, i, i, i, i, i, f, i, i, p, i, p],
             "cisr_channel_chunk_slots": [i, i],
             "cisr_channel_scan": [p, i, p, i, p, i, p, i, p, i, p, i, p, ll, p, p, i, i, i, i, i, f, i, p],
             "cisr_mingru_scan": [p, i, p, p, p, i, p, p, p, i, i, i, i, p, i, i, p],
@@ -1361,7 +1361,7 @@ def _rec():
             fn.restype = C.c_int
         h.cisr_linear_scan_carry.argtypes = [i, i, i, i, i, i, C.POINTER(ll)]
         h.cisr_linear_scan_carry.restype = ll
-        h.cisr_channel_chunk_floats.argtypes = [i, i, i]
+        h.cisr_channel_chunk_floats.argtypes = [i, i, i, i]
         h.cisr_channel_chunk_floats.restype = ll
         _recurrence = h
     return _recurrence
@@ -1681,14 +1681,15 @@ def channel_columns(segments, heads, cols):
             return width
 
 
-def _channel_operands(name, q, k, v, decay, write, state, seg_start, state_slots, heads, R, C_, share):
-    """Checked pointers and strides that the forms of the delta rule with decays a channel share."""
+def _channel_operands(name, q, k, v, decay, write, state, seg_start, state_slots, heads, R, C_, share, scalar=False):
+    """Checked pointers and strides that the forms of the delta rule with decays a channel (and, by chunks, of the rule and
+    of the linear scan with one decay a head: `scalar`) share.  `write` None: no such operand."""
     T, segments = v.shape[0], state_slots.shape[0]
     if heads % share or R > 256:
         raise KernelError(f"{name}: heads must divide into their groups and a state has at most 256 rows")
     args = (*_rows_of(q, "q", heads // share * R), *_rows_of(k, "k", heads // share * R), *_rows_of(v, "v", heads * C_),
-            *_rows_of(decay, "decay", heads * R), *_rows_of(write, "write", heads))
-    if any(t.shape[0] != T for t in (q, k, decay, write)):
+            *_rows_of(decay, "decay", heads if scalar else heads * R), *((None, 0) if write is None else _rows_of(write, "write", heads)))
+    if any(t.shape[0] != T for t in (q, k, decay)) or (write is not None and write.shape[0] != T):
         raise KernelError(f"{name}: operands differ in rows")
     if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or state.shape[1] < heads * R * C_ or not state.is_cuda:
         raise KernelError(f"{name}: the state must be float [slots, >= heads * R * C]")
@@ -1714,6 +1715,7 @@ def channel_delta_scan(q, k, v, decay, write, out, state, seg_start, state_slots
     return out
 
 
+CHUNK_ROWS = 16               # rows of a chunk (csrc/recurrence_chunk.hip)
 CHANNEL_CHUNK_ROWS = 32       # rows beyond one a segment from which a step's portions are walked chunk by chunk
 CHANNEL_SLAB = 160            # chunks whose operands wait in memory at one time (2,048 rows of one request and some)
 
@@ -1724,25 +1726,40 @@ def channel_chunked(rows, segments, decode_only):
     return not decode_only and rows - segments >= CHANNEL_CHUNK_ROWS
 
 
-def channel_chunk_work(rows, segments, heads, rows_of_state, cols_of_state, slab=CHANNEL_SLAB):
-    """Floats of `work` that channel_delta_chunks needs for a step of `rows` rows in `segments` segments."""
+def channel_chunk_work(rows, segments, heads, rows_of_state, cols_of_state, slab=CHANNEL_SLAB, delta=True):
+    """Floats of `work` that channel_delta_chunks (linear_chunks: delta False) needs for a step of `rows` rows in `segments`
+    segments."""
     slots = int(_rec().cisr_channel_chunk_slots(int(rows), int(segments)))
-    return min(slots, int(slab)) * int(_rec().cisr_channel_chunk_floats(int(heads), int(rows_of_state), int(cols_of_state)))
+    return min(slots, int(slab)) * int(_rec().cisr_channel_chunk_floats(int(heads), int(rows_of_state), int(cols_of_state), int(delta)))
+
+
+def _chunks(name, q, k, v, decay, write, out, state, seg_start, state_slots, heads, R, Cc, work, share, q_scale, slab, delta):
+    T, segments = v.shape[0], state_slots.shape[0]
+    scalar = decay.shape[1] == heads
+    args, where = _channel_operands(name, q, k, v, decay, write, state, seg_start, state_slots, heads, R, Cc, share, scalar)
+    op, ldo = _rows_of(out, "out", heads * Cc)
+    if out.shape[0] != T or work.numel() < channel_chunk_work(T, segments, heads, R, Cc, slab, delta):
+        raise KernelError(f"{name}: too few result rows, or too little work space")
+    _check(_rec().cisr_channel_chunks(*args, op, ldo, *where, T, segments, heads, R, Cc, int(share), float(q_scale), int(delta),
+                                      int(not scalar), _dev(work, "work", torch.float32), int(slab), _stream()), name)
+    return out
 
 
 def channel_delta_chunks(q, k, v, decay, write, out, state, seg_start, state_slots, heads, rows_of_state, cols_of_state, work, share=1,
                          q_scale=1.0, slab=CHANNEL_SLAB):
-    """channel_delta_scan in chunks of 16 rows on the matrix cores with float operands: the same results up to rounding.
-    work: float, at least channel_chunk_work(...) elements; `slab`: chunks that one pair of launches takes."""
-    R, Cc = int(rows_of_state), int(cols_of_state)
-    T, segments = v.shape[0], state_slots.shape[0]
-    args, where = _channel_operands("channel_delta_chunks", q, k, v, decay, write, state, seg_start, state_slots, heads, R, Cc, share)
-    op, ldo = _rows_of(out, "out", heads * Cc)
-    if out.shape[0] != T or work.numel() < channel_chunk_work(T, segments, heads, R, Cc, slab):
-        raise KernelError("channel_delta_chunks: too few result rows, or too little work space")
-    _check(_rec().cisr_channel_chunks(*args, op, ldo, *where, T, segments, heads, R, Cc, int(share), float(q_scale),
-                                      _dev(work, "work", torch.float32), int(slab), _stream()), "channel_delta_chunks")
-    return out
+    """channel_delta_scan (decay [T, heads * R]) or delta_scan (decay [T, heads]) in chunks of 16 rows on the matrix cores with
+    float operands: the same results up to rounding.  work: float, at least channel_chunk_work(...) elements; `slab`:
+    chunks that one pair of launches takes."""
+    return _chunks("channel_delta_chunks", q, k, v, decay, write, out, state, seg_start, state_slots, heads, int(rows_of_state),
+                   int(cols_of_state), work, share, q_scale, slab, True)
+
+
+def linear_chunks(q, k, v, decay, out, state, seg_start, state_slots, heads, rows_of_state, cols_of_state, work, share=1, step=None,
+                  q_scale=1.0, slab=CHANNEL_SLAB):
+    """linear_scan in chunks of 16 rows on the matrix cores with float operands: the same results up to rounding.  work: float,
+    at least channel_chunk_work(..., delta=False) elements; `slab`: chunks that one pair of launches takes."""
+    return _chunks("linear_chunks", q, k, v, decay, step, out, state, seg_start, state_slots, heads, int(rows_of_state),
+                   int(cols_of_state), work, share, q_scale, slab, False)
 
 
 def channel_step_ok(state, rows_of_state, cols_of_state):

@@ -1,7 +1,7 @@
 """Mixers that keep a state of fixed size per request instead of keys and values.
 
-The first three are the same recurrence per head, S_t = diag(a_t) S_(t-1) + k_t v_t^T, o_t = S_t^T q_t, run by one kernel
-(ops.linear_scan) over the rows of a step as they come (portions and single tokens of several requests), with
+The first three are the same recurrence per head, S_t = diag(a_t) S_(t-1) + k_t v_t^T, o_t = S_t^T q_t, run by the same
+kernels (ops.linear_scan, ops.linear_chunks) over the rows of a step as they come (portions and single tokens of several requests), with
 the state in the cache manager's state slots, in float in every mode:
 
   GatedLinearAttention   a_t a vector over the key channels, sigmoid(z_t)^(1/tau), z_t from a low-rank projection
@@ -14,8 +14,8 @@ the state in the cache manager's state slots, in float in every mode:
                          causal convolution with silu whose last inputs are part of the state; y = o + D x, times
                          silu(z), RMS-normed in equal parts of the row, then the output projection.
 
-  GatedDeltaRule         S <- g_t S; u = beta_t (v_t - S^T k_t); S <- S + k_t u^T; o_t = S^T q_t, a kernel of its own
-                         (ops.delta_scan): g_t = exp(-exp(A_log) softplus(a_t + dt_bias)) and beta_t = sigmoid(b_t) one
+  GatedDeltaRule         S <- g_t S; u = beta_t (v_t - S^T k_t); S <- S + k_t u^T; o_t = S^T q_t, kernels of its own
+                         (ops.delta_scan, portions by ops.channel_delta_chunks): g_t = exp(-exp(A_log) softplus(a_t + dt_bias)) and beta_t = sigmoid(b_t) one
                          number a head; q, k, v come out of a short causal convolution with silu (its last inputs are
                          part of the state), q and k are made unit vectors per head, q scaled by dim^(-1/2); each
                          head's result RMS-normed, times silu of a gate projection, then the output projection.
@@ -32,6 +32,8 @@ the state in the cache manager's state slots, in float in every mode:
 The projections and the convolution's inputs are products with float results; decays, step sizes, gates of the
 recurrence and the norms are float arithmetic; the operands of the output projections are the compute dtype.
 """
+from dataclasses import dataclass
+
 import torch
 
 from ..cache.pages import StateNeed
@@ -44,15 +46,51 @@ def _float(t):
     return t.to(torch.float32).contiguous()
 
 
-def _scan(ctx, tag, q, k, v, decay, out, state, heads, rows, cols, **kw):
-    """ops.linear_scan over the step's segments; the segments of a step with long portions are walked in pieces."""
+@dataclass(frozen=True)
+class DeltaByChunks:
+    """Whether a step's delta rule of `heads` heads is walked chunk by chunk (launch value 1) or row by row (0): a step array
+    (engine.context.StepArray) without words.  Row by row a step lasts as long as its longest portion or, with many heads
+    and segments, as its rows take all together; chunk by chunk as its chunks take to prepare and walk.  Measured on an
+    MI355X at 32 and 16 heads of 128 x 128 (row by row / by chunks, us; the constants below are fits): one portion of 48
+    rows 26 / 24 and 24 / 23, of 128 58 / 28 and 55 / 27, of 2,048 840 / 180 and 787 / 144; eight of 32 37 / 57 and 26 / 39,
+    of 256 216 / 190 and 145 / 102; 32 of 64 164 / 264 and 88 / 129."""
+    heads: int
+
+    def words(self, rows, segments):
+        return 0
+
+    def launch_value(self, batch):
+        if batch.decode_only:
+            return 0
+        longest, chunks = max(batch.counts), sum(-(-n // ops.CHUNK_ROWS) for n in batch.counts)
+        by_rows = max(8 + 0.41 * longest, 0.0028 * self.heads * sum(batch.counts))
+        return int(20 + max(0.042 * self.heads * chunks, longest / 16) < by_rows)
+
+    def fill(self, out, batch, value):
+        pass
+
+
+def _chunk_work(ctx, rows, heads, state_rows, state_cols, delta):
+    """What a walk by chunks keeps between its two kernels: scratch memory of the runner, one buffer for every program and layer."""
+    return ctx.scratch.get("chunks", ops.channel_chunk_work(rows.shape[0], ctx.n_segments, heads, state_rows, state_cols, delta=delta),
+                           torch.float32, rows.device)
+
+
+def _scan(ctx, tag, q, k, v, decay, out, state, heads, rows, cols, silu=False, step=None, **kw):
+    """ops.linear_scan over the step's segments: portions chunk by chunk on the matrix cores (at every size measured, one
+    portion of 33 rows to 32 of 64 and one of 4,096, faster than row by row: `ops.linear_chunks`), else row by row, where the
+    segments of a step with long portions are walked in pieces."""
     T = v.shape[0]
+    if not silu and ops.channel_chunked(T, ctx.n_segments, ctx.decode_only):
+        work = _chunk_work(ctx, v, heads, rows, cols, False)
+        return ops.linear_chunks(q, k, v, decay, out, state, ctx.seg_start, ctx.state_slots, heads, rows, cols, work, step=step, **kw)
     piece = ops.scan_piece(T, ctx.decode_only)
     carry = None
     if piece:
         n, n_decay = ops.scan_carry(T, piece, heads, rows, cols, decay.shape[1] != heads)
         carry = (ctx.buffer(tag + ".carry", (n,), torch.float32), ctx.buffer(tag + ".carry_decay", (n_decay,), torch.float32))
-    return ops.linear_scan(q, k, v, decay, out, state, ctx.seg_start, ctx.state_slots, heads, rows, cols, piece=piece, carry=carry, **kw)
+    return ops.linear_scan(q, k, v, decay, out, state, ctx.seg_start, ctx.state_slots, heads, rows, cols, piece=piece, carry=carry,
+                           silu=silu, step=step, **kw)
 
 
 class GatedLinearAttention(Mixer):
@@ -274,6 +312,10 @@ class GatedDeltaRule(Mixer):
         self.qk, self.inner = kv_heads * dim, heads * vdim
         self.channels = 2 * self.qk + self.inner           # what the convolution runs over: q, k, v
         self.names = {**self.NAMES, **(names or {})}
+        self.by_chunks = DeltaByChunks(heads)
+
+    def step_arrays(self):
+        return [] if self.by_chunks is None else [self.by_chunks]
 
     def _tensor(self, which):
         return f"{self.name}.{self.names[which]}"
@@ -322,8 +364,13 @@ class GatedDeltaRule(Mixer):
                       gates=(proj[:, ch:ch + nh], self.dt_bias, self.a_log, step, decay), single_rows=ctx.decode_only)
         ops.unit_heads(qkv[:, :2 * qk], 2 * self.kv_heads, self.dim, eps=self.unit_eps)
         o = ctx.buffer("delta.o", (T, inner), torch.float32)
-        ops.delta_scan(qkv[:, :qk], qkv[:, qk:2 * qk], qkv[:, 2 * qk:], decay, proj[:, ch + nh:ch + 2 * nh], o, state,
-                       ctx.seg_start, ctx.state_slots, nh, self.dim, self.vdim, share=nh // self.kv_heads, q_scale=self.dim ** -0.5)
+        operands = (qkv[:, :qk], qkv[:, qk:2 * qk], qkv[:, 2 * qk:], decay, proj[:, ch + nh:ch + 2 * nh], o, state,
+                    ctx.seg_start, ctx.state_slots, nh, self.dim, self.vdim)
+        law = dict(share=nh // self.kv_heads, q_scale=self.dim ** -0.5)
+        if ctx.step_array(self.by_chunks)[1]:
+            ops.channel_delta_chunks(*operands, _chunk_work(ctx, o, nh, self.dim, self.vdim, True), **law)
+        else:
+            ops.delta_scan(*operands, **law)
         act = ops.group_norm_gate(o, proj[:, ch + 2 * nh:ch + 2 * nh + inner], self.norm_weight, ctx.buffer("delta.act", (T, inner), ctx.dtype),
                                   nh, self.eps, gate_first=False, shared_weight=True)
         return act
@@ -348,6 +395,7 @@ class ChannelDeltaRule(GatedDeltaRule):
     def __init__(self, name, hidden, heads, kv_heads, dim, vdim, taps, eps, unit_eps=1e-6, rank=None, names=None):
         """`rank`: the inner size of the low-rank projections where no file says it (`dim` unless given)."""
         super().__init__(name, hidden, heads, kv_heads, dim, vdim, taps, eps, unit_eps=unit_eps, names=names)
+        self.by_chunks = None
         self.rank = int(rank) if rank is not None else dim
 
     def tensor_specs(self):

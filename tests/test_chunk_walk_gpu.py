@@ -1,0 +1,89 @@
+"""The walk of a recurrence by chunks of 16 rows (csrc/recurrence_chunk.hip) against the recurrences row by row in 64 bits: the delta
+rule with one decay a head and the linear scan with either kind of decay (the rule with a decay a channel has tests of its own)."""
+import numpy as np
+import pytest
+import torch
+
+from plain_ditazen import delta_scan
+from plain_novosun import decayed_outer_scan
+
+DEV = "cuda:0"
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(torch.float32).to(DEV)
+
+
+def ints(a):
+    return torch.tensor(list(a), dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("law, heads, share, R, C", [
+    ("delta", 4, 2, 128, 128), ("delta", 3, 1, 20, 13), ("delta", 2, 2, 256, 33), ("channel", 3, 1, 128, 80), ("channel", 2, 1, 5, 3),
+    ("channel", 2, 2, 200, 17), ("head", 6, 6, 128, 64), ("head", 4, 2, 16, 65), ("head", 1, 1, 77, 16)])
+def test_chunks_against_the_recurrence_row_by_row(law, heads, share, R, C):
+    """Segments of none, one, fifteen, sixteen, seventeen rows and several chunks, in slabs that cut them, from states that are
+    not zero; some decays are zero; work space and results hold NaN before.  The bound is that of the scans row by row."""
+    from runtime.kernels import ops
+    rng = np.random.default_rng(R + C)
+    counts, slots = [17, 0, 1, 83, 15, 16], [3, 6, 0, 5, 1, 4]
+    T, starts = sum(counts), np.concatenate(([0], np.cumsum(counts)))
+    vec, is_delta = law == "channel", law == "delta"
+    groups = heads // share
+    q, k, v = (rng.standard_normal((T, n, d)) for n, d in ((groups, R), (groups, R), (heads, C)))
+    k /= np.sqrt((k * k).sum(-1, keepdims=True))
+    g = rng.uniform(0.6, 1.0, (T, heads, R if vec else 1))
+    g[rng.random(g.shape) < 0.02] = 0.0
+    b = rng.standard_normal((T, heads)) * 2 if is_delta else rng.uniform(0.1, 2.0, (T, heads))
+    begun = rng.standard_normal((7, heads, R, C))
+    state = torch.full((7, heads * R * C + 3), 9.0, device=DEV)
+    state[:, :heads * R * C] = dev(begun.reshape(7, -1))
+    out = torch.full((T, heads * C), float("nan"), device=DEV)
+    wide = torch.full((T, groups * R * 2 + 5), 7.0, device=DEV)                     # (q and k as columns of wider rows)
+    wide[:, 1:1 + groups * R], wide[:, 2 + groups * R:2 + 2 * groups * R] = dev(q.reshape(T, -1)), dev(k.reshape(T, -1))
+    operands = (wide[:, 1:1 + groups * R], wide[:, 2 + groups * R:2 + 2 * groups * R], dev(v.reshape(T, -1)), dev(g.reshape(T, -1)))
+    work = torch.full((ops.channel_chunk_work(T, len(counts), heads, R, C, slab=5, delta=is_delta),), float("nan"), device=DEV)
+    sizes, kw = (state, ints(starts), ints(slots), heads, R, C, work), dict(share=share, q_scale=0.37, slab=5)
+    if is_delta:
+        ops.channel_delta_chunks(*operands, dev(b), out, *sizes, **kw)
+    else:
+        ops.linear_chunks(*operands, out, *sizes, step=None if vec else dev(b), **kw)
+    got, after = out.cpu().numpy().reshape(T, heads, C), state.cpu().numpy()
+    for s, slot in enumerate(slots):
+        rows = slice(starts[s], starts[s + 1])
+        for h in range(heads):
+            S = begun[slot, h]
+            for t in range(rows.start, rows.stop):
+                kk, qq, dd = k[t, h // share], q[t, h // share], np.broadcast_to(g[t, h], (R,))
+                S = dd[:, None] * S
+                u = (v[t, h] - S.T @ kk) / (1.0 + np.exp(-b[t, h])) if is_delta else v[t, h] * (1.0 if vec else b[t, h])
+                S = S + np.outer(kk, u)
+                want = 0.37 * (S.T @ qq)
+                assert np.abs(got[t, h] - want).max() < 2e-5 * max(1.0, np.abs(want).max()), (s, t, h)
+            mine = after[slot, h * R * C:(h + 1) * R * C].reshape(R, C)
+            assert np.abs(mine - S).max() < 2e-5 * np.abs(S).max(), (s, h)
+    assert (after[:, heads * R * C:] == 9.0).all() and np.array_equal(after[[2, 6], :-3], begun[[2, 6]].reshape(2, -1).astype(np.float32))
+
+
+def test_the_oracle_is_the_designs_recurrence():
+    """The loop above is the designs' plain recurrences (from a state of zero, for one head)."""
+    rng = np.random.default_rng(1)
+    q, k, v, g, b = rng.standard_normal((9, 4)), rng.standard_normal((9, 4)), rng.standard_normal((9, 3)), rng.uniform(0.5, 1, (9, 1)), rng.uniform(0.1, 0.9, 9)
+    for is_delta in (True, False):
+        S, out = np.zeros((4, 3)), []
+        for t in range(9):
+            S = g[t][:, None] * S
+            S = S + np.outer(k[t], b[t] * (v[t] - S.T @ k[t]) if is_delta else v[t])
+            out.append(S.T @ q[t])
+        want = delta_scan(q, k, v, b, g[:, 0]) if is_delta else decayed_outer_scan(q, k, v, np.repeat(g, 4, 1))
+        np.testing.assert_allclose(out, want, rtol=1e-10, atol=1e-12)
+
+
+def test_which_steps_walk_the_delta_rule_by_chunks():
+    from runtime.engine.context import Batch
+    from runtime.parts.recurrent import DeltaByChunks
+    value = lambda heads, counts: DeltaByChunks(heads).launch_value(Batch(counts, [0] * len(counts), None, all(n == 1 for n in counts), {}))
+    assert value(32, [2048]) == value(32, [1] * 37 + [1024]) == value(16, [256] * 8) == 1
+    assert value(32, [1] * 64) == value(32, [20]) == value(32, [32] * 8) == value(16, [64] * 32) == 0
+    assert DeltaByChunks(32).words(100, 3) == 0
