@@ -137,19 +137,27 @@ class CacheManager:
             return self._append_one_each(items, commit)
         if not self.can_append(items):
             raise OutOfPages("not enough free KV pages for this step")
-        result = []
+        result, copied = [], {}
         for request, n in items:
             length = self.lengths[request]
             done = Appended(request, length, n, state_slot=self.slots.slot_of(request))
             for gid, group in enumerate(self.groups):
                 slots, copies = group.append(request, length, n)
                 done.slots[gid] = slots
-                if copies and self._copy_pages is not None:
-                    self._copy_pages(group, copies)
+                if copies:
+                    copied.setdefault(gid, []).extend(copies)
             if commit:
                 self.lengths[request] = length + n
             result.append(done)
+        self._run_copies(copied)
         return result
+
+    def _run_copies(self, copied):
+        """The page copies of a step, {group id: [(src, dst)]}, all of a group's at once.  (A source is shared while it is
+        copied and a destination fresh, so no copy of a step reads what another writes.)"""
+        if self._copy_pages is not None:
+            for gid, copies in copied.items():
+                self._copy_pages(self.groups[gid], copies)
 
     def commit(self, done):
         """The step that fills the slots of `done` (append_many with commit=False) is on its way: the tokens count.
@@ -188,7 +196,7 @@ class CacheManager:
                     fresh += 1
             if fresh > len(group.pool.free):
                 raise OutOfPages("not enough free KV pages for this step")
-        result = []
+        result, copied = [], {}
         for request, _ in items:
             length = lengths[request]
             done = Appended(request, length, 1, state_slot=self.slots.slot_of(request))
@@ -198,13 +206,12 @@ class CacheManager:
                     table.append(group.pool.allocate())
                     group._touch(request)
                 elif group.pool.refs[table[-1]] > 1:      # the shared, partly filled last page: copy on write
-                    slots, copies = group.append(request, length, 1)
-                    if copies and self._copy_pages is not None:
-                        self._copy_pages(group, copies)
+                    copied.setdefault(gid, []).extend(group.append(request, length, 1)[1])
                 done.slots[gid] = [table[-1] * P + length % P]
             if commit:
                 lengths[request] = length + 1
             result.append(done)
+        self._run_copies(copied)
         return result
 
     def trim(self, request):

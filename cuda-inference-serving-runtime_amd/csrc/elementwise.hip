@@ -591,24 +591,50 @@ extern "C" int cisr_rope_scatter(void* qkv, const int* positions, const int* slo
 }
 
 // ------------------------------------------------------------- page copy
-// Copy whole pages inside one cache tensor laid out [slabs, pages, page_elems]:
-// for every slab, page dst[i] := page src[i].  Used for copy-on-write of a
-// shared, partly filled page (reference: runtime/cache.py:70-75).
-__global__ void page_copy_kernel(uint32_t* __restrict__ pool, const int* __restrict__ src,
-                                 const int* __restrict__ dst, size_t page_words, size_t slab_words) {
-    const int pair = blockIdx.x, slab = blockIdx.y;
-    const uint32_t* s = pool + slab * slab_words + (size_t)src[pair] * page_words;
-    uint32_t* d = pool + slab * slab_words + (size_t)dst[pair] * page_words;
-    for (size_t i = threadIdx.x; i < page_words; i += blockDim.x) d[i] = s[i];
+// Copy whole pages inside one cache tensor laid out [slabs, pages, page bytes]: for every slab, page dst[i] := page src[i].
+// Used for copy-on-write of shared, partly filled pages (reference: runtime/cache.py:70-75): all the pages of a step in one
+// launch, their numbers among the kernel's arguments (an upload of two lists is two copies that the host waits for).  Bound
+// by the way to memory: a block copies 16 KB, a thread four 16-byte words that are on their way together.  A step in which
+// 62 requests leave shared pages at the 1.7B sizes (62 x 48 pages of 64 KB, read and written): 62 launches of 28.5 us (4
+// bytes a thread and trip, a block a page, and twice as many uploads) -> one of 70.
+#define COPY_PAIRS 128
+struct PagePairs { int src[COPY_PAIRS], dst[COPY_PAIRS]; };
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+page_copy_kernel(T* __restrict__ pool, PagePairs pairs, size_t page_words, size_t slab_words) {
+    const T* s = pool + blockIdx.y * slab_words + (size_t)pairs.src[blockIdx.x] * page_words;
+    T* d = pool + blockIdx.y * slab_words + (size_t)pairs.dst[blockIdx.x] * page_words;
+    const size_t at = (size_t)blockIdx.z * 1024 + threadIdx.x;
+    T v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = s[at + 256 * i < page_words ? at + 256 * i : page_words - 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (at + 256 * i < page_words) d[at + 256 * i] = v[i];
 }
 
+// src, dst: host memory.
 extern "C" int cisr_page_copy(void* pool, const int* src, const int* dst, int n_pairs, int slabs,
                               long long page_bytes, long long slab_bytes, hipStream_t stream) {
     if (n_pairs <= 0 || slabs <= 0) return 0;
-    if (page_bytes % 4 || slab_bytes % 4) return (int)hipErrorInvalidValue;
-    page_copy_kernel<<<dim3(n_pairs, slabs), 256, 0, stream>>>((uint32_t*)pool, src, dst,
-        (size_t)(page_bytes / 4), (size_t)(slab_bytes / 4));
-    return CISR_LAUNCH_CHECK();
+    if (page_bytes % 4 || slab_bytes % 4 || page_bytes <= 0) return (int)hipErrorInvalidValue;
+    const bool wide = page_bytes % 16 == 0 && slab_bytes % 16 == 0 && (uintptr_t)pool % 16 == 0;
+    const long long words = page_bytes / (wide ? 16 : 4), parts = (words + 1023) / 1024;
+    if (parts > 65535) return (int)hipErrorInvalidValue;
+    for (int first = 0; first < n_pairs; first += COPY_PAIRS)
+        for (int slab = 0; slab < slabs; slab += 65535) {
+            PagePairs pairs = {};
+            const int n = n_pairs - first < COPY_PAIRS ? n_pairs - first : COPY_PAIRS;
+            for (int i = 0; i < n; ++i) { pairs.src[i] = src[first + i]; pairs.dst[i] = dst[first + i]; }
+            const dim3 grid(n, slabs - slab < 65535 ? slabs - slab : 65535, (unsigned)parts);
+            char* base = (char*)pool + (long long)slab * slab_bytes;
+            if (wide) page_copy_kernel<uint4><<<grid, 256, 0, stream>>>((uint4*)base, pairs, (size_t)words, (size_t)(slab_bytes / 16));
+            else page_copy_kernel<uint32_t><<<grid, 256, 0, stream>>>((uint32_t*)base, pairs, (size_t)words, (size_t)(slab_bytes / 4));
+            const int err = CISR_LAUNCH_CHECK();
+            if (err) return err;
+        }
+    return 0;
 }
 
 // ------------------------------------------------------------- conversions

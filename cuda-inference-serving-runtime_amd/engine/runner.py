@@ -124,9 +124,7 @@ class ModelRunner:
         return self.cache.length(request)
 
     def _copy_pages(self, group, copies):
-        src = torch.tensor([c[0] for c in copies], dtype=torch.int32, device=self.device)
-        dst = torch.tensor([c[1] for c in copies], dtype=torch.int32, device=self.device)
-        ops.page_copy(group.storage, src, dst, group.need.slabs(len(group.sites)), group.pool.n_pages)
+        ops.page_copy(group.storage, [c[0] for c in copies], [c[1] for c in copies], group.need.slabs(len(group.sites)), group.pool.n_pages)
 
     def carry(self, array):
         """From the next step on, every step's metadata holds the step array `array`."""

@@ -311,15 +311,19 @@ def rope_scatter(qkv, positions, slots, cos, sin, kcache, vcache, heads, kv_head
 
 
 def page_copy(pool, src, dst, slabs, pages_per_slab):
-    """pool viewed as [slabs, pages_per_slab, page]: page dst[i] := page src[i] in every slab."""
-    n = src.shape[0]
+    """pool viewed as [slabs, pages_per_slab, page]: page dst[i] := page src[i] in every slab.  src, dst: page numbers
+    (sequences, or tensors, which are read back first); no page is both a source and a destination."""
+    src, dst = ([int(x) for x in (t.tolist() if isinstance(t, torch.Tensor) else t)] for t in (src, dst))
+    n = len(src)
     total = pool.numel() * pool.element_size()
     if total % (slabs * pages_per_slab):
         raise KernelError("page_copy: pool does not divide into slabs and pages")
+    if len(dst) != n or any(not 0 <= x < pages_per_slab for x in src + dst):
+        raise KernelError("page_copy: as many sources as destinations, all of them pages of the pool")
     slab_bytes = total // slabs
     page_bytes = slab_bytes // pages_per_slab
-    _check(lib().cisr_page_copy(_dev(pool, "pool"), _dev(src, "src", torch.int32, (n,)), _dev(dst, "dst", torch.int32, (n,)),
-                                n, slabs, page_bytes, slab_bytes, _stream()), "page_copy")
+    numbers = C.c_int * n
+    _check(lib().cisr_page_copy(_dev(pool, "pool"), numbers(*src), numbers(*dst), n, slabs, page_bytes, slab_bytes, _stream()), "page_copy")
 
 
 def f32_to_bf16(x, out):

@@ -1294,6 +1294,19 @@ def test_page_copy(ops):
     assert torch.equal(pool[:, :, [1, 2, 4]], before[:, :, [1, 2, 4]])
 
 
+@pytest.mark.parametrize("slabs, pages, words, pairs", [(3, 5, 1, 2), (2, 300, 10, 140), (1, 4, 4 * 1024 + 4, 1), (48, 9, 16384, 4), (2, 6, 1027, 3)])
+def test_page_copies_of_a_step_in_one_call(ops, slabs, pages, words, pairs):
+    """Pages of one word, of whole and broken 16-byte runs, of more than a block's share; more pairs than a launch takes."""
+    pool = torch.randint(-2 ** 31, 2 ** 31 - 1, (slabs, pages, words), dtype=torch.int32, device=DEV)
+    before, order = pool.clone(), np.random.default_rng(words).permutation(pages).tolist()
+    src, dst = order[:pairs], order[-pairs:]
+    ops.page_copy(pool, src, dst, slabs, pages)
+    before[:, dst] = before[:, src].clone()
+    assert torch.equal(pool, before)
+    with pytest.raises(ops.KernelError):
+        ops.page_copy(pool, [0], [pages], slabs, pages)
+
+
 def test_kernels_refuse_what_they_cannot_take(ops):
     from runtime.kernels.ops import KernelError
     with pytest.raises(KernelError, match="head size"):
