@@ -46,10 +46,9 @@ route_kernel(const float* __restrict__ logits, int ld, const float* __restrict__
     }
 }
 
-__global__ void __launch_bounds__(1024)
-arrange_kernel(const int* __restrict__ chosen, int pairs, int experts, int max_tiles, int* __restrict__ pair_of_pos,
-               int* __restrict__ tile_expert) {
-    extern __shared__ int lds[];          // counts[E], then start[E] (in places), then cursor[E]
+// lds: counts[E], then start[E] (in places), then cursor[E]; `chosen` in memory or in LDS.  All 1,024 threads call it.
+__device__ __forceinline__ void arrange_pairs(const int* chosen, int pairs, int experts, int max_tiles, int* __restrict__ pair_of_pos,
+                                              int* __restrict__ tile_expert, int* lds) {
     int* counts = lds;
     int* start = lds + experts;
     int* cursor = lds + 2 * experts;
@@ -82,6 +81,58 @@ arrange_kernel(const int* __restrict__ chosen, int pairs, int experts, int max_t
     }
 }
 
+__global__ void __launch_bounds__(1024)
+arrange_kernel(const int* __restrict__ chosen, int pairs, int experts, int max_tiles, int* __restrict__ pair_of_pos,
+               int* __restrict__ tile_expert) {
+    extern __shared__ int lds[];
+    arrange_pairs(chosen, pairs, experts, max_tiles, pair_of_pos, tile_expert, lds);
+}
+
+// Route and arrange of a step of few rows in one block: the logits (and bias) come into LDS all at once, where a thread a row
+// chooses as route_kernel does, then the pairs are arranged.  24 rows of 16 experts: 6.3 + 4.7 us as two kernels (a thread's
+// logits come one trip after the other) -> 7.3.
+#define ROUTE_ONE_BLOCK 8192         // rows times experts, at most
+__global__ void __launch_bounds__(1024)
+route_arrange_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ bias, int* __restrict__ chosen,
+                     float* __restrict__ weights, int rows, int experts, int top, int max_tiles, int* __restrict__ pair_of_pos,
+                     int* __restrict__ tile_expert) {
+    extern __shared__ int lds[];                                  // arrange's 3 E, the choices [rows * top], the logits [rows * (E + 1)]
+    int* picked = lds + 3 * experts;
+    float* z = (float*)(picked + rows * top);
+    for (int i = threadIdx.x; i < rows * experts; i += 1024) {
+        const int row = i / experts, e = i % experts;
+        z[row * (experts + 1) + e] = logits[(size_t)row * ld + e] + (bias ? bias[e] : 0.f);
+    }
+    __syncthreads();
+    for (int row = threadIdx.x; row < rows; row += 1024) {
+        const float* lr = z + row * (experts + 1);
+        int ids[MAX_TOP];
+        float vals[MAX_TOP];
+        for (int k = 0; k < top; ++k) {
+            int best = -1;
+            float bv = -INFINITY;
+            for (int e = 0; e < experts; ++e) {
+                bool taken = false;
+                for (int j = 0; j < k; ++j) taken |= ids[j] == e;
+                if (taken) continue;
+                const float v = lr[e];
+                if (best < 0 || v > bv) { best = e; bv = v; }
+            }
+            ids[k] = best;
+            vals[k] = bv;
+        }
+        float den = 0.f;
+        const float largest = vals[0];
+        for (int k = 0; k < top; ++k) { vals[k] = expf(vals[k] - largest); den += vals[k]; }
+        for (int k = 0; k < top; ++k) {
+            picked[row * top + k] = chosen[(size_t)row * top + k] = ids[k];
+            weights[(size_t)row * top + k] = vals[k] / den;
+        }
+    }
+    __syncthreads();
+    arrange_pairs(picked, rows * top, experts, max_tiles, pair_of_pos, tile_expert, lds);
+}
+
 extern "C" int cisr_experts_route(const float* logits, int ld, const float* bias, int* chosen, float* weights, int rows,
                                   int experts, int top, int max_tiles, int* pair_of_pos, int* tile_expert, hipStream_t stream) {
     if (rows <= 0) return 0;
@@ -89,6 +140,12 @@ extern "C" int cisr_experts_route(const float* logits, int ld, const float* bias
     if (experts <= 0 || top <= 0 || top > MAX_TOP || top > experts || experts > 4096 || (arrange && (!tile_expert ||
         (long long)max_tiles * EX_TILE < (long long)rows * top + (long long)experts * (EX_TILE - 1))))
         return (int)hipErrorInvalidValue;
+    // (the choices, the logits and what arrange needs fit 64 KB: 8,192 logits, up to sixteen choices of 512 rows of 16 experts)
+    const size_t together = ((size_t)3 * experts + (size_t)rows * top + (size_t)rows * (experts + 1)) * sizeof(int);
+    if (arrange && (long long)rows * experts <= ROUTE_ONE_BLOCK && together <= 65536) {
+        route_arrange_kernel<<<1, 1024, together, stream>>>(logits, ld, bias, chosen, weights, rows, experts, top, max_tiles, pair_of_pos, tile_expert);
+        return CISR_LAUNCH_CHECK();
+    }
     route_kernel<<<(rows + 255) / 256, 256, 0, stream>>>(logits, ld, bias, chosen, weights, rows, experts, top);
     int err = CISR_LAUNCH_CHECK();
     if (err || !arrange) return err;

@@ -93,6 +93,7 @@ def _declare(h):
         "cisr_experts_route_scored": [p, i, p, p, p, i, i, i, i, i, i, i, i, f, i, p, p, p],
         "cisr_experts_route_product": [p, i, p, i, i, p, p, p, p, i, i, i, i, i, i, i, i, f, i, p, p, p],
         "cisr_attn_merge_gated": [p, p, p, i, i, i, i, p, i, i, p],
+        "cisr_experts_few": [p, i, p, p, p, i, i, p, i, i, i, i, i, i, f, f, f, p],
         "cisr_experts_gemm_gated": [p, i, p, p, p, i, p, i, i, i, i, f, f, f, p],
         "cisr_side_rows": [p, i, p, p, p, i, i, p, i, i, i, i, i, p],
         "cisr_experts_add": [p, p, p, p, p, p, i, i, i, i, i, p, f, p, i, p],
@@ -2195,6 +2196,28 @@ def experts_rows_gated(a, w, chosen, out, law, top=0):
     return out
 
 
+# A step's tiles stream the experts' matrices up to this many pairs an expert on the mean, and up to this inner size.  Measured
+# on an MI355X (the other kernel / the streaming one, us): 16 experts of 4096 x 2048, 48 pairs 64 / 50, 128 pairs 68 / 57, 256
+# pairs 69 / 61, 400 pairs 70 / 81; gated, of 2 x 1024 x 2048, 96 pairs 42 / 35, 512 pairs 45 / 38, 1,024 pairs 48 / 62; of
+# 2048 x 1024, 96 and 512 pairs 20 / 16 and 21 / 25; 64 experts of 1024 x 512, 256 pairs 16.6 / 17.1, 1,024 pairs 18 / 20.  With
+# an inner size of 4,096 a wave's stream is too long for the few waves there are: 48 pairs against 2048 x 4096 63 / 69.
+EXPERT_FEW_PAIRS, EXPERT_FEW_K = 8, 2048
+
+
+def experts_few_ok(a, w, tiles):
+    """Whether the experts' tiles run the kernel that streams the matrices (csrc/experts_few.hip): bf16 with 16-byte rows, and
+    few pairs an expert.  (`tiles` = experts + pairs / 64 rounded up: a function of a captured program's rows.)"""
+    experts, _, k = w.shape
+    return (experts_gemm_gated_ok(a, w) and 8 <= k <= EXPERT_FEW_K and EXPERT_TILE * (tiles - experts) <= EXPERT_FEW_PAIRS * experts)
+
+
+def _experts_few(a, w, pair_of_pos, tile_expert, out, top, scatter, n, act, law=(0.0, 0.0, 0.0)):
+    _check(lib().cisr_experts_few(a.data_ptr(), a.stride(0), _dev(w, "w"), _dev(tile_expert, "tile_expert", torch.int32),
+                                  _dev(pair_of_pos, "pair_of_pos", torch.int32), int(top), int(bool(scatter)), _dev(out, "out"), out.stride(0),
+                                  tile_expert.shape[0], n, w.shape[2], act, _storage(out, "out"), *(float(v) for v in law), _stream()), "experts_few")
+    return out
+
+
 def experts_gemm(a, w, pair_of_pos, tile_expert, out, top=0, scatter=False, act=False):
     """out[row of place] = act(a[row of place] . w[expert of the place's tile]^T) over the places that experts_route
     laid out.  w [experts, N, K]; `top` > 0: a place's operand is row pair // top of `a` (the step's rows), else the
@@ -2210,6 +2233,8 @@ def experts_gemm(a, w, pair_of_pos, tile_expert, out, top=0, scatter=False, act=
         raise KernelError("experts_gemm: the places do not fit the tiles")
     if (top <= 0 and a.shape[0] < places) or (not scatter and out.shape[0] < places):
         raise KernelError("experts_gemm: operands by place need a row a place")
+    if experts_few_ok(a, w, tiles):
+        return _experts_few(a, w, pair_of_pos, tile_expert, out, top, scatter, n, int(bool(act)))
     _check(lib().cisr_experts_gemm(_dev(a, "a") if a.is_contiguous() else a.data_ptr(), a.stride(0), _dev(w, "w"),
                                    _dev(tile_expert, "tile_expert", torch.int32), _dev(pair_of_pos, "pair_of_pos", torch.int32),
                                    int(top), int(bool(scatter)), _dev(out, "out"), out.stride(0), tiles, n, k, int(bool(act)),
@@ -2232,6 +2257,8 @@ def experts_gemm_gated(a, w, pair_of_pos, tile_expert, out, law, top=0):
         raise KernelError("experts_gemm_gated: shape not supported")
     if out.dim() != 2 or out.shape[1] != n2 // 2 or out.shape[0] < places or (top <= 0 and a.shape[0] < places):
         raise KernelError("experts_gemm_gated: operands and results by place need a row a place")
+    if experts_few_ok(a, w, tiles):
+        return _experts_few(a, w, pair_of_pos, tile_expert, _dev(out, "out", torch.bfloat16) and out, top, False, n2 // 2, 2, law)
     _check(lib().cisr_experts_gemm_gated(a.data_ptr(), a.stride(0), _dev(w, "w"), _dev(tile_expert, "tile_expert", torch.int32),
                                          _dev(pair_of_pos, "pair_of_pos", torch.int32), int(top), _dev(out, "out", torch.bfloat16), out.stride(0),
                                          tiles, n2 // 2, k, *(float(v) for v in law), _stream()), "experts_gemm_gated")
