@@ -241,6 +241,17 @@ extern "C" int cisr_attn_merge(const float* part_o, const float* part_ml, void* 
     return CISR_LAUNCH_CHECK();
 }
 
+// merge of float partials (natural logarithms) of csrc/attention_f32.hip
+extern "C" int cisr_attn_merge_f32(const float* part_o, const float* part_ml, float* out, int rows, int heads, int dim, int splits,
+                                   hipStream_t stream) {
+    if (rows <= 0) return 0;
+    if (heads > 65535 || splits < 1) return (int)hipErrorInvalidValue;
+    const int threads = merge_threads(dim);
+    if (splits <= 16) attn_merge_kernel<float, false, false><<<dim3(rows, heads), threads, 0, stream>>>(part_o, part_ml, out, heads, dim, splits);
+    else attn_merge_kernel<float, false, true><<<dim3(rows, heads), threads, 0, stream>>>(part_o, part_ml, out, heads, dim, splits);
+    return CISR_LAUNCH_CHECK();
+}
+
 // the same with the heads packed to vdim coordinates and gated element by element (float gates)
 extern "C" int cisr_attn_merge_gated(const float* part_o, const float* part_ml, void* out, int rows, int heads, int dim, int splits,
                                      const float* gate, int ld_gate, int vdim, hipStream_t stream) {

@@ -210,6 +210,12 @@ def rowwise_splits(waves, span):
     return int(min(32, -(-span // 256), max(1, 4096 // waves)))
 
 
+def f32_splits(blocks, span):
+    """Blocks that share a tile's keys in the float matrix-instruction kernel: until there is a block for every compute unit,
+    each of whose eight waves keeps three 16-key steps (a merge costs what two steps take)."""
+    return int(max(1, min(256 // max(blocks, 1), span // 384, 32)))
+
+
 def rows_launch(blocks, span, heads_per_chunk, head_dim):
     """Matrix-core decode kernel: (wavefronts a block, blocks along the keys).  Few rows:
     eight waves share a row's keys inside one block; when that still leaves the GPU idle
@@ -333,6 +339,16 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
     law = dict(head_bias=head_bias, slopes=slopes, sink=sink, keep_first=keep_first)
     common = (q, q_row_stride, kcache, vcache, view.tables, ctx.seg_of_row, ctx.positions, out, heads, kv_heads, head_dim,
               view.page_size, window, scale)
+    if (head_bias is None and slopes is None and sink is None and not keep_first
+            and ops.attention_f32_ok(q, q_row_stride, kcache, vcache, head_dim, view.page_size)):
+        tasks, _ = ctx.step_array(TileTasks(16 // min(heads // kv_heads, 16)))
+        tasks = tasks.view(-1, 4)
+        blocks = (rows if ctx.decode_only else tasks.shape[0]) * kv_heads * -(-(heads // kv_heads) // 16)
+        splits = f32_splits(blocks, span)
+        workspace = _split_workspace(ctx, rows, heads, splits, head_dim) if splits > 1 else None
+        ops.attention_f32(q, q_row_stride, kcache, vcache, view.tables, ctx.positions, tasks, out, heads, kv_heads, head_dim, view.page_size,
+                          window, scale, splits, workspace)
+        return None
     if not ops.mfma_attention_supported(out.dtype, head_dim, view.page_size):
         splits = rowwise_splits(rows * heads, span)
         workspace = _split_workspace(ctx, rows, heads, splits, head_dim) if splits > 1 else None

@@ -55,6 +55,9 @@ def _declare(h):
         "cisr_gemm_bf16_swiglu_tile": [p, i, p, i, p, i, i, i, i, i, i, p],
         "cisr_gemm_skinny_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, p, f, p, p],
         "cisr_qkv_rope_skinny": [p, i, p, i, p, i, i, i, p, f, p, p, p, p, p, p, i, i, i, i, i, p],
+        "cisr_attn_f32": [p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, f, i, p],
+        "cisr_attn_f32_ok": [i, i],
+        "cisr_attn_merge_f32": [p, p, p, i, i, i, i, p],
         "cisr_attn_merge": [p, p, p, i, i, i, i, p, p],
         "cisr_argmax": [p, p, p, i, p, p, i, i, p],
         "cisr_sample": [p, p, p, p, p, p, i, i, i, p],
@@ -380,6 +383,38 @@ def attention_rowwise(q, q_row_stride, kcache, vcache, tables, seg_of_row, posit
         _check(lib().cisr_attn_rowwise(*args, None if slopes is None else _dev(slopes, "slopes", torch.float32, (heads,)),
                                        None if sink is None else _dev(sink, "sink", torch.float32, (heads,)), int(keep_first), _stream()),
                "attention_rowwise")
+    return out
+
+
+def attention_f32_ok(q, q_row_stride, kcache, vcache, dim, page_size):
+    """Whether attention_f32 takes these operands (the softmax law only)."""
+    return (q.dtype == torch.float32 and q_row_stride % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in (q, kcache, vcache))
+            and bool(lib().cisr_attn_f32_ok(int(dim), int(page_size))))
+
+
+def attention_f32(q, q_row_stride, kcache, vcache, tables, positions, tasks, out, heads, kv_heads, dim, page_size, window, scale,
+                  splits=1, workspace=None):
+    """attention_rowwise's softmax law for float operands on the float matrix instruction, over `tasks` (int32 [n, 4]: tiles of
+    rows of one segment, at most 16 // min(heads / kv_heads, 16) rows each; rows that no task names are left alone)."""
+    rows, pages = out.shape[0], kcache.shape[0]
+    if not attention_f32_ok(q, q_row_stride, kcache, vcache, dim, page_size) or heads % kv_heads:
+        raise KernelError("attention_f32: operands not supported")
+    if q.numel() < (rows - 1) * q_row_stride + heads * dim:
+        raise KernelError("attention: q buffer too small for its stride")
+    po = pm = None
+    if splits > 1:
+        part_o, part_ml = workspace
+        po, pm = _dev(part_o, "part_o", torch.float32), _dev(part_ml, "part_ml", torch.float32)
+        if part_o.numel() < rows * heads * splits * dim or part_ml.numel() < rows * heads * splits * 2:
+            raise KernelError("attention: split workspace too small")
+    op = _dev(out, "out", torch.float32, (rows, heads * dim))
+    _check(lib().cisr_attn_f32(q.data_ptr(), q_row_stride, _dev(kcache, "kcache", torch.float32, (pages, kv_heads, page_size, dim)),
+                               _dev(vcache, "vcache", torch.float32, (pages, kv_heads, dim, page_size)), _dev(tables, "tables", torch.int32),
+                               _dev(positions, "positions", torch.int32, (rows,)), _dev(tasks, "tasks", torch.int32, (tasks.shape[0], 4)),
+                               tasks.shape[0], op, po, pm, heads, kv_heads, dim, page_size, tables.shape[1], int(window or 0), float(scale),
+                               int(splits), _stream()), "attention_f32")
+    if splits > 1:
+        _check(lib().cisr_attn_merge_f32(po, pm, op, rows, heads, dim, int(splits), _stream()), "attention_merge")
     return out
 
 

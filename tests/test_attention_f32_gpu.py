@@ -1,0 +1,66 @@
+"""The 32-bit path's attention on the float matrix instruction (csrc/attention_f32.hip) against attention row by row in 64 bits."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from test_kernels_gpu import DEV, f64, paged_case, reference_attention, rnd, tol
+
+pytestmark = pytest.mark.gpu
+
+
+def tasks_of(rows, per):
+    """Tiles of at most `per` neighbouring rows of one segment, a tile of no segment among them."""
+    tasks, at = [(-1, 0, 0, 0)], 0
+    while at < len(rows):
+        n = 1
+        while n < per and at + n < len(rows) and rows[at + n][0] == rows[at][0] and rows[at + n][1] == rows[at][1] + n:
+            n += 1
+        tasks.append((rows[at][0], at, n, 0))
+        at += n
+    return torch.tensor(tasks, dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim, page_size", [(9, 3, 64, 16), (4, 4, 32, 4), (8, 1, 128, 8), (20, 1, 96, 64), (16, 1, 64, 32), (34, 2, 32, 16)])
+@pytest.mark.parametrize("window", [None, 1, 9, 40])
+def test_attention_f32(heads, kv_heads, dim, page_size, window):
+    """Segments of one key to several hundred (more than a turn of the eight waves), tiles of whole prompts and of their ends, single
+    rows; groups of heads that fill a tile, leave some of it and take two; windows whose earlier pages are gone; more splits
+    than a short segment has keys.  Scores spread by 2.8, so that maxima move: up to about 13, whose rounding (a few of 2^-24 of it) moves a
+    weight by up to 3e-6 of itself and a result, values of up to 4, by 1e-5; the row-wise kernel's bound else."""
+    from runtime.kernels import ops
+    _, kt, vt, tables, _ = paged_case(heads, kv_heads, dim, page_size, [17, 7, 1, 330], torch.float32, seed=dim + heads)
+    group = heads // kv_heads
+    scale = 0.7 / math.sqrt(dim)
+    at = {0: range(10, 17), 1: range(4, 7), 2: [0], 3: [*(() if window else range(5)), 200, *range(290, 330)]}
+    rows = [(seg, pos) for seg, where in at.items() for pos in where]
+    qt = rnd(len(rows), heads, dim, seed=3, scale=4.0)
+    want = reference_attention(qt, kt, vt, tables, rows, page_size, window=window, scale=scale)
+    if window:                                             # pages that no row of a segment sees are gone, and hold NaN
+        tables = tables.clone()
+        for seg in range(tables.shape[0]):
+            low = min(pos for s, pos in rows if s == seg) + 1 - window
+            for j in range(max(0, low) // page_size):
+                kt[tables[seg, j]] = vt[tables[seg, j]] = float("nan")
+                tables[seg, j] = -1
+    T = len(rows)
+    pos = torch.tensor([r[1] for r in rows], dtype=torch.int32, device=DEV)
+    tasks = tasks_of(rows, 16 // min(group, 16))
+    wide = torch.full((T, heads * dim + 8), float("nan"), device=DEV)
+    wide[:, 4:4 + heads * dim] = qt.reshape(T, -1)
+    for splits in (1, 3, 33):
+        out = torch.full((T, heads * dim), 7.0, device=DEV)
+        ws = (torch.full((T * heads * splits * dim,), float("nan"), device=DEV), torch.full((T * heads * splits * 2,), float("nan"), device=DEV))
+        ops.attention_f32(wide.view(-1)[4:], wide.stride(0), kt, vt, tables, pos, tasks, out, heads, kv_heads, dim, page_size, window, scale, splits, ws)
+        np.testing.assert_allclose(f64(out).reshape(T, heads, dim), want, rtol=tol(torch.float32)["rtol"], atol=1e-5, err_msg=f"splits={splits}")
+
+
+def test_what_attention_f32_takes():
+    from runtime.kernels import ops
+    q = torch.zeros(4, 64, device=DEV)
+    kc = vc = torch.zeros(2, 1, 16, 64, device=DEV)
+    assert ops.attention_f32_ok(q, 64, kc, vc, 64, 16)
+    assert not any(ops.attention_f32_ok(q, 64, kc, vc, dim, page) for dim, page in ((48, 16), (256, 16), (64, 2), (64, 12)))
+    assert not ops.attention_f32_ok(q.bfloat16(), 64, kc, vc, 64, 16) and not ops.attention_f32_ok(q, 66, kc, vc, 64, 16)
+    assert not ops.attention_f32_ok(q.view(-1)[1:], 64, kc, vc, 64, 16)
