@@ -2,8 +2,8 @@
 // numpy/cupy argmax does in the reference, runtime/engine.py:99) and temperature
 // sampling p = softmax(logits / T) drawn by inverse CDF with a counter-based
 // random number per (seed, counter), so a request's draw does not depend on
-// what else is in the batch.  One block of 256 threads per row; every thread
-// owns one contiguous slice of the vocabulary, which fixes the summation order.
+// what else is in the batch.  The vocabulary is cut into 256 contiguous slices,
+// each summed in order, which fixes the summation order.
 #include "common.h"
 #include "cisr_noalloc.h"
 #include <stdio.h>
@@ -22,16 +22,18 @@ __device__ __forceinline__ float uniform01(uint64_t seed, uint64_t counter) {
     return (float)(h >> 40) * (1.0f / 16777216.0f);
 }
 
+template <int NT = 256>
 __device__ __forceinline__ void argmax_block(const float* __restrict__ x, int n, float* smax, int* sidx,
                                              float& best, int& best_idx) {
     float bv = -INFINITY; int bi = 0x7fffffff;
-    for (int i = threadIdx.x; i < n; i += 256) {
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += NT) {
         float v = x[i];
         if (bi == 0x7fffffff || v > bv) { bv = v; bi = i; }  // indices ascend: a tie keeps the lower one
     }
     smax[threadIdx.x] = bv; sidx[threadIdx.x] = bi;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
+    for (int s = NT / 2; s > 0; s >>= 1) {
         if (threadIdx.x < s) {
             float ov = smax[threadIdx.x + s]; int oi = sidx[threadIdx.x + s];
             float mv = smax[threadIdx.x]; int mi = sidx[threadIdx.x];
@@ -145,58 +147,105 @@ extern "C" int cisr_argmax_noalloc(const float* logits, int* out, int rows, int 
     return CISR_LAUNCH_CHECK();
 }
 
-__global__ void __launch_bounds__(256)
+// A block of 1,024 threads a row.  The weights exp((x - best) / T) are made by all of them, SAMPLE_STEP of every slice at a
+// time, read and left in LDS side by side; a thread a slice then adds its own in order, so the sums are those of a thread
+// that walks its slice alone.  The chosen slice's weights are made the same way before one thread walks them.  Bound by trips
+// to memory (three passes over the row out of the cache): 49,152 logits 100 us with 256 threads walking a slice each and one
+// walking the chosen one (78 in a graph of such calls, 38 so).
+#define SAMPLE_THREADS 1024
+#define SAMPLE_STEP 32
+__global__ void __launch_bounds__(SAMPLE_THREADS)
 sample_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
               const unsigned long long* __restrict__ seeds, const unsigned long long* __restrict__ counters,
               int* __restrict__ out, const int* __restrict__ index, int out_n, int vocab) {
-    __shared__ float smax[256];
-    __shared__ int sidx[256];
+    __shared__ float smax[SAMPLE_THREADS];
+    __shared__ int sidx[SAMPLE_THREADS];
     __shared__ float ssum[256];
-    const int row = blockIdx.x;
+    __shared__ float weight[256][SAMPLE_STEP + 1];
+    __shared__ float run_at;
+    __shared__ int slice_at;
+    const int row = blockIdx.x, tid = threadIdx.x;
     const int dst = index ? index[row] : row;
     if (dst < 0 || dst >= out_n) return;       // the whole block: no barrier is passed by a part of it
     const float* x = logits + (size_t)row * vocab;
     float best; int best_idx;
-    argmax_block(x, vocab, smax, sidx, best, best_idx);
+    argmax_block<SAMPLE_THREADS>(x, vocab, smax, sidx, best, best_idx);
     const float temp = temperature[row];
     if (!(temp > 0.f)) {  // greedy
-        if (threadIdx.x == 0) out[dst] = best_idx == 0x7fffffff ? 0 : best_idx;
+        if (tid == 0) out[dst] = best_idx == 0x7fffffff ? 0 : best_idx;
         return;
     }
     const float inv_t = 1.0f / temp;
     const int per = (vocab + 255) / 256;
-    const int lo = threadIdx.x * per, hi = min(vocab, lo + per);
-    float part = 0.f;
-    for (int i = lo; i < hi; ++i) part += expf((x[i] - best) * inv_t);
-    ssum[threadIdx.x] = part;
+    constexpr int TURNS = 256 * SAMPLE_STEP / SAMPLE_THREADS;        // words a thread makes of a step
+    float part = 0.f;                                                // (of slice tid, tid < 256)
+    for (int j0 = 0; j0 < per; j0 += SAMPLE_STEP) {
+        float v[TURNS];
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i) {
+            const int idx = tid + SAMPLE_THREADS * i, at = idx / SAMPLE_STEP * per + j0 + idx % SAMPLE_STEP;
+            v[i] = x[min(at, vocab - 1)];
+        }
+        __syncthreads();                                             // (the step before is added up)
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i) {
+            const int idx = tid + SAMPLE_THREADS * i;
+            weight[idx / SAMPLE_STEP][idx % SAMPLE_STEP] = expf((v[i] - best) * inv_t);
+        }
+        __syncthreads();
+        if (tid < 256) {
+            const int n = min(min(per - j0, SAMPLE_STEP), vocab - (tid * per + j0));
+#pragma unroll 8
+            for (int j = 0; j < n; ++j) part += weight[tid][j];
+        }
+    }
+    if (tid < 256) ssum[tid] = part;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         float total = 0.f;
+#pragma unroll 8
         for (int t = 0; t < 256; ++t) total += ssum[t];
         const float target = uniform01(seeds[row], counters[row]) * total;
-        // find the slice, then the token inside it; fall back to the last token
-        // with non-zero mass if rounding pushes the target past the end
-        float run = 0.f; int choice = -1;
+        // find the slice
+        float run = 0.f;
         int t = 0;
         for (; t < 256; ++t) { if (run + ssum[t] > target) break; run += ssum[t]; }
-        if (t < 256) {
-            const int a = t * per, b = min(vocab, a + per);
-            for (int i = a; i < b; ++i) {
-                run += expf((x[i] - best) * inv_t);
-                if (run > target) { choice = i; break; }
-            }
-            if (choice < 0) choice = b - 1;
-        }
-        if (choice < 0) choice = best_idx;
-        out[dst] = choice;
+        smax[0] = target;
+        run_at = run;
+        slice_at = t;
     }
+    __syncthreads();
+    const int t = slice_at;
+    const float target = smax[0];
+    int choice = -1;                                                 // (of thread 0)
+    if (t < 256) {
+        // then the token inside it; fall back to the last token with non-zero mass if rounding pushes the target past the end
+        const int a = t * per, b = min(vocab, a + per);
+        float run = run_at;
+        float* slice = &weight[0][0];
+        constexpr int ROOM = 256 * (SAMPLE_STEP + 1);
+        for (int a0 = a; a0 < b; a0 += ROOM) {
+            const int n = min(b - a0, ROOM);
+            __syncthreads();
+            for (int i = tid; i < n; i += SAMPLE_THREADS) slice[i] = expf((x[a0 + i] - best) * inv_t);
+            __syncthreads();
+            if (tid == 0 && choice < 0)
+                for (int i = 0; i < n; ++i) {
+                    run += slice[i];
+                    if (run > target) { choice = a0 + i; break; }
+                }
+        }
+        if (choice < 0) choice = b - 1;
+    }
+    if (choice < 0) choice = best_idx;
+    if (tid == 0) out[dst] = choice;
 }
 
 extern "C" int cisr_sample(const float* logits, const float* temperature, const unsigned long long* seeds,
                            const unsigned long long* counters, int* out, const int* index, int out_n, int rows, int vocab,
                            hipStream_t stream) {
     if (rows <= 0) return 0;
-    sample_kernel<<<rows, 256, 0, stream>>>(logits, temperature, seeds, counters, out, index, index ? out_n : rows, vocab);
+    sample_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(logits, temperature, seeds, counters, out, index, index ? out_n : rows, vocab);
     return CISR_LAUNCH_CHECK();
 }
 
