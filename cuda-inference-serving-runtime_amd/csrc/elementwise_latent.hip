@@ -269,6 +269,19 @@ __global__ void __launch_bounds__(256) gelu_kernel(const T* __restrict__ x, T* _
     if (i < n) store_f32(out + i, unary_activation(load_f32(x + i), kind + 1));
 }
 
+// The same for bf16 in 16-byte words: 2,048 rows of 8,192 39.5 us an element a thread (2-byte accesses), 19.6 so.
+__global__ void __launch_bounds__(256) gelu_bf16x8_kernel(const uint4* __restrict__ x, uint4* __restrict__ out, size_t n8, int kind) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const uint4 v = x[i];
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        y[e] = pack_bf16x2(unary_activation(__uint_as_float(w[e] << 16), kind + 1), unary_activation(__uint_as_float(w[e] & 0xffff0000u), kind + 1));
+    out[i] = make_uint4(y[0], y[1], y[2], y[3]);
+}
+
 // out = act(x + bias[column]) for a product whose bias keeps the activation out of its epilogue; the sum is float
 template <typename T>
 __global__ void __launch_bounds__(256) bias_act_kernel(const T* __restrict__ x, const float* __restrict__ bias, T* __restrict__ out,
@@ -290,6 +303,10 @@ extern "C" int cisr_gelu(const void* x, void* out, long long n, int kind, int dt
     if (n <= 0) return 0;
     if (kind < 0 || kind > 2) return (int)hipErrorInvalidValue;
     const unsigned blocks = (unsigned)((n + 255) / 256);
+    if (dtype != DT_F32 && n % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0) {
+        gelu_bf16x8_kernel<<<(unsigned)((n / 8 + 255) / 256), 256, 0, stream>>>((const uint4*)x, (uint4*)out, (size_t)n / 8, kind);
+        return CISR_LAUNCH_CHECK();
+    }
     if (dtype == DT_F32) gelu_kernel<float><<<blocks, 256, 0, stream>>>((const float*)x, (float*)out, (size_t)n, kind);
     else gelu_kernel<bf16_t><<<blocks, 256, 0, stream>>>((const bf16_t*)x, (bf16_t*)out, (size_t)n, kind);
     return CISR_LAUNCH_CHECK();

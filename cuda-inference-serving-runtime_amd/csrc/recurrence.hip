@@ -92,6 +92,84 @@ conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* _
     out[(size_t)t * channels + idx] = y / (1.0f + expf(-y));
 }
 
+// The same for portions, four channels a thread and CONV_ROWS rows of the step a block: an input is read once (the taps - 1
+// before a block's first row again), eight rows' 16-byte loads are on their way together.  The same sums in the same order.
+// Channels, row stride and first column multiples of 4, pointers 16-byte aligned.  The last blocks of y make the gates.
+// 2,048 rows of 8,192 channels, four taps: 90 us with a thread a (row, channel), 45 so (134 MB).
+#define CONV_ROWS 16
+typedef __attribute__((ext_vector_type(4))) float conv_f32x4;
+template <int TAPS>
+__global__ void __launch_bounds__(256)
+conv_silu_rows_kernel(const float* __restrict__ in, int ld, int first, const float* __restrict__ w, const float* __restrict__ bias,
+                      const float* __restrict__ conv_state, long long slot_stride, float* __restrict__ out,
+                      const int* __restrict__ seg_of_row, const int* __restrict__ seg_start, const int* __restrict__ state_slots,
+                      int rows, int channels, int heads, int dt_first, const float* __restrict__ dt_bias,
+                      const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay) {
+    const int t0 = blockIdx.x * CONV_ROWS, t1 = min(t0 + CONV_ROWS, rows);
+    const int channel_blocks = (channels / 4 + 255) / 256;
+    if ((int)blockIdx.y >= channel_blocks) {
+        const int h = ((int)blockIdx.y - channel_blocks) * 256 + threadIdx.x;
+        if (h >= heads) return;
+        for (int t = t0; t < t1; ++t) {
+            if (seg_of_row[t] < 0) continue;
+            const float z = in[(size_t)t * ld + dt_first + h] + dt_bias[h];
+            const float dt = z > 20.f ? z : log1pf(expf(z));
+            step[(size_t)t * heads + h] = dt;
+            decay[(size_t)t * heads + h] = expf(-expf(a_log[h]) * dt);
+        }
+        return;
+    }
+    const int c = ((int)blockIdx.y * 256 + threadIdx.x) * 4;
+    if (c >= channels) return;
+    const float* x0 = in + first + c;
+    float taps[4][TAPS];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) taps[i][j] = w[(size_t)(c + i) * TAPS + j];
+    const conv_f32x4 b = bias ? *(const conv_f32x4*)(bias + c) : (conv_f32x4){0.f, 0.f, 0.f, 0.f};
+    conv_f32x4 before[TAPS - 1];                     // the inputs of the TAPS - 1 rows before, whoever's they are
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) before[j] = *(const conv_f32x4*)(x0 + (size_t)max(t0 - (TAPS - 1) + j, 0) * ld);
+    for (int tb = t0; tb < t1; tb += 8) {
+        conv_f32x4 x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = *(const conv_f32x4*)(x0 + (size_t)min(tb + i, rows - 1) * ld);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int t = tb + i;
+            if (t >= t1) break;                      // (uniform)
+            const int seg = seg_of_row[t];
+            conv_f32x4 use[TAPS];
+#pragma unroll
+            for (int j = 0; j < TAPS - 1; ++j) use[j] = before[j];
+            use[TAPS - 1] = x[i];
+#pragma unroll
+            for (int j = 0; j + 1 < TAPS - 1; ++j) before[j] = before[j + 1];
+            before[TAPS - 2] = x[i];
+            if (seg < 0) continue;
+            const int rel = t - seg_start[seg];
+            if (rel < TAPS - 1) {                    // (uniform: a portion's first rows reach back into the request's state)
+                const float* st = conv_state + (long long)state_slots[seg] * slot_stride + c;
+#pragma unroll
+                for (int j = 0; j < TAPS - 1; ++j)
+                    if (rel - (TAPS - 1) + j < 0) {
+                        const float* from = st + (size_t)(rel + j) * channels;
+                        use[j] = (conv_f32x4){from[0], from[1], from[2], from[3]};
+                    }
+            }
+            conv_f32x4 y = b;
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) y[k] += taps[k][j] * use[j][k];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) y[k] = y[k] / (1.0f + expf(-y[k]));
+            *(conv_f32x4*)(out + (size_t)t * channels + c) = y;
+        }
+    }
+}
+
 // After the convolution has read it: the state becomes the last taps - 1 inputs of (state, portion).
 __global__ void __launch_bounds__(256)
 conv_state_kernel(const float* __restrict__ in, int ld, int first, float* __restrict__ conv_state, long long slot_stride,
@@ -127,8 +205,19 @@ extern "C" int cisr_conv_silu(const float* in, int ld, int first, const float* w
             out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay);
         return CISR_LAUNCH_CHECK();
     }
-    conv_silu_kernel<false><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride,
-        out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay);
+    if (taps >= 2 && taps <= 4 && channels % 4 == 0 && ld % 4 == 0 && first % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+        (!bias || (uintptr_t)bias % 16 == 0)) {
+        const dim3 blocks((rows + CONV_ROWS - 1) / CONV_ROWS, (channels / 4 + 255) / 256 + (heads + 255) / 256);
+#define CONV_ROWS_OF(TAPS) conv_silu_rows_kernel<TAPS><<<blocks, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride, \
+            out, seg_of_row, seg_start, state_slots, rows, channels, heads, dt_first, dt_bias, a_log, step, decay)
+        if (taps == 2) CONV_ROWS_OF(2);
+        else if (taps == 3) CONV_ROWS_OF(3);
+        else CONV_ROWS_OF(4);
+#undef CONV_ROWS_OF
+    } else {
+        conv_silu_kernel<false><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride,
+            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay);
+    }
     int err = CISR_LAUNCH_CHECK();
     if (err || taps == 1) return err;
     conv_state_kernel<<<dim3(segments, (channels + 255) / 256), 256, 0, stream>>>(in, ld, first, conv_state, slot_stride, seg_start,
@@ -165,12 +254,39 @@ __global__ void decay_gate_low_rank_kernel(const float* __restrict__ low, int ld
     a[i] = expf((fminf(u, 0.f) - log1pf(expf(-fabsf(u)))) * inv_tau);
 }
 
+// The same with GATE_ROWS rows a thread, which share the matrix's words: 2,368 rows of 1,024 decays through a rank of 16 20 us a
+// decay a thread, 14 so.  The same sums in the same order.
+#define GATE_ROWS 8
+__global__ void __launch_bounds__(256)
+decay_gate_low_rank_rows_kernel(const float* __restrict__ low, int ld, int rank, const float* __restrict__ up,
+                                const float* __restrict__ bias, float* __restrict__ a, int rows, int cols, float inv_tau) {
+    const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * GATE_ROWS;
+    if (c >= cols) return;
+    float u[GATE_ROWS];
+    const float b = bias ? bias[c] : 0.f;
+#pragma unroll
+    for (int i = 0; i < GATE_ROWS; ++i) u[i] = b;
+#pragma unroll 4
+    for (int r = 0; r < rank; ++r) {
+        const float w = up[(size_t)r * cols + c];
+#pragma unroll
+        for (int i = 0; i < GATE_ROWS; ++i) u[i] += w * low[(size_t)min(t0 + i, rows - 1) * ld + r];     // (uniform over the block)
+    }
+#pragma unroll
+    for (int i = 0; i < GATE_ROWS; ++i)
+        if (t0 + i < rows) a[(size_t)(t0 + i) * cols + c] = expf((fminf(u[i], 0.f) - log1pf(expf(-fabsf(u[i])))) * inv_tau);
+}
+
 extern "C" int cisr_decay_gate_low_rank(const float* low, int ld, int rank, const float* up, const float* bias, float* a,
                                         int rows, int cols, float tau, hipStream_t stream) {
     const size_t n = (size_t)rows * cols;
     if (n == 0) return 0;
     if (!(tau > 0.f) || rank <= 0) return (int)hipErrorInvalidValue;
-    decay_gate_low_rank_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(low, ld, rank, up, bias, a, cols, n, 1.0f / tau);
+    // (from a block for every other compute unit on)
+    if ((long long)((cols + 255) / 256) * ((rows + GATE_ROWS - 1) / GATE_ROWS) >= 128 && rows <= 65535 * GATE_ROWS)
+        decay_gate_low_rank_rows_kernel<<<dim3((cols + 255) / 256, (rows + GATE_ROWS - 1) / GATE_ROWS), 256, 0, stream>>>(low, ld, rank, up, bias, a, rows, cols, 1.0f / tau);
+    else
+        decay_gate_low_rank_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(low, ld, rank, up, bias, a, cols, n, 1.0f / tau);
     return CISR_LAUNCH_CHECK();
 }
 
@@ -222,10 +338,89 @@ group_norm_gate_kernel(const float* __restrict__ y, const float* __restrict__ ga
     }
 }
 
+// The same in 16-byte words with a part's elements in registers: NT neighbouring threads (half a wave, a wave or the block of
+// 256) a part of up to 4 NT E elements.  Parts, row strides and the skip's span multiples of 4, pointers
+// 16-byte aligned.  2,048 rows of 32 parts of 128 31 us with a word a lane, 18.6 so; 2,368 rows of one part of 4,096 44 and 27.5.
+typedef __attribute__((ext_vector_type(4))) float gng_f32x4;
+template <typename T, bool GATE_FIRST, int NT, int E>
+__global__ void __launch_bounds__(256)
+group_norm_gate_words_kernel(const float* __restrict__ y, const float* __restrict__ gate, int ldg, const float* __restrict__ w,
+                             int shared, const float* __restrict__ skip, int skip_span, const float* __restrict__ x, int ldx,
+                             T* __restrict__ out, int groups, int size, float eps, int sigmoid, long long parts) {
+    __shared__ float red[4];
+    const int lane = threadIdx.x % NT;
+    const long long own = (long long)blockIdx.x * (256 / NT) + threadIdx.x / NT, part = own < parts ? own : parts - 1;
+    const long long t = part / groups;
+    const int col0 = (int)(part % groups) * size;
+    gng_f32x4 u[E], z[E], wt[E], s[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int d = min(4 * (lane + NT * e), size - 4);
+        u[e] = *(const gng_f32x4*)(y + part * size + d);
+        z[e] = *(const gng_f32x4*)(gate + t * ldg + col0 + d);
+        wt[e] = *(const gng_f32x4*)(w + (shared ? d : col0 + d));
+        s[e] = (gng_f32x4){0.f, 0.f, 0.f, 0.f};
+        if (skip) {
+            const float f = skip[(col0 + d) / skip_span];
+            s[e] = *(const gng_f32x4*)(x + t * ldx + col0 + d);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s[e][k] *= f;
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool in = 4 * (lane + NT * e) < size;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float g = (sigmoid ? 1.0f : z[e][k]) / (1.0f + expf(-z[e][k]));
+            float v = u[e][k] + s[e][k];
+            if (GATE_FIRST) v *= g;
+            ss += in ? v * v : 0.f;
+            u[e][k] = v;
+            z[e][k] = g;
+        }
+    }
+    float sum = ss;
+    if constexpr (NT == 256) sum = block_sum<256>(ss, red);
+    else
+#pragma unroll
+        for (int off = NT / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, WAVE);
+    if (own >= parts) return;
+    const float scale = 1.0f / sqrtf(sum / (float)size + eps);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int d = 4 * (lane + NT * e);
+        if (d >= size) continue;
+        gng_f32x4 v;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = u[e][k] * scale * wt[e][k] * (GATE_FIRST ? 1.0f : z[e][k]);
+        T* o = out + part * size + d;
+        if constexpr (sizeof(T) == 4) *(gng_f32x4*)o = v;
+        else *(uint2*)o = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    }
+}
+
 template <typename T, bool GATE_FIRST>
 static void launch_group_norm_gate(const float* y, const float* gate, int ldg, const float* w, int shared, const float* skip,
                                    int skip_span, const float* x, int ldx, T* out, int rows, int groups, int size, float eps,
                                    int sigmoid, hipStream_t stream) {
+    const bool words = size % 4 == 0 && size <= 4096 && ldg % 4 == 0 && (!skip || (ldx % 4 == 0 && skip_span % 4 == 0 && (uintptr_t)x % 16 == 0)) &&
+                       (uintptr_t)y % 16 == 0 && (uintptr_t)gate % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % (4 * sizeof(T)) == 0;
+    const long long parts = (long long)rows * groups;
+    // (a step of few rows keeps the blocks of a part each, which spread it over more compute units: from a part for each on)
+    if (words && parts >= 256 && parts < 0x7fffffff) {
+#define GNGW(NT, E) group_norm_gate_words_kernel<T, GATE_FIRST, NT, E><<<(unsigned)((parts + 256 / NT - 1) / (256 / NT)), 256, 0, stream>>>(y, gate, ldg, w, shared, skip, \
+        skip_span, x, ldx, out, groups, size, eps, sigmoid, parts)
+        if (size <= 128) GNGW(32, 1);
+        else if (size <= 256) GNGW(64, 1);
+        else if (size <= 512) GNGW(64, 2);
+        else if (size <= 1024) GNGW(256, 1);
+        else if (size <= 2048) GNGW(256, 2);
+        else GNGW(256, 4);
+#undef GNGW
+        return;
+    }
     const dim3 grid(rows, groups);
     const size_t lds = (size_t)size * sizeof(float);
 #define GNG(NT, KEEP) group_norm_gate_kernel<T, GATE_FIRST, NT, KEEP><<<grid, NT, KEEP ? lds : 0, stream>>>(y, gate, ldg, w, shared, skip, skip_span, x, ldx, out, size, eps, sigmoid)

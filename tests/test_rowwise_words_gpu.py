@@ -1,0 +1,94 @@
+"""The row-wise kernels of the recurrent mixers and the gelu where they run in 16-byte words, at the edges of those forms."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def close(got, want, tol):
+    got, want = got.double().cpu(), want.double().cpu()
+    assert ((got - want).abs().max() / want.abs().max().clamp_min(1e-30)).item() < tol
+
+
+def ints(a):
+    return torch.tensor([int(x) for x in a], dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("channels, taps, heads, bias", [(4, 2, 0, True), (1028, 4, 3, True), (300, 3, 300, False), (8, 4, 1, False)])
+def test_short_convolution_in_words(channels, taps, heads, bias):
+    """Portions shorter than the taps, of one row, of more rows than a block takes, that begin inside a block and at its first
+    row; rows of no segment; inputs and state as columns of wider rows."""
+    from runtime.kernels import ops
+    counts, slots = [5, 1, 43, 0, 16, 2, 33], [2, 0, 5, 1, 6, 3, 4]
+    pad, T = 3, sum(counts) + 3
+    starts = np.concatenate(([0], np.cumsum(counts)))
+    seg = np.concatenate([np.repeat(np.arange(len(counts)), counts), [-1] * pad])
+    wide = torch.randn(T, 4 + channels + heads + (-(channels + heads) % 4), device=DEV)
+    x, dt = wide[:, 4:4 + channels], wide[:, 4 + channels:4 + channels + heads]
+    w, b = torch.randn(channels, taps, device=DEV), torch.randn(channels, device=DEV) if bias else None
+    state = torch.randn(7, (taps - 1) * channels + 5, device=DEV)
+    before, out = state.clone(), torch.full((T, channels), 9.0, device=DEV)
+    gates = None
+    if heads:
+        step, decay = torch.full((T, heads), 9.0, device=DEV), torch.full((T, heads), 9.0, device=DEV)
+        dt_bias, a_log = torch.randn(heads, device=DEV), torch.randn(heads, device=DEV)
+        gates = (dt, dt_bias, a_log, step, decay)
+    ops.conv_silu(x, w, b, state[:, :(taps - 1) * channels], out, ints(seg), ints(starts), ints(slots), gates=gates)
+    for s, slot in enumerate(slots):
+        lo, hi = starts[s], starts[s + 1]
+        old = before[slot, :(taps - 1) * channels].view(taps - 1, channels).double()
+        inputs = torch.cat((old, x[lo:hi].double()))
+        z = sum(inputs[j:j + hi - lo] * w[:, j].double() for j in range(taps)) + (0.0 if b is None else b.double())
+        if hi > lo:
+            close(out[lo:hi], torch.nn.functional.silu(z), 2e-6)
+            close(state[slot, :(taps - 1) * channels].view(taps - 1, channels), inputs[-(taps - 1):], 1e-9)
+        if heads and hi > lo:
+            d = torch.nn.functional.softplus(dt[lo:hi].double() + dt_bias.double())
+            close(step[lo:hi], d, 2e-6)
+            close(decay[lo:hi], torch.exp(-a_log.double().exp() * d), 2e-6)
+    assert (out[-pad:] == 9.0).all() and (state[1] == before[1]).all() and (not heads or bool((step[-pad:] == 9.0).all()))
+
+
+@pytest.mark.parametrize("groups, size", [(300, 4), (33, 128), (9, 132), (40, 256), (3, 260), (2, 1000), (1, 1028), (1, 2048), (1, 4096), (5, 100)])
+@pytest.mark.parametrize("gate_first, sigmoid, skip, shared, dtype", [(True, False, True, False, torch.bfloat16), (False, True, False, True, torch.float32),
+                                                                     (False, False, True, False, torch.bfloat16)])
+def test_group_norm_and_gate_in_words(groups, size, gate_first, sigmoid, skip, shared, dtype):
+    from runtime.kernels import ops
+    rows, width = max(2, -(-259 // groups)), groups * size
+    y, w = torch.randn(rows, width, device=DEV), torch.randn(size if shared else width, device=DEV)
+    gate, x = torch.randn(rows, width + 8, device=DEV)[:, 4:4 + width], torch.randn(rows, width + 4, device=DEV)[:, :width]
+    d = torch.randn(groups, device=DEV)
+    out = torch.empty(rows, width, device=DEV, dtype=dtype)
+    ops.group_norm_gate(y, gate, w, out, groups, 1e-5, gate_first=gate_first, shared_weight=shared, sigmoid=sigmoid, skip=(d, x) if skip else None)
+    u, z = y.double(), gate.double()
+    if skip:
+        u = u + d.double().repeat_interleave(size) * x.double()
+    law = torch.sigmoid(z) * (1.0 if sigmoid else z)
+    if gate_first:
+        u = u * law
+    u = u.view(rows, groups, size)
+    u = (u * torch.rsqrt(u.square().mean(-1, keepdim=True) + 1e-5)).view(rows, width) * (w.double().repeat(groups) if shared else w.double())
+    close(out, u if gate_first else u * law, 3e-6 if dtype == torch.float32 else 5e-3)
+
+
+@pytest.mark.parametrize("rows, cols, rank", [(1025, 256, 16), (513, 520, 3), (130, 2049, 17), (3, 100, 5)])
+def test_low_rank_decays_several_rows_a_thread(rows, cols, rank):
+    from runtime.kernels import ops
+    low, up, bias = torch.randn(rows, rank + 3, device=DEV)[:, 1:1 + rank], torch.randn(rank, cols, device=DEV), torch.randn(cols, device=DEV)
+    out = ops.decay_gate_low_rank(low, up, bias, torch.empty(rows, cols, device=DEV), 16.0)
+    close(out, torch.exp(torch.nn.functional.logsigmoid(low.double() @ up.double() + bias.double()) / 16.0), 2e-6)
+
+
+@pytest.mark.parametrize("n", [8, 2048 * 8 + 8, 12])
+@pytest.mark.parametrize("form", ["gelu", "gelu_tanh"])
+def test_gelu_of_bf16_words(n, form):
+    from runtime.kernels import ops
+    x = (torch.randn(1, n, device=DEV) * 3).bfloat16()
+    out = ops.gelu(x, torch.empty_like(x), form)
+    z = x.double()
+    want = 0.5 * z * (1 + torch.erf(z / math.sqrt(2.0))) if form == "gelu" else 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z ** 3)))
+    close(out, want, 5e-3)
