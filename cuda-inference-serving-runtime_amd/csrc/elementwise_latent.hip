@@ -81,11 +81,110 @@ layernorm_wave_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     }
 }
 
+// A block a row, the row in registers (R words of four floats a thread): x += what the product before left unfinished, if
+// anything (slices > 0: partial sums [slices][rows][dim], added in slice order and then to x; delta: a bf16 product), then the
+// norm as above.  Few rows take it without a product as well: a row is spread over 256 lanes instead of 64.
+// Bound by its loads' one round trip.  Measured on an MI355X in captured decode steps of 8 rows of 2,048: the norm alone 6.3 us a
+// wave a row (two blocks in all) -> 4.5; behind a product cut in slices 4.5 instead of 6.3 and the finishing kernel's 4.6 (the
+// step 7.66 -> 7.15 ms); 2,048 rows behind a bf16 product 10.2 instead of 8.5 (the sum) and 8.4.
+template <typename OUT, int R, bool DELTA>
+__global__ void __launch_bounds__(256)
+layernorm_row_kernel(float* x, const float* __restrict__ parts, int slices, const bf16_t* __restrict__ delta, const float* __restrict__ w,
+                     const float* __restrict__ b, OUT* __restrict__ out, int n_rows, int dim, float eps) {
+    typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+    __shared__ float red[4];
+    const int row = blockIdx.x, tid = threadIdx.x, words = dim / 4;
+    f32x4_t* xr = (f32x4_t*)(x + (size_t)row * dim);
+    const f32x4_t* pr = (const f32x4_t*)parts + (size_t)row * words;
+    const size_t slice = (size_t)n_rows * words;
+    f32x4_t v[R], ww[R], bb[R], sum[R];
+    uint2 d[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int c = min(tid + 256 * i, words - 1);      // past the row: a copy of its last word, not counted or stored
+        v[i] = xr[c];
+        if (DELTA) d[i] = ((const uint2*)(delta + (size_t)row * dim))[c];
+        ww[i] = ((const f32x4_t*)w)[c];
+        bb[i] = b ? ((const f32x4_t*)b)[c] : (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        sum[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    }
+    for (int s0 = 0; s0 < slices; s0 += 4) {
+        f32x4_t p[R][4];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) p[i][j] = pr[(size_t)min(s0 + j, slices - 1) * slice + min(tid + 256 * i, words - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (s0 + j >= slices) break;
+#pragma unroll
+            for (int i = 0; i < R; ++i) sum[i] += p[i][j];
+        }
+    }
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        if (slices > 0) v[i] = sum[i] + v[i];
+        if (DELTA) v[i] += (f32x4_t){__uint_as_float(d[i].x << 16), __uint_as_float(d[i].x & 0xffff0000u), __uint_as_float(d[i].y << 16),
+                                     __uint_as_float(d[i].y & 0xffff0000u)};
+        if (tid + 256 * i >= words) continue;
+        if (slices > 0 || DELTA) xr[tid + 256 * i] = v[i];
+        total += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+    }
+    const float mean = block_sum<256>(total, red) / dim;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        v[i] -= mean;
+        if (tid + 256 * i >= words) continue;
+        q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    }
+    const float inv = rsqrtf(block_sum<256>(q, red) / dim + eps);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int at = tid + 256 * i;
+        if (at >= words) continue;
+        const f32x4_t y = v[i] * inv * ww[i] + bb[i];
+        if (sizeof(OUT) == 4) ((f32x4_t*)((float*)out + (size_t)row * dim))[at] = y;
+        else ((uint2*)((bf16_t*)out + (size_t)row * dim))[at] = make_uint2(pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w));
+    }
+}
+
+template <typename OUT>
+static int launch_layernorm_rows(float* x, const float* parts, int slices, const bf16_t* delta, const float* w, const float* b, OUT* out,
+                                 int n_rows, int dim, float eps, hipStream_t stream) {
+    const int per = (dim / 4 + 255) / 256;
+#define LN_ROW(R) do { if (delta) layernorm_row_kernel<OUT, R, true><<<n_rows, 256, 0, stream>>>(x, parts, slices, delta, w, b, out, n_rows, dim, eps); \
+                       else layernorm_row_kernel<OUT, R, false><<<n_rows, 256, 0, stream>>>(x, parts, slices, nullptr, w, b, out, n_rows, dim, eps); } while (0)
+    if (per <= 1) LN_ROW(1);
+    else if (per <= 2) LN_ROW(2);
+    else if (per <= 4) LN_ROW(4);
+    else LN_ROW(8);
+#undef LN_ROW
+    return CISR_LAUNCH_CHECK();
+}
+
+// x[n_rows, dim] += parts[slices][n_rows][dim] (slices > 0) or delta (bf16, or null), then out = layernorm(x).  dim % 4 == 0,
+// dim <= 8192, 16-byte aligned operands.
+extern "C" int cisr_layernorm_partials(float* x, const float* parts, int slices, const void* delta, const float* w, const float* b,
+                                       void* out, int n_rows, int dim, float eps, int out_dtype, hipStream_t stream) {
+    if (n_rows <= 0) return 0;
+    if (slices < 0 || (slices > 0) == (delta != nullptr) || (slices > 0 && !parts) || dim <= 0 || dim % 4 || dim > 8192 || (uintptr_t)x % 16 ||
+        (uintptr_t)parts % 16 || (uintptr_t)delta % 8 || (uintptr_t)w % 16 || (uintptr_t)b % 16 || (uintptr_t)out % 16)
+        return (int)hipErrorInvalidValue;
+    if (out_dtype == DT_F32) return launch_layernorm_rows<float>(x, parts, slices, (const bf16_t*)delta, w, b, (float*)out, n_rows, dim, eps, stream);
+    return launch_layernorm_rows<bf16_t>(x, parts, slices, (const bf16_t*)delta, w, b, (bf16_t*)out, n_rows, dim, eps, stream);
+}
+
 template <typename OUT>
 static int launch_layernorm(const float* x, const float* w, const float* b, OUT* out, const int* rows, int n_out, int dim,
                             float eps, hipStream_t stream) {
     const bool aligned = dim % 4 == 0 && ((uintptr_t)x) % 16 == 0 && ((uintptr_t)w) % 16 == 0 && (!b || ((uintptr_t)b) % 16 == 0) &&
                          ((uintptr_t)out) % 16 == 0;
+    // Up to 64 rows in order: a block a row (6.3 -> 4.5 us at 8 rows).  More rows fill the chip a wave a row, without the two
+    // barriers of a block's sums; under 1,024 columns a wave holds a row in four loads a lane.
+    if (aligned && !rows && n_out <= 64 && dim >= 1024 && dim <= 8192)
+        return launch_layernorm_rows(const_cast<float*>(x), nullptr, 0, nullptr, w, b, out, n_out, dim, eps, stream);    // (x is not written)
     const int per_lane = (dim / 4 + WAVE - 1) / WAVE;
     const unsigned blocks = (unsigned)((n_out + 3) / 4);
 #define LN_WAVE(CH) layernorm_wave_kernel<OUT, CH><<<blocks, 256, 0, stream>>>(x, w, b, out, rows, n_out, dim, eps)

@@ -76,6 +76,7 @@ def _declare(h):
         "cisr_glu_clamped": [p, p, i, i, f, f, f, i, p],
         "cisr_qk_norm_scatter": [p, i, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f, i, i, i, i, p, f, i, p],
         "cisr_head_gate": [p, p, i, i, p, i, i, i, i, i, i, p],
+        "cisr_layernorm_partials": [p, p, i, p, p, p, p, i, i, f, i, p],
         "cisr_layernorm": [p, p, p, p, p, i, i, f, i, p],
         "cisr_rms_slice": [p, i, i, p, p, i, i, f, i, p],
         "cisr_latent_keys": [p, i, i, p, p, i, p, p, p, p, p, p, p, i, i, i, i, i, i, i, i, i, i, f, i, p],
@@ -1252,6 +1253,23 @@ def layernorm(x, weight, out, eps, rows=None, bias=None):
     _check(lib().cisr_layernorm(_dev(x, "x", torch.float32), _dev(weight, "weight", torch.float32, (dim,)), bp,
                                 _dev(out, "out", None, (n_out, dim)), rp, n_out, dim, float(eps), _storage(out, "out"),
                                 _stream()), "layernorm")
+    return out
+
+
+def layernorm_partials(x, partials, weight, out, eps, bias=None):
+    """x += what gemm_unfinished left (in place), out = layernorm(x) * weight (+ bias): one kernel."""
+    parts, slices = partials
+    rows, dim = x.shape
+    if not partials_ok(x) or out.data_ptr() % 16:
+        raise KernelError("layernorm_partials: contiguous float rows of a multiple of 4 (at most 8192)")
+    if slices and parts.numel() < slices * rows * dim:
+        raise KernelError("layernorm_partials: too few partial sums")
+    pp = _dev(parts, "partials", torch.float32) if slices else None
+    dp = None if slices else _dev(parts, "product", torch.bfloat16, (rows, dim))
+    bp = None if bias is None else _dev(bias, "bias", torch.float32, (dim,))
+    _check(lib().cisr_layernorm_partials(x.data_ptr(), pp, int(slices), dp, _dev(weight, "weight", torch.float32, (dim,)), bp,
+                                         _dev(out, "out", None, (rows, dim)), rows, dim, float(eps), _storage(out, "out"), _stream()),
+           "layernorm_partials")
     return out
 
 

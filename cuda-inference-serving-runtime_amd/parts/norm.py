@@ -44,7 +44,8 @@ class RMSNorm(Part):
 class LayerNorm(Part):
     """The centred norm with a weight and, with `bias`, a bias.  `gain`: a constant that multiplies the result (it rides
     in the weight and the bias): a model whose head scales its logits gives it to its last norm, since the head is linear.
-    No product takes this norm over (it states no `fusable_as`) and it adds no partial sums."""
+    No product takes this norm over (it states no `fusable_as`)."""
+    adds_partials = True    # forward adds the partial sums of a product left unfinished before it (ctx.add_product)
 
     def __init__(self, name, dim, eps, tensor=None, bias=False, bias_tensor=None, gain=1.0):
         self.name, self.dim, self.eps, self.gain = name, dim, float(eps), float(gain)
@@ -65,8 +66,13 @@ class LayerNorm(Part):
 
     def forward(self, x, ctx, rows=None, tag="norm"):
         n_out = x.shape[0] if rows is None else rows.shape[0]
+        out = ctx.buffer(tag, (n_out, self.dim), ctx.dtype)
+        if rows is None and ops.partials_ok(x):
+            partials = ctx.take_unfinished(x)
+            if partials is not None:
+                return ops.layernorm_partials(x, partials, self.weight, out, self.eps, bias=self.bias)
         ctx.settle(x)
-        return ops.layernorm(x, self.weight, ctx.buffer(tag, (n_out, self.dim), ctx.dtype), self.eps, rows, bias=self.bias)
+        return ops.layernorm(x, self.weight, out, self.eps, rows, bias=self.bias)
 
 
 class StreamsNorm(RMSNorm):

@@ -92,3 +92,19 @@ def test_gelu_of_bf16_words(n, form):
     z = x.double()
     want = 0.5 * z * (1 + torch.erf(z / math.sqrt(2.0))) if form == "gelu" else 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z ** 3)))
     close(out, want, 5e-3)
+
+
+@pytest.mark.parametrize("rows, dim, slices", [(1, 4, 1), (8, 2048, 3), (64, 1024, 5), (3, 8192, 2), (5, 1028, 9), (70, 2052, 0), (2, 4, 0)])
+@pytest.mark.parametrize("bias, dtype", [(True, torch.float32), (False, torch.bfloat16)])
+def test_layernorm_behind_a_product_left_unfinished(rows, dim, slices, bias, dtype):
+    """Partial sums (more than four, fewer, one) and a bf16 product, added before the norm; without one, the same rows."""
+    from runtime.kernels import ops
+    x, w, b = torch.randn(rows, dim, device=DEV) + 3, torch.randn(dim, device=DEV), torch.randn(dim, device=DEV) if bias else None
+    parts = torch.randn(slices, rows, dim, device=DEV) if slices else torch.randn(rows, dim, device=DEV).bfloat16()
+    v = x.double() + (parts.double().sum(0) if slices else parts.double())
+    out = ops.layernorm_partials(x, (parts.view(-1) if slices else parts, slices), w, torch.empty(rows, dim, device=DEV, dtype=dtype), 1e-5, bias=b)
+    close(x, v, 5e-7)
+    want = torch.nn.functional.layer_norm(v, (dim,), w.double(), None if b is None else b.double(), 1e-5)
+    tol = 5e-6 if dtype == torch.float32 else 5e-3       # (four values of mean 3: their deviations keep 1e-6 of themselves)
+    close(out, want, tol)
+    close(ops.layernorm(x, w, torch.empty_like(out), 1e-5, bias=b), want, tol)
