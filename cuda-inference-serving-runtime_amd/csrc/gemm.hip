@@ -46,13 +46,15 @@ __host__ __device__ inline int patch_side(int tiles) {
 }
 
 // Block tile (16 WM TM) x (32 TN), BK deep; WM x 2 waves (WM = 2 or 4), each wave TM x TN tiles of 16 x 16.
-// The larger the block tile, the fewer bytes come from L2 per product: 128 x 128 is bound by the L2 at about
-// a third of the matrix cores' peak, 256 x 128 moves a quarter less.
-// Operands go global memory -> registers -> LDS -> matrix-core operands.
-// The pipeline hides the global-memory latency inside one block, because small problems leave a
-// compute unit with a single block: PF tiles of global loads are in flight in a ring of registers,
-// and two LDS buffers let the next tile be written while the current one is multiplied, with one
-// barrier per tile.
+// Operands go global memory -> registers -> LDS -> matrix-core operands: PF tiles of global loads are in flight in a ring of
+// registers, and two LDS buffers let the next tile be written while the current one is multiplied, with one barrier per tile.
+// The products that come here leave a compute unit one or two blocks, so the time is the chain of a block's turns (copy, barrier,
+// LDS reads, products) and not the matrix cores.  What shortens it: eight waves a block, so that a SIMD has a second wave to run
+// in the waits of the first; 128 of the inner size a turn in the small tiles, half as many barriers; exact waits (below).
+// Measured on an MI355X, rows x columns x inner size, four waves and 64 a turn before: 1,741 x 576 x 1,536 16.3 -> 8.8 us, 1,741 x
+// 960 x 576 8.8 -> 7.4, 100 x 2,048 x 2,048 12.6 -> 8.0, 300 x 2,048 x 2,048 16.1 -> 11.0, 4,000 x 4,096 x 2,048 144 -> 94 (0.71
+// PFLOP/s), 1,741 x 1,536 x 576 with SwiGLU 17.8 -> 16.1, 100 x 4,096 x 2,048 with it 17.3 -> 10.8.  Reading a turn's operands
+// ahead of the next tile's copies (two tiles deep in LDS) was 5-25 % slower: the copies' waits then stand before the products.
 // SWIGLU: W holds two blocks of N rows, `dual_off` rows apart (gate, then up).  A wave's first TN/2
 // column tiles take gate rows and its last TN/2 the up rows of the same output columns, so a lane ends
 // with gate and up of one output element in its registers and writes silu(gate) * up (both rounded to
@@ -62,7 +64,7 @@ __host__ __device__ inline int patch_side(int tiles) {
 // activation is applied before the store.  Zeros: one product, no gate, no activation.
 struct HeadBatch { long long a, w, c; const float* gate; int ldg; int act; };
 
-template <int TM, int TN, int BK, typename TC, bool VEC, bool SWIGLU = false, int WM = 2>
+template <int TM, int TN, int BK, typename TC, bool VEC, bool SWIGLU = false, int WM = 2, int PF = 3>
 __global__ void __launch_bounds__(WM * 128)
 gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
                  TC* C, int ldc, const float* R, int ldr, int M, int N, int K, int dual_off = 0, GateLaw law = {},
@@ -85,7 +87,6 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict
     static_assert((BM * CPR) % NT == 0 && (BN * CPR) % NT == 0, "a tile is a whole number of 16-byte chunks per thread");
     constexpr int A_PER_THREAD = BM * CPR / NT;
     constexpr int W_PER_THREAD = BN * CPR / NT;
-    constexpr int PF = 3;                                  // tiles of global loads in flight
     __shared__ __attribute__((aligned(16))) bf16_t As[2][BM * BK];
     __shared__ __attribute__((aligned(16))) bf16_t Ws[2][BN * BK];
 
@@ -97,15 +98,15 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict
     // 8 x 8 (sides as even as the tile counts allow, so that few slots fall outside the matrix): the sixty-odd blocks that run on an XCD at one time then share 8 row bands of A and 8 of W
     // (16 bands from memory for 64 tiles) instead of one band of A and 64 of W.
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
-    const int gm = patch_side(tiles_m), gn = patch_side(tiles_n);
-    const int patches_n = (tiles_n + gn - 1) / gn, patches = ((tiles_m + gm - 1) / gm) * patches_n;
-    const int slots = patches * gm * gn;                   // tile slots (those outside the matrix do nothing)
-    const int per_xcd = (slots + 7) / 8;
+    const int tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
     const int slot = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (slot >= slots) return;                             // the grid is rounded up to a multiple of 8
-    const int patch = slot / (gm * gn), in_patch = slot % (gm * gn);
-    const int tile_m = (patch / patches_n) * gm + in_patch % gm, tile_n = (patch % patches_n) * gn + in_patch / gm;
-    if (tile_m >= tiles_m || tile_n >= tiles_n) return;
+    if (slot >= tiles) return;                             // the grid is rounded up to a multiple of 8
+    // (the last patches of a row or column are cut to the matrix: a slot outside it would leave its compute unit idle
+    // while another takes two tiles)
+    const int gm = patch_side(tiles_m), gn = patch_side(tiles_n);
+    const int band = slot / (gm * tiles_n), rows = min(gm, tiles_m - band * gm);
+    const int in_band = slot - band * gm * tiles_n, patch = in_band / (rows * gn), in_patch = in_band - patch * rows * gn;
+    const int tile_m = band * gm + in_patch % rows, tile_n = patch * gn + in_patch / rows;
     const int m0 = tile_m * BM, n0 = tile_n * BN_OUT;
 
     f32x4 acc[TM][TN];
@@ -135,51 +136,53 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict
         }
     };
 #pragma unroll
-    for (int s = 0; s < PF; ++s) fetch(s * BK, ra[s], rw[s]);   // beyond K: zeros, never used
+    for (int s = 0; s < PF; ++s) fetch(s * BK, ra[s], rw[s]);   // beyond K: the last chunk again (VEC) or zeros, never used
 
-    int it = 0;
-    for (int k0 = 0; k0 < K; k0 += PF * BK) {
+    auto turn = [&](int t, u32x4 (&ta)[A_PER_THREAD], u32x4 (&tw)[W_PER_THREAD], bool ask) {
+        const int kk0 = t * BK, buf = t & 1;
 #pragma unroll
-        for (int s = 0; s < PF; ++s) {
-            const int kk0 = k0 + s * BK;
-            if (kk0 < K) {
-                const int buf = it & 1;
-                ++it;
-#pragma unroll
-                for (int i = 0; i < A_PER_THREAD; ++i) {
-                    const int c = tid + i * NT;
-                    const uint32_t keep = (VEC && kk0 + (c % CPR) * 8 >= K) ? 0u : 0xffffffffu;
-                    u32x4 v = ra[s][i];
-                    v.x &= keep; v.y &= keep; v.z &= keep; v.w &= keep;
-                    *(u32x4*)(&As[buf][lds_at(c / CPR, c % CPR)]) = v;
-                }
-#pragma unroll
-                for (int i = 0; i < W_PER_THREAD; ++i) {
-                    const int c = tid + i * NT;
-                    *(u32x4*)(&Ws[buf][lds_at(c / CPR, c % CPR)]) = rw[s][i];   // A is zero there: enough
-                }
-                // one barrier a tile: whoever writes this buffer again (two tiles on) has passed
-                // the next tile's barrier, which every wave reaches only after reading this one
-                __syncthreads();
-                if (kk0 + PF * BK < K) fetch(kk0 + PF * BK, ra[s], rw[s]);
-#pragma unroll
-                for (int kk = 0; kk < BK; kk += 32) {
-                    bf16x8 fa[TM], fw[TN];
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-                        fa[i] = *(const bf16x8*)(&As[buf][lds_at(wm * TM * 16 + i * 16 + r, kk / 8 + g)]);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        fw[j] = *(const bf16x8*)(&Ws[buf][lds_at(wn * TN * 16 + j * 16 + r, kk / 8 + g)]);
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fw[j], acc[i][j], 0, 0, 0);
-                }
-            }
+        for (int i = 0; i < A_PER_THREAD; ++i) {
+            const int c = tid + i * NT;
+            const uint32_t keep = (VEC && kk0 + (c % CPR) * 8 >= K) ? 0u : 0xffffffffu;
+            u32x4 v = ta[i];
+            v.x &= keep; v.y &= keep; v.z &= keep; v.w &= keep;
+            *(u32x4*)(&As[buf][lds_at(c / CPR, c % CPR)]) = v;
         }
-    }
+#pragma unroll
+        for (int i = 0; i < W_PER_THREAD; ++i) {
+            const int c = tid + i * NT;
+            *(u32x4*)(&Ws[buf][lds_at(c / CPR, c % CPR)]) = tw[i];   // A is zero there: enough
+        }
+        // one barrier a tile: whoever writes this buffer again (two tiles on) has passed
+        // the next tile's barrier, which every wave reaches only after reading this one
+        __syncthreads();
+        if (ask) fetch(kk0 + PF * BK, ta, tw);
+#pragma unroll
+        for (int kk = 0; kk < BK; kk += 32) {
+            bf16x8 fa[TM], fw[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                fa[i] = *(const bf16x8*)(&As[buf][lds_at(wm * TM * 16 + i * 16 + r, kk / 8 + g)]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                fw[j] = *(const bf16x8*)(&Ws[buf][lds_at(wn * TN * 16 + j * 16 + r, kk / 8 + g)]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fw[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // Every turn of the loop asks for PF tiles and uses PF, with no branch between: only then are the waits counted exactly
+    // (a load asked for under a condition makes the next wait one for all that is in flight).  The last turn asks for nothing.
+    const int k_tiles = (K + BK - 1) / BK;
+    int t = 0;
+    for (; t + PF < k_tiles; t += PF)
+#pragma unroll
+        for (int s = 0; s < PF; ++s) turn(t + s, ra[s], rw[s], true);
+#pragma unroll
+    for (int s = 0; s < PF; ++s)
+        if (t + s < k_tiles) turn(t + s, ra[s], rw[s], false);
     if (SWIGLU) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -240,46 +243,40 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict
     }
 }
 
-// tile slots of the kernel's patch numbering (whole patches)
-static long long tile_slots(long long tiles_m, long long tiles_n) {
-    const long long gm = patch_side((int)tiles_m), gn = patch_side((int)tiles_n);
-    return ((tiles_m + gm - 1) / gm) * ((tiles_n + gn - 1) / gn) * gm * gn;
-}
-
-template <int TM, int TN, int BK, int WM = 2>
+template <int TM, int TN, int BK, int WM = 2, int PF = 3>
 static int launch_bf16(const bf16_t* A, int lda, const bf16_t* W, int ldw, void* C, int ldc, const float* R,
                        int ldr, int M, int N, int K, int out_dtype, hipStream_t stream, HeadBatch heads = {}, int n_heads = 1) {
     constexpr int BM = WM * TM * 16, BN = 2 * TN * 16, NT = WM * 128;
-    const long long slots = tile_slots((M + BM - 1) / BM, (N + BN - 1) / BN);
-    if (slots > (1ll << 30) || n_heads < 1 || n_heads > 65535) return (int)hipErrorInvalidValue;
-    dim3 grid((unsigned)((slots + 7) / 8 * 8), n_heads);
+    const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    if (tiles > (1ll << 30) || n_heads < 1 || n_heads > 65535) return (int)hipErrorInvalidValue;
+    dim3 grid((unsigned)((tiles + 7) / 8 * 8), n_heads);
     const bool vec = lda % 8 == 0 && ldw % 8 == 0 && K % 8 == 0 && ((uintptr_t)A) % 16 == 0 && ((uintptr_t)W) % 16 == 0 &&
                      heads.a % 8 == 0 && heads.w % 8 == 0;
     const GateLaw law{};
     if (out_dtype == DT_F32) {
-        if (vec) gemm_bf16_kernel<TM, TN, BK, float, true, false, WM><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (float*)C, ldc, R, ldr, M, N, K, 0, law, heads);
-        else gemm_bf16_kernel<TM, TN, BK, float, false, false, WM><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (float*)C, ldc, R, ldr, M, N, K, 0, law, heads);
+        if (vec) gemm_bf16_kernel<TM, TN, BK, float, true, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (float*)C, ldc, R, ldr, M, N, K, 0, law, heads);
+        else gemm_bf16_kernel<TM, TN, BK, float, false, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (float*)C, ldc, R, ldr, M, N, K, 0, law, heads);
     } else {
-        if (vec) gemm_bf16_kernel<TM, TN, BK, bf16_t, true, false, WM><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (bf16_t*)C, ldc, R, ldr, M, N, K, 0, law, heads);
-        else gemm_bf16_kernel<TM, TN, BK, bf16_t, false, false, WM><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (bf16_t*)C, ldc, R, ldr, M, N, K, 0, law, heads);
+        if (vec) gemm_bf16_kernel<TM, TN, BK, bf16_t, true, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (bf16_t*)C, ldc, R, ldr, M, N, K, 0, law, heads);
+        else gemm_bf16_kernel<TM, TN, BK, bf16_t, false, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (bf16_t*)C, ldc, R, ldr, M, N, K, 0, law, heads);
     }
     return CISR_LAUNCH_CHECK();
 }
 
 // C[M, N] = silu(A . Wg^T) * (A . Wu^T), W = [Wg; Wu] with `dual_off` rows between the blocks; bf16 in and out,
 // 16-byte aligned rows with K % 8 == 0.
-template <int TM, int TN, int BK, int WM = 2>
+template <int TM, int TN, int BK, int WM = 2, int PF = 3>
 static int launch_bf16_swiglu(const bf16_t* A, int lda, const bf16_t* W, int ldw, bf16_t* C, int ldc, int M, int N, int K,
                               int dual_off, GateLaw law, hipStream_t stream) {
     constexpr int BM = WM * TM * 16, BN_OUT = TN * 16;
-    const long long slots = tile_slots((M + BM - 1) / BM, (N + BN_OUT - 1) / BN_OUT);
-    if (slots > (1ll << 30)) return (int)hipErrorInvalidValue;
-    dim3 grid((unsigned)((slots + 7) / 8 * 8));
-    gemm_bf16_kernel<TM, TN, BK, bf16_t, true, true, WM><<<grid, WM * 128, 0, stream>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, law);
+    const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN_OUT - 1) / BN_OUT);
+    if (tiles > (1ll << 30)) return (int)hipErrorInvalidValue;
+    dim3 grid((unsigned)((tiles + 7) / 8 * 8));
+    gemm_bf16_kernel<TM, TN, BK, bf16_t, true, true, WM, PF><<<grid, WM * 128, 0, stream>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, law);
     return CISR_LAUNCH_CHECK();
 }
 
-// `tile`: 0 picks by the rule below; TM * 100 + TN * 10 + WM asks for that block tile (a tile that is not built: an error).
+// `tile`: 0 picks by the rule below; otherwise a block tile by its code (a tile that is not built: an error).
 static int swiglu_tile_entry(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N, int K,
                              int dual_off, int tile, GateLaw law, hipStream_t stream);
 
@@ -302,15 +299,20 @@ static int swiglu_tile_entry(const void* A, int lda, const void* W, int ldw, voi
     const bf16_t* a = (const bf16_t*)A; const bf16_t* w = (const bf16_t*)W;
     auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((2 * N + bn - 1) / bn); };
     if (tile == 0) {
-        if (blocks(128, 128) >= 512) tile = 442;
-        else if (blocks(128, 64) >= 512) tile = 422;
-        else if (blocks(64, 64) < 256) tile = 122;
-        else tile = 222;
+        // As below, over the columns of both halves: 300 rows, 1,536 outputs, K 576: 32 x 64 (480 blocks) 6.8 us, 64 x 64 (240) 6.1,
+        // 128 x 64 7.8.  Between one round and two of 128 x 128 the last round is mostly idle, and 128 x 64 is faster (1,741 rows
+        // there, 336 blocks: 15.7 against 16.6; 600 rows, 4,096 outputs, K 2,048: 39.7 against 41.6); from two on it is not (4,000
+        // rows: 27.8 against 24.9).
+        if (blocks(32, 64) <= 256) tile = 122;
+        else if (blocks(64, 64) <= 256) tile = 222;
+        else if (blocks(128, 64) <= 256 || (blocks(128, 128) > 256 && blocks(128, 128) < 512)) tile = 422;
+        else tile = 442;
     }
-#define SWIGLU_TILE(TM, TN, WM) \
-    case TM * 100 + TN * 10 + WM: return launch_bf16_swiglu<TM, TN, 64, WM>(a, lda, w, ldw, (bf16_t*)C, ldc, M, N, K, dual_off, law, stream);
+#define SWIGLU_TILE(CODE, TM, TN, BK, WM, PF) \
+    case CODE: return launch_bf16_swiglu<TM, TN, BK, WM, PF>(a, lda, w, ldw, (bf16_t*)C, ldc, M, N, K, dual_off, law, stream);
+    // (128 x 128: 32 of the inner size a turn keeps two blocks on a unit; 2,000 rows, 4,096 outputs, K 2,048: 64 deep 94 us, 32 deep 87)
     switch (tile) {
-        SWIGLU_TILE(1, 2, 2) SWIGLU_TILE(2, 2, 2) SWIGLU_TILE(4, 2, 2) SWIGLU_TILE(4, 4, 2)
+        SWIGLU_TILE(122, 1, 2, 64, 2, 3) SWIGLU_TILE(222, 1, 2, 128, 4, 2) SWIGLU_TILE(422, 2, 2, 64, 4, 2) SWIGLU_TILE(442, 2, 4, 32, 4, 4)
     }
 #undef SWIGLU_TILE
     return (int)hipErrorInvalidValue;
@@ -321,31 +323,42 @@ extern "C" int cisr_gemm_bf16_swiglu(const void* A, int lda, const void* W, int 
     return cisr_gemm_bf16_swiglu_tile(A, lda, W, ldw, C, ldc, M, N, K, dual_off, 0, stream);
 }
 
-// Tile choice: the largest tile that still gives the 256 compute units a few blocks each; when even 64 x 64 leaves
-// most of them idle (a portion of a few hundred rows against small weights), 32 x 64 and 32 x 32 (measured on an
-// MI355X at 128 and 512 rows: 10-30 % faster there, slower from about one block a compute unit on).
-// `tile`: 0 picks by this rule; TM * 100 + TN * 10 + WM asks for that block tile (a tile that is not built: an error).
+// The codes name a block tile: rows / 32, columns / 32, and a 2 (112: 32 x 32, 422: 128 x 64).
+// Tile choice: the smallest that needs no more blocks than there are compute units: a block alone on its unit takes the longer the
+// larger its tile, and a second round costs more than a larger tile does.  1,741 rows, us: 576 columns (K 1,536) 32 x 32 12.4, 64 x
+// 32 10.4, 64 x 64 (252 blocks) 8.8, 128 x 64 12.8; 960 columns (K 576) 64 x 64 (420 blocks) 9.8, 128 x 64 (210) 7.4, 128 x 128 10.3.
+// 300 rows x 960: 32 x 32 (300 blocks) 5.1, 64 x 32 (150) 4.6, 64 x 64 5.4.  Where even 128 x 64 needs more, 128 x 128 (4,000 x
+// 2,048, K 512: 128 x 64 in two rounds 17.7, 128 x 128 in one 18.8; K 2,048, 512 blocks against 1,024: 48.6 against 52.8).  Up to 32
+// rows a tile has 32 of them (32 x 12,000, K 1,024: 32 x 64 6.6, 64 x 64 6.8).
+static int pick_tile(int M, int N, int heads) {
+    auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * heads; };
+    if (blocks(32, 32) <= 256) return 112;
+    if (M <= 32) return 122;
+    if (blocks(64, 32) <= 256) return 212;
+    if (blocks(64, 64) <= 256) return 222;
+    if (blocks(128, 64) <= 256) return 422;
+    return 442;
+}
+
+static int launch_tile(int tile, const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R, int ldr, int M, int N,
+                       int K, int out_dtype, hipStream_t stream, HeadBatch batch = {}, int heads = 1) {
+    const bf16_t* a = (const bf16_t*)A; const bf16_t* w = (const bf16_t*)W;
+#define GEMM_TILE(CODE, TM, TN, BK, WM, PF) \
+    case CODE: return launch_bf16<TM, TN, BK, WM, PF>(a, lda, w, ldw, C, ldc, R, ldr, M, N, K, out_dtype, stream, batch, heads);
+    switch (tile) {
+        GEMM_TILE(112, 1, 1, 128, 2, 3) GEMM_TILE(122, 1, 2, 64, 2, 3) GEMM_TILE(212, 1, 1, 128, 4, 2) GEMM_TILE(222, 1, 2, 128, 4, 2)
+        GEMM_TILE(422, 2, 2, 64, 4, 2) GEMM_TILE(442, 2, 4, 64, 4, 2)
+    }
+#undef GEMM_TILE
+    return (int)hipErrorInvalidValue;
+}
+
+// `tile`: 0 picks by the rule above; otherwise a block tile by its code (a tile that is not built: an error).
 extern "C" int cisr_gemm_bf16_tile(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R,
                                    int ldr, int M, int N, int K, int out_dtype, int tile, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || (R && out_dtype != DT_F32)) return (int)hipErrorInvalidValue;
-    const bf16_t* a = (const bf16_t*)A; const bf16_t* w = (const bf16_t*)W;
-    auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    if (tile == 0) {
-        if (M <= 32) tile = 122;
-        else if (blocks(128, 128) >= 512) tile = 442;
-        else if (blocks(128, 64) >= 512) tile = 422;
-        else if (blocks(32, 64) <= 64) tile = 112;
-        else if (blocks(64, 64) < 256) tile = 122;
-        else tile = 222;
-    }
-#define GEMM_TILE(TM, TN, WM) \
-    case TM * 100 + TN * 10 + WM: return launch_bf16<TM, TN, 64, WM>(a, lda, w, ldw, C, ldc, R, ldr, M, N, K, out_dtype, stream);
-    switch (tile) {
-        GEMM_TILE(1, 1, 2) GEMM_TILE(1, 2, 2) GEMM_TILE(2, 2, 2) GEMM_TILE(4, 2, 2) GEMM_TILE(4, 4, 2)
-    }
-#undef GEMM_TILE
-    return (int)hipErrorInvalidValue;
+    return launch_tile(tile ? tile : pick_tile(M, N, 1), A, lda, W, ldw, C, ldc, R, ldr, M, N, K, out_dtype, stream);
 }
 
 // A product a head in one launch: C[m, h * c_head + n] = sum_k A[m, h * a_head + k] W[h][n][k] (W [heads, N, K] contiguous),
@@ -354,22 +367,8 @@ extern "C" int cisr_gemm_bf16_heads(const void* A, int lda, int a_head, const vo
                                     const float* gate, int ldg, int M, int N, int K, int heads, int out_dtype, hipStream_t stream) {
     if (M <= 0 || N <= 0 || heads <= 0) return 0;
     if (K <= 0) return (int)hipErrorInvalidValue;
-    const bf16_t* a = (const bf16_t*)A; const bf16_t* w = (const bf16_t*)W;
     const HeadBatch batch{a_head, (long long)N * K, c_head, gate, ldg, ACT_NONE};
-    auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * heads; };
-    int tile;
-    if (M <= 32) tile = 122;
-    else if (blocks(128, 128) >= 512) tile = 442;
-    else if (blocks(128, 64) >= 512) tile = 422;
-    else if (blocks(64, 64) < 256) tile = 122;
-    else tile = 222;
-#define HEADS_TILE(TM, TN, WM) \
-    case TM * 100 + TN * 10 + WM: return launch_bf16<TM, TN, 64, WM>(a, lda, w, K, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch, heads);
-    switch (tile) {
-        HEADS_TILE(1, 2, 2) HEADS_TILE(2, 2, 2) HEADS_TILE(4, 2, 2) HEADS_TILE(4, 4, 2)
-    }
-#undef HEADS_TILE
-    return (int)hipErrorInvalidValue;
+    return launch_tile(pick_tile(M, N, heads), A, lda, W, K, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch, heads);
 }
 
 // C = act(A . W^T) with an ungated activation (ACT_GELU, ACT_GELU_TANH, ACT_RELU2) as the epilogue; the tile is picked as for the
@@ -378,22 +377,8 @@ extern "C" int cisr_gemm_bf16_act(const void* A, int lda, const void* W, int ldw
                                   int out_dtype, int act, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || act < ACT_GELU || act > ACT_RELU2) return (int)hipErrorInvalidValue;
-    const bf16_t* a = (const bf16_t*)A; const bf16_t* w = (const bf16_t*)W;
     const HeadBatch batch{0, 0, 0, nullptr, 0, act};
-    auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    int tile;
-    if (M <= 32) tile = 122;
-    else if (blocks(128, 128) >= 512) tile = 442;
-    else if (blocks(128, 64) >= 512) tile = 422;
-    else if (blocks(64, 64) < 256) tile = 122;
-    else tile = 222;
-#define ACT_TILE(TM, TN, WM) \
-    case TM * 100 + TN * 10 + WM: return launch_bf16<TM, TN, 64, WM>(a, lda, w, ldw, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch, 1);
-    switch (tile) {
-        ACT_TILE(1, 2, 2) ACT_TILE(2, 2, 2) ACT_TILE(4, 2, 2) ACT_TILE(4, 4, 2)
-    }
-#undef ACT_TILE
-    return (int)hipErrorInvalidValue;
+    return launch_tile(pick_tile(M, N, 1), A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch);
 }
 
 extern "C" int cisr_gemm_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R,

@@ -1167,6 +1167,23 @@ def test_gemm_bf16(ops, M, N, K):
     np.testing.assert_allclose(f64(out), want + f64(r), rtol=1e-4, atol=1e-4 * math.sqrt(K))
 
 
+@pytest.mark.parametrize("tile, rows, cols", [(112, 32, 32), (122, 32, 64), (212, 64, 32), (222, 64, 64), (422, 128, 64), (442, 128, 128), (0, 64, 64)])
+@pytest.mark.parametrize("K", [8, 136, 384, 520, 75])
+def test_gemm_bf16_of_more_tiles_than_a_patch(ops, tile, rows, cols, K):
+    """Nine and eleven tiles a side (patches cut to the matrix), inner sizes of one turn, of as many as are asked for ahead, of one
+    more, and without whole 16-byte chunks; the residual's rows that no tile owns stay."""
+    torch.manual_seed(K)
+    M, N = 8 * rows + 5, 10 * cols + 3
+    a, w = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(N, K, device=DEV).bfloat16()
+    out = torch.full((M + 1, N), 7.0, device=DEV)
+    assert ops.lib().cisr_gemm_bf16_tile(a.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), N, out.data_ptr(), N, M, N, K, 0, tile,
+                                         torch.cuda.current_stream().cuda_stream) == 0
+    want = 7.0 + a.double() @ w.double().T
+    # float accumulation of K products of standard normals: at most K roundings of half an ulp of a sum below 8 sqrt(K)
+    assert (out[:M] - want).abs().max().item() <= K * 2 ** -24 * 8 * K ** 0.5 + 1e-6
+    assert (out[M] == 7.0).all()
+
+
 @pytest.mark.parametrize("tile", [112, 122, 222, 422, 442])
 def test_gemm_bf16_every_block_tile_alone(ops, tile):
     """The rule picks a block tile by the shape; here each built tile (rows / 16 a wave x 100, columns / 16 a wave x 10,
