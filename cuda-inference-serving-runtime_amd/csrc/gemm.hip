@@ -328,15 +328,16 @@ extern "C" int cisr_gemm_bf16_swiglu(const void* A, int lda, const void* W, int 
 // larger its tile, and a second round costs more than a larger tile does.  1,741 rows, us: 576 columns (K 1,536) 32 x 32 12.4, 64 x
 // 32 10.4, 64 x 64 (252 blocks) 8.8, 128 x 64 12.8; 960 columns (K 576) 64 x 64 (420 blocks) 9.8, 128 x 64 (210) 7.4, 128 x 128 10.3.
 // 300 rows x 960: 32 x 32 (300 blocks) 5.1, 64 x 32 (150) 4.6, 64 x 64 5.4.  Where even 128 x 64 needs more, 128 x 128 (4,000 x
-// 2,048, K 512: 128 x 64 in two rounds 17.7, 128 x 128 in one 18.8; K 2,048, 512 blocks against 1,024: 48.6 against 52.8).  Up to 32
-// rows a tile has 32 of them (32 x 12,000, K 1,024: 32 x 64 6.6, 64 x 64 6.8).
+// 2,048, K 512: 128 x 64 in two rounds 17.7, 128 x 128 in one 18.8; K 2,048, 512 blocks against 1,024: 48.6 against 52.8).  Between
+// one round and two of 128 x 128 its last round is mostly idle: 128 x 64 (7,936 x 576, K 1,536, 310 blocks against 620: 36.5 against
+// 32.2; 5,000 x 960, K 576: 19.5 against 15.1).  Up to 32 rows a tile has 32 of them (32 x 12,000, K 1,024: 32 x 64 6.6, 64 x 64 6.8).
 static int pick_tile(int M, int N, int heads) {
     auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * heads; };
     if (blocks(32, 32) <= 256) return 112;
     if (M <= 32) return 122;
     if (blocks(64, 32) <= 256) return 212;
     if (blocks(64, 64) <= 256) return 222;
-    if (blocks(128, 64) <= 256) return 422;
+    if (blocks(128, 64) <= 256 || (blocks(128, 128) > 256 && blocks(128, 128) < 512)) return 422;
     return 442;
 }
 
