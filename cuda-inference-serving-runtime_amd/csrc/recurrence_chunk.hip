@@ -18,15 +18,23 @@
 // The operands lie in memory as the walk's lanes want them, 16 bytes a lane side by side: read in rows of the chunk instead,
 // each load of the walk touches four times the lines.
 // Measured on an MI355X, us of both kernels (in brackets the scans that walk row by row): 2,048 rows of one request, the delta
-// rule with 32 heads of 128 x 128 and a decay a channel 213 with the operands in rows of the chunk, 180 so (840); gated
-// linear attention, 8 heads of 128 x 256, 108 (290), three requests of 782 rows 94 (361); state-space duality, 64 heads of
-// 128 x 64, 193 (495) and 241 (477).  The walk's bound is its chain a chunk (0.7 to 1 us), with many heads what the two
-// kernels write and read in between (30 KB a chunk and head at 128 x 64).
+// rule with 32 heads of 128 x 128 and a decay a channel 207, with a decay a head 176 (840); gated linear attention, 8 heads
+// of 128 x 256, 111 (290), three requests of 782 rows 99 (361); state-space duality, 64 heads of 128 x 64, 170 (495) and
+// 224 (477).  The walk's bound is its chain a chunk (0.7 to 1 us), with many heads what the two kernels write and read in
+// between (30 KB a chunk and head at 128 x 64).
+//
+// Sums: the scans round the state once a row, the walk twice a chunk (what its rows write is summed apart from it); products with
+// the state are a sum a tile of sixteen rows; scores and products of decays are made in double where that is cheap.  Relative
+// error of 1,500 rows' results against 64 bits, row by row / so: delta rule, 8 heads of 128 x 128, decays from 0.999 to 1
+// 3.2e-7 / 1.9e-7, from 0.8 to 1 1.13e-7 / 1.02e-7; gated linear attention, 4 heads of 128 x 256, 5.1e-7 / 2.3e-7 and 9.7e-8 /
+// 8.6e-8; state-space duality, 16 heads of 128 x 64, 5.1e-7 / 2.2e-7 and 1.00e-7 / 8.2e-8.
 #include "common.h"
+#include <type_traits>
 
 #define CHUNK 16
 
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(4))) double f64x4_t;
 
 struct ChunkArgs {
     const float* q; int ldq;          // q[t * ldq + (head / share) * R + r]
@@ -75,8 +83,17 @@ __device__ __forceinline__ float lanes_moved(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
 }
 
+template <int CTRL>
+__device__ __forceinline__ double lanes_moved(double x) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
 // the sum over the 16 lanes of an aligned row, in each of them
-__device__ __forceinline__ float row_sum(float x) {
+template <typename T>
+__device__ __forceinline__ T row_sum(T x) {
     x += lanes_moved<0xB1>(x);                   // quad_perm [1, 0, 3, 2]
     x += lanes_moved<0x4E>(x);                   // quad_perm [2, 3, 0, 1]
     x += lanes_moved<0x141>(x);                  // row_half_mirror
@@ -84,11 +101,24 @@ __device__ __forceinline__ float row_sum(float x) {
     return x;
 }
 
+// The row of its chunk that stands in slot s of the walk's operands.  A matrix instruction of the walk takes slots i, 4 + i, 8 + i
+// and 12 + i (float i of the four that a lane holds of its result), which are rows 4 i .. 4 i + 3: sums over a chunk's
+// rows run in the order of time, so that under strong decays the large terms come last and are rounded few times.
+__host__ __device__ constexpr int row_of_slot(int s) { return 4 * (s % 4) + s / 4; }
+
+// Scores, products of decays and the inverse of I + A are double and rounded once (with a decay a head the scores are Gram matrices,
+// on v_mfma_f64_16x16x4_f64): what is rounded here is an error that all columns of a chunk share, which row by row no two of
+// them do.  (The delta rule with a decay a channel makes them in float: two scores a pair of rows, each with products of
+// decays of its own, are most of its work.)
 template <bool DELTA, bool VEC>
 __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    __shared__ float sA[CHUNK][CHUNK + 1], sBeta[CHUNK];
-    __shared__ __attribute__((aligned(16))) float sM[CHUNK][CHUNK];
+    using Wide = std::conditional_t<VEC && DELTA, float, double>;
+    __shared__ Wide sA[DELTA ? CHUNK : 1][CHUNK + 1];
+    __shared__ double sD[CHUNK], sE[CHUNK], sG[VEC ? 1 : CHUNK];
+    __shared__ double gram[VEC ? 1 : 4][VEC ? 1 : CHUNK * CHUNK];
+    __shared__ __attribute__((aligned(16))) float sM[DELTA ? CHUNK : 1][CHUNK];
+    __shared__ float sBeta[CHUNK];
     const int slot = p.slot0 + blockIdx.y, head = blockIdx.x, tid = threadIdx.x;
     const int seg = segment_of_slot(p.seg_start, p.segments, slot);
     const int t0 = p.seg_start[seg] + (slot - p.seg_start[seg] / CHUNK - seg) * CHUNK, t1 = p.seg_start[seg + 1];
@@ -103,26 +133,30 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
     for (int idx = tid; idx < CHUNK * Rp; idx += 256) {
         const int i = idx / Rp, r = idx % Rp, tt = min(i, n - 1), rr = min(r, R - 1);
         const bool in = r < R && i < n;
-        const float k = kh[tt * p.ldk + rr], q = qh[tt * p.ldq + rr], g = gh[tt * p.ldg + (VEC ? rr : 0)];
+        const float k = kh[tt * p.ldk + rr], q = qh[tt * p.ldq + rr];
         sk[i * RS + r] = in ? k : 0.f;
         sq[i * RS + r] = in ? q * p.q_scale : 0.f;
-        sg[i * RS + r] = in ? g : 1.f;
+        if (VEC) {
+            const float g = gh[tt * p.ldg + rr];
+            sg[i * RS + r] = in ? g : 1.f;
+        }
     }
     if (DELTA && tid < CHUNK) sBeta[tid] = tid < n ? 1.0f / (1.0f + expf(-p.b[(size_t)(t0 + tid) * p.ldb + head])) : 0.f;
     if (!DELTA && tid < CHUNK) sBeta[tid] = tid < n && p.b ? p.b[(size_t)(t0 + tid) * p.ldb + head] : 1.f;     // (the step sizes)
+    if (!VEC && tid < CHUNK) sG[tid] = tid < n ? (double)gh[tid * p.ldg] : 1.0;
     __syncthreads();
     const ChunkLayout<DELTA> at(Rp, p.Cp);
     float* work = p.work + ((size_t)blockIdx.y * p.heads + head) * at.floats;
     float* wP = work + at.pr;
-    // column i of A and P: sixteen neighbouring threads, each with every sixteenth run of four channels, carry k_i down the
-    // rows behind i (times their decays) and meet
-    {
+    if constexpr (VEC) {
+        // column i of A and P: sixteen neighbouring threads, each with every sixteenth run of four channels, carry k_i down the
+        // rows behind i (times their decays) and meet
         const int i = tid / 16, part = tid % 16;
         f32x4_t x[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) x[j] = 64 * j + 4 * part < Rp ? *(const f32x4_t*)(sk + i * RS + 64 * j + 4 * part) : (f32x4_t){0.f, 0.f, 0.f, 0.f};
         for (int t = 0; t < CHUNK; ++t) {
-            float a = 0.f, b = 0.f;
+            Wide a = 0, b = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int r = 64 * j + 4 * part;
@@ -130,54 +164,91 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
                 if (r >= Rp || t < i) continue;
                 const f32x4_t k = *(const f32x4_t*)(sk + t * RS + r), q = *(const f32x4_t*)(sq + t * RS + r);
                 if (t > i) x[j] *= *(const f32x4_t*)(sg + t * RS + r);
-                if (DELTA) a += (x[j][0] * k[0] + x[j][1] * k[1]) + (x[j][2] * k[2] + x[j][3] * k[3]);
-                b += (x[j][0] * q[0] + x[j][1] * q[1]) + (x[j][2] * q[2] + x[j][3] * q[3]);
+                if constexpr (DELTA) {
+                    a += (x[j][0] * k[0] + x[j][1] * k[1]) + (x[j][2] * k[2] + x[j][3] * k[3]);
+                    b += (x[j][0] * q[0] + x[j][1] * q[1]) + (x[j][2] * q[2] + x[j][3] * q[3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) b += (double)x[j][e] * q[e];
+                }
             }
             if (DELTA) a = row_sum(a);
             b = row_sum(b);
             if (part == t) {
                 if (DELTA) sA[t][i] = sBeta[t] * a;                // (only i < t is read)
-                wP[(i / 4 * 16 + t) * 4 + i % 4] = b;              // (0 for i > t)
+                const int row = row_of_slot(t), col = row_of_slot(i);          // (its own inverse)
+                wP[(col / 4 * 16 + row) * 4 + col % 4] = (float)b; // (0 for i > t)
             }
         }
+    } else {
+        // q k^T and, for A, k k^T, a part of the channels a wave
+        const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+        const bool score = !DELTA || wave < 2;
+        const int parts = DELTA ? 2 : 4, part = wave % parts;
+        const float* left = (score ? sq : sk) + lane % 16 * RS + lane / 16;
+        const float* right = sk + lane % 16 * RS + lane / 16;
+        f64x4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int r = part * (Rp / parts); r < (part + 1) * (Rp / parts); r += 4)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)left[r], (double)right[r], acc, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gram[wave][(4 * e + lane / 16) * CHUNK + lane % 16] = acc[e];      // (element e: row 4 e + lane / 16)
+        __syncthreads();
+        const int t = tid / CHUNK, i = tid % CHUNK;
+        double d = 1.0, ahead = 1.0, so_far = 1.0;
+#pragma unroll
+        for (int u = 0; u < CHUNK; ++u) {
+            const double g = sG[u];
+            d *= u > i && u <= t ? g : 1.0;
+            so_far *= u <= i ? g : 1.0;
+            ahead *= u > i ? g : 1.0;
+        }
+        if (t == 0) { sD[i] = so_far; sE[i] = ahead; }
+        const double b = DELTA ? gram[0][tid] + gram[1][tid] : (gram[0][tid] + gram[1][tid]) + (gram[2][tid] + gram[3][tid]);
+        if (DELTA) sA[t][i] = sBeta[t] * (d * (gram[2][tid] + gram[3][tid]));              // (only i < t is read)
+        const int row = row_of_slot(t), col = row_of_slot(i);                                      // (its own inverse)
+        wP[(col / 4 * 16 + row) * 4 + col % 4] = i <= t ? (float)(b * d) : 0.f;
     }
     __syncthreads();
     // column j of the inverse of the unit triangle I + A by forward substitution, times beta_j
     if (DELTA && tid < CHUNK) {
-        float x[CHUNK];
+        Wide x[CHUNK];
 #pragma unroll
-        for (int t = 0; t < CHUNK; ++t) {
-            float s = t == tid ? 1.f : 0.f;
+        for (int t = 0; t < CHUNK; ++t) x[t] = t == tid ? 1 : 0;
 #pragma unroll
-            for (int i = 0; i < t; ++i) s -= sA[t][i] * x[i];
-            x[t] = s;
-            __builtin_amdgcn_sched_barrier(0);                     // (the rows' operands are not asked for all at once: registers)
+        for (int i = 0; i < CHUNK; ++i) {
+#pragma unroll
+            for (int t = i + 1; t < CHUNK; ++t) x[t] -= sA[t][i] * x[i];
+            __builtin_amdgcn_sched_barrier(0);                     // (the columns' operands are not asked for all at once: registers)
         }
 #pragma unroll
-        for (int t = 0; t < CHUNK; ++t) sM[t][tid] = x[t] * sBeta[tid];
+        for (int t = 0; t < CHUNK; ++t) sM[t][tid] = (float)(x[t] * sBeta[tid]);
     }
-    __syncthreads();
+    if (DELTA) __syncthreads();
     // a thread a channel (M Kg and the other operands over the state's rows, which take the place of k, q and the decays) or a
     // column of v (M V)
     for (int idx = tid; idx < Rp + p.Cp; idx += 256) {
         const bool key = idx < Rp;
         const int c = key ? idx : idx - Rp;
-        float x[CHUNK], kd[CHUNK];
+        float x[CHUNK];
         if (key) {
-            float d = 1.f;
+            float kd[CHUNK];
+            Wide d = 1;
 #pragma unroll
             for (int i = CHUNK - 1; i >= 0; --i) {
-                kd[i] = sk[i * RS + c] * d;
-                d *= sg[i * RS + c];
+                if (!VEC) d = sE[i];
+                kd[i] = (float)(sk[i * RS + c] * d);
+                if (VEC) d *= sg[i * RS + c];
             }
-            d = 1.f;
+            d = 1;
 #pragma unroll
             for (int i = 0; i < CHUNK; ++i) {
-                d *= sg[i * RS + c];
-                if (DELTA) x[i] = sk[i * RS + c] * d;
-                sq[i * RS + c] *= d;
+                if (VEC) d *= sg[i * RS + c];
+                else d = sD[i];
+                if (DELTA) x[i] = (float)(sk[i * RS + c] * d);
+                sq[i * RS + c] = (float)(sq[i * RS + c] * d);
             }
-            work[at.g + c] = d;
+            work[at.g + c] = (float)d;
 #pragma unroll
             for (int i = 0; i < CHUNK; ++i) sg[i * RS + c] = kd[i];
         } else {
@@ -188,13 +259,15 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
         float y[CHUNK];
 #pragma unroll
         for (int t = 0; t < CHUNK; ++t) {
-            float s = DELTA ? 0.f : x[t] * sBeta[t];
             if (DELTA) {
+                float s = 0.f;
 #pragma unroll
                 for (int i = 0; i <= t; ++i) s += sM[t][i] * x[i];
+                y[t] = s;
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                y[t] = x[t] * sBeta[t];
             }
-            y[t] = s;
-            if (DELTA) __builtin_amdgcn_sched_barrier(0);
         }
         if (key) {
 #pragma unroll
@@ -202,16 +275,17 @@ __global__ void __launch_bounds__(256, 4) channel_chunk_kernel(ChunkArgs p) {
         } else {
             f32x4_t* wv = (f32x4_t*)(work + at.u) + c / 16 * WAVE + c % 16;
 #pragma unroll
-            for (int t = 0; t < CHUNK; t += 4) wv[t * 4] = (f32x4_t){y[t], y[t + 1], y[t + 2], y[t + 3]};
+            for (int s = 0; s < CHUNK; s += 4) wv[s * 4] = (f32x4_t){y[row_of_slot(s)], y[row_of_slot(s + 1)], y[row_of_slot(s + 2)], y[row_of_slot(s + 3)]};
         }
     }
     __syncthreads();
     for (int unit = tid; unit < Rp * 4; unit += 256) {             // (CHUNK * Rp floats in 16 bytes each)
         const int tile = unit / WAVE, a = unit % 16, b = unit % WAVE / 16 * 4;
-        ((f32x4_t*)(work + at.q))[unit] = *(const f32x4_t*)(sq + a * RS + tile * 16 + b);
-        if (DELTA) ((f32x4_t*)work)[unit] = *(const f32x4_t*)(sk + a * RS + tile * 16 + b);
-        const float* kd = sg + b * RS + tile * 16 + a;
-        ((f32x4_t*)(work + at.kd))[unit] = (f32x4_t){kd[0], kd[RS], kd[2 * RS], kd[3 * RS]};
+        const int row = row_of_slot(a);
+        ((f32x4_t*)(work + at.q))[unit] = *(const f32x4_t*)(sq + row * RS + tile * 16 + b);
+        if (DELTA) ((f32x4_t*)work)[unit] = *(const f32x4_t*)(sk + row * RS + tile * 16 + b);
+        const float* kd = sg + b / 4 * RS + tile * 16 + a;         // (slots b .. b + 3: rows b / 4, 4 + b / 4, ..)
+        ((f32x4_t*)(work + at.kd))[unit] = (f32x4_t){kd[0], kd[4 * RS], kd[8 * RS], kd[12 * RS]};
     }
 }
 
@@ -254,13 +328,14 @@ __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int d = 0; d < AHEAD; ++d) fetch(ring[d], first + d);
         f32x4_t u = {0.f, 0.f, 0.f, 0.f}, pr = u;
         auto finish = [&](int slot, int par) {       // o of the chunk before, whose shares are there now
-            f32x4_t y = (share_o[par][0][lane] + share_o[par][1][lane]) + (share_o[par][2][lane] + share_o[par][3][lane]);
+            f32x4_t own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) y = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[i], u[i], y, 0, 0, 0);
-            const int row = t0 + (slot - base) * CHUNK + 4 * kg;
+            for (int i = 0; i < 4; ++i) own = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[i], u[i], own, 0, 0, 0);
+            const f32x4_t y = ((share_o[par][0][lane] + share_o[par][1][lane]) + (share_o[par][2][lane] + share_o[par][3][lane])) + own;
+            const int row = t0 + (slot - base) * CHUNK + kg;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (row + i < t1 && c < C) p.out[(size_t)(row + i) * p.ldo + (size_t)head * C + c] = y[i];
+            for (int i = 0; i < 4; ++i)                  // (slot 4 kg + i of the chunk)
+                if (row + 4 * i < t1 && c < C) p.out[(size_t)(row + 4 * i) * p.ldo + (size_t)head * C + c] = y[i];
         };
         for (int turn = first; turn < last; turn += AHEAD)
 #pragma unroll
@@ -313,27 +388,40 @@ __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     };
     auto walk = [&](Operands& now, int par) {
-        f32x4_t w = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f};
-        if (DELTA) {
+        const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+        // (a sum a tile of sixteen rows of S, then theirs)
+        auto with_state = [&](const f32x4_t (&left)[NT]) {
+            f32x4_t part[NT];
 #pragma unroll
-            for (int j = 0; j < NT; ++j)
+            for (int j = 0; j < NT; ++j) part[j] = zero;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kg[j][i], S[j][i], w, 0, 0, 0);
-            share_w[par][wave][lane] = w;
-        }
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) part[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(left[j][i], S[j][i], part[j], 0, 0, 0);
+            if constexpr (NT == 4) return (part[0] + part[1]) + (part[2] + part[3]);
+            else if constexpr (NT == 3) return (part[0] + part[1]) + part[2];
+            else if constexpr (NT == 2) return part[0] + part[1];
+            else return part[0];
+        };
+        if constexpr (DELTA) share_w[par][wave][lane] = with_state(now.kg);
         __syncthreads();           // (the other parity's shares were read before the barrier before this one's writes)
         const f32x4_t u = writes(now.u, par);
+        share_o[par][wave][lane] = with_state(now.qg);
+        // what the chunk's rows write is summed apart from S, eight rows and eight: S is rounded twice a chunk instead of sixteen times
+        f32x4_t early[NT], late[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) early[j] = late[j] = zero;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                early[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kd[j][i] * mine[j], u[i], early[j], 0, 0, 0);
+                late[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kd[j][2 + i] * mine[j], u[2 + i], late[j], 0, 0, 0);
+            }
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(now.qg[j][i], S[j][i], o, 0, 0, 0);
-        share_o[par][wave][lane] = o;
-#pragma unroll
-        for (int j = 0; j < NT; ++j) S[j] *= now.g[j];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.kd[j][i] * mine[j], u[i], S[j], 0, 0, 0);
+            for (int i = 0; i < 4; ++i) S[j][i] = fmaf(S[j][i], now.g[j][i], early[j][i]) + late[j][i];
     };
 #pragma unroll
     for (int d = 0; d < AHEAD; ++d) {

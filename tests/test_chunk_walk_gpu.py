@@ -66,6 +66,48 @@ def test_chunks_against_the_recurrence_row_by_row(law, heads, share, R, C):
     assert (after[:, heads * R * C:] == 9.0).all() and np.array_equal(after[[2, 6], :-3], begun[[2, 6]].reshape(2, -1).astype(np.float32))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("law, heads, share, R, C", [("delta", 4, 2, 128, 128), ("delta", 2, 1, 64, 64), ("channel", 2, 1, 128, 128), ("head", 8, 8, 128, 64)])
+@pytest.mark.parametrize("decays", ["near one", "0.8 to one", "any"])
+def test_chunks_are_no_further_from_64_bits_than_the_walk_row_by_row(law, heads, share, R, C, decays):
+    """The same operands through both forms, 300 rows from a state that is not zero.  Results: the relative error of the chunks is at
+    most that of the rows.  The state: within a tenth of it (under strong decays both round a state's last rows a few times,
+    and which of the two ends closer depends on the draw)."""
+    from runtime.kernels import ops
+    T, vec, is_delta = 300, law == "channel", law == "delta"
+    gen = torch.Generator(device=DEV).manual_seed(R + C + heads)
+    draw = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    unit = lambda x: torch.nn.functional.normalize(x, dim=-1).reshape(T, -1).contiguous()
+    q, k, v = unit(draw(T, heads // share, R)), unit(draw(T, heads // share, R)), draw(T, heads * C)
+    u = torch.rand(T, heads * R if vec else heads, device=DEV, generator=gen)
+    g = {"near one": 1 - 1e-3 * u, "0.8 to one": 0.8 + 0.2 * u, "any": u ** 3}[decays]
+    b = draw(T, heads) if is_delta else draw(T, heads).abs() + 0.1
+    begun = 0.3 * draw(1, heads * R * C)
+    S, want = begun.double().view(heads, R, C), []
+    for t in range(T):
+        kk, qq = (x[t].double().view(-1, R).repeat_interleave(share, 0) for x in (k, q))
+        S = S * g[t].double().view(heads, -1, 1)
+        w = v[t].double().view(heads, C)
+        w = torch.sigmoid(b[t].double())[:, None] * (w - (S * kk[:, :, None]).sum(1)) if is_delta else w if vec else w * b[t].double()[:, None]
+        S = S + kk[:, :, None] * w[:, None, :]
+        want.append((S * qq[:, :, None]).sum(1).reshape(-1))
+    want, end = torch.stack(want), S.reshape(1, -1)
+    where, sizes = (ints([0, T]), ints([0])), (heads, R, C)
+    errors = []
+    for chunks in (False, True):
+        state, out = begun.clone(), torch.empty(T, heads * C, device=DEV)
+        work = torch.empty(ops.channel_chunk_work(T, 1, *sizes, delta=is_delta), device=DEV)
+        if is_delta:
+            args = (q, k, v, g, b, out, state, *where, *sizes)
+            ops.channel_delta_chunks(*args, work, share=share) if chunks else ops.delta_scan(*args, share=share)
+        else:
+            args, kw = (q, k, v, g, out, state, *where, *sizes), dict(share=share, step=None if vec else b)
+            ops.linear_chunks(*args, work, **kw) if chunks else ops.linear_scan(*args, **kw)
+        errors.append([((x.double() - y).norm() / y.norm()).item() for x, y in ((out, want), (state, end))])
+    (rows_out, rows_state), (out, state) = errors
+    assert out <= rows_out and state <= 1.1 * rows_state, errors
+
+
 def test_the_oracle_is_the_designs_recurrence():
     """The loop above is the designs' plain recurrences (from a state of zero, for one head)."""
     rng = np.random.default_rng(1)
