@@ -79,11 +79,16 @@ attn_f32_kernel(AttnF32Args p) {
         for (int c = 0; c < DT; ++c) fv[c] = *(const af_f32x4*)(vr + (size_t)16 * c * P);
     };
     auto use = [&](int s, af_f32x4 (&fk)[DT], af_f32x4 (&fv)[DT]) {
-        af_f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+        // (a sum for every second sixteen of coordinates: half the chain of instructions, and of roundings)
+        af_f32x4 sc = {0.f, 0.f, 0.f, 0.f}, odd = sc;
 #pragma unroll
-        for (int c = 0; c < DT; ++c)
+        for (int c = 0; c < DT; c += 2)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[c][e], fq[c][e], sc, 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+                sc = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[c][e], fq[c][e], sc, 0, 0, 0);
+                odd = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[c + 1][e], fq[c + 1][e], odd, 0, 0, 0);
+            }
+        sc += odd;
         // sc[e]: item r, key s * 16 + 4 g + e
         float best = -INFINITY;
 #pragma unroll

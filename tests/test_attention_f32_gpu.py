@@ -64,3 +64,26 @@ def test_what_attention_f32_takes():
     assert not any(ops.attention_f32_ok(q, 64, kc, vc, dim, page) for dim, page in ((48, 16), (256, 16), (64, 2), (64, 12)))
     assert not ops.attention_f32_ok(q.bfloat16(), 64, kc, vc, 64, 16) and not ops.attention_f32_ok(q, 66, kc, vc, 64, 16)
     assert not ops.attention_f32_ok(q.view(-1)[1:], 64, kc, vc, 64, 16)
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim", [(9, 3, 64), (32, 8, 128), (8, 1, 128), (4, 4, 32)])
+def test_no_further_from_64_bits_than_the_row_wise_kernel(heads, kv_heads, dim):
+    """Single rows of wide scores (spread 3) at a few hundred keys, where a score's own rounding decides: the relative error is at
+    most the row-wise kernel's on the same operands."""
+    from runtime.kernels import ops
+    lengths, page = [200, 320, 77, 450], 16
+    _, kt, vt, tables, _ = paged_case(heads, kv_heads, dim, page, lengths, torch.float32, seed=dim)
+    rows = [(s, n - 1) for s, n in enumerate(lengths)]
+    q, scale = rnd(len(rows), heads, dim, seed=3, scale=3.0), 1.0 / math.sqrt(dim)
+    want = reference_attention(q, kt, vt, tables, rows, page, scale=scale)
+    ints = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    pos, flat, errors = ints([p for _, p in rows]), q.reshape(len(rows), -1).contiguous(), []
+    for tiles in (False, True):
+        out = torch.empty(len(rows), heads * dim, device=DEV)
+        args = (out, heads, kv_heads, dim, page, None, scale)
+        if tiles:
+            ops.attention_f32(flat, heads * dim, kt, vt, tables, pos, tasks_of(rows, 16 // min(heads // kv_heads, 16)), *args)
+        else:
+            ops.attention_rowwise(flat, heads * dim, kt, vt, tables, ints([s for s, _ in rows]), pos, *args)
+        errors.append(np.linalg.norm(f64(out).reshape(want.shape) - want) / np.linalg.norm(want))
+    assert errors[1] <= errors[0], errors
