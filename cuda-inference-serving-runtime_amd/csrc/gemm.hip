@@ -300,13 +300,17 @@ static int swiglu_tile_entry(const void* A, int lda, const void* W, int ldw, voi
     auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((2 * N + bn - 1) / bn); };
     if (tile == 0) {
         // As below, over the columns of both halves: 300 rows, 1,536 outputs, K 576: 32 x 64 (480 blocks) 6.8 us, 64 x 64 (240) 6.1,
-        // 128 x 64 7.8.  Between one round and two of 128 x 128 the last round is mostly idle, and 128 x 64 is faster (1,741 rows
-        // there, 336 blocks: 15.7 against 16.6; 600 rows, 4,096 outputs, K 2,048: 39.7 against 41.6); from two on it is not (4,000
-        // rows: 27.8 against 24.9).
+        // 128 x 64 7.8; 300 rows, 3,072 outputs: 64 x 64 (480 blocks, two a unit) 9.5, 128 x 64 (288) 12.4, 128 x 128 12.8.  With one
+        // round of 128 x 128, 128 x 64 up to K 576 (1,000 rows, 1,536 outputs: 12.0 against 12.4), 128 x 128 from there (1,000 rows,
+        // 2,048 outputs, K 1,024: 17.5 against 17.1; 500 rows, 4,096 outputs, K 2,048: 32.8 against 29.5).  With a second round that
+        // is mostly idle 128 x 64 (1,500 rows, 2,048 outputs, K 1,024, 384 blocks: 24.1 against 25.6), from 400 blocks on 128 x 128
+        // (1,777 rows, 448 blocks: 29.8 against 26.0; 4,000 rows of 1,536 outputs, K 576: 29.0 against 26.3).
         if (blocks(32, 64) <= 256) tile = 122;
         else if (blocks(64, 64) <= 256) tile = 222;
-        else if (blocks(128, 64) <= 256 || (blocks(128, 128) > 256 && blocks(128, 128) < 512)) tile = 422;
-        else tile = 442;
+        else if (blocks(128, 64) <= 256) tile = 422;
+        else if (blocks(64, 64) <= 512) tile = 222;
+        else if (blocks(128, 128) <= 256) tile = K <= 576 ? 422 : 442;
+        else tile = blocks(128, 128) < 400 ? 422 : 442;
     }
 #define SWIGLU_TILE(CODE, TM, TN, BK, WM, PF) \
     case CODE: return launch_bf16_swiglu<TM, TN, BK, WM, PF>(a, lda, w, ldw, (bf16_t*)C, ldc, M, N, K, dual_off, law, stream);
@@ -327,18 +331,27 @@ extern "C" int cisr_gemm_bf16_swiglu(const void* A, int lda, const void* W, int 
 // Tile choice: the smallest that needs no more blocks than there are compute units: a block alone on its unit takes the longer the
 // larger its tile, and a second round costs more than a larger tile does.  1,741 rows, us: 576 columns (K 1,536) 32 x 32 12.4, 64 x
 // 32 10.4, 64 x 64 (252 blocks) 8.8, 128 x 64 12.8; 960 columns (K 576) 64 x 64 (420 blocks) 9.8, 128 x 64 (210) 7.4, 128 x 128 10.3.
-// 300 rows x 960: 32 x 32 (300 blocks) 5.1, 64 x 32 (150) 4.6, 64 x 64 5.4.  Where even 128 x 64 needs more, 128 x 128 (4,000 x
-// 2,048, K 512: 128 x 64 in two rounds 17.7, 128 x 128 in one 18.8; K 2,048, 512 blocks against 1,024: 48.6 against 52.8).  Between
-// one round and two of 128 x 128 its last round is mostly idle: 128 x 64 (7,936 x 576, K 1,536, 310 blocks against 620: 36.5 against
-// 32.2; 5,000 x 960, K 576: 19.5 against 15.1).  Up to 32 rows a tile has 32 of them (32 x 12,000, K 1,024: 32 x 64 6.6, 64 x 64 6.8).
-static int pick_tile(int M, int N, int heads) {
+// 300 rows x 960: 32 x 32 (300 blocks) 5.1, 64 x 32 (150) 4.6, 64 x 64 5.4.  Up to 32 rows a tile has 32 of them (32 x 12,000, K
+// 1,024: 32 x 64 6.6, 64 x 64 6.8).
+// Where 128 x 64 needs more than one round, us of 64 x 64 / 128 x 64 / 128 x 128:
+//   64 x 64 twice a unit at once (its LDS leaves room for two): 1,300 x 1,536 (504, 264 and 132 blocks), K 576 11.9 / 12.5 / 12.3, K
+//   1,536 18.7 / 24.3 / 21.5; 1,500 rows (576 of 64 x 64) are too many for that: 25.8 / 24.0 / 21.6;
+//   one round of 128 x 128: the same up to K 576 (2,000 x 2,048, 512 and 256 blocks, K 512: 18.3 / 12.7 / 13.1; 1,777 x 1,536, 336
+//   and 168, K 576: 16.1 / 12.9 / 12.8), above it the larger tile's fewer bytes (2,000 x 2,048, K 1,024 27.0 / 20.5 / 19.8, K 2,048
+//   41.0 / 31.8 / 29.0; 1,777 x 1,536, K 1,536 25.9 / 24.0 / 22.3);
+//   more than one: 128 x 64 up to K 1,536 (4,000 x 2,048, 1,024 and 512 blocks, K 512: 24.2 / 26.0; 6,000 x 1,536, 1,128 and 564, K
+//   1,536: 54.1 / 61.2; 8,000 x 1,536: 66.1 / 64.3) and where the second round of 128 x 128 is mostly idle (7,936 x 576, K 1,536,
+//   558 and 310 blocks: 32.2 / 36.5), else 128 x 128 (8,000 x 1,024, K 2,048, 1,008 and 504: 56.4 / 54.1).
+static int pick_tile(int M, int N, int K, int heads) {
     auto blocks = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * heads; };
     if (blocks(32, 32) <= 256) return 112;
     if (M <= 32) return 122;
     if (blocks(64, 32) <= 256) return 212;
     if (blocks(64, 64) <= 256) return 222;
-    if (blocks(128, 64) <= 256 || (blocks(128, 128) > 256 && blocks(128, 128) < 512)) return 422;
-    return 442;
+    if (blocks(128, 64) <= 256) return 422;
+    if (blocks(64, 64) <= 512) return 222;
+    if (blocks(128, 128) <= 256) return K <= 576 ? 422 : 442;
+    return K <= 1536 || blocks(128, 128) < 400 ? 422 : 442;
 }
 
 static int launch_tile(int tile, const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R, int ldr, int M, int N,
@@ -359,7 +372,7 @@ extern "C" int cisr_gemm_bf16_tile(const void* A, int lda, const void* W, int ld
                                    int ldr, int M, int N, int K, int out_dtype, int tile, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || (R && out_dtype != DT_F32)) return (int)hipErrorInvalidValue;
-    return launch_tile(tile ? tile : pick_tile(M, N, 1), A, lda, W, ldw, C, ldc, R, ldr, M, N, K, out_dtype, stream);
+    return launch_tile(tile ? tile : pick_tile(M, N, K, 1), A, lda, W, ldw, C, ldc, R, ldr, M, N, K, out_dtype, stream);
 }
 
 // A product a head in one launch: C[m, h * c_head + n] = sum_k A[m, h * a_head + k] W[h][n][k] (W [heads, N, K] contiguous),
@@ -369,7 +382,7 @@ extern "C" int cisr_gemm_bf16_heads(const void* A, int lda, int a_head, const vo
     if (M <= 0 || N <= 0 || heads <= 0) return 0;
     if (K <= 0) return (int)hipErrorInvalidValue;
     const HeadBatch batch{a_head, (long long)N * K, c_head, gate, ldg, ACT_NONE};
-    return launch_tile(pick_tile(M, N, heads), A, lda, W, K, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch, heads);
+    return launch_tile(pick_tile(M, N, K, heads), A, lda, W, K, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch, heads);
 }
 
 // C = act(A . W^T) with an ungated activation (ACT_GELU, ACT_GELU_TANH, ACT_RELU2) as the epilogue; the tile is picked as for the
@@ -379,7 +392,7 @@ extern "C" int cisr_gemm_bf16_act(const void* A, int lda, const void* W, int ldw
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || act < ACT_GELU || act > ACT_RELU2) return (int)hipErrorInvalidValue;
     const HeadBatch batch{0, 0, 0, nullptr, 0, act};
-    return launch_tile(pick_tile(M, N, 1), A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch);
+    return launch_tile(pick_tile(M, N, K, 1), A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, out_dtype, stream, batch);
 }
 
 extern "C" int cisr_gemm_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R,

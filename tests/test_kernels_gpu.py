@@ -1184,11 +1184,10 @@ def test_gemm_bf16_of_more_tiles_than_a_patch(ops, tile, rows, cols, K):
     assert (out[M] == 7.0).all()
 
 
-@pytest.mark.parametrize("tile", [112, 122, 222, 422, 442])
+@pytest.mark.parametrize("tile", [112, 122, 212, 222, 422, 442])
 def test_gemm_bf16_every_block_tile_alone(ops, tile):
-    """The rule picks a block tile by the shape; here each built tile (rows / 16 a wave x 100, columns / 16 a wave x 10,
-    waves along the rows) multiplies shapes that no tile divides, with and without the residual, and the activation
-    where the tile pairs column tiles."""
+    """The rule picks a block tile by the shape; here each built tile (its code: rows / 32 x 100 + columns / 32 x 10 + 2) multiplies
+    shapes that no tile divides, with and without the residual, and the activation where the tile pairs column tiles."""
     stream = torch.cuda.current_stream().cuda_stream
     for M, N, K in ((150, 200, 136), (70, 1000, 72), (333, 96, 520)):
         a, w, r = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2), rnd(M, N, seed=3)
