@@ -95,8 +95,14 @@ conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* _
 // The same for portions, four channels a thread and CONV_ROWS rows of the step a block: an input is read once (the taps - 1
 // before a block's first row again), eight rows' 16-byte loads are on their way together.  The same sums in the same order.
 // Channels, row stride and first column multiples of 4, pointers 16-byte aligned.  The last blocks of y make the gates.
-// 2,048 rows of 8,192 channels, four taps: 90 us with a thread a (row, channel), 45 so (134 MB).
+// 2,048 rows of 8,192 channels, four taps: 90 us with a thread a (row, channel), 45 so (134 MB).  A block's walk takes 12 to 14 us
+// however few blocks there are, more where it meets portions that begin (their first rows wait for the state, one after the
+// other; 16 single rows 22 us).  Steps of fewer inputs than that is worth keep a thread a (row, channel): 128 rows of 8,192 channels
+// 10.1 us against 13.1 (200 rows 14.8 against 13.9), 1,024 of 1,024 9.6 against 12.7 (1,500 rows 13.2 against 12.8); 24 single
+// rows beside 256, 8,192 channels, 18.9 against 25.2 (beside 512 28.8 against 26.9).
 #define CONV_ROWS 16
+#define CONV_WORDS (3ll << 19)               // inputs of a step of one portion
+#define CONV_WORDS_A_PORTION 170000ll        // and for each of up to sixteen more
 typedef __attribute__((ext_vector_type(4))) float conv_f32x4;
 template <int TAPS>
 __global__ void __launch_bounds__(256)
@@ -205,7 +211,8 @@ extern "C" int cisr_conv_silu(const float* in, int ld, int first, const float* w
             out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay);
         return CISR_LAUNCH_CHECK();
     }
-    if (taps >= 2 && taps <= 4 && channels % 4 == 0 && ld % 4 == 0 && first % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+    const bool enough = (long long)rows * channels >= CONV_WORDS + CONV_WORDS_A_PORTION * min(segments - 1, 16);
+    if (enough && taps >= 2 && taps <= 4 && channels % 4 == 0 && ld % 4 == 0 && first % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0 &&
         (!bias || (uintptr_t)bias % 16 == 0)) {
         const dim3 blocks((rows + CONV_ROWS - 1) / CONV_ROWS, (channels / 4 + 255) / 256 + (heads + 255) / 256);
 #define CONV_ROWS_OF(TAPS) conv_silu_rows_kernel<TAPS><<<blocks, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride, \
@@ -282,8 +289,11 @@ extern "C" int cisr_decay_gate_low_rank(const float* low, int ld, int rank, cons
     const size_t n = (size_t)rows * cols;
     if (n == 0) return 0;
     if (!(tau > 0.f) || rank <= 0) return (int)hipErrorInvalidValue;
-    // (from a block for every other compute unit on)
-    if ((long long)((cols + 255) / 256) * ((rows + GATE_ROWS - 1) / GATE_ROWS) >= 128 && rows <= 65535 * GATE_ROWS)
+    // From a block for every compute unit on, and from about 12,000 blocks times rank on.  A decay a thread / so: rank 16, 512 rows of
+    // 1,024 (256 blocks) 5.5 / 6.9, 782 of 2,048 (784) 11.3 / 10.8; rank 32, 300 rows of 2,048 (304) 8.3 / 8.9, 512 (512) 11.3 /
+    // 9.2; rank 128, 64 rows of 4,096 (128) 11.4 / 12.3, 130 (272) 21.7 / 12.9.
+    const long long blocks = (long long)((cols + 255) / 256) * ((rows + GATE_ROWS - 1) / GATE_ROWS);
+    if (blocks >= 256 && blocks * rank >= 12000 && rows <= 65535 * GATE_ROWS)
         decay_gate_low_rank_rows_kernel<<<dim3((cols + 255) / 256, (rows + GATE_ROWS - 1) / GATE_ROWS), 256, 0, stream>>>(low, ld, rank, up, bias, a, rows, cols, 1.0f / tau);
     else
         decay_gate_low_rank_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(low, ld, rank, up, bias, a, cols, n, 1.0f / tau);

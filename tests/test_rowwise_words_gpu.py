@@ -18,10 +18,12 @@ def ints(a):
     return torch.tensor([int(x) for x in a], dtype=torch.int32, device=DEV)
 
 
-@pytest.mark.parametrize("channels, taps, heads, bias", [(4, 2, 0, True), (1028, 4, 3, True), (300, 3, 300, False), (8, 4, 1, False)])
+@pytest.mark.parametrize("channels, taps, heads, bias", [(4, 2, 0, True), (1028, 4, 3, True), (300, 3, 300, False), (8, 4, 1, False),
+                                                         (27000, 2, 0, True), (26004, 4, 3, True), (26500, 3, 300, False)])
 def test_short_convolution_in_words(channels, taps, heads, bias):
     """Portions shorter than the taps, of one row, of more rows than a block takes, that begin inside a block and at its first
-    row; rows of no segment; inputs and state as columns of wider rows."""
+    row; rows of no segment; inputs and state as columns of wider rows.  Few channels keep a thread an input (the step is too
+    small for the form in words), many take the words."""
     from runtime.kernels import ops
     counts, slots = [5, 1, 43, 0, 16, 2, 33], [2, 0, 5, 1, 6, 3, 4]
     pad, T = 3, sum(counts) + 3
