@@ -77,7 +77,7 @@ def test_group_norm_and_gate_in_words(groups, size, gate_first, sigmoid, skip, s
     close(out, u if gate_first else u * law, 3e-6 if dtype == torch.float32 else 5e-3)
 
 
-@pytest.mark.parametrize("rows, cols, rank", [(1025, 256, 16), (513, 520, 3), (130, 2049, 17), (3, 100, 5)])
+@pytest.mark.parametrize("rows, cols, rank", [(1025, 256, 16), (513, 520, 3), (130, 2049, 17), (3, 100, 5), (2051, 1024, 16), (1033, 700, 40)])
 def test_low_rank_decays_several_rows_a_thread(rows, cols, rank):
     from runtime.kernels import ops
     low, up, bias = torch.randn(rows, rank + 3, device=DEV)[:, 1:1 + rank], torch.randn(rank, cols, device=DEV), torch.randn(cols, device=DEV)
