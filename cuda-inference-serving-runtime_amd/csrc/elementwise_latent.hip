@@ -377,7 +377,10 @@ __global__ void __launch_bounds__(256) gelu_kernel(const T* __restrict__ x, T* _
     if (i < n) store_f32(out + i, unary_activation(load_f32(x + i), kind + 1));
 }
 
-// The same for bf16 in 16-byte words: 2,048 rows of 8,192 39.5 us an element a thread (2-byte accesses), 19.6 so.
+// The same for bf16 in 16-byte words: 2,048 rows of 8,192 39.5 us an element a thread (2-byte accesses), 19.6 so.  A thread's eight
+// gelus are a chain of their own: under GELU_WORDS elements an element a thread is faster (64 rows of 2,048 3.2 us against 4.3,
+// 512 of 2,048 4.0 against 4.3).
+#define GELU_WORDS (2ll << 20)
 __global__ void __launch_bounds__(256) gelu_bf16x8_kernel(const uint4* __restrict__ x, uint4* __restrict__ out, size_t n8, int kind) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n8) return;
@@ -411,7 +414,7 @@ extern "C" int cisr_gelu(const void* x, void* out, long long n, int kind, int dt
     if (n <= 0) return 0;
     if (kind < 0 || kind > 2) return (int)hipErrorInvalidValue;
     const unsigned blocks = (unsigned)((n + 255) / 256);
-    if (dtype != DT_F32 && n % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0) {
+    if (dtype != DT_F32 && n >= GELU_WORDS && n % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0) {
         gelu_bf16x8_kernel<<<(unsigned)((n / 8 + 255) / 256), 256, 0, stream>>>((const uint4*)x, (uint4*)out, (size_t)n / 8, kind);
         return CISR_LAUNCH_CHECK();
     }

@@ -85,7 +85,7 @@ def test_low_rank_decays_several_rows_a_thread(rows, cols, rank):
     close(out, torch.exp(torch.nn.functional.logsigmoid(low.double() @ up.double() + bias.double()) / 16.0), 2e-6)
 
 
-@pytest.mark.parametrize("n", [8, 2048 * 8 + 8, 12])
+@pytest.mark.parametrize("n", [8, 2048 * 8 + 8, 12, (2 << 20) + 8, (2 << 20) + 12])
 @pytest.mark.parametrize("form", ["gelu", "gelu_tanh"])
 def test_gelu_of_bf16_words(n, form):
     from runtime.kernels import ops
