@@ -152,16 +152,21 @@ extern "C" int cisr_argmax_noalloc(const float* logits, int* out, int rows, int 
 // that walks its slice alone.  The chosen slice's weights are made the same way before one thread walks them.  Bound by trips
 // to memory (three passes over the row out of the cache): 49,152 logits 100 us with 256 threads walking a slice each and one
 // walking the chosen one (78 in a graph of such calls, 38 so).
-#define SAMPLE_THREADS 1024
+// Vocabularies of up to SAMPLE_SMALL (SMALL: 256 threads, which make and add their slice of up to 14 weights alone): there the
+// larger block and its meetings cost more than they save, 1,000 logits 13.1 us against 15.7, 3,000 15.0 against 16.3 (4,000:
+// 16.8 against 16.6).
+#define SAMPLE_SMALL 3584
 #define SAMPLE_STEP 32
-__global__ void __launch_bounds__(SAMPLE_THREADS)
+template <bool SMALL>
+__global__ void __launch_bounds__(SMALL ? 256 : 1024)
 sample_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
               const unsigned long long* __restrict__ seeds, const unsigned long long* __restrict__ counters,
               int* __restrict__ out, const int* __restrict__ index, int out_n, int vocab) {
-    __shared__ float smax[SAMPLE_THREADS];
-    __shared__ int sidx[SAMPLE_THREADS];
+    constexpr int THREADS = SMALL ? 256 : 1024;
+    __shared__ float smax[THREADS];
+    __shared__ int sidx[THREADS];
     __shared__ float ssum[256];
-    __shared__ float weight[256][SAMPLE_STEP + 1];
+    __shared__ float weight[SMALL ? 1 : 256][SAMPLE_STEP + 1];
     __shared__ float run_at;
     __shared__ int slice_at;
     const int row = blockIdx.x, tid = threadIdx.x;
@@ -169,7 +174,7 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
     if (dst < 0 || dst >= out_n) return;       // the whole block: no barrier is passed by a part of it
     const float* x = logits + (size_t)row * vocab;
     float best; int best_idx;
-    argmax_block<SAMPLE_THREADS>(x, vocab, smax, sidx, best, best_idx);
+    argmax_block<THREADS>(x, vocab, smax, sidx, best, best_idx);
     const float temp = temperature[row];
     if (!(temp > 0.f)) {  // greedy
         if (tid == 0) out[dst] = best_idx == 0x7fffffff ? 0 : best_idx;
@@ -177,26 +182,31 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
     }
     const float inv_t = 1.0f / temp;
     const int per = (vocab + 255) / 256;
-    constexpr int TURNS = 256 * SAMPLE_STEP / SAMPLE_THREADS;        // words a thread makes of a step
+    constexpr int TURNS = 256 * SAMPLE_STEP / THREADS;               // words a thread makes of a step
     float part = 0.f;                                                // (of slice tid, tid < 256)
-    for (int j0 = 0; j0 < per; j0 += SAMPLE_STEP) {
-        float v[TURNS];
+    if constexpr (SMALL) {
+        const int lo = tid * per, hi = min(vocab, lo + per);
+        for (int i = lo; i < hi; ++i) part += expf((x[i] - best) * inv_t);
+    } else {
+        for (int j0 = 0; j0 < per; j0 += SAMPLE_STEP) {
+            float v[TURNS];
 #pragma unroll
-        for (int i = 0; i < TURNS; ++i) {
-            const int idx = tid + SAMPLE_THREADS * i, at = idx / SAMPLE_STEP * per + j0 + idx % SAMPLE_STEP;
-            v[i] = x[min(at, vocab - 1)];
-        }
-        __syncthreads();                                             // (the step before is added up)
+            for (int i = 0; i < TURNS; ++i) {
+                const int idx = tid + THREADS * i, at = idx / SAMPLE_STEP * per + j0 + idx % SAMPLE_STEP;
+                v[i] = x[min(at, vocab - 1)];
+            }
+            __syncthreads();                                         // (the step before is added up)
 #pragma unroll
-        for (int i = 0; i < TURNS; ++i) {
-            const int idx = tid + SAMPLE_THREADS * i;
-            weight[idx / SAMPLE_STEP][idx % SAMPLE_STEP] = expf((v[i] - best) * inv_t);
-        }
-        __syncthreads();
-        if (tid < 256) {
-            const int n = min(min(per - j0, SAMPLE_STEP), vocab - (tid * per + j0));
+            for (int i = 0; i < TURNS; ++i) {
+                const int idx = tid + THREADS * i;
+                weight[idx / SAMPLE_STEP][idx % SAMPLE_STEP] = expf((v[i] - best) * inv_t);
+            }
+            __syncthreads();
+            if (tid < 256) {
+                const int n = min(min(per - j0, SAMPLE_STEP), vocab - (tid * per + j0));
 #pragma unroll 8
-            for (int j = 0; j < n; ++j) part += weight[tid][j];
+                for (int j = 0; j < n; ++j) part += weight[tid][j];
+            }
         }
     }
     if (tid < 256) ssum[tid] = part;
@@ -210,10 +220,24 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
         float run = 0.f;
         int t = 0;
         for (; t < 256; ++t) { if (run + ssum[t] > target) break; run += ssum[t]; }
-        smax[0] = target;
-        run_at = run;
-        slice_at = t;
+        if constexpr (SMALL) {                                       // then the token inside it, as below
+            int choice = -1;
+            if (t < 256) {
+                const int a = t * per, b = min(vocab, a + per);
+                for (int i = a; i < b; ++i) {
+                    run += expf((x[i] - best) * inv_t);
+                    if (run > target) { choice = i; break; }
+                }
+                if (choice < 0) choice = b - 1;
+            }
+            out[dst] = choice < 0 ? best_idx : choice;
+        } else {
+            smax[0] = target;
+            run_at = run;
+            slice_at = t;
+        }
     }
+    if constexpr (SMALL) return;
     __syncthreads();
     const int t = slice_at;
     const float target = smax[0];
@@ -227,7 +251,7 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
         for (int a0 = a; a0 < b; a0 += ROOM) {
             const int n = min(b - a0, ROOM);
             __syncthreads();
-            for (int i = tid; i < n; i += SAMPLE_THREADS) slice[i] = expf((x[a0 + i] - best) * inv_t);
+            for (int i = tid; i < n; i += THREADS) slice[i] = expf((x[a0 + i] - best) * inv_t);
             __syncthreads();
             if (tid == 0 && choice < 0)
                 for (int i = 0; i < n; ++i) {
@@ -245,7 +269,9 @@ extern "C" int cisr_sample(const float* logits, const float* temperature, const 
                            const unsigned long long* counters, int* out, const int* index, int out_n, int rows, int vocab,
                            hipStream_t stream) {
     if (rows <= 0) return 0;
-    sample_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(logits, temperature, seeds, counters, out, index, index ? out_n : rows, vocab);
+    const int slots = index ? out_n : rows;
+    if (vocab <= SAMPLE_SMALL) sample_kernel<true><<<rows, 256, 0, stream>>>(logits, temperature, seeds, counters, out, index, slots, vocab);
+    else sample_kernel<false><<<rows, 1024, 0, stream>>>(logits, temperature, seeds, counters, out, index, slots, vocab);
     return CISR_LAUNCH_CHECK();
 }
 

@@ -1302,6 +1302,24 @@ def test_sampling_kernel(ops):
     assert one[0] == five[2]
 
 
+@pytest.mark.parametrize("V", [1, 7, 300, 3584, 3585, 8192, 40001])
+def test_sampled_tokens_stand_where_the_distribution_says(ops, V):
+    """Both forms of the kernel (up to 3,584 logits and more), the last slices short or empty.  The random number of a draw lies in its
+    token's interval of the distribution in 64 bits, give or take the roundings of the sums: a slice of V / 256 weights, then
+    256 slices, added twice."""
+    from runtime.sampling import uniform01
+    z, temp = rnd(40, V, seed=V, scale=2.0), torch.linspace(0.3, 1.7, 40, device=DEV)
+    ints = lambda a: torch.tensor(a, dtype=torch.int64, device=DEV)
+    out = ops.sample(z, temp, ints([77] * 40), ints(range(40)), torch.empty(40, dtype=torch.int32, device=DEV)).cpu().numpy()
+    x = f64(z) / f64(temp)[:, None]
+    cdf = np.cumsum(np.exp(x - x.max(1, keepdims=True)), 1)
+    cdf /= cdf[:, -1:]
+    tol = 2 * (-(-V // 256) + 256) * 2.0 ** -24 + 1e-5          # (1e-5: the exponentials, of arguments up to 60)
+    for row, token in enumerate(out):
+        u = uniform01(77, row)
+        assert (cdf[row, token - 1] if token else 0.0) - tol <= u <= cdf[row, token] + tol, (row, token, u)
+
+
 def test_page_copy(ops):
     pool = rnd(3, 2, 5, 2, 4, 8, dtype=torch.bfloat16)   # [sites, k/v, pages, kv_heads, page, dim]
     before = pool.clone()
