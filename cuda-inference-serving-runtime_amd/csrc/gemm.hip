@@ -64,7 +64,7 @@ __host__ __device__ inline int patch_side(int tiles) {
 // activation is applied before the store.  Zeros: one product, no gate, no activation.
 struct HeadBatch { long long a, w, c; const float* gate; int ldg; int act; };
 
-template <int TM, int TN, int BK, typename TC, bool VEC, bool SWIGLU = false, int WM = 2, int PF = 3>
+template <int TM, int TN, int BK, typename TC, bool VEC, bool TAIL, bool SWIGLU = false, int WM = 2, int PF = 3>
 __global__ void __launch_bounds__(WM * 128)
 gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
                  TC* C, int ldc, const float* R, int ldr, int M, int N, int K, int dual_off = 0, GateLaw law = {},
@@ -140,19 +140,15 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict
 
     auto turn = [&](int t, u32x4 (&ta)[A_PER_THREAD], u32x4 (&tw)[W_PER_THREAD], bool ask) {
         const int kk0 = t * BK, buf = t & 1;
+        // TAIL (K is no multiple of BK): chunks beyond K, which only the last tile has and the loop's turns (ask) never see, are
+        // cleared on both sides: zero times an infinite weight of the row's last chunk, which they repeat, is no number.
+        auto put = [&](bf16_t* to, int c, const u32x4& chunk) {
+            *(u32x4*)(to + lds_at(c / CPR, c % CPR)) = chunk & (TAIL && !ask && kk0 + c % CPR * 8 >= K ? 0u : 0xffffffffu);
+        };
 #pragma unroll
-        for (int i = 0; i < A_PER_THREAD; ++i) {
-            const int c = tid + i * NT;
-            const uint32_t keep = (VEC && kk0 + (c % CPR) * 8 >= K) ? 0u : 0xffffffffu;
-            u32x4 v = ta[i];
-            v.x &= keep; v.y &= keep; v.z &= keep; v.w &= keep;
-            *(u32x4*)(&As[buf][lds_at(c / CPR, c % CPR)]) = v;
-        }
+        for (int i = 0; i < A_PER_THREAD; ++i) put(As[buf], tid + i * NT, ta[i]);
 #pragma unroll
-        for (int i = 0; i < W_PER_THREAD; ++i) {
-            const int c = tid + i * NT;
-            *(u32x4*)(&Ws[buf][lds_at(c / CPR, c % CPR)]) = tw[i];   // A is zero there: enough
-        }
+        for (int i = 0; i < W_PER_THREAD; ++i) put(Ws[buf], tid + i * NT, tw[i]);
         // one barrier a tile: whoever writes this buffer again (two tiles on) has passed
         // the next tile's barrier, which every wave reaches only after reading this one
         __syncthreads();
@@ -253,13 +249,13 @@ static int launch_bf16(const bf16_t* A, int lda, const bf16_t* W, int ldw, void*
     const bool vec = lda % 8 == 0 && ldw % 8 == 0 && K % 8 == 0 && ((uintptr_t)A) % 16 == 0 && ((uintptr_t)W) % 16 == 0 &&
                      heads.a % 8 == 0 && heads.w % 8 == 0;
     const GateLaw law{};
-    if (out_dtype == DT_F32) {
-        if (vec) gemm_bf16_kernel<TM, TN, BK, float, true, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (float*)C, ldc, R, ldr, M, N, K, 0, law, heads);
-        else gemm_bf16_kernel<TM, TN, BK, float, false, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (float*)C, ldc, R, ldr, M, N, K, 0, law, heads);
-    } else {
-        if (vec) gemm_bf16_kernel<TM, TN, BK, bf16_t, true, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (bf16_t*)C, ldc, R, ldr, M, N, K, 0, law, heads);
-        else gemm_bf16_kernel<TM, TN, BK, bf16_t, false, false, WM, PF><<<grid, NT, 0, stream>>>(A, lda, W, ldw, (bf16_t*)C, ldc, R, ldr, M, N, K, 0, law, heads);
-    }
+#define GEMM_OF(TC, VEC, TAIL) gemm_bf16_kernel<TM, TN, BK, TC, VEC, TAIL, false, WM, PF><<<grid, NT, 0, stream>>>( \
+        A, lda, W, ldw, (TC*)C, ldc, R, ldr, M, N, K, 0, law, heads)
+#define GEMM_TO(TC) do { if (!vec) GEMM_OF(TC, false, false); else if (K % BK) GEMM_OF(TC, true, true); else GEMM_OF(TC, true, false); } while (0)
+    if (out_dtype == DT_F32) GEMM_TO(float);
+    else GEMM_TO(bf16_t);
+#undef GEMM_TO
+#undef GEMM_OF
     return CISR_LAUNCH_CHECK();
 }
 
@@ -272,7 +268,8 @@ static int launch_bf16_swiglu(const bf16_t* A, int lda, const bf16_t* W, int ldw
     const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN_OUT - 1) / BN_OUT);
     if (tiles > (1ll << 30)) return (int)hipErrorInvalidValue;
     dim3 grid((unsigned)((tiles + 7) / 8 * 8));
-    gemm_bf16_kernel<TM, TN, BK, bf16_t, true, true, WM, PF><<<grid, WM * 128, 0, stream>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, law);
+    if (K % BK) gemm_bf16_kernel<TM, TN, BK, bf16_t, true, true, true, WM, PF><<<grid, WM * 128, 0, stream>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, law);
+    else gemm_bf16_kernel<TM, TN, BK, bf16_t, true, false, true, WM, PF><<<grid, WM * 128, 0, stream>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, law);
     return CISR_LAUNCH_CHECK();
 }
 

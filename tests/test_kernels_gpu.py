@@ -1210,6 +1210,23 @@ def test_gemm_bf16_every_block_tile_alone(ops, tile):
     assert ops.lib().cisr_gemm_bf16_tile(a.data_ptr(), 64, w.data_ptr(), 64, out.data_ptr(), 48, None, 0, 40, 48, 64, 0, 999, stream) != 0
 
 
+@pytest.mark.parametrize("tile", [112, 122, 212, 222, 422, 442])
+@pytest.mark.parametrize("K", [8, 136, 576])
+def test_gemm_bf16_of_infinite_weights(ops, tile, K):
+    """An infinite weight in the last chunk of a row, which loads beyond the inner size repeat: its column is infinite with the sign
+    of the operand, the others are what they are without it."""
+    stream = torch.cuda.current_stream().cuda_stream
+    a, w = rnd(70, K, dtype=torch.bfloat16, seed=1), rnd(90, K, dtype=torch.bfloat16, seed=2)
+    outs = []
+    for _ in range(2):
+        outs.append(torch.empty(70, 90, device=DEV))
+        assert ops.lib().cisr_gemm_bf16_tile(a.data_ptr(), K, w.data_ptr(), K, outs[-1].data_ptr(), 90, None, 0, 70, 90, K, 0, tile, stream) == 0
+        w[5, K - 1] = float("inf")
+    want = outs[0].clone()
+    want[:, 5] = torch.where(a[:, K - 1] > 0, float("inf"), float("-inf"))
+    assert (a[:, K - 1] != 0).all() and torch.equal(outs[1], want)
+
+
 def test_gemm_strided_rows_and_bad_operands(ops):
     from runtime.kernels.ops import KernelError
     big = rnd(9, 50, dtype=torch.bfloat16)
