@@ -14,7 +14,8 @@
 // channel whose decays vanish within a chunk costs neither range nor precision.  A first kernel makes, chunk by chunk and
 // all side by side, what does not need the state: M V, M Kg, D q, P, D(15, i) k and D(15); a second walks a segment's chunks
 // in order, a block a (head, 16 columns of S): its waves own the rows of S in turn, two products with S0 (one without DELTA),
-// one meeting through LDS, one product into S.  Rows behind a segment's end count as k = q = v = 0 with decays of one.
+// one meeting through LDS, one product into S.  Rows behind a segment's end count as k = q = v = 0 with decays of one.  A row
+// does not see the rows behind it, whatever they hold: where a write is not finite, scores and writes are summed row by row.
 // The operands lie in memory as the walk's lanes want them, 16 bytes a lane side by side: read in rows of the chunk instead,
 // each load of the walk touches four times the lines.
 // Measured on an MI355X, us of both kernels (in brackets the scans that walk row by row): 2,048 rows of one request, the delta
@@ -331,6 +332,21 @@ __global__ void __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))
             f32x4_t own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < 4; ++i) own = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[i], u[i], own, 0, 0, 0);
+            if (__builtin_expect(__any((own[0] * 0.f + own[1] * 0.f) + (own[2] * 0.f + own[3] * 0.f) != 0.f), 0)) {
+                // a write that is no finite number, times the zeros of P, reaches the rows before it: once more, row by row
+                own = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {        // slot 4 b + j, row 4 j + b of the chunk
+                        const float write = __shfl(u[j], 16 * b + m, WAVE);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float score = __shfl(pr[j], 16 * b + 4 * kg + i, WAVE);
+                            if (4 * j + b <= 4 * i + kg) own[i] += score * write;
+                        }
+                    }
+            }
             const f32x4_t y = ((share_o[par][0][lane] + share_o[par][1][lane]) + (share_o[par][2][lane] + share_o[par][3][lane])) + own;
             const int row = t0 + (slot - base) * CHUNK + kg;
 #pragma unroll

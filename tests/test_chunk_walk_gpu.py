@@ -108,6 +108,40 @@ def test_chunks_are_no_further_from_64_bits_than_the_walk_row_by_row(law, heads,
     assert out <= rows_out and state <= 1.1 * rows_state, errors
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("is_delta, vec", [(True, False), (True, True), (False, False), (False, True)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_rows_do_not_see_what_is_not_finite_behind_them(is_delta, vec, value):
+    """A value, key, query or decay of row 22 (in the middle of a chunk) that is no finite number: the rows before it are what they
+    are without it, and so are the other columns where a value holds it."""
+    from runtime.kernels import ops
+    T, heads, R, C = 40, 2, 32, 32
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    draw = lambda *shape: torch.randn(*shape, device=DEV, generator=gen)
+    q, k, v = draw(T, heads * R) / 6, draw(T, heads * R) / 6, draw(T, heads * C)
+    g, b = 0.9 + 0.1 * torch.rand(T, heads * R if vec else heads, device=DEV, generator=gen), draw(T, heads)
+    begun = draw(1, heads * R * C)
+
+    def run(q, k, v, g):
+        state, out = begun.clone(), torch.empty(T, heads * C, device=DEV)
+        work = torch.empty(ops.channel_chunk_work(T, 1, heads, R, C, delta=is_delta), device=DEV)
+        where = (out, state, ints([0, T]), ints([0]), heads, R, C, work)
+        if is_delta:
+            ops.channel_delta_chunks(q, k, v, g, b, *where)
+        else:
+            ops.linear_chunks(q, k, v, g, *where)
+        return out
+
+    want = run(q, k, v, g)
+    for which in range(4):
+        operands = [q.clone(), k.clone(), v.clone(), g.clone()]
+        operands[which][22, 0] = value
+        got = run(*operands)
+        assert (got[:22] - want[:22]).abs().max().item() < 1e-5 * want.abs().max().item(), which
+        if which == 2:
+            assert (got[:, 1:] - want[:, 1:]).abs().max().item() < 1e-5 * want.abs().max().item() and not got[22, 0].isfinite()
+
+
 def test_the_oracle_is_the_designs_recurrence():
     """The loop above is the designs' plain recurrences (from a state of zero, for one head)."""
     rng = np.random.default_rng(1)
