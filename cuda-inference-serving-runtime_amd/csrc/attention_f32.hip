@@ -8,11 +8,13 @@
 // 4 g + 3, g = lane / 16, which is what the second product wants as its left operand: the weights go from one instruction to
 // the other in the registers where they are.  Both products take their inner index as 4 g + e of a sixteen, so keys (a row of
 // the page) and values (transposed in the page) are 16-byte loads; the next step's are in flight while this one is computed.
+// An item does not see what it must not, whatever that holds: a wave whose result is not finite makes it again item by item.
 // Bound by the two matrix products and a chain of one trip to memory a step and wave.
 //
 // Measured on an MI355X, 9 heads of 64 over 3: 130 rows at 128 to 350 keys beside two decoding rows 79 us with a wave a (row,
 // head), lanes along the keys, each lane walking a key of its own -> 12.3; two rows at 350 keys 28 + 5 (two splits, merge) -> 13.0.
 #include "common.h"
+#include <type_traits>
 
 #define AF_WAVES 8
 
@@ -29,6 +31,12 @@ struct AttnF32Args {
     float scale;
     int splits;
 };
+
+// What a wave wrote to LDS before is there for its own lanes after.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // DT sixteens of a head's coordinates
 template <int DT>
@@ -52,12 +60,12 @@ attn_f32_kernel(AttnF32Args p) {
     const int begin = first + blockIdx.z * share, stop = min(begin + share, first + steps);
     const int P = 1 << p.page_shift;
     const int* table = p.tables + (size_t)seg * p.width;
-    af_f32x4 fq[DT];
-    {
+    af_f32x4 fq[DT];                                                  // (a wave without a step does not wait for it)
+    auto ask_q = [&]() __attribute__((always_inline)) {
         const float* qr = p.q + (size_t)row_of(r) * p.q_row_stride + (size_t)head_of(r) * D + 4 * g;
 #pragma unroll
         for (int c = 0; c < DT; ++c) fq[c] = *(const af_f32x4*)(qr + 16 * c);
-    }
+    };
     af_f32x4 o[DT];
 #pragma unroll
     for (int c = 0; c < DT; ++c) o[c] = (af_f32x4){0.f, 0.f, 0.f, 0.f};
@@ -69,7 +77,7 @@ attn_f32_kernel(AttnF32Args p) {
         pk = table[key_of(s * 16 + r) >> p.page_shift];
         pv = table[key_of(s * 16 + 4 * g) >> p.page_shift];
     };
-    auto ask = [&](int s, int pk, int pv, af_f32x4 (&fk)[DT], af_f32x4 (&fv)[DT]) {
+    auto ask = [&](int s, int pk, int pv, af_f32x4 (&fk)[DT], af_f32x4 (&fv)[DT]) __attribute__((always_inline)) {
         const int tk = key_of(s * 16 + r), tv = key_of(s * 16 + 4 * g) & ~3;      // (pages of whole fours)
         const float* kr = p.kcache + (((size_t)pk * p.kv_heads + kvh) * P + (tk & (P - 1))) * D + 4 * g;
         const float* vr = p.vcache + (((size_t)pv * p.kv_heads + kvh) * D + r) * P + (tv & (P - 1));
@@ -78,7 +86,8 @@ attn_f32_kernel(AttnF32Args p) {
 #pragma unroll
         for (int c = 0; c < DT; ++c) fv[c] = *(const af_f32x4*)(vr + (size_t)16 * c * P);
     };
-    auto use = [&](int s, af_f32x4 (&fk)[DT], af_f32x4 (&fv)[DT]) {
+    // careful: the second product item by item over the keys that it sees
+    auto use = [&](int s, af_f32x4 (&fk)[DT], af_f32x4 (&fv)[DT], auto careful) __attribute__((always_inline)) {
         // (a sum for every second sixteen of coordinates: half the chain of instructions, and of roundings)
         af_f32x4 sc = {0.f, 0.f, 0.f, 0.f}, odd = sc;
 #pragma unroll
@@ -125,15 +134,41 @@ attn_f32_kernel(AttnF32Args p) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) fv[c][e] = s * 16 + 4 * g + e < end ? fv[c][e] : 0.f;
         }
+        if constexpr (!decltype(careful)::value) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int c = 0; c < DT; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[e], fv[c][e], o[c], 0, 0, 0);
+                for (int c = 0; c < DT; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[e], fv[c][e], o[c], 0, 0, 0);
+        } else {
+            // (through LDS, where the wave's result goes at the end: weights by item, -1 for none; values by key, a sixteen at a time)
+            float* weights = &so[wave][0][0];
+            float* values = weights + 256;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = s * 16 + 4 * g + e;
+                weights[r * 16 + 4 * g + e] = t <= pos && (p.window <= 0 || t > pos - p.window) ? sc[e] : -1.f;
+            }
+#pragma unroll
+            for (int c = 0; c < DT; ++c) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) values[(4 * g + e) * 16 + r] = fv[c][e];
+                wave_order();
+#pragma unroll 1
+                for (int t = 0; t < 16; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float weight = weights[(4 * g + e) * 16 + t];
+                        if (!(weight < 0.f)) o[c][e] += weight * values[t * 16 + r];
+                    }
+                wave_order();
+            }
+        }
     };
     af_f32x4 ka[DT], va[DT], kb[DT], vb[DT];
     int s = begin + wave, pk = 0, pv = 0;
     if (s < stop) {
         ask_pages(s, pk, pv);
+        ask_q();
         ask(s, pk, pv, ka, va);
         ask_pages(min(s + AF_WAVES, stop - 1), pk, pv);
     }
@@ -143,13 +178,30 @@ attn_f32_kernel(AttnF32Args p) {
             ask(s + AF_WAVES, pk, pv, kb, vb);
             ask_pages(min(s + 2 * AF_WAVES, stop - 1), pk, pv);
         }
-        use(s, ka, va);
+        use(s, ka, va, std::false_type{});
         if (!more) break;
         if (s + 2 * AF_WAVES < stop) {
             ask(s + 2 * AF_WAVES, pk, pv, ka, va);
             ask_pages(min(s + 3 * AF_WAVES, stop - 1), pk, pv);
         }
-        use(s + AF_WAVES, kb, vb);
+        use(s + AF_WAVES, kb, vb, std::false_type{});
+    }
+    // A value that is not finite, times the zero weight of an item that does not see its key, is no number: then once more, with care
+    af_f32x4 finite = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < DT; ++c) finite += o[c] * 0.f;
+    if (__builtin_expect(__any((finite.x + finite.y) + (finite.z + finite.w) != 0.f), 0)) {
+#pragma unroll
+        for (int c = 0; c < DT; ++c) o[c] = (af_f32x4){0.f, 0.f, 0.f, 0.f};
+        m = -INFINITY;
+        l = 0.f;
+        ask_q();
+#pragma unroll 1
+        for (int t = begin + wave; t < stop; t += AF_WAVES) {
+            ask_pages(t, pk, pv);
+            ask(t, pk, pv, ka, va);
+            use(t, ka, va, std::true_type{});
+        }
     }
     l += __shfl_xor(l, 16, WAVE);
     l += __shfl_xor(l, 32, WAVE);

@@ -87,3 +87,25 @@ def test_no_further_from_64_bits_than_the_row_wise_kernel(heads, kv_heads, dim):
             ops.attention_rowwise(flat, heads * dim, kt, vt, tables, ints([s for s, _ in rows]), pos, *args)
         errors.append(np.linalg.norm(f64(out).reshape(want.shape) - want) / np.linalg.norm(want))
     assert errors[1] <= errors[0], errors
+
+
+@pytest.mark.parametrize("window", [None, 6])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_rows_do_not_see_what_is_not_finite_where_they_do_not_look(window, value):
+    """Rows 30 to 45 of a prompt, sixteen a tile, and a value of key 36 that is no finite number: the rows that do not see that key
+    are what they are without it, and so are the other coordinates."""
+    from runtime.kernels import ops
+    heads, dim, page = 2, 32, 16
+    _, kt, vt, tables, _ = paged_case(heads, heads, dim, page, [46], torch.float32, seed=1)
+    pos = torch.arange(30, 46, dtype=torch.int32, device=DEV)
+    q = rnd(16, heads * dim, seed=2)
+    tasks, outs = torch.tensor([(0, 0, 16, 0)], dtype=torch.int32, device=DEV), []
+    for _ in range(2):
+        outs.append(torch.empty(16, heads * dim, device=DEV))
+        ops.attention_f32(q, heads * dim, kt, vt, tables, pos, tasks, outs[-1], heads, heads, dim, page, window, dim ** -0.5)
+        vt[tables[0, 2], 1, 3, 36 - 32] = value
+    want, got = outs
+    sees = (pos >= 36) & (pos - 36 < (window or 99))
+    assert (got[~sees] - want[~sees]).abs().max().item() < 1e-5 and not got[sees, dim + 3].isfinite().any()
+    other = torch.arange(heads * dim, device=DEV) != dim + 3
+    assert (got[:, other] - want[:, other]).abs().max().item() < 1e-5
