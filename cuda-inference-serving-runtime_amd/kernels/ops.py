@@ -2278,8 +2278,8 @@ def experts_gemm(a, w, pair_of_pos, tile_expert, out, top=0, scatter=False, act=
     experts, n, k = w.shape
     tiles = tile_expert.shape[0]
     places = tiles * EXPERT_TILE
-    if a.dtype != w.dtype or a.dim() != 2 or a.shape[1] != k or a.stride(1) != 1 or not w.is_contiguous():
-        raise KernelError("experts_gemm: operands of one dtype, [rows, K] against [experts, N, K]")
+    if not a.is_cuda or a.dtype != w.dtype or a.dim() != 2 or a.shape[1] != k or a.stride(1) != 1 or not w.is_contiguous():
+        raise KernelError("experts_gemm: GPU operands of one dtype, [rows, K] against [experts, N, K]")
     if out.dim() != 2 or out.shape[1] != n or not out.is_contiguous() or (a.dtype == torch.float32 and out.dtype != torch.float32):
         raise KernelError("experts_gemm: out is [rows, N], float for float operands")
     if pair_of_pos.numel() != places:
@@ -2306,7 +2306,7 @@ def experts_gemm_gated(a, w, pair_of_pos, tile_expert, out, law, top=0):
     experts, n2, k = w.shape
     tiles = tile_expert.shape[0]
     places = tiles * EXPERT_TILE
-    if not experts_gemm_gated_ok(a, w) or a.dim() != 2 or a.shape[1] != k or n2 % 2 or not w.is_contiguous() or pair_of_pos.numel() != places:
+    if not a.is_cuda or not experts_gemm_gated_ok(a, w) or a.dim() != 2 or a.shape[1] != k or n2 % 2 or not w.is_contiguous() or pair_of_pos.numel() != places:
         raise KernelError("experts_gemm_gated: shape not supported")
     if out.dim() != 2 or out.shape[1] != n2 // 2 or out.shape[0] < places or (top <= 0 and a.shape[0] < places):
         raise KernelError("experts_gemm_gated: operands and results by place need a row a place")

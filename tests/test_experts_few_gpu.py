@@ -91,3 +91,16 @@ def test_gated_norm_with_its_row_in_registers(dim):
     v = (share[:, :2, None].double() * y[:, :2].double()).sum(1) * torch.sigmoid(g.double() + gb.double()) + 2.0 * x.double()
     want = v * torch.rsqrt(v.square().mean(1, keepdim=True) + 1e-5) * w.double()
     assert ((got[0][0] - want).abs().max() / want.abs().max()).item() < 1e-5
+
+
+def test_operands_on_the_host_are_refused():
+    from runtime.kernels import ops
+    w = torch.zeros(16, 16, 64, device=DEV, dtype=torch.bfloat16)
+    tiles = ops.expert_tiles(2, 1, 16)
+    pp, te = torch.full((tiles * 64,), -1, dtype=torch.int32, device=DEV), torch.full((tiles,), -1, dtype=torch.int32, device=DEV)
+    a, out = torch.zeros(2, 64, dtype=torch.bfloat16), torch.zeros(tiles * 64, 16, device=DEV, dtype=torch.bfloat16)
+    assert ops.experts_few_ok(a, w, tiles)
+    with pytest.raises(ops.KernelError):
+        ops.experts_gemm(a, w, pp, te, out, top=1)
+    with pytest.raises(ops.KernelError):
+        ops.experts_gemm_gated(a, w, pp, te, out[:, :8].contiguous(), (7.0, 1.0, 0.0), top=1)
