@@ -8,6 +8,7 @@ graph.  Nothing here computes on the CPU.  One kind of call leaves the kernels o
 products of more than 64 rows, which go to the vendor's library through torch.mm (see library_ok).
 """
 import ctypes as C
+import operator
 
 import torch
 
@@ -315,10 +316,17 @@ def rope_scatter(qkv, positions, slots, cos, sin, kcache, vcache, heads, kv_head
                                    int(bool(interleaved)), dt, _stream()), "rope_scatter")
 
 
+def _page_numbers(pages, name):
+    if isinstance(pages, torch.Tensor):
+        _dev(pages, name, torch.int32, (pages.numel(),))
+        return pages.tolist()
+    return [operator.index(x) for x in pages]
+
+
 def page_copy(pool, src, dst, slabs, pages_per_slab):
     """pool viewed as [slabs, pages_per_slab, page]: page dst[i] := page src[i] in every slab.  src, dst: page numbers
     (sequences, or tensors, which are read back first); no page is both a source and a destination."""
-    src, dst = ([int(x) for x in (t.tolist() if isinstance(t, torch.Tensor) else t)] for t in (src, dst))
+    src, dst = (_page_numbers(t, name) for t, name in ((src, "src"), (dst, "dst")))
     n = len(src)
     total = pool.numel() * pool.element_size()
     if total % (slabs * pages_per_slab):

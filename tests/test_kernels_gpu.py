@@ -1358,6 +1358,16 @@ def test_page_copies_of_a_step_in_one_call(ops, slabs, pages, words, pairs):
         ops.page_copy(pool, [0], [pages], slabs, pages)
 
 
+def test_page_numbers_are_whole(ops):
+    pool = torch.zeros(2, 4, 8, dtype=torch.int32, device=DEV)
+    one, two = (torch.tensor([n], dtype=torch.int32, device=DEV) for n in (1, 2))
+    for bad in (one.float(), one.long(), one.cpu(), one[None].repeat(1, 2)):
+        with pytest.raises(ops.KernelError):
+            ops.page_copy(pool, bad, two, 2, 4)
+    with pytest.raises(TypeError):
+        ops.page_copy(pool, [1.5], [2], 2, 4)
+
+
 def test_kernels_refuse_what_they_cannot_take(ops):
     from runtime.kernels.ops import KernelError
     with pytest.raises(KernelError, match="head size"):
