@@ -47,50 +47,80 @@ def _float(t):
 
 
 @dataclass(frozen=True)
-class DeltaByChunks:
-    """Whether a step's delta rule of `heads` heads is walked chunk by chunk (launch value 1) or row by row (0): a step array
-    (engine.context.StepArray) without words.  Row by row a step lasts as long as its longest portion or, with many heads
-    and segments, as its rows take all together; chunk by chunk as its chunks take to prepare and walk.  Measured on an
-    MI355X at 32 and 16 heads of 128 x 128 (row by row / by chunks, us; the constants below are fits): one portion of 48
-    rows 26 / 24 and 24 / 23, of 128 58 / 28 and 55 / 27, of 2,048 840 / 180 and 787 / 144; eight of 32 37 / 57 and 26 / 39,
-    of 256 216 / 190 and 145 / 102; 32 of 64 164 / 264 and 88 / 129."""
+class ByChunks:
+    """Whether a step's recurrence of `heads` heads of `rows` x `cols` is walked chunk by chunk (launch value 1) or row by row
+    (0): a step array (engine.context.StepArray) without words.  Row by row a step lasts as long as its longest portion or, with
+    many heads and segments, as its rows take all together; chunk by chunk as its chunks take to prepare and walk, and a
+    segment of one row is a chunk of sixteen.  So a portion alone goes by chunks, a few dozen rows beside as many single ones
+    do not.  The rule: by chunks if
+
+        longest (chain + chain_rows rows / 128) + work heads rows cols (all rows) / 10^6 > 10 + operands heads chunks words / 1000
+
+    (`words`: floats of a channel's and a column's operands), fitted to 38 batches at 16 sizes on an MI355X, a portion of 32 rows or more
+    in each: it picks the slower form by more than 5 % in 7 of 608, by 13 % at worst.  Row by row / by chunks, us:
+
+                                            1 x 48    1 x 2,048   8 x 32   8 x 256    24 x 1 + 64   64 x 1 + 64   64 x 1 + 512
+      delta rule, 32 heads of 128 x 128     26 / 18   840 / 175   37 / 53  222 / 185  83 / 114      103 / 267     488 / 307
+      delta rule, 16 heads of 128 x 128     24 / 18   788 / 146   25 / 33  144 / 99   63 / 66       81 / 146      435 / 172
+      a decay a channel, 8 of 128 x 256     38 / 22   1401 / 107  37 / 33  244 / 84   76 / 60       101 / 123     492 / 140
+      a decay a head, 64 of 128 x 64        40 / 15   1392 / 161  44 / 48  274 / 197  91 / 100      130 / 235     532 / 280
+      a decay a head, 16 of 64 x 129        32 / 12   1178 / 83   31 / 23  212 / 70   58 / 40       71 / 87       402 / 100
+    """
     heads: int
+    rows: int = 128
+    cols: int = 128
+
+    LEAST = 32                # rows of a step's longest portion, at least (fewer were not measured)
+
+    def law(self):
+        """(chain, chain_rows, work, operands, words)"""
+        raise NotImplementedError
 
     def words(self, rows, segments):
         return 0
 
     def launch_value(self, batch):
-        if batch.decode_only:
+        if batch.decode_only or max(batch.counts) < self.LEAST:
             return 0
-        longest, chunks = max(batch.counts), sum(-(-n // ops.CHUNK_ROWS) for n in batch.counts)
-        by_rows = max(8 + 0.41 * longest, 0.0028 * self.heads * sum(batch.counts))
-        return int(20 + max(0.042 * self.heads * chunks, longest / 16) < by_rows)
+        chain, chain_rows, work, operands, words = self.law()
+        chunks = sum(-(-n // ops.CHUNK_ROWS) for n in batch.counts)
+        by_rows = max(batch.counts) * (chain + chain_rows * self.rows / 128) + work * self.heads * self.rows * self.cols * sum(batch.counts) / 1e6
+        return int(by_rows > 10 + operands * self.heads * chunks * words / 1e3)
 
     def fill(self, out, batch, value):
         pass
 
 
+@dataclass(frozen=True)
+class DeltaByChunks(ByChunks):
+    """ByChunks of the delta rule with a decay a head."""
+
+    def law(self):
+        return 0.18, 0.228, 0.145, 0.101, 3 * self.rows + self.cols
+
+
+@dataclass(frozen=True)
+class LinearByChunks(ByChunks):
+    """ByChunks of the linear scan; `vector`: a decay a channel, else one a head."""
+    vector: bool = False
+
+    def law(self):
+        return (0.55, 0.0, 0.234, 0.185, 2 * self.rows + self.cols) if self.vector else (0.2, 1.66, 0.56, 0.305, 2 * self.rows + self.cols)
+
+
 def _chunk_work(ctx, rows, heads, state_rows, state_cols, delta):
-    """What a walk by chunks keeps between its two kernels: scratch memory of the runner, one buffer for every program and layer."""
+    """What a walk by chunks keeps between its two kernels: scratch memory of the runner, one buffer for every program and layer
+    (of the step's largest mixer, 160 chunks at most, in a power of two: 256 MB at 64 heads of 128 x 64 or 32 of 128 x 128)."""
     return ctx.scratch.get("chunks", ops.channel_chunk_work(rows.shape[0], ctx.n_segments, heads, state_rows, state_cols, delta=delta),
                            torch.float32, rows.device)
 
 
-def _scan(ctx, tag, q, k, v, decay, out, state, heads, rows, cols, silu=False, step=None, **kw):
-    """ops.linear_scan over the step's segments: portions chunk by chunk on the matrix cores (at every size measured, one
-    portion of 33 rows to 32 of 64 and one of 4,096, faster than row by row: `ops.linear_chunks`), else row by row, where the
-    segments of a step with long portions are walked in pieces."""
-    T = v.shape[0]
-    if not silu and ops.channel_chunked(T, ctx.n_segments, ctx.decode_only):
-        work = _chunk_work(ctx, v, heads, rows, cols, False)
-        return ops.linear_chunks(q, k, v, decay, out, state, ctx.seg_start, ctx.state_slots, heads, rows, cols, work, step=step, **kw)
-    piece = ops.scan_piece(T, ctx.decode_only)
-    carry = None
-    if piece:
-        n, n_decay = ops.scan_carry(T, piece, heads, rows, cols, decay.shape[1] != heads)
-        carry = (ctx.buffer(tag + ".carry", (n,), torch.float32), ctx.buffer(tag + ".carry_decay", (n_decay,), torch.float32))
-    return ops.linear_scan(q, k, v, decay, out, state, ctx.seg_start, ctx.state_slots, heads, rows, cols, piece=piece, carry=carry,
-                           silu=silu, step=step, **kw)
+def _scan(ctx, by_chunks, q, k, v, decay, out, state, heads, rows, cols, **kw):
+    """ops.linear_scan over the step's segments, row by row or (`by_chunks`, a LinearByChunks) chunk by chunk on the matrix cores."""
+    where = (out, state, ctx.seg_start, ctx.state_slots, heads, rows, cols)
+    if ctx.step_array(by_chunks)[1]:
+        return ops.linear_chunks(q, k, v, decay, *where, _chunk_work(ctx, v, heads, rows, cols, False), **kw)
+    return ops.linear_scan(q, k, v, decay, *where, **kw)
 
 
 class GatedLinearAttention(Mixer):
@@ -103,6 +133,10 @@ class GatedLinearAttention(Mixer):
         self.name, self.hidden, self.heads, self.dim, self.vdim = name, hidden, heads, dim, vdim
         self.tau, self.eps, self.rank = float(tau), float(eps), int(rank)
         self.names = {**self.NAMES, **(names or {})}
+        self.by_chunks = LinearByChunks(heads, dim, vdim, vector=True)
+
+    def step_arrays(self):
+        return [self.by_chunks]
 
     def _tensor(self, which):
         return f"{self.name}.{self.names[which]}"
@@ -141,7 +175,7 @@ class GatedLinearAttention(Mixer):
         decay = ops.decay_gate_low_rank(proj[:, 2 * K + 2 * V:], self.w_up, self.bias, ctx.buffer("gla.decay", (T, K), torch.float32), self.tau)
         state = ctx.cache.state_storage[site]
         o = ctx.buffer("gla.o", (T, V), torch.float32)
-        _scan(ctx, "gla", proj[:, :K], proj[:, K:2 * K], proj[:, 2 * K:2 * K + V], decay, o, state.view(state.shape[0], -1),
+        _scan(ctx, self.by_chunks, proj[:, :K], proj[:, K:2 * K], proj[:, 2 * K:2 * K + V], decay, o, state.view(state.shape[0], -1),
               self.heads, self.dim, self.vdim, q_scale=self.dim ** -0.5)
         act = ops.group_norm_gate(o, proj[:, 2 * K + V:2 * K + 2 * V], self.norm_weight, ctx.buffer("gla.act", (T, V), ctx.dtype),
                                   self.heads, self.eps, gate_first=False, shared_weight=True)
@@ -210,7 +244,12 @@ class LightningAttention(Mixer):
         q, k, v, sizes = proj[:, :K], proj[:, K:2 * K], proj[:, 2 * K:2 * K + V], (self.heads, self.dim, self.vdim)
         form = ops.lightning_form(q, v, o, state, T, ctx.n_segments, ctx.decode_only, self.vdim)
         if form == "scan":
-            _scan(ctx, "la", q, k, v, self.decay_row.expand(T, self.heads), o, state, *sizes, silu=True)
+            # (short portions and single rows; a long one among them is walked in pieces)
+            decay, piece, carry = self.decay_row.expand(T, self.heads), ops.scan_piece(T, ctx.decode_only), None
+            if piece:
+                carry = tuple(ctx.buffer("la.carry" + name, (n,), torch.float32)
+                              for name, n in zip(("", "_decay"), ops.scan_carry(T, piece, *sizes, False)))
+            ops.linear_scan(q, k, v, decay, o, state, ctx.seg_start, ctx.state_slots, *sizes, piece=piece, carry=carry, silu=True)
         else:
             carry = None
             if form == "chunks":
@@ -242,6 +281,10 @@ class StateSpaceDuality(Mixer):
         self.inner = heads * vdim
         self.channels = self.inner + 2 * groups * state          # what the convolution runs over: x, B, C
         self.names = {**self.NAMES, **(names or {})}
+        self.by_chunks = LinearByChunks(heads, state, vdim)
+
+    def step_arrays(self):
+        return [self.by_chunks]
 
     def _tensor(self, which):
         return f"{self.name}.{self.names[which]}"
@@ -280,7 +323,7 @@ class StateSpaceDuality(Mixer):
                       ctx.seg_start, ctx.state_slots, gates=(proj[:, inner + ch:], self.dt_bias, self.a_log, step, decay),
                       single_rows=ctx.decode_only)
         y = ctx.buffer("ssd.o", (T, inner), torch.float32)
-        _scan(ctx, "ssd", xbc[:, inner + GN:], xbc[:, inner:inner + GN], xbc[:, :inner], decay, y, state,
+        _scan(ctx, self.by_chunks, xbc[:, inner + GN:], xbc[:, inner:inner + GN], xbc[:, :inner], decay, y, state,
               nh, self.state, self.vdim, share=nh // self.groups, step=step)
         act = ops.group_norm_gate(y, proj[:, :inner], self.norm_weight, ctx.buffer("ssd.act", (T, inner), ctx.dtype),
                                   self.norm_groups, self.eps, gate_first=True, skip=(self.skip, xbc[:, :inner]))
@@ -312,7 +355,7 @@ class GatedDeltaRule(Mixer):
         self.qk, self.inner = kv_heads * dim, heads * vdim
         self.channels = 2 * self.qk + self.inner           # what the convolution runs over: q, k, v
         self.names = {**self.NAMES, **(names or {})}
-        self.by_chunks = DeltaByChunks(heads)
+        self.by_chunks = DeltaByChunks(heads, dim, vdim)
 
     def step_arrays(self):
         return [] if self.by_chunks is None else [self.by_chunks]
@@ -538,6 +581,10 @@ class MatrixMemory(Mixer):
         self.name, self.hidden, self.heads, self.dim, self.vdim = name, hidden, heads, dim, vdim
         self.cap, self.eps, self.floor = float(gate_cap), float(eps), float(floor)
         self.names = {**self.NAMES, **(names or {})}
+        self.by_chunks = LinearByChunks(heads, dim, vdim + 1)
+
+    def step_arrays(self):
+        return [self.by_chunks]
 
     def _tensor(self, which):
         return f"{self.name}.{self.names[which]}"
@@ -585,7 +632,7 @@ class MatrixMemory(Mixer):
         ops.mlstm_gates(proj[:, gates:gates + nh], proj[:, gates + nh:gates + 2 * nh], self.bias_i, self.bias_f, proj[:, 2 * K:2 * K + W],
                         decay, step, top, vx, state[:, K * C:], ctx.seg_start, ctx.state_slots, nh, V, self.cap, single_rows=ctx.decode_only)
         o = ctx.buffer("mm.o", (T, nh * C), torch.float32)
-        _scan(ctx, "mm", proj[:, :K], proj[:, K:2 * K], vx, decay, o, state, nh, R, C, step=step, q_scale=R ** -0.5)
+        _scan(ctx, self.by_chunks, proj[:, :K], proj[:, K:2 * K], vx, decay, o, state, nh, R, C, step=step, q_scale=R ** -0.5)
         act = ops.mlstm_finish(o, top, proj[:, 2 * K + W:2 * K + 2 * W], self.norm_weight, ctx.buffer("mm.act", (T, W), ctx.dtype),
                                nh, V, self.eps, self.floor)
         return ops.gemm(act, self.w_out, ctx.buffer("mm.y", (T, self.hidden), torch.float32), scratch=ctx.scratch)

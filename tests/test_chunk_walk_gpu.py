@@ -156,6 +156,37 @@ def test_the_oracle_is_the_designs_recurrence():
         np.testing.assert_allclose(out, want, rtol=1e-10, atol=1e-12)
 
 
+# row by row, by chunks: us on an MI355X of (portions) at (law, heads, rows, columns of a state)
+BATCHES = [[48], [2048], [32] * 8, [256] * 8, [1] * 24 + [64], [1] * 64 + [64], [1] * 64 + [512]]
+MEASURED = {
+    ("delta", 32, 128, 128): [(26, 18), (840, 175), (37, 53), (222, 185), (83, 114), (103, 267), (488, 307)],
+    ("delta", 16, 128, 128): [(24, 18), (788, 146), (25, 33), (144, 99), (63, 66), (81, 146), (435, 172)],
+    ("channel", 8, 128, 256): [(38, 22), (1401, 107), (37, 33), (244, 84), (76, 60), (101, 123), (492, 140)],
+    ("head", 64, 128, 64): [(40, 15), (1392, 161), (44, 48), (274, 197), (91, 100), (130, 235), (532, 280)],
+    ("head", 16, 64, 129): [(32, 12), (1178, 83), (31, 23), (212, 70), (58, 40), (71, 87), (402, 100)]}
+
+
+@pytest.mark.parametrize("law, heads, R, C", MEASURED)
+def test_the_form_chosen_is_the_faster_one(law, heads, R, C):
+    """Portions alone and beside single rows: what the rule picks takes at most a tenth longer than the other form was measured to."""
+    from runtime.engine.context import Batch
+    from runtime.parts.recurrent import DeltaByChunks, LinearByChunks
+    rule = DeltaByChunks(heads, R, C) if law == "delta" else LinearByChunks(heads, R, C, vector=law == "channel")
+    for counts, times in zip(BATCHES, MEASURED[law, heads, R, C]):
+        picked = rule.launch_value(Batch(counts, [0] * len(counts), None, False, {}))
+        assert times[picked] <= 1.1 * min(times), counts
+    assert rule.launch_value(Batch([1] * 9, [5] * 9, None, True, {})) == rule.launch_value(Batch([2] * 64, [0] * 64, None, False, {})) == 0
+
+
+def test_every_mixer_of_these_laws_names_its_rule():
+    """The rule's answer is part of a captured program's key from the first step on."""
+    from runtime.parts.recurrent import DeltaByChunks, GatedDeltaRule, GatedLinearAttention, LinearByChunks, MatrixMemory, StateSpaceDuality
+    assert GatedDeltaRule("n", 64, 4, 2, 16, 24, 4, 1e-5).step_arrays() == [DeltaByChunks(4, 16, 24)]
+    assert GatedLinearAttention("n", 64, 2, 16, 24, 16.0, 1e-5).step_arrays() == [LinearByChunks(2, 16, 24, vector=True)]
+    assert StateSpaceDuality("n", 64, 4, 16, 24, 2, 4, 1, 1e-5).step_arrays() == [LinearByChunks(4, 24, 16)]
+    assert MatrixMemory("n", 64, 2, 16, 24, 15.0, 1e-5).step_arrays() == [LinearByChunks(2, 16, 25)]
+
+
 def test_which_steps_walk_the_delta_rule_by_chunks():
     from runtime.engine.context import Batch
     from runtime.parts.recurrent import DeltaByChunks
