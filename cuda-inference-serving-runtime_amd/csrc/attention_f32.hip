@@ -1,7 +1,7 @@
 // Softmax attention over the paged cache for the 32-bit path, on the float matrix instruction (v_mfma_f32_16x16x4_f32: whole
 // floats in, float sums).  A block is one tile of up to 16 items (rows of one segment times the query heads that share a
-// key head) and a split of its keys; its eight waves take the 16-key steps in turn, each with a running maximum, sum and
-// result of its own, which meet in LDS at the end.  Several splits leave partial results for the merge of
+// key head) and a split of its keys; its waves (eight, or two or four) take the 16-key steps in turn, each with a
+// running maximum, sum and result of its own, which meet in LDS at the end.  Several splits leave partial results for the merge of
 // csrc/attention_rowwise.hip.
 //
 // A step is S^T = K Q^T and O += P V.  With S^T a lane holds the scores of one item (column lane % 16) against the keys 4 g ..
@@ -13,10 +13,11 @@
 //
 // Measured on an MI355X, 9 heads of 64 over 3: 130 rows at 128 to 350 keys beside two decoding rows 79 us with a wave a (row,
 // head), lanes along the keys, each lane walking a key of its own -> 12.3; two rows at 350 keys 28 + 5 (two splits, merge) -> 13.0.
+// Where many blocks have short contexts a block has two or four waves (kernels.attention.f32_waves).
 #include "common.h"
 #include <type_traits>
 
-#define AF_WAVES 8
+#define AF_WAVES 8                      // at most
 
 typedef __attribute__((ext_vector_type(4))) float af_f32x4;
 
@@ -38,12 +39,12 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// DT sixteens of a head's coordinates
-template <int DT>
-__global__ void __launch_bounds__(AF_WAVES * WAVE)
+// DT sixteens of a head's coordinates, W waves
+template <int DT, int W>
+__global__ void __launch_bounds__(W * WAVE)
 attn_f32_kernel(AttnF32Args p) {
     constexpr int D = 16 * DT;
-    __shared__ float so[AF_WAVES][16][D + 4], sm[AF_WAVES][16], sl[AF_WAVES][16];
+    __shared__ float so[W][16][D + 4], sm[W][16], sl[W][16];
     const int seg = p.tasks[4 * blockIdx.x], row0 = p.tasks[4 * blockIdx.x + 1], n_rows = p.tasks[4 * blockIdx.x + 2];
     if (seg < 0 || n_rows <= 0) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, r = lane % 16, g = lane / 16;
@@ -174,21 +175,21 @@ attn_f32_kernel(AttnF32Args p) {
         ask_pages(s, pk, pv);
         ask_q();
         ask(s, pk, pv, ka, va);
-        ask_pages(min(s + AF_WAVES, stop - 1), pk, pv);
+        ask_pages(min(s + W, stop - 1), pk, pv);
     }
-    for (; s < stop; s += 2 * AF_WAVES) {
-        const bool more = s + AF_WAVES < stop;                        // (uniform over the wave)
+    for (; s < stop; s += 2 * W) {
+        const bool more = s + W < stop;                        // (uniform over the wave)
         if (more) {
-            ask(s + AF_WAVES, pk, pv, kb, vb);
-            ask_pages(min(s + 2 * AF_WAVES, stop - 1), pk, pv);
+            ask(s + W, pk, pv, kb, vb);
+            ask_pages(min(s + 2 * W, stop - 1), pk, pv);
         }
         use(s, ka, va, std::false_type{});
         if (!more) break;
-        if (s + 2 * AF_WAVES < stop) {
-            ask(s + 2 * AF_WAVES, pk, pv, ka, va);
-            ask_pages(min(s + 3 * AF_WAVES, stop - 1), pk, pv);
+        if (s + 2 * W < stop) {
+            ask(s + 2 * W, pk, pv, ka, va);
+            ask_pages(min(s + 3 * W, stop - 1), pk, pv);
         }
-        use(s + AF_WAVES, kb, vb, std::false_type{});
+        use(s + W, kb, vb, std::false_type{});
     }
     // A value that is not finite, times the zero weight of an item that does not see its key, is no number: then once more, with care
     af_f32x4 finite = {0.f, 0.f, 0.f, 0.f};
@@ -201,7 +202,7 @@ attn_f32_kernel(AttnF32Args p) {
         l = 0.f;
         ask_q();
 #pragma unroll 1
-        for (int t = begin + wave; t < stop; t += AF_WAVES) {
+        for (int t = begin + wave; t < stop; t += W) {
             ask_pages(t, pk, pv);
             ask(t, pk, pv, ka, va);
             use(t, ka, va, std::true_type{});
@@ -215,14 +216,14 @@ attn_f32_kernel(AttnF32Args p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) so[wave][4 * g + e][16 * c + r] = o[c][e];
     __syncthreads();
-    for (int idx = tid; idx < 16 * D; idx += AF_WAVES * WAVE) {
+    for (int idx = tid; idx < 16 * D; idx += W * WAVE) {
         const int i = idx / D, d = idx % D;
         if (!live(i)) continue;
         float best = -INFINITY, den = 0.f, num = 0.f;
 #pragma unroll
-        for (int w = 0; w < AF_WAVES; ++w) best = fmaxf(best, sm[w][i]);
+        for (int w = 0; w < W; ++w) best = fmaxf(best, sm[w][i]);
 #pragma unroll
-        for (int w = 0; w < AF_WAVES; ++w) {                          // in the order of the waves
+        for (int w = 0; w < W; ++w) {                          // in the order of the waves
             const float f = sm[w][i] == -INFINITY ? 0.f : expf(sm[w][i] - best);
             den += f * sl[w][i];
             num += f * so[w][i][d];
@@ -248,9 +249,10 @@ extern "C" int cisr_attn_f32_ok(int dim, int page_size) {
 // splits, 2] receive what attn_merge_kernel (natural logarithms) takes: rows that no task names are left alone.
 extern "C" int cisr_attn_f32(const float* q, int q_row_stride, const float* kcache, const float* vcache, const int* tables,
                              const int* positions, const int* tasks, int n_tasks, float* out, float* part_o, float* part_ml, int heads,
-                             int kv_heads, int dim, int page_size, int width, int window, float scale, int splits, hipStream_t stream) {
+                             int kv_heads, int dim, int page_size, int width, int window, float scale, int splits, int waves,
+                             hipStream_t stream) {
     if (n_tasks <= 0) return 0;
-    if (!cisr_attn_f32_ok(dim, page_size) || kv_heads <= 0 || heads % kv_heads || splits < 1 || splits > 65535 || q_row_stride % 4 ||
+    if (!cisr_attn_f32_ok(dim, page_size) || kv_heads <= 0 || heads % kv_heads || splits < 1 || splits > 65535 || q_row_stride % 4 || (waves != 2 && waves != 4 && waves != AF_WAVES) ||
         ((uintptr_t)q) % 16 || ((uintptr_t)kcache) % 16 || ((uintptr_t)vcache) % 16 || (splits > 1 && (!part_o || !part_ml)))
         return (int)hipErrorInvalidValue;
     const int group = heads / kv_heads, per_chunk = group < 16 ? group : 16, chunks = (group + per_chunk - 1) / per_chunk;
@@ -260,9 +262,15 @@ extern "C" int cisr_attn_f32(const float* q, int q_row_stride, const float* kcac
     const AttnF32Args p{q, q_row_stride, kcache, vcache, tables, positions, tasks, out, part_o, part_ml, heads, kv_heads, per_chunk, chunks,
                         shift, width, window, scale, splits};
     const dim3 grid(n_tasks, kv_heads * chunks, splits);
-    if (dim == 32) attn_f32_kernel<2><<<grid, AF_WAVES * WAVE, 0, stream>>>(p);
-    else if (dim == 64) attn_f32_kernel<4><<<grid, AF_WAVES * WAVE, 0, stream>>>(p);
-    else if (dim == 96) attn_f32_kernel<6><<<grid, AF_WAVES * WAVE, 0, stream>>>(p);
-    else attn_f32_kernel<8><<<grid, AF_WAVES * WAVE, 0, stream>>>(p);
+#define AF_OF(DT) do { \
+        if (waves == 2) attn_f32_kernel<DT, 2><<<grid, 2 * WAVE, 0, stream>>>(p); \
+        else if (waves == 4) attn_f32_kernel<DT, 4><<<grid, 4 * WAVE, 0, stream>>>(p); \
+        else attn_f32_kernel<DT, AF_WAVES><<<grid, AF_WAVES * WAVE, 0, stream>>>(p); \
+    } while (0)
+    if (dim == 32) AF_OF(2);
+    else if (dim == 64) AF_OF(4);
+    else if (dim == 96) AF_OF(6);
+    else AF_OF(8);
+#undef AF_OF
     return CISR_LAUNCH_CHECK();
 }

@@ -216,6 +216,17 @@ def f32_splits(blocks, span):
     return int(max(1, min(256 // max(blocks, 1), span // 384, 32)))
 
 
+def f32_waves(blocks, span, head_dim):
+    """Wavefronts of a block of that kernel.  A compute unit holds two blocks of eight, and where there are more and contexts are
+    short most of their waves have no step: from 384 blocks on, up to 512 keys, four, or two with heads of 128 coordinates and from
+    768 blocks on.  Single rows, us of 8 / 4 / 2 waves (row by row): 32 heads of 64, 64 rows of 16 keys 21.5 / 11.2 / 9.7 (10.0), of 256
+    60 / 44 / 48 (87); 9 heads over 3, 128 rows of 64 keys 7.8 / 6.4 / 8.4 (14.8); 32 heads of 128 over 8, 64 rows of 64 keys 12.8 /
+    14.4 / 12.0 (41).  (At 8 keys row by row stays ahead of any: 8.0 against 9.5 us for the 64 rows.)"""
+    if blocks < 384 or span > 512:
+        return 8
+    return 4 if blocks < 768 and head_dim < 128 else 2
+
+
 def rows_launch(blocks, span, heads_per_chunk, head_dim):
     """Matrix-core decode kernel: (wavefronts a block, blocks along the keys).  Few rows:
     eight waves share a row's keys inside one block; when that still leaves the GPU idle
@@ -347,7 +358,7 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
         splits = f32_splits(blocks, span)
         workspace = _split_workspace(ctx, rows, heads, splits, head_dim) if splits > 1 else None
         ops.attention_f32(q, q_row_stride, kcache, vcache, view.tables, ctx.positions, tasks, out, heads, kv_heads, head_dim, view.page_size,
-                          window, scale, splits, workspace)
+                          window, scale, splits, workspace, f32_waves(blocks, span, head_dim))
         return None
     if not ops.mfma_attention_supported(out.dtype, head_dim, view.page_size):
         splits = rowwise_splits(rows * heads, span)

@@ -56,7 +56,7 @@ def _declare(h):
         "cisr_gemm_bf16_swiglu_tile": [p, i, p, i, p, i, i, i, i, i, i, p],
         "cisr_gemm_skinny_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, p, f, p, p],
         "cisr_qkv_rope_skinny": [p, i, p, i, p, i, i, i, p, f, p, p, p, p, p, p, i, i, i, i, i, p],
-        "cisr_attn_f32": [p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, f, i, p],
+        "cisr_attn_f32": [p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, f, i, i, p],
         "cisr_attn_f32_ok": [i, i],
         "cisr_attn_merge_f32": [p, p, p, i, i, i, i, p],
         "cisr_attn_merge": [p, p, p, i, i, i, i, p, p],
@@ -402,9 +402,10 @@ def attention_f32_ok(q, q_row_stride, kcache, vcache, dim, page_size):
 
 
 def attention_f32(q, q_row_stride, kcache, vcache, tables, positions, tasks, out, heads, kv_heads, dim, page_size, window, scale,
-                  splits=1, workspace=None):
+                  splits=1, workspace=None, waves=8):
     """attention_rowwise's softmax law for float operands on the float matrix instruction, over `tasks` (int32 [n, 4]: tiles of
-    rows of one segment, at most 16 // min(heads / kv_heads, 16) rows each; rows that no task names are left alone)."""
+    rows of one segment, at most 16 // min(heads / kv_heads, 16) rows each; rows that no task names are left alone).  `waves` (2, 4 or
+    8): wavefronts that share a tile's keys, sixteen a turn each."""
     rows, pages = out.shape[0], kcache.shape[0]
     if not attention_f32_ok(q, q_row_stride, kcache, vcache, dim, page_size) or heads % kv_heads:
         raise KernelError("attention_f32: operands not supported")
@@ -421,7 +422,7 @@ def attention_f32(q, q_row_stride, kcache, vcache, tables, positions, tasks, out
                                _dev(vcache, "vcache", torch.float32, (pages, kv_heads, dim, page_size)), _dev(tables, "tables", torch.int32),
                                _dev(positions, "positions", torch.int32, (rows,)), _dev(tasks, "tasks", torch.int32, (tasks.shape[0], 4)),
                                tasks.shape[0], op, po, pm, heads, kv_heads, dim, page_size, tables.shape[1], int(window or 0), float(scale),
-                               int(splits), _stream()), "attention_f32")
+                               int(splits), int(waves), _stream()), "attention_f32")
     if splits > 1:
         _check(lib().cisr_attn_merge_f32(po, pm, op, rows, heads, dim, int(splits), _stream()), "attention_merge")
     return out

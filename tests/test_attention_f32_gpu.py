@@ -109,3 +109,34 @@ def test_rows_do_not_see_what_is_not_finite_where_they_do_not_look(window, value
     assert (got[~sees] - want[~sees]).abs().max().item() < 1e-5 and not got[sees, dim + 3].isfinite().any()
     other = torch.arange(heads * dim, device=DEV) != dim + 3
     assert (got[:, other] - want[:, other]).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim", [(9, 3, 64), (4, 4, 32), (8, 1, 128), (6, 2, 96)])
+@pytest.mark.parametrize("waves", [2, 4])
+def test_attention_f32_with_fewer_waves(heads, kv_heads, dim, waves):
+    """Blocks of two and four waves, with no step for some of them and with several for each, whole and with split keys: the result in 64 bits
+    (weights as in test_attention_f32), and the bits of eight waves where no wave has a second step."""
+    from runtime.kernels import ops
+    page, lengths = 16, [1, 16, 17, 16 * waves, 16 * waves + 1, 130]
+    _, kt, vt, tables, _ = paged_case(heads, kv_heads, dim, page, lengths, torch.float32, seed=dim)
+    rows = [(seg, pos) for seg, n in enumerate(lengths) for pos in range(max(0, n - 7), n)]
+    q, scale = rnd(len(rows), heads, dim, seed=4), dim ** -0.5
+    want = reference_attention(q, kt, vt, tables, rows, page, scale=scale)
+    pos = torch.tensor([r[1] for r in rows], dtype=torch.int32, device=DEV)
+    tasks, flat, outs = tasks_of(rows, 16 // min(heads // kv_heads, 16)), q.reshape(len(rows), -1).contiguous(), {}
+    for splits, w in ((1, waves), (3, waves), (1, 8)):
+        out = torch.full((len(rows), heads * dim), 7.0, device=DEV)
+        ws = (torch.empty(len(rows) * heads * splits * dim, device=DEV), torch.empty(len(rows) * heads * splits * 2, device=DEV))
+        ops.attention_f32(flat, heads * dim, kt, vt, tables, pos, tasks, out, heads, kv_heads, dim, page, None, scale, splits, ws, w)
+        np.testing.assert_allclose(f64(out).reshape(want.shape), want, rtol=tol(torch.float32)["rtol"], atol=1e-5, err_msg=f"splits={splits}")
+        outs[splits, w] = out
+    short = torch.tensor([lengths[seg] <= 16 * waves for seg, _ in rows], device=DEV)
+    assert torch.equal(outs[1, waves][short], outs[1, 8][short])
+    with pytest.raises(ops.KernelError):
+        ops.attention_f32(flat, heads * dim, kt, vt, tables, pos, tasks, out, heads, kv_heads, dim, page, None, scale, waves=3)
+
+
+def test_many_blocks_of_short_contexts_have_few_waves():
+    from runtime.kernels.attention import f32_waves
+    assert [f32_waves(n, 256, 64) for n in (1, 383, 384, 767, 768, 8192)] == [8, 8, 4, 4, 2, 2]
+    assert f32_waves(384, 256, 128) == 2 and f32_waves(8192, 513, 64) == f32_waves(383, 16, 128) == 8
