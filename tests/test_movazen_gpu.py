@@ -481,14 +481,14 @@ def test_prompt_then_tokens_one_by_one_and_portions_down_to_two_tokens(folders, 
 
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_long_portion_walked_in_pieces(folders, dtype):
-    """A portion long enough for the memory's scan to walk it in pieces side by side, after a shorter one that leaves a
-    state, beside a second request's portion in the same step."""
+    """A portion that the memory takes in several chunks side by side, after a shorter one that leaves a state, beside a second
+    request's portion in the same step."""
     from runtime.engine import StepEntry
     from runtime.kernels import ops
     name = "a"
     V = CONFIGS[name]["vocab"]
     long, other = decisive_tokens(folders[name], 31, 700, V), decisive_tokens(folders[name], 32, 300, V)
-    assert ops.scan_piece(600 + 300, False) > 0
+    assert ops.lightning_form(None, None, None, None, 600 + 300, 2, False, 0) == "chunks" and 300 > ops.LIGHTNING_CHUNK
     runner = make_runner(folders[name], dtype, pages=70)
     runner.create("l"); runner.create("o")
     got = [runner.step([StepEntry("l", long[:100], list(range(100)))]).cpu().numpy()]

@@ -405,14 +405,17 @@ def test_prompt_then_tokens_one_by_one_and_portions_down_to_two_tokens(folders, 
 
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_long_portion_walked_in_pieces(folders, dtype):
-    """A portion long enough for the memory's scan to walk it in pieces side by side, after a shorter one that leaves a
-    state, beside a second request's portion in the same step."""
+    """Portions that the memory walks chunk by chunk: a long one after a shorter one that leaves a state, beside a second
+    request's in the same step."""
     from runtime.engine import StepEntry
-    from runtime.kernels import ops
+    from runtime.engine.context import Batch
+    from runtime.parts.recurrent import LinearByChunks
     name = "a"
     V = CONFIGS[name]["vocab"]
     long, other = random_tokens(31, 700, V), random_tokens(32, 300, V)
-    assert ops.scan_piece(600 + 300, False) > 0
+    memory = next(l["mixer"]["right"] for l in CONFIGS[name]["layers"] if l["type"] == "parallel")
+    rule = LinearByChunks(memory["heads"], memory["dim"], memory["vdim"] + 1)
+    assert rule.launch_value(Batch([100], [0], None, False, {})) and rule.launch_value(Batch([600, 300], [100, 0], None, False, {}))
     runner = make_runner(folders[name], dtype, pages=70)
     runner.create("l"); runner.create("o")
     got = [runner.step([StepEntry("l", long[:100], list(range(100)))]).cpu().numpy()]
