@@ -142,7 +142,7 @@ __device__ __forceinline__ void few_tile(const FewArgs& p, int e, int tile, int 
 template <typename TC, int ACT>
 __global__ void __launch_bounds__(EXF_WAVES * WAVE)
 experts_few_kernel(FewArgs p) {
-    __shared__ exf_u32x4 lds[EXF_WAVES * 6 * 128];                    // (at most six pieces a wave: 48 KB)
+    __shared__ exf_u32x4 lds[EXF_WAVES * 6 * 128];                    // (at most six pieces a wave: 12 KB)
     const int tile = blockIdx.x, e = p.tile_expert[tile];
     if (e < 0) return;
     // a tile's pairs come first, padding behind them
