@@ -228,13 +228,12 @@ attn_f32_kernel(AttnF32Args p) {
             den += f * sl[w][i];
             num += f * so[w][i][d];
         }
-        const float y = den > 0.f ? num / den : 0.f;
         const size_t at = (size_t)row_of(i) * p.heads + head_of(i);
-        if (p.splits == 1) {
-            p.out[at * D + d] = y;
-        } else {
+        if (p.splits == 1) {                                          // (an item sees its own key: a sum of zero is of scores that are all -inf)
+            p.out[at * D + d] = num / den;
+        } else {                                                      // (a split may hold no key that the item sees)
             const size_t part = at * p.splits + blockIdx.z;
-            p.part_o[part * D + d] = y;
+            p.part_o[part * D + d] = den > 0.f ? num / den : 0.f;
             if (d == 0) { p.part_ml[part * 2] = best; p.part_ml[part * 2 + 1] = den; }
         }
     }

@@ -111,6 +111,34 @@ def test_rows_do_not_see_what_is_not_finite_where_they_do_not_look(window, value
     assert (got[:, other] - want[:, other]).abs().max().item() < 1e-5
 
 
+@pytest.mark.parametrize("where", ["query", "key", "value", "scores of -inf"])
+def test_what_is_not_finite_reaches_the_rows_that_see_it(where):
+    """A query, a key or a value that is no number, and scores that are all -inf, whose weights are none: no number as row by row, in the same
+    rows and coordinates."""
+    from runtime.kernels import ops
+    heads, dim, page, n = 2, 32, 16, 40
+    _, kt, vt, tables, _ = paged_case(heads, heads, dim, page, [n], torch.float32, seed=1)
+    pos = torch.arange(20, n, dtype=torch.int32, device=DEV)
+    q = rnd(n - 20, heads * dim, seed=2)
+    if where == "query":
+        q[3, 5] = float("nan")
+    elif where == "key":
+        kt[tables[0, 1], 1, 30 - 16, 7] = float("nan")
+    elif where == "value":
+        vt[tables[0, 1], 1, 7, 30 - 16] = float("nan")
+    else:
+        kt[:, 0, :, 0] = -float("inf")
+        q[:, 0] = q[:, 0].abs() + 0.1
+    tasks, seg = torch.tensor([(0, 0, 16, 0), (0, 16, 4, 0)], dtype=torch.int32, device=DEV), torch.zeros(n - 20, dtype=torch.int32, device=DEV)
+    want, args = torch.empty(n - 20, heads * dim, device=DEV), (heads, heads, dim, page, None, dim ** -0.5)
+    ops.attention_rowwise(q, heads * dim, kt, vt, tables, seg, pos, want, *args)
+    assert want.isnan().any() and not want.isnan().all()
+    for waves in (2, 8):
+        got = torch.empty(n - 20, heads * dim, device=DEV)
+        ops.attention_f32(q, heads * dim, kt, vt, tables, pos, tasks, got, *args, waves=waves)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.allclose(got, want, rtol=1e-4, atol=1e-5, equal_nan=True)
+
+
 @pytest.mark.parametrize("heads, kv_heads, dim", [(9, 3, 64), (4, 4, 32), (8, 1, 128), (6, 2, 96)])
 @pytest.mark.parametrize("waves", [2, 4])
 def test_attention_f32_with_fewer_waves(heads, kv_heads, dim, waves):
