@@ -30,7 +30,8 @@ class AttentionTuning:
     tile_waves: int = 4                   # wavefronts that share one tile's keys
     item_tiles: int = 2                   # 16-item tiles a wave of long portions (small heads)
     # In a mixed step a decoded token is a tile whose keys one block walks; from this context on the one-token
-    # segments get a launch of their own instead, which splits their keys over blocks
+    # segments get a launch of their own instead, which splits their keys over blocks (from twice that on where there
+    # are 24 of them and more: they are blocks enough, and run beside the portions)
     split_single_from: int = 4096
     rows_launch: Optional[tuple] = None   # (wavefronts a block, blocks along the keys) of decode rows
     stream_loads: Optional[bool] = None   # decode rows read keys and values with non-temporal loads (None: by the rule)
@@ -76,7 +77,10 @@ def fill_tasks(tasks, counts, rows_per_tile, starts=None, skip_single=False):
 class SingleRows:
     """Step array: the rows of the one-token segments of a mixed step (then -1), when they get an attention launch
     of their own: all of them, if one of them has a context of `split_from` keys or more; none in a step of
-    one-token segments only, or of short contexts.  Its launch value is how many entries such a launch covers."""
+    one-token segments only, or of short contexts.  Its launch value is how many entries such a launch covers.
+    From 24 of them on `split_from` counts twice (30 rows of 5,000 keys beside a portion, us together / apart: 9 heads of 64
+    over 3 and 2,048 rows 65 / 105, 32 heads of 64 and 512 rows 216 / 276, 32 heads of 128 over 8 and 512 rows 152 / 169; but 8 of
+    6,000 and 1,024 rows 71 / 39, 107 / 113, 155 / 90, and 20 of 15,000 171 / 69, 458 / 462, 408 / 293)."""
     split_from: int
 
     def words(self, rows, segments):
@@ -84,7 +88,8 @@ class SingleRows:
 
     def launch_value(self, batch):
         singles = [start + 1 for start, count in zip(batch.starts, batch.counts) if count == 1]
-        if not singles or len(singles) == len(batch.counts) or max(singles) < self.split_from:
+        split_from = self.split_from * (2 if len(singles) >= 24 else 1)
+        if not singles or len(singles) == len(batch.counts) or max(singles) < split_from:
             return 0
         return len(singles)
 
@@ -93,6 +98,22 @@ class SingleRows:
         if value:
             own = [int(batch.first_row[s]) for s, c in enumerate(batch.counts) if c == 1]
             out[:len(own)] = own
+
+
+@dataclass(frozen=True)
+class SingleTokens:
+    """Step array without contents whose launch value is the number of one-token segments in a step that has portions
+    too, otherwise 0: what picks a mixed step's form is its portions and how many blocks the others bring (prompt_form)."""
+
+    def words(self, rows, segments):
+        return 0
+
+    def launch_value(self, batch):
+        singles = sum(count == 1 for count in batch.counts)
+        return singles if singles < len(batch.counts) else 0
+
+    def fill(self, out, batch, value):
+        pass
 
 
 @dataclass(frozen=True)
@@ -142,15 +163,32 @@ class TileTasks:
 
 # -- rules ------------------------------------------------------------------------------------------------------
 
-def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tuning=DEFAULT_TUNING):
+def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tuning=DEFAULT_TUNING, singles=0):
     """Which form of the matrix-core kernel the prompt rows of a step take, (kind, n, halves): ("tiles", n, 1): a block
     is one tile of 16 n items (a token row and a query head) whose waves split its keys; ("block", n, 1): 64 n items,
     four waves that own different rows and share keys and values through LDS; ("square", n, halves): 64 n items on
     the 32 x 32 instruction with waves of their own for the copies, as one half or as two that take the even and the
-    odd steps.  `span`: the longest context of the step."""
+    odd steps.  `span`: the longest context of the step.  `singles`: how many of the segments are single tokens that
+    share the launch; the others' rows decide, with the singles' blocks counted beside theirs."""
+    rows, n_segments = max(1, rows - singles), max(1, n_segments - singles)
     group = heads // kv_heads
     heads_per_chunk = min(group, 16)
     long_portions = rows >= 16 * n_segments
+    if singles and head_dim <= 128 and page_size >= 8 and (long_portions or singles >= n_segments) and tuning.square_tiles is None:
+        # Decoded tokens beside portions: a block of the square form gives all its waves to a tile of one row, and the
+        # single rows' reads run beside the portions' products.  Small blocks (64 items, four waves) leave the compute units room
+        # for both; two halves where all the blocks are few and long.  us, before (a single row walked by one wave of a tile) -> now,
+        # with 128 items in brackets: 32 heads of 64, 37 rows of 900 keys and a portion of 1,024: 123 -> 74 (82); 30 of
+        # 1,300 and one of 30: 99 -> 61 (61); 16 of 200 and one of 256: 22 -> 16 (18); 32 heads of 128 over 8: 78 -> 60
+        # (67), 68 -> 44 in halves (46), 22 -> 16 (18).  Below 256 blocks the forms of few blocks below stay ahead (9 heads
+        # over 3, 16 of 200 and 256: 11.8 against 13.0); with large heads, so do larger blocks where a row's chain of steps is
+        # long (30 of 2,400 and 1,024: 98 against 85 with 128 items) or the portions fill the GPU (8 of 2,000 and 2,048: 82 against
+        # 73 with 192).
+        chunks = kv_heads * -(-group // heads_per_chunk)
+        blocks = -(-rows // (64 // heads_per_chunk)) * chunks
+        together = blocks + singles * chunks
+        if together >= 256 and (head_dim <= 64 or (span <= 2048 and blocks < 1000)):
+            return "square", 1, 2 if together <= 384 and span >= 1024 else 1
     if long_portions and head_dim <= 128:
         # enough long portions to fill the GPU with blocks of 64 items (or more): the waves of a block own different
         # rows and share each step's keys and values through LDS.  Otherwise (few heads, short portions) the waves
@@ -399,7 +437,11 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
         workspace = _split_workspace(ctx, n_single, heads, splits, head_dim) if splits > 1 else None
         ops.attention_mfma(*common, None, splits, workspace, waves, row_ids=single_rows[:n_single],
                            stream_loads=stream(n_single * chunks, waves, splits), **law)
-    form = prompt_form(rows, ctx.n_segments, span, heads, kv_heads, head_dim, view.page_size, tuning)
+    _, alone = ctx.step_array(SingleTokens())
+    if n_single:
+        form = prompt_form(max(1, rows - alone), max(1, ctx.n_segments - alone), span, heads, kv_heads, head_dim, view.page_size, tuning)
+    else:
+        form = prompt_form(rows, ctx.n_segments, span, heads, kv_heads, head_dim, view.page_size, tuning, alone)
     if head_bias is not None and form[0] != "tiles":
         form = ("tiles", 2 if tuning.item_tiles == 2 and head_dim <= 64 else 1, 1)
     if (slopes is not None or keep_first) and form[0] == "block":

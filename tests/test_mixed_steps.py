@@ -1,0 +1,58 @@
+"""Attention of steps that hold decoded tokens beside prompt portions: the rule that picks their form, and single rows inside the
+square form (all waves of a block take one row's keys) at the edges of its key steps, pages and head groups."""
+import pytest
+import torch
+
+from runtime.engine.context import Batch
+from runtime.kernels.attention import AttentionTuning, SingleRows, SingleTokens, prompt_form
+
+
+def test_single_tokens_of_a_step():
+    """The launch value counts the one-token segments, and only where portions share the step."""
+    def value(counts):
+        return SingleTokens().launch_value(Batch(counts, [0] * len(counts), None, all(c == 1 for c in counts), {}))
+    assert [value(c) for c in ([1, 5, 1], [1, 5, 9, 2], [5, 9], [7], [1, 1], [1])] == [2, 1, 0, 0, 0, 0]
+    assert SingleTokens().words(64, 8) == 0
+
+
+def test_single_rows_share_the_launch_up_to_twice_the_context_when_they_are_many():
+    def value(n, context):
+        return SingleRows(100).launch_value(Batch([1] * n + [6], [context - 1] * n + [0], None, False, {}))
+    assert [value(23, 99), value(23, 100), value(24, 199), value(24, 200), value(1, 100)] == [0, 23, 0, 24, 1]
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim, singles, rows, span, form", [
+    (32, 32, 64, 37, 1024, 2048, ("square", 1, 1)),
+    (32, 32, 64, 16, 256, 256, ("square", 1, 1)),       # 640 blocks, short contexts
+    (32, 8, 128, 16, 256, 1024, ("square", 1, 2)),      # 256 blocks
+    (32, 8, 128, 37, 1024, 2048, ("square", 1, 1)),
+    (32, 8, 128, 30, 1024, 4096, ("square", 2, 1)),     # large heads, long rows: the portions' own form
+    (9, 3, 64, 37, 1024, 2048, ("square", 1, 2)),       # 255 blocks
+    (9, 3, 64, 16, 256, 256, ("tiles", 2, 1)),
+    (32, 32, 64, 30, 30, 2048, ("square", 1, 1)),
+    (32, 32, 256, 30, 300, 2048, ("tiles", 1, 1)),
+])
+def test_form_of_mixed_steps_at_measured_points(heads, kv_heads, dim, singles, rows, span, form):
+    assert tuple(prompt_form(rows + singles, 1 + singles, span, heads, kv_heads, dim, 16, singles=singles)) == form
+    assert prompt_form(rows + singles, 1 + singles, span, heads, kv_heads, dim, 4, singles=singles)[0] != "square"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, kv_heads, D", [(9, 3, 64), (32, 8, 128), (4, 4, 32), (20, 1, 96), (6, 2, 72)])
+def test_single_rows_in_square_tiles(heads, kv_heads, D):
+    """Single rows of 1 to 300 keys (no key but their own, a step less one, a step, one more, a wave's second step) beside portions
+    whose last tile is one row too, in every size of block and in halves; then a step that takes the form by the rule."""
+    from test_long_attention_gpu import Step, attend, check
+    keys = [1, 2, 15, 16, 17, 31, 32, 33, 64, 127, 255, 256, 257, 300]
+    per = 64 // min(heads // kv_heads, 16)
+    step = Step([1] * 7 + [per + 1] + [1] * 7 + [3, 2 * per + 1], [k - 1 for k in keys[:7]] + [40] + [k - 1 for k in keys[7:]] + [500, 0])
+    for n, halves in ((1, 1), (1, 2), (2, 1), (2, 2), (3, 1), (4, 1)):
+        if D > 64 and (n == 4 or (n == 2 and halves == 2)):
+            continue
+        got, want = attend(step, heads, kv_heads, D, seed=n, tuning=AttentionTuning(square_tiles=n, square_halves=halves))
+        check(got, want, f"{heads}/{kv_heads}x{D}, blocks of {64 * n} items, {halves} halves")
+    step = Step([1] * 90 + [200], [7 * i for i in range(90)] + [100])
+    if kv_heads >= 3:
+        assert prompt_form(290, 91, step.span_hint, heads, kv_heads, D, 16, singles=90)[0] == "square"
+    got, want = attend(step, heads, kv_heads, D, seed=9)
+    check(got, want, f"{heads}/{kv_heads}x{D}, 90 single rows and 200")
