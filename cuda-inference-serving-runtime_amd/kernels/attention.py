@@ -27,6 +27,7 @@ class AttentionTuning:
     block_tiles: Optional[int] = None     # long portions through LDS-shared tiles of 64 x this items
     square_tiles: Optional[int] = None    # long portions of long contexts through 32 x 32 tiles, 64 x this items a block (0: never)
     square_halves: Optional[int] = None   # two halves a block in that form (even and odd steps): 1, 2
+    deep_tiles: Optional[bool] = None     # portions with heads of more than 128 coordinates through LDS-shared tiles of 64 items
     tile_waves: int = 4                   # wavefronts that share one tile's keys
     item_tiles: int = 2                   # 16-item tiles a wave of long portions (small heads)
     # In a mixed step a decoded token is a tile whose keys one block walks; from this context on the one-token
@@ -168,7 +169,7 @@ def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tu
     is one tile of 16 n items (a token row and a query head) whose waves split its keys; ("block", n, 1): 64 n items,
     four waves that own different rows and share keys and values through LDS; ("square", n, halves): 64 n items on
     the 32 x 32 instruction with waves of their own for the copies, as one half or as two that take the even and the
-    odd steps.  `span`: the longest context of the step.  `singles`: how many of the segments are single tokens that
+    odd steps; ("deep", 1, 1): "block" for heads of more than 128 coordinates.  `span`: the longest context of the step.  `singles`: how many of the segments are single tokens that
     share the launch; the others' rows decide, with the singles' blocks counted beside theirs."""
     rows, n_segments = max(1, rows - singles), max(1, n_segments - singles)
     group = heads // kv_heads
@@ -231,6 +232,15 @@ def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tu
         block_tiles = (2 if blocks >= 2048 else 1 if blocks >= 512 else 0) if tuning.block_tiles is None else tuning.block_tiles
         if block_tiles:
             return "block", block_tiles, 1
+    if long_portions and head_dim > 128 and page_size >= 8:
+        # Large heads: the block of 64 items takes 1.4 us a step, a tile's four waves 0.8 (each step's keys straight from the
+        # caches, for 16 items).  It is ahead once the tiles wait for the caches: us as tiles / deep, 16 heads of 256 over one key
+        # head, 1,000 rows (250 blocks) 91 / 56, 700 and 1,300 rows 186 / 77, 4,096 rows 811 / 292; 8 heads of 192 over 2, 2,048 rows
+        # (256 blocks) 107 / 77.  At 128 blocks it depends on the chain: 512 rows of 16 heads over one 40 / 33, 256 rows of 24 heads
+        # of 160 over one 25 / 18, the same rows behind 3,000 keys 90 / 107.
+        blocks = -(-rows // (64 // heads_per_chunk)) * kv_heads * -(-group // heads_per_chunk)
+        if blocks >= (96 if span <= 512 else 192) if tuning.deep_tiles is None else tuning.deep_tiles:
+            return "deep", 1, 1
     return "tiles", 2 if tuning.item_tiles == 2 and long_portions and head_dim <= 64 else 1, 1
 
 
@@ -444,12 +454,13 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
         form = prompt_form(rows, ctx.n_segments, span, heads, kv_heads, head_dim, view.page_size, tuning, alone)
     if head_bias is not None and form[0] != "tiles":
         form = ("tiles", 2 if tuning.item_tiles == 2 and head_dim <= 64 else 1, 1)
-    if (slopes is not None or keep_first) and form[0] == "block":
-        form = ("square", form[1], 1)         # (that law's build has no block tiles on the 16 x 16 instruction)
+    if (slopes is not None or keep_first) and form[0] in ("block", "deep"):
+        # (that law's build has no such tiles)
+        form = ("square", form[1], 1) if form[0] == "block" else ("tiles", 1, 1)
     kind, item_tiles, halves = form
     tasks, _ = ctx.step_array(TileTasks(rows_per_tile_of(form, heads, kv_heads), singles))
     ops.attention_mfma(*common, tasks.view(-1, 4), waves=tuning.tile_waves,
-                       block_tiles={"tiles": False, "block": True, "square": 32}[kind], item_tiles=item_tiles, key_groups=halves,
+                       block_tiles={"tiles": False, "block": True, "square": 32, "deep": "deep"}[kind], item_tiles=item_tiles, key_groups=halves,
                        **law)
     return None
 

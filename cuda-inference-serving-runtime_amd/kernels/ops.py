@@ -934,7 +934,8 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
     """Matrix-core attention (bf16).  tasks int32 [n, 4] = (segment, first row, rows, 0) runs tiles of
     prompt rows: one tile of 16/GC rows a block whose waves share the keys (with item_tiles=2, head sizes up to
     64: 32/GC rows, two item tiles a wave), or with `block_tiles` (head sizes up to 128) one tile of
-    64 item_tiles / GC rows a block whose four waves own different rows and share keys and values through LDS
+    64 item_tiles / GC rows a block whose four waves own different rows and share keys and values through LDS ("deep": the
+    same with 64 items and head sizes above 128)
     (GC = query heads per key head, at most 16); tasks None runs one block
     per row (decode) of `waves` wavefronts (4 or 8) with `splits` blocks along the keys; splits > 1 needs
     workspace = (partials float, statistics float) and a merge.  `row_ids` (int32 [n], with tasks None): only
@@ -981,10 +982,15 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
     if tasks is not None:
         if item_tiles not in ((1, 2, 3, 4) if block_tiles == 32 else (1, 2)) or (item_tiles == 2 and dim > 64 and not block_tiles):
             raise KernelError("attention_mfma: two item tiles a wave need a head size of at most 64")
-        if block_tiles and dpad > 128:
+        if block_tiles == "deep":
+            if dpad <= 128 or law_name != "softmax" or item_tiles != 1:
+                raise KernelError("attention_mfma: deep tiles are 64 items of the softmax law with heads of more than 128 coordinates")
+        elif block_tiles and dpad > 128:
             raise KernelError("attention_mfma: block tiles need a head size of at most 128")
         n_tasks, splits = tasks.shape[0], 1
         mode = (2 if item_tiles == 1 else 4) if block_tiles else (3 if item_tiles == 2 else 0)
+        if block_tiles == "deep":
+            mode = 12
         if block_tiles == 32:
             # the 32 x 32 matrix instruction: 128/GC rows a block and four waves (item_tiles 2), or 64/GC rows and two
             if out.numel() >= 2 ** 31:

@@ -30,7 +30,8 @@ def test_single_rows_share_the_launch_up_to_twice_the_context_when_they_are_many
     (9, 3, 64, 37, 1024, 2048, ("square", 1, 2)),       # 255 blocks
     (9, 3, 64, 16, 256, 256, ("tiles", 2, 1)),
     (32, 32, 64, 30, 30, 2048, ("square", 1, 1)),
-    (32, 32, 256, 30, 300, 2048, ("tiles", 1, 1)),
+    (32, 32, 256, 30, 300, 2048, ("tiles", 1, 1)),      # 160 blocks
+    (32, 32, 256, 30, 400, 2048, ("deep", 1, 1)),
 ])
 def test_form_of_mixed_steps_at_measured_points(heads, kv_heads, dim, singles, rows, span, form):
     assert tuple(prompt_form(rows + singles, 1 + singles, span, heads, kv_heads, dim, 16, singles=singles)) == form
