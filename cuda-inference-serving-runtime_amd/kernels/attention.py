@@ -12,6 +12,7 @@ step's context for them (`ctx.step_array`), and the step function carries them i
 on without knowing what they hold.  The reference has one attention kernel and no such choice
 (kernels/ops.cu:35-80).
 """
+import functools
 from dataclasses import dataclass
 from typing import Optional
 
@@ -134,6 +135,66 @@ class RowsLongestFirst:
         if batch.decode_only:
             order = np.argsort(-np.asarray(batch.starts, dtype=np.int64), kind="stable")
             out[:len(order)] = np.asarray(batch.first_row, dtype=np.int64)[order]
+
+
+@functools.lru_cache(maxsize=1024)      # (rules of sizes alone, asked for again in every step's metadata)
+def _pieces_launch(pieces, rows, span):
+    if pieces.seen:
+        span = min(span, pieces.seen)
+    blocks = rows * pieces.chunks
+    waves, splits = rows_launch(blocks, span, pieces.heads_per_chunk, pieces.head_dim)
+    room = rows_room(blocks, span, waves, splits, pieces.head_dim)
+    return None if room is None else (room[0], max(rows, -(-room[1] // pieces.chunks)), room[2], splits)
+
+
+@dataclass(frozen=True)
+class RowPieces:
+    """Step array: how the blocks of a decode step are dealt to its rows by the 32-key steps that each has to walk: int32 [rows +
+    1], the first block of every row (rows that pad a step have none) and the end.  Which launch that is for follows from rows
+    and the longest context, rounded up to a power of two (`launch`): where a row's keys are not cut the array stays empty.
+    `chunks`: blocks a row and part has; `seen`: how many keys a row sees at most (0: all)."""
+    chunks: int
+    heads_per_chunk: int
+    head_dim: int
+    window: int
+    seen: int
+
+    def launch(self, rows, longest):
+        """(wavefronts a block, blocks a key head, least steps a wave, nominal splits) of `rows` rows up to `longest` keys, or None."""
+        return _pieces_launch(self, rows, max(256, 1 << (int(longest) - 1).bit_length()))
+
+    def words(self, rows, segments):
+        return rows + 1
+
+    def launch_value(self, batch):
+        return None
+
+    def fill(self, out, batch, value):
+        """A part is a multiple of the block's waves in steps (each wave then walks as many), the smallest for which the parts of all
+        rows are no more than there are blocks; a row has at most 16, or 32 where rows are few and a wave has two steps and
+        more (their merge costs more than a second step)."""
+        rows = len(out) - 1
+        launch = self.launch(rows, max(batch.starts) + 1) if batch.decode_only else None
+        if launch is None:
+            out[:] = 0
+            return
+        waves, blocks, a_wave, _ = launch
+        ends = np.array(batch.starts) + 1
+        steps = ends + 31
+        if self.window:
+            steps -= np.maximum(ends - self.window, 0) & ~31
+        steps >>= 5
+        a_wave = max(a_wave, -(-int(steps.sum()) // (waves * blocks)))
+        if a_wave == 1 and int(steps.max()) > 32 * waves:
+            a_wave = 2                # (more than sixteen parts of two steps a wave instead of sixteen longer ones)
+        while True:
+            ends = np.minimum((steps + (waves * a_wave - 1)) // (waves * a_wave), 32 if rows < 16 and a_wave > 1 else 16).cumsum()
+            if ends[-1] <= blocks:
+                break
+            a_wave += max(1, a_wave // 8)
+        out[0] = 0
+        out[1:len(ends) + 1] = ends
+        out[len(ends) + 1:] = ends[-1]
 
 
 @dataclass(frozen=True)
@@ -325,6 +386,42 @@ def rows_launch(blocks, span, heads_per_chunk, head_dim):
     return waves, splits
 
 
+def rows_room(blocks, span, waves, splits, head_dim):
+    """Whether a decode step that `rows_launch` gives (waves, splits) deals its blocks to the rows by their lengths, and how:
+    (wavefronts a block, blocks that the launch has room for, least 32-key steps a wave), or None: unsplit.
+    The launch is filled once: 512 blocks of four waves (256 with more than 128 coordinates, where a compute unit holds one),
+    256 of eight, 768 of four with small heads, 1,024 where runs are long.  us of a step of rows between 0.4 and 1.6 times a mean, equal
+    splits -> by pieces: 32 heads of 128 over 8, 12 rows of 5,000 keys 76 -> 53, 24 of 3,000 93 -> 62, 3 of 700 11.1 -> 10.9, one of 30,000
+    among eight of 500 125 -> 40; 9 of 64 over 3, 100 rows of 1,500 37 -> 30, 64 of 7,000 75 -> 64; one key head of 256, 24 rows of 2,000
+    44 -> 24.  Rows of one length, where only a merge that looks its parts up is added: 8 rows of 5,000 keys 36.2 -> 36.8, 16 of
+    2,000 31.9 -> 31.7.
+    Small heads of many rows that are not split otherwise are, from 4,096 keys on: 32 heads of 64, 12 rows of 2,000 47 -> 41, 16 of
+    4,500 112 -> 100, 16 and 32 of 2,100 keys each 49 -> 50 and 93 -> 92; below, whole rows longest first are ahead (16 of 1,000 29.2 against 31.9, 64 of 1,216 109 against 114), and
+    so they are with large heads of one length (64 rows of 1,500, 32 heads of 128 over 8: 71 against 78)."""
+    if splits == 1:
+        return (4, 1536, 2) if head_dim <= 64 and span >= 4096 and 256 < blocks <= 1024 else None
+    if head_dim > 64:
+        return 4, (512 if head_dim <= 128 else 256), (1 if blocks < 128 else 2)
+    if waves == 8:
+        return 8, 256, 1
+    return 4, (1024 if blocks * splits > 768 else 768), 2
+
+
+def row_pieces(heads, kv_heads, head_dim, window, keep_first=0):
+    """The RowPieces of an attention layer."""
+    group = heads // kv_heads
+    per_chunk = min(group, 16)
+    window = int(window or 0)
+    return RowPieces(kv_heads * -(-group // per_chunk), per_chunk, head_dim, window, window + 31 + keep_first if window else 0)
+
+
+def step_arrays(tuning, operand, *layer):
+    """The step arrays that an attention layer names beforehand.  `operand`: one of its matrices (decode rows on the matrix cores,
+    which RowPieces is for, are those of bfloat16 ones); `layer`: what `row_pieces` takes."""
+    pieces = [row_pieces(*layer)] if operand is not None and operand.dtype == torch.bfloat16 and tuning.rows_launch is None else []
+    return [SingleRows(tuning.split_single_from), SingleTokens(), RowsLongestFirst()] + pieces
+
+
 def rows_stream_loads(blocks, span, waves, splits, head_dim):
     """Whether the decode kernel launched as `blocks` x `splits` blocks of `waves` wavefronts reads keys and values with
     non-temporal loads (no block reads them again; the caches then do not keep them).  Measured inside decode steps
@@ -431,6 +528,14 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
                 ops.attention_mfma(*common, None, fused, workspace, waves, merge=False,
                                    stream_loads=stream(rows * chunks, waves, fused), **law)
                 return workspace[0], workspace[1], fused
+        pieces = row_pieces(heads, kv_heads, head_dim, window, keep_first)
+        launch = pieces.launch(rows, ctx.span_hint) if tuning.rows_launch is None else None
+        if launch is not None:
+            waves, blocks, _, splits = launch
+            firsts, _ = ctx.step_array(pieces)
+            ops.attention_mfma(*common, waves=waves, workspace=_split_workspace(ctx, blocks, heads, 1, head_dim), merge_gate=merge_gate,
+                               pieces=(firsts[:rows + 1], blocks), stream_loads=stream(rows * chunks, waves, splits), **law)
+            return None if merge_gate is None else GATED
         workspace = _split_workspace(ctx, rows, heads, splits, head_dim) if splits > 1 else None
         order = None
         if splits == 1 and rows * chunks >= tuning.order_rows_from:

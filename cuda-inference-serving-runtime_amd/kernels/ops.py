@@ -60,6 +60,7 @@ def _declare(h):
         "cisr_attn_f32_ok": [i, i],
         "cisr_attn_merge_f32": [p, p, p, i, i, i, i, p],
         "cisr_attn_merge": [p, p, p, i, i, i, i, p, p],
+        "cisr_attn_merge_pieces": [p, p, p, i, i, i, p, i, p, i, i, p],
         "cisr_argmax": [p, p, p, i, p, p, i, i, p],
         "cisr_sample": [p, p, p, p, p, p, i, i, i, p],
         "cisr_take_tokens": [p, p, p, i, i, p],
@@ -930,7 +931,7 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
 def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, positions, out, heads, kv_heads, dim,
                    page_size, window, scale, tasks=None, splits=1, workspace=None, waves=4, block_tiles=False,
                    item_tiles=1, row_ids=None, merge=True, key_groups=1, stream_loads=False, head_bias=None, slopes=None, sink=None,
-                   keep_first=0, merge_gate=None):
+                   keep_first=0, merge_gate=None, pieces=None):
     """Matrix-core attention (bf16).  tasks int32 [n, 4] = (segment, first row, rows, 0) runs tiles of
     prompt rows: one tile of 16/GC rows a block whose waves share the keys (with item_tiles=2, head sizes up to
     64: 32/GC rows, two item tiles a wave), or with `block_tiles` (head sizes up to 128) one tile of
@@ -949,7 +950,10 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
     `slopes`, `sink`, `keep_first`: as in attention_rowwise; with slopes or kept keys every form but the block tiles of 64 and
     128 items on the 16 x 16 instruction runs (a build of its own).  `merge_gate` = (gates float view [T, heads * vdim], packed
     bf16 [T, heads * vdim], vdim) with splits > 1 and all rows: the merge packs the heads' first vdim coordinates, gates them
-    element by element and writes `packed`; `out` is not written."""
+    element by element and writes `packed`; `out` is not written.
+    `pieces` = (firsts int32 [rows + 1], blocks) (rows mode over all rows, with workspace): row r's keys are cut into firsts[r + 1] -
+    firsts[r] parts (at most 32; none: the row has no keys and becomes zeros), a block a part; `blocks` is what the launch
+    has for a key head and the workspace for every head, at least firsts[rows]."""
     rows = out.shape[0]
     law_name = "sigmoid" if head_bias is not None else "distance" if slopes is not None or keep_first else "softmax"
     if law_name == "sigmoid" and (sink is not None or slopes is not None or keep_first):
@@ -979,6 +983,8 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
     law = ((_dev(head_bias, "head_bias", torch.float32, (heads,)),) if law_name == "sigmoid" else
            (sp, _dev(slopes, "slopes", torch.float32, (heads,)), int(keep_first)) if law_name == "distance" else (sp,))
     po = pm = tp = None
+    if pieces is not None and tasks is not None:
+        raise KernelError("attention_mfma: pieces are dealt in rows mode")
     if tasks is not None:
         if item_tiles not in ((1, 2, 3, 4) if block_tiles == 32 else (1, 2)) or (item_tiles == 2 and dim > 64 and not block_tiles):
             raise KernelError("attention_mfma: two item tiles a wave need a head size of at most 64")
@@ -1008,7 +1014,13 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
         if row_ids is not None:
             n_tasks = row_ids.numel()
             tp = _dev(row_ids, "row_ids", torch.int32, (n_tasks,))
-        if splits > 1:
+        if pieces is not None:
+            firsts, n_tasks = pieces
+            splits = 1
+            if row_ids is not None or not merge:
+                raise KernelError("attention_mfma: pieces are dealt to all rows of a step and merged here")
+            tp = _dev(firsts, "pieces", torch.int32, (rows + 1,))
+        if splits > 1 or pieces is not None:
             if workspace is None:
                 raise KernelError("attention: split runs need a workspace")
             part_o, part_ml = workspace
@@ -1019,10 +1031,20 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
               _dev(vcache, "vcache", None, (pages, kv_heads, dim, page_size)), _dev(tables, "tables", torch.int32),
               tables.shape[1], tp, n_tasks, _dev(seg_of_row, "seg_of_row", torch.int32, (rows,)),
               _dev(positions, "positions", torch.int32, (rows,)), _dev(out, "out", None, (rows, heads * dim)), po, pm,
-              heads, kv_heads, dim, page_size.bit_length() - 1, int(window or 0), float(scale), int(splits),
-              11 if mode == 1 and stream_loads else mode, int(waves),
+              heads, kv_heads, dim, page_size.bit_length() - 1, int(window or 0), float(scale), rows if pieces is not None else int(splits),
+              (13 if pieces is not None else 1) + (0 if not stream_loads else 1 if pieces is not None else 10) if mode == 1 else mode, int(waves),
               int(mode == 1 and splits > 1 and not merge), _stream(), *law), "attention_mfma")
-    if mode == 1 and splits > 1 and merge:
+    if pieces is not None:
+        gp, ldg, vdim, into = None, 0, 0, out.data_ptr()
+        if merge_gate is not None:
+            gates, packed, vdim = merge_gate
+            gp, ldg = _rows_of(gates, "gates", heads * vdim)
+            if head_bias is not None or gates.shape[0] != rows or vdim > dim:
+                raise KernelError("attention_mfma: a gated merge is one of the softmax law over all rows")
+            into = _dev(packed, "packed", torch.bfloat16, (rows, heads * vdim))
+        _check(lib().cisr_attn_merge_pieces(po, pm, into, rows, heads, dim, tp, int(head_bias is not None), gp, ldg, int(vdim), _stream()),
+               "attention_merge")
+    elif mode == 1 and splits > 1 and merge:
         if merge_gate is not None:
             gates, packed, vdim = merge_gate
             gp, ldg = _rows_of(gates, "gates", heads * vdim)

@@ -40,7 +40,7 @@ class PagedAttention(Mixer):
         return kernel.kernel_units(self.head_dim, dtype)
 
     def step_arrays(self):
-        return [kernel.SingleRows(self.tuning.split_single_from), kernel.SingleTokens(), kernel.RowsLongestFirst()]
+        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.head_dim, self.window)
 
     def cache_need(self):
         return KVNeed(self.kv_heads, self.head_dim, self.window) if self.own_kv else None
@@ -192,7 +192,7 @@ class NormedGatedAttention(Mixer):
         return kernel.kernel_units(self.pad, dtype, "softmax" if self.slopes is None else "distance")
 
     def step_arrays(self):
-        return [kernel.SingleRows(self.tuning.split_single_from), kernel.SingleTokens(), kernel.RowsLongestFirst()]
+        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.pad, self.window, self.keep_first)
 
     def cache_need(self):
         if self.keep_first:
@@ -330,7 +330,7 @@ class LatentAttention(Mixer):
         return kernel.kernel_units(self.pad, dtype)
 
     def step_arrays(self):
-        return [kernel.SingleRows(self.tuning.split_single_from), kernel.SingleTokens(), kernel.RowsLongestFirst()]
+        return kernel.step_arrays(self.tuning, self.w_small, self.heads, 1, self.pad, self.window)
 
     def cache_need(self):
         return KVNeed(1, self.pad, self.window)
@@ -454,7 +454,7 @@ class SigmoidAttention(Mixer):
         return kernel.kernel_units(self.pad, dtype, "sigmoid")
 
     def step_arrays(self):
-        return [kernel.SingleRows(self.tuning.split_single_from), kernel.SingleTokens(), kernel.RowsLongestFirst()]
+        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.pad, self.window)
 
     def cache_need(self):
         return KVNeed(self.kv_heads, self.pad, self.keep) if self.own_kv else None
