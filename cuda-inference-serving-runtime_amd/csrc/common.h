@@ -30,6 +30,12 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
+// Where a sum over `units` pieces of a row of `of` (which matrix, which group of its rows) begins; it goes round from there.
+// Rows of a power of two in bytes lie on the same few memory channels at the same piece, and blocks that all begin at the
+// first piece ask the same channels for everything at once: 16 matrices of 2048 x 4096 bf16 in 67 us (3.7 TB/s), 42 with
+// beginnings spread over the row.
+__device__ __forceinline__ int first_unit(int matrix, int group, int units) { return (int)((unsigned)(group + 9 * matrix) % (unsigned)units); }
+
 __device__ __forceinline__ float load_f32(const float* p) { return *p; }
 __device__ __forceinline__ float load_f32(const bf16_t* p) { return bf16_to_f32(*p); }
 __device__ __forceinline__ void store_f32(float* p, float v) { *p = v; }

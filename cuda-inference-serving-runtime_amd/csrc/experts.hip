@@ -724,6 +724,7 @@ expert_gemm_mfma_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
     const int r = lane % 16, g = lane / 16;
     const int lr = tid / 8, lc = (tid % 8) * 8;               // this thread's chunks of a tile: rows lr + 32 i, first k
     const int n0 = column_block * EX_BN;
+    const int units = (K + EX_BK - 1) / EX_BK, begin = first_unit(e, column_block, units) * EX_BK;
     const bf16_t* ap[2 * MT];
     const bf16_t* wp[4];
 #pragma unroll
@@ -749,7 +750,7 @@ expert_gemm_mfma_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
     // is shorter than a trip to the L2); MT 2 has registers for one set, and more arithmetic a step
     u32x4 va0[2 * MT], vw0[4], va1[2 * MT], vw1[4];
     auto fetch = [&](int k0, u32x4 (&va)[2 * MT], u32x4 (&vw)[4]) {
-        const int k = k0 + lc;
+        const int at = k0 + begin, k = (at < units * EX_BK ? at : at - units * EX_BK) + lc;
 #pragma unroll
         for (int i = 0; i < 2 * MT; ++i) va[i] = (ap[i] && k < K) ? *(const u32x4*)(ap[i] + k) : zero;
 #pragma unroll

@@ -6,10 +6,10 @@
 // rows of the matrix, eight neighbouring lanes a row); the lanes that the matrix instruction wants them in get them through
 // LDS, in slots of the wave's own.  (Loaded in the instruction's layout, sixteen rows in neighbouring lanes, the cache serves
 // a load at a quarter of its rate.)  Rows past the tile's last pair are not loaded: 16, 32 or 64 rows are multiplied as the
-// tile needs.  A sum is one chain of matrix instructions over K in order, as in the other kernel: the same bits.
+// tile needs.  A sum is one chain of matrix instructions over K from `first_unit` on, as in the other kernel: the same bits.
 //
-// Measured on an MI355X, 16 experts of 4096 x 2048, 48 pairs: 64 us in tiles of 64 x 128 (two 64-deep steps of a block in
-// flight), 50 so (268 MB, 5.0 TB/s).
+// Measured on an MI355X, 16 experts, 48 pairs: matrices of 4096 x 2048 in 42 us (6.0 TB/s; 54 when every sum began at the first
+// unit, 52 in tiles of 64 x 128), of 2048 x 4096 in 42 (67 and 68).
 #include "common.h"
 
 #define EXF_TILE 64
@@ -45,6 +45,8 @@ __device__ __forceinline__ void few_tile(const FewArgs& p, int e, int tile, int 
     const int lrow = lane / 8, chunk = lane % 8;
     const int n0 = (blockIdx.y * EXF_WAVES + wave) * 16;
     if (n0 >= p.N) return;
+    const int begin = first_unit(e, n0 / (ACT == FEW_GATED ? 64 : 128), units);
+    auto place_of = [&](int u) { const int at = u + begin; return at < units ? at : at - units; };
     const bf16_t* We = p.W + (size_t)e * NT * p.N * K;
     const bf16_t* w_row[NT][2];
 #pragma unroll
@@ -69,7 +71,7 @@ __device__ __forceinline__ void few_tile(const FewArgs& p, int e, int tile, int 
         for (int j = 0; j < NT; ++j) acc[i][j] = (exf_f32x4){0.f, 0.f, 0.f, 0.f};
     exf_u32x4 fw[DEPTH][NT][2], fa[DEPTH][MT][2];
     auto ask = [&](int d, int u) {
-        const int k = min(min(u, units - 1) * 64 + 8 * chunk, K - 8);
+        const int k = min(place_of(min(u, units - 1)) * 64 + 8 * chunk, K - 8);
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -80,8 +82,9 @@ __device__ __forceinline__ void few_tile(const FewArgs& p, int e, int tile, int 
             for (int h = 0; h < 2; ++h) fa[d][i][h] = *(const exf_u32x4*)(a_row[i][h] + k);
     };
     auto use = [&](int d, int u) {
-        const bool tail = u * 64 + 64 > K;                            // (uniform: K's last, partly filled unit)
-        const uint32_t keep = !tail || u * 64 + 8 * chunk < K ? 0xffffffffu : 0u;
+        const int k0 = place_of(u) * 64;
+        const bool tail = k0 + 64 > K;                                // (uniform: K's last, partly filled unit)
+        const uint32_t keep = !tail || k0 + 8 * chunk < K ? 0xffffffffu : 0u;
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -142,13 +145,13 @@ __device__ __forceinline__ void few_tile(const FewArgs& p, int e, int tile, int 
 template <typename TC, int ACT>
 __global__ void __launch_bounds__(EXF_WAVES * WAVE)
 experts_few_kernel(FewArgs p) {
-    __shared__ exf_u32x4 lds[EXF_WAVES * 6 * 128];                    // (at most six pieces a wave: 12 KB)
+    __shared__ exf_u32x4 lds[EXF_WAVES * (ACT == FEW_GATED ? 6 : 5) * 128];   // (at most so many pieces a wave: 12 or 10 KB, sixteen blocks a compute unit)
     const int tile = blockIdx.x, e = p.tile_expert[tile];
     if (e < 0) return;
     // a tile's pairs come first, padding behind them
     const int places = __popcll(__ballot(p.pair_of_pos[tile * EXF_TILE + threadIdx.x % WAVE] >= 0));
     if (places <= 0) return;
-    if (places <= 16) few_tile<1, ACT == FEW_GATED ? 4 : 6, TC, ACT>(p, e, tile, places, lds);
+    if (places <= 16) few_tile<1, 4, TC, ACT>(p, e, tile, places, lds);
     else if (places <= 32) few_tile<2, ACT == FEW_GATED ? 3 : 4, TC, ACT>(p, e, tile, places, lds);
     else few_tile<4, 2, TC, ACT>(p, e, tile, places, lds);
 }

@@ -2286,19 +2286,19 @@ def experts_rows_gated(a, w, chosen, out, law, top=0):
     return out
 
 
-# A step's tiles stream the experts' matrices up to this many pairs an expert on the mean, and up to this inner size.  Measured
-# on an MI355X (the other kernel / the streaming one, us): 16 experts of 4096 x 2048, 48 pairs 64 / 50, 128 pairs 68 / 57, 256
-# pairs 69 / 61, 400 pairs 70 / 81; gated, of 2 x 1024 x 2048, 96 pairs 42 / 35, 512 pairs 45 / 38, 1,024 pairs 48 / 62; of
-# 2048 x 1024, 96 and 512 pairs 20 / 16 and 21 / 25; 64 experts of 1024 x 512, 256 pairs 16.6 / 17.1, 1,024 pairs 18 / 20.  With
-# an inner size of 4,096 a wave's stream is too long for the few waves there are: 48 pairs against 2048 x 4096 63 / 69.
-EXPERT_FEW_PAIRS, EXPERT_FEW_K = 8, 2048
+# A step's tiles stream the experts' matrices up to this many pairs an expert on the mean.  Measured on an MI355X (the other kernel /
+# the streaming one, us): 16 experts of 4096 x 2048, 48 pairs 52 / 42, 128 pairs 52 / 49, 256 pairs 52 / 58; of 2048 x 4096, results
+# by pair, 68 / 42, 68 / 47 and 70 / 59, 400 pairs 71 / 74; gated, of 2 x 1024 x 2048, 96 pairs 38 / 27, 512 pairs 40 / 34, 1,024
+# pairs 41 / 64; of 2048 x 1024, 96 pairs 23 / 16, 512 pairs 25 / 26; 64 experts of 1024 x 512, 96 pairs 17 / 14; 8 of 4096 x 14336,
+# 48 pairs 232 / 153, 256 pairs 242 / 262.
+EXPERT_FEW_PAIRS = 8
 
 
 def experts_few_ok(a, w, tiles):
     """Whether the experts' tiles run the kernel that streams the matrices (csrc/experts_few.hip): bf16 with 16-byte rows, and
     few pairs an expert.  (`tiles` = experts + pairs / 64 rounded up: a function of a captured program's rows.)"""
     experts, _, k = w.shape
-    return (experts_gemm_gated_ok(a, w) and 8 <= k <= EXPERT_FEW_K and EXPERT_TILE * (tiles - experts) <= EXPERT_FEW_PAIRS * experts)
+    return (experts_gemm_gated_ok(a, w) and k >= 8 and EXPERT_TILE * (tiles - experts) <= EXPERT_FEW_PAIRS * experts)
 
 
 def _experts_few(a, w, pair_of_pos, tile_expert, out, top, scatter, n, act, law=(0.0, 0.0, 0.0)):
