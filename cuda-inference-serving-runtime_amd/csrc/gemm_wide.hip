@@ -11,6 +11,10 @@
 //   - the work items (slice, unit), slice-major, are dealt to the blocks in equal contiguous runs, one block a
 //     compute unit; a block walks over its units of W, the loads of the next unit in flight while the matrix
 //     cores work on this one and the waves' partial tiles meet in LDS;
+//   - W comes in whole lines (eight rows a load, eight neighbouring lanes a row), non-temporally, and goes through LDS of
+//     the wave's own into the instruction's layout.  In that layout straight from memory, through the caches: us at 12
+//     rows before -> now: 28672 x 4096 gated 49.5 -> 42.3 (5.6 TB/s), 128256 x 4096 201 -> 175, 4096 x 14336 32.2 -> 27.0,
+//     49152 x 2048 40.7 -> 33.6;
 //   - with one slice the block finishes the result itself; with several, every slice writes its partial
 //     sums and a second small kernel adds them in slice order and finishes.
 // Sums are formed in a fixed order (waves in order inside a slice, slices in order), so a row's result
@@ -87,12 +91,18 @@ __device__ __forceinline__ void wide_finish(const WideArgs& p, int m, int n, flo
     else ((bf16_t*)p.C)[(size_t)m * p.ldc + n] = f32_to_bf16(v);
 }
 
+__device__ __forceinline__ void wide_wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // MT 16-row tiles of A; NW waves; SPW k-steps a wave and slice (even); NB blocks of W
 template <int MT, int NW, int SPW, int NB, bool ROPE>
 __global__ void __launch_bounds__(NW * 64)
 gemm_wide_kernel(WideArgs p) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     float (*red)[NB][MT][4][WAVE] = reinterpret_cast<float (*)[NB][MT][4][WAVE]>(smem);   // [wave][block][tile][e][lane]
+    u32x4* turn = reinterpret_cast<u32x4*>(smem + NW * NB * MT * 4 * WAVE);                 // [wave][2][block][16 rows][8 chunks]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;   // (uniform: scalar loop control)
     const int r = lane % 16, g = lane / 16;
     const int M = p.M, N = p.N, K = p.K;
@@ -130,14 +140,21 @@ gemm_wide_kernel(WideArgs p) {
                 af[j][t] = v;
             }
         }
+        // a lane's 16 bytes of a pair of steps of W: rows lane / 8 and 8 + lane / 8 of the unit, chunk lane % 8
+        int kline[SPW / 2];
+#pragma unroll
+        for (int j = 0; j < SPW / 2; ++j) kline[j] = min((wave + NW * (i0 + j)) * 64 + lane % 8 * 8, K - 8);
         auto load_w = [&](u32x4 (&w)[NB][SPW], int u) {
-            // rows past N are read again and never stored
-            const int n = ROPE ? wide_rope_row(p, u, r) : min(u * 16 + r, N - 1);
-            const bf16_t* row = p.W + (size_t)n * p.ldw;
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
+            for (int h = 0; h < 2; ++h) {
+                // rows past N are read again and never stored
+                const int n = ROPE ? wide_rope_row(p, u, 8 * h + lane / 8) : min(u * 16 + 8 * h + lane / 8, N - 1);
+                const bf16_t* row = p.W + (size_t)n * p.ldw;
 #pragma unroll
-                for (int j = 0; j < SPW; ++j) w[b][j] = *(const u32x4*)(row + (size_t)b * p.dual_off * p.ldw + koff[j]);
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int j = 0; j < SPW / 2; ++j) w[b][2 * j + h] = __builtin_nontemporal_load((const u32x4*)(row + (size_t)b * p.dual_off * p.ldw + kline[j]));
+            }
         };
         auto compute = [&](u32x4 (&w)[NB][SPW], int u) {
             f32x4 acc[NB][MT];
@@ -146,13 +163,28 @@ gemm_wide_kernel(WideArgs p) {
 #pragma unroll
                 for (int t = 0; t < MT; ++t) acc[b][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < SPW; ++j)
+            for (int j = 0; j < SPW; j += 2) {
+                // the pair's lines through the wave's own LDS into the instruction's layout (slots spread over the banks)
+                u32x4* mine = turn + (size_t)(wave * 2 + (j / 2) % 2) * NB * 128;
 #pragma unroll
-                for (int t = 0; t < MT; ++t)
+                for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int b = 0; b < NB; ++b)
-                        acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[j][t]),
-                                                                            __builtin_bit_cast(bf16x8, w[b][j]), acc[b][t], 0, 0, 0);
+                    for (int h = 0; h < 2; ++h) mine[b * 128 + 64 * h + (lane / 8) * 8 + ((lane % 8) ^ (lane / 8))] = w[b][j + h];
+                wide_wave_order();
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    u32x4 x[NB];
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) x[b] = mine[b * 128 + r * 8 + ((4 * ks + g) ^ (r % 8))];
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+#pragma unroll
+                        for (int b = 0; b < NB; ++b)
+                            acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[j + ks][t]),
+                                                                                __builtin_bit_cast(bf16x8, x[b]), acc[b][t], 0, 0, 0);
+                }
+                wide_wave_order();
+            }
             if (!first) __syncthreads();                          // every wave has read the sums of the unit before
             first = false;
 #pragma unroll
@@ -249,7 +281,7 @@ static int wide_launch(WideArgs a, size_t workspace_floats, bool plan_only, long
     if (partial > workspace_floats || (partial && !a.P) || (a.leave_partials && !partial)) return (int)hipErrorInvalidValue;
     const long long items = (long long)a.units * a.slices;
     const int cus = wide_cus();
-    const size_t shmem = (size_t)NW * NB * MT * 4 * WAVE * sizeof(float);
+    const size_t shmem = (size_t)NW * NB * (MT * 4 * WAVE * sizeof(float) + 2 * 16 * 128);
     if (shmem > 65536) {
         hipError_t e = hipFuncSetAttribute((const void*)gemm_wide_kernel<MT, NW, SPW, NB, ROPE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
