@@ -45,6 +45,15 @@ extern "C" int cisr_gemv_ok(int M, int N, int K) {
     return M <= gemv_rows && (long long)N * K * 2 >= gemv_bytes && (K >= gemv_inner || gemv_bytes == 0) && cisr_gemv_takes(M, K);
 }
 
+// Of the products that the matrix-vector kernel may take, those it is ahead on: the ones with the norm fused, and without, up to two
+// rows of gated ones and of long inner sizes (the kernels by lines cut those or have few blocks).  us of it / of the kernels by lines
+// (gemm_skinny.inc, gemm_wide.hip), 1 row: 8192 x 2048 9.9 / 7.5, 12352 x 2048 14.1 / 10.8, 4096 x 4096 9.1 / 8.1, 2048 x 2048 4.6 /
+// 4.3, 49152 x 2048 47 / 33, 16384 x 2048 gated 14.9 / 15.0, 2048 x 8192 8.5 / 11.4, 4096 x 14336 22 / 25; 4 rows: 41 / 25 for the last,
+// 12 / 12 for the one before, 16.5 / 15.3 gated; normed, 6144 x 4096, 1 row 12.3 / 18.3.
+extern "C" int cisr_gemv_ahead(int M, int N, int K, int norm, int gated) {
+    return cisr_gemv_ok(M, N, K) && (norm || gemv_bytes == 0 || (M <= 2 && (gated || K >= 3 * N)));
+}
+
 // Few rows against small weights with a narrow output: a block for every 16 columns would leave most compute
 // units idle, so the narrow kernels take over (a block for every 4 columns).  Measured on an MI355X in captured
 // chains: the down projection of the 135M sizes (8 rows, 576 x 1536) 4.3 us with 36 blocks of 16 columns.
@@ -99,7 +108,7 @@ static int skinny_entry(const void* A, int lda, const void* W, int ldw, void* C,
     a.A = A; a.lda = lda; a.W = (const bf16_t*)W; a.ldw = ldw; a.C = C; a.ldc = ldc; a.R = R; a.ldr = ldr;
     a.M = M; a.N = N; a.K = K; a.dual_off = dual_off; a.norm_w = norm_w; a.eps = eps; a.rows = rows; a.law = law; a.act = act;
     const int epi = dual_off > 0 ? EPI_SWIGLU : EPI_STORE;
-    if (cisr_gemv_ok(M, dual_off > 0 ? 2 * N : N, K)) return cisr_gemv_launch(a, N, norm_w != nullptr, epi, out_dtype, 0, stream);
+    if (cisr_gemv_ahead(M, dual_off > 0 ? 2 * N : N, K, norm_w != nullptr, dual_off > 0)) return cisr_gemv_launch(a, N, norm_w != nullptr, epi, out_dtype, 0, stream);
     if (narrow_wanted(M, dual_off > 0 ? 2 * N : N, K, norm_w != nullptr)) return launch_narrow(a, (N + 3) / 4, norm_w != nullptr, epi, out_dtype, stream);
     const int blocks = (N + 15) / 16;
     return launch_rows(a, blocks, norm_w != nullptr, epi, out_dtype, stream);
@@ -122,7 +131,7 @@ extern "C" int cisr_qkv_rope_skinny(const void* A, int lda, const void* W, int l
     a.positions = positions; a.slots = slots; a.cos_tab = cos_tab; a.sin_tab = sin_tab;
     a.kcache = (bf16_t*)kcache; a.vcache = (bf16_t*)vcache; a.heads = heads; a.kv_heads = kv_heads;
     a.head_dim = head_dim; a.page_size = page_size; a.max_pos = max_pos;
-    if (cisr_gemv_ok(M, a.N, K)) return cisr_gemv_launch(a, a.N / 2, norm_w != nullptr, EPI_ROPE, DT_BF16, 0, stream);
+    if (cisr_gemv_ahead(M, a.N, K, norm_w != nullptr, 0)) return cisr_gemv_launch(a, a.N / 2, norm_w != nullptr, EPI_ROPE, DT_BF16, 0, stream);
     if (narrow_wanted(M, a.N, K, norm_w != nullptr)) return launch_narrow(a, a.N / 4, norm_w != nullptr, EPI_ROPE, DT_BF16, stream);
     const int blocks = (heads + 2 * kv_heads) * (head_dim / 16);
     return launch_rows(a, blocks, norm_w != nullptr, EPI_ROPE, DT_BF16, stream);

@@ -122,6 +122,8 @@ def _declare(h):
     h.cisr_gemm_wide_workspace.restype = C.c_longlong
     h.cisr_gemv_ok.argtypes = [i, i, i]
     h.cisr_gemv_ok.restype = C.c_int
+    h.cisr_gemv_ahead.argtypes = [i, i, i, i, i]
+    h.cisr_gemv_ahead.restype = C.c_int
     h.cisr_gemv_set.argtypes = [i, ll]
     h.cisr_gemv_set.restype = None
 
@@ -669,7 +671,7 @@ def wide_ok(m, w, swiglu=False, after_norm=False):
     `after_norm`: the rows are the output of an RMSNorm, which the other kernel would fuse (it then reads the
     float residual and the norm's weights for every 16 rows of W, which costs it more than bf16 rows do)."""
     n, k = w.shape
-    if gemv_ok(m, n, k):   # up to four rows against large weights: the matrix-vector kernel takes them
+    if lib().cisr_gemv_ahead(int(m), int(n), int(k), int(after_norm), int(swiglu)):   # the matrix-vector kernel takes them
         return False
     least = WIDE_MIN_BYTES_FEW_ROWS if m <= 16 else WIDE_MIN_BYTES if m <= 32 else WIDE_MIN_BYTES_MANY_ROWS
     if m <= 16 and n < 16 * _compute_units(w.device) and k >= 4096:
@@ -690,8 +692,7 @@ GEMV_ROWS, GEMV_MIN_BYTES = 4, 4 << 20
 def gemv_ok(m, n, k):
     """Whether a product of m rows with weights [n, k] runs the matrix-vector kernel (up to four rows against weights
     of 4 MB and more with an inner size of at least 1024: a wave owns whole rows of the weights; see csrc/gemv.hip
-    and the measurements in csrc/gemm_skinny.hip).  The weight-streaming entry points choose it themselves; callers ask only to know that
-    the wide kernel and its separate norm are not wanted."""
+    and the measurements in csrc/gemm_skinny.hip).  The weight-streaming entry points choose it themselves, where it is ahead."""
     return bool(lib().cisr_gemv_ok(int(m), int(n), int(k)))
 
 
