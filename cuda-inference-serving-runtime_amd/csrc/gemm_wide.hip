@@ -96,7 +96,10 @@ __device__ __forceinline__ void wide_wave_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// MT 16-row tiles of A; NW waves; SPW k-steps a wave and slice (even); NB blocks of W
+// MT 16-row tiles of A; NW waves; SPW k-steps a wave and slice (even); NB blocks of W.  A wave's steps of a unit are loaded at once, or
+// where the registers hold only half of them (with A's) in two halves, each while the other is multiplied: longer slices, fewer
+// partial sums and second kernels.  us at 12 rows: 128256 x 4096 175 -> 161 (6.5 TB/s; it spilled), 28672 x 4096 gated 42.5 -> 40.7 (one
+// slice of K instead of two and a second kernel).
 template <int MT, int NW, int SPW, int NB, bool ROPE>
 __global__ void __launch_bounds__(NW * 64)
 gemm_wide_kernel(WideArgs p) {
@@ -109,6 +112,7 @@ gemm_wide_kernel(WideArgs p) {
     constexpr int TSTEP = NW / 4;                                 // NW is a multiple of 4
     constexpr int TPW = (MT + TSTEP - 1) / TSTEP;                 // tiles a wave finishes
     const int e2 = wave % 4, t2 = wave / 4;
+    constexpr int HALVES = SPW * NW >= 128 || SPW * MT >= 32 ? 2 : 1, CW = SPW / HALVES;      // steps that are loaded at once
     bool first = true;
 
     // this block's run of work items; item i is unit i % units of slice i / units
@@ -144,7 +148,7 @@ gemm_wide_kernel(WideArgs p) {
         int kline[SPW / 2];
 #pragma unroll
         for (int j = 0; j < SPW / 2; ++j) kline[j] = min((wave + NW * (i0 + j)) * 64 + lane % 8 * 8, K - 8);
-        auto load_w = [&](u32x4 (&w)[NB][SPW], int u) {
+        auto load_w = [&](u32x4 (&w)[NB][CW], int u, int half) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 // rows past N are read again and never stored
@@ -153,17 +157,19 @@ gemm_wide_kernel(WideArgs p) {
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int j = 0; j < SPW / 2; ++j) w[b][2 * j + h] = __builtin_nontemporal_load((const u32x4*)(row + (size_t)b * p.dual_off * p.ldw + kline[j]));
+                    for (int j = 0; j < CW / 2; ++j)
+                        w[b][2 * j + h] = __builtin_nontemporal_load((const u32x4*)(row + (size_t)b * p.dual_off * p.ldw + kline[half * (CW / 2) + j]));
             }
         };
-        auto compute = [&](u32x4 (&w)[NB][SPW], int u) {
-            f32x4 acc[NB][MT];
+        f32x4 acc[NB][MT];
+        auto compute = [&](u32x4 (&w)[NB][CW], int u, int half) {
+            if (half == 0)
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
+                for (int b = 0; b < NB; ++b)
 #pragma unroll
-                for (int t = 0; t < MT; ++t) acc[b][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                    for (int t = 0; t < MT; ++t) acc[b][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < SPW; j += 2) {
+            for (int j = 0; j < CW; j += 2) {
                 // the pair's lines through the wave's own LDS into the instruction's layout (slots spread over the banks)
                 u32x4* mine = turn + (size_t)(wave * 2 + (j / 2) % 2) * NB * 128;
 #pragma unroll
@@ -180,11 +186,12 @@ gemm_wide_kernel(WideArgs p) {
                     for (int t = 0; t < MT; ++t)
 #pragma unroll
                         for (int b = 0; b < NB; ++b)
-                            acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[j + ks][t]),
+                            acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[half * CW + j + ks][t]),
                                                                                 __builtin_bit_cast(bf16x8, x[b]), acc[b][t], 0, 0, 0);
                 }
                 wide_wave_order();
             }
+            if (half < HALVES - 1) return;
             if (!first) __syncthreads();                          // every wave has read the sums of the unit before
             first = false;
 #pragma unroll
@@ -222,14 +229,23 @@ gemm_wide_kernel(WideArgs p) {
                 }
             }
         };
-        u32x4 wa[NB][SPW], wb[NB][SPW];
-        load_w(wa, u0);
-        for (int u = u0; u < u1; u += 2) {                        // u0 < u1; the bounds are uniform over the block
-            if (u + 1 < u1) load_w(wb, u + 1);
-            compute(wa, u);
-            if (u + 1 < u1) {
-                if (u + 2 < u1) load_w(wa, u + 2);
-                compute(wb, u + 1);
+        u32x4 wa[NB][CW], wb[NB][CW];
+        load_w(wa, u0, 0);
+        if constexpr (HALVES == 2) {
+            for (int u = u0; u < u1; ++u) {
+                load_w(wb, u, 1);
+                compute(wa, u, 0);
+                if (u + 1 < u1) load_w(wa, u + 1, 0);
+                compute(wb, u, 1);
+            }
+        } else {
+            for (int u = u0; u < u1; u += 2) {                    // u0 < u1; the bounds are uniform over the block
+                if (u + 1 < u1) load_w(wb, u + 1, 0);
+                compute(wa, u, 0);
+                if (u + 1 < u1) {
+                    if (u + 2 < u1) load_w(wa, u + 2, 0);
+                    compute(wb, u + 1, 0);
+                }
             }
         }
     }
@@ -296,20 +312,19 @@ static int wide_launch(WideArgs a, size_t workspace_floats, bool plan_only, long
     return CISR_LAUNCH_CHECK();
 }
 
-// Rounds a slice (SPW / 2), by a model of the busiest block's time fitted to measurements on an MI355X (it picks
-// the fastest of 1, 2, 4 rounds in 27 of 30 products of the 135M, 1.7B and 8B sizes at 8, 32 and 64 rows, and is
-// within 3 % of it in the others).  In units of a round (every block streams NW * 2 KB of each block of W, at
-// about 5 TB/s over the whole GPU):
+// Rounds a slice (SPW / 2), by a model of the busiest block's time fitted to measurements on an MI355X (sixty products of the
+// 1.7B, 8B and Ditazen sizes at 8 to 64 rows: 0.4 % slower than the fastest of 1, 2, 4, 8 rounds on the mean, 9 % at worst).  In
+// units of a round (every block streams NW * 2 KB of each block of W, at 6.5 TB/s over the whole GPU):
 //   items of the block x (rounds a slice + the fixed cost of a unit: barriers and the sums through LDS)
-//   + the activations of each slice the run touches (rows / 16 of a round of W for each of its rounds)
+//   + the activations of each slice the run touches (half of rows / 16 of a round of W for each of its rounds)
 //   + half a slice more for a block with a single unit (nothing overlaps its loads)
-//   + with several slices: the second kernel, and the partial sums written and read once.
+//   + with several slices: the second kernel (5 us), and the partial sums written and read once.
 // The rounds of a last slice past K are loaded from clamped addresses and add nothing, but cost like the others.
 template <int MT, int NW, int MAXSPW, int NB, bool ROPE>
 static int wide_steps(const WideArgs& a, size_t workspace_floats, bool plan_only, long long* need, hipStream_t stream) {
     const int pairs = (a.K + 63) / 64, rounds = (pairs + NW - 1) / NW, cus = wide_cus();
-    const double round_us = (double)NW * 2048.0 * NB * cus / 5e12 * 1e6;
-    const double unit_cost = 0.4 / round_us, second_kernel = 4.0 / round_us;
+    const double round_us = (double)NW * 2048.0 * NB * cus / 6.5e12 * 1e6;
+    const double unit_cost = 0.1 / round_us, second_kernel = 5.0 / round_us;
     const int rows = a.M < 16 * MT ? a.M : 16 * MT;
     int best = 1;
     double best_cost = -1.0;
@@ -317,11 +332,12 @@ static int wide_steps(const WideArgs& a, size_t workspace_floats, bool plan_only
         const int slices = (rounds + r - 1) / r;
         const long long items = (long long)a.units * slices;
         const long long run = (items + cus - 1) / cus;
-        double cost = (double)run * (r + unit_cost) + (double)((run + a.units - 1) / a.units) * rows / 16.0 * r / NB;
+        double cost = (double)run * (r + unit_cost) + 0.5 * (double)((run + a.units - 1) / a.units) * rows / 16.0 * r / NB;
         if (run == 1) cost += 0.5 * r;
-        if (slices > 1) cost += second_kernel + 0.1 * slices + (double)slices * a.M * a.N * 8.0 / ((double)NW * 2048.0 * cus);
+        if (slices > 1) cost += second_kernel + 0.1 * slices + (double)slices * a.M * a.N * NB * 4.0 / ((double)NW * 2048.0 * cus);
         if (best_cost < 0 || cost < best_cost) { best = r; best_cost = cost; }
     }
+    if constexpr (MAXSPW >= 16) if (best == 8) return wide_launch<MT, NW, 16, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
     if constexpr (MAXSPW >= 8) if (best == 4) return wide_launch<MT, NW, 8, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
     if constexpr (MAXSPW >= 4) if (best >= 2) return wide_launch<MT, NW, 4, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
     return wide_launch<MT, NW, 2, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
@@ -342,7 +358,7 @@ static int wide_dispatch(const WideArgs& a, size_t workspace_floats, bool plan_o
         }
     } else {
         switch (mt) {
-            case 1: return wide_steps<1, 8, 8, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
+            case 1: return wide_steps<1, 8, 16, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
             case 2: return wide_steps<2, 8, 4, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
             case 3: return wide_steps<3, 8, 4, NB, ROPE>(a, workspace_floats, plan_only, need, stream);
             default: return wide_steps<4, 8, 4, NB, ROPE>(a, workspace_floats, plan_only, need, stream);

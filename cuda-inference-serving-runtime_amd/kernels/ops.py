@@ -656,11 +656,12 @@ def gemm(a, w, out, residual=None, after_norm=False, scratch=None):
 
 # Weights of at least this many bytes are streamed by the kernel that keeps the activations in registers
 # (norm, rotary embedding and cache write are then kernels of their own); smaller ones by the kernels that
-# fuse them, which cost fewer launches.  Measured on an MI355X against the other kernel in captured graphs:
-# with at most 16 rows the activations are a small part of the traffic and the fused kernels hold out up to
-# about 64 MB; with 17 to 32 rows the wide kernel wins from about 12 MB on, with more from about 30 MB on
-# (a block then holds so much of the activations that it needs many rows of W to spread their cost over).
+# fuse them, which cost fewer launches.  us of the other kernel / the wide one on an MI355X, without a norm: 6144 x 4096 13.5 / 12.4
+# at 8 rows, 16.1 / 12.8 at 16; 4096 x 4096 8.6 / 8.8 and 9.8 / 9.2; 12352 x 2048 11.2 / 12.1 and 13.6 / 12.2; 6144 x 2048 7.6 / 8.2
+# and 8.9 / 8.0; at 32 rows 6144 x 2048 11.6 / 9.8, 3072 x 2048 8.0 / 9.1; with more rows from about 30 MB on (a block then
+# holds so much of the activations that it needs many rows of W to spread their cost over).
 WIDE_MIN_BYTES_FEW_ROWS = 64 << 20
+WIDE_MIN_BYTES_LONG = 24 << 20      # more than 8 rows, or an inner size of 4,096 and more
 WIDE_MIN_BYTES = 12 << 20
 WIDE_MIN_BYTES_MANY_ROWS = 30 << 20
 _wide_plans = {}
@@ -674,6 +675,8 @@ def wide_ok(m, w, swiglu=False, after_norm=False):
     if lib().cisr_gemv_ahead(int(m), int(n), int(k), int(after_norm), int(swiglu)):   # the matrix-vector kernel takes them
         return False
     least = WIDE_MIN_BYTES_FEW_ROWS if m <= 16 else WIDE_MIN_BYTES if m <= 32 else WIDE_MIN_BYTES_MANY_ROWS
+    if 4 < m <= 16 and not after_norm and (m > 8 or k >= 4096):
+        least = min(least, WIDE_MIN_BYTES_LONG)
     if m <= 16 and n < 16 * _compute_units(w.device) and k >= 4096:
         # a narrow output with a long inner size: the fused kernels have a block for every 16 columns and
         # cannot fill the GPU; this one cuts K as well
