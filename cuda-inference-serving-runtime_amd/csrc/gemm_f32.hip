@@ -16,6 +16,12 @@
 // 4.6 / 7.8, 3072 x 576 60 / 58 / 61 -> 4.2 / 5.1 / 13.4, 576 x 1536 158 / 152 / 170 -> 5.7 / 7.1 / 14.7; the head of two
 // rows, 49152 x 576, 94 -> 28 (4.0 TB/s); 2,048 rows against 8192 x 2048 1,797 -> 786 (87 of 157 TFLOP/s).  Relative error
 // against 64 bits 4.3e-7 -> 1.6e-7 (K = 576), 8.1e-7 -> 2.1e-7 (K = 2,048): K's runs are sums of their own.
+//
+// GATED and ROTARY products make two rows of W a column, the gate's and the up's or a rotary pair's two halves: half of a tile's sixteens
+// (in tiles of one sixteen, half of its rows) are the first rows, the others the second, and the wave that finishes a sixteen
+// holds both sums.  The activation, or the rotation
+// with the keys' and values' way into their pages, is then no kernel of its own (2 rows at 576 x 3072 / 960: 2.1 and 3.2 us a layer and
+// two gaps between kernels of about 1.5; 130 rows 4.7 and 4.9).
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
@@ -25,9 +31,14 @@ struct GemmF32Args {
     const float* W; int ldw;
     float* C; int ldc;
     const float* R; int ldr;         // residual added at the end, or null; may be C
-    int M, N, K;
+    int M, N, K;                     // N: columns of the product, or of the first rows (GATED), or pairs (ROTARY)
     int m_tiles;
+    // ROTARY: W = [Wq; Wk; Wv], C the queries; pair i of a head is coordinates (i, i + dim / 2)
+    const int* positions; const int* slots; const float* cos_tab; const float* sin_tab;
+    float* kcache; float* vcache;
+    int heads, kv_heads, dim, page_size, max_pos;
 };
+enum { F32_PLAIN = 0, F32_GATED = 1, F32_ROTARY = 2 };
 
 // Four floats of row `row` at k; VEC: one 16-byte load, rows 16-byte aligned and K a multiple of 4.  Addresses are
 // clamped, never branched around; what lies past K is cleared by `clear_tail`.
@@ -53,12 +64,42 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-template <int TM, int TN, int WK, int DEPTH, bool VEC>
+// The pair (a, b) of row m, pair n (of all heads' pairs), turned by the angle (c, s): queries to C, keys and values to `slot`.
+__device__ __forceinline__ void finish_pair(const GemmF32Args& p, int m, int n, float a, float b, float c, float s, int slot) {
+    const int half = p.dim / 2, head = n / half, i = n % half;
+    if (head < p.heads + p.kv_heads) {
+        const float x = fmaf(a, c, -(b * s));         // (as the rotary kernel's sums are contracted: the same bits)
+        b = fmaf(b, c, a * s);
+        a = x;
+    }
+    if (head < p.heads) {
+        float* q = p.C + (size_t)m * p.ldc + head * p.dim + i;
+        q[0] = a;
+        q[half] = b;
+        return;
+    }
+    if (slot < 0) return;
+    const int page = slot / p.page_size, off = slot % p.page_size;
+    if (head < p.heads + p.kv_heads) {
+        float* k = p.kcache + (((size_t)page * p.kv_heads + head - p.heads) * p.page_size + off) * p.dim + i;
+        k[0] = a;
+        k[half] = b;
+    } else {
+        float* v = p.vcache + (((size_t)page * p.kv_heads + head - p.heads - p.kv_heads) * p.dim + i) * p.page_size + off;
+        v[0] = a;
+        v[(size_t)half * p.page_size] = b;
+    }
+}
+
+template <int TM, int TN, int WK, int DEPTH, bool VEC, int FORM = F32_PLAIN>
 __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
     extern __shared__ __attribute__((aligned(16))) char gf_lds[];
+    constexpr bool HALVES = FORM != F32_PLAIN && TN == 1;            // the sixteen's first eight rows of W and its last
+    constexpr int OT = FORM == F32_PLAIN || HALVES ? TN : TN / 2;    // sixteens of columns (eights with HALVES)
+    constexpr int OC = HALVES ? 8 : 16;
     gf_f32x4* meet = (gf_f32x4*)gf_lds;                              // [WK][TM * TN][64], after the waves are through
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, r = lane % 16, g = lane / 16;
-    const int m0 = (blockIdx.x % p.m_tiles) * TM * 16, n0 = (blockIdx.x / p.m_tiles) * TN * 16;   // (neighbours share rows of W)
+    const int m0 = (blockIdx.x % p.m_tiles) * TM * 16, n0 = (blockIdx.x / p.m_tiles) * OT * OC;   // (neighbours share rows of W)
     const int K = p.K, sixteens = (K + 15) / 16;
     const int first = (int)((long long)sixteens * wave / WK), last = (int)((long long)sixteens * (wave + 1) / WK);
     // Neighbouring lanes load neighbouring words of a row (lane: row lane / 4, four k from 4 (lane % 4)); the instruction wants
@@ -72,7 +113,12 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) a_row[i] = p.A + (size_t)min(m0 + i * 16 + lrow, p.M - 1) * p.lda;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) w_row[j] = p.W + (size_t)min(n0 + j * 16 + lrow, p.N - 1) * p.ldw;
+    for (int j = 0; j < TN; ++j) {
+        const int n = min(n0 + j % OT * OC + lrow % OC, p.N - 1), half = p.dim / 2;
+        const bool second = HALVES ? lrow >= 8 : j >= OT;
+        const int row = FORM == F32_PLAIN ? n : FORM == F32_GATED ? n + (second ? p.N : 0) : n / half * p.dim + n % half + (second ? half : 0);
+        w_row[j] = p.W + (size_t)row * p.ldw;
+    }
     gf_f32x4 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -113,10 +159,30 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
                 for (int j = 0; j < TN; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[i][e], xw[j][e], acc[i][j], 0, 0, 0);
     };
+    const int t = tid / WAVE, i = t / OT, j = t % OT;                // (the first TM OT waves finish a sixteen by sixteen each)
+    static_assert(TM * OT <= WK, "a wave finishes at most one sixteen by sixteen");
+    const bool finishes = t < TM * OT;
+    const int n = n0 + j * OC + r % OC, m = m0 + i * 16 + 4 * g;
+    // (the rows' positions are asked for before the operands and the angles behind the first of them, not at the end)
+    int pos[4] = {0, 0, 0, 0}, slot[4] = {-1, -1, -1, -1};
+    float turn_c[4] = {1.f, 1.f, 1.f, 1.f}, turn_s[4] = {0.f, 0.f, 0.f, 0.f};
+    if (FORM == F32_ROTARY && finishes)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pos[e] = p.positions[min(m + e, p.M - 1)];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
         ask(d, first + d);
         __builtin_amdgcn_sched_barrier(0);
+    }
+    if (FORM == F32_ROTARY && finishes) {
+        const int half = p.dim / 2, angle = min(n, p.N - 1) % half;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const size_t at = (size_t)min(max(pos[e], 0), p.max_pos - 1) * half + angle;
+            turn_c[e] = p.cos_tab[at];
+            turn_s[e] = p.sin_tab[at];
+            if (p.kv_heads > 0) slot[e] = p.slots[min(m + e, p.M - 1)];
+        }
     }
     // whole turns ask for the turn behind them (past the last sixteen: that one again, so that every wait counts the same
     // loads); the last turn asks for nothing: a wave with up to DEPTH sixteens is one trip to memory
@@ -134,10 +200,6 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
         if (turn + d < last) use(d, turn + d);                       // (uniform over the wave)
     // element 4 g + e of a lane's four is row 4 g + e, column r of its sixteen by sixteen
     constexpr int ITEMS = TM * TN * WAVE;
-    const int t = tid / WAVE, i = t / TN, j = t % TN;                // (the first TM TN waves finish a sixteen by sixteen each)
-    static_assert(TM * TN <= WK, "a wave finishes at most one sixteen by sixteen");
-    const bool finishes = t < TM * TN;
-    const int n = n0 + j * 16 + r, m = m0 + i * 16 + 4 * g;
     float resid[4] = {0.f, 0.f, 0.f, 0.f};
     if (finishes && p.R && n < p.N)
 #pragma unroll
@@ -148,30 +210,51 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
         for (int jj = 0; jj < TN; ++jj) meet[(wave * TM * TN + ii * TN + jj) * WAVE + lane] = acc[ii][jj];
     __syncthreads();
-    if (!finishes || n >= p.N) return;
-    gf_f32x4 part[WK];
+    if (!finishes || (!HALVES && n >= p.N)) return;
+    auto total = [&](int tile) {
+        gf_f32x4 part[WK];
 #pragma unroll
-    for (int w = 0; w < WK; ++w) part[w] = meet[w * ITEMS + tid];
+        for (int w = 0; w < WK; ++w) part[w] = meet[w * ITEMS + tile * WAVE + lane];
 #pragma unroll
-    for (int half = WK / 2; half > 0; half /= 2)
+        for (int half = WK / 2; half > 0; half /= 2)
 #pragma unroll
-        for (int w = 0; w < half; ++w) part[w] += part[w + half];
+            for (int w = 0; w < half; ++w) part[w] += part[w + half];
+        return part[0];
+    };
+    const gf_f32x4 sum = total(i * TN + j);
+    if constexpr (FORM == F32_PLAIN) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (m + e < p.M) p.C[(size_t)(m + e) * p.ldc + n] = part[0][e] + resid[e];
+        for (int e = 0; e < 4; ++e)
+            if (m + e < p.M) p.C[(size_t)(m + e) * p.ldc + n] = sum[e] + resid[e];
+    } else {
+        gf_f32x4 second;
+        if constexpr (HALVES) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) second[e] = __shfl_xor(sum[e], 8, WAVE);
+        } else {
+            second = total(i * TN + OT + j);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (m + e >= p.M || (HALVES && (r >= 8 || n >= p.N))) continue;
+            if constexpr (FORM == F32_GATED) p.C[(size_t)(m + e) * p.ldc + n] = sum[e] / (1.0f + expf(-sum[e])) * second[e];
+            else finish_pair(p, m + e, n, sum[e], second[e], turn_c[e], turn_s[e], slot[e]);
+        }
+    }
 }
 
-template <int TM, int TN, int WK, int DEPTH, bool VEC>
+template <int TM, int TN, int WK, int DEPTH, bool VEC, int FORM = F32_PLAIN>
 static int launch_f32(GemmF32Args p, hipStream_t stream) {
+    constexpr int COLUMNS = FORM == F32_PLAIN ? 16 * TN : 8 * TN;
     p.m_tiles = (p.M + 16 * TM - 1) / (16 * TM);
-    const long long blocks = (long long)p.m_tiles * ((p.N + 16 * TN - 1) / (16 * TN));
+    const long long blocks = (long long)p.m_tiles * ((p.N + COLUMNS - 1) / COLUMNS);
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
     constexpr int lds = WK * (TM * TN > TM + TN ? TM * TN : TM + TN) * WAVE * (int)sizeof(gf_f32x4);
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_kernel<TM, TN, WK, DEPTH, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        const hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_kernel<TM, TN, WK, DEPTH, VEC, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return (int)e;
     }
-    gemm_f32_kernel<TM, TN, WK, DEPTH, VEC><<<(unsigned)blocks, WK * WAVE, lds, stream>>>(p);
+    gemm_f32_kernel<TM, TN, WK, DEPTH, VEC, FORM><<<(unsigned)blocks, WK * WAVE, lds, stream>>>(p);
     return CISR_LAUNCH_CHECK();
 }
 
@@ -183,6 +266,42 @@ static int launch_f32_tile(const GemmF32Args& p, hipStream_t stream) {
     if (p.M > 16 && m32 * n64 >= 512) return launch_f32<2, 4, WK, 2, VEC>(p, stream);
     if (p.M > 16 && m32 * n32 >= 64) return launch_f32<2, 2, WK, 4, VEC>(p, stream);
     return launch_f32<1, 1, WK, 8, VEC>(p, stream);
+}
+
+// The same with two rows of W a column.
+template <int WK, bool VEC, int FORM>
+static int launch_f32_pairs(const GemmF32Args& p, hipStream_t stream) {
+    const long long m32 = (p.M + 31) / 32, n32 = (p.N + 15) / 16, n64 = (p.N + 31) / 32;
+    if (p.M > 16 && m32 * n64 >= 512) return launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+    if (p.M > 16 && m32 * n32 >= 64) return launch_f32<2, 2, WK, 4, VEC, FORM>(p, stream);
+    return launch_f32<1, 1, WK, 8, VEC, FORM>(p, stream);
+}
+template <int FORM>
+static int launch_f32_pairs(const GemmF32Args& p, hipStream_t stream) {
+    const bool vec = p.K % 4 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0 && (uintptr_t)p.A % 16 == 0 && (uintptr_t)p.W % 16 == 0;
+    if (p.K >= 1024) return vec ? launch_f32_pairs<16, true, FORM>(p, stream) : launch_f32_pairs<16, false, FORM>(p, stream);
+    return vec ? launch_f32_pairs<8, true, FORM>(p, stream) : launch_f32_pairs<8, false, FORM>(p, stream);
+}
+
+// C[M, N] = silu(A . Wg^T) * (A . Wu^T) with W = [Wg; Wu], 2 N rows
+extern "C" int cisr_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0) return (int)hipErrorInvalidValue;
+    GemmF32Args p{A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, 0};
+    return launch_f32_pairs<F32_GATED>(p, stream);
+}
+
+// W = [Wq; Wk; Wv] (kv_heads 0: Wq alone): queries and keys turned over the whole head by the rows' positions, queries to C, keys
+// and values to the pages at `slots`
+extern "C" int cisr_gemm_f32_rope(const float* A, int lda, const float* W, int ldw, float* q_out, int ldq, int M, int K, const int* positions,
+                                  const int* slots, const float* cos_tab, const float* sin_tab, float* kcache, float* vcache, int heads,
+                                  int kv_heads, int dim, int page_size, int max_pos, hipStream_t stream) {
+    if (M <= 0 || heads <= 0) return 0;
+    if (K <= 0 || dim <= 0 || dim % 2 || kv_heads < 0 || page_size <= 0 || max_pos <= 0 || !positions || (kv_heads && (!slots || !kcache || !vcache)))
+        return (int)hipErrorInvalidValue;
+    GemmF32Args p{A, lda, W, ldw, q_out, ldq, nullptr, 0, M, (heads + 2 * kv_heads) * dim / 2, K, 0,
+                  positions, slots, cos_tab, sin_tab, kcache, vcache, heads, kv_heads, dim, page_size, max_pos};
+    return launch_f32_pairs<F32_ROTARY>(p, stream);
 }
 
 // Waves a tile: sixteen from an inner size of 1,024 on, else eight (so that a wave has at least two sixteens at the small

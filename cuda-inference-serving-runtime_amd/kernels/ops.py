@@ -50,6 +50,8 @@ def _declare(h):
         "cisr_bias_add": [p, p, ll, i, i, i, p],
         "cisr_attn_rowwise": [p, i, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f, i, i, p, p, i, p],
         "cisr_gemm_f32": [p, i, p, i, p, i, p, i, i, i, i, p],
+        "cisr_gemm_f32_swiglu": [p, i, p, i, p, i, i, i, i, p],
+        "cisr_gemm_f32_rope": [p, i, p, i, p, i, i, i, p, p, p, p, p, p, i, i, i, i, i, p],
         "cisr_gemm_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_bf16_swiglu": [p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_bf16_tile": [p, i, p, i, p, i, p, i, i, i, i, i, i, p],
@@ -878,6 +880,10 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         return out
     if gate_up is None:
         raise KernelError("gemm_swiglu: this shape needs a buffer [M, 2I] for the product of gate and up")
+    if a.dtype == torch.float32 and law is None and w_gate_up.is_cuda and w_gate_up.stride(1) == 1 and a.is_cuda and a.stride(1) == 1:
+        _check(lib().cisr_gemm_f32_swiglu(a.data_ptr(), a.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), _dev(out, "out"), out.stride(0),
+                                          m, inter, k, _stream()), "gemm_swiglu")
+        return out
     gemm(a, w_gate_up, gate_up, scratch=scratch)
     return activate(gate_up, out)
 
@@ -893,11 +899,37 @@ def qkv_rope_fused_ok(a, w, head_dim, cos, normed):
             and a.dtype == (torch.float32 if normed else torch.bfloat16))
 
 
+def qkv_rope_f32_ok(a, w, head_dim, cos):
+    """Whether qkv_rope takes these operands as the 32-bit product with the rotation as its epilogue."""
+    return (a.is_cuda and w.is_cuda and a.dtype == torch.float32 and w.dtype == torch.float32 and a.dim() == 2 and a.stride(1) == 1
+            and w.stride(1) == 1 and head_dim % 2 == 0 and 2 * cos.shape[1] == head_dim and 0 < a.shape[0])
+
+
+def _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size):
+    m, k = a.shape
+    kp = vp = sp = None
+    if kcache is not None:
+        pages = kcache.shape[0]
+        kp = _dev(kcache, "kcache", torch.float32, (pages, kv_heads, page_size, dim))
+        vp = _dev(vcache, "vcache", torch.float32, (pages, kv_heads, dim, page_size))
+        sp = _dev(slots, "slots", torch.int32, (m,))
+    n_kv, max_pos = (kv_heads if kcache is not None else 0), cos.shape[0]
+    if tuple(w.shape) != ((heads + 2 * n_kv) * dim, k):
+        raise KernelError("qkv_rope: shapes do not fit")
+    _check(lib().cisr_gemm_f32_rope(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), _dev(q_out, "q_out", torch.float32, (m, heads * dim)),
+                                    heads * dim, m, k, _dev(positions, "positions", torch.int32, (m,)), sp, _dev(cos, "cos", torch.float32),
+                                    _dev(sin, "sin", torch.float32, (max_pos, dim // 2)), kp, vp, heads, n_kv, dim, page_size, max_pos,
+                                    _stream()), "qkv_rope")
+    return q_out
+
+
 def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm=None, scratch=None):
     """One kernel for a decode step's projections: (RMSNorm of the float residual `a` if `norm` = (weight, eps),
     else `a` is bf16 and normed), product with w = [Wq; Wk; Wv], rotary embedding of q and k, q into
     q_out [M, heads*dim], k and v into the cache at `slots`.  kcache None: w = Wq only (a layer reading
     another layer's cache)."""
+    if norm is None and qkv_rope_f32_ok(a, w, dim, cos):
+        return _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size)
     m, k = a.shape
     has_kv = kcache is not None
     n_kv = kv_heads if has_kv else 0

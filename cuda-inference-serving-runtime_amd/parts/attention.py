@@ -83,7 +83,9 @@ class PagedAttention(Mixer):
     def _fused_projection_ok(self, a, normed):
         cos, _ = self.position.tables()
         # (the fused kernels turn split-half pairs only; another pairing takes the general rotary kernel)
-        return not self._interleaved and not self.bias and ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed)
+        if self._interleaved or self.bias:
+            return False
+        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
 
     def fuses_norm(self, norm, residual, ctx):
         return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True)
@@ -99,7 +101,7 @@ class PagedAttention(Mixer):
         else:
             kcache_w, vcache_w, slots = kcache, vcache, view.slots
         if norm is not None or self._fused_projection_ok(h, False):
-            # few rows: norm, projections, rotary embedding and the cache write are one kernel
+            # few rows (in 32 bits any): norm, projections, rotary embedding and the cache write are one kernel
             q, q_stride = ctx.buffer("attn.q", (T, nh * D), ctx.dtype), nh * D
             ops.qkv_rope(residual if norm is not None else h, self.w_in, q, ctx.positions, slots, cos, sin,
                          kcache_w, vcache_w, nh, nkv, D, view.page_size,
