@@ -390,11 +390,11 @@ def rows_room(blocks, span, waves, splits, head_dim):
     """Whether a decode step that `rows_launch` gives (waves, splits) deals its blocks to the rows by their lengths, and how:
     (wavefronts a block, blocks that the launch has room for, least 32-key steps a wave), or None: unsplit.
     The launch is filled once: 512 blocks of four waves (256 with more than 128 coordinates, where a compute unit holds one),
-    256 of eight, 768 of four with small heads, 1,024 where runs are long.  us of a step of rows between 0.4 and 1.6 times a mean, equal
+    256 of eight, 768 of four with small heads, twice where runs are long.  us of a step of rows between 0.4 and 1.6 times a mean, equal
     splits -> by pieces: 32 heads of 128 over 8, 12 rows of 5,000 keys 76 -> 53, 24 of 3,000 93 -> 62, 3 of 700 11.1 -> 10.9, one of 30,000
-    among eight of 500 125 -> 40; 9 of 64 over 3, 100 rows of 1,500 37 -> 30, 64 of 7,000 75 -> 64; one key head of 256, 24 rows of 2,000
+    among eight of 500 125 -> 40; 9 of 64 over 3, 100 rows of 1,500 37 -> 30, 64 of 7,000 75 -> 65, 64 of 24,000 239 -> 196; one key head of 256, 24 rows of 2,000
     44 -> 24.  Rows of one length, where only a merge that looks its parts up is added: 8 rows of 5,000 keys 36.2 -> 36.8, 16 of
-    2,000 31.9 -> 31.7.
+    2,000 31.9 -> 31.7; 9 of 64 over 3, 64 of 8,000 69 -> 71, 64 of 32,100 259 -> 256, 32 of 9,000 44 -> 48.
     Small heads of many rows that are not split otherwise are, from 4,096 keys on: 32 heads of 64, 12 rows of 2,000 47 -> 41, 16 of
     4,500 112 -> 100, 16 and 32 of 2,100 keys each 49 -> 50 and 93 -> 92; below, whole rows longest first are ahead (16 of 1,000 29.2 against 31.9, 64 of 1,216 109 against 114), and
     so they are with large heads of one length (64 rows of 1,500, 32 heads of 128 over 8: 71 against 78)."""
@@ -404,7 +404,7 @@ def rows_room(blocks, span, waves, splits, head_dim):
         return 4, (512 if head_dim <= 128 else 256), (1 if blocks < 128 else 2)
     if waves == 8:
         return 8, 256, 1
-    return 4, (1024 if blocks * splits > 768 else 768), 2
+    return (4, 1536, 4) if blocks * splits > 768 else (4, 768, 2)
 
 
 def row_pieces(heads, kv_heads, head_dim, window, keep_first=0):
