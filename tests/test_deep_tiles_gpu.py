@@ -96,3 +96,33 @@ def test_deep_tiles_are_refused_where_they_do_not_exist():
         with pytest.raises(ops.KernelError):
             ops.attention_mfma(q, D, cache, cache.view(1, 1, D, 16), ints.view(4, 1), ints, ints, q.clone(), 1, 1, D, 16, None, 1.0,
                                torch.zeros(1, 4, dtype=torch.int32, device=DEV), block_tiles="deep", **kw)
+
+
+def _microseconds(step, heads, kv_heads, D):
+    from runtime.kernels import attention
+    from test_long_attention_gpu import View, make_cache
+    K, V, tables = make_cache(step, kv_heads, D, 1)
+    q = torch.randn(step.n_rows, heads * D, device=DEV).bfloat16()
+    out = torch.empty_like(q)
+    tuning = AttentionTuning(deep_tiles=True, split_single_from=1 << 30)
+    launch = lambda: attention.paged_attention(step, q, heads * D, K, V, View(tables), out, heads, kv_heads, D, None, D ** -0.5, tuning=tuning)
+    launch()
+    torch.cuda.synchronize()
+    best = math.inf
+    for _ in range(5):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(20):
+            launch()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, begin.elapsed_time(end) * 50)
+    return best
+
+
+@pytest.mark.gpu
+def test_all_waves_of_a_block_walk_a_single_rows_keys():
+    """Decoded tokens of 2,000 keys run beside a portion of 1,024 rows; walked by one wave of four they take 1.5 times what it does."""
+    from test_long_attention_gpu import Step
+    alone = _microseconds(Step([1024], [0]), 16, 1, 256)
+    assert _microseconds(Step([1] * 8 + [1024], [1999] * 8 + [0]), 16, 1, 256) < 1.35 * alone
