@@ -126,3 +126,41 @@ def test_all_waves_of_a_block_walk_a_single_rows_keys():
     from test_long_attention_gpu import Step
     alone = _microseconds(Step([1024], [0]), 16, 1, 256)
     assert _microseconds(Step([1] * 8 + [1024], [1999] * 8 + [0]), 16, 1, 256) < 1.35 * alone
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, kv_heads, D, window", [(16, 1, 256, None), (6, 2, 200, None), (3, 3, 160, None), (16, 1, 256, 40), (3, 3, 192, 50)])
+def test_deep_tiles_keep_what_is_not_finite_from_other_waves_rows(heads, kv_heads, D, window):
+    """Values of some keys hold NaN and infinities.  They reach the rows that see them, and at most the rows that share their sixteen items (with
+    16 heads a key head none: a wave's items are one row): not a block's earlier rows, nor those whose window has passed them."""
+    from runtime.kernels import attention
+    from test_long_attention_gpu import P, Step, View, make_cache
+    step, gc = Step([150, 1, 90], [0, 33, 64]), min(heads // kv_heads, 16)
+    K, V, tables = make_cache(step, kv_heads, D, 4)
+    for s, key, d, what in [(0, 3, 5, math.nan), (0, 17, 40, math.inf), (0, 70, 9, -math.inf), (0, 141, D - 1, math.nan), (1, 33, 0, math.nan), (2, 100, 77, math.inf),
+                            (2, 153, 78, math.nan)]:
+        V[tables[s, key // P].item(), :, d, key % P] = what
+    q = torch.randn(step.n_rows, heads * D, device=DEV).bfloat16()
+    out = torch.empty_like(q)
+    attention.paged_attention(step, q, heads * D, K, V, View(tables), out, heads, kv_heads, D, window, D ** -0.5, tuning=AttentionTuning(deep_tiles=True))
+    got, row, kept = out.double().cpu().view(-1, heads, D), 0, 0
+    for s, (start, count) in enumerate(zip(step.starts, step.counts)):
+        pages = tables[s, :-(-(start + count) // P)].long()
+        keys = K[pages].double().cpu().permute(0, 2, 1, 3).reshape(-1, kv_heads, D)
+        values = V[pages].double().cpu().permute(0, 3, 1, 2).reshape(-1, kv_heads, D)
+        for i in range(count):
+            for h in range(heads):
+                at, per = h * kv_heads // heads, 64 // gc
+                wave = (i % per * gc + h % gc) // 16
+                first, last = (min(i // per * per + item // gc, i // per * per + per - 1, count - 1) for item in (16 * wave, 16 * wave + 15))
+                low, near = (0 if window is None else max(0, start + x + 1 - window) for x in (i, first))
+                k, v = keys[low:start + i + 1, at], values[low:start + i + 1, at]
+                sees, may = ~torch.isfinite(v).all(0), ~torch.isfinite(values[near:start + last + 1, at]).all(0)
+                odd = ~torch.isfinite(got[row, h])
+                assert (odd >= sees).all() and (odd <= may).all(), (s, i, h)
+                want = torch.softmax(k @ q[row].double().cpu().view(heads, D)[h] * D ** -0.5, 0) @ v
+                # (a weight as two bf16 numbers and the output's rounding, 2^-9)
+                assert (got[row, h] - want)[~odd].abs().max() < 8e-3 * max(1.0, want[~odd].abs().max())
+                kept += int((~may).sum())
+            row += 1
+    assert kept > 0
