@@ -36,7 +36,7 @@ class AttentionTuning:
     # are 24 of them and more: they are blocks enough, and run beside the portions)
     split_single_from: int = 4096
     rows_launch: Optional[tuple] = None   # (wavefronts a block, blocks along the keys) of decode rows
-    stream_loads: Optional[bool] = None   # decode rows read keys and values with non-temporal loads (None: by the rule)
+    stream_loads: Optional[bool] = None   # decode rows, and single rows in the square form, read with non-temporal loads (None: by the rules)
     # A step of single tokens whose keys are not split runs a block for every (row, key head), the key heads of a row
     # side by side.  From this many blocks on (more than one block a compute unit) the rows are listed longest first,
     # so that the launch does not end with the blocks of a long row alone (64 rows of 228 to 2,304 keys at the 1.7B
@@ -437,6 +437,16 @@ def rows_stream_loads(blocks, span, waves, splits, head_dim):
     return blocks * splits >= 160 and 2 * steps <= 5 * waves * splits
 
 
+def single_rows_stream(blocks):
+    """Whether the single rows of a mixed step in the square form, `blocks` blocks of them (the step's number rounded up), read keys
+    and values with non-temporal loads.  The waves' loads take half lines; few blocks leave the caches room to hold a line until its other half is
+    asked for, many do not.  us non-temporal / plain: 32 heads of 128 over 8, 8 rows of 4,000 keys and a portion of 256 71 / 60, 8 of 2,000
+    and 1,024 50 / 48, 16 of 3,000 and 256 63 / 58, 30 of 900 and 256 30 / 33, 30 of 2,000 and 2,048 107 / 117; 9 heads of 64 over 3,
+    8 of 4,000 and 1,024 34 / 23, 50 of 3,000 and 1,024 35 / 31; 32 heads of 64, 3 of 3,000 and 256 30 / 26, 8 of 900 and 30 20 / 21, 30 of 3,000
+    and 256 128 / 136.  Where the number is rounded up to 256 the line is crossed early: 20 of 2,000 and 256, 32 heads of 128 over 8, 46 / 38."""
+    return blocks >= 256
+
+
 def fused_merge_splits(splits, rows, accepts):
     """How many of the `splits` blocks along a decode row's keys the product that follows may merge itself
     (`accepts(n)` says whether it takes n), or None: then the merge kernel runs.  That product merges 2, 4 or 8
@@ -564,7 +574,8 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
         form = ("square", form[1], 1) if form[0] == "block" else ("tiles", 1, 1)
     kind, item_tiles, halves = form
     tasks, _ = ctx.step_array(TileTasks(rows_per_tile_of(form, heads, kv_heads), singles))
-    ops.attention_mfma(*common, tasks.view(-1, 4), waves=tuning.tile_waves,
+    stream_single = kind == "square" and (tuning.stream_loads if tuning.stream_loads is not None else single_rows_stream(alone * chunks))
+    ops.attention_mfma(*common, tasks.view(-1, 4), waves=tuning.tile_waves, stream_loads=stream_single,
                        block_tiles={"tiles": False, "block": True, "square": 32, "deep": "deep"}[kind], item_tiles=item_tiles, key_groups=halves,
                        **law)
     return None

@@ -1043,7 +1043,7 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
                 raise KernelError("attention_mfma: one or two key groups, two with 64 or 128 items a block")
             if dpad > 64 and (item_tiles == 4 or (item_tiles == 2 and key_groups == 2)):
                 raise KernelError("attention_mfma: blocks of more than eight waves need a head size of at most 64")
-            mode = {(1, 1): 6, (2, 1): 5, (3, 1): 10, (4, 1): 7, (1, 2): 8, (2, 2): 9}[(item_tiles, key_groups)]
+            mode = {(1, 1): 6, (2, 1): 5, (3, 1): 10, (4, 1): 7, (1, 2): 8, (2, 2): 9}[(item_tiles, key_groups)] + (16 if stream_loads else 0)
         tp = _dev(tasks, "tasks", torch.int32, (n_tasks, 4))
     else:
         n_tasks, mode = rows, 1

@@ -57,3 +57,18 @@ def test_single_rows_in_square_tiles(heads, kv_heads, D):
         assert prompt_form(290, 91, step.span_hint, heads, kv_heads, D, 16, singles=90)[0] == "square"
     got, want = attend(step, heads, kv_heads, D, seed=9)
     check(got, want, f"{heads}/{kv_heads}x{D}, 90 single rows and 200")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, kv_heads, D, singles, streams", [(32, 8, 128, 8, False), (32, 8, 128, 32, True), (9, 3, 64, 64, False), (32, 32, 64, 8, True)])
+def test_few_single_rows_read_with_plain_loads(monkeypatch, heads, kv_heads, D, singles, streams):
+    """Which loads the single rows of the square form take, and that their results do not depend on it."""
+    from runtime.kernels import ops
+    from test_long_attention_gpu import Step, attend
+    step, seen, launch = Step([1] * singles + [1024], [37 * i for i in range(singles)] + [700]), [], ops.attention_mfma
+    monkeypatch.setattr(ops, "attention_mfma", lambda *a, **kw: (seen.append((kw.get("block_tiles"), kw.get("stream_loads"))), launch(*a, **kw))[1])
+    by_rule, _ = attend(step, heads, kv_heads, D, seed=3)
+    assert seen == [(32, streams)]
+    for stream in (False, True):
+        got, _ = attend(step, heads, kv_heads, D, seed=3, tuning=AttentionTuning(stream_loads=stream))
+        assert torch.equal(got, by_rule)
