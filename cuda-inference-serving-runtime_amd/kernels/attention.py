@@ -230,8 +230,11 @@ def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tu
     is one tile of 16 n items (a token row and a query head) whose waves split its keys; ("block", n, 1): 64 n items,
     four waves that own different rows and share keys and values through LDS; ("square", n, halves): 64 n items on
     the 32 x 32 instruction with waves of their own for the copies, as one half or as two that take the even and the
-    odd steps; ("deep", 1, 1): "block" for heads of more than 128 coordinates.  `span`: the longest context of the step.  `singles`: how many of the segments are single tokens that
-    share the launch; the others' rows decide, with the singles' blocks counted beside theirs."""
+    odd steps; ("deep", 1, 1): "block" for heads of more than 128 coordinates.  `span`: the longest context of the step.
+    `singles`: how many of the segments are single tokens that share the launch; the others' rows decide, with the singles' blocks counted
+    beside theirs (but how large a tile is follows from all rows: a single row is a tile too.  9 heads of 64 over 3, 16 rows of 900 keys
+    beside 256, us with 32 items / 16: 11.5 / 9.2, of 3,000 22.8 / 18.5; 8 of 900 beside 1,024 13.9 / 15.8)."""
+    tile_items = 2 if tuning.item_tiles == 2 and head_dim <= 64 and rows >= 16 * n_segments else 1
     rows, n_segments = max(1, rows - singles), max(1, n_segments - singles)
     group = heads // kv_heads
     heads_per_chunk = min(group, 16)
@@ -243,14 +246,22 @@ def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tu
         # with 128 items in brackets: 32 heads of 64, 37 rows of 900 keys and a portion of 1,024: 123 -> 74 (82); 30 of
         # 1,300 and one of 30: 99 -> 61 (61); 16 of 200 and one of 256: 22 -> 16 (18); 32 heads of 128 over 8: 78 -> 60
         # (67), 68 -> 44 in halves (46), 22 -> 16 (18).  Below 256 blocks the forms of few blocks below stay ahead (9 heads
-        # over 3, 16 of 200 and 256: 11.8 against 13.0); with large heads, so do larger blocks where a row's chain of steps is
-        # long (30 of 2,400 and 1,024: 98 against 85 with 128 items) or the portions fill the GPU (8 of 2,000 and 2,048: 82 against
-        # 73 with 192).
+        # over 3, 16 of 200 and 256: 11.8 against 13.0), and tiles where the portions are small (fewer than 128 blocks of 64 items; us in this
+        # form / in tiles: 32 heads of 64, 8 rows of 900 and a portion of 30 20 / 15, of 100 20 / 16; 32 of 128 over 8, 20 of
+        # 2,000 and 30 45 / 37; 8 of 128, 30 of 900 and 256 34 / 29), unless the single rows are more blocks than
+        # compute units and their contexts not short (32 heads of 64, 16 of 900 and 30: 25 / 26, of 200 12 / 10).  With large heads larger blocks are ahead where a row's chain
+        # of steps is long (30 of 2,400 and 1,024: 98 against 85 with 128 items) or the portions fill the GPU (8 of 2,000 and 2,048: 82
+        # against 73 with 192; beside fewer than 192 blocks of single rows from 512 blocks on: 8 of 2,000 and 1,024 41 / 33, 16 of
+        # 2,000 48 / 42, but 24 53 / 63).
+        # In halves: 30 of 200 and 2,048, 9 heads over 3, 30 / 24, of 2,000 31 / 28; 8 of 128, 16 of 900 and 2,048 46 / 38; with 256
+        # blocks of single rows and more they lose (8 of 128, 30 of 900 and 256: 27 / 35).
         chunks = kv_heads * -(-group // heads_per_chunk)
         blocks = -(-rows // (64 // heads_per_chunk)) * chunks
-        together = blocks + singles * chunks
-        if together >= 256 and (head_dim <= 64 or (span <= 2048 and blocks < 1000)):
-            return "square", 1, 2 if together <= 384 and span >= 1024 else 1
+        alone = singles * chunks
+        fill = blocks + alone >= 256 and (blocks >= 128 or (alone > 256 and span >= 512))
+        if fill and (head_dim <= 64 or (span <= 2048 and blocks < (1000 if alone >= 192 else 512))):
+            few = alone < 256 and (blocks + alone <= 384 or (blocks <= 320 and blocks + alone <= 512))
+            return "square", 1, 2 if few and span >= 1024 else 1
     if long_portions and head_dim <= 128:
         # enough long portions to fill the GPU with blocks of 64 items (or more): the waves of a block own different
         # rows and share each step's keys and values through LDS.  Otherwise (few heads, short portions) the waves
@@ -302,7 +313,7 @@ def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tu
         blocks = -(-rows // (64 // heads_per_chunk)) * kv_heads * -(-group // heads_per_chunk)
         if blocks >= (96 if span <= 512 else 192) if tuning.deep_tiles is None else tuning.deep_tiles:
             return "deep", 1, 1
-    return "tiles", 2 if tuning.item_tiles == 2 and long_portions and head_dim <= 64 else 1, 1
+    return "tiles", tile_items, 1
 
 
 def rows_per_tile_of(form, heads, kv_heads):

@@ -38,6 +38,25 @@ def test_form_of_mixed_steps_at_measured_points(heads, kv_heads, dim, singles, r
     assert prompt_form(rows + singles, 1 + singles, span, heads, kv_heads, dim, 4, singles=singles)[0] != "square"
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, singles, rows, span, form", [
+    (9, 3, 64, 16, 256, 1024, ("tiles", 2, 1)),         # 272 rows of 17 segments
+    (9, 3, 64, 16, 255, 1024, ("tiles", 1, 1)),         # 271: a single row is a tile of 16 items
+    (9, 3, 64, 32, 288, 1024, ("tiles", 1, 1)),
+    (9, 3, 64, 32, 2048, 1024, ("square", 1, 2)),       # 294 blocks beside 96: halves
+    (8, 8, 128, 16, 2048, 1024, ("square", 1, 2)),
+    (8, 8, 128, 32, 2048, 1024, ("square", 1, 1)),      # 256 blocks of single rows
+    (32, 32, 64, 8, 56, 1024, ("tiles", 1, 1)),         # a small portion
+    (32, 32, 64, 8, 192, 1024, ("tiles", 2, 1)),        # 96 blocks
+    (32, 32, 64, 8, 256, 1024, ("square", 1, 1)),
+    (32, 32, 64, 16, 48, 256, ("tiles", 1, 1)),         # 512 blocks of single rows, short contexts
+    (32, 32, 64, 16, 48, 1024, ("square", 1, 1)),
+    (32, 8, 128, 8, 1024, 2048, ("square", 2, 1)),      # 512 blocks beside 64: the portions' own form
+    (32, 8, 128, 32, 1024, 2048, ("square", 1, 1)),     # beside 256
+])
+def test_single_rows_are_no_reason_for_a_slower_form(heads, kv_heads, dim, singles, rows, span, form):
+    assert tuple(prompt_form(rows + singles, 1 + singles, span, heads, kv_heads, dim, 16, singles=singles)) == form
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads, kv_heads, D", [(9, 3, 64), (32, 8, 128), (4, 4, 32), (20, 1, 96), (6, 2, 72)])
 def test_single_rows_in_square_tiles(heads, kv_heads, D):
