@@ -455,7 +455,7 @@ def single_rows_stream(blocks):
     and 1,024 50 / 48, 16 of 3,000 and 256 63 / 58, 30 of 900 and 256 30 / 33, 30 of 2,000 and 2,048 107 / 117; 9 heads of 64 over 3,
     8 of 4,000 and 1,024 34 / 23, 50 of 3,000 and 1,024 35 / 31; 32 heads of 64, 3 of 3,000 and 256 30 / 26, 8 of 900 and 30 20 / 21, 30 of 3,000
     and 256 128 / 136.  Where the number is rounded up to 256 the line is crossed early: 20 of 2,000 and 256, 32 heads of 128 over 8, 46 / 38."""
-    return blocks >= 256
+    return blocks >= 256 or blocks == 0      # (none: one kernel for the portions of all steps)
 
 
 def fused_merge_splits(splits, rows, accepts):
