@@ -13,7 +13,7 @@ on without knowing what they hold.  The reference has one attention kernel and n
 (kernels/ops.cu:35-80).
 """
 import functools
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import Optional
 
 import numpy as np
@@ -31,9 +31,8 @@ class AttentionTuning:
     deep_tiles: Optional[bool] = None     # portions with heads of more than 128 coordinates through LDS-shared tiles of 64 items
     tile_waves: int = 4                   # wavefronts that share one tile's keys
     item_tiles: int = 2                   # 16-item tiles a wave of long portions (small heads)
-    # In a mixed step a decoded token is a tile whose keys one block walks; from this context on the one-token
-    # segments get a launch of their own instead, which splits their keys over blocks (from twice that on where there
-    # are 24 of them and more: they are blocks enough, and run beside the portions)
+    # In a mixed step a decoded token is a tile whose keys one block walks; from about this context on the one-token
+    # segments get a launch of their own instead, which splits their keys over blocks (SingleRows, single_rows)
     split_single_from: int = 4096
     rows_launch: Optional[tuple] = None   # (wavefronts a block, blocks along the keys) of decode rows
     stream_loads: Optional[bool] = None   # decode rows, and single rows in the square form, read with non-temporal loads (None: by the rules)
@@ -80,18 +79,46 @@ class SingleRows:
     """Step array: the rows of the one-token segments of a mixed step (then -1), when they get an attention launch
     of their own: all of them, if one of them has a context of `split_from` keys or more; none in a step of
     one-token segments only, or of short contexts.  Its launch value is how many entries such a launch covers.
-    From 24 of them on `split_from` counts twice (30 rows of 5,000 keys beside a portion, us together / apart: 9 heads of 64
-    over 3 and 2,048 rows 65 / 105, 32 heads of 64 and 512 rows 216 / 276, 32 heads of 128 over 8 and 512 rows 152 / 169; but 8 of
-    6,000 and 1,024 rows 71 / 39, 107 / 113, 155 / 90, and 20 of 15,000 171 / 69, 458 / 462, 408 / 293)."""
+    `layer` = (heads, key heads, head size, whether it is one of large heads without a window): `split_from` is multiplied (`least`) where the rows'
+    blocks fill the GPU without being split, or run long beside the portions'.  Layers that share a list go by the first one's.
+    us together / apart, rows of so many keys beside a portion:
+    from 192 blocks and 24 rows on twice: 24 of 4,100 and 64, 32 heads of 128 over 8 (192 blocks) 77 / 96, of 8,000 and 1,024 177 / 196; 64 of
+    8,000 and 64, 9 heads over 3, 74 / 75; but with 72 blocks, 24 of 8,000 and 64, 55 / 42, with 24 (16 heads of 256 over one) 227 / 67;
+    from 64 blocks on in the square form one and a half times: 24 of 4,100 and 1,024, 9 heads of 64 over 3, 32 / 40, of 8,000 55 / 52.
+    Large heads count half (single_rows): 16 of 256 over one, 8 of 2,000 and 64 50 / 23, of 3,000 and 512 73 / 45, of 1,000 and 512 30 / 41;
+    but from twice that on (the whole `split_from` of other layers) where the portions take as long as such rows: 400 blocks (8 of 3,000 and 2,048
+    105 / 121, of 4,100 138 / 124), or 64 beside as many of single rows (8 of 192 over 2, 40 of 2,000 and 1,024 58 / 76, of 4,100 112 / 108),
+    and from a quarter more beside deep tiles (8 of 2,000 and 1,024 63 / 67, of 3,000 87 / 71)."""
     split_from: int
+    layer: Optional[tuple] = field(default=None, compare=False)
 
     def words(self, rows, segments):
         return segments
 
+    def least(self, singles, batch):
+        """The context from which on `singles` one-token segments of this batch have a launch of their own."""
+        if self.layer is None:
+            return self.split_from * (2 if singles >= 24 else 1)
+        heads, kv_heads, head_dim, large = self.layer
+        group = heads // kv_heads
+        chunks = kv_heads * -(-group // min(group, 16))
+        unit = 2 * self.split_from if large else self.split_from
+        if singles * chunks >= 192:
+            return unit * (2 if singles >= 24 else 1)
+        if not large and (singles < 24 or singles * chunks < 64):
+            return unit
+        rows, longest = sum(batch.counts), max(start + count for start, count in zip(batch.starts, batch.counts))
+        kind, _, _ = prompt_form(rows, len(batch.counts), 1 << (longest - 1).bit_length(), heads, kv_heads, head_dim, 16, singles=singles)
+        if not large:
+            return unit * 3 // 2 if kind == "square" else unit
+        blocks = -(-(rows - singles) // (64 // min(group, 16))) * chunks
+        if singles * chunks >= 64 and blocks >= 64 or blocks >= 400:
+            return unit
+        return unit * 5 // 8 if kind == "deep" else unit // 2
+
     def launch_value(self, batch):
         singles = [start + 1 for start, count in zip(batch.starts, batch.counts) if count == 1]
-        split_from = self.split_from * (2 if len(singles) >= 24 else 1)
-        if not singles or len(singles) == len(batch.counts) or max(singles) < split_from:
+        if not singles or len(singles) == len(batch.counts) or max(singles) < self.split_from or max(singles) < self.least(len(singles), batch):
             return 0
         return len(singles)
 
@@ -430,7 +457,13 @@ def step_arrays(tuning, operand, *layer):
     """The step arrays that an attention layer names beforehand.  `operand`: one of its matrices (decode rows on the matrix cores,
     which RowPieces is for, are those of bfloat16 ones); `layer`: what `row_pieces` takes."""
     pieces = [row_pieces(*layer)] if operand is not None and operand.dtype == torch.bfloat16 and tuning.rows_launch is None else []
-    return [SingleRows(tuning.split_single_from), SingleTokens(), RowsLongestFirst()] + pieces
+    return [single_rows(tuning, *layer[:4]), SingleTokens(), RowsLongestFirst()] + pieces
+
+
+def single_rows(tuning, heads, kv_heads, head_dim, window):
+    """The SingleRows of an attention layer.  (Of large heads without a window: half the context.  A window's keys are walked soon.)"""
+    large = head_dim > 128 and not window
+    return SingleRows(tuning.split_single_from // (2 if large else 1), (heads, kv_heads, head_dim, large))
 
 
 def rows_stream_loads(blocks, span, waves, splits, head_dim):
@@ -565,13 +598,13 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
         ops.attention_mfma(*common, None, splits, workspace, waves, row_ids=order, stream_loads=stream(rows * chunks, waves, splits),
                            merge_gate=gated, **law)
         return None if gated is None else GATED
-    singles = SingleRows(tuning.split_single_from)
-    single_rows, n_single = ctx.step_array(singles)
+    singles = single_rows(tuning, heads, kv_heads, head_dim, window)
+    apart, n_single = ctx.step_array(singles)
     if n_single:
         # the decoded tokens of this mixed step: a launch of their own that splits their keys
         waves, splits = tuning.rows_launch or rows_launch(n_single * chunks, span, heads_per_chunk, head_dim)
         workspace = _split_workspace(ctx, n_single, heads, splits, head_dim) if splits > 1 else None
-        ops.attention_mfma(*common, None, splits, workspace, waves, row_ids=single_rows[:n_single],
+        ops.attention_mfma(*common, None, splits, workspace, waves, row_ids=apart[:n_single],
                            stream_loads=stream(n_single * chunks, waves, splits), **law)
     _, alone = ctx.step_array(SingleTokens())
     if n_single:

@@ -38,6 +38,31 @@ def test_form_of_mixed_steps_at_measured_points(heads, kv_heads, dim, singles, r
     assert prompt_form(rows + singles, 1 + singles, span, heads, kv_heads, dim, 4, singles=singles)[0] != "square"
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, window, singles, portion, least", [
+    (16, 1, 256, None, 24, 64, 2048),          # 24 blocks
+    (16, 1, 256, None, 40, 1024, 2560),        # deep tiles beside them
+    (16, 1, 256, None, 8, 2048, 4096),         # which take longer than the rows
+    (16, 1, 256, 1024, 8, 64, 4096),
+    (8, 2, 192, None, 40, 1024, 4096),         # 80 blocks beside 128
+    (8, 2, 192, None, 40, 64, 2048),
+    (32, 32, 256, None, 8, 64, 4096),          # 256 blocks
+    (8, 8, 192, None, 24, 256, 8192),          # 192
+    (9, 3, 64, None, 24, 64, 4096),            # 72 blocks, tiles
+    (9, 3, 64, None, 24, 1024, 6144),          # the square form
+    (9, 3, 64, None, 64, 64, 8192),            # 192 blocks
+    (9, 3, 64, None, 8, 1024, 4096),
+    (32, 8, 128, None, 23, 1024, 4096),
+    (32, 8, 128, None, 24, 64, 8192),
+])
+def test_single_rows_leave_the_launch_by_blocks_and_form(heads, kv_heads, dim, window, singles, portion, least):
+    from runtime.kernels.attention import DEFAULT_TUNING, step_arrays
+    array = step_arrays(DEFAULT_TUNING, None, heads, kv_heads, dim, window)[0]
+
+    def value(context):
+        return array.launch_value(Batch([1] * singles + [portion], [context - 1] * singles + [0], None, False, {}))
+    assert (value(least - 1), value(least)) == (0, singles)
+
+
 @pytest.mark.parametrize("heads, kv_heads, dim, singles, rows, span, form", [
     (9, 3, 64, 16, 256, 1024, ("tiles", 2, 1)),         # 272 rows of 17 segments
     (9, 3, 64, 16, 255, 1024, ("tiles", 1, 1)),         # 271: a single row is a tile of 16 items
