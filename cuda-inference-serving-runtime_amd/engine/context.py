@@ -46,6 +46,7 @@ class Batch:
     first_row: object     # int32 [segments]: row of each segment's first token
     decode_only: bool     # every segment brings exactly one token
     launch_values: dict   # StepArray -> its launch value for this step
+    rows: int = 0         # rows that the step is padded to (0: not padded)
 
 
 class StepContext:

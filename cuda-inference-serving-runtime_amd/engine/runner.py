@@ -261,7 +261,7 @@ class ModelRunner:
     def _launch_values(self, done):
         """What the parts' launches depend on beside rows, segments and contexts: the launch value of every carried
         step array that has one (context.StepArray), for this batch."""
-        batch = Batch([d.count for d in done], [d.start for d in done], None, all(d.count == 1 for d in done), {})
+        batch = Batch([d.count for d in done], [d.start for d in done], None, all(d.count == 1 for d in done), {}, _bucket(sum(d.count for d in done)))
         for array in self.carried:
             batch.launch_values[array] = array.launch_value(batch)
         return batch.launch_values
@@ -339,7 +339,7 @@ class ModelRunner:
                 slots[n_rows:] = -1
                 tables[n_seg:] = -1
         # what the parts asked for: first every launch value, then the arrays (one may read another's value)
-        batch = Batch(counts, starts, first_row, decode_only, {})
+        batch = Batch(counts, starts, first_row, decode_only, {}, T)
         for array in carried:
             own = array.launch_value(batch)
             batch.launch_values[array] = own if launch_values is None or own is None else launch_values.get(array, 0)

@@ -13,6 +13,7 @@ on without knowing what they hold.  The reference has one attention kernel and n
 (kernels/ops.cu:35-80).
 """
 import functools
+import math
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -171,7 +172,9 @@ def _pieces_launch(pieces, rows, span):
     blocks = rows * pieces.chunks
     waves, splits = rows_launch(blocks, span, pieces.heads_per_chunk, pieces.head_dim)
     room = rows_room(blocks, span, waves, splits, pieces.head_dim)
-    return None if room is None else (room[0], max(rows, -(-room[1] // pieces.chunks)), room[2], splits)
+    if room is None:
+        return None, 0.0
+    return (room[0], max(rows, -(-room[1] // pieces.chunks)), room[2], splits), rows_even(blocks, span, waves, splits, pieces.head_dim)
 
 
 @dataclass(frozen=True)
@@ -179,7 +182,8 @@ class RowPieces:
     """Step array: how the blocks of a decode step are dealt to its rows by the 32-key steps that each has to walk: int32 [rows +
     1], the first block of every row (rows that pad a step have none) and the end.  Which launch that is for follows from rows
     and the longest context, rounded up to a power of two (`launch`): where a row's keys are not cut the array stays empty.
-    `chunks`: blocks a row and part has; `seen`: how many keys a row sees at most (0: all)."""
+    Its launch value says whether the step's rows differ enough for that (rows_even): where they do not, it stays empty too, and
+    every row's keys are cut alike.  `chunks`: blocks a row and part has; `seen`: how many keys a row sees at most (0: all)."""
     chunks: int
     heads_per_chunk: int
     head_dim: int
@@ -188,20 +192,34 @@ class RowPieces:
 
     def launch(self, rows, longest):
         """(wavefronts a block, blocks a key head, least steps a wave, nominal splits) of `rows` rows up to `longest` keys, or None."""
-        return _pieces_launch(self, rows, max(256, 1 << (int(longest) - 1).bit_length()))
+        return _pieces_launch(self, rows, max(256, 1 << (int(longest) - 1).bit_length()))[0]
 
     def words(self, rows, segments):
         return rows + 1
 
     def launch_value(self, batch):
-        return None
+        if not batch.decode_only:
+            return 0
+        longest, n = max(batch.starts) + 1, len(batch.counts)
+        rows = batch.rows or n
+        even = _pieces_launch(self, rows, max(256, 1 << (longest - 1).bit_length()))[1]
+        if even is None:              # (whole rows: the blocks of the rows that there are, dealt to 256 compute units)
+            blocks = n * self.chunks
+            if blocks <= 0.85 * 256 * -(-blocks // 256):
+                return 1
+            even = 0.66 if rows * self.chunks <= 512 else 0.0
+        if self.seen and longest > self.seen:
+            longest, keys = self.seen, sum(min(start + 1, self.seen) for start in batch.starts)
+        else:
+            keys = sum(batch.starts) + n
+        return int(keys <= even * rows * longest)
 
     def fill(self, out, batch, value):
         """A part is a multiple of the block's waves in steps (each wave then walks as many), the smallest for which the parts of all
         rows are no more than there are blocks; a row has at most 16, or 32 where rows are few and a wave has two steps and
         more (their merge costs more than a second step)."""
         rows = len(out) - 1
-        launch = self.launch(rows, max(batch.starts) + 1) if batch.decode_only else None
+        launch = self.launch(rows, max(batch.starts) + 1) if batch.decode_only and value != 0 else None
         if launch is None:
             out[:] = 0
             return
@@ -429,13 +447,11 @@ def rows_room(blocks, span, waves, splits, head_dim):
     (wavefronts a block, blocks that the launch has room for, least 32-key steps a wave), or None: unsplit.
     The launch is filled once: 512 blocks of four waves (256 with more than 128 coordinates, where a compute unit holds one),
     256 of eight, 768 of four with small heads, twice where runs are long.  us of a step of rows between 0.4 and 1.6 times a mean, equal
-    splits -> by pieces: 32 heads of 128 over 8, 12 rows of 5,000 keys 76 -> 53, 24 of 3,000 93 -> 62, 3 of 700 11.1 -> 10.9, one of 30,000
+    splits -> by pieces: 32 heads of 128 over 8, 12 rows of 5,000 keys 76 -> 53, 24 of 3,000 93 -> 62, one of 30,000
     among eight of 500 125 -> 40; 9 of 64 over 3, 100 rows of 1,500 37 -> 30, 64 of 7,000 75 -> 65, 64 of 24,000 239 -> 196; one key head of 256, 24 rows of 2,000
-    44 -> 24.  Rows of one length, where only a merge that looks its parts up is added: 8 rows of 5,000 keys 36.2 -> 36.8, 16 of
-    2,000 31.9 -> 31.7; 9 of 64 over 3, 64 of 8,000 69 -> 71, 64 of 32,100 259 -> 256, 32 of 9,000 44 -> 48.
-    Small heads of many rows that are not split otherwise are, from 4,096 keys on: 32 heads of 64, 12 rows of 2,000 47 -> 41, 16 of
-    4,500 112 -> 100, 16 and 32 of 2,100 keys each 49 -> 50 and 93 -> 92; below, whole rows longest first are ahead (16 of 1,000 29.2 against 31.9, 64 of 1,216 109 against 114), and
-    so they are with large heads of one length (64 rows of 1,500, 32 heads of 128 over 8: 71 against 78)."""
+    44 -> 24.  Small heads of many rows that are not split otherwise may be, from 4,096 keys on (below, whole rows longest first are ahead: 32 heads
+    of 64, 16 of 1,000 29.2 against 31.9, 64 of 1,216 109 against 114), and so they are with large heads (64 rows of 1,500, 32 heads of 128
+    over 8: 71 against 78)."""
     if splits == 1:
         return (4, 1536, 2) if head_dim <= 64 and span >= 4096 and 256 < blocks <= 1024 else None
     if head_dim > 64:
@@ -443,6 +459,35 @@ def rows_room(blocks, span, waves, splits, head_dim):
     if waves == 8:
         return 8, 256, 1
     return (4, 1536, 4) if blocks * splits > 768 else (4, 768, 2)
+
+
+def rows_even(blocks, span, waves, splits, head_dim):
+    """How even the rows of a decode step may be for its blocks to be dealt by lengths: the most that their keys are of as many rows (the
+    padding ones too) of the longest one's length; 1: always, 0: never, None: for whole rows, which RowPieces decides.  Equal rows gain nothing
+    and pay for a merge that looks their parts up.  us equal splits / by pieces, that share in brackets: 9 heads of 64 over 3, 32 rows of 9,000
+    keys 43.9 / 46.3 (1.0), 45.7 / 47.2 (0.84), 51 / 48.5 (0.63); 64 of 8,000 72 / 73.4 (1.0), 85 / 75.6 (0.63); 12 heads of 64, 32 of 5,000 94.8 /
+    101.7 (0.72), 100.4 / 99 (0.63); 32 of 128 over 8, 4 of 3,000 17.7 / 19.3 (1.0), 18.1 / 19.5 (0.87), 20.9 / 20.2 (0.69), 12 of 5,000 and four that
+    pad 60.1 / 52.3 (0.75).  Never where a wave has a step at most, and nothing is to be evened out (16 of 128 over 4, 8 of 1,000 12.0 / 13.1 (0.66)).
+    Always with more than 16 splits, whose merge by one loop takes longer than the pieces' (32 of 128 over 8, one of 8,000 18.2 / 16.3;
+    with more than 128 coordinates only there and where rows differ: 16 of 256 over one, 8 of 6,000 21.4 / 22.5 (1.0), 23.2 / 22.3 (0.74)); where
+    the waves' second turn is nearly empty (33 steps of a window for 32 waves: 15.8 / 14.7); and with more than 128 coordinates and more
+    blocks than compute units (32 of 1,500 24.7 / 21.8 (1.0), but 16 of 1,500 14.6 / 16.8).  Blocks of eight waves otherwise never
+    (12 heads of 64, 8 of 3,000 24.1 / 29.0 (0.74)).
+    Whole rows (small heads): where the blocks of the rows that there are leave compute units a sixth idle or more (32 heads of 64, 12 rows of
+    5,000 101.6 / 87.1, 20 of 4,500 139 / 126; but 16 of 2,100 50 / 53, 24 of 4,500 147 / 149, 32 of 4,500 193 / 196 and of mixed lengths 196 / 218), or,
+    up to 512 blocks, lengths differ much (16 of 4,500 103 / 107 (0.84), 112 / 104 (0.64))."""
+    if splits == 1:
+        return None
+    turns = -(-span // 32) / (waves * splits)
+    if head_dim > 128 and blocks * splits > 256:
+        return 1.0
+    if turns <= 1:
+        return 0.0
+    if math.ceil(turns) >= 1.3 * turns or (head_dim <= 128 and splits > 16):
+        return 1.0
+    if head_dim > 128:
+        return 0.76 if splits > 16 else 0.0
+    return 0.76 if head_dim > 64 else 0.715 if waves == 4 else 0.0
 
 
 def row_pieces(heads, kv_heads, head_dim, window, keep_first=0):
@@ -584,11 +629,11 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
                 return workspace[0], workspace[1], fused
         pieces = row_pieces(heads, kv_heads, head_dim, window, keep_first)
         launch = pieces.launch(rows, ctx.span_hint) if tuning.rows_launch is None else None
-        if launch is not None:
-            waves, blocks, _, splits = launch
-            firsts, _ = ctx.step_array(pieces)
+        firsts, dealt = ctx.step_array(pieces) if launch is not None else (None, 0)
+        if dealt:
+            waves, blocks, _, nominal = launch
             ops.attention_mfma(*common, waves=waves, workspace=_split_workspace(ctx, blocks, heads, 1, head_dim), merge_gate=merge_gate,
-                               pieces=(firsts[:rows + 1], blocks), stream_loads=stream(rows * chunks, waves, splits), **law)
+                               pieces=(firsts[:rows + 1], blocks), stream_loads=stream(rows * chunks, waves, nominal), **law)
             return None if merge_gate is None else GATED
         workspace = _split_workspace(ctx, rows, heads, splits, head_dim) if splits > 1 else None
         order = None

@@ -41,6 +41,61 @@ def test_steps_with_portions_have_no_pieces():
     assert (out == 0).all()
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, window, lengths, rows, dealt", [
+    (9, 3, 64, 0, [8000] * 64, 64, 0),                                  # rows of one length: cut alike
+    (9, 3, 64, 0, [4000, 12000] * 32, 64, 1),
+    (9, 3, 64, 0, [9000] * 32, 32, 0),
+    (9, 3, 64, 0, [8000] * 4, 4, 0),
+    (9, 3, 64, 0, [8200] * 4, 4, 1),                                    # 21 splits
+    (12, 12, 64, 0, [3000] * 4 + [2000] * 4, 8, 0),                     # blocks of eight waves
+    (32, 8, 128, 0, [5000] * 8, 8, 0),
+    (32, 8, 128, 0, [5000] * 12, 12, 0),
+    (32, 8, 128, 0, [5000] * 12, 16, 1),                                # four rows that pad
+    (32, 8, 128, 0, [3000] * 4, 4, 0),
+    (32, 8, 128, 0, [700, 300, 200], 4, 0),                             # a step a wave
+    (32, 32, 64, 0, [2100] * 16, 16, 0),                                # whole rows: two blocks a compute unit
+    (32, 32, 64, 0, [5000] * 12, 16, 1),                                # one and a half
+    (32, 32, 64, 0, [6900, 2100] * 8, 16, 1),
+    (32, 32, 64, 0, [6900, 2100] * 16, 32, 0),                          # 1,024 blocks: they even out by themselves
+    (16, 1, 256, 0, [1500] * 8, 8, 0),
+    (16, 1, 256, 0, [1500] * 32, 32, 1),                                # 512 blocks of which a compute unit holds one
+    (16, 1, 256, 1024, [1500] * 8, 8, 1),                               # 33 steps for 32 waves
+    (16, 4, 128, 1024, [1100] * 24, 32, 1),
+])
+def test_blocks_are_dealt_by_lengths_where_rows_differ(heads, kv_heads, dim, window, lengths, rows, dealt):
+    n, pieces = len(lengths), row_pieces(heads, kv_heads, dim, window)
+    batch = Batch([1] * n, [x - 1 for x in lengths], np.arange(n, dtype=np.int32), True, {}, rows)
+    assert pieces.launch_value(batch) == dealt
+    out = np.full(pieces.words(rows, rows), 7, dtype=np.int32)
+    pieces.fill(out, batch, dealt)
+    assert (out == 0).all() if not dealt else (out[-1] > n or dealt == 1)
+    assert pieces.launch_value(Batch([1, 2], [900, 0], np.array([0, 1], dtype=np.int32), False, {}, 4)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads, kv_heads, D, length, law", [(9, 3, 64, 9000, None), (32, 8, 128, 3000, "gate"), (16, 1, 256, 1500, None)])
+def test_rows_of_one_length_are_cut_alike(heads, kv_heads, D, length, law):
+    """The same call, and the same bits, as with the launch rule's splits given."""
+    from runtime.kernels import attention
+    from test_long_attention_gpu import DEV, Step, View, make_cache
+    n = 4 if D == 128 else 32 if D == 64 else 8
+    step = Step([1] * n, [length - 1] * n)
+    K, V, tables = make_cache(step, kv_heads, D, seed=1)
+    q = (torch.randn(n, heads * D, device=DEV) * 2.0).bfloat16()
+    gates, packed = torch.randn(n, heads * D, device=DEV), [torch.zeros(n, heads * D, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    outs = []
+    chunks = kv_heads * -(-(heads // kv_heads) // 16)
+    given = attention.rows_launch(n * chunks, step.span_hint, min(heads // kv_heads, 16), D)
+    for i, tuning in enumerate((attention.DEFAULT_TUNING, attention.AttentionTuning(rows_launch=given))):
+        out = torch.zeros(n, heads * D, dtype=torch.bfloat16, device=DEV)
+        left = attention.paged_attention(step, q, heads * D, K, V, View(tables), out, heads, kv_heads, D, None, D ** -0.5, tuning=tuning,
+                                         merge_gate=None if law is None else (gates, packed[i], D))
+        assert (left == attention.GATED) == (law == "gate")
+        outs.append(packed[i] if law else out)
+    assert outs[0].any() and torch.equal(*outs)
+    assert any(isinstance(a, RowPieces) and not dealt for a, (_, dealt) in step.arrays.items())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads, kv_heads, D, lengths, window, law", [
     (32, 8, 128, [7750, 31, 2300, 5001, 1, 640], None, None),          # groups of 4: pieces of many sizes, a row of one key
@@ -52,8 +107,9 @@ def test_steps_with_portions_have_no_pieces():
     (8, 2, 128, [5000, 64, 1300], None, "gate"),                       # packed and gated by the merge
     (8, 2, 64, [5000, 900, 1300], 1024, "slopes"),
 ])
-def test_rows_of_mixed_lengths_by_pieces(heads, kv_heads, D, lengths, window, law):
+def test_rows_of_mixed_lengths_by_pieces(monkeypatch, heads, kv_heads, D, lengths, window, law):
     from runtime.kernels import attention
+    monkeypatch.setattr(RowPieces, "launch_value", lambda self, batch: 1)           # (also where the rows' lengths are no reason for it)
     from test_long_attention_gpu import DEV, Step, View, make_cache
     n = len(lengths)
     step = Step([1] * n, [x - 1 for x in lengths])
@@ -74,7 +130,7 @@ def test_rows_of_mixed_lengths_by_pieces(heads, kv_heads, D, lengths, window, la
     extra = {"sink": dict(sink=bias), "sigmoid": dict(head_bias=bias), "gate": dict(merge_gate=(gates, packed, vdim)),
              "slopes": dict(slopes=slopes, keep_first=17)}.get(law, {})
     attention.paged_attention(step, q, heads * D, K, V, View(tables), out, heads, kv_heads, D, window, scale, **extra)
-    assert any(isinstance(a, RowPieces) for a in step.arrays), "this step is meant to be dealt by pieces"
+    assert any(isinstance(a, RowPieces) and dealt for a, (_, dealt) in step.arrays.items()), "this step is meant to be dealt by pieces"
     group = heads // kv_heads
     want = torch.zeros(rows, heads, D, dtype=torch.float64, device=DEV)
     for s, length in enumerate(lengths):
