@@ -172,6 +172,8 @@ def _pieces_launch(pieces, rows, span):
     blocks = rows * pieces.chunks
     waves, splits = rows_launch(blocks, span, pieces.heads_per_chunk, pieces.head_dim)
     room = rows_room(blocks, span, waves, splits, pieces.head_dim)
+    if pieces.merges and splits > 1 and fused_merge_splits(splits, rows, lambda n: ops.merged_rows_ok(rows, pieces.merges, n)) is not None:
+        room = None                   # (the product behind merges the rows itself, and those are cut alike)
     if room is None:
         return None, 0.0
     return (room[0], max(rows, -(-room[1] // pieces.chunks)), room[2], splits), rows_even(blocks, span, waves, splits, pieces.head_dim)
@@ -183,12 +185,14 @@ class RowPieces:
     1], the first block of every row (rows that pad a step have none) and the end.  Which launch that is for follows from rows
     and the longest context, rounded up to a power of two (`launch`): where a row's keys are not cut the array stays empty.
     Its launch value says whether the step's rows differ enough for that (rows_even): where they do not, it stays empty too, and
-    every row's keys are cut alike.  `chunks`: blocks a row and part has; `seen`: how many keys a row sees at most (0: all)."""
+    every row's keys are cut alike.  `chunks`: blocks a row and part has; `seen`: how many keys a row sees at most (0: all);
+    `merges`: what the product behind can merge itself (ops.merges_into; None: nothing)."""
     chunks: int
     heads_per_chunk: int
     head_dim: int
     window: int
     seen: int
+    merges: Optional[tuple] = None
 
     def launch(self, rows, longest):
         """(wavefronts a block, blocks a key head, least steps a wave, nominal splits) of `rows` rows up to `longest` keys, or None."""
@@ -490,17 +494,17 @@ def rows_even(blocks, span, waves, splits, head_dim):
     return 0.76 if head_dim > 64 else 0.715 if waves == 4 else 0.0
 
 
-def row_pieces(heads, kv_heads, head_dim, window, keep_first=0):
+def row_pieces(heads, kv_heads, head_dim, window, keep_first=0, merges=None):
     """The RowPieces of an attention layer."""
     group = heads // kv_heads
     per_chunk = min(group, 16)
     window = int(window or 0)
-    return RowPieces(kv_heads * -(-group // per_chunk), per_chunk, head_dim, window, window + 31 + keep_first if window else 0)
+    return RowPieces(kv_heads * -(-group // per_chunk), per_chunk, head_dim, window, window + 31 + keep_first if window else 0, merges)
 
 
 def step_arrays(tuning, operand, *layer):
     """The step arrays that an attention layer names beforehand.  `operand`: one of its matrices (decode rows on the matrix cores,
-    which RowPieces is for, are those of bfloat16 ones); `layer`: what `row_pieces` takes."""
+    which RowPieces is for, are those of bfloat16 ones); `layer`: what `row_pieces` takes (and paged_attention is given)."""
     pieces = [row_pieces(*layer)] if operand is not None and operand.dtype == torch.bfloat16 and tuning.rows_launch is None else []
     return [single_rows(tuning, *layer[:4]), SingleTokens(), RowsLongestFirst()] + pieces
 
@@ -571,7 +575,7 @@ GATED = "gated"       # paged_attention: the heads' results were packed and gate
 
 
 def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_heads, head_dim, window, scale,
-                    defer_merge=None, tuning=DEFAULT_TUNING, head_bias=None, slopes=None, sink=None, keep_first=0, merge_gate=None):
+                    defer_merge=None, tuning=DEFAULT_TUNING, head_bias=None, slopes=None, sink=None, keep_first=0, merge_gate=None, merges=None):
     """out[r] = attention of row r's queries over its request's cached keys up to its own position (or the last
     `window` of them).  `ctx` is the step's context (rows, segments, positions, buffers, step arrays), `view` the
     cache group as the step sees it (block tables, page size).
@@ -585,6 +589,7 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
     `defer_merge(splits) -> bool`: the caller's next product can merge the partial results of a decode step whose
     keys are split over `splits` blocks itself (ops.gemm_merged).  Where that is so, no merge kernel runs, `out`
     is left alone and (partial outputs bf16, statistics float, splits) is returned; otherwise None.
+    `merges`: what that product's weights are (ops.merges_into), as the layer told `step_arrays`.
 
     `merge_gate` = (gates, packed, vdim): where the keys of a decode step are split, the merge packs and gates the heads
     itself (ops.attention_mfma) and GATED is returned; otherwise `out` is written and the caller gates."""
@@ -627,7 +632,7 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
                 ops.attention_mfma(*common, None, fused, workspace, waves, merge=False,
                                    stream_loads=stream(rows * chunks, waves, fused), **law)
                 return workspace[0], workspace[1], fused
-        pieces = row_pieces(heads, kv_heads, head_dim, window, keep_first)
+        pieces = row_pieces(heads, kv_heads, head_dim, window, keep_first, merges)
         launch = pieces.launch(rows, ctx.span_hint) if tuning.rows_launch is None else None
         firsts, dealt = ctx.step_array(pieces) if launch is not None else (None, 0)
         if dealt:

@@ -1097,8 +1097,22 @@ def attention_mfma(q, q_row_stride, kcache, vcache, tables, seg_of_row, position
 
 def gemm_merged_ok(m, w, heads, dim, splits):
     """Whether gemm_merged takes m rows of `splits` partial attention results of heads x dim against the bf16 weights w."""
-    return (w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == heads * dim and w.stride(1) == 1 and w.stride(0) % 8 == 0
-            and w.data_ptr() % 16 == 0 and bool(lib().cisr_gemm_merged_ok(int(m), int(w.shape[0]), int(heads), int(dim), int(splits))))
+    merges = merges_into(w, heads, dim)
+    return merges is not None and merged_rows_ok(m, merges, splits)
+
+
+def merges_into(w, heads, dim):
+    """(columns, heads, dim) if the bf16 weights w are ones that gemm_merged may be given for heads x dim, else None."""
+    if (w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == heads * dim and w.stride(1) == 1 and w.stride(0) % 8 == 0
+            and w.data_ptr() % 16 == 0):
+        return int(w.shape[0]), int(heads), int(dim)
+    return None
+
+
+def merged_rows_ok(m, merges, splits):
+    """Whether gemm_merged takes m rows of `splits` partial results against weights that `merges_into` says `merges` of."""
+    columns, heads, dim = merges
+    return bool(lib().cisr_gemm_merged_ok(int(m), columns, heads, dim, int(splits)))
 
 
 def gemm_merged(partials, heads, dim, w, out, residual=None):

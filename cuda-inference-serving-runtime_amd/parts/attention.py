@@ -33,14 +33,14 @@ class PagedAttention(Mixer):
         self.position, self.window, self.own_kv = position, window, own_kv
         self.scale = float(scale) if scale is not None else 1.0 / math.sqrt(head_dim)
         self.bias, self.out_bias = bool(bias), bool(out_bias)
-        self.w_in = self.w_out = self.b_in = self.b_out = None
+        self.w_in = self.w_out = self.b_in = self.b_out = self.merges = None
         self.tuning = tuning if tuning is not None else kernel.DEFAULT_TUNING   # what the kernel's launch rules may be told
 
     def kernel_units(self, dtype):
         return kernel.kernel_units(self.head_dim, dtype)
 
     def step_arrays(self):
-        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.head_dim, self.window)
+        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.head_dim, self.window, 0, self.merges)
 
     def cache_need(self):
         return KVNeed(self.kv_heads, self.head_dim, self.window) if self.own_kv else None
@@ -68,6 +68,7 @@ class PagedAttention(Mixer):
         parts = [matrix_operand(tensors[f"{self.name}.{p}.weight"], dtype) for p in names]
         self.w_in = torch.cat(parts, dim=0).contiguous() if len(parts) > 1 else parts[0]
         self.w_out = matrix_operand(tensors[f"{self.name}.o_proj.weight"], dtype)
+        self.merges = ops.merges_into(self.w_out, self.heads, self.head_dim)
         if self.bias:   # (a bias keeps the type it is stored in; it is added in float)
             self.b_in = torch.cat([tensors[f"{self.name}.{p}.bias"] for p in names], dim=0).contiguous()
         if self.out_bias:
@@ -118,7 +119,7 @@ class PagedAttention(Mixer):
         # a decode step of few rows may leave the partial results of its split keys to the output projection
         unmerged = kernel.paged_attention(ctx, q, q_stride, kcache, vcache, view, out, nh, nkv, D, self.window, self.scale,
                                           defer_merge=lambda splits: ops.gemm_merged_ok(T, self.w_out, nh, D, splits),
-                                          tuning=self.tuning)
+                                          tuning=self.tuning, merges=self.merges)
         if unmerged is not None:
             residual = ops.gemm_merged(unmerged, nh, D, self.w_out, residual, residual)
         else:
@@ -185,7 +186,7 @@ class NormedGatedAttention(Mixer):
             raise ValueError("a layer's cache keeps at least the keys the layer itself looks back over")
         self.names = {**self.NAMES, **(names or {})}
         self.tuning = tuning or kernel.DEFAULT_TUNING
-        self.w_in = self.w_out = self.q_weight = self.k_weight = self.b_in = None
+        self.w_in = self.w_out = self.q_weight = self.k_weight = self.b_in = self.merges = None
 
     def _tensor(self, which):
         return f"{self.name}.{self.names[which]}"
@@ -194,7 +195,7 @@ class NormedGatedAttention(Mixer):
         return kernel.kernel_units(self.pad, dtype, "softmax" if self.slopes is None else "distance")
 
     def step_arrays(self):
-        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.pad, self.window, self.keep_first)
+        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.pad, self.window, self.keep_first, self.merges)
 
     def cache_need(self):
         if self.keep_first:
@@ -230,6 +231,8 @@ class NormedGatedAttention(Mixer):
         device = self.w_in.device
         self.slope_t, self.sink_t = (None if n is None else torch.tensor(n, dtype=torch.float32, device=device) for n in (self.slopes, self.sink))
         self.w_out = matrix_operand(tensors[self._tensor("o")], dtype)
+        if not self.head_gate and self.pad == self.vdim:
+            self.merges = ops.merges_into(self.w_out, self.heads, self.vdim)
         if self.bias:
             self.b_in = torch.cat([tensors[self._tensor(p) + ".b"].to(torch.float32) for p in inputs]).contiguous()
         if self.qk_norm and self.qk_norm != "plain":
@@ -268,10 +271,10 @@ class NormedGatedAttention(Mixer):
         gates = qkv[:, first_gate:first_gate + self.gate_rows] if self.head_gate else None
         act = ctx.buffer("gattn.act", (T, nh * V), ctx.dtype) if gates is not None or pad != V else out
         merge_gate = (gates, act, V) if self.head_gate == "element" and self.float_rows and ctx.dtype == torch.bfloat16 else None
-        merges = None if self.head_gate or pad != V else (lambda splits: ops.gemm_merged_ok(T, self.w_out, nh, V, splits))
+        merges = None if self.merges is None else (lambda splits: ops.gemm_merged_ok(T, self.w_out, nh, V, splits))
         unmerged = kernel.paged_attention(ctx, q, nh * pad, kcache, vcache, view, out, nh, nkv, pad, self.window, self.scale,
                                           defer_merge=merges, tuning=self.tuning, slopes=self.slope_t, sink=self.sink_t,
-                                          keep_first=self.keep_first, merge_gate=merge_gate)
+                                          keep_first=self.keep_first, merge_gate=merge_gate, merges=self.merges)
         if unmerged is kernel.GATED:
             return ctx.product_for_norm(act, self.w_out, "gattn.y")
         if unmerged is not None:

@@ -72,6 +72,17 @@ def test_blocks_are_dealt_by_lengths_where_rows_differ(heads, kv_heads, dim, win
     assert pieces.launch_value(Batch([1, 2], [900, 0], np.array([0, 1], dtype=np.int32), False, {}, 4)) == 0
 
 
+def test_no_list_is_made_where_the_product_behind_merges():
+    """Four rows of 1,000 to 5,000 keys, 32 heads of 128 over 8: the output projection takes the rows' partial results as they are."""
+    batch = Batch([1] * 4, [4999, 999, 1999, 999], np.arange(4, dtype=np.int32), True, {}, 4)
+    assert row_pieces(32, 8, 128, None).launch_value(batch) == 1
+    merged = row_pieces(32, 8, 128, None, merges=(4096, 32, 128))
+    out = np.full(5, 7, dtype=np.int32)
+    merged.fill(out, batch, None)
+    assert merged.launch(4, 5000) is None and merged.launch_value(batch) == 0 and (out == 0).all()
+    assert merged.launch(16, 5000) == row_pieces(32, 8, 128, None).launch(16, 5000) is not None        # (more rows than it merges)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads, kv_heads, D, length, law", [(9, 3, 64, 9000, None), (32, 8, 128, 3000, "gate"), (16, 1, 256, 1500, None)])
 def test_rows_of_one_length_are_cut_alike(heads, kv_heads, D, length, law):
