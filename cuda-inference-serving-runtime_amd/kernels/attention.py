@@ -502,11 +502,16 @@ def row_pieces(heads, kv_heads, head_dim, window, keep_first=0, merges=None):
     return RowPieces(kv_heads * -(-group // per_chunk), per_chunk, head_dim, window, window + 31 + keep_first if window else 0, merges)
 
 
-def step_arrays(tuning, operand, *layer):
-    """The step arrays that an attention layer names beforehand.  `operand`: one of its matrices (decode rows on the matrix cores,
-    which RowPieces is for, are those of bfloat16 ones); `layer`: what `row_pieces` takes (and paged_attention is given)."""
-    pieces = [row_pieces(*layer)] if operand is not None and operand.dtype == torch.bfloat16 and tuning.rows_launch is None else []
-    return [single_rows(tuning, *layer[:4]), SingleTokens(), RowsLongestFirst()] + pieces
+def step_arrays(tuning, operand, *layer, law="softmax"):
+    """The step arrays that an attention layer names beforehand: what its steps read, as the numbers among them are part of a captured program's key.
+    `operand`: one of its matrices (these lists are for the matrix cores, and so for bfloat16); `layer`: what `row_pieces` takes (and
+    paged_attention is given); `law`: as in `kernel_units`."""
+    heads, kv_heads, head_dim, window = layer[:4]
+    if operand is not None and not kernel_units(head_dim, operand.dtype):
+        return []
+    tokens = [] if law == "sigmoid" else [SingleTokens()]
+    pieces = [row_pieces(*layer)] if operand is not None and tuning.rows_launch is None else []
+    return [single_rows(tuning, heads, kv_heads, head_dim, window)] + tokens + [RowsLongestFirst()] + pieces
 
 
 def single_rows(tuning, heads, kv_heads, head_dim, window):
@@ -656,10 +661,12 @@ def paged_attention(ctx, q, q_row_stride, kcache, vcache, view, out, heads, kv_h
         workspace = _split_workspace(ctx, n_single, heads, splits, head_dim) if splits > 1 else None
         ops.attention_mfma(*common, None, splits, workspace, waves, row_ids=apart[:n_single],
                            stream_loads=stream(n_single * chunks, waves, splits), **law)
-    _, alone = ctx.step_array(SingleTokens())
+    alone = 0
     if n_single:
-        form = prompt_form(max(1, rows - alone), max(1, ctx.n_segments - alone), span, heads, kv_heads, head_dim, view.page_size, tuning)
+        form = prompt_form(max(1, rows - n_single), max(1, ctx.n_segments - n_single), span, heads, kv_heads, head_dim, view.page_size, tuning)
     else:
+        if head_bias is None:         # (that law's prompt rows run as tiles in any case)
+            _, alone = ctx.step_array(SingleTokens())
         form = prompt_form(rows, ctx.n_segments, span, heads, kv_heads, head_dim, view.page_size, tuning, alone)
     if head_bias is not None and form[0] != "tiles":
         form = ("tiles", 2 if tuning.item_tiles == 2 and head_dim <= 64 else 1, 1)

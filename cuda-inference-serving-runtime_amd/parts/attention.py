@@ -459,7 +459,7 @@ class SigmoidAttention(Mixer):
         return kernel.kernel_units(self.pad, dtype, "sigmoid")
 
     def step_arrays(self):
-        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.pad, self.window)
+        return kernel.step_arrays(self.tuning, self.w_out, self.heads, self.kv_heads, self.pad, self.window, law="sigmoid")
 
     def cache_need(self):
         return KVNeed(self.kv_heads, self.pad, self.keep) if self.own_kv else None

@@ -21,6 +21,17 @@ def test_single_rows_share_the_launch_up_to_twice_the_context_when_they_are_many
     assert [value(23, 99), value(23, 100), value(24, 199), value(24, 200), value(1, 100)] == [0, 23, 0, 24, 1]
 
 
+def test_layers_name_the_numbers_that_they_read_and_no_others():
+    """A step's launch values are part of its captured program's key."""
+    from runtime.kernels.attention import DEFAULT_TUNING, RowPieces, RowsLongestFirst, step_arrays
+
+    def named(dtype, head_dim=64, **law):
+        return [type(a) for a in step_arrays(DEFAULT_TUNING, torch.zeros(1, 1, dtype=dtype), 8, 2, head_dim, None, **law)]
+    assert named(torch.bfloat16) == [SingleRows, SingleTokens, RowsLongestFirst, RowPieces]
+    assert named(torch.bfloat16, law="sigmoid") == [SingleRows, RowsLongestFirst, RowPieces]
+    assert named(torch.float32) == named(torch.bfloat16, 20) == []          # (row by row, or the 32-bit tiles)
+
+
 @pytest.mark.parametrize("heads, kv_heads, dim, singles, rows, span, form", [
     (32, 32, 64, 37, 1024, 2048, ("square", 1, 1)),
     (32, 32, 64, 16, 256, 256, ("square", 1, 1)),       # 640 blocks, short contexts
