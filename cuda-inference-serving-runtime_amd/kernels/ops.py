@@ -669,12 +669,17 @@ WIDE_MIN_BYTES_MANY_ROWS = 30 << 20
 _wide_plans = {}
 
 
-def wide_ok(m, w, swiglu=False, after_norm=False):
+def wide_ok(m, w, swiglu=False, after_norm=False, fused=False):
     """Whether a product of m rows with the bf16 weights w runs the wide weight-streaming kernel.
     `after_norm`: the rows are the output of an RMSNorm, which the other kernel would fuse (it then reads the
-    float residual and the norm's weights for every 16 rows of W, which costs it more than bf16 rows do)."""
+    float residual and the norm's weights for every 16 rows of W, which costs it more than bf16 rows do).
+    `fused`: it still may: the norm has not run, and the matrix-vector kernel is asked with it."""
     n, k = w.shape
-    if lib().cisr_gemv_ahead(int(m), int(n), int(k), int(after_norm), int(swiglu)):   # the matrix-vector kernel takes them
+    if gemv_ahead(m, n, k, fused, swiglu):
+        return False
+    if m <= GEMV_ROWS and after_norm and not fused and (swiglu or k < 2048):
+        # us of the other kernel / this one at 3 and 4 rows: 16384 x 2048 gated 13.7 / 14.9, 28672 x 4096 gated 40.3 / 39.6, 32768 x 1024 12.8 / 14.7; but
+        # 128256 x 4096 177 / 157, 32768 x 2048 27.1 / 23.7, 49152 x 2048 36.5 / 34.7
         return False
     least = WIDE_MIN_BYTES_FEW_ROWS if m <= 16 else WIDE_MIN_BYTES if m <= 32 else WIDE_MIN_BYTES_MANY_ROWS
     if 4 < m <= 16 and not after_norm and (m > 8 or k >= 4096):
@@ -683,7 +688,7 @@ def wide_ok(m, w, swiglu=False, after_norm=False):
         # a narrow output with a long inner size: the fused kernels have a block for every 16 columns and
         # cannot fill the GPU; this one cuts K as well
         least = min(least, max(WIDE_MIN_BYTES, 16 << 20))
-    if m >= 4 and after_norm and k >= 2048:     # (one or two rows of the residual cost the fused kernel next to nothing)
+    if (m > 4 or (m == 4 and fused)) and after_norm and k >= 2048:     # (few rows of the residual cost the fused kernel next to nothing)
         least = min(least, max(WIDE_MIN_BYTES, 24 << 20))
     if (w.dtype != torch.bfloat16 or not 0 < m <= SKINNY_ROWS or w.numel() * 2 < least or k % 8 or w.stride(0) % 8
             or w.data_ptr() % 16 or w.stride(1) != 1):
@@ -695,10 +700,15 @@ GEMV_ROWS, GEMV_MIN_BYTES = 4, 4 << 20
 
 
 def gemv_ok(m, n, k):
-    """Whether a product of m rows with weights [n, k] runs the matrix-vector kernel (up to four rows against weights
-    of 4 MB and more with an inner size of at least 1024: a wave owns whole rows of the weights; see csrc/gemv.hip
-    and the measurements in csrc/gemm_skinny.hip).  The weight-streaming entry points choose it themselves, where it is ahead."""
+    """Whether the matrix-vector kernel may be given a product of m rows with weights [n, k] (up to four rows against weights
+    of 4 MB and more with an inner size of at least 1024: a wave owns whole rows of the weights; see csrc/gemv.hip)."""
     return bool(lib().cisr_gemv_ok(int(m), int(n), int(k)))
+
+
+def gemv_ahead(m, n, k, normed=False, gated=False):
+    """Whether such a product runs the matrix-vector kernel: of those it may be given the ones that it is ahead on (`normed`: with the RMSNorm
+    fused; the measurements are in csrc/gemm_skinny.hip).  The weight-streaming entry points ask the same."""
+    return bool(lib().cisr_gemv_ahead(int(m), int(n), int(k), int(normed), int(gated)))
 
 
 def set_gemv(rows=GEMV_ROWS, least_bytes=GEMV_MIN_BYTES):
@@ -794,7 +804,7 @@ def _norm_args(x, norm, k):
 def fused_norm_ok(x, w, rows_out):
     """Whether the weight-streaming kernel can take RMSNorm(x) . w^T with the norm fused (and large weights
     do not make the norm as a kernel of its own and the wide kernel the better choice)."""
-    return (not wide_ok(rows_out, w, after_norm=True) and w.dtype == torch.bfloat16 and rows_out <= SKINNY_ROWS and x.dtype == torch.float32 and x.shape[1] % 8 == 0
+    return (not wide_ok(rows_out, w, after_norm=True, fused=True) and w.dtype == torch.bfloat16 and rows_out <= SKINNY_ROWS and x.dtype == torch.float32 and x.shape[1] % 8 == 0
             and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0)
 
 
@@ -891,7 +901,7 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
 def qkv_rope_fused_ok(a, w, head_dim, cos, normed):
     """Whether the fused projection + rotary + scatter kernel takes this shape."""
     m, k = a.shape
-    if normed and wide_ok(m, w, after_norm=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
+    if normed and wide_ok(m, w, after_norm=True, fused=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
         return False
     return (w.dtype == torch.bfloat16 and m <= SKINNY_ROWS and k % 8 == 0 and head_dim % 16 == 0
             and 2 * cos.shape[1] == head_dim and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0

@@ -172,3 +172,38 @@ def test_which_products_take_this_kernel(ops):
         assert not ops.gemv_ok(1, 6144, 4096)
     finally:
         ops.set_gemv(8, 0)
+
+
+# rows, weights, whether the norm is fused, whether the product is gated, whether the matrix-vector kernel is ahead
+AHEAD = [(1, 2048, 2048, False, False, False), (1, 2048, 2048, True, False, True), (1, 49152, 2048, False, False, False), (4, 49152, 2048, True, False, True),
+         (2, 6144, 4096, False, False, False), (4, 6144, 4096, True, False, True), (5, 6144, 4096, True, False, False),
+         (2, 16384, 2048, False, True, True), (3, 16384, 2048, False, True, False), (2, 4096, 14336, False, False, True), (3, 4096, 14336, False, False, False),
+         (2, 4096, 12288, False, False, True), (2, 4096, 12280, False, False, False), (1, 49152, 576, True, False, False)]
+
+
+def test_which_products_the_matrix_vector_kernel_is_ahead_on(ops):
+    ops.set_gemv()
+    try:
+        for m, n, k, normed, gated, ahead in AHEAD:
+            assert ops.gemv_ahead(m, n, k, normed, gated) == ahead, (m, n, k, normed, gated)
+    finally:
+        ops.set_gemv(8, 0)
+
+
+def test_rows_whose_norm_has_run_are_asked_about_as_such(ops):
+    """Up to four rows against a large head: with the norm fused they are the matrix-vector kernel's, without it the wide kernel's, and no product is
+    refused by both."""
+    ops.set_gemv()
+    try:
+        for n, k, swiglu, wide in [(32768, 2048, False, True), (32768, 1024, False, False), (32768, 2048, True, False), (6144, 4096, False, False)]:
+            w = torch.empty(n, k, dtype=torch.bfloat16, device=DEV)
+            for m in (1, 2, 3, 4):
+                assert ops.wide_ok(m, w, swiglu, after_norm=True) == wide
+                assert not ops.wide_ok(m, w, swiglu, after_norm=True, fused=True) and ops.gemv_ahead(m, n, k, True, swiglu)
+                assert ops.fused_norm_ok(torch.empty(m, k, device=DEV), w, m)
+        w, x = rnd(32768, 2048, dtype=torch.bfloat16, scale=2048 ** -0.5), rnd(3, 2048, dtype=torch.bfloat16)
+        got = ops.gemm(x, w, torch.empty(3, 32768, device=DEV), after_norm=True)
+        # sums of 2,048 exact products in float32
+        np.testing.assert_allclose(f64(got), f64(x) @ f64(w).T, rtol=1e-4, atol=1e-4)
+    finally:
+        ops.set_gemv(8, 0)
