@@ -890,7 +890,10 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         return out
     if gate_up is None:
         raise KernelError("gemm_swiglu: this shape needs a buffer [M, 2I] for the product of gate and up")
-    if a.dtype == torch.float32 and law is None and w_gate_up.is_cuda and w_gate_up.stride(1) == 1 and a.is_cuda and a.stride(1) == 1:
+    if (a.dtype == torch.float32 and law is None and w_gate_up.is_cuda and w_gate_up.stride(1) == 1 and a.is_cuda and a.stride(1) == 1
+            and a.untyped_storage().data_ptr() != out.untyped_storage().data_ptr()):      # (its blocks read `a` while others write)
+        if tuple(gate_up.shape) != (m, two_i) or gate_up.dtype != torch.float32 or not gate_up.is_cuda or gate_up.stride(1) != 1:
+            raise KernelError("gemm_swiglu: gate_up is float rows [M, 2I] on the GPU")
         _check(lib().cisr_gemm_f32_swiglu(a.data_ptr(), a.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), _dev(out, "out"), out.stride(0),
                                           m, inter, k, _stream()), "gemm_swiglu")
         return out

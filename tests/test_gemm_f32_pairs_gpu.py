@@ -24,6 +24,7 @@ def test_gated_product(rows, inter, K):
     want = torch.nn.functional.silu(z[:, :inter]) * z[:, inter:]
     # sums of K products in at least eight runs: 3e-7; the exponential's and the quotient's roundings are of that size
     assert off(out, want) < 1e-6 and off(out, want) < 1.05 * off(apart, want) + 1e-9
+    assert torch.equal(out, apart)
     with pytest.raises(ops.KernelError):
         ops.gemm_swiglu(a, w, out)
 
@@ -55,11 +56,24 @@ def test_projection_with_rotation_and_pages(rows, heads, kv_heads, dim, K, own):
             ops.rope_scatter(both, pos, slots if own else None, cos, sin, *cache, heads, kv_heads, dim, page)
             q = both[:, :heads * dim].contiguous()
         made.append((q, k, v))
-    # the same sums; the rotation is two products and a sum, which may be contracted either way (2^-24 of the larger one)
+    # the same sums, and the rotation's two products and sum are contracted alike
     for x, y in zip(*made):
-        assert torch.isfinite(x).all() and (x - y).abs().max() <= 1e-6 * y.abs().max()
-    assert torch.equal(made[0][2], made[1][2])
+        assert torch.isfinite(x).all() and torch.equal(x, y)
     z = (a.double() @ w.double().T)[:, :heads * dim].view(rows, heads, dim)
     c, s = cos.double()[pos.long()][:, None], sin.double()[pos.long()][:, None]
     lo, hi = z[..., :dim // 2], z[..., dim // 2:]
     assert off(made[0][0].view(rows, heads, dim), torch.cat([lo * c - hi * s, hi * c + lo * s], -1)) < 1e-6
+
+
+def test_gated_product_refuses_and_takes_what_it_did_with_two_kernels():
+    """The buffer for the product of gate and up is checked although nothing is written to it; a result may lie where the rows were."""
+    from runtime.kernels import ops
+    rows, width = 19, 48
+    a, w = torch.randn(rows, width, device=DEV), torch.randn(2 * width, width, device=DEV)
+    both, out = torch.empty(rows, 2 * width, device=DEV), torch.empty(rows, width, device=DEV)
+    for wrong in (both[:, :width], both[:-1], both.double(), both.bfloat16(), both.cpu(), torch.empty(2 * width, rows, device=DEV).t()):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_swiglu(a, w, out, gate_up=wrong)
+    ops.gemm_swiglu(a, w, out, gate_up=both)
+    ops.gemm_swiglu(a, w, a, gate_up=both)
+    assert torch.equal(a, out)
