@@ -5,7 +5,7 @@ new tokens at positions start..start+count-1.  Flattened, that gives T token
 rows.  All per-row and per-segment metadata sits in int32 device tensors; parts
 never look at request identities.
 """
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 
 import numpy as np
 import torch
@@ -47,6 +47,7 @@ class Batch:
     decode_only: bool     # every segment brings exactly one token
     launch_values: dict   # StepArray -> its launch value for this step
     rows: int = 0         # rows that the step is padded to (0: not padded)
+    made: dict = field(default_factory=dict)      # what one array's filling may leave for another's of this step
 
 
 class StepContext:

@@ -58,20 +58,21 @@ def fill_tasks(tasks, counts, rows_per_tile, starts=None, skip_single=False):
     number of keys they attend to, most first: blocks are handed out in this order, and the
     long ones must not be the last to start.  `skip_single`: segments of one row get no tile
     (they are attended to by a launch of their own)."""
-    n = row = 0
-    for seg, count in enumerate(counts):
-        tiles = 0 if skip_single and count == 1 else -(-count // rows_per_tile)
-        firsts = np.arange(tiles, dtype=np.int64) * rows_per_tile
-        tasks[n:n + tiles, 0] = seg
-        tasks[n:n + tiles, 1] = row + firsts
-        tasks[n:n + tiles, 2] = np.minimum(rows_per_tile, count - firsts)
-        tasks[n:n + tiles, 3] = 0 if starts is None else int(starts[seg]) + firsts + 1
-        n += tiles
-        row += count
-    if starts is not None and n > 1:
-        first_row = np.concatenate(([0], np.cumsum(counts)))[tasks[:n, 0]]
-        keys = np.asarray(starts, dtype=np.int64)[tasks[:n, 0]] + (tasks[:n, 1] - first_row) + tasks[:n, 2]
-        tasks[:n] = tasks[:n][np.argsort(-keys, kind="stable")]
+    counts = np.asarray(counts, dtype=np.int64)
+    tiles = -(-counts // rows_per_tile)
+    if skip_single:
+        tiles[counts == 1] = 0
+    n = int(tiles.sum())
+    seg = np.repeat(np.arange(len(counts)), tiles)
+    firsts = (np.arange(n) - np.repeat(np.cumsum(tiles) - tiles, tiles)) * rows_per_tile
+    made = np.zeros((n, 4), dtype=np.int64)
+    made[:, 0] = seg
+    made[:, 1] = (np.cumsum(counts) - counts)[seg] + firsts
+    made[:, 2] = np.minimum(rows_per_tile, counts[seg] - firsts)
+    if starts is not None:
+        made[:, 3] = np.asarray(starts, dtype=np.int64)[seg] + firsts + 1
+        made = made[np.argsort(-(made[:, 3] + made[:, 2]), kind="stable")]
+    tasks[:n] = made
     return n
 
 
@@ -118,8 +119,10 @@ class SingleRows:
         return unit * 5 // 8 if kind == "deep" else unit // 2
 
     def launch_value(self, batch):
+        if batch.decode_only or max(batch.starts) + 1 < self.split_from:
+            return 0
         singles = [start + 1 for start, count in zip(batch.starts, batch.counts) if count == 1]
-        if not singles or len(singles) == len(batch.counts) or max(singles) < self.split_from or max(singles) < self.least(len(singles), batch):
+        if not singles or max(singles) < self.split_from or max(singles) < self.least(len(singles), batch):
             return 0
         return len(singles)
 
@@ -139,8 +142,7 @@ class SingleTokens:
         return 0
 
     def launch_value(self, batch):
-        singles = sum(count == 1 for count in batch.counts)
-        return singles if singles < len(batch.counts) else 0
+        return 0 if batch.decode_only else batch.counts.count(1)
 
     def fill(self, out, batch, value):
         pass
@@ -212,10 +214,11 @@ class RowPieces:
             if blocks <= 0.85 * 256 * -(-blocks // 256):
                 return 1
             even = 0.66 if rows * self.chunks <= 512 else 0.0
-        if self.seen and longest > self.seen:
-            longest, keys = self.seen, sum(min(start + 1, self.seen) for start in batch.starts)
-        else:
-            keys = sum(batch.starts) + n
+        if even in (0.0, 1.0):
+            return int(even)
+        keys, seen = sum(batch.starts) + n, self.seen
+        if seen and longest > seen:
+            longest, keys = seen, sum([start + 1 if start < seen else seen for start in batch.starts])
         return int(keys <= even * rows * longest)
 
     def fill(self, out, batch, value):
@@ -267,8 +270,14 @@ class TileTasks:
             tasks[:n, 2] = 1
             tasks[:n, 3] = 0
         else:
+            # (layers whose single rows leave the launch by different rules mostly decide alike: one list for both is made once)
             skip = self.singles is not None and batch.launch_values.get(self.singles, 0) > 0
+            made = batch.made.get((self.rows_per_tile, skip))
+            if made is not None and len(made) == len(out):
+                out[:] = made
+                return
             n = fill_tasks(tasks, batch.counts, self.rows_per_tile, batch.starts, skip_single=skip)
+            batch.made[self.rows_per_tile, skip] = out
         tasks[n:] = (-1, 0, 0, 0)
 
 

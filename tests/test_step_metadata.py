@@ -90,6 +90,29 @@ def test_step_arrays_of_the_attention_kernels():
     assert sorted(tasks[tasks[:, 0] >= 0][:, 0].tolist()) == [0, 1, 1, 2, 3]
 
 
+def test_a_steps_tiles_are_made_once_for_layers_that_decide_alike(monkeypatch):
+    from runtime.kernels import attention
+    made, fill = [], attention.fill_tasks
+    monkeypatch.setattr(attention, "fill_tasks", lambda *a, **kw: (made.append(1), fill(*a, **kw))[1])
+    near, far = SingleRows(100), SingleRows(1000)
+    lists = [TileTasks(4, near), TileTasks(4, far), TileTasks(4), TileTasks(8, far)]
+
+    def filled(contexts):
+        starts = [c - 1 for c in contexts] + [0]
+        batch = Batch([1] * len(contexts) + [9], starts, np.arange(len(starts), dtype=np.int32), False, {})
+        for s in (near, far):
+            batch.launch_values[s] = s.launch_value(batch)
+        made.clear()
+        outs = [np.full(t.words(16, 4), 99, dtype=np.int32) for t in lists]
+        for t, out in zip(lists, outs):
+            t.fill(out, batch, None)
+        return outs, len(made)
+    (a, b, c, d), n = filled([50, 60])
+    assert n == 2 and (a == b).all() and (a == c).all() and (a.reshape(-1, 4)[:, 2] == 1).sum() == 3 and (d.reshape(-1, 4)[:, 0] == -1).any()
+    (a, b, c, d), n = filled([50, 600])
+    assert n == 3 and (b == c).all() and (a.reshape(-1, 4)[:, 2] == 1).sum() == 1
+
+
 def test_rows_of_a_decode_step_longest_first():
     """The order in which an unsplit decode launch hands out its blocks: rows by keys, most first, rows of equal
     length in their own order, then the padding rows of a captured program; a mixed step lists every row in place."""
