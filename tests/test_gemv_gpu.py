@@ -207,3 +207,17 @@ def test_rows_whose_norm_has_run_are_asked_about_as_such(ops):
         np.testing.assert_allclose(f64(got), f64(x) @ f64(w).T, rtol=1e-4, atol=1e-4)
     finally:
         ops.set_gemv(8, 0)
+
+
+@pytest.mark.parametrize("N, K", [(576, 1536), (1000, 1032), (2048, 2048), (6144, 520), (24, 4096)])
+def test_rows_in_groups_that_read_the_same_weights(ops, N, K):
+    """Narrow outputs of 17 to 64 rows run as groups of rows, whose loads of the weights are ordinary ones."""
+    a, w, r = rnd(64, K, dtype=torch.bfloat16, seed=6), rnd(N, K, dtype=torch.bfloat16, seed=7, scale=K ** -0.5), rnd(64, N, seed=8)
+    want, of = f64(r) + f64(a) @ f64(w).T, {}
+    for M in (17, 32, 33, 48, 49, 64):
+        of[M] = r[:M].clone()
+        ops.gemm(a[:M], w, of[M], residual=of[M])
+        # sums of K exact products in float32
+        np.testing.assert_allclose(f64(of[M]), want[:M], rtol=1e-4, atol=1e-4)
+        if N <= 2048:       # (sixteen waves a block: one order of a sum, whatever rows are beside it)
+            assert torch.equal(of[M][:17], of[17])
