@@ -365,9 +365,9 @@ def prompt_form(rows, n_segments, span, heads, kv_heads, head_dim, page_size, tu
     if long_portions and head_dim > 128 and page_size >= 8:
         # Large heads: the block of 64 items takes 1.4 us a step, a tile's four waves 0.8 (each step's keys straight from the
         # caches, for 16 items).  It is ahead once the tiles wait for the caches: us as tiles / deep, 16 heads of 256 over one key
-        # head, 1,000 rows (250 blocks) 91 / 56, 700 and 1,300 rows 186 / 77, 4,096 rows 811 / 292; 8 heads of 192 over 2, 2,048 rows
-        # (256 blocks) 107 / 77.  At 128 blocks it depends on the chain: 512 rows of 16 heads over one 40 / 33, 256 rows of 24 heads
-        # of 160 over one 25 / 18, the same rows behind 3,000 keys 90 / 107.
+        # head, 1,000 rows (250 blocks) 91 / 50, 700 and 1,300 rows 186 / 72, 4,096 rows 811 / 282; 8 heads of 192 over 2, 2,048 rows
+        # (256 blocks) 107 / 75.  At 128 blocks it depends on the chain: 512 rows of 16 heads over one 40 / 29, 256 rows of 24 heads
+        # of 160 over one 25 / 14, the same rows behind 3,000 keys 75 / 106.
         blocks = -(-rows // (64 // heads_per_chunk)) * kv_heads * -(-group // heads_per_chunk)
         if blocks >= (96 if span <= 512 else 192) if tuning.deep_tiles is None else tuning.deep_tiles:
             return "deep", 1, 1
@@ -550,7 +550,8 @@ def single_rows_stream(blocks):
     asked for, many do not.  us non-temporal / plain: 32 heads of 128 over 8, 8 rows of 4,000 keys and a portion of 256 71 / 60, 8 of 2,000
     and 1,024 50 / 48, 16 of 3,000 and 256 63 / 58, 30 of 900 and 256 30 / 33, 30 of 2,000 and 2,048 107 / 117; 9 heads of 64 over 3,
     8 of 4,000 and 1,024 34 / 23, 50 of 3,000 and 1,024 35 / 31; 32 heads of 64, 3 of 3,000 and 256 30 / 26, 8 of 900 and 30 20 / 21, 30 of 3,000
-    and 256 128 / 136.  Where the number is rounded up to 256 the line is crossed early: 20 of 2,000 and 256, 32 heads of 128 over 8, 46 / 38."""
+    and 256 128 / 136.  Where the number is rounded up to 256 the line is crossed early: 20 of 2,000 and 256, 32 heads of 128 over 8, 46 / 38;
+    and below it the one place found where plain loads lose is halves beside about a block a compute unit (8 heads of 128, 16 of 900 and 1,024 23 / 26)."""
     return blocks >= 256 or blocks == 0      # (none: one kernel for the portions of all steps)
 
 
