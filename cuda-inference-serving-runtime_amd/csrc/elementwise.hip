@@ -215,33 +215,52 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ x, const TD* __restrict__
     for (int d = threadIdx.x; d < dim; d += 256) store_f32(dst + d, xr[d] * scale * w[d]);
 }
 
-// The same for a bf16 delta and rows of a multiple of four, 16-byte aligned (8 for the delta): one wavefront a
-// row, as rmsnorm_wave_kernel, which it equals bit for bit on the summed rows.
-template <typename T, int R>
+// The same for a bf16 delta or (SUMS) the float sums of `slices` slices [slices][n_rows][dim], added in slice order and then to x, and rows
+// of a multiple of four, 16-byte aligned (8 for the bf16 delta): one wavefront a row, as rmsnorm_wave_kernel, which it equals bit
+// for bit on the summed rows.  For steps of many rows; 1,061 rows of 2,048 with two slices move 39 MB.
+template <typename T, int R, bool SUMS>
 __global__ void __launch_bounds__(256)
-add_rmsnorm_wave_kernel(float* x, const bf16_t* __restrict__ delta, const float* __restrict__ w, T* __restrict__ y,
+add_rmsnorm_wave_kernel(float* x, const void* __restrict__ delta, int slices, const float* __restrict__ w, T* __restrict__ y,
                         int n_rows, int dim, float eps) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;   // (uniform: the row's loads of indices are scalar)
     const int row = blockIdx.x * 4 + wave;
     if (row >= n_rows) return;
     const int n4 = dim / 4;
     float4* xr = (float4*)(x + (size_t)row * dim);
-    const uint2* dr = (const uint2*)(delta + (size_t)row * dim);
+    const uint2* dr = (const uint2*)delta + (size_t)row * n4;
     const float4* w4 = (const float4*)w;
-    float4 v[R], g[R];
-    uint2 d[R];
+    float4 v[R], g[R], sum[SUMS ? R : 1];
+    uint2 d[SUMS ? 1 : R];
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         const int c = min(lane + WAVE * i, n4 - 1);   // past the row: a copy of its last chunk, not counted or stored
         v[i] = xr[c];
-        d[i] = dr[c];
+        if (SUMS) sum[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        else d[i] = dr[c];
         g[i] = w4[c];
     }
+    if (SUMS)
+        for (int s = 0; s < slices; s += 2) {          // two slices' loads at a time; an odd last one is read twice and added once
+            const float4* pr = (const float4*)delta + ((size_t)s * n_rows + row) * n4;
+            const float4* pn = (const float4*)delta + ((size_t)min(s + 1, slices - 1) * n_rows + row) * n4;
+            float4 p[R], q[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i) { p[i] = pr[min(lane + WAVE * i, n4 - 1)]; q[i] = pn[min(lane + WAVE * i, n4 - 1)]; }
+#pragma unroll
+            for (int i = 0; i < R; ++i) { sum[i].x += p[i].x; sum[i].y += p[i].y; sum[i].z += p[i].z; sum[i].w += p[i].w; }
+            if (s + 1 < slices)
+#pragma unroll
+                for (int i = 0; i < R; ++i) { sum[i].x += q[i].x; sum[i].y += q[i].y; sum[i].z += q[i].z; sum[i].w += q[i].w; }
+        }
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-        v[i].x += __uint_as_float(d[i].x << 16); v[i].y += __uint_as_float(d[i].x & 0xffff0000u);
-        v[i].z += __uint_as_float(d[i].y << 16); v[i].w += __uint_as_float(d[i].y & 0xffff0000u);
+        if (SUMS) {
+            v[i] = make_float4(sum[i].x + v[i].x, sum[i].y + v[i].y, sum[i].z + v[i].z, sum[i].w + v[i].w);
+        } else {
+            v[i].x += __uint_as_float(d[i].x << 16); v[i].y += __uint_as_float(d[i].x & 0xffff0000u);
+            v[i].z += __uint_as_float(d[i].y << 16); v[i].w += __uint_as_float(d[i].y & 0xffff0000u);
+        }
         if (lane + WAVE * i >= n4) continue;
         xr[lane + WAVE * i] = v[i];
         ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
@@ -261,16 +280,18 @@ add_rmsnorm_wave_kernel(float* x, const bf16_t* __restrict__ delta, const float*
     }
 }
 
-template <typename T>
-static int launch_add_rmsnorm_wave(float* x, const bf16_t* delta, const float* w, T* y, int rows, int dim, float eps,
+template <typename T, bool SUMS>
+static int launch_add_rmsnorm_wave(float* x, const void* delta, int slices, const float* w, T* y, int rows, int dim, float eps,
                                    hipStream_t stream) {
     const int blocks = (rows + 3) / 4, chunks = (dim / 4 + WAVE - 1) / WAVE;
-    if (chunks <= 1) add_rmsnorm_wave_kernel<T, 1><<<blocks, 256, 0, stream>>>(x, delta, w, y, rows, dim, eps);
-    else if (chunks <= 2) add_rmsnorm_wave_kernel<T, 2><<<blocks, 256, 0, stream>>>(x, delta, w, y, rows, dim, eps);
-    else if (chunks <= 4) add_rmsnorm_wave_kernel<T, 4><<<blocks, 256, 0, stream>>>(x, delta, w, y, rows, dim, eps);
-    else if (chunks <= 8) add_rmsnorm_wave_kernel<T, 8><<<blocks, 256, 0, stream>>>(x, delta, w, y, rows, dim, eps);
-    else if (chunks <= 16) add_rmsnorm_wave_kernel<T, 16><<<blocks, 256, 0, stream>>>(x, delta, w, y, rows, dim, eps);
-    else add_rmsnorm_wave_kernel<T, 32><<<blocks, 256, 0, stream>>>(x, delta, w, y, rows, dim, eps);
+#define ADD_NORM(R) add_rmsnorm_wave_kernel<T, R, SUMS><<<blocks, 256, 0, stream>>>(x, delta, slices, w, y, rows, dim, eps)
+    if (chunks <= 1) ADD_NORM(1);
+    else if (chunks <= 2) ADD_NORM(2);
+    else if (chunks <= 4) ADD_NORM(4);
+    else if (chunks <= 8) ADD_NORM(8);
+    else if (chunks <= 16) ADD_NORM(16);
+    else ADD_NORM(32);
+#undef ADD_NORM
     return CISR_LAUNCH_CHECK();
 }
 
@@ -281,8 +302,18 @@ extern "C" int cisr_add_rmsnorm_bf16(float* x, const void* delta, const float* w
     if (rows <= 0) return 0;
     if (dim <= 0 || dim % 4 || dim > 8192 || (uintptr_t)x % 16 || (uintptr_t)delta % 8 || (uintptr_t)w % 16 || (uintptr_t)y % 16)
         return (int)hipErrorInvalidValue;
-    if (out_dtype == DT_F32) return launch_add_rmsnorm_wave<float>(x, (const bf16_t*)delta, w, (float*)y, rows, dim, eps, stream);
-    return launch_add_rmsnorm_wave<bf16_t>(x, (const bf16_t*)delta, w, (bf16_t*)y, rows, dim, eps, stream);
+    if (out_dtype == DT_F32) return launch_add_rmsnorm_wave<float, false>(x, delta, 0, w, (float*)y, rows, dim, eps, stream);
+    return launch_add_rmsnorm_wave<bf16_t, false>(x, delta, 0, w, (bf16_t*)y, rows, dim, eps, stream);
+}
+
+// The same with the sums of `slices` slices, parts[slices][rows][dim] (float, 16-byte aligned), in the delta's place.
+extern "C" int cisr_add_rmsnorm_sums(float* x, const float* parts, int slices, const float* w, void* y, int rows, int dim, float eps,
+                                     int out_dtype, hipStream_t stream) {
+    if (rows <= 0) return 0;
+    if (slices < 1 || dim <= 0 || dim % 4 || dim > 8192 || (uintptr_t)x % 16 || (uintptr_t)parts % 16 || (uintptr_t)w % 16 || (uintptr_t)y % 16)
+        return (int)hipErrorInvalidValue;
+    if (out_dtype == DT_F32) return launch_add_rmsnorm_wave<float, true>(x, parts, slices, w, (float*)y, rows, dim, eps, stream);
+    return launch_add_rmsnorm_wave<bf16_t, true>(x, parts, slices, w, (bf16_t*)y, rows, dim, eps, stream);
 }
 
 extern "C" int cisr_add_rmsnorm(float* x, const void* delta, const float* w, void* y, int rows, int dim,

@@ -1,0 +1,23 @@
+// Arguments of the ring products (gemm_ring.inc) and the entry points of the units that hold their tiles (so that the tiles
+// compile in parallel).
+#pragma once
+#include "common.h"
+
+enum { RING_STORE = 0, RING_GATED = 1, RING_FLOAT = 2 };
+
+struct RingArgs {
+    const bf16_t* A; int lda;
+    const bf16_t* W; int ldw;
+    void* C; int ldc;                  // bf16 (RING_STORE, RING_GATED) or float (RING_FLOAT)
+    const float* R; int ldr;           // RING_FLOAT with one slice: a residual, which may be C itself; else null
+    int M, N, K;
+    int dual_off; GateLaw law;         // RING_GATED: W = [gate; up], `dual_off` rows apart; the activation's law
+    int act;                           // RING_STORE: an ungated activation (ACT_*) before the store
+    int slices;                        // RING_FLOAT: parts of the inner size; slice s writes C + s M ldc
+};
+
+// one function per unit; false: the unit does not hold this tile
+int cisr_ring_launch_a(const RingArgs& a, int tile, int mode, hipStream_t stream);
+int cisr_ring_launch_b(const RingArgs& a, int tile, int mode, hipStream_t stream);
+int cisr_ring_launch_c(const RingArgs& a, int tile, int mode, hipStream_t stream);
+int cisr_ring_launch_d(const RingArgs& a, int tile, int mode, hipStream_t stream);

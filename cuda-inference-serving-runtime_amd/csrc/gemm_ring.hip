@@ -1,0 +1,96 @@
+// Which tile and how many slices a ring product (gemm_ring.inc) takes, and its entry points.
+#include "gemm_ring.h"
+#include <algorithm>
+#include <cmath>
+
+namespace {
+
+// What a round of blocks takes (one a compute unit, 256 of them), us on an MI355X: `start` and `step` for every 64 of the inner size
+// with all units busy, `half` with half of them (less contention and a higher clock).  Measured with bf16 results, 16 x 16 and
+// 8 x 16 tiles, inner sizes of 576, 2,048 and 8,192; `start` has the launch, the first copies and the stores.
+struct Tile { int rows, cols; float start, step, half; };
+constexpr Tile TILES[] = {
+    {64, 64, 3.4f, 0.235f, 0.180f},    {64, 128, 4.4f, 0.355f, 0.272f},   {128, 64, 3.9f, 0.344f, 0.264f},   {96, 128, 4.9f, 0.415f, 0.325f},
+    {128, 128, 5.6f, 0.496f, 0.377f},  {160, 128, 6.1f, 0.589f, 0.437f},  {192, 128, 6.7f, 0.671f, 0.507f},  {224, 128, 7.6f, 0.776f, 0.588f},
+    {256, 128, 8.1f, 0.894f, 0.671f},  {64, 256, 5.2f, 0.590f, 0.590f},   {96, 256, 6.2f, 0.739f, 0.700f},   {128, 256, 7.9f, 0.859f, 0.780f},
+    {160, 256, 8.6f, 1.029f, 0.855f},  {192, 256, 9.1f, 1.228f, 1.228f},  {224, 256, 10.2f, 1.389f, 1.308f}, {256, 256, 11.4f, 1.505f, 1.347f},
+    {288, 256, 12.3f, 1.665f, 1.395f},
+};
+constexpr int UNITS = 256, MOST_SLICES = 8, LEAST_STEPS = 4;
+
+struct Plan { int tile, slices; float us; };
+
+float rounds_us(const Tile& t, long long blocks, int steps) {
+    const long long full = blocks / UNITS, rest = blocks % UNITS;
+    float us = full * (t.start + steps * t.step);
+    if (rest) us += t.start + steps * (t.half + (t.step - t.half) * std::max(0.f, 2.f * rest / UNITS - 1.f));
+    return us;
+}
+
+// The least of the model's times.  `slices` 0: any number of them, whose float sums are written and read once more (at 5 TB/s) by a
+// kernel that mostly runs anyway (the norm that follows).
+Plan plan_of(int M, int N, int K, bool gated, int slices) {
+    Plan best{0, 1, INFINITY};
+    const int steps = K / 64, cols = gated ? 2 * N : N;
+    for (const Tile& t : TILES) {
+        const long long tiles = (long long)((M + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols);
+        for (int s = slices ? slices : 1; s <= (slices ? slices : MOST_SLICES); ++s) {
+            if (s > 1 && steps / s < LEAST_STEPS) break;
+            float us = rounds_us(t, tiles * s, (steps + s - 1) / s);
+            if (s > 1) us += (float)s * M * N * 8 / 5e6f + 0.5f;
+            if (us < best.us) best = {t.rows * 1000 + t.cols, s, us};
+        }
+    }
+    return best;
+}
+
+bool fits(const RingArgs& a, int out_bytes) {
+    const long long reach = ((long long)std::max(a.dual_off, 0) + 512) * a.ldw * 2;
+    return a.M > 0 && a.N > 0 && a.N % 4 == 0 && a.K > 0 && a.K % 64 == 0 && a.lda >= a.K && a.ldw >= a.K && a.lda % 8 == 0 && a.ldw % 8 == 0 &&
+           (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0 && a.ldc >= a.N && a.ldc % 4 == 0 && (uintptr_t)a.C % (4 * out_bytes) == 0 &&
+           (!a.R || (a.ldr % 4 == 0 && (uintptr_t)a.R % 16 == 0)) && (long long)a.lda * 2 * 512 < 0x7fffffffll && reach < 0x7fffffffll;
+}
+
+int launch(const RingArgs& a, int tile, int mode, hipStream_t stream) {
+    const int rows = tile / 1000, cols = tile % 1000;
+    if (cols == 256 && rows >= 224) return cisr_ring_launch_a(a, tile, mode, stream);
+    if (cols == 256 && rows >= 96) return cisr_ring_launch_b(a, tile, mode, stream);
+    if (cols == 256 || (cols == 128 && rows >= 192)) return cisr_ring_launch_c(a, tile, mode, stream);
+    return cisr_ring_launch_d(a, tile, mode, stream);
+}
+
+}  // namespace
+
+// How many slices a product whose inner size may be cut is best cut into.  0: not a shape of these kernels.
+extern "C" int cisr_gemm_ring_slices(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % 4) return 0;
+    return plan_of(M, N, K, false, 0).slices;
+}
+
+// C = A . W^T, bf16 or float; R (float C only) is added, and may be C; `act` (bf16 C only): an ungated activation.  `tile` 0: the model's.
+extern "C" int cisr_gemm_ring_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R, int ldr, int M, int N,
+                                   int K, int out_dtype, int act, int tile, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    const bool wide = out_dtype == DT_F32;
+    const RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, C, ldc, R, ldr, M, N, K, 0, GateLaw{}, act, 1};
+    if (!fits(a, wide ? 4 : 2) || (R && !wide) || (act && wide) || act < ACT_NONE || act > ACT_RELU2) return (int)hipErrorInvalidValue;
+    return launch(a, tile ? tile : plan_of(M, N, K, false, 1).tile, wide ? RING_FLOAT : RING_STORE, stream);
+}
+
+// C = act(A . Wg^T, A . Wu^T), W = [Wg; Wu] with `dual_off` rows between the blocks; the law as GateLaw.
+extern "C" int cisr_gemm_ring_bf16_gated(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N, int K, int dual_off,
+                                         float limit, float slope, float shift, int tile, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    const RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, GateLaw{limit, slope, shift}, 0, 1};
+    if (!fits(a, 2) || dual_off < N) return (int)hipErrorInvalidValue;
+    return launch(a, tile ? tile : plan_of(M, N, K, true, 1).tile, RING_GATED, stream);
+}
+
+// The product's partial sums, parts[slices][M][N] (float): to be added in slice order by the kernel that reads them next.
+extern "C" int cisr_gemm_ring_partials_bf16(const void* A, int lda, const void* W, int ldw, float* parts, int M, int N, int K, int slices,
+                                            int tile, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    const RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, parts, N, nullptr, 0, M, N, K, 0, GateLaw{}, 0, slices};
+    if (!fits(a, 4) || slices < 1 || slices > K / 64) return (int)hipErrorInvalidValue;
+    return launch(a, tile ? tile : plan_of(M, N, K, false, slices).tile, RING_FLOAT, stream);
+}

@@ -56,6 +56,11 @@ def _declare(h):
         "cisr_gemm_bf16_swiglu": [p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_bf16_tile": [p, i, p, i, p, i, p, i, i, i, i, i, i, p],
         "cisr_gemm_bf16_swiglu_tile": [p, i, p, i, p, i, i, i, i, i, i, p],
+        "cisr_gemm_ring_slices": [i, i, i],
+        "cisr_add_rmsnorm_sums": [p, p, i, p, p, i, i, f, i, p],
+        "cisr_gemm_ring_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, i, p],
+        "cisr_gemm_ring_bf16_gated": [p, i, p, i, p, i, i, i, i, i, f, f, f, i, p],
+        "cisr_gemm_ring_partials_bf16": [p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_skinny_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, p, f, p, p],
         "cisr_qkv_rope_skinny": [p, i, p, i, p, i, i, i, p, f, p, p, p, p, p, p, i, i, i, i, i, p],
         "cisr_attn_f32": [p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, f, i, i, p],
@@ -222,10 +227,20 @@ def partials_ok(x):
             and x.data_ptr() % 16 == 0)
 
 
+def _sums_of(partials, x):
+    """(partial sums or bf16 product, slices or 0) of what gemm_unfinished left for the rows x."""
+    parts, slices = partials
+    if not isinstance(parts, RingSums):
+        return parts, slices
+    if (parts.rows, parts.cols) != tuple(x.shape):
+        raise KernelError("the partial sums belong to other rows")
+    return parts.parts, parts.slices
+
+
 def add_partials(x, partials):
     """x += what gemm_unfinished left (float rows, in place): the partial sums in slice order, or (slices 0) the
-    bf16 product."""
-    parts, slices = partials
+    bf16 product or a RingSums."""
+    parts, slices = _sums_of(partials, x)
     rows, dim = x.shape
     if slices == 0:
         return residual_add(x, parts)
@@ -238,7 +253,7 @@ def add_partials(x, partials):
 
 def rmsnorm_partials(x, partials, weight, out, eps):
     """x += what gemm_unfinished left (in place), out = rmsnorm(x) * weight: one kernel."""
-    parts, slices = partials
+    parts, slices = _sums_of(partials, x)
     rows, dim = x.shape
     if not partials_ok(x) or out.data_ptr() % 16:
         raise KernelError("rmsnorm_partials: contiguous float rows of a multiple of 4 (at most 8192)")
@@ -249,6 +264,10 @@ def rmsnorm_partials(x, partials, weight, out, eps):
         return out
     if parts.numel() < slices * rows * dim:
         raise KernelError("rmsnorm_partials: too few partial sums")
+    if isinstance(partials[0], RingSums):           # (many rows: a wavefront a row)
+        _check(lib().cisr_add_rmsnorm_sums(x.data_ptr(), _dev(parts, "partials", torch.float32), int(slices), wp, op, rows, dim,
+                                           float(eps), _storage(out, "out"), _stream()), "rmsnorm_partials")
+        return out
     _check(lib().cisr_rmsnorm_partials(x.data_ptr(), _dev(parts, "partials", torch.float32), int(slices), wp, op,
                                        rows, dim, float(eps), _storage(out, "out"), _stream()), "rmsnorm_partials")
     return out
@@ -599,6 +618,98 @@ def library_ok(m, w, gated=False, plain=False, floats=False):
             and w.numel() * 2 >= least_bytes)
 
 
+# bf16 products of many rows whose operands go from memory straight into a ring in LDS (csrc/gemm_ring.inc): from this many rows on.
+RING_MIN_ROWS = 65
+RING_MIN_OUTPUTS, RING_MIN_OUTPUTS_K = 500_000, 40
+RING_MIN_OUTPUTS_SHORT, RING_SHORT_K = 250_000, 1024
+RING_PLAIN_FLOPS, RING_PLAIN_COLS = 15e9, 2048
+RING_MOST_FLOPS, RING_GATED_FLOPS = 300e9, 210e9
+
+
+def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
+    """Whether the ring product is the fastest for m rows against the bf16 weights w ([N, K]; `gated`: gate and up).  `fused`: a kernel
+    after the library's product (activation, residual sum) is an epilogue here; `floats`: float results; `cut`: the inner size
+    may be cut.  Measured on an MI355X over 65 to 4,096 rows of the sizes of all designs, us of the other kernels / this one:
+      few outputs stay with the kernels of small tiles: 300 x 960, K 576 5.0 / 5.3, 600 x 960 6.2 / 5.6; 256 x 2,048, K 8,192 28 / 35, 400 rows
+      37 / 33 (the library cuts the inner size); with a short one against the library from half as many on: 256 x 1,024, K 1,024 8.0 / 6.4;
+      what is added to a residual is cut here too, and beats the library at any number of rows: 65 x 2,048, K 8,192 22.7 / 15.5, 1,061 rows
+      66 / 50, 2,048 rows 82 / 70;
+      gate and up with their activation: 128 x 16,384, K 2,048 25.8 / 20.2, 1,061 rows 83 / 66, 2,345 rows 177 / 153, 907 x 28,672,
+      K 4,096 (213 GFLOP) 192 / 213, 2,048 rows 377 / 409;
+      a product that ends with its store: 1,000 x 4,096, K 1,024 13.8 / 13.3, 2,000 rows (17 GFLOP) 21 / 22, 4,000 rows 29 / 35; 2,345 x 2,048, K 2,048
+      29 / 24; float results 2,000 x 8,512, K 2,048 81 / 63, 4,000 rows 138 / 128."""
+    cols, k = w.shape
+    flops, outputs = 2.0 * m * cols * k, m * cols
+    if m < RING_MIN_ROWS or w.dtype != torch.bfloat16 or flops > (RING_GATED_FLOPS if gated else RING_MOST_FLOPS):
+        return False
+    library = library_ok(m, w, gated=gated, plain=not (fused or gated), floats=floats)
+    if library and (gated or cut):
+        return True
+    if outputs < (RING_MIN_OUTPUTS_SHORT if library and k <= RING_SHORT_K else RING_MIN_OUTPUTS + RING_MIN_OUTPUTS_K * k):
+        return False
+    return not library or fused or floats or flops <= RING_PLAIN_FLOPS or cols <= RING_PLAIN_COLS
+
+
+def ring_fits(a, w, out):
+    """Whether the ring product takes these operands (shapes are the caller's to check): an inner size of a multiple of 64, a multiple
+    of four columns, 16-byte rows, results stored four at a time."""
+    n, k = out.shape[1], a.shape[1]
+    return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda and w.is_cuda and out.is_cuda and k % 64 == 0 and n % 4 == 0
+            and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1 and _skinny_ok(a, w) and a.stride(0) >= k and w.stride(0) >= k
+            and out.stride(0) >= n and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0
+            and max(a.stride(0), w.stride(0)) * 1024 < 1 << 31 and (w.shape[0] + 512) * w.stride(0) * 2 < 1 << 31)
+
+
+class RingSums:
+    """A ring product [rows, cols] cut along its inner size: `parts` float [slices * rows * cols], to be added in slice order."""
+
+    def __init__(self, parts, slices, rows, cols):
+        self.parts, self.slices, self.rows, self.cols = parts, int(slices), int(rows), int(cols)
+
+
+def ring_sums(a, w, make_buffer):
+    """The RingSums of a . w^T in floats of the caller's (`make_buffer(floats)`), or None where the product is best not cut."""
+    (m, k), n = a.shape, w.shape[0]
+    slices = int(lib().cisr_gemm_ring_slices(m, n, k))
+    return RingSums(gemm_ring_partials(a, w, make_buffer(slices * m * n), slices), slices, m, n) if slices > 1 else None
+
+
+def gemm_ring(a, w, out, residual=None, act=0, tile=0):
+    """out = a . w^T (+ residual, float rows that may be `out`) by the ring product; `act` (bf16 results): an ungated activation.
+    `tile`: rows * 1000 + columns of a block (0: the fastest by the kernel's model of itself)."""
+    (m, k), n = a.shape, w.shape[0]
+    if (tuple(out.shape) != (m, n) or w.shape[1] != k or not ring_fits(a, w, out) or (act and out.dtype != torch.bfloat16)
+            or (residual is not None and (residual.dtype != torch.float32 or out.dtype != torch.float32 or tuple(residual.shape) != (m, n)
+                                          or residual.stride(1) != 1 or residual.stride(0) % 4 or residual.data_ptr() % 16 or not residual.is_cuda))):
+        raise KernelError("gemm_ring: shape not supported")
+    rp, ldr = (residual.data_ptr(), residual.stride(0)) if residual is not None else (None, 0)
+    _check(lib().cisr_gemm_ring_bf16(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), rp, ldr, m, n, k,
+                                     _storage(out, "out"), int(act), int(tile), _stream()), "gemm_ring")
+    return out
+
+
+def gemm_ring_gated(a, w, out, law=None, tile=0):
+    """out[M, I] = act(a . Wg^T, a . Wu^T), w = [Wg; Wu], by the ring product; `law` as gemm_swiglu."""
+    (m, k), inter = a.shape, w.shape[0] // 2
+    if tuple(out.shape) != (m, inter) or tuple(w.shape) != (2 * inter, k) or out.dtype != torch.bfloat16 or not ring_fits(a, w, out):
+        raise KernelError("gemm_ring_gated: shape not supported")
+    lim, slope, shift = (float(x) for x in law or (0.0, 0.0, 0.0))
+    _check(lib().cisr_gemm_ring_bf16_gated(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), m, inter, k,
+                                           inter, lim, slope, shift, int(tile), _stream()), "gemm_ring_gated")
+    return out
+
+
+def gemm_ring_partials(a, w, parts, slices, tile=0):
+    """parts (contiguous floats [slices * M * N] and more) = the partial sums of a . w^T cut into `slices` along its inner size."""
+    (m, k), n = a.shape, w.shape[0]
+    flat = _dev(parts, "partial sums", torch.float32)
+    if w.shape[1] != k or parts.numel() < slices * m * n or not 1 <= slices <= k // 64 or not ring_fits(a, w, parts.view(-1)[:m * n].view(m, n)):
+        raise KernelError("gemm_ring_partials: shape not supported")
+    _check(lib().cisr_gemm_ring_partials_bf16(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), flat, m, n, k, int(slices), int(tile),
+                                              _stream()), "gemm_ring_partials")
+    return parts
+
+
 def _scratch_bf16(scratch, device, rows, cols):
     return (scratch or DEFAULT_SCRATCH).get("library", rows * cols, torch.bfloat16, device)[:rows * cols].view(rows, cols)
 
@@ -628,6 +739,12 @@ def gemm(a, w, out, residual=None, after_norm=False, scratch=None):
             raise KernelError("gemm: float operands need a float output")
         code = lib().cisr_gemm_f32(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
                                    rp, ldr, m, n, k, _stream())
+    elif (a.dtype == torch.bfloat16 and ring_ahead(m, w, fused=residual is not None, floats=out.dtype == torch.float32, cut=residual is not None)
+          and ring_fits(a, w, out) and (residual is None or (ldr % 4 == 0 and rp % 16 == 0))):
+        sums = None
+        if residual is not None and residual is out and partials_ok(out):
+            sums = ring_sums(a, w, lambda floats: _wide_workspace(scratch, a.device, floats))
+        return gemm_ring(a, w, out, residual) if sums is None else add_partials(out, (sums, 0))
     elif (a.dtype == torch.bfloat16 and library_ok(m, w, plain=residual is None, floats=out.dtype == torch.float32) and a.is_contiguous() and out.is_contiguous()
           and (residual is None or residual is out)):
         if residual is None:
@@ -759,13 +876,16 @@ def _gemm_wide(a, w, out, residual, swiglu, what, scratch=None):
 def gemm_unfinished(a, w, residual, scratch=None):
     """The product a . w^T that is to be added to the float rows `residual`, left unfinished where adding it takes a
     kernel of its own: the wide kernel's partial sums of a product cut into slices, (partial sums [slices, M, N],
-    slices), or the library's bf16 product, (product [M, N], 0); rmsnorm_partials or add_partials then are that
-    kernel.  None (nothing done) for every other product: call gemm."""
+    slices), the ring product's, (a RingSums, 0), or the library's bf16 product, (product [M, N], 0); rmsnorm_partials or
+    add_partials then are that kernel.  None (nothing done) for every other product: call gemm."""
     m, k = a.shape
     n = w.shape[0]
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape[1] != k or tuple(residual.shape) != (m, n)
             or not partials_ok(residual)):
         return None
+    if ring_ahead(m, w, fused=True, cut=True) and ring_fits(a, w, residual):
+        sums = ring_sums(a, w, lambda floats: _wide_workspace(scratch, a.device, floats))
+        return None if sums is None else (sums, 0)       # (one that is not cut: gemm adds it in the product's epilogue)
     if library_ok(m, w):
         if not a.is_contiguous():
             return None
@@ -853,6 +973,8 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         return out
     if out.dtype != a.dtype or a.dtype != w_gate_up.dtype:
         raise KernelError("gemm_swiglu: dtypes differ")
+    if a.dtype == torch.bfloat16 and ring_ahead(m, w_gate_up, gated=True) and ring_fits(a, w_gate_up, out):
+        return gemm_ring_gated(a, w_gate_up, out, law)
     activate = swiglu if law is None else (lambda gu, o: glu_clamped(gu, o, *law))
     if a.dtype == torch.bfloat16 and library_ok(m, w_gate_up, gated=True) and a.is_contiguous():
         product = _scratch_bf16(scratch, a.device, m, two_i)
@@ -1223,6 +1345,10 @@ def gemm_for_norm(a, w, out, make_buffer, scratch=None):
             _check(lib().cisr_gemm_wide_partials_bf16(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), m, n, k,
                                                       _dev(work, "partial sums", torch.float32), work.numel(), _stream()), "gemm_for_norm")
             return Partials(work, need // (m * n), m, n)
+    if (a.dtype == torch.bfloat16 and n <= PARTIALS_MAX_COLS and tuple(out.shape) == (m, n) and w.shape[1] == k
+            and ring_ahead(m, w, fused=True, floats=True, cut=True) and ring_fits(a, w, out)):
+        sums = ring_sums(a, w, make_buffer)
+        return gemm_ring(a, w, out) if sums is None else Partials(sums.parts, sums.slices, m, n)
     return gemm(a, w, out, scratch=scratch)
 
 
@@ -1358,7 +1484,7 @@ def layernorm(x, weight, out, eps, rows=None, bias=None):
 
 def layernorm_partials(x, partials, weight, out, eps, bias=None):
     """x += what gemm_unfinished left (in place), out = layernorm(x) * weight (+ bias): one kernel."""
-    parts, slices = partials
+    parts, slices = _sums_of(partials, x)
     rows, dim = x.shape
     if not partials_ok(x) or out.data_ptr() % 16:
         raise KernelError("layernorm_partials: contiguous float rows of a multiple of 4 (at most 8192)")
@@ -1450,8 +1576,11 @@ def gemm_gelu(a, w, out, kind="gelu", scratch=None, product=None):
     m, k = a.shape
     n = w.shape[0]
     fused = (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and tuple(out.shape) == (m, n)
-             and w.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1 and not library_ok(m, w))
+             and w.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1)
     act = 1 + GELU_KINDS[kind]
+    if fused and ring_ahead(m, w, fused=True) and ring_fits(a, w, out):
+        return gemm_ring(a, w, out, act=act)
+    fused = fused and not library_ok(m, w)
     if fused and m <= SKINNY_ROWS and _skinny_ok(a, w) and not wide_ok(m, w):
         _check(lib().cisr_gemm_skinny_bf16_act(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
                                                m, n, k, BF16, act, _stream()), "gemm_gelu")

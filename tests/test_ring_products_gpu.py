@@ -1,0 +1,169 @@
+"""The ring products (bf16 products of many rows, csrc/gemm_ring.inc) against products in 64 bits: every tile at the edges of its
+rows, columns and inner size, every epilogue, slices of the inner size and what adds them, and the rule that picks them."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+TILES = [64064, 64128, 128064, 96128, 128128, 160128, 192128, 224128, 256128, 64256, 96256, 128256, 160256, 192256, 224256, 256256, 288256]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from runtime.kernels import ops
+    return ops
+
+
+def operands(M, N, K, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(M, K, generator=g, device=DEV).bfloat16(), torch.randn(N, K, generator=g, device=DEV).bfloat16(),
+            torch.randn(M, N, generator=g, device=DEV))
+
+
+def close(got, want, K, half=False):
+    """Float accumulation of K products of standard normals: at most K roundings of half an ulp of a sum below 8 sqrt(K); a bf16
+    result is rounded once more."""
+    bound = K * 2.0 ** -24 * 8 * K ** 0.5 + 1e-6
+    return ((got.double() - want).abs() <= bound + (2.0 ** -8 * want.abs() if half else 0.0)).all().item()
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("K", [64, 128, 320, 576])
+def test_every_tile_at_its_edges(ops, tile, K):
+    """Rows and columns that no tile divides (and fewer than a tile has), inner sizes of one step, of as many as the ring holds, and
+    of more; the rows and columns that no tile owns stay."""
+    rows, cols = tile // 1000, tile % 1000
+    for M, N in ((2 * rows + 5, 2 * cols + 12), (7, 20)):
+        a, w, r = operands(M, N, K, seed=K + M)
+        want = a.double() @ w.double().T
+        held = torch.full((M + 1, N + 8), 7.0, device=DEV)
+        out = held[:M, :N]
+        out.copy_(r)
+        ops.gemm_ring(a, w, out, residual=out, tile=tile)
+        assert close(out, want + r.double(), K) and (held[M:] == 7.0).all() and (held[:, N:] == 7.0).all()
+        half = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.gemm_ring(a, w, half[:M, :N], tile=tile)
+        assert close(half[:M, :N], want, K, half=True) and (half[M:] == 7.0).all() and (half[:, N:] == 7.0).all()
+        ops.gemm_ring(a, w, half[:M, :N], act=3, tile=tile)                      # relu(z)^2 of the rounded product
+        z = want.float().bfloat16().double().clamp(min=0.0)
+        # z may round to the neighbouring bf16 (2^-7 of it, twice that of its square), the square is rounded (2^-8)
+        assert (((half[:M, :N].double() - z * z).abs() <= 6 * 2.0 ** -8 * z * z + 1e-3).all()).item()
+        inter = N // 2 // 4 * 4
+        act = torch.full((M + 1, inter + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        wg = torch.cat([w[:inter], w[-inter:]]).contiguous()
+        gate, up = (x.float().bfloat16().double() for x in (a.double() @ wg[:inter].double().T, a.double() @ wg[inter:].double().T))
+        for law in (None, (7.0, 1.702, 1.0)):
+            ops.gemm_ring_gated(a, wg, act[:M, :inter], law, tile=tile)
+            if law is None:
+                ref = gate / (1 + torch.exp(-gate)) * up
+            else:
+                g, u = gate.clamp(max=7.0), up.clamp(-7.0, 7.0)
+                ref = g / (1 + torch.exp(-1.702 * g)) * (u + 1.0)
+            # gate and up may round to the neighbouring bf16 (2^-8 of each), and the result is rounded
+            assert ((act[:M, :inter].double() - ref).abs() <= 2.0 ** -5 * ref.abs() + 2.0 ** -6 * (gate.abs() + up.abs()) + 1e-3).all()
+            assert (act[M:] == 7.0).all() and (act[:, inter:] == 7.0).all()
+
+
+@pytest.mark.parametrize("tile", [64064, 128128, 128256, 288256])
+@pytest.mark.parametrize("slices", [1, 2, 3, 9])
+def test_slices_and_the_norm_that_adds_them(ops, tile, slices):
+    """Partial sums add up to the product; the norm of many rows equals, bit for bit, the sum made alone and the norm of it."""
+    M, N, K = 131, 260, 576
+    a, w, r = operands(M, N, K, seed=slices)
+    parts = torch.full((slices * M * N + 8,), 7.0, device=DEV)
+    ops.gemm_ring_partials(a, w, parts, slices, tile=tile)
+    assert close(parts[:slices * M * N].view(slices, M, N).double().sum(0), a.double() @ w.double().T, K) and (parts[slices * M * N:] == 7.0).all()
+    left = (ops.RingSums(parts, slices, M, N), 0)
+    weight = 1 + 0.1 * torch.randn(N, device=DEV)
+    for dtype in (torch.bfloat16, torch.float32):
+        alone = ops.add_partials(r.clone(), left)
+        want = ops.rmsnorm(alone, weight, torch.empty(M, N, dtype=dtype, device=DEV), 1e-5)
+        x = r.clone()
+        got = ops.rmsnorm_partials(x, left, weight, torch.empty(M, N, dtype=dtype, device=DEV), 1e-5)
+        assert torch.equal(x, alone) and torch.equal(got, want)
+        x = r.clone()
+        centred = ops.layernorm_partials(x, left, weight, torch.empty(M, N, dtype=dtype, device=DEV), 1e-5)
+        assert torch.equal(x, alone)
+        ref = torch.nn.functional.layer_norm(alone.double(), (N,), weight.double(), eps=1e-5)
+        assert (centred.double() - ref).abs().max().item() <= (2.0 ** -7 * ref.abs().max().item() if dtype == torch.bfloat16 else 1e-5)
+    with pytest.raises(ops.KernelError):
+        ops.add_partials(torch.zeros(M, N + 4, device=DEV), left)
+
+
+@pytest.mark.parametrize("dim", [4, 576, 1028, 8192])
+def test_norm_of_sums_over_the_widths(ops, dim):
+    M, slices = 5, 4
+    parts, r, weight = torch.randn(slices, M, dim, device=DEV), torch.randn(M, dim, device=DEV), torch.randn(dim, device=DEV)
+    left, x = (ops.RingSums(parts.view(-1), slices, M, dim), 0), r.clone()
+    got = ops.rmsnorm_partials(x, left, weight, torch.empty(M, dim, device=DEV), 1e-5)
+    want = parts[0] + parts[1] + parts[2] + parts[3] + r
+    assert torch.equal(x, want) and torch.equal(got, ops.rmsnorm(want, weight, torch.empty(M, dim, device=DEV), 1e-5))
+
+
+def test_what_is_not_taken(ops):
+    a, w, r = operands(70, 64, 128)
+    for bad in ((a[:, :96], w[:, :96], r), (a, w[:62], r[:, :62]), (a[:, 1:65], w[:, :64], r), (a.float(), w.float(), r),
+                (a, w, torch.empty(64, 70, device=DEV).t())):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_ring(*bad)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_ring(a, w, r, tile=32032)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_ring(a, w, torch.empty(70, 64, dtype=torch.bfloat16, device=DEV), residual=r)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_ring_partials(a, w, torch.empty(70 * 64 * 2, device=DEV), 3)
+    assert not ops.ring_fits(a[:, :96], w[:, :96], r) and ops.ring_fits(a, w, r)
+
+
+@pytest.mark.parametrize("M, N, K", [(65, 2048, 2048), (65, 4096, 2048), (700, 1024, 1024), (700, 960, 576), (1061, 576, 1536), (400, 2048, 1024)])
+def test_calls_that_came_to_these_kernels_against_the_others(ops, M, N, K, monkeypatch):
+    """The same calls with the ring products off: rows with a stride, results in views, the residual apart from the output."""
+    a, w, r = operands(M, N, K, seed=M)
+    wide = torch.randn(M, K + 64, device=DEV).bfloat16()
+    wide[:, 64:] = a
+    held = torch.zeros(M, N + 16, device=DEV)
+    gu = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    assert ops.ring_ahead(M, w, fused=True, cut=True) and ops.ring_ahead(M, w, gated=True)
+
+    def calls():
+        x = r.clone()
+        yield ops.gemm(wide[:, 64:], w, x, residual=x)
+        yield ops.gemm(a, w, held[:, 16:], residual=r).clone()
+        yield ops.gemm(a, w, torch.empty(M, N, device=DEV))
+        yield ops.gemm(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV))
+        yield ops.gemm_swiglu(a, w, torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV), gate_up=gu)
+        yield ops.gemm_swiglu(a, w, torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV), gate_up=gu, law=ops.GELU_TANH_LAW)
+        yield ops.gemm_gelu(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), product=gu)
+    here = list(calls())
+    monkeypatch.setattr(ops, "RING_MIN_ROWS", 1 << 30)
+    for i, (got, want) in enumerate(zip(here, calls())):
+        scale = want.double().square().mean().sqrt().item()
+        assert (got.double() - want.double()).norm().item() <= 2.0 ** -7 * want.double().norm().item(), i
+        assert (got.double() - want.double()).abs().max().item() <= 2.0 ** -5 * max(scale, want.abs().max().item()), i
+
+
+def test_on_every_replay_of_a_captured_graph(ops):
+    M, N, K = 300, 2048, 8192
+    a, w, r = operands(M, N, K)
+    a.mul_(0.1)
+    x, gu = r.clone(), torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV)
+
+    def step():
+        ops.gemm(a, w, x, residual=x)
+        ops.gemm_swiglu(a, w, gu)
+    step()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for i in range(4):
+        a.copy_(torch.randn(M, K, device=DEV) * 0.1)
+        x.copy_(r)
+        step()
+        torch.cuda.synchronize()
+        want = x.clone(), gu.clone()
+        x.copy_(r)
+        gu.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(x, want[0]) and torch.equal(gu, want[1]), i
