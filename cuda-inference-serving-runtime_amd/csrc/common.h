@@ -97,11 +97,30 @@ __device__ __forceinline__ float unary_activation(float z, int act) {
     return 0.5f * z * (1.0f + tanhf(0.79788456080286536f * (z + 0.044715f * z * z * z)));
 }
 
+// The gelu with the error function where the result is rounded to bf16: z / 2 erfc(-z / sqrt 2), with erfc(x) = t 2^(p(t) - x^2 / ln 2),
+// t = 1 / (1 + x / 2), for x >= 0 and 2 - erfc(|x|) below; p is a polynomial fitted here (Chebyshev nodes, t from 1/8 to 1) to
+// log2(e^(x^2) erfc(x) / t).  Relative error of erfc 4e-6, also where it is small, where 1 + erf(z) has lost its digits.  A sixth of
+// erff's instructions: as the epilogue of 1,999 x 8,192, K 2,048 the activation took 30 us of 86.
+__device__ __forceinline__ float gelu_to_bf16(float z) {
+    const float x = fabsf(z) * 0.70710678118654752f, t = __builtin_amdgcn_rcpf(fmaf(0.5f, x, 1.0f));
+    float p = 0.0669854358f;
+    p = fmaf(p, t, -0.578201771f); p = fmaf(p, t, 1.67653584f); p = fmaf(p, t, -2.0672853f); p = fmaf(p, t, 0.893760622f);
+    p = fmaf(p, t, -0.20385237f); p = fmaf(p, t, 0.600722373f); p = fmaf(p, t, 1.43684995f); p = fmaf(p, t, -1.82551515f);
+    const float tail = t * __builtin_amdgcn_exp2f(fmaf(-x * 1.4426950408889634f, x, p));
+    return 0.5f * z * (z < 0.f ? tail : 2.0f - tail);
+}
+
+// the activation of a result of type TC
+template <typename TC>
+__device__ __forceinline__ float activation_to(float z, int act) {
+    return sizeof(TC) == 2 && act == ACT_GELU ? gelu_to_bf16(z) : unary_activation(z, act);
+}
+
 // as the epilogue of a product: the sum is rounded to the output's type first, as the path of two kernels does
 template <typename TC>
 __device__ __forceinline__ float activated(float v, int act) {
     if (sizeof(TC) == 2) v = bf16_to_f32(f32_to_bf16(v));
-    return unary_activation(v, act);
+    return activation_to<TC>(v, act);
 }
 
 #define CISR_LAUNCH_CHECK() ((int)hipGetLastError())

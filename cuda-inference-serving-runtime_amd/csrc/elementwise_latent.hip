@@ -374,7 +374,7 @@ extern "C" int cisr_heads_product(const void* a, int lda, int a_head, const void
 template <typename T>
 __global__ void __launch_bounds__(256) gelu_kernel(const T* __restrict__ x, T* __restrict__ out, size_t n, int kind) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) store_f32(out + i, unary_activation(load_f32(x + i), kind + 1));
+    if (i < n) store_f32(out + i, activation_to<T>(load_f32(x + i), kind + 1));
 }
 
 // The same for bf16 in 16-byte words: 2,048 rows of 8,192 39.5 us an element a thread (2-byte accesses), 19.6 so.  A thread's eight
@@ -389,7 +389,7 @@ __global__ void __launch_bounds__(256) gelu_bf16x8_kernel(const uint4* __restric
     uint32_t y[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        y[e] = pack_bf16x2(unary_activation(__uint_as_float(w[e] << 16), kind + 1), unary_activation(__uint_as_float(w[e] & 0xffff0000u), kind + 1));
+        y[e] = pack_bf16x2(activation_to<bf16_t>(__uint_as_float(w[e] << 16), kind + 1), activation_to<bf16_t>(__uint_as_float(w[e] & 0xffff0000u), kind + 1));
     out[i] = make_uint4(y[0], y[1], y[2], y[3]);
 }
 
@@ -398,7 +398,7 @@ template <typename T>
 __global__ void __launch_bounds__(256) bias_act_kernel(const T* __restrict__ x, const float* __restrict__ bias, T* __restrict__ out,
                                                        size_t n, int cols, int kind) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) store_f32(out + i, unary_activation(load_f32(x + i) + bias[i % cols], kind + 1));
+    if (i < n) store_f32(out + i, activation_to<T>(load_f32(x + i) + bias[i % cols], kind + 1));
 }
 
 extern "C" int cisr_bias_act(const void* x, const float* bias, void* out, long long n, int cols, int kind, int dtype, hipStream_t stream) {

@@ -167,3 +167,20 @@ def test_on_every_replay_of_a_captured_graph(ops):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(x, want[0]) and torch.equal(gu, want[1]), i
+
+
+def test_gelu_of_every_bf16_number(ops):
+    """The gelu of bf16 results against 64 bits over all bf16 numbers from 2^-20 to 16 and their negatives: rounded to the nearest
+    bf16 but for sums near a tie (the kernel's 4e-6 relative against a rounding of 2^-9: fewer than one in a hundred), never
+    further than the next one."""
+    bits = torch.arange(0x3580, 0x4181, dtype=torch.int32)
+    z = torch.cat([bits, bits | 0x8000]).to(torch.int16).view(torch.bfloat16).to(DEV)
+    want = 0.5 * z.double() * torch.special.erfc(-z.double() * 0.5 ** 0.5)
+    want = torch.where(want.abs() < 1e-36, 0.0, want)
+    got = ops.gelu(z, torch.empty_like(z)).double()
+    got = torch.where(got.abs() < 1e-36, 0.0, got)
+    near = want.float().bfloat16().double()
+    assert ((got - want).abs() <= 2.0 ** -7 * want.abs()).all() and (got != near).float().mean().item() < 0.01
+    special = torch.tensor([0.0, float("inf"), float("nan")], dtype=torch.bfloat16, device=DEV)
+    out = ops.gelu(special, torch.empty_like(special))
+    assert out[0] == 0 and out[1] == float("inf") and out[2].isnan()
