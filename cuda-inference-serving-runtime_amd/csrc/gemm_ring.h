@@ -3,7 +3,7 @@
 #pragma once
 #include "common.h"
 
-enum { RING_STORE = 0, RING_GATED = 1, RING_FLOAT = 2 };
+enum { RING_STORE = 0, RING_GATED = 1, RING_FLOAT = 2, RING_ROPE = 3 };
 
 struct RingArgs {
     const bf16_t* A; int lda;
@@ -14,6 +14,9 @@ struct RingArgs {
     int dual_off; GateLaw law;         // RING_GATED: W = [gate; up], `dual_off` rows apart; the activation's law
     int act;                           // RING_STORE: an ungated activation (ACT_*) before the store
     int slices;                        // RING_FLOAT: parts of the inner size; slice s writes C + s M ldc
+    // RING_ROPE: W = [Wq; Wk; Wv] (or Wq alone, kv_heads 0); C: q, rows of ldc; k and v go into the pages at `slots`
+    const int* positions; const int* slots; const float* cos_tab; const float* sin_tab;
+    bf16_t* kcache; bf16_t* vcache; int heads, kv_heads, dim, page_size, max_pos;
 };
 
 // one function per unit; false: the unit does not hold this tile

@@ -94,3 +94,20 @@ extern "C" int cisr_gemm_ring_partials_bf16(const void* A, int lda, const void* 
     if (!fits(a, 4) || slices < 1 || slices > K / 64) return (int)hipErrorInvalidValue;
     return launch(a, tile ? tile : plan_of(M, N, K, false, slices).tile, RING_FLOAT, stream);
 }
+
+// The projection W = [Wq; Wk; Wv] of bf16 rows with the rotary embedding (pairs (i, i + dim / 2) of whole heads) and the cache write:
+// q into q_out (rows of ldq), k and v into the pages at `slots` (a negative one: nowhere); kv_heads 0: W = Wq only.
+extern "C" int cisr_gemm_ring_rope(const void* A, int lda, const void* W, int ldw, void* q_out, int ldq, int M, int K, const int* positions,
+                                   const int* slots, const float* cos_tab, const float* sin_tab, void* kcache, void* vcache, int heads,
+                                   int kv_heads, int dim, int page_size, int max_pos, int tile, hipStream_t stream) {
+    if (M <= 0 || heads <= 0) return 0;
+    if (dim <= 0 || dim % 32 || kv_heads < 0 || max_pos <= 0 || !positions || !cos_tab || !sin_tab || (uintptr_t)cos_tab % 16 || (uintptr_t)sin_tab % 16 ||
+        (kv_heads && (!slots || !kcache || !vcache || page_size <= 0 || (uintptr_t)kcache % 8)) || ldq < heads * dim)
+        return (int)hipErrorInvalidValue;
+    RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, q_out, ldq, nullptr, 0, M, heads * dim, K, 0, GateLaw{}, 0, 1,
+               positions, slots, cos_tab, sin_tab, (bf16_t*)kcache, (bf16_t*)vcache, heads, kv_heads, dim, std::max(page_size, 1), max_pos};
+    if (!fits(a, 2)) return (int)hipErrorInvalidValue;
+    a.N = (heads + 2 * kv_heads) * dim;
+    if (((long long)a.N + 512) * ldw * 2 >= 0x7fffffffll) return (int)hipErrorInvalidValue;
+    return launch(a, tile ? tile : plan_of(M, a.N, K, false, 1).tile, RING_ROPE, stream);
+}

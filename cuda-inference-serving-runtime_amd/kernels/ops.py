@@ -60,6 +60,7 @@ def _declare(h):
         "cisr_add_rmsnorm_sums": [p, p, i, p, p, i, i, f, i, p],
         "cisr_gemm_ring_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, i, p],
         "cisr_gemm_ring_bf16_gated": [p, i, p, i, p, i, i, i, i, i, f, f, f, i, p],
+        "cisr_gemm_ring_rope": [p, i, p, i, p, i, i, i, p, p, p, p, p, p, i, i, i, i, i, i, p],
         "cisr_gemm_ring_partials_bf16": [p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_skinny_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, p, f, p, p],
         "cisr_qkv_rope_skinny": [p, i, p, i, p, i, i, i, p, f, p, p, p, p, p, p, i, i, i, i, i, p],
@@ -623,7 +624,7 @@ RING_MIN_ROWS = 65
 RING_MIN_OUTPUTS, RING_MIN_OUTPUTS_K = 500_000, 40
 RING_MIN_OUTPUTS_SHORT, RING_SHORT_K = 250_000, 1024
 RING_PLAIN_FLOPS, RING_PLAIN_COLS = 15e9, 2048
-RING_MOST_FLOPS, RING_GATED_FLOPS = 300e9, 210e9
+RING_MOST_FLOPS, RING_GATED_FLOPS, RING_ROPE_FLOPS = 300e9, 210e9, 95e9
 
 
 def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
@@ -686,6 +687,16 @@ def gemm_ring(a, w, out, residual=None, act=0, tile=0):
     _check(lib().cisr_gemm_ring_bf16(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), rp, ldr, m, n, k,
                                      _storage(out, "out"), int(act), int(tile), _stream()), "gemm_ring")
     return out
+
+
+def ring_rope_ok(a, w, head_dim, cos):
+    """Whether qkv_rope runs the ring product with the rotation and the cache write as its epilogue: bf16 rows, whole heads of a multiple
+    of 32 coordinates.  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
+    rows 40.8 / 36.6, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.8; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
+    (m, k), n = a.shape, w.shape[0]
+    return (m >= RING_MIN_ROWS and 2.0 * m * n * k <= RING_ROPE_FLOPS and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda
+            and w.is_cuda and k % 64 == 0 and head_dim % 32 == 0 and 2 * cos.shape[1] == head_dim and a.stride(1) == 1 and w.stride(1) == 1
+            and _skinny_ok(a, w) and a.stride(0) >= k and w.stride(0) >= k and a.stride(0) * 1024 < 1 << 31 and (n + 512) * w.stride(0) * 2 < 1 << 31)
 
 
 def gemm_ring_gated(a, w, out, law=None, tile=0):
@@ -1028,6 +1039,8 @@ def qkv_rope_fused_ok(a, w, head_dim, cos, normed):
     m, k = a.shape
     if normed and wide_ok(m, w, after_norm=True, fused=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
         return False
+    if not normed and ring_rope_ok(a, w, head_dim, cos):
+        return True
     return (w.dtype == torch.bfloat16 and m <= SKINNY_ROWS and k % 8 == 0 and head_dim % 16 == 0
             and 2 * cos.shape[1] == head_dim and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0
             and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0
@@ -1059,7 +1072,7 @@ def _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads
 
 
 def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm=None, scratch=None):
-    """One kernel for a decode step's projections: (RMSNorm of the float residual `a` if `norm` = (weight, eps),
+    """One kernel for a step's projections (few rows, or the ring product): (RMSNorm of the float residual `a` if `norm` = (weight, eps),
     else `a` is bf16 and normed), product with w = [Wq; Wk; Wv], rotary embedding of q and k, q into
     q_out [M, heads*dim], k and v into the cache at `slots`.  kcache None: w = Wq only (a layer reading
     another layer's cache)."""
@@ -1080,6 +1093,12 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
         vp = _dev(vcache, "vcache", torch.bfloat16, (pages, kv_heads, dim, page_size))
         sp = _dev(slots, "slots", torch.int32, (m,))
     max_pos = cos.shape[0]
+    if norm is None and ring_rope_ok(a, w, dim, cos):
+        _check(lib().cisr_gemm_ring_rope(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), _dev(q_out, "q_out", torch.bfloat16, (m, heads * dim)),
+                                         heads * dim, m, k, _dev(positions, "positions", torch.int32, (m,)), sp, _dev(cos, "cos", torch.float32),
+                                         _dev(sin, "sin", torch.float32, (max_pos, dim // 2)), kp, vp, heads, n_kv, dim, page_size, max_pos, 0,
+                                         _stream()), "qkv_rope")
+        return q_out
     if norm is None and wide_ok(m, w, after_norm=True):
         need = _wide_plan(m, w.shape[0], k, False)
         work = _wide_workspace(scratch, a.device, need)

@@ -184,3 +184,38 @@ def test_gelu_of_every_bf16_number(ops):
     special = torch.tensor([0.0, float("inf"), float("nan")], dtype=torch.bfloat16, device=DEV)
     out = ops.gelu(special, torch.empty_like(special))
     assert out[0] == 0 and out[1] == float("inf") and out[2].isnan()
+
+
+@pytest.mark.parametrize("M, K, heads, kv, dim, page", [(65, 64, 3, 1, 32, 16), (200, 576, 9, 3, 64, 16), (97, 128, 2, 2, 96, 8), (300, 512, 4, 0, 64, 16),
+                                                        (131, 256, 8, 2, 128, 32), (80, 192, 1, 1, 160, 16), (700, 576, 9, 3, 64, 16)])
+def test_rotation_and_cache_write_in_the_epilogue(ops, M, K, heads, kv, dim, page, monkeypatch):
+    """Against the product and the rotary kernel: rows in runs of slots and out of order, rows without a slot, whole pages that stay."""
+    a, w, _ = operands(M, (heads + 2 * kv) * dim, K, seed=M)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    angle = torch.rand(2 * M, dim // 2, generator=g, device=DEV) * 6.3
+    cos, sin = angle.cos().contiguous(), angle.sin().contiguous()
+    positions = torch.randint(0, 2 * M, (M,), generator=g, device=DEV, dtype=torch.int32)
+    pages = M // page + 3
+    slots = torch.arange(M, device=DEV, dtype=torch.int32) + page + 3
+    slots[M // 2:] = slots[M // 2:].flip(0).clone()
+    slots[::17] = -1
+
+    def run():
+        keys = torch.full((pages, max(kv, 1), page, dim), 7.0, dtype=torch.bfloat16, device=DEV)
+        values = torch.full((pages, max(kv, 1), dim, page), 7.0, dtype=torch.bfloat16, device=DEV)
+        pools = (keys, values) if kv else (None, None)
+        if ops.qkv_rope_fused_ok(a, w, dim, cos, False):
+            q = ops.qkv_rope(a, w, torch.empty(M, heads * dim, dtype=torch.bfloat16, device=DEV), positions, slots if kv else None, cos, sin,
+                             *pools, heads, kv, dim, page)
+        else:
+            rows = ops.gemm(a, w, torch.empty(M, w.shape[0], dtype=torch.bfloat16, device=DEV))
+            ops.rope_scatter(rows, positions, slots if kv else None, cos, sin, *pools, heads, kv, dim, page)
+            q = rows[:, :heads * dim]
+        return q.double(), keys.double(), values.double()
+    assert ops.ring_rope_ok(a, w, dim, cos)
+    here = run()
+    monkeypatch.setattr(ops, "RING_MIN_ROWS", 1 << 30)
+    for got, want in zip(here, run()):
+        # the other path rounds the product to bf16 before it turns it (2^-8 of either coordinate of a pair) and both round the result
+        assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * 2 * want.abs().max()).all()
+        assert (got - want).norm() <= 2.0 ** -7 * want.norm()
