@@ -10,21 +10,28 @@ namespace {
 // 8 x 16 tiles, inner sizes of 576, 2,048 and 8,192; `start` has the launch, the first copies and the stores.
 struct Tile { int rows, cols; float start, step, half; };
 constexpr Tile TILES[] = {
-    {64, 64, 3.4f, 0.235f, 0.180f},    {64, 128, 4.4f, 0.355f, 0.272f},   {128, 64, 3.9f, 0.344f, 0.264f},   {96, 128, 4.9f, 0.415f, 0.325f},
-    {128, 128, 5.6f, 0.496f, 0.377f},  {160, 128, 6.1f, 0.589f, 0.437f},  {192, 128, 6.7f, 0.671f, 0.507f},  {224, 128, 7.6f, 0.776f, 0.588f},
-    {256, 128, 8.1f, 0.894f, 0.671f},  {64, 256, 5.2f, 0.590f, 0.590f},   {96, 256, 6.2f, 0.739f, 0.700f},   {128, 256, 7.9f, 0.859f, 0.780f},
-    {160, 256, 8.6f, 1.029f, 0.855f},  {192, 256, 9.1f, 1.228f, 1.228f},  {224, 256, 10.2f, 1.389f, 1.308f}, {256, 256, 11.4f, 1.505f, 1.347f},
-    {288, 256, 12.3f, 1.665f, 1.395f},
+    {64, 32, 3.3f, 0.190f, 0.170f},    {64, 64, 3.4f, 0.230f, 0.180f},    {64, 128, 4.2f, 0.350f, 0.275f},   {128, 64, 3.9f, 0.344f, 0.264f},
+    {96, 128, 4.9f, 0.415f, 0.325f},   {128, 128, 5.6f, 0.496f, 0.377f},  {160, 128, 6.1f, 0.589f, 0.437f},  {192, 128, 6.7f, 0.671f, 0.507f},
+    {224, 128, 7.6f, 0.776f, 0.588f},  {256, 128, 8.1f, 0.894f, 0.671f},  {64, 256, 5.2f, 0.590f, 0.590f},   {96, 256, 6.2f, 0.739f, 0.700f},
+    {128, 256, 7.9f, 0.859f, 0.780f},  {160, 256, 8.6f, 1.029f, 0.855f},  {192, 256, 9.1f, 1.228f, 1.228f},  {224, 256, 10.2f, 1.389f, 1.308f},
+    {256, 256, 11.4f, 1.505f, 1.347f}, {288, 256, 12.3f, 1.665f, 1.395f},
 };
 constexpr int UNITS = 256, MOST_SLICES = 8, LEAST_STEPS = 4;
 
 struct Plan { int tile, slices; float us; };
 
-float rounds_us(const Tile& t, long long blocks, int steps) {
-    const long long full = blocks / UNITS, rest = blocks % UNITS;
-    float us = full * (t.start + steps * t.step);
-    if (rest) us += t.start + steps * (t.half + (t.step - t.half) * std::max(0.f, 2.f * rest / UNITS - 1.f));
-    return us;
+// With one tile of rows every block streams its rows of W from memory alone: a step then is no shorter than the way there (measured
+// 0.29, 0.48 and 0.77 us with 64, 128 and 256 columns); and the rows of W that a round reads come at 5.6 TB/s at best.
+float round_us(const Tile& t, int blocks, int tiles_m, int steps) {
+    float step = t.half + (t.step - t.half) * std::max(0.f, 2.f * blocks / UNITS - 1.f);
+    if (tiles_m == 1) step = std::max(step, 0.13f + 0.0025f * t.cols);
+    return t.start + steps * std::max(step, (float)blocks / tiles_m * t.cols * 128 / 5.6e6f);
+}
+
+float rounds_us(const Tile& t, long long blocks, int tiles_m, int steps) {
+    const long long full = blocks / UNITS;
+    const int rest = (int)(blocks % UNITS);
+    return (full ? full * round_us(t, UNITS, tiles_m, steps) : 0.f) + (rest ? round_us(t, rest, std::min(tiles_m, rest), steps) : 0.f);
 }
 
 // The least of the model's times.  `slices` 0: any number of them, whose float sums are written and read once more (at 5 TB/s) by a
@@ -33,10 +40,11 @@ Plan plan_of(int M, int N, int K, bool gated, int slices) {
     Plan best{0, 1, INFINITY};
     const int steps = K / 64, cols = gated ? 2 * N : N;
     for (const Tile& t : TILES) {
-        const long long tiles = (long long)((M + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols);
+        const int tiles_m = (M + t.rows - 1) / t.rows;
+        const long long tiles = (long long)tiles_m * ((cols + t.cols - 1) / t.cols);
         for (int s = slices ? slices : 1; s <= (slices ? slices : MOST_SLICES); ++s) {
             if (s > 1 && steps / s < LEAST_STEPS) break;
-            float us = rounds_us(t, tiles * s, (steps + s - 1) / s);
+            float us = rounds_us(t, tiles * s, tiles_m, (steps + s - 1) / s);
             if (s > 1) us += (float)s * M * N * 8 / 5e6f + 0.5f;
             if (us < best.us) best = {t.rows * 1000 + t.cols, s, us};
         }

@@ -625,6 +625,11 @@ RING_MIN_OUTPUTS, RING_MIN_OUTPUTS_K = 500_000, 40
 RING_MIN_OUTPUTS_SHORT, RING_SHORT_K = 250_000, 1024
 RING_PLAIN_FLOPS, RING_PLAIN_COLS = 15e9, 2048
 RING_MOST_FLOPS, RING_GATED_FLOPS, RING_ROPE_FLOPS = 300e9, 210e9, 95e9
+# Of 17 to 64 rows the products of large weights, in bytes (by kind: see ring_ahead); the smaller ones only from more than 32 rows on.
+RING_FEW_ROWS, RING_HALF_ROWS = 17, 33
+RING_FEW_GATED, RING_HALF_GATED = 64 << 20, 16 << 20
+RING_FEW_CUT = 32 << 20
+RING_FEW_PLAIN, RING_FEW_PLAIN_MOST = 24 << 20, 64 << 20
 
 
 def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
@@ -638,9 +643,20 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
       gate and up with their activation: 128 x 16,384, K 2,048 25.8 / 20.2, 1,061 rows 83 / 66, 2,345 rows 177 / 153, 907 x 28,672,
       K 4,096 (213 GFLOP) 192 / 213, 2,048 rows 377 / 409;
       a product that ends with its store: 1,000 x 4,096, K 1,024 13.8 / 13.3, 2,000 rows (17 GFLOP) 21 / 22, 4,000 rows 29 / 35; 2,345 x 2,048, K 2,048
-      29 / 24; float results 2,000 x 8,512, K 2,048 81 / 63, 4,000 rows 138 / 128."""
+      29 / 24; float results 2,000 x 8,512, K 2,048 81 / 63, 4,000 rows 138 / 128;
+      17 to 64 rows, where a block streams its rows of W alone: gate and up 18 x 16,384, K 2,048 18.3 / 14.4, 64 rows 20.8 / 15.8, 64 x
+      28,672, K 4,096 55 / 46, 32 x 8,192, K 1,024 6.6 / 6.7, 40 rows 8.4 / 6.9; added to a residual, the norm included, 18 x 2,048, K 8,192
+      14.5 / 13.6, 64 rows 19.7 / 14.6, 64 x 4,096, K 14,336 46 / 31 (32 x 2,048, K 2,048 8.5 / 9.2); others 32 x 6,144,
+      K 2,048 10.3 / 8.9, 64 rows 16.4 / 9.3, 18 x 49,152 35 / 40, 64 rows 49 / 42, 64 x 2,048 7.6 / 9.5.  Fewer rows read W as fast elsewhere."""
     cols, k = w.shape
     flops, outputs = 2.0 * m * cols * k, m * cols
+    if m <= SKINNY_ROWS:
+        size, half = 2 * cols * k, m >= RING_HALF_ROWS
+        if m < RING_FEW_ROWS or w.dtype != torch.bfloat16:
+            return False
+        if gated or cut:
+            return size >= ((RING_HALF_GATED if half else RING_FEW_GATED) if gated else RING_FEW_CUT)
+        return size >= RING_FEW_PLAIN and (half or size <= RING_FEW_PLAIN_MOST)
     if m < RING_MIN_ROWS or w.dtype != torch.bfloat16 or flops > (RING_GATED_FLOPS if gated else RING_MOST_FLOPS):
         return False
     library = library_ok(m, w, gated=gated, plain=not (fused or gated), floats=floats)
@@ -691,10 +707,11 @@ def gemm_ring(a, w, out, residual=None, act=0, tile=0):
 
 def ring_rope_ok(a, w, head_dim, cos):
     """Whether qkv_rope runs the ring product with the rotation and the cache write as its epilogue: bf16 rows, whole heads of a multiple
-    of 32 coordinates.  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
+    of 32 coordinates; up to 64 rows large weights only (64 x 6,144, K 2,048 17.7 / 10.0, 18 rows 10.1 / 9.6, K 4,096 17.0 / 16.2).  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
     rows 40.8 / 36.6, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.8; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
     (m, k), n = a.shape, w.shape[0]
-    return (m >= RING_MIN_ROWS and 2.0 * m * n * k <= RING_ROPE_FLOPS and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda
+    many = m >= RING_MIN_ROWS if m > SKINNY_ROWS else m >= RING_FEW_ROWS and 2 * n * k >= RING_FEW_PLAIN
+    return (many and 2.0 * m * n * k <= RING_ROPE_FLOPS and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda
             and w.is_cuda and k % 64 == 0 and head_dim % 32 == 0 and 2 * cos.shape[1] == head_dim and a.stride(1) == 1 and w.stride(1) == 1
             and _skinny_ok(a, w) and a.stride(0) >= k and w.stride(0) >= k and a.stride(0) * 1024 < 1 << 31 and (n + 512) * w.stride(0) * 2 < 1 << 31)
 
@@ -896,7 +913,9 @@ def gemm_unfinished(a, w, residual, scratch=None):
         return None
     if ring_ahead(m, w, fused=True, cut=True) and ring_fits(a, w, residual):
         sums = ring_sums(a, w, lambda floats: _wide_workspace(scratch, a.device, floats))
-        return None if sums is None else (sums, 0)       # (one that is not cut: gemm adds it in the product's epilogue)
+        if sums is None:
+            return None                     # (not cut: gemm adds it in the product's epilogue)
+        return (sums, 0) if m > SKINNY_ROWS else (sums.parts, sums.slices)      # (few rows: a block a row adds them)
     if library_ok(m, w):
         if not a.is_contiguous():
             return None
@@ -1356,6 +1375,10 @@ def gemm_for_norm(a, w, out, make_buffer, scratch=None):
     finished into `out` (float [M, N]) and `out` is returned."""
     m, k = a.shape
     n = w.shape[0]
+    if (a.dtype == torch.bfloat16 and n <= PARTIALS_MAX_COLS and tuple(out.shape) == (m, n) and w.shape[1] == k
+            and ring_ahead(m, w, fused=True, floats=True, cut=True) and ring_fits(a, w, out)):
+        sums = ring_sums(a, w, make_buffer)
+        return gemm_ring(a, w, out) if sums is None else Partials(sums.parts, sums.slices, m, n)
     if (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and 0 < m <= SKINNY_ROWS and n <= PARTIALS_MAX_COLS
             and not library_ok(m, w) and _skinny_ok(a, w) and wide_ok(m, w)):
         need = _wide_plan(m, n, k, False)
@@ -1364,10 +1387,6 @@ def gemm_for_norm(a, w, out, make_buffer, scratch=None):
             _check(lib().cisr_gemm_wide_partials_bf16(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), m, n, k,
                                                       _dev(work, "partial sums", torch.float32), work.numel(), _stream()), "gemm_for_norm")
             return Partials(work, need // (m * n), m, n)
-    if (a.dtype == torch.bfloat16 and n <= PARTIALS_MAX_COLS and tuple(out.shape) == (m, n) and w.shape[1] == k
-            and ring_ahead(m, w, fused=True, floats=True, cut=True) and ring_fits(a, w, out)):
-        sums = ring_sums(a, w, make_buffer)
-        return gemm_ring(a, w, out) if sums is None else Partials(sums.parts, sums.slices, m, n)
     return gemm(a, w, out, scratch=scratch)
 
 
