@@ -258,29 +258,39 @@ static int launch_f32(GemmF32Args p, hipStream_t stream) {
     return CISR_LAUNCH_CHECK();
 }
 
-// The tile: 32 x 64 where that leaves two blocks a compute unit, 32 x 32 where it leaves a quarter of them a block, else 16 x 16
-// (up to 16 rows always: the other rows of a tile would be padding).
-template <int WK, bool VEC>
+// The tile (sixteens of rows x sixteens of W's rows): the smallest that needs no more blocks than there are compute units, as a block alone
+// on its unit takes the longer the larger its tile, and a second round costs more.  192 rows, us of the tile before / now: 576 x 576 2 x 2
+// (108 blocks) 8.2 / 1 x 2 (216) 6.4, 576 x 1,536 15.2 / 1 x 2 11.3, 960 x 576 8.7 / 2 x 2 with two sixteens in flight instead of four 7.9,
+// 3,072 x 576 gated 2 x 2 (576) 18.1 / 3 x 4 (192) 15.8; 2,048 x 2,048 33 / 3 x 2 24; 512 x 576, K 1,536 26.6 / 3 x 2 18.9.  Beyond one round
+// the others: 512 x 3,072, K 576 2 x 2 29.8, 2 x 4 31.4; K 2,048 512 x 8,192 2 x 4 207, 4 x 2 210, 192 x 8,192 2 x 4 90, 4 x 2 84.5.  Up to 16
+// rows the tile has 16 of them.  A tile never changes a sum: its order is K's.  (Rows that are not aligned: two tiles only.)
+template <int WK, bool VEC, int FORM>
 static int launch_f32_tile(const GemmF32Args& p, hipStream_t stream) {
-    const long long m32 = (p.M + 31) / 32, n32 = (p.N + 31) / 32, n64 = (p.N + 63) / 64;
-    if (p.M > 16 && m32 * n64 >= 512) return launch_f32<2, 4, WK, 2, VEC>(p, stream);
-    if (p.M > 16 && m32 * n32 >= 64) return launch_f32<2, 2, WK, 4, VEC>(p, stream);
-    return launch_f32<1, 1, WK, 8, VEC>(p, stream);
+    const int cols = FORM == F32_PLAIN ? p.N : 2 * p.N;
+    auto one_round = [&](int tm, int tn) { return (long long)((p.M + 16 * tm - 1) / (16 * tm)) * ((cols + 16 * tn - 1) / (16 * tn)) <= 256; };
+    constexpr int DEEP = WK == 16 ? 8 : 4;               // sixteens in flight where a wave has few operands each
+    if (p.M <= 16 || one_round(1, 1)) return launch_f32<1, 1, WK, DEEP, VEC, FORM>(p, stream);
+    if constexpr (VEC) {
+        if (one_round(1, 2)) return launch_f32<1, 2, WK, 4, VEC, FORM>(p, stream);
+        if (one_round(2, 2)) return launch_f32<2, 2, WK, 2, VEC, FORM>(p, stream);
+        if (one_round(3, 2)) return launch_f32<3, 2, WK, 2, VEC, FORM>(p, stream);
+        if (one_round(4, 2)) return launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream);
+        if constexpr (WK == 8 && FORM != F32_PLAIN) {    // (a wave finishes at most one sixteen by sixteen of columns)
+            if (one_round(3, 4)) return launch_f32<3, 4, WK, 2, VEC, FORM>(p, stream);
+            if (one_round(4, 4)) return launch_f32<4, 4, WK, 2, VEC, FORM>(p, stream);
+        }
+        if constexpr (WK == 16) return p.M <= 256 ? launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream) : launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+    }
+    return launch_f32<2, 2, WK, 2, VEC, FORM>(p, stream);
 }
 
-// The same with two rows of W a column.
-template <int WK, bool VEC, int FORM>
-static int launch_f32_pairs(const GemmF32Args& p, hipStream_t stream) {
-    const long long m32 = (p.M + 31) / 32, n32 = (p.N + 15) / 16, n64 = (p.N + 31) / 32;
-    if (p.M > 16 && m32 * n64 >= 512) return launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
-    if (p.M > 16 && m32 * n32 >= 64) return launch_f32<2, 2, WK, 4, VEC, FORM>(p, stream);
-    return launch_f32<1, 1, WK, 8, VEC, FORM>(p, stream);
-}
+// Waves a tile: sixteen from an inner size of 1,024 on, else eight (so that a wave has at least two sixteens at the small
+// models' 576).
 template <int FORM>
-static int launch_f32_pairs(const GemmF32Args& p, hipStream_t stream) {
+static int launch_f32_form(const GemmF32Args& p, hipStream_t stream) {
     const bool vec = p.K % 4 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0 && (uintptr_t)p.A % 16 == 0 && (uintptr_t)p.W % 16 == 0;
-    if (p.K >= 1024) return vec ? launch_f32_pairs<16, true, FORM>(p, stream) : launch_f32_pairs<16, false, FORM>(p, stream);
-    return vec ? launch_f32_pairs<8, true, FORM>(p, stream) : launch_f32_pairs<8, false, FORM>(p, stream);
+    if (p.K >= 1024) return vec ? launch_f32_tile<16, true, FORM>(p, stream) : launch_f32_tile<16, false, FORM>(p, stream);
+    return vec ? launch_f32_tile<8, true, FORM>(p, stream) : launch_f32_tile<8, false, FORM>(p, stream);
 }
 
 // C[M, N] = silu(A . Wg^T) * (A . Wu^T) with W = [Wg; Wu], 2 N rows
@@ -288,7 +298,7 @@ extern "C" int cisr_gemm_f32_swiglu(const float* A, int lda, const float* W, int
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return (int)hipErrorInvalidValue;
     GemmF32Args p{A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, 0};
-    return launch_f32_pairs<F32_GATED>(p, stream);
+    return launch_f32_form<F32_GATED>(p, stream);
 }
 
 // W = [Wq; Wk; Wv] (kv_heads 0: Wq alone): queries and keys turned over the whole head by the rows' positions, queries to C, keys
@@ -301,17 +311,13 @@ extern "C" int cisr_gemm_f32_rope(const float* A, int lda, const float* W, int l
         return (int)hipErrorInvalidValue;
     GemmF32Args p{A, lda, W, ldw, q_out, ldq, nullptr, 0, M, (heads + 2 * kv_heads) * dim / 2, K, 0,
                   positions, slots, cos_tab, sin_tab, kcache, vcache, heads, kv_heads, dim, page_size, max_pos};
-    return launch_f32_pairs<F32_ROTARY>(p, stream);
+    return launch_f32_form<F32_ROTARY>(p, stream);
 }
 
-// Waves a tile: sixteen from an inner size of 1,024 on, else eight (so that a wave has at least two sixteens at the small
-// models' 576).
 extern "C" int cisr_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
                              const float* R, int ldr, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return (int)hipErrorInvalidValue;
     const GemmF32Args p{A, lda, W, ldw, C, ldc, R, ldr, M, N, K, 0};
-    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
-    if (K >= 1024) return vec ? launch_f32_tile<16, true>(p, stream) : launch_f32_tile<16, false>(p, stream);
-    return vec ? launch_f32_tile<8, true>(p, stream) : launch_f32_tile<8, false>(p, stream);
+    return launch_f32_form<F32_PLAIN>(p, stream);
 }
