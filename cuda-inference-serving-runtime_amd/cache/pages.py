@@ -99,6 +99,39 @@ class PagePool:
         self.peak = max(self.peak, self.n_pages - len(self.free))
         return page
 
+    def allocate_many(self, n):
+        """The pages that n calls of allocate would hand out, in their order."""
+        if n > len(self.free):
+            raise OutOfPages("KV page pool exhausted")
+        pages = self.free[:-n - 1:-1]
+        del self.free[len(self.free) - n:]
+        refs = self.refs
+        for page in pages:
+            refs[page] = 1
+        self.peak = max(self.peak, self.n_pages - len(self.free))
+        return pages
+
+    def share_all(self, pages):
+        """share of every page of a table (negative entries are none)."""
+        refs = self.refs
+        for page in pages:
+            if page >= 0:
+                if refs[page] <= 0:
+                    raise AssertionError(f"page {page} is shared while free")
+                refs[page] += 1
+
+    def drop_all(self, pages):
+        """drop of every page of a table (negative entries are none), in its order."""
+        refs, free = self.refs, self.free
+        for page in pages:
+            if page >= 0:
+                held = refs[page]
+                if held <= 0:
+                    raise AssertionError(f"page {page} is freed twice")
+                refs[page] = held - 1
+                if held == 1:
+                    free.append(page)
+
     def share(self, page):
         if self.refs[page] <= 0:
             raise AssertionError(f"page {page} is shared while free")
@@ -192,8 +225,8 @@ class CacheGroup:
                 self.trim(request, length)
 
     def append(self, request, length, n_new):
-        """Slots of the n_new tokens at logical positions length.. and the page
-        copies (src, dst) that must run on the device before they are written."""
+        """Slots of the n_new tokens at logical positions length.. (a list; of a prompt portion, more than 32 tokens, an
+        int32 array) and the page copies (src, dst) that must run on the device before they are written."""
         table, P = self.tables[request], self.page_size
         copies = []
         if n_new > 0 and length % P and self.pool.refs[table[-1]] > 1:
@@ -202,12 +235,14 @@ class CacheGroup:
             self.pool.drop(old)
             table[-1] = new
             self._touch(request)
-        while len(table) * P < length + n_new:
-            table.append(self.pool.allocate())
+        more = -(-(length + n_new) // P) - len(table)
+        if more > 0:
+            table += self.pool.allocate_many(more)
             self._touch(request)
-        if n_new > 32:      # a prompt portion: the same, vectorised
-            at = np.arange(length, length + n_new, dtype=np.int64)
-            slots = (np.asarray(table, dtype=np.int64)[at // P] * P + at % P).tolist()
+        if n_new > 32:      # a prompt portion: the same, page by page
+            first = length // P
+            pages = np.array(table[first:], dtype=np.int32) * np.int32(P)
+            slots = (pages[:, None] + np.arange(P, dtype=np.int32)).reshape(-1)[length - first * P:length - first * P + n_new]
         else:
             slots = [table[(length + i) // P] * P + (length + i) % P for i in range(n_new)]
         return slots, copies
@@ -221,16 +256,12 @@ class CacheGroup:
         if source in self.given_back:
             self.given_back[target] = self.given_back[source]
         self._touch(target)
-        for page in self.tables[target]:
-            if page >= 0:
-                self.pool.share(page)
+        self.pool.share_all(self.tables[target])
 
     def release(self, request):
         self.versions.pop(request, None)
         self.given_back.pop(request, None)
-        for page in self.tables.pop(request):
-            if page >= 0:
-                self.pool.drop(page)
+        self.pool.drop_all(self.tables.pop(request))
 
     def check(self):
         expected = [0] * self.pool.n_pages

@@ -348,3 +348,46 @@ def test_fork_of_a_request_whose_window_has_passed_pages():
     m.release("a"); m.check()
     m.release("b"); m.check()
     assert [g.pool.used for g in m.groups] == [0, 0]
+
+
+def test_pages_in_bulk_are_those_one_at_a_time():
+    """Portions take, share and give back their pages in bulk: the same pages in the same order as one call a page, and the
+    slots of a long portion are an array of the same numbers, from any position in a page."""
+    import random
+    import numpy as np
+    from runtime.cache.pages import PagePool, OutOfPages, CacheGroup, KVNeed
+    rng = random.Random(3)
+    bulk, single = PagePool(50), PagePool(50)
+    held = []
+    for _ in range(300):
+        n = rng.randrange(0, 9)
+        if n <= len(single.free) and rng.random() < 0.6:
+            pages = bulk.allocate_many(n)
+            assert pages == [single.allocate() for _ in range(n)]
+            held.append(pages)
+            if rng.random() < 0.3:
+                bulk.share_all([-1] + pages)
+                for page in pages:
+                    single.share(page)
+                held.append(pages)
+        elif held:
+            pages = held.pop(rng.randrange(len(held)))
+            bulk.drop_all(pages[:1] + [-1] + pages[1:])
+            for page in pages:
+                single.drop(page)
+        assert (bulk.free, bulk.refs, bulk.peak) == (single.free, single.refs, single.peak)
+    with pytest.raises(OutOfPages):
+        bulk.allocate_many(len(bulk.free) + 1)
+    with pytest.raises(AssertionError):
+        PagePool(2).drop_all([0])
+    with pytest.raises(AssertionError):
+        PagePool(2).share_all([0])
+    for P in (1, 4, 16):
+        for length in (0, 1, P - 1, 3 * P + P // 2):
+            group = CacheGroup(KVNeed(1, 8), [0], 200, P)
+            group.create("a")
+            if length:
+                group.append("a", 0, length)
+            slots, _ = group.append("a", length, 77)
+            table = group.tables["a"]
+            assert slots.dtype == np.int32 and slots.tolist() == [table[i // P] * P + i % P for i in range(length, length + 77)]
