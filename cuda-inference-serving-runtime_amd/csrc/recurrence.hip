@@ -95,7 +95,12 @@ conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* _
 // The same for portions, four channels a thread and CONV_ROWS rows of the step a block: an input is read once (the taps - 1
 // before a block's first row again), eight rows' 16-byte loads are on their way together.  The same sums in the same order.
 // Channels, row stride and first column multiples of 4, pointers 16-byte aligned.  The last blocks of y make the gates.
-// 2,048 rows of 8,192 channels, four taps: 90 us with a thread a (row, channel), 45 so (134 MB).  A block's walk takes 12 to 14 us
+// A block all of whose rows are one portion's, none of them within the portion's first, looks nothing up row by row and asks for a
+// row eight rows before its turn; in the others a portion that begins inside brings its state when its first row comes.  (With the
+// state's rows chosen input by input a wave of four taps held 174 registers, two waves a SIMD; so 82, and the stream of
+// memory is what bounds it.)  2,048 rows of 8,192 channels, four taps (134 MB): 90 us with a thread a (row, channel), 45 with rows looked
+// up and the state chosen input by input, 34 so; fifty portions of 40 rows 42.5 / 39.0, 2,368 rows of 6,144 35.3 / 29.0, 4,096 of 8,192
+// 76 / 60 (both with the state's own kernel).  A block's walk takes 12 to 14 us
 // however few blocks there are, more where it meets portions that begin (their first rows wait for the state, one after the
 // other; 16 single rows 22 us).  Steps of fewer inputs than that is worth keep a thread a (row, channel): 128 rows of 8,192 channels
 // 10.1 us against 13.1 (200 rows 14.8 against 13.9), 1,024 of 1,024 9.6 against 12.7 (1,500 rows 13.2 against 12.8); 24 single
@@ -134,44 +139,66 @@ conv_silu_rows_kernel(const float* __restrict__ in, int ld, int first, const flo
 #pragma unroll
         for (int j = 0; j < TAPS; ++j) taps[i][j] = w[(size_t)(c + i) * TAPS + j];
     const conv_f32x4 b = bias ? *(const conv_f32x4*)(bias + c) : (conv_f32x4){0.f, 0.f, 0.f, 0.f};
-    conv_f32x4 before[TAPS - 1];                     // the inputs of the TAPS - 1 rows before, whoever's they are
+    auto row = [&](int t) { return *(const conv_f32x4*)(x0 + (size_t)t * ld); };
+    auto finish = [&](int t, const conv_f32x4 (&use)[TAPS]) __attribute__((always_inline)) {
+        conv_f32x4 y = b;
 #pragma unroll
-    for (int j = 0; j < TAPS - 1; ++j) before[j] = *(const conv_f32x4*)(x0 + (size_t)max(t0 - (TAPS - 1) + j, 0) * ld);
+        for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) y[k] += taps[k][j] * use[j][k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y[k] = y[k] / (1.0f + expf(-y[k]));
+        *(conv_f32x4*)(out + (size_t)t * channels + c) = y;
+    };
+    const int mine = seg_of_row[min(t0 + (int)threadIdx.x % CONV_ROWS, t1 - 1)], whose = __builtin_amdgcn_readfirstlane(mine);
+    if (whose >= 0 && t1 - t0 == CONV_ROWS && __all(mine == whose) && t0 - seg_start[whose] >= TAPS - 1) {
+        // the block's rows are one portion's and reach back into rows of it only: nothing to look up row by row
+        conv_f32x4 x[CONV_ROWS + TAPS - 1];          // (a row is asked for eight rows before its turn)
+#pragma unroll
+        for (int i = 0; i < TAPS - 1 + 8; ++i) x[i] = row(t0 - (TAPS - 1) + i);
+#pragma unroll
+        for (int i = 0; i < CONV_ROWS; ++i) {
+            conv_f32x4 use[TAPS];
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) use[j] = x[i + j];
+            finish(t0 + i, use);
+            if (i + 8 < CONV_ROWS) x[i + TAPS - 1 + 8] = row(t0 + i + 8);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
+    // the inputs of the TAPS - 1 rows before: a portion's first rows reach back into the request's state, rel of them behind it
+    conv_f32x4 before[TAPS - 1];
+    auto from_state = [&](int seg, int rel) __attribute__((always_inline)) {
+        const float* st = conv_state + (long long)state_slots[seg] * slot_stride + c;
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j)
+            if (rel + j < TAPS - 1) {
+                const float* from = st + (size_t)(rel + j) * channels;
+                before[j] = (conv_f32x4){from[0], from[1], from[2], from[3]};
+            }
+    };
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) before[j] = row(max(t0 - (TAPS - 1) + j, 0));
+    const int rel0 = whose < 0 ? 0 : t0 - seg_start[whose];
+    if (rel0 > 0 && rel0 < TAPS - 1) from_state(whose, rel0);
     for (int tb = t0; tb < t1; tb += 8) {
         conv_f32x4 x[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = *(const conv_f32x4*)(x0 + (size_t)min(tb + i, rows - 1) * ld);
+        for (int i = 0; i < 8; ++i) x[i] = row(min(tb + i, rows - 1));
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int t = tb + i;
             if (t >= t1) break;                      // (uniform)
             const int seg = seg_of_row[t];
+            if (seg >= 0 && t == seg_start[seg]) from_state(seg, 0);
             conv_f32x4 use[TAPS];
 #pragma unroll
             for (int j = 0; j < TAPS - 1; ++j) use[j] = before[j];
             use[TAPS - 1] = x[i];
 #pragma unroll
-            for (int j = 0; j + 1 < TAPS - 1; ++j) before[j] = before[j + 1];
-            before[TAPS - 2] = x[i];
-            if (seg < 0) continue;
-            const int rel = t - seg_start[seg];
-            if (rel < TAPS - 1) {                    // (uniform: a portion's first rows reach back into the request's state)
-                const float* st = conv_state + (long long)state_slots[seg] * slot_stride + c;
-#pragma unroll
-                for (int j = 0; j < TAPS - 1; ++j)
-                    if (rel - (TAPS - 1) + j < 0) {
-                        const float* from = st + (size_t)(rel + j) * channels;
-                        use[j] = (conv_f32x4){from[0], from[1], from[2], from[3]};
-                    }
-            }
-            conv_f32x4 y = b;
-#pragma unroll
-            for (int j = 0; j < TAPS; ++j)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) y[k] += taps[k][j] * use[j][k];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) y[k] = y[k] / (1.0f + expf(-y[k]));
-            *(conv_f32x4*)(out + (size_t)t * channels + c) = y;
+            for (int j = 0; j < TAPS - 1; ++j) before[j] = use[j + 1];
+            if (seg >= 0) finish(t, use);
         }
     }
 }

@@ -55,6 +55,22 @@ def test_short_convolution_in_words(channels, taps, heads, bias):
     assert (out[-pad:] == 9.0).all() and (state[1] == before[1]).all() and (not heads or bool((step[-pad:] == 9.0).all()))
 
 
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("before", [1, 3, 13, 15, 16])
+def test_short_convolution_wherever_a_portion_begins(taps, before):
+    """A portion of 70 rows behind another one of `before` rows, against the same portion alone: the rows that lie in blocks of its own
+    there lie in shared ones here, blocks whose first row is its second or fourth among them.  The same sums, so the same bits."""
+    from runtime.kernels import ops
+    channels, n = 26004, 70
+    x, w, b = torch.randn(before + n, channels, device=DEV), torch.randn(channels, taps, device=DEV), torch.randn(channels, device=DEV)
+    kept, outs = torch.randn(2, (taps - 1) * channels, device=DEV), []
+    for rows, counts, slots in ((x, [before, n], [1, 0]), (x[before:].contiguous(), [n], [0])):
+        out, state = torch.empty_like(rows), kept.clone()
+        ops.conv_silu(rows, w, b, state, out, ints(np.repeat(np.arange(len(counts)), counts)), ints(np.cumsum([0] + counts)), ints(slots))
+        outs.append((out[-n:], state[0]))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 @pytest.mark.parametrize("groups, size", [(300, 4), (33, 128), (9, 132), (40, 256), (3, 260), (2, 1000), (1, 1028), (1, 2048), (1, 4096), (5, 100)])
 @pytest.mark.parametrize("gate_first, sigmoid, skip, shared, dtype", [(True, False, True, False, torch.bfloat16), (False, True, False, True, torch.float32),
                                                                      (False, False, True, False, torch.bfloat16)])
