@@ -371,7 +371,7 @@ __global__ void swiglu_kernel(const T* __restrict__ gu, T* __restrict__ act, int
     size_t row = i / inter; int col = (int)(i % inter);
     const T* base = gu + row * (size_t)(2 * inter);
     float g = load_f32(base + col), u = load_f32(base + inter + col);
-    store_f32(act + i, g / (1.0f + expf(-g)) * u);
+    store_f32(act + i, times_sigmoid<T>(g, g) * u);
 }
 
 // the same for bf16, eight elements a thread with 16-byte accesses (inter % 8 == 0, aligned pointers)
@@ -388,7 +388,7 @@ __global__ void __launch_bounds__(256) swiglu_bf16x8_kernel(const bf16_t* __rest
     for (int k = 0; k < 4; ++k) {
         const float g0 = __uint_as_float(gw[k] << 16), g1 = __uint_as_float(gw[k] & 0xffff0000u);
         const float u0 = __uint_as_float(uw[k] << 16), u1 = __uint_as_float(uw[k] & 0xffff0000u);
-        out[k] = pack_bf16x2(g0 / (1.0f + expf(-g0)) * u0, g1 / (1.0f + expf(-g1)) * u1);
+        out[k] = pack_bf16x2(times_sigmoid_to_bf16(g0, g0) * u0, times_sigmoid_to_bf16(g1, g1) * u1);
     }
     *(u32x4_t*)(act + i * 8) = (u32x4_t){out[0], out[1], out[2], out[3]};
 }

@@ -175,7 +175,7 @@ __global__ void glu_clamped_kernel(const T* __restrict__ gu, T* __restrict__ act
     const size_t row = i / inter;
     const int col = (int)(i % inter);
     const T* base = gu + row * (size_t)(2 * inter);
-    store_f32(act + i, gated_activation(load_f32(base + col), load_f32(base + inter + col), law));
+    store_f32(act + i, gated_activation<T>(load_f32(base + col), load_f32(base + inter + col), law));
 }
 
 // the same for bf16, eight elements a thread with 16-byte accesses (inter % 8 == 0, aligned pointers)
@@ -192,8 +192,8 @@ glu_clamped_bf16x8_kernel(const bf16_t* __restrict__ gu, bf16_t* __restrict__ ac
     uint32_t out[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-        out[k] = pack_bf16x2(gated_activation(__uint_as_float(gw[k] << 16), __uint_as_float(uw[k] << 16), law),
-                             gated_activation(__uint_as_float(gw[k] & 0xffff0000u), __uint_as_float(uw[k] & 0xffff0000u), law));
+        out[k] = pack_bf16x2(gated_activation<bf16_t>(__uint_as_float(gw[k] << 16), __uint_as_float(uw[k] << 16), law),
+                             gated_activation<bf16_t>(__uint_as_float(gw[k] & 0xffff0000u), __uint_as_float(uw[k] & 0xffff0000u), law));
     *(u32x4_t*)(act + i * 8) = (u32x4_t){out[0], out[1], out[2], out[3]};
 }
 

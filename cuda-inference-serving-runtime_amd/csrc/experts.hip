@@ -805,7 +805,7 @@ expert_gemm_mfma_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
 #pragma unroll
                 for (int j = 0; j < 4; j += 2) {
                     const int n = n0 / 2 + wn * 32 + j * 8 + r;
-                    if (n < N / 2) store_f32(C + (size_t)m * ldc + n, gated_activation(acc[i][j][x], acc[i][j + 1][x], law));
+                    if (n < N / 2) store_f32(C + (size_t)m * ldc + n, gated_activation<TC>(acc[i][j][x], acc[i][j + 1][x], law));
                 }
             } else {
 #pragma unroll
@@ -873,7 +873,7 @@ expert_rows_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restri
     for (int j = 0; j < 4; ++j) sum[j] = wave_sum(sum[j]);
     if (GATED) {
         if (lane < 2 && n_first + lane < N)
-            store_f32(C + (size_t)pair * ldc + n_first + lane, gated_activation(lane ? sum[1] : sum[0], lane ? sum[3] : sum[2], law));
+            store_f32(C + (size_t)pair * ldc + n_first + lane, gated_activation<TC>(lane ? sum[1] : sum[0], lane ? sum[3] : sum[2], law));
         return;
     }
     if (lane < 4 && n_first + lane < N)

@@ -137,7 +137,7 @@ __device__ __forceinline__ void few_tile(const FewArgs& p, int e, int tile, int 
             const int pos = tile * EXF_TILE + place;
             float v = acc[i][0][x];
             if (ACT == FEW_RELU2) { v = fmaxf(v, 0.f); v *= v; }
-            if (ACT == FEW_GATED) v = gated_activation(v, acc[i][NT - 1][x], p.law);
+            if (ACT == FEW_GATED) v = gated_activation<TC>(v, acc[i][NT - 1][x], p.law);
             store_f32((TC*)p.C + (size_t)(p.scatter ? p.pair_of_pos[pos] : pos) * p.ldc + n, v);
         }
 }

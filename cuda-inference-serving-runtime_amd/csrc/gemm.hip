@@ -190,7 +190,7 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict
                 for (int e = 0; e < 4; ++e) {
                     const int m = m0 + wm * TM * 16 + i * 16 + g * 4 + e;
                     const float gq = bf16_to_f32(f32_to_bf16(acc[i][j][e])), uq = bf16_to_f32(f32_to_bf16(acc[i][j + TN / 2][e]));
-                    if (m < M) store_f32(C + (size_t)m * ldc + n, gated_activation(gq, uq, law));
+                    if (m < M) store_f32(C + (size_t)m * ldc + n, gated_activation<TC>(gq, uq, law));
                 }
             }
         return;

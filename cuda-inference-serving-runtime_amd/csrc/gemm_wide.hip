@@ -84,7 +84,7 @@ __device__ __forceinline__ void wide_finish(const WideArgs& p, int m, int n, flo
     if (NB == 2) {
         // gate and up are rounded to bf16 before the activation, as the two-kernel path does
         const float gq = bf16_to_f32(f32_to_bf16(v)), uq = bf16_to_f32(f32_to_bf16(u));
-        v = gated_activation(gq, uq, p.law);
+        v = gated_activation<bf16_t>(gq, uq, p.law);
     }
     if (p.R) v += p.R[(size_t)m * p.ldr + n];
     if (p.out_dtype == DT_F32) ((float*)p.C)[(size_t)m * p.ldc + n] = v;

@@ -221,3 +221,38 @@ def test_rotation_and_cache_write_in_the_epilogue(ops, M, K, heads, kv, dim, pag
         # the other path rounds the product to bf16 before it turns it (2^-8 of either coordinate of a pair) and both round the result
         assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * 2 * want.abs().max()).all()
         assert (got - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.parametrize("law", [None, (7.0, 1.702, 1.0), (-1.0, 0.0, 0.0)])
+def test_gates_of_every_size_against_64_bits(law):
+    """Gates from -1e30 to 1e30 with both signs' smallest, and infinite ones, as products with one term: the activation's own error stays
+    below what rounding its result to bf16, eight bits, may cost (2^-8 of it, and 4e-6 for the exponential, whose argument the other two laws
+    round before it, times its size)."""
+    from runtime.kernels import ops
+    k, inter = 64, 128
+    a = torch.zeros(80, k, device="cuda:0", dtype=torch.bfloat16)
+    for m in range(80):
+        a[m, m % k] = 1.0
+    g = torch.randn(k, inter, device="cuda:0") * torch.logspace(-3, 1.7, k, device="cuda:0")[:, None]
+    g[0, :12] = torch.tensor([0.0, -0.0, 1e-30, -1e-30, 1e-4, -1e-4, 80.0, -80.0, 1000.0, -1000.0, 1e30, -1e30], device="cuda:0")
+    g[1, :6] = torch.tensor([-86.0, -87.5, -88.0, -89.0, 88.0, 89.0], device="cuda:0")
+    g[63] = torch.where(torch.arange(inter, device="cuda:0") % 2 == 0, 3e38, -3e38)
+    u = torch.randn(k, inter, device="cuda:0")
+    w = torch.cat((g.t(), u.t())).bfloat16().contiguous()
+    a[63, 63] = 3e38                                          # (3e38 squared is past the largest float: gates of plus and minus infinity)
+    w[inter:, 63] = 1e-38
+    out = torch.empty(80, inter, device="cuda:0", dtype=torch.bfloat16)
+    ops.gemm_ring_gated(a, w, out, law)
+    rows = torch.arange(80, device="cuda:0") % k
+    gate, up = w[:inter].t().double()[rows], w[inter:].t().double()[rows]
+    gate[rows == 63] *= float("inf")
+    up[rows == 63] = (w[inter:, 63].double() * a[63, 63].double()).bfloat16().double()
+    limit, slope, shift = law or (0.0, 0.0, 0.0)
+    if limit > 0:
+        gate, up = gate.clamp(max=limit), up.clamp(-limit, limit) + shift
+    z = slope * gate if limit > 0 else 1.5957691216057308 * (gate + 0.044715 * gate ** 3) if limit < 0 else gate
+    want, got = gate * torch.sigmoid(z) * up, out.double()
+    dull = want.isnan() | want.isinf()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    bound = want.abs() * (2.0 ** -8 + 4e-6 + 2.0 ** -22 * z.abs().clamp(max=88.0)) + 1e-35
+    assert ((got - want).abs() <= bound)[~dull].all()
