@@ -453,16 +453,13 @@ def attention_f32(q, q_row_stride, kcache, vcache, tables, positions, tasks, out
     return out
 
 
-# Large bf16 products of many rows go to the vendor's library through torch.mm (the reference's linears are
-# library calls too: cuBLAS through runtime/blas.py:44-56, or CuPy's matmul, runtime/model.py:108): from this many rows on, with weights of at least LIBRARY_MIN_BYTES;
-# the residual sum or the activation is then a kernel after the product.  Measured on an MI355X at 2048 rows:
-# 1,270-1,480 TFLOP/s against 830-920 of the tiled kernel here on the 8B shapes (a prompt step of 30.6 against
-# 39.9 ms); at 65-255 rows with weights streamed from HBM it is up to 2.5 times as fast on narrow outputs with
-# a long inner size, which leave the tiled kernel few tiles (it does not cut K).  With at most 64 rows the
-# weight-streaming kernels here are as fast or faster (8 rows: 50 against 67 us for gate and up of the 8B
-# sizes), as are all products of small weights, and both save the kernel after the product.  The least weights are
-# those of the 1.7B sizes' output projection (8 MB: 10.7 against 13.9 us at 128 rows, 29 against 33 at 2,048, the
-# residual sum included; the products of the 135M sizes, 0.7 to 3.5 MB, are as fast or faster here).  0 rows: never.
+# What bf16 products of many rows go to the vendor's library through torch.mm where the ring product does not take them (the reference's
+# linears are library calls too: cuBLAS through runtime/blas.py:44-56, or CuPy's matmul, runtime/model.py:108): from this many rows
+# on, with weights of at least LIBRARY_MIN_BYTES; the residual sum or the activation is then a kernel after the product.  What is left
+# of them is in `ring_ahead`: large products that end with their store, gate and up above 210 GFLOP (1,270 to 1,480 TFLOP/s there at
+# 2,048 rows of the 8B shapes), inner sizes that are no multiple of 64.  Against the tiled kernel, which is what runs below these
+# lines: 8 MB (the 1.7B sizes' output projection) 10.7 against 13.9 us at 128 rows, 29 against 33 at 2,048, the residual sum
+# included; smaller weights are as fast or faster there.  0 rows: never.
 LIBRARY_MIN_ROWS = 65
 LIBRARY_MIN_BYTES = 8 << 20
 LIBRARY_GATED_MIN_ROWS, LIBRARY_GATED_MIN_BYTES = 33, 64 << 20
@@ -641,7 +638,7 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
       what is added to a residual is cut here too, and beats the library at any number of rows: 65 x 2,048, K 8,192 22.7 / 15.5, 1,061 rows
       66 / 50, 2,048 rows 82 / 70;
       gate and up with their activation: 128 x 16,384, K 2,048 25.8 / 20.2, 1,061 rows 83 / 66, 2,345 rows 177 / 153, 907 x 28,672,
-      K 4,096 (213 GFLOP) 192 / 213, 2,048 rows 377 / 409;
+      K 4,096 (213 GFLOP) 192 / 213, 2,048 rows 377 / 409 (with the present form of the activation this one takes 3 to 6 % less: 907 rows 202);
       a product that ends with its store: 1,000 x 4,096, K 1,024 13.8 / 13.3, 2,000 rows (17 GFLOP) 21 / 22, 4,000 rows 29 / 35; 2,345 x 2,048, K 2,048
       29 / 24; float results 2,000 x 8,512, K 2,048 81 / 63, 4,000 rows 138 / 128;
       17 to 64 rows, where a block streams its rows of W alone: gate and up 18 x 16,384, K 2,048 18.3 / 14.4, 64 rows 20.8 / 15.8, 64 x
@@ -708,7 +705,7 @@ def gemm_ring(a, w, out, residual=None, act=0, tile=0):
 def ring_rope_ok(a, w, head_dim, cos):
     """Whether qkv_rope runs the ring product with the rotation and the cache write as its epilogue: bf16 rows, whole heads of a multiple
     of 32 coordinates; up to 64 rows large weights only (64 x 6,144, K 2,048 17.7 / 10.0, 18 rows 10.1 / 9.6, K 4,096 17.0 / 16.2).  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
-    rows 40.8 / 36.6, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.8; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
+    rows 40.8 / 36.2, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.6; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
     (m, k), n = a.shape, w.shape[0]
     many = m >= RING_MIN_ROWS if m > SKINNY_ROWS else m >= RING_FEW_ROWS and 2 * n * k >= RING_FEW_PLAIN
     return (many and 2.0 * m * n * k <= RING_ROPE_FLOPS and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda
@@ -1369,7 +1366,7 @@ PARTIALS_MAX_COLS = 4096      # rows that post_norm_add holds in registers: only
 
 
 def gemm_for_norm(a, w, out, make_buffer, scratch=None):
-    """a . w^T for a reader that can add partial sums (post_norm_add): where the wide kernel cuts the product along
+    """a . w^T for a reader that can add partial sums (post_norm_add): where the ring or the wide kernel cuts the product along
     its inner size, its slices' partial sums are left in a buffer of the caller's (`make_buffer(floats)`: not the
     shared scratch, which the next wide product would overwrite) and a Partials is returned; every other product is
     finished into `out` (float [M, N]) and `out` is returned."""
