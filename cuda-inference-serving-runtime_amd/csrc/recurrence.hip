@@ -150,9 +150,10 @@ conv_silu_rows_kernel(const float* __restrict__ in, int ld, int first, const flo
         for (int k = 0; k < 4; ++k) y[k] = y[k] / (1.0f + expf(-y[k]));
         *(conv_f32x4*)(out + (size_t)t * channels + c) = y;
     };
-    const int mine = seg_of_row[min(t0 + (int)threadIdx.x % CONV_ROWS, t1 - 1)], whose = __builtin_amdgcn_readfirstlane(mine);
-    if (whose >= 0 && t1 - t0 == CONV_ROWS && __all(mine == whose) && t0 - seg_start[whose] >= TAPS - 1) {
-        // the block's rows are one portion's and reach back into rows of it only: nothing to look up row by row
+    const int whose = seg_of_row[t0];
+    if (whose >= 0 && t0 - seg_start[whose] >= TAPS - 1 && t0 + CONV_ROWS <= seg_start[whose + 1]) {
+        // the block's rows are one portion's and reach back into rows of it only: nothing to look up row by row.  (Told from the
+        // portion's ends, which all lanes read: of a row's last wave only the lanes that still have channels are left to vote.)
         conv_f32x4 x[CONV_ROWS + TAPS - 1];          // (a row is asked for eight rows before its turn)
 #pragma unroll
         for (int i = 0; i < TAPS - 1 + 8; ++i) x[i] = row(t0 - (TAPS - 1) + i);

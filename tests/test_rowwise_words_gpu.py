@@ -71,6 +71,30 @@ def test_short_convolution_wherever_a_portion_begins(taps, before):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("taps", [2, 4])
+@pytest.mark.parametrize("channels", [26116, 26144, 26172, 26112])
+def test_short_convolution_where_few_lanes_are_left(channels, taps):
+    """A row's last wave with 1, 8, 15 and all lanes; blocks that begin deep in a portion, in whose first, ninth, middle and last rows the
+    next portion or the padding begins.  Against 64 bits, the last channels apart; the padding stays."""
+    from runtime.kernels import ops
+    counts, pad = [24, 23, 32, 17, 25, 30], 5                   # portions from rows 24, 47, 79, 96, 121 on, padding from row 151
+    T, starts = sum(counts) + pad, np.concatenate(([0], np.cumsum(counts)))
+    assert [int(s) % 16 for s in starts[1:]] == [8, 15, 15, 0, 9, 7]
+    x, w, b = torch.randn(T, channels, device=DEV), torch.randn(channels, taps, device=DEV), torch.randn(channels, device=DEV)
+    state = torch.randn(len(counts), (taps - 1) * channels, device=DEV)
+    before, out = state.clone(), torch.full((T, channels), 9.0, device=DEV)
+    ops.conv_silu(x, w, b, state, out, ints(np.concatenate([np.repeat(np.arange(len(counts)), counts), [-1] * pad])), ints(starts),
+                  ints(range(len(counts))))
+    for s, n in enumerate(counts):
+        lo = int(starts[s])
+        inputs = torch.cat((before[s].view(taps - 1, channels).double(), x[lo:lo + n].double()))
+        want = torch.nn.functional.silu(sum(inputs[j:j + n] * w[:, j].double() for j in range(taps)) + b.double())
+        last = channels // 256 * 256 if channels % 256 else channels - 256
+        close(out[lo:lo + n, :last], want[:, :last], 2e-6)
+        close(out[lo:lo + n, last:], want[:, last:], 2e-6)
+    assert (out[-pad:] == 9.0).all()
+
+
 @pytest.mark.parametrize("groups, size", [(300, 4), (33, 128), (9, 132), (40, 256), (3, 260), (2, 1000), (1, 1028), (1, 2048), (1, 4096), (5, 100)])
 @pytest.mark.parametrize("gate_first, sigmoid, skip, shared, dtype", [(True, False, True, False, torch.bfloat16), (False, True, False, True, torch.float32),
                                                                      (False, False, True, False, torch.bfloat16)])
