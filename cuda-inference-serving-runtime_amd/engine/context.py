@@ -101,7 +101,9 @@ class StepContext:
         """residual += a . w^T, in place.  Where the product is cut along its inner size and the norm that reads the
         residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer."""
         if getattr(self.next_norm, "adds_partials", False):
-            partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch)
+            partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch, finish=True)
+            if partials is ops.ADDED:
+                return residual
             if partials is not None:
                 self.leave_unfinished(residual, partials)
                 return residual

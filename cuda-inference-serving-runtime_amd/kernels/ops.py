@@ -656,22 +656,33 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
         return size >= RING_FEW_PLAIN and (half or size <= RING_FEW_PLAIN_MOST)
     if m < RING_MIN_ROWS or w.dtype != torch.bfloat16 or flops > (RING_GATED_FLOPS if gated else RING_MOST_FLOPS):
         return False
-    library = library_ok(m, w, gated=gated, plain=not (fused or gated), floats=floats)
-    if library and (gated or cut):
+    many = outputs >= RING_MIN_OUTPUTS + RING_MIN_OUTPUTS_K * k
+    beats_library = gated or cut or fused or floats or flops <= RING_PLAIN_FLOPS or cols <= RING_PLAIN_COLS
+    if many and beats_library:
         return True
-    if outputs < (RING_MIN_OUTPUTS_SHORT if library and k <= RING_SHORT_K else RING_MIN_OUTPUTS + RING_MIN_OUTPUTS_K * k):
-        return False
-    return not library or fused or floats or flops <= RING_PLAIN_FLOPS or cols <= RING_PLAIN_COLS
+    library = library_ok(m, w, gated=gated, plain=not (fused or gated), floats=floats)
+    if many or not library:
+        return many and not library
+    return gated or cut or (beats_library and k <= RING_SHORT_K and outputs >= RING_MIN_OUTPUTS_SHORT)
+
+
+def _ring_operands(a, w, out):
+    """(pointer and row stride of a, of w, of out) where the ring product takes these operands (shapes are the caller's to check), else
+    None: an inner size of a multiple of 64, a multiple of four columns, 16-byte rows, results stored four at a time.  Asked once a product: a step that runs kernel by kernel waits for it."""
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not (a.is_cuda and w.is_cuda and out.is_cuda):
+        return None
+    k, n, item = a.shape[1], out.shape[1], out.element_size()
+    (lda, a1), (ldw, w1), (ldc, c1) = a.stride(), w.stride(), out.stride()
+    pa, pw, pc = a.data_ptr(), w.data_ptr(), out.data_ptr()
+    if (k % 64 or n % 4 or a1 != 1 or w1 != 1 or c1 != 1 or (lda | ldw) % 8 or (pa | pw) % 16 or lda < k or ldw < k or ldc < n or ldc % 4
+            or pc % (4 * item) or max(lda, ldw) * 1024 >= 1 << 31 or (w.shape[0] + 512) * ldw * 2 >= 1 << 31):
+        return None
+    return pa, lda, pw, ldw, pc, ldc
 
 
 def ring_fits(a, w, out):
-    """Whether the ring product takes these operands (shapes are the caller's to check): an inner size of a multiple of 64, a multiple
-    of four columns, 16-byte rows, results stored four at a time."""
-    n, k = out.shape[1], a.shape[1]
-    return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda and w.is_cuda and out.is_cuda and k % 64 == 0 and n % 4 == 0
-            and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1 and _skinny_ok(a, w) and a.stride(0) >= k and w.stride(0) >= k
-            and out.stride(0) >= n and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0
-            and max(a.stride(0), w.stride(0)) * 1024 < 1 << 31 and (w.shape[0] + 512) * w.stride(0) * 2 < 1 << 31)
+    """Whether the ring product takes these operands (shapes are the caller's to check)."""
+    return _ring_operands(a, w, out) is not None
 
 
 class RingSums:
@@ -681,24 +692,31 @@ class RingSums:
         self.parts, self.slices, self.rows, self.cols = parts, int(slices), int(rows), int(cols)
 
 
-def ring_sums(a, w, make_buffer):
-    """The RingSums of a . w^T in floats of the caller's (`make_buffer(floats)`), or None where the product is best not cut."""
-    (m, k), n = a.shape, w.shape[0]
+def _ring_sums(at, m, n, k, make_buffer):
+    """The RingSums of a product whose operands are `at` in floats of the caller's (`make_buffer(floats)`), or None where it is best
+    not cut."""
     slices = int(lib().cisr_gemm_ring_slices(m, n, k))
-    return RingSums(gemm_ring_partials(a, w, make_buffer(slices * m * n), slices), slices, m, n) if slices > 1 else None
+    if slices <= 1:
+        return None
+    parts = make_buffer(slices * m * n)
+    if parts.numel() < slices * m * n:
+        raise KernelError("ring product: too small a buffer for the partial sums")
+    _check(lib().cisr_gemm_ring_partials_bf16(*at[:4], _dev(parts, "partial sums", torch.float32), m, n, k, slices, 0, _stream()),
+           "gemm_ring_partials")
+    return RingSums(parts, slices, m, n)
 
 
 def gemm_ring(a, w, out, residual=None, act=0, tile=0):
     """out = a . w^T (+ residual, float rows that may be `out`) by the ring product; `act` (bf16 results): an ungated activation.
     `tile`: rows * 1000 + columns of a block (0: the fastest by the kernel's model of itself)."""
     (m, k), n = a.shape, w.shape[0]
-    if (tuple(out.shape) != (m, n) or w.shape[1] != k or not ring_fits(a, w, out) or (act and out.dtype != torch.bfloat16)
+    at = _ring_operands(a, w, out) if tuple(out.shape) == (m, n) and w.shape[1] == k else None
+    if (at is None or (act and out.dtype != torch.bfloat16)
             or (residual is not None and (residual.dtype != torch.float32 or out.dtype != torch.float32 or tuple(residual.shape) != (m, n)
                                           or residual.stride(1) != 1 or residual.stride(0) % 4 or residual.data_ptr() % 16 or not residual.is_cuda))):
         raise KernelError("gemm_ring: shape not supported")
     rp, ldr = (residual.data_ptr(), residual.stride(0)) if residual is not None else (None, 0)
-    _check(lib().cisr_gemm_ring_bf16(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), rp, ldr, m, n, k,
-                                     _storage(out, "out"), int(act), int(tile), _stream()), "gemm_ring")
+    _check(lib().cisr_gemm_ring_bf16(*at, rp, ldr, m, n, k, _storage(out, "out"), int(act), int(tile), _stream()), "gemm_ring")
     return out
 
 
@@ -708,19 +726,28 @@ def ring_rope_ok(a, w, head_dim, cos):
     rows 40.8 / 36.2, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.6; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
     (m, k), n = a.shape, w.shape[0]
     many = m >= RING_MIN_ROWS if m > SKINNY_ROWS else m >= RING_FEW_ROWS and 2 * n * k >= RING_FEW_PLAIN
-    return (many and 2.0 * m * n * k <= RING_ROPE_FLOPS and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.is_cuda
-            and w.is_cuda and k % 64 == 0 and head_dim % 32 == 0 and 2 * cos.shape[1] == head_dim and a.stride(1) == 1 and w.stride(1) == 1
-            and _skinny_ok(a, w) and a.stride(0) >= k and w.stride(0) >= k and a.stride(0) * 1024 < 1 << 31 and (n + 512) * w.stride(0) * 2 < 1 << 31)
+    if (not many or 2.0 * m * n * k > RING_ROPE_FLOPS or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not (a.is_cuda and w.is_cuda)
+            or k % 64 or head_dim % 32 or 2 * cos.shape[1] != head_dim):
+        return False
+    (lda, a1), (ldw, w1) = a.stride(), w.stride()
+    return (a1 == 1 and w1 == 1 and (lda | ldw) % 8 == 0 and (a.data_ptr() | w.data_ptr()) % 16 == 0 and lda >= k and ldw >= k
+            and lda * 1024 < 1 << 31 and (n + 512) * ldw * 2 < 1 << 31)
 
 
 def gemm_ring_gated(a, w, out, law=None, tile=0):
     """out[M, I] = act(a . Wg^T, a . Wu^T), w = [Wg; Wu], by the ring product; `law` as gemm_swiglu."""
     (m, k), inter = a.shape, w.shape[0] // 2
-    if tuple(out.shape) != (m, inter) or tuple(w.shape) != (2 * inter, k) or out.dtype != torch.bfloat16 or not ring_fits(a, w, out):
+    fits = tuple(out.shape) == (m, inter) and tuple(w.shape) == (2 * inter, k) and out.dtype == torch.bfloat16
+    at = _ring_operands(a, w, out) if fits else None
+    if at is None:
         raise KernelError("gemm_ring_gated: shape not supported")
-    lim, slope, shift = (float(x) for x in law or (0.0, 0.0, 0.0))
-    _check(lib().cisr_gemm_ring_bf16_gated(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), m, inter, k,
-                                           inter, lim, slope, shift, int(tile), _stream()), "gemm_ring_gated")
+    return _ring_gated(at, m, inter, k, out, law, tile)
+
+
+def _ring_gated(at, m, inter, k, out, law, tile=0):
+    lim, slope, shift = law or (0.0, 0.0, 0.0)
+    _check(lib().cisr_gemm_ring_bf16_gated(*at, m, inter, k, inter, float(lim), float(slope), float(shift), int(tile), _stream()),
+           "gemm_ring_gated")
     return out
 
 
@@ -765,11 +792,12 @@ def gemm(a, w, out, residual=None, after_norm=False, scratch=None):
         code = lib().cisr_gemm_f32(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
                                    rp, ldr, m, n, k, _stream())
     elif (a.dtype == torch.bfloat16 and ring_ahead(m, w, fused=residual is not None, floats=out.dtype == torch.float32, cut=residual is not None)
-          and ring_fits(a, w, out) and (residual is None or (ldr % 4 == 0 and rp % 16 == 0))):
-        sums = None
+          and (at := _ring_operands(a, w, out)) is not None and (residual is None or (ldr % 4 == 0 and rp % 16 == 0))):
         if residual is not None and residual is out and partials_ok(out):
-            sums = ring_sums(a, w, lambda floats: _wide_workspace(scratch, a.device, floats))
-        return gemm_ring(a, w, out, residual) if sums is None else add_partials(out, (sums, 0))
+            sums = _ring_sums(at, m, n, k, lambda floats: _wide_workspace(scratch, a.device, floats))
+            if sums is not None:
+                return add_partials(out, (sums, 0))
+        code = lib().cisr_gemm_ring_bf16(*at, rp, ldr, m, n, k, _storage(out, "out"), 0, 0, _stream())
     elif (a.dtype == torch.bfloat16 and library_ok(m, w, plain=residual is None, floats=out.dtype == torch.float32) and a.is_contiguous() and out.is_contiguous()
           and (residual is None or residual is out)):
         if residual is None:
@@ -898,20 +926,27 @@ def _gemm_wide(a, w, out, residual, swiglu, what, scratch=None):
     return out
 
 
-def gemm_unfinished(a, w, residual, scratch=None):
+ADDED = (None, -1)      # gemm_unfinished: the product is added already
+
+
+def gemm_unfinished(a, w, residual, scratch=None, finish=False):
     """The product a . w^T that is to be added to the float rows `residual`, left unfinished where adding it takes a
     kernel of its own: the wide kernel's partial sums of a product cut into slices, (partial sums [slices, M, N],
     slices), the ring product's, (a RingSums, 0), or the library's bf16 product, (product [M, N], 0); rmsnorm_partials or
-    add_partials then are that kernel.  None (nothing done) for every other product: call gemm."""
+    add_partials then are that kernel.  None (nothing done) for every other product: call gemm.  `finish`: a ring product that is
+    best not cut is added to `residual` at once (ADDED), so that gemm need not ask the same again."""
     m, k = a.shape
     n = w.shape[0]
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape[1] != k or tuple(residual.shape) != (m, n)
             or not partials_ok(residual)):
         return None
-    if ring_ahead(m, w, fused=True, cut=True) and ring_fits(a, w, residual):
-        sums = ring_sums(a, w, lambda floats: _wide_workspace(scratch, a.device, floats))
-        if sums is None:
-            return None                     # (not cut: gemm adds it in the product's epilogue)
+    if ring_ahead(m, w, fused=True, cut=True) and (at := _ring_operands(a, w, residual)) is not None:
+        sums = _ring_sums(at, m, n, k, lambda floats: _wide_workspace(scratch, a.device, floats))
+        if sums is None:                    # (not cut: added in the product's epilogue)
+            if not finish:
+                return None
+            _check(lib().cisr_gemm_ring_bf16(*at, at[4], at[5], m, n, k, F32, 0, 0, _stream()), "gemm_unfinished")
+            return ADDED
         return (sums, 0) if m > SKINNY_ROWS else (sums.parts, sums.slices)      # (few rows: a block a row adds them)
     if library_ok(m, w):
         if not a.is_contiguous():
@@ -1000,8 +1035,8 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         return out
     if out.dtype != a.dtype or a.dtype != w_gate_up.dtype:
         raise KernelError("gemm_swiglu: dtypes differ")
-    if a.dtype == torch.bfloat16 and ring_ahead(m, w_gate_up, gated=True) and ring_fits(a, w_gate_up, out):
-        return gemm_ring_gated(a, w_gate_up, out, law)
+    if a.dtype == torch.bfloat16 and ring_ahead(m, w_gate_up, gated=True) and (at := _ring_operands(a, w_gate_up, out)) is not None:
+        return _ring_gated(at, m, inter, k, out, law)
     activate = swiglu if law is None else (lambda gu, o: glu_clamped(gu, o, *law))
     if a.dtype == torch.bfloat16 and library_ok(m, w_gate_up, gated=True) and a.is_contiguous():
         product = _scratch_bf16(scratch, a.device, m, two_i)
@@ -1057,6 +1092,11 @@ def qkv_rope_fused_ok(a, w, head_dim, cos, normed):
         return False
     if not normed and ring_rope_ok(a, w, head_dim, cos):
         return True
+    return _few_rope_ok(a, w, head_dim, cos, normed)
+
+
+def _few_rope_ok(a, w, head_dim, cos, normed):
+    m, k = a.shape
     return (w.dtype == torch.bfloat16 and m <= SKINNY_ROWS and k % 8 == 0 and head_dim % 16 == 0
             and 2 * cos.shape[1] == head_dim and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0
             and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0
@@ -1097,7 +1137,9 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     m, k = a.shape
     has_kv = kcache is not None
     n_kv = kv_heads if has_kv else 0
-    if not qkv_rope_fused_ok(a, w, dim, cos, norm is not None) or tuple(w.shape) != ((heads + 2 * n_kv) * dim, k):
+    ring = norm is None and ring_rope_ok(a, w, dim, cos)
+    if (not (ring or (_few_rope_ok(a, w, dim, cos, False) if norm is None else qkv_rope_fused_ok(a, w, dim, cos, True)))
+            or tuple(w.shape) != ((heads + 2 * n_kv) * dim, k)):
         raise KernelError("qkv_rope: shape not supported by the fused kernel")
     wp, eps = (None, 0.0)
     if norm is not None:
@@ -1109,7 +1151,7 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
         vp = _dev(vcache, "vcache", torch.bfloat16, (pages, kv_heads, dim, page_size))
         sp = _dev(slots, "slots", torch.int32, (m,))
     max_pos = cos.shape[0]
-    if norm is None and ring_rope_ok(a, w, dim, cos):
+    if ring:
         _check(lib().cisr_gemm_ring_rope(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), _dev(q_out, "q_out", torch.bfloat16, (m, heads * dim)),
                                          heads * dim, m, k, _dev(positions, "positions", torch.int32, (m,)), sp, _dev(cos, "cos", torch.float32),
                                          _dev(sin, "sin", torch.float32, (max_pos, dim // 2)), kp, vp, heads, n_kv, dim, page_size, max_pos, 0,
@@ -1373,9 +1415,12 @@ def gemm_for_norm(a, w, out, make_buffer, scratch=None):
     m, k = a.shape
     n = w.shape[0]
     if (a.dtype == torch.bfloat16 and n <= PARTIALS_MAX_COLS and tuple(out.shape) == (m, n) and w.shape[1] == k
-            and ring_ahead(m, w, fused=True, floats=True, cut=True) and ring_fits(a, w, out)):
-        sums = ring_sums(a, w, make_buffer)
-        return gemm_ring(a, w, out) if sums is None else Partials(sums.parts, sums.slices, m, n)
+            and ring_ahead(m, w, fused=True, floats=True, cut=True) and (at := _ring_operands(a, w, out)) is not None):
+        sums = _ring_sums(at, m, n, k, make_buffer)
+        if sums is not None:
+            return Partials(sums.parts, sums.slices, m, n)
+        _check(lib().cisr_gemm_ring_bf16(*at, None, 0, m, n, k, _storage(out, "out"), 0, 0, _stream()), "gemm_ring")
+        return out
     if (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and 0 < m <= SKINNY_ROWS and n <= PARTIALS_MAX_COLS
             and not library_ok(m, w) and _skinny_ok(a, w) and wide_ok(m, w)):
         need = _wide_plan(m, n, k, False)
@@ -1613,8 +1658,9 @@ def gemm_gelu(a, w, out, kind="gelu", scratch=None, product=None):
     fused = (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and tuple(out.shape) == (m, n)
              and w.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1)
     act = 1 + GELU_KINDS[kind]
-    if fused and ring_ahead(m, w, fused=True) and ring_fits(a, w, out):
-        return gemm_ring(a, w, out, act=act)
+    if fused and ring_ahead(m, w, fused=True) and (at := _ring_operands(a, w, out)) is not None:
+        _check(lib().cisr_gemm_ring_bf16(*at, None, 0, m, n, k, BF16, act, 0, _stream()), "gemm_gelu")
+        return out
     fused = fused and not library_ok(m, w)
     if fused and m <= SKINNY_ROWS and _skinny_ok(a, w) and not wide_ok(m, w):
         _check(lib().cisr_gemm_skinny_bf16_act(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),

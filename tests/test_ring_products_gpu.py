@@ -144,6 +144,24 @@ def test_calls_that_came_to_these_kernels_against_the_others(ops, M, N, K, monke
         assert (got.double() - want.double()).abs().max().item() <= 2.0 ** -5 * max(scale, want.abs().max().item()), i
 
 
+def test_a_product_is_asked_about_once(ops, monkeypatch):
+    """A step that runs kernel by kernel waits for the host: a product's operands are looked at once, whatever it ends in."""
+    a, w, r = operands(300, 2048, 576)
+    a2, w2, _ = operands(300, 2048, 8192)                                       # (cut along its inner size)
+    asked, ask = [], ops._ring_operands
+    monkeypatch.setattr(ops, "_ring_operands", lambda *x: (asked.append(1), ask(*x))[1])
+    monkeypatch.setattr(ops, "ring_fits", None)
+    half = torch.empty(300, 2048, dtype=torch.bfloat16, device=DEV)
+    calls = [lambda: ops.gemm(a, w, r, residual=r), lambda: ops.gemm(a, w, half), lambda: ops.gemm(a2, w2, r, residual=r),
+             lambda: ops.gemm_swiglu(a, w, half[:, :1024].contiguous()), lambda: ops.gemm_unfinished(a, w, r, finish=True),
+             lambda: ops.gemm_unfinished(a2, w2, r, finish=True)]
+    results = [call() for call in calls]
+    assert len(asked) == len(calls) and results[-2] is ops.ADDED and isinstance(results[-1][0], ops.RingSums)
+    want = r + a.float() @ w.float().T
+    assert ops.gemm_unfinished(a, w, r, finish=True) is ops.ADDED
+    assert (r - want).abs().max() <= 1e-2
+
+
 def test_on_every_replay_of_a_captured_graph(ops):
     M, N, K = 300, 2048, 8192
     a, w, r = operands(M, N, K)
