@@ -86,7 +86,7 @@ class ModelRunner:
                                   zero_state=lambda t, s: t[s].zero_(),
                                   copy_state=lambda t, a, b: t[b].copy_(t[a]))
         self.workspace = Workspace(self.device)
-        self.scratch = ops.ScratchPool()   # what products need beyond their operands (never shared with another runner)
+        self.scratch = ops.ScratchPool(ring=not getattr(model, "routes", False))   # what products need beyond their operands (never shared with another runner)
         self.max_context = model.max_positions
         self.table_width = -(-self.max_context // page_size)
         self._staging = []

@@ -575,10 +575,12 @@ class ScratchPool:
     sum into the residual, the wide kernel's partial sums, the slice winners of the argmax.  A buffer is handed out
     again to every later call that it is large enough for, and none is freed before `clear`: captured programs keep
     the addresses.  A step function owns one pool (calls on its stream are ordered, so they can share buffers);
-    calls that name no pool share DEFAULT_SCRATCH."""
+    calls that name no pool share DEFAULT_SCRATCH.  `ring`: whether the products of its steps may be ring products
+    (csrc/gemm_ring.inc); a model that sends rows to experts takes none (see Model.routes)."""
 
-    def __init__(self):
+    def __init__(self, ring=True):
         self.buffers = {}   # (kind, device, dtype) -> [tensors]
+        self.ring = bool(ring)
 
     def get(self, kind, elements, dtype, device):
         pool = self.buffers.setdefault((kind, device, dtype), [])
@@ -627,6 +629,10 @@ RING_FEW_ROWS, RING_HALF_ROWS = 17, 33
 RING_FEW_GATED, RING_HALF_GATED = 64 << 20, 16 << 20
 RING_FEW_CUT = 32 << 20
 RING_FEW_PLAIN, RING_FEW_PLAIN_MOST = 24 << 20, 64 << 20
+
+
+def _ring_open(scratch):
+    return scratch is None or scratch.ring
 
 
 def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
@@ -791,7 +797,7 @@ def gemm(a, w, out, residual=None, after_norm=False, scratch=None):
             raise KernelError("gemm: float operands need a float output")
         code = lib().cisr_gemm_f32(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
                                    rp, ldr, m, n, k, _stream())
-    elif (a.dtype == torch.bfloat16 and ring_ahead(m, w, fused=residual is not None, floats=out.dtype == torch.float32, cut=residual is not None)
+    elif (a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w, fused=residual is not None, floats=out.dtype == torch.float32, cut=residual is not None)
           and (at := _ring_operands(a, w, out)) is not None and (residual is None or (ldr % 4 == 0 and rp % 16 == 0))):
         if residual is not None and residual is out and partials_ok(out):
             sums = _ring_sums(at, m, n, k, lambda floats: _wide_workspace(scratch, a.device, floats))
@@ -940,7 +946,7 @@ def gemm_unfinished(a, w, residual, scratch=None, finish=False):
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape[1] != k or tuple(residual.shape) != (m, n)
             or not partials_ok(residual)):
         return None
-    if ring_ahead(m, w, fused=True, cut=True) and (at := _ring_operands(a, w, residual)) is not None:
+    if _ring_open(scratch) and ring_ahead(m, w, fused=True, cut=True) and (at := _ring_operands(a, w, residual)) is not None:
         sums = _ring_sums(at, m, n, k, lambda floats: _wide_workspace(scratch, a.device, floats))
         if sums is None:                    # (not cut: added in the product's epilogue)
             if not finish:
@@ -1035,7 +1041,7 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         return out
     if out.dtype != a.dtype or a.dtype != w_gate_up.dtype:
         raise KernelError("gemm_swiglu: dtypes differ")
-    if a.dtype == torch.bfloat16 and ring_ahead(m, w_gate_up, gated=True) and (at := _ring_operands(a, w_gate_up, out)) is not None:
+    if a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w_gate_up, gated=True) and (at := _ring_operands(a, w_gate_up, out)) is not None:
         return _ring_gated(at, m, inter, k, out, law)
     activate = swiglu if law is None else (lambda gu, o: glu_clamped(gu, o, *law))
     if a.dtype == torch.bfloat16 and library_ok(m, w_gate_up, gated=True) and a.is_contiguous():
@@ -1085,12 +1091,12 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
     return activate(gate_up, out)
 
 
-def qkv_rope_fused_ok(a, w, head_dim, cos, normed):
-    """Whether the fused projection + rotary + scatter kernel takes this shape."""
+def qkv_rope_fused_ok(a, w, head_dim, cos, normed, scratch=None):
+    """Whether the fused projection + rotary + scatter kernel takes this shape (`scratch`: the pool that qkv_rope is given)."""
     m, k = a.shape
     if normed and wide_ok(m, w, after_norm=True, fused=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
         return False
-    if not normed and ring_rope_ok(a, w, head_dim, cos):
+    if not normed and _ring_open(scratch) and ring_rope_ok(a, w, head_dim, cos):
         return True
     return _few_rope_ok(a, w, head_dim, cos, normed)
 
@@ -1137,7 +1143,7 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     m, k = a.shape
     has_kv = kcache is not None
     n_kv = kv_heads if has_kv else 0
-    ring = norm is None and ring_rope_ok(a, w, dim, cos)
+    ring = norm is None and _ring_open(scratch) and ring_rope_ok(a, w, dim, cos)
     if (not (ring or (_few_rope_ok(a, w, dim, cos, False) if norm is None else qkv_rope_fused_ok(a, w, dim, cos, True)))
             or tuple(w.shape) != ((heads + 2 * n_kv) * dim, k)):
         raise KernelError("qkv_rope: shape not supported by the fused kernel")
@@ -1415,7 +1421,7 @@ def gemm_for_norm(a, w, out, make_buffer, scratch=None):
     m, k = a.shape
     n = w.shape[0]
     if (a.dtype == torch.bfloat16 and n <= PARTIALS_MAX_COLS and tuple(out.shape) == (m, n) and w.shape[1] == k
-            and ring_ahead(m, w, fused=True, floats=True, cut=True) and (at := _ring_operands(a, w, out)) is not None):
+            and _ring_open(scratch) and ring_ahead(m, w, fused=True, floats=True, cut=True) and (at := _ring_operands(a, w, out)) is not None):
         sums = _ring_sums(at, m, n, k, make_buffer)
         if sums is not None:
             return Partials(sums.parts, sums.slices, m, n)
@@ -1658,7 +1664,7 @@ def gemm_gelu(a, w, out, kind="gelu", scratch=None, product=None):
     fused = (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and tuple(out.shape) == (m, n)
              and w.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1)
     act = 1 + GELU_KINDS[kind]
-    if fused and ring_ahead(m, w, fused=True) and (at := _ring_operands(a, w, out)) is not None:
+    if fused and _ring_open(scratch) and ring_ahead(m, w, fused=True) and (at := _ring_operands(a, w, out)) is not None:
         _check(lib().cisr_gemm_ring_bf16(*at, None, 0, m, n, k, BF16, act, 0, _stream()), "gemm_gelu")
         return out
     fused = fused and not library_ok(m, w)

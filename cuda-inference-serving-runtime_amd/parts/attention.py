@@ -81,15 +81,15 @@ class PagedAttention(Mixer):
     def _interleaved(self):
         return getattr(self.position, "pairing", "split_half") == "interleaved"
 
-    def _fused_projection_ok(self, a, normed):
+    def _fused_projection_ok(self, a, normed, scratch):
         cos, _ = self.position.tables()
         # (the fused kernels turn split-half pairs only; another pairing takes the general rotary kernel)
         if self._interleaved or self.bias:
             return False
-        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
+        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed, scratch) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
 
     def fuses_norm(self, norm, residual, ctx):
-        return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True)
+        return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True, ctx.scratch)
 
     def forward(self, h, residual, ctx, site, norm=None):
         T = residual.shape[0]
@@ -101,7 +101,7 @@ class PagedAttention(Mixer):
             kcache_w = vcache_w = slots = None
         else:
             kcache_w, vcache_w, slots = kcache, vcache, view.slots
-        if norm is not None or self._fused_projection_ok(h, False):
+        if norm is not None or self._fused_projection_ok(h, False, ctx.scratch):
             # few rows (in 32 bits any): norm, projections, rotary embedding and the cache write are one kernel
             q, q_stride = ctx.buffer("attn.q", (T, nh * D), ctx.dtype), nh * D
             ops.qkv_rope(residual if norm is not None else h, self.w_in, q, ctx.positions, slots, cos, sin,

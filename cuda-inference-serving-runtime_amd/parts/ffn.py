@@ -181,6 +181,7 @@ class RoutedExperts(FeedForward):
     adds the sublayer's result (ops.WeightedRows).  `ride(weight)`: further rows for the router's product, whose
     float results are then `rider`.  `names`: (router, expert prefix, up, down), the tensors' names under `name`;
     expert j's matrices are `<name>.<prefix>j.<up|down>`."""
+    routes = True            # sends rows to experts of their choice
 
     def __init__(self, name, hidden, intermediate, experts, top, names=("router", "e", "up", "down")):
         if not 0 < top <= min(experts, 16):
@@ -259,6 +260,7 @@ class ScoredExperts(FeedForward):
     [gate; up] a expert with the activation as its epilogue (float32: a kernel after it).  `names`: (router, correction, expert
     prefix, gate, up, down)."""
     leaves_rows = True       # `output` takes `unsummed`
+    routes = True            # sends rows to experts of their choice
 
     def __init__(self, name, hidden, intermediate, experts, top, identity=0, groups=None, shared=None, correction=True,
                  names=("router", "correction", "e", "gate", "up", "down"), scores="softmax", group_pairs=False, floor=None, law=None,

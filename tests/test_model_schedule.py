@@ -46,3 +46,12 @@ def test_what_a_reading_layer_expects_is_checked_against_what_is_kept():
         build([ScheduleEntry(1, reads=1), ScheduleEntry(0)])
     with pytest.raises(ValueError, match="earlier entry"):
         build([ScheduleEntry(0), ScheduleEntry(1, reads=0), ScheduleEntry(1, reads=1)])   # the entry it names keeps none
+
+
+def test_which_models_send_rows_to_experts():
+    """A model says whether one of its parts routes rows, however deep the part lies."""
+    from runtime.config.presets import preset, preset_names
+    from runtime.engine.loading import build_from_config_dict
+    routed = {name for name in preset_names() if build_from_config_dict(preset(name))[2].routes}
+    assert routed == {"movazen-tiny", "noresun-tiny", "zovozen-tiny"}
+    assert not build([]).routes

@@ -162,6 +162,49 @@ def test_a_product_is_asked_about_once(ops, monkeypatch):
     assert (r - want).abs().max() <= 1e-2
 
 
+def test_models_that_route_rows_take_no_ring_products(ops, monkeypatch):
+    """Every entry point given a pool without ring products, and a step of a model with experts: the bits are those of the other kernels."""
+    from runtime.engine import ModelRunner, StepEntry, random_model
+    asked, ask = [], ops._ring_operands
+    monkeypatch.setattr(ops, "_ring_operands", lambda *x: (asked.append(1), ask(*x))[1])
+    M, heads, dim = 500, 8, 64
+    a, w, r = operands(M, 3 * heads * dim, 512)
+    angle = torch.rand(M, dim // 2, device=DEV)
+    cos, sin = angle.cos(), angle.sin()
+    half = lambda cols: torch.empty(M, cols, dtype=torch.bfloat16, device=DEV)      # noqa: E731
+
+    def calls(pool):
+        yield lambda: ops.gemm(a, w, r.clone(), residual=r, scratch=pool)
+        yield lambda: ops.gemm(a, w, half(w.shape[0]), scratch=pool)
+        yield lambda: ops.gemm_swiglu(a, w, half(w.shape[0] // 2), scratch=pool)
+        yield lambda: ops.gemm_gelu(a, w, half(w.shape[0]), scratch=pool, product=half(w.shape[0]))
+        yield lambda: ops.gemm_for_norm(a, w, torch.empty_like(r), lambda n: torch.empty(n, device=DEV), scratch=pool)
+        yield lambda: ops.gemm_unfinished(a, w, r.clone(), scratch=pool, finish=True)
+    open_, closed = ops.ScratchPool(), ops.ScratchPool(ring=False)
+    for i, call in enumerate(calls(open_)):
+        call()
+        assert len(asked) == i + 1
+    kept = [call() for call in calls(closed)]
+    assert len(asked) == i + 1 and kept[-1] is None
+    assert ops.qkv_rope_fused_ok(a, w, dim, cos, False, open_) and not ops.qkv_rope_fused_ok(a, w, dim, cos, False, closed)
+    with pytest.raises(ops.KernelError):
+        ops.qkv_rope(a, w, half(heads * dim), torch.zeros(M, dtype=torch.int32, device=DEV), None, cos, sin, None, None, 3 * heads, 0, dim, 16, scratch=closed)
+    mlp = {"kind": "moe", "expert": {"ff": 512}, "router": {"experts": 8, "top": 2}}
+    raw = {"architecture": "Noresun", "vocab": 1024, "width": 1024, "postln_alpha": 2.0, "norm": {"eps": 1e-5}, "max_positions": 512,
+           "embedding": {"scale": 1.0, "bigram": {"buckets": 509, "mul_prev": 13, "mul_cur": 5}},
+           "layers": [{"type": "mingru", "mixer": {"width": 1024}, "mlp": mlp}] * 2}
+    del asked[:]
+    results = []
+    for ring in (False, True):
+        runner = ModelRunner(random_model(raw, seed=3, std=0.03), n_pages=40, page_size=16, max_requests=2)
+        assert not runner.scratch.ring
+        runner.scratch.ring = ring
+        runner.create("a")
+        results.append(runner.step([StepEntry("a", [i * 7 % 1024 for i in range(300)], [0, 150, 299])]).clone())
+        assert bool(asked) == ring
+    assert not torch.equal(*results)
+
+
 def test_on_every_replay_of_a_captured_graph(ops):
     M, N, K = 300, 2048, 8192
     a, w, r = operands(M, N, K)
