@@ -726,14 +726,14 @@ def gemm_ring(a, w, out, residual=None, act=0, tile=0):
     return out
 
 
-def ring_rope_ok(a, w, head_dim, cos):
+def ring_rope_ok(a, w, head_dim, cos, sin=None):
     """Whether qkv_rope runs the ring product with the rotation and the cache write as its epilogue: bf16 rows, whole heads of a multiple
-    of 32 coordinates; up to 64 rows large weights only (64 x 6,144, K 2,048 17.7 / 10.0, 18 rows 10.1 / 9.6, K 4,096 17.0 / 16.2).  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
+    of 32 coordinates, tables on 16 bytes; up to 64 rows large weights only (64 x 6,144, K 2,048 17.7 / 10.0, 18 rows 10.1 / 9.6, K 4,096 17.0 / 16.2).  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
     rows 40.8 / 36.2, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.6; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
     (m, k), n = a.shape, w.shape[0]
     many = m >= RING_MIN_ROWS if m > SKINNY_ROWS else m >= RING_FEW_ROWS and 2 * n * k >= RING_FEW_PLAIN
     if (not many or 2.0 * m * n * k > RING_ROPE_FLOPS or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not (a.is_cuda and w.is_cuda)
-            or k % 64 or head_dim % 32 or 2 * cos.shape[1] != head_dim):
+            or k % 64 or head_dim % 32 or 2 * cos.shape[1] != head_dim or cos.data_ptr() % 16 or (sin is not None and sin.data_ptr() % 16)):
         return False
     (lda, a1), (ldw, w1) = a.stride(), w.stride()
     return (a1 == 1 and w1 == 1 and (lda | ldw) % 8 == 0 and (a.data_ptr() | w.data_ptr()) % 16 == 0 and lda >= k and ldw >= k
@@ -1091,12 +1091,13 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
     return activate(gate_up, out)
 
 
-def qkv_rope_fused_ok(a, w, head_dim, cos, normed, scratch=None):
-    """Whether the fused projection + rotary + scatter kernel takes this shape (`scratch`: the pool that qkv_rope is given)."""
+def qkv_rope_fused_ok(a, w, head_dim, cos, normed, scratch=None, sin=None):
+    """Whether the fused projection + rotary + scatter kernel takes this shape and, where `sin` is at hand, these tables (`scratch`: the pool that
+    qkv_rope is given)."""
     m, k = a.shape
     if normed and wide_ok(m, w, after_norm=True, fused=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
         return False
-    if not normed and _ring_open(scratch) and ring_rope_ok(a, w, head_dim, cos):
+    if not normed and _ring_open(scratch) and ring_rope_ok(a, w, head_dim, cos, sin):
         return True
     return _few_rope_ok(a, w, head_dim, cos, normed)
 
@@ -1143,7 +1144,9 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     m, k = a.shape
     has_kv = kcache is not None
     n_kv = kv_heads if has_kv else 0
-    ring = norm is None and _ring_open(scratch) and ring_rope_ok(a, w, dim, cos)
+    # (queries and key pages that are not on 8 bytes, or other tables: up to 64 rows the kernels of few rows)
+    ring = (norm is None and _ring_open(scratch) and ring_rope_ok(a, w, dim, cos, sin) and q_out.data_ptr() % 8 == 0
+            and (not has_kv or kcache.data_ptr() % 8 == 0))
     if (not (ring or (_few_rope_ok(a, w, dim, cos, False) if norm is None else qkv_rope_fused_ok(a, w, dim, cos, True)))
             or tuple(w.shape) != ((heads + 2 * n_kv) * dim, k)):
         raise KernelError("qkv_rope: shape not supported by the fused kernel")

@@ -82,11 +82,11 @@ class PagedAttention(Mixer):
         return getattr(self.position, "pairing", "split_half") == "interleaved"
 
     def _fused_projection_ok(self, a, normed, scratch):
-        cos, _ = self.position.tables()
+        cos, sin = self.position.tables()
         # (the fused kernels turn split-half pairs only; another pairing takes the general rotary kernel)
         if self._interleaved or self.bias:
             return False
-        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed, scratch) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
+        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed, scratch, sin) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
 
     def fuses_norm(self, norm, residual, ctx):
         return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True, ctx.scratch)

@@ -284,6 +284,39 @@ def test_rotation_and_cache_write_in_the_epilogue(ops, M, K, heads, kv, dim, pag
         assert (got - want).norm() <= 2.0 ** -7 * want.norm()
 
 
+@pytest.mark.parametrize("odd", ["cos", "sin", "q", "keys"])
+@pytest.mark.parametrize("M", [64, 200])
+def test_rotation_with_operands_between_words(ops, M, odd):
+    """Tables, queries or key pages that do not begin on the words the epilogue moves take another route: the layer's projection beside the
+    rotary kernel, or up to 64 rows the kernels of few rows."""
+    heads, kv, dim, page, K = 32, 32, 64, 16, 2048
+
+    def at_odd(t, name):
+        flat = torch.empty(t.numel() + 2, dtype=t.dtype, device=DEV)
+        view = flat[1:1 + t.numel()].view(t.shape) if odd == name else flat[:t.numel()].view(t.shape)
+        return view.copy_(t)
+    a, w, _ = operands(M, (heads + 2 * kv) * dim, K, seed=M)
+    angle = torch.rand(2 * M, dim // 2, device=DEV) * 6.3
+    cos, sin = at_odd(angle.cos(), "cos"), at_odd(angle.sin(), "sin")
+    positions, slots = torch.arange(M, device=DEV, dtype=torch.int32), torch.arange(M, device=DEV, dtype=torch.int32)
+    keys = at_odd(torch.zeros(M // page + 1, kv, page, dim, dtype=torch.bfloat16, device=DEV), "keys")
+    values = torch.zeros(M // page + 1, kv, dim, page, dtype=torch.bfloat16, device=DEV)
+    q = at_odd(torch.zeros(M, heads * dim, dtype=torch.bfloat16, device=DEV), "q")
+    if M > 64:
+        if odd in ("cos", "sin"):           # (what PagedAttention asks before it chooses)
+            assert not ops.qkv_rope_fused_ok(a, w, dim, cos, False, None, sin)
+        with pytest.raises(ops.KernelError):
+            ops.qkv_rope(a, w, q, positions, slots, cos, sin, keys, values, heads, kv, dim, page)
+        return
+    ops.qkv_rope(a, w, q, positions, slots, cos, sin, keys, values, heads, kv, dim, page)
+    rows = ops.gemm(a, w, torch.empty(M, w.shape[0], dtype=torch.bfloat16, device=DEV))
+    ref_keys, ref_values = torch.zeros_like(keys), torch.zeros_like(values)
+    ops.rope_scatter(rows, positions, slots, angle.cos(), angle.sin(), ref_keys, ref_values, heads, kv, dim, page)
+    for got, want in ((q, rows[:, :heads * dim]), (keys, ref_keys), (values, ref_values)):
+        # (rounded to bf16 before the turn on one side only, and both round the result: as in the test above)
+        assert ((got.double() - want.double()).abs() <= 2.0 ** -7 * want.double().abs() + 2.0 ** -8 * 2 * want.double().abs().max()).all()
+
+
 @pytest.mark.parametrize("law", [None, (7.0, 1.702, 1.0), (-1.0, 0.0, 0.0)])
 def test_gates_of_every_size_against_64_bits(law):
     """Gates from -1e30 to 1e30 with both signs' smallest, and infinite ones, as products with one term: the activation's own error stays
