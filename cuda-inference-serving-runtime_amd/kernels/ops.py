@@ -674,14 +674,16 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
 
 def _ring_operands(a, w, out):
     """(pointer and row stride of a, of w, of out) where the ring product takes these operands (shapes are the caller's to check), else
-    None: an inner size of a multiple of 64, a multiple of four columns, 16-byte rows, results stored four at a time.  Asked once a product: a step that runs kernel by kernel waits for it."""
+    None: an inner size of a multiple of 64, a multiple of four columns, 16-byte rows, results stored four at a time that do not lie
+    where the rows do (its blocks read `a` while others write).  Asked once a product: a step that runs kernel by kernel waits for it."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not (a.is_cuda and w.is_cuda and out.is_cuda):
         return None
-    k, n, item = a.shape[1], out.shape[1], out.element_size()
+    (m, k), n, item = a.shape, out.shape[1], out.element_size()
     (lda, a1), (ldw, w1), (ldc, c1) = a.stride(), w.stride(), out.stride()
     pa, pw, pc = a.data_ptr(), w.data_ptr(), out.data_ptr()
     if (k % 64 or n % 4 or a1 != 1 or w1 != 1 or c1 != 1 or (lda | ldw) % 8 or (pa | pw) % 16 or lda < k or ldw < k or ldc < n or ldc % 4
-            or pc % (4 * item) or max(lda, ldw) * 1024 >= 1 << 31 or (w.shape[0] + 512) * ldw * 2 >= 1 << 31):
+            or pc % (4 * item) or max(lda, ldw) * 1024 >= 1 << 31 or (w.shape[0] + 512) * ldw * 2 >= 1 << 31
+            or (pc < pa + 2 * (m * lda - lda + k) and pa < pc + item * (m * ldc - ldc + n))):
         return None
     return pa, lda, pw, ldw, pc, ldc
 

@@ -284,6 +284,23 @@ def test_rotation_and_cache_write_in_the_epilogue(ops, M, K, heads, kv, dim, pag
         assert (got - want).norm() <= 2.0 ** -7 * want.norm()
 
 
+def test_a_result_may_lie_where_the_rows_were(ops):
+    """Gate and up, and the gelu, of large weights into the buffer of their rows: the product goes to a buffer of its own first, as it
+    did before there were ring products, whose blocks would read rows that others have replaced."""
+    a, w, _ = operands(300, 4096, 2048)
+    for call, inner in ((lambda x, out: ops.gemm_swiglu(x, w, out), w), (lambda x, out: ops.gemm_gelu(x, w[:2048], out, product=torch.empty_like(out)), w)):
+        for shift in (0, 64 * 2048):                    # all of it, and rows that overlap by all but 64
+            held = torch.empty(300 * 2048 + shift, dtype=torch.bfloat16, device=DEV)
+            x, out = held[:300 * 2048].view(300, 2048).copy_(a), held[shift:].view(300, 2048)
+            assert not ops.ring_fits(x, inner, out) and ops.ring_fits(a, inner, torch.empty_like(a))
+            want = call(a, torch.empty_like(a)).double()
+            got = call(x, out).double()
+            # (sums in another order, rounded to bf16 twice: gate and up, and the result)
+            assert (got - want).norm() <= 2.0 ** -7 * want.norm() and (got - want).abs().max() <= 2.0 ** -5 * want.abs().max()
+    beside = torch.empty(300, 4096, dtype=torch.bfloat16, device=DEV)
+    assert not ops.ring_fits(beside[:, :2048], w, beside[:, 2048:])         # (columns of the same rows: told apart no further)
+
+
 @pytest.mark.parametrize("odd", ["cos", "sin", "q", "keys"])
 @pytest.mark.parametrize("M", [64, 200])
 def test_rotation_with_operands_between_words(ops, M, odd):
