@@ -344,8 +344,9 @@ class PostNormBlock(Part):
         """x <- norm(alpha x + gate * result) in place; returns the new rows in the activations' type."""
         if isinstance(result, ops.Biased):
             result = ops.bias_add(result.rows, result.bias)
-        if isinstance(result, ops.Partials):
-            raise TypeError("a sublayer of this arrangement gives finished rows (or weighted rows), no partial sums")
+        if isinstance(result, ops.Partials):      # (products cut along their inner size, of few rows or many: added before the gate)
+            rows = ctx.buffer(f"post.rows{which}", x.shape, torch.float32).zero_()
+            result = ops.add_partials(rows, (result.parts, result.slices))
         gate = bias = None
         if which in self.gates:
             weight, bias = self.gates[which]

@@ -186,3 +186,36 @@ def test_stored_32bit_matrix_runs_in_bf16_by_rounding(tmp_path, folders):
     assert torch.equal(m16.layers[0].ffn.w_down.cpu(), tensors[name].to(torch.bfloat16))
     assert m16.layers[0].ffn_norm.weight.dtype == torch.float32
     assert torch.equal(m16.layers[0].ffn_norm.weight.cpu(), tensors["model.layers.0.post_attention_layernorm.weight"])
+
+
+@pytest.mark.parametrize("rows, inner", [(6, 8192), (300, 8192)])
+def test_the_norm_after_a_sum_of_a_product_left_in_slices(folders, rows, inner, monkeypatch, no_gemv):
+    """A block that norms after the sum takes a mixer whose product is cut along its inner size, of few rows (the wide kernel) or many
+    (the ring product): the same rows, within the order of the sums, as with the product finished by the mixer."""
+    from runtime.engine import load_model, ModelRunner, StepEntry
+    from runtime.kernels import ops
+    from runtime.parts import RMSNorm, Mixer
+    from runtime.parts.block import PostNormBlock
+    for limit in ("WIDE_MIN_BYTES", "WIDE_MIN_BYTES_FEW_ROWS", "WIDE_MIN_BYTES_MANY_ROWS"):
+        monkeypatch.setattr(ops, limit, 0)
+    runner = ModelRunner(load_model(folders["a"], dtype="bfloat16"), n_pages=64, page_size=16)
+    runner.create("u")
+    ctx = runner._context([StepEntry("u", [1] * 6, [])], runner.cache.append_many([("u", 6)]))
+    torch.manual_seed(rows)
+    hidden = 1024
+    a, w = torch.randn(rows, inner, device=DEV).bfloat16(), (torch.randn(hidden, inner, device=DEV) * 0.02).bfloat16()
+    left = []
+
+    class Product(Mixer):
+        def output(self, h, ctx, site):
+            left.append(ctx.product_for_norm(a, w, "t.y") if self.cut else ops.gemm(a, w, torch.empty(rows, hidden, device=DEV)))
+            return left[-1]
+
+    mixer, norm = Product(), RMSNorm("n", hidden, 1e-5)
+    norm.weight = 1 + 0.1 * torch.randn(hidden, device=DEV)
+    block = PostNormBlock("b", hidden, norm, mixer, alpha=1.5)
+    start, results = torch.randn(rows, hidden, device=DEV), []
+    for mixer.cut in (False, True):
+        results.append(block.forward(start.clone(), ctx, 0).clone())
+    assert isinstance(left[1], ops.Partials) and left[1].slices > 1, "this product was meant to be cut into slices"
+    torch.testing.assert_close(results[1], results[0], rtol=1e-4, atol=1e-4)
