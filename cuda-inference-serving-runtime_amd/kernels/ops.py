@@ -253,7 +253,9 @@ def add_partials(x, partials):
 
 
 def rmsnorm_partials(x, partials, weight, out, eps):
-    """x += what gemm_unfinished left (in place), out = rmsnorm(x) * weight: one kernel."""
+    """x += what gemm_unfinished left (in place), out = rmsnorm(x) * weight: one kernel (a weight that does not lie on 16 bytes: two)."""
+    if weight.data_ptr() % 16:
+        return rmsnorm(add_partials(x, partials), weight, out, eps)
     parts, slices = _sums_of(partials, x)
     rows, dim = x.shape
     if not partials_ok(x) or out.data_ptr() % 16:
@@ -1574,7 +1576,10 @@ def layernorm(x, weight, out, eps, rows=None, bias=None):
 
 
 def layernorm_partials(x, partials, weight, out, eps, bias=None):
-    """x += what gemm_unfinished left (in place), out = layernorm(x) * weight (+ bias): one kernel."""
+    """x += what gemm_unfinished left (in place), out = layernorm(x) * weight (+ bias): one kernel (a weight or bias that does not lie
+    on 16 bytes: two)."""
+    if weight.data_ptr() % 16 or (bias is not None and bias.data_ptr() % 16):
+        return layernorm(add_partials(x, partials), weight, out, eps, bias=bias)
     parts, slices = _sums_of(partials, x)
     rows, dim = x.shape
     if not partials_ok(x) or out.data_ptr() % 16:

@@ -101,6 +101,25 @@ def test_norm_of_sums_over_the_widths(ops, dim):
     assert torch.equal(x, want) and torch.equal(got, ops.rmsnorm(want, weight, torch.empty(M, dim, device=DEV), 1e-5))
 
 
+def test_norm_of_sums_with_weights_between_words(ops):
+    """Norm weights that are views into one buffer, as a program may bind them: the sum and the norm, as two kernels."""
+    M, N, K = 300, 260, 8192
+    a, w, r = operands(M, N, K)
+    held = torch.randn(2 * N + 2, device=DEV)
+    weight, bias = held[1:1 + N], held[1 + N:1 + 2 * N]
+    parts = torch.empty(2 * M * N, device=DEV)
+    ops.gemm_ring_partials(a, w, parts, 2)
+    product = (a.float() @ w.float().T).bfloat16()
+    for left in ((ops.RingSums(parts, 2, M, N), 0), (parts, 2), (product, 0)):
+        alone = ops.add_partials(r.clone(), left)
+        for norm, alone_norm in ((lambda x, out: ops.rmsnorm_partials(x, left, weight, out, 1e-5), lambda x, out: ops.rmsnorm(x, weight, out, 1e-5)),
+                                 (lambda x, out: ops.layernorm_partials(x, left, weight, out, 1e-5, bias=bias),
+                                  lambda x, out: ops.layernorm(x, weight, out, 1e-5, bias=bias))):
+            x = r.clone()
+            got = norm(x, torch.empty(M, N, dtype=torch.bfloat16, device=DEV))
+            assert torch.equal(x, alone) and torch.equal(got, alone_norm(alone, torch.empty_like(got)))
+
+
 def test_what_is_not_taken(ops):
     a, w, r = operands(70, 64, 128)
     for bad in ((a[:, :96], w[:, :96], r), (a, w[:62], r[:, :62]), (a[:, 1:65], w[:, :64], r), (a.float(), w.float(), r),
