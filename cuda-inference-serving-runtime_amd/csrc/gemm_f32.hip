@@ -261,25 +261,44 @@ static int launch_f32(GemmF32Args p, hipStream_t stream) {
 // The tile (sixteens of rows x sixteens of W's rows): the smallest that needs no more blocks than there are compute units, as a block alone
 // on its unit takes the longer the larger its tile, and a second round costs more.  192 rows, us of the tile before / now: 576 x 576 2 x 2
 // (108 blocks) 8.2 / 1 x 2 (216) 6.4, 576 x 1,536 15.2 / 1 x 2 11.3, 960 x 576 8.7 / 2 x 2 with two sixteens in flight instead of four 7.9,
-// 3,072 x 576 gated 2 x 2 (576) 18.1 / 3 x 4 (192) 15.8; 2,048 x 2,048 33 / 3 x 2 24; 512 x 576, K 1,536 26.6 / 3 x 2 18.9.  Beyond one round
-// the others: 512 x 3,072, K 576 2 x 2 29.8, 2 x 4 31.4; K 2,048 512 x 8,192 2 x 4 207, 4 x 2 210, 192 x 8,192 2 x 4 90, 4 x 2 84.5.  Up to 16
-// rows the tile has 16 of them.  A tile never changes a sum: its order is K's.  (Rows that are not aligned: two tiles only.)
+// 3,072 x 576 gated 2 x 2 (576) 18.1 / 3 x 4 (192) 15.8; 2,048 x 2,048 33 / 3 x 2 24; 512 x 576, K 1,536 26.6 / 3 x 2 18.9.  (3 x 4 only where
+// 2 x 2 would be more than 512, 4 x 4 where it would be more than 800: 90 x 4,608 x 768 gated, 432 of them, 18.2 / 17.0; 256 x 3,072 x 576, 768,
+// 20.2 / 18.0; 1,024 x 960, 960, 19.6 / 20.8.)
+// Beyond one round, K below 1,024: 2 x 4 has two blocks a unit and is ahead where these are many (1,024 x 3,072 x 576, 1,536 of them, 49.5, with 2 x 2
+// 52.5; 2,048 x 2,048 x 1,000 105 / 110) or fill their last round of 512 well (4,096 x 512 x 512, 1,024, 31.2 / 33.3; 1,800 x 1,000 x 1,000, 912, 56.4 / 60.7;
+// 1,300 rows, 656, 43.8 / 46.3), 2 x 2 else (384 x 3,072 x 576, 576, 28.3 / 25.0; 700 rows, 1,056, 40.6 / 39.7; K 512 to 960 up to half a round:
+// 1,024 x 1,536 x 576, 768, 31.5 / 29.1).  K from 1,024 on: 4 x 2 for up to 256 rows that fill it (192 x 8,192 x 2,048 84.5, 2 x 4 90; 130 x 6,144 x 1,024
+// 43.8, 2 x 2 37.8); else 2 x 2 with four sixteens in flight up to 400 blocks of 2 x 4 (300 x 2,048 x 2,048 48.6, 2 x 4 55.2, K 8,192
+// 148 / 195), then 2 x 4 (1,500 x 576 x 1,536, 423 blocks, 44.2, 2 x 2 55.2; 512 x 8,192 x 2,048 207, 4 x 2 210).
+// Rows that are not aligned load word by word: three tiles, 2 x 4 from 512 of them on (512 x 3,072 x 577 58.4, 2 x 2 69.9; 1,024 x 8,192 x 1,030 572 / 658).
+// Up to 16 rows the tile has 16 of them.  A tile never changes a sum: its order is K's.
 template <int WK, bool VEC, int FORM>
 static int launch_f32_tile(const GemmF32Args& p, hipStream_t stream) {
     const int cols = FORM == F32_PLAIN ? p.N : 2 * p.N;
-    auto one_round = [&](int tm, int tn) { return (long long)((p.M + 16 * tm - 1) / (16 * tm)) * ((cols + 16 * tn - 1) / (16 * tn)) <= 256; };
+    auto blocks = [&](int tm, int tn) { return (long long)((p.M + 16 * tm - 1) / (16 * tm)) * ((cols + 16 * tn - 1) / (16 * tn)); };
+    auto one_round = [&](int tm, int tn) { return blocks(tm, tn) <= 256; };
     constexpr int DEEP = WK == 16 ? 8 : 4;               // sixteens in flight where a wave has few operands each
+    const long long wide = blocks(2, 4);
     if (p.M <= 16 || one_round(1, 1)) return launch_f32<1, 1, WK, DEEP, VEC, FORM>(p, stream);
-    if constexpr (VEC) {
+    if constexpr (!VEC) {
+        if (wide >= 512) return launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+        if constexpr (WK == 16)                           // (192 x 2,048 x 4,099 152 us with two sixteens in flight, 146 with four)
+            if (p.K >= 2048 && blocks(2, 2) >= 128) return launch_f32<2, 2, WK, 4, VEC, FORM>(p, stream);
+    } else {
         if (one_round(1, 2)) return launch_f32<1, 2, WK, 4, VEC, FORM>(p, stream);
         if (one_round(2, 2)) return launch_f32<2, 2, WK, 2, VEC, FORM>(p, stream);
         if (one_round(3, 2)) return launch_f32<3, 2, WK, 2, VEC, FORM>(p, stream);
         if (one_round(4, 2)) return launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream);
         if constexpr (WK == 8 && FORM != F32_PLAIN) {    // (a wave finishes at most one sixteen by sixteen of columns)
-            if (one_round(3, 4)) return launch_f32<3, 4, WK, 2, VEC, FORM>(p, stream);
-            if (one_round(4, 4)) return launch_f32<4, 4, WK, 2, VEC, FORM>(p, stream);
+            if (one_round(3, 4) && blocks(2, 2) > 512) return launch_f32<3, 4, WK, 2, VEC, FORM>(p, stream);
+            if (one_round(4, 4) && blocks(2, 2) > 800) return launch_f32<4, 4, WK, 2, VEC, FORM>(p, stream);
         }
-        if constexpr (WK == 16) return p.M <= 256 ? launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream) : launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+        if constexpr (WK == 16) {
+            if (p.M <= 256 && wide > 400 && blocks(4, 2) <= wide) return launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream);
+            return wide <= 400 ? launch_f32<2, 2, WK, 4, VEC, FORM>(p, stream) : launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+        }
+        const int over = (int)(wide % 512), most = p.K >= 512 && p.K <= 960 ? 256 : 128;
+        if (wide >= 1200 || (wide >= 512 && (over == 0 || over > most))) return launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
     }
     return launch_f32<2, 2, WK, 2, VEC, FORM>(p, stream);
 }
