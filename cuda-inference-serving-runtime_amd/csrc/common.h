@@ -76,18 +76,21 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 struct GateLaw { float limit, slope, shift; };
 
 // g sigmoid(z) where it goes on to bf16.  exp(-z) = 2^t exp(rho) with t = -z / ln 2 rounded and rho what the rounding left, in two
-// pieces of ln 2; then the quotient from the approximate reciprocal and one correction.  Relative error at most 2.1e-7 (g / (1 + expf(-z)):
-// 1.9e-7); over 2^24 products silu(g) u of normal g (0.3 to 10 wide) and u the error of the bf16 results against 64 bits is the same in all
-// ten digits.  Beyond |z| = 88 the sigmoid is 0 or 1; the maximum keeps g = inf from inf - inf.  As the epilogue of a product
-// nothing runs beside it: with this, and the law asked for once a row, the gated ring product takes 12.9 us for 14.8 at 1,777 x 3,072, K 576,
-// 74.5 for 78.2 at 1,061 x 16,384, K 2,048, 155 for 165 at 2,345 rows, 202 for 213 at 907 x 28,672, K 4,096.
+// pieces of ln 2; then the quotient from the approximate reciprocal and one correction, both of a quarter of the divisor, as the
+// reciprocal of 1 + exp(87.4) and beyond is below the smallest normal number.  Relative error at most 2.1e-7 (g / (1 + expf(-z)):
+// 1.9e-7) down to z = -88.72; below, where the exponential is past the largest float, the sigmoid is 0 as there.  Over 2^24 products silu(g) u of
+// normal g (0.3 to 30 wide) and u the error of the bf16 results against 64 bits is the same in all ten digits.  The maximum keeps g = inf from
+// inf - inf.  As the epilogue of a product nothing runs beside it: with this, and the law asked for once a row, the gated ring product
+// takes 13.2 us for 14.8 at 1,777 x 3,072, K 576 (13.0 without the quarter, whose results between z = -87.34 and -88.72 were 0),
+// 74.5 for 78.2 at 1,061 x 16,384, K 2,048, 155 for 165 at 2,345 rows, 203 for 213 at 907 x 28,672, K 4,096.
 __device__ __forceinline__ float times_sigmoid_to_bf16(float g, float z) {
-    z = __builtin_amdgcn_fmed3f(z, -88.f, 88.f);
-    const float t = z * -1.44269502f, rho = fmaf(t, 1.90465432e-9f, fmaf(t, -0.693147182f, -z));
+    const float c = __builtin_amdgcn_fmed3f(z, -88.7228f, 88.f);
+    const float t = c * -1.44269502f, rho = fmaf(t, 1.90465432e-9f, fmaf(t, -0.693147182f, -c));
     float e = __builtin_amdgcn_exp2f(t);
     e = fmaf(e, rho, e);
-    const float d = 1.0f + e, r = __builtin_amdgcn_rcpf(d), q = g * r;
-    return fmaf(fmaxf(fmaf(-d, q, g), -3.0e38f), r, q);
+    const float d = fmaf(e, 0.25f, 0.25f), h = 0.25f * g;
+    const float r = z < -88.7228f ? 0.f : __builtin_amdgcn_rcpf(d), q = h * r;
+    return fmaf(fmaxf(fmaf(-d, q, h), -3.0e38f), r, q);
 }
 
 template <typename TC>
@@ -121,9 +124,10 @@ __device__ __forceinline__ float unary_activation(float z, int act) {
 }
 
 // The gelu with the error function where the result is rounded to bf16: z / 2 erfc(-z / sqrt 2), with erfc(x) = t 2^(p(t) - x^2 / ln 2),
-// t = 1 / (1 + x / 2), for x >= 0 and 2 - erfc(|x|) below; p is a polynomial fitted here (Chebyshev nodes, t from 1/8 to 1) to
-// log2(e^(x^2) erfc(x) / t).  Relative error of erfc 4e-6, also where it is small, where 1 + erf(z) has lost its digits.  A sixth of
-// erff's instructions: as the epilogue of 1,999 x 8,192, K 2,048 the activation took 30 us of 86.
+// t = 1 / (1 + x / 2), for x >= 0 and 2 - erfc(|x|) below, the form of W. H. Press et al., Numerical Recipes; p is a polynomial fitted here
+// (Chebyshev nodes, t from 1/8 to 1) to log2(e^(x^2) erfc(x) / t).  Relative error of erfc(-z / sqrt 2) in 32 bits: 6e-7 for z > -1, 1.4e-6 to
+// -5, 4.5e-6 to -8, 1.4e-5 to -13.2 (x^2 / ln 2 is rounded where it is large); 1 + erff(z / sqrt 2) has 1.4e-7 for z > -1, 7e-6 to -3,
+// 4e-2 to -5 and no digit beyond.  A sixth of erff's instructions: as the epilogue of 1,999 x 8,192, K 2,048 the activation took 30 us of 86.
 __device__ __forceinline__ float gelu_to_bf16(float z) {
     const float x = fabsf(z) * 0.70710678118654752f, t = __builtin_amdgcn_rcpf(fmaf(0.5f, x, 1.0f));
     float p = 0.0669854358f;

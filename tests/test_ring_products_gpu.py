@@ -252,7 +252,7 @@ def test_on_every_replay_of_a_captured_graph(ops):
 
 def test_gelu_of_every_bf16_number(ops):
     """The gelu of bf16 results against 64 bits over all bf16 numbers from 2^-20 to 16 and their negatives: rounded to the nearest
-    bf16 but for sums near a tie (the kernel's 4e-6 relative against a rounding of 2^-9: fewer than one in a hundred), never
+    bf16 but for sums near a tie (the kernel's 1.4e-5 relative at most against a rounding of 2^-9: fewer than one in a hundred), never
     further than the next one."""
     bits = torch.arange(0x3580, 0x4181, dtype=torch.int32)
     z = torch.cat([bits, bits | 0x8000]).to(torch.int16).view(torch.bfloat16).to(DEV)
@@ -365,7 +365,7 @@ def test_gates_of_every_size_against_64_bits(law):
         a[m, m % k] = 1.0
     g = torch.randn(k, inter, device="cuda:0") * torch.logspace(-3, 1.7, k, device="cuda:0")[:, None]
     g[0, :12] = torch.tensor([0.0, -0.0, 1e-30, -1e-30, 1e-4, -1e-4, 80.0, -80.0, 1000.0, -1000.0, 1e30, -1e30], device="cuda:0")
-    g[1, :6] = torch.tensor([-86.0, -87.5, -88.0, -89.0, 88.0, 89.0], device="cuda:0")
+    g[1, :7] = torch.tensor([-86.0, -87.5, -88.0, -88.5, -89.0, 88.0, 89.0], device="cuda:0")
     g[63] = torch.where(torch.arange(inter, device="cuda:0") % 2 == 0, 3e38, -3e38)
     u = torch.randn(k, inter, device="cuda:0")
     w = torch.cat((g.t(), u.t())).bfloat16().contiguous()
@@ -384,5 +384,8 @@ def test_gates_of_every_size_against_64_bits(law):
     want, got = gate * torch.sigmoid(z) * up, out.double()
     dull = want.isnan() | want.isinf()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
-    bound = want.abs() * (2.0 ** -8 + 4e-6 + 2.0 ** -22 * z.abs().clamp(max=88.0)) + 1e-35
+    # (where exp(-z) is past the largest float the sigmoid is 0; results below the smallest normal number may be)
+    bound = want.abs() * (2.0 ** -8 + 4e-6 + 2.0 ** -22 * z.abs().clamp(max=88.0) + (z < -88.72).double()) + 2.0 ** -126
     assert ((got - want).abs() <= bound)[~dull].all()
+    near = (z < -87.0) & (z > -88.72)
+    assert law is not None or (near.any() and (got[near] != 0).all())
