@@ -19,7 +19,7 @@ struct RingArgs {
     bf16_t* kcache; bf16_t* vcache; int heads, kv_heads, dim, page_size, max_pos;
 };
 
-// one function per unit; false: the unit does not hold this tile
+// one function per unit: 0 or a HIP error; hipErrorInvalidValue: the unit does not hold this tile (nothing is launched)
 int cisr_ring_launch_a(const RingArgs& a, int tile, int mode, hipStream_t stream);
 int cisr_ring_launch_b(const RingArgs& a, int tile, int mode, hipStream_t stream);
 int cisr_ring_launch_c(const RingArgs& a, int tile, int mode, hipStream_t stream);
