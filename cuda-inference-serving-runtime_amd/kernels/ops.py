@@ -577,7 +577,7 @@ class ScratchPool:
     sum into the residual, the wide kernel's partial sums, the slice winners of the argmax.  A buffer is handed out
     again to every later call that it is large enough for, and none is freed before `clear`: captured programs keep
     the addresses.  A step function owns one pool (calls on its stream are ordered, so they can share buffers);
-    calls that name no pool share DEFAULT_SCRATCH.  `ring`: whether the products of its steps may be ring products
+    calls that name no pool share DEFAULT_SCRATCH, but for the partial sums of a ring product.  `ring`: whether the products of its steps may be ring products
     (csrc/gemm_ring.inc); a model that sends rows to experts takes none (see Model.routes)."""
 
     def __init__(self, ring=True):
@@ -702,6 +702,14 @@ class RingSums:
         self.parts, self.slices, self.rows, self.cols = parts, int(slices), int(rows), int(cols)
 
 
+def _ring_workspace(scratch, device, floats):
+    """Floats for the partial sums of a ring product: the pool's, or without one this call's own.  (Most products that are cut here
+    ran in a kernel that needs no memory before, so callers on several streams that name no pool must not meet in one buffer.)"""
+    if scratch is None:
+        return torch.empty(floats, dtype=torch.float32, device=device)
+    return _wide_workspace(scratch, device, floats)
+
+
 def _ring_sums(at, m, n, k, make_buffer):
     """The RingSums of a product whose operands are `at` in floats of the caller's (`make_buffer(floats)`), or None where it is best
     not cut."""
@@ -804,7 +812,7 @@ def gemm(a, w, out, residual=None, after_norm=False, scratch=None):
     elif (a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w, fused=residual is not None, floats=out.dtype == torch.float32, cut=residual is not None)
           and (at := _ring_operands(a, w, out)) is not None and (residual is None or (ldr % 4 == 0 and rp % 16 == 0))):
         if residual is not None and residual is out and partials_ok(out):
-            sums = _ring_sums(at, m, n, k, lambda floats: _wide_workspace(scratch, a.device, floats))
+            sums = _ring_sums(at, m, n, k, lambda floats: _ring_workspace(scratch, a.device, floats))
             if sums is not None:
                 return add_partials(out, (sums, 0))
         code = lib().cisr_gemm_ring_bf16(*at, rp, ldr, m, n, k, _storage(out, "out"), 0, 0, _stream())
@@ -951,7 +959,7 @@ def gemm_unfinished(a, w, residual, scratch=None, finish=False):
             or not partials_ok(residual)):
         return None
     if _ring_open(scratch) and ring_ahead(m, w, fused=True, cut=True) and (at := _ring_operands(a, w, residual)) is not None:
-        sums = _ring_sums(at, m, n, k, lambda floats: _wide_workspace(scratch, a.device, floats))
+        sums = _ring_sums(at, m, n, k, lambda floats: _ring_workspace(scratch, a.device, floats))
         if sums is None:                    # (not cut: added in the product's epilogue)
             if not finish:
                 return None

@@ -91,6 +91,24 @@ def test_slices_and_the_norm_that_adds_them(ops, tile, slices):
         ops.add_partials(torch.zeros(M, N + 4, device=DEV), left)
 
 
+def test_sums_of_calls_without_a_pool_lie_apart(ops, monkeypatch):
+    """Two products that are cut, neither of them added yet, as callers on two streams have them that name no pool: each holds its own
+    partial sums, and none lie in the buffers that such calls share."""
+    M, N, K = 2000, 448, 8192
+    a, w, r = operands(M, N, K)
+    b = a.flip(0).contiguous()
+    monkeypatch.setattr(ops, "DEFAULT_SCRATCH", ops.ScratchPool())
+    left = [ops.gemm_unfinished(x, w, r) for x in (a, b)]
+    x = r.clone()
+    ops.gemm(a, w, x, residual=x)
+    assert not any(kind == "wide" for kind, _, _ in ops.DEFAULT_SCRATCH.buffers)
+    assert all(isinstance(sums, ops.RingSums) and sums.slices > 1 for sums, _ in left)
+    got = [ops.add_partials(torch.zeros_like(r), part) for part in left]
+    for rows, out in zip((a, b), got):
+        assert close(out, rows.double() @ w.double().T, K)
+    assert torch.equal(x, ops.add_partials(r.clone(), left[0]))
+
+
 @pytest.mark.parametrize("dim", [4, 576, 1028, 8192])
 def test_norm_of_sums_over_the_widths(ops, dim):
     M, slices = 5, 4
