@@ -626,6 +626,7 @@ RING_MIN_OUTPUTS, RING_MIN_OUTPUTS_K = 500_000, 40
 RING_MIN_OUTPUTS_SHORT, RING_SHORT_K = 250_000, 1024
 RING_PLAIN_FLOPS, RING_PLAIN_COLS = 15e9, 2048
 RING_MOST_FLOPS, RING_GATED_FLOPS, RING_ROPE_FLOPS = 300e9, 210e9, 95e9
+RING_GATED_LONG_K, RING_GATED_LONG_FLOPS = 4096, 175e9
 # Of 17 to 64 rows the products of large weights, in bytes (by kind: see ring_ahead); the smaller ones only from more than 32 rows on.
 RING_FEW_ROWS, RING_HALF_ROWS = 17, 33
 RING_FEW_GATED, RING_HALF_GATED = 64 << 20, 16 << 20
@@ -637,16 +638,20 @@ def _ring_open(scratch):
     return scratch is None or scratch.ring
 
 
-def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
+def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False, library_rows=True):
     """Whether the ring product is the fastest for m rows against the bf16 weights w ([N, K]; `gated`: gate and up).  `fused`: a kernel
     after the library's product (activation, residual sum) is an epilogue here; `floats`: float results; `cut`: the inner size
-    may be cut.  Measured on an MI355X over 65 to 4,096 rows of the sizes of all designs, us of the other kernels / this one:
+    may be cut; `library_rows`: whether the rows are such as the library is given.  Measured on an MI355X over 65 to 4,096 rows of the sizes of all designs, us of the other kernels / this one:
       few outputs stay with the kernels of small tiles: 300 x 960, K 576 5.0 / 5.3, 600 x 960 6.2 / 5.6; 256 x 2,048, K 8,192 28 / 35, 400 rows
       37 / 33 (the library cuts the inner size); with a short one against the library from half as many on: 256 x 1,024, K 1,024 8.0 / 6.4;
       what is added to a residual is cut here too, and beats the library at any number of rows: 65 x 2,048, K 8,192 22.7 / 15.5, 1,061 rows
       66 / 50, 2,048 rows 82 / 70;
-      gate and up with their activation: 128 x 16,384, K 2,048 25.8 / 20.2, 1,061 rows 83 / 66, 2,345 rows 177 / 153, 907 x 28,672,
-      K 4,096 (213 GFLOP) 192 / 213, 2,048 rows 377 / 409 (with the present form of the activation this one takes 3 to 6 % less: 907 rows 202);
+      gate and up with their activation, K 2,048: 128 x 16,384 25.8 / 20.2, 1,061 rows 83 / 66, 2,345 rows 181 / 144, 3,072 rows (206 GFLOP)
+      173 / 170, 4,096 rows 227 / 225; K 4,096 and more: 576 x 28,672 (135 GFLOP) 147 / 115, 640 rows 149 / 142, 720 rows (169) 164 / 182, 750 rows
+      164 / 183, 850 rows 188 / 198, 907 rows 195 / 209, 1,777 rows 420 / 386, 2,048 rows 377 / 413; 1,100 x 16,384 (148) 146 / 115, 1,200 rows 150 / 142,
+      1,400 rows (188) 170 / 171, 1,500 rows 170 / 179; 1,000 x 22,016 (180) 176 / 176, 1,100 rows 187 / 194; 600 x 27,648, K 5,120 (170) 186 / 174, 700 rows
+      198 / 229; 450 x 36,864 (170) 187 / 185, 500 rows 198 / 231.  (Each side jumps where its tiles need another round, so that single sizes on
+      either side of the line lie up to 10 % wrong, 192 and 256 x 36,864 23 %.)
       a product that ends with its store: 1,000 x 4,096, K 1,024 13.8 / 13.3, 2,000 rows (17 GFLOP) 21 / 22, 4,000 rows 29 / 35; 2,345 x 2,048, K 2,048
       29 / 24; float results 2,000 x 8,512, K 2,048 81 / 63, 4,000 rows 138 / 128;
       17 to 64 rows, where a block streams its rows of W alone: gate and up 18 x 16,384, K 2,048 18.3 / 14.4, 64 rows 20.8 / 15.8, 64 x
@@ -663,6 +668,8 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False):
             return size >= ((RING_HALF_GATED if half else RING_FEW_GATED) if gated else RING_FEW_CUT)
         return size >= RING_FEW_PLAIN and (half or size <= RING_FEW_PLAIN_MOST)
     if m < RING_MIN_ROWS or w.dtype != torch.bfloat16 or flops > (RING_GATED_FLOPS if gated else RING_MOST_FLOPS):
+        return False
+    if gated and k >= RING_GATED_LONG_K and flops > RING_GATED_LONG_FLOPS and library_rows and library_ok(m, w, gated=True):
         return False
     many = outputs >= RING_MIN_OUTPUTS + RING_MIN_OUTPUTS_K * k
     beats_library = gated or cut or fused or floats or flops <= RING_PLAIN_FLOPS or cols <= RING_PLAIN_COLS
@@ -1053,7 +1060,7 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         return out
     if out.dtype != a.dtype or a.dtype != w_gate_up.dtype:
         raise KernelError("gemm_swiglu: dtypes differ")
-    if a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w_gate_up, gated=True) and (at := _ring_operands(a, w_gate_up, out)) is not None:
+    if a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w_gate_up, gated=True, library_rows=a.is_contiguous()) and (at := _ring_operands(a, w_gate_up, out)) is not None:
         return _ring_gated(at, m, inter, k, out, law)
     activate = swiglu if law is None else (lambda gu, o: glu_clamped(gu, o, *law))
     if a.dtype == torch.bfloat16 and library_ok(m, w_gate_up, gated=True) and a.is_contiguous():

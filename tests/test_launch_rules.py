@@ -2,6 +2,7 @@
 measurements settled them (profiles/prompt_attention_forms_and_the_rule_that_picks.txt and
 profiles/decode_attention_launch_shapes_and_the_rule_that_picks.txt), so that a change of a rule shows."""
 import pytest
+import torch
 
 from runtime.kernels.attention import fused_merge_splits, prompt_form, rows_launch, rows_stream_loads
 
@@ -79,3 +80,26 @@ def test_decode_attention_streams_keys_and_values_at_measured_points(blocks, key
 def test_splits_that_the_output_projection_merges_itself(splits, rows, fused):
     assert fused_merge_splits(splits, rows, lambda n: True) == fused
     assert fused_merge_splits(splits, rows, lambda n: False) is None
+
+
+@pytest.mark.parametrize("rows, columns, k, ring", [
+    (3100, 16384, 2048, True),         # 208 GFLOP with a short inner size: ahead of the library by up to 25 %
+    (4096, 16384, 2048, False),
+    (640, 28672, 4096, True),
+    (777, 28672, 4096, False),         # 183 GFLOP with a long one: the library by 4 to 15 %
+    (907, 28672, 4096, False),
+    (1500, 16384, 4096, False),
+    (500, 36864, 5120, False),
+])
+def test_ring_product_of_gate_and_up_at_measured_points(rows, columns, k, ring):
+    from runtime.kernels import ops
+    w = torch.empty(columns, k, dtype=torch.bfloat16, device="meta")
+    assert ops.ring_ahead(rows, w, gated=True) is ring
+
+
+def test_ring_product_of_gate_and_up_where_the_library_takes_no_operands():
+    """Rows or weights that are views: the other side is not the library, and the product stays here."""
+    from runtime.kernels import ops
+    w = torch.empty(28672, 4224, dtype=torch.bfloat16, device="meta")
+    assert ops.ring_ahead(777, w[:, :4096], gated=True)
+    assert ops.ring_ahead(777, w[:, :4096].contiguous(), gated=True, library_rows=False)
