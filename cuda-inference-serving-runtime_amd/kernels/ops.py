@@ -627,6 +627,7 @@ RING_MIN_OUTPUTS_SHORT, RING_SHORT_K = 250_000, 1024
 RING_PLAIN_FLOPS, RING_PLAIN_COLS = 15e9, 2048
 RING_MOST_FLOPS, RING_GATED_FLOPS, RING_ROPE_FLOPS = 300e9, 210e9, 95e9
 RING_GATED_LONG_K, RING_GATED_LONG_FLOPS = 4096, 175e9
+RING_GELU_OUTPUTS, RING_RELU2_OUTPUTS = 10.5e6, 24e6
 # Of 17 to 64 rows the products of large weights, in bytes (by kind: see ring_ahead); the smaller ones only from more than 32 rows on.
 RING_FEW_ROWS, RING_HALF_ROWS = 17, 33
 RING_FEW_GATED, RING_HALF_GATED = 64 << 20, 16 << 20
@@ -1677,6 +1678,21 @@ def heads_product(a, a_head, w, out, out_head, gate=None):
 GELU_KINDS = {"gelu": 0, "gelu_erf": 0, "gelu_tanh": 1, "relu2": 2}      # ungated activations (relu2: relu(z)^2)
 
 
+def activation_apart(a, w, out, product, kind):
+    """Whether gemm_gelu's activation is better a kernel after the library's product than the ring product's epilogue, where nothing runs
+    beside it: many results, and operands that both kernels take.  Measured on an MI355X, us as two kernels / as the epilogue; gelu
+    1,280 x 8,192, K 2,048 (10.5 M results) 52 / 51, 1,500 rows 57 / 61, 2,048 rows 67 / 74, 4,096 rows 122 / 145; 2,345 x 4,096, K 1,024 (9.6 M) 33 / 33,
+    3,000 rows 37 / 38, 4,096 rows 45 / 50; 777 x 12,288, K 3,072 (9.5 M) 66 / 65, 2,048 rows 142 / 161; 1,024 x 16,384, K 4,096 114 / 127 (the tanh
+    form the same 2 to 4 % lower); relu2, which costs less, 2,345 x 8,192 (19 M) 84 / 82, 3,000 rows (25 M) 100 / 101, 4,096 rows 121 / 133; 2,345 x 10,752,
+    K 2,688 (25 M) 127 / 134; 2,700 x 12,288 (33 M) 190 / 187.  (1,500 x 12,288, 18 M, is the one size of gelu above its line where the epilogue is
+    ahead: 131 / 126.)"""
+    (m, k), n = a.shape, w.shape[0]
+    if product is None or m * n <= (RING_RELU2_OUTPUTS if kind == "relu2" else RING_GELU_OUTPUTS):
+        return False
+    return (n > RING_PLAIN_COLS and 2.0 * m * n * k > RING_PLAIN_FLOPS and product.dtype == out.dtype == a.dtype == torch.bfloat16
+            and product.shape == out.shape and a.is_contiguous() and product.is_contiguous() and out.is_contiguous() and library_ok(m, w))
+
+
 def gemm_gelu(a, w, out, kind="gelu", scratch=None, product=None):
     """out[M, N] = gelu(a . w^T), out of the operands' dtype.  bf16 products of this repository's own kernels (few rows
     against weights that the wide kernel does not take; many rows against weights that the library does not take) apply
@@ -1689,7 +1705,8 @@ def gemm_gelu(a, w, out, kind="gelu", scratch=None, product=None):
     fused = (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and tuple(out.shape) == (m, n)
              and w.shape[1] == k and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1)
     act = 1 + GELU_KINDS[kind]
-    if fused and _ring_open(scratch) and ring_ahead(m, w, fused=True) and (at := _ring_operands(a, w, out)) is not None:
+    if (fused and _ring_open(scratch) and ring_ahead(m, w, fused=True) and not activation_apart(a, w, out, product, kind)
+            and (at := _ring_operands(a, w, out)) is not None):
         _check(lib().cisr_gemm_ring_bf16(*at, None, 0, m, n, k, BF16, act, 0, _stream()), "gemm_gelu")
         return out
     fused = fused and not library_ok(m, w)

@@ -103,3 +103,22 @@ def test_ring_product_of_gate_and_up_where_the_library_takes_no_operands():
     w = torch.empty(28672, 4224, dtype=torch.bfloat16, device="meta")
     assert ops.ring_ahead(777, w[:, :4096], gated=True)
     assert ops.ring_ahead(777, w[:, :4096].contiguous(), gated=True, library_rows=False)
+
+
+@pytest.mark.parametrize("kind, rows, columns, k, apart", [
+    ("gelu", 1280, 8192, 2048, False),
+    ("gelu", 1999, 8192, 2048, True),          # 16 M results: 67 us as two kernels, 74 with the epilogue
+    ("gelu_tanh", 4096, 4096, 1024, True),
+    ("relu2", 1999, 8192, 2048, False),
+    ("relu2", 4096, 8192, 2048, True),
+    ("gelu", 8000, 2048, 2048, False),         # a narrow product that ends with its store is the ring product's in any case
+])
+def test_activation_of_a_large_product_at_measured_points(kind, rows, columns, k, apart):
+    from runtime.kernels import ops
+    half = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device="meta")
+    a, w, out, product = half(rows, k), half(columns, k), half(rows, columns), half(rows, columns)
+    assert ops.activation_apart(a, w, out, product, kind) is apart
+    # what only the epilogue takes stays with it: no buffer, results or rows in a view
+    assert not ops.activation_apart(a, w, out, None, kind)
+    assert not ops.activation_apart(a, w, half(rows, columns + 8)[:, 8:], product, kind)
+    assert not ops.activation_apart(half(rows, k + 64)[:, 64:], w, out, product, kind)

@@ -181,6 +181,26 @@ def test_calls_that_came_to_these_kernels_against_the_others(ops, M, N, K, monke
         assert (got.double() - want.double()).abs().max().item() <= 2.0 ** -5 * max(scale, want.abs().max().item()), i
 
 
+@pytest.mark.parametrize("kind", ["gelu", "gelu_tanh", "relu2"])
+def test_activation_of_a_large_product_on_either_side_of_its_line(ops, kind):
+    """As a kernel after the library's product and as the epilogue, which results in a view and calls without a buffer keep: the product
+    rounded to bf16 either way, from sums of another order (one rounding apart), then the activation."""
+    M, N, K = 3001, 8192, 2048
+    a, w = operands(M, 8, K)[0], operands(N, 8, K, seed=1)[0] * 0.02
+    product, out, held = (torch.empty(M, n, dtype=torch.bfloat16, device=DEV) for n in (N, N, N + 8))
+    assert ops.activation_apart(a, w, out, product, kind)
+    got = ops.gemm_gelu(a, w, out, kind, product=product)
+    z = (a.float() @ w.float().T).double()
+    act = {"gelu": lambda x: x * 0.5 * torch.erfc(-x / 2 ** 0.5), "gelu_tanh": lambda x: torch.nn.functional.gelu(x, approximate="tanh"),
+           "relu2": lambda x: x.clamp(min=0).square()}[kind]
+    want = act(z)
+    # z is off by its rounding (2^-8 of it) and the sums' order (K 2^-24 of what a sum of 0.02 sqrt K passes through); slopes to 1.13, relu2 2 z
+    slope = 2 * z.abs() if kind == "relu2" else 1.13
+    bound = 2.0 ** -8 * want.abs() + (2.0 ** -8 * z.abs() + 1e-4) * (slope + 2.0 ** -8) + 1e-6
+    for result in (got, ops.gemm_gelu(a, w, held[:, 8:], kind, product=product), ops.gemm_gelu(a, w, torch.empty_like(out), kind)):
+        assert ((result.double() - want).abs() <= bound).all()
+
+
 def test_a_product_is_asked_about_once(ops, monkeypatch):
     """A step that runs kernel by kernel waits for the host: a product's operands are looked at once, whatever it ends in."""
     a, w, r = operands(300, 2048, 576)
