@@ -632,7 +632,7 @@ RING_GELU_OUTPUTS, RING_RELU2_OUTPUTS = 10.5e6, 24e6
 RING_FEW_ROWS, RING_HALF_ROWS = 17, 33
 RING_FEW_GATED, RING_HALF_GATED = 64 << 20, 16 << 20
 RING_FEW_CUT = 32 << 20
-RING_FEW_PLAIN, RING_FEW_PLAIN_MOST = 24 << 20, 64 << 20
+RING_FEW_PLAIN, RING_FEW_PLAIN_MOST, RING_FEW_FLOAT = 24 << 20, 64 << 20, 48 << 20
 
 
 def _ring_open(scratch):
@@ -658,7 +658,8 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False, library_
       17 to 64 rows, where a block streams its rows of W alone: gate and up 18 x 16,384, K 2,048 18.3 / 14.4, 64 rows 20.8 / 15.8, 64 x
       28,672, K 4,096 55 / 46, 32 x 8,192, K 1,024 6.6 / 6.7, 40 rows 8.4 / 6.9; added to a residual, the norm included, 18 x 2,048, K 8,192
       14.5 / 13.6, 64 rows 19.7 / 14.6, 64 x 4,096, K 14,336 46 / 31 (32 x 2,048, K 2,048 8.5 / 9.2); others 32 x 6,144,
-      K 2,048 10.3 / 8.9, 64 rows 16.4 / 9.3, 18 x 49,152 35 / 40, 64 rows 49 / 42, 64 x 2,048 7.6 / 9.5.  Fewer rows read W as fast elsewhere."""
+      K 2,048 10.3 / 8.9, 64 rows 16.4 / 9.3, 18 x 49,152 35 / 40, 64 rows 49 / 42, 64 x 2,048 7.6 / 9.5; float results of up to 32 rows, 17 x 8,512,
+      K 2,048 11.6 / 12.8, 32 rows 12.7 / 13.9, 24 x 10,240 12.9 / 13.4, 17 x 49,152, K 576 17.8 / 14.4.  Fewer rows read W as fast elsewhere."""
     cols, k = w.shape
     flops, outputs = 2.0 * m * cols * k, m * cols
     if m <= SKINNY_ROWS:
@@ -667,7 +668,7 @@ def ring_ahead(m, w, gated=False, fused=False, floats=False, cut=False, library_
             return False
         if gated or cut:
             return size >= ((RING_HALF_GATED if half else RING_FEW_GATED) if gated else RING_FEW_CUT)
-        return size >= RING_FEW_PLAIN and (half or size <= RING_FEW_PLAIN_MOST)
+        return size >= RING_FEW_PLAIN and (half or (size <= RING_FEW_PLAIN_MOST and (not floats or size >= RING_FEW_FLOAT)))
     if m < RING_MIN_ROWS or w.dtype != torch.bfloat16 or flops > (RING_GATED_FLOPS if gated else RING_MOST_FLOPS):
         return False
     if gated and k >= RING_GATED_LONG_K and flops > RING_GATED_LONG_FLOPS and library_rows and library_ok(m, w, gated=True):

@@ -122,3 +122,16 @@ def test_activation_of_a_large_product_at_measured_points(kind, rows, columns, k
     assert not ops.activation_apart(a, w, out, None, kind)
     assert not ops.activation_apart(a, w, half(rows, columns + 8)[:, 8:], product, kind)
     assert not ops.activation_apart(half(rows, k + 64)[:, 64:], w, out, product, kind)
+
+
+@pytest.mark.parametrize("rows, columns, k, floats, ring", [
+    (17, 8512, 2048, True, False),         # 33 MB of weights, float results: 11.6 us in the streaming kernel, 12.8 here
+    (32, 10240, 2048, True, False),
+    (33, 8512, 2048, True, True),
+    (17, 49152, 576, True, True),          # 54 MB: 17.8 / 14.4
+    (32, 6144, 2048, False, True),         # bf16 results
+])
+def test_ring_product_of_few_rows_at_measured_points(rows, columns, k, floats, ring):
+    from runtime.kernels import ops
+    w = torch.empty(columns, k, dtype=torch.bfloat16, device="meta")
+    assert ops.ring_ahead(rows, w, floats=floats) is ring
