@@ -750,7 +750,9 @@ def gemm_ring(a, w, out, residual=None, act=0, tile=0):
 def ring_rope_ok(a, w, head_dim, cos, sin=None):
     """Whether qkv_rope runs the ring product with the rotation and the cache write as its epilogue: bf16 rows, whole heads of a multiple
     of 32 coordinates, tables on 16 bytes; up to 64 rows large weights only (64 x 6,144, K 2,048 17.7 / 10.0, 18 rows 10.1 / 9.6, K 4,096 17.0 / 16.2).  us with the product and the rotation as kernels of their own / as one: 65 x 6,144, K 2,048 22.9 / 11.0, 1,061
-    rows 40.8 / 36.2, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.6; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99."""
+    rows 40.8 / 36.2, 4,096 rows 109 / 106; 1,777 x 960, K 576 13.6 / 8.6; 1,777 x 6,144, K 4,096 (89 GFLOP) 93 / 91, 2,048 rows 97 / 99,
+    4,096 rows 181 / 195; 4,096 x 5,120, K 3,072 130 / 142; 1,500 x 15,360, K 5,120 220 / 246 (single sizes above the line lie on the other side: 3,000 x 6,144,
+    K 4,096 161 / 145, 1,061 x 15,360, K 5,120 194 / 156)."""
     (m, k), n = a.shape, w.shape[0]
     many = m >= RING_MIN_ROWS if m > SKINNY_ROWS else m >= RING_FEW_ROWS and 2 * n * k >= RING_FEW_PLAIN
     if (not many or 2.0 * m * n * k > RING_ROPE_FLOPS or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not (a.is_cuda and w.is_cuda)
