@@ -37,6 +37,9 @@ struct GemmF32Args {
     const int* positions; const int* slots; const float* cos_tab; const float* sin_tab;
     float* kcache; float* vcache;
     int heads, kv_heads, dim, page_size, max_pos;
+    // NORM
+    const float* norm_w; float eps, inv_k;
+    const int* rows;                 // row m of A is row rows[m] of x; null: row m
 };
 enum { F32_PLAIN = 0, F32_GATED = 1, F32_ROTARY = 2 };
 
@@ -91,7 +94,12 @@ __device__ __forceinline__ void finish_pair(const GemmF32Args& p, int m, int n, 
     }
 }
 
-template <int TM, int TN, int WK, int DEPTH, bool VEC, int FORM = F32_PLAIN>
+#define GF_RUN 256                       // NORM: most of K that a wave may take (a word a lane)
+
+// 16-byte words of LDS: the waves' operands on their way, and then their tiles
+constexpr int gf_lds_items(int tm, int tn, int wk) { return wk * (tm * tn > tm + tn ? tm * tn : tm + tn) * WAVE; }
+
+template <int TM, int TN, int WK, int DEPTH, bool VEC, int FORM, bool NORM>
 __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
     extern __shared__ __attribute__((aligned(16))) char gf_lds[];
     constexpr bool HALVES = FORM != F32_PLAIN && TN == 1;            // the sixteen's first eight rows of W and its last
@@ -111,7 +119,10 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
     const float* a_row[TM];
     const float* w_row[TN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) a_row[i] = p.A + (size_t)min(m0 + i * 16 + lrow, p.M - 1) * p.lda;
+    for (int i = 0; i < TM; ++i) {
+        const int m = min(m0 + i * 16 + lrow, p.M - 1);
+        a_row[i] = p.A + (size_t)(NORM && FORM == F32_PLAIN && p.rows ? p.rows[m] : m) * p.lda;
+    }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int n = min(n0 + j % OT * OC + lrow % OC, p.N - 1), half = p.dim / 2;
@@ -125,6 +136,9 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = (gf_f32x4){0.f, 0.f, 0.f, 0.f};
     gf_f32x4 fa[DEPTH][TM], fw[DEPTH][TN];
+    float squares[TM];                                               // NORM: of the lane's words of its rows
+#pragma unroll
+    for (int i = 0; i < TM; ++i) squares[i] = 0.f;
     auto ask = [&](int d, int s) {
         const int k = min(s, sixteens - 1) * 16 + lk;
 #pragma unroll
@@ -132,7 +146,13 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) fa[d][i] = gf_load<VEC>(a_row[i], k, K);
     };
+    // NORM: the wave's run of the norm's weights waits in LDS (in registers beside the operands they made tiles of sixteen waves spill)
+    float* const ssq = (float*)((gf_f32x4*)gf_lds + gf_lds_items(TM, TN, WK));      // [WK][TM * 16] sums of squares
+    float* const run = ssq + WK * TM * 16 + wave * GF_RUN - first * 16;              // [WK][GF_RUN], from its first sixteen on
+    gf_f32x4 next = {0.f, 0.f, 0.f, 0.f};
     auto use = [&](int d, int s) {
+        const gf_f32x4 norm = next;
+        if constexpr (NORM) next = *(const gf_f32x4*)(run + min(s + 1, last - 1) * 16 + lk);
         if (s * 16 + 16 > K) {                                       // (uniform: K's last, partly filled sixteen)
             const int k = s * 16 + lk;
 #pragma unroll
@@ -140,6 +160,13 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
             for (int i = 0; i < TM; ++i) fa[d][i] = gf_clear_tail(fa[d][i], k, K);
         }
+        if constexpr (NORM)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const gf_f32x4 x = fa[d][i];
+                squares[i] += (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+                fa[d][i] = x * norm;
+            }
 #pragma unroll
         for (int j = 0; j < TN; ++j) put[j * WAVE] = fw[d][j];
 #pragma unroll
@@ -169,10 +196,17 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
     if (FORM == F32_ROTARY && finishes)
 #pragma unroll
         for (int e = 0; e < 4; ++e) pos[e] = p.positions[min(m + e, p.M - 1)];
+    gf_f32x4 mine;
+    if constexpr (NORM) mine = gf_load<VEC>(p.norm_w, first * 16 + 4 * lane, K);
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
         ask(d, first + d);
         __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (NORM) {
+        *(gf_f32x4*)(run + first * 16 + 4 * lane) = mine;
+        wave_order();
+        next = *(const gf_f32x4*)(run + first * 16 + lk);
     }
     if (FORM == F32_ROTARY && finishes) {
         const int half = p.dim / 2, angle = min(n, p.N - 1) % half;
@@ -200,6 +234,14 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
         if (turn + d < last) use(d, turn + d);                       // (uniform over the wave)
     // element 4 g + e of a lane's four is row 4 g + e, column r of its sixteen by sixteen
     constexpr int ITEMS = TM * TN * WAVE;
+    if constexpr (NORM)
+#pragma unroll
+        for (int ii = 0; ii < TM; ++ii) {                            // (a row's words of a sixteen are its quad's)
+            float x = squares[ii];
+            x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xb1, 0xf, 0xf, false));     // quad_perm 1, 0, 3, 2
+            x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4e, 0xf, 0xf, false));     // quad_perm 2, 3, 0, 1
+            if (lane % 4 == 0) ssq[(wave * TM + ii) * 16 + lrow] = x;
+        }
     float resid[4] = {0.f, 0.f, 0.f, 0.f};
     if (finishes && p.R && n < p.N)
 #pragma unroll
@@ -210,7 +252,20 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
         for (int jj = 0; jj < TN; ++jj) meet[(wave * TM * TN + ii * TN + jj) * WAVE + lane] = acc[ii][jj];
     __syncthreads();
-    if (!finishes || (!HALVES && n >= p.N)) return;
+    if (!finishes) return;
+    gf_f32x4 factor = {1.f, 1.f, 1.f, 1.f};
+    if constexpr (NORM) {
+        // (a row a lane, and all lanes change them, those past the last column too: four rows a lane, with the library's root and quotients, are 0.7 us)
+        float all = 0.f;
+#pragma unroll
+        for (int w = 0; w < WK; ++w) all += ssq[(w * TM + i) * 16 + r];
+        const float mean = fmaf(all, p.inv_k, p.eps), half = 0.5f * mean;
+        float f = __builtin_amdgcn_rsqf(mean);
+        if (mean < INFINITY) f = fmaf(f, fmaf(-half * f, f, 0.5f), f);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) factor[e] = __shfl(f, 4 * g + e, WAVE);
+    }
+    if (!HALVES && n >= p.N) return;
     auto total = [&](int tile) {
         gf_f32x4 part[WK];
 #pragma unroll
@@ -221,7 +276,8 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
             for (int w = 0; w < half; ++w) part[w] += part[w + half];
         return part[0];
     };
-    const gf_f32x4 sum = total(i * TN + j);
+    gf_f32x4 sum = total(i * TN + j);
+    if constexpr (NORM) sum *= factor;
     if constexpr (FORM == F32_PLAIN) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -232,7 +288,7 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) second[e] = __shfl_xor(sum[e], 8, WAVE);
         } else {
-            second = total(i * TN + OT + j);
+            second = total(i * TN + OT + j) * factor;
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -243,18 +299,18 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
     }
 }
 
-template <int TM, int TN, int WK, int DEPTH, bool VEC, int FORM = F32_PLAIN>
+template <int TM, int TN, int WK, int DEPTH, bool VEC, int FORM, bool NORM>
 static int launch_f32(GemmF32Args p, hipStream_t stream) {
     constexpr int COLUMNS = FORM == F32_PLAIN ? 16 * TN : 8 * TN;
     p.m_tiles = (p.M + 16 * TM - 1) / (16 * TM);
     const long long blocks = (long long)p.m_tiles * ((p.N + COLUMNS - 1) / COLUMNS);
     if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
-    constexpr int lds = WK * (TM * TN > TM + TN ? TM * TN : TM + TN) * WAVE * (int)sizeof(gf_f32x4);
+    constexpr int lds = gf_lds_items(TM, TN, WK) * (int)sizeof(gf_f32x4) + (NORM ? WK * (TM * 16 + GF_RUN) * (int)sizeof(float) : 0);
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_kernel<TM, TN, WK, DEPTH, VEC, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        const hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_kernel<TM, TN, WK, DEPTH, VEC, FORM, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return (int)e;
     }
-    gemm_f32_kernel<TM, TN, WK, DEPTH, VEC, FORM><<<(unsigned)blocks, WK * WAVE, lds, stream>>>(p);
+    gemm_f32_kernel<TM, TN, WK, DEPTH, VEC, FORM, NORM><<<(unsigned)blocks, WK * WAVE, lds, stream>>>(p);
     return CISR_LAUNCH_CHECK();
 }
 
@@ -272,51 +328,63 @@ static int launch_f32(GemmF32Args p, hipStream_t stream) {
 // 148 / 195), then 2 x 4 (1,500 x 576 x 1,536, 423 blocks, 44.2, 2 x 2 55.2; 512 x 8,192 x 2,048 207, 4 x 2 210).
 // Rows that are not aligned load word by word: three tiles, 2 x 4 from 512 of them on (512 x 3,072 x 577 58.4, 2 x 2 69.9; 1,024 x 8,192 x 1,030 572 / 658).
 // Up to 16 rows the tile has 16 of them.  A tile never changes a sum: its order is K's.
-template <int WK, bool VEC, int FORM>
+template <int WK, bool VEC, int FORM, bool NORM>
 static int launch_f32_tile(const GemmF32Args& p, hipStream_t stream) {
     const int cols = FORM == F32_PLAIN ? p.N : 2 * p.N;
     auto blocks = [&](int tm, int tn) { return (long long)((p.M + 16 * tm - 1) / (16 * tm)) * ((cols + 16 * tn - 1) / (16 * tn)); };
     auto one_round = [&](int tm, int tn) { return blocks(tm, tn) <= 256; };
     constexpr int DEEP = WK == 16 ? 8 : 4;               // sixteens in flight where a wave has few operands each
     const long long wide = blocks(2, 4);
-    if (p.M <= 16 || one_round(1, 1)) return launch_f32<1, 1, WK, DEEP, VEC, FORM>(p, stream);
+    if (p.M <= 16 || one_round(1, 1)) return launch_f32<1, 1, WK, DEEP, VEC, FORM, NORM>(p, stream);
     if constexpr (!VEC) {
-        if (wide >= 512) return launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+        if (wide >= 512) return launch_f32<2, 4, WK, 2, VEC, FORM, NORM>(p, stream);
         if constexpr (WK == 16)                           // (192 x 2,048 x 4,099 152 us with two sixteens in flight, 146 with four)
-            if (p.K >= 2048 && blocks(2, 2) >= 128) return launch_f32<2, 2, WK, 4, VEC, FORM>(p, stream);
+            if (p.K >= 2048 && blocks(2, 2) >= 128) return launch_f32<2, 2, WK, 4, VEC, FORM, NORM>(p, stream);
     } else {
-        if (one_round(1, 2)) return launch_f32<1, 2, WK, 4, VEC, FORM>(p, stream);
-        if (one_round(2, 2)) return launch_f32<2, 2, WK, 2, VEC, FORM>(p, stream);
-        if (one_round(3, 2)) return launch_f32<3, 2, WK, 2, VEC, FORM>(p, stream);
-        if (one_round(4, 2)) return launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream);
+        if (one_round(1, 2)) return launch_f32<1, 2, WK, 4, VEC, FORM, NORM>(p, stream);
+        if (one_round(2, 2)) return launch_f32<2, 2, WK, 2, VEC, FORM, NORM>(p, stream);
+        if (one_round(3, 2)) return launch_f32<3, 2, WK, 2, VEC, FORM, NORM>(p, stream);
+        if (one_round(4, 2)) return launch_f32<4, 2, WK, 2, VEC, FORM, NORM>(p, stream);
         if constexpr (WK == 8 && FORM != F32_PLAIN) {    // (a wave finishes at most one sixteen by sixteen of columns)
-            if (one_round(3, 4) && blocks(2, 2) > 512) return launch_f32<3, 4, WK, 2, VEC, FORM>(p, stream);
-            if (one_round(4, 4) && blocks(2, 2) > 800) return launch_f32<4, 4, WK, 2, VEC, FORM>(p, stream);
+            if (one_round(3, 4) && blocks(2, 2) > 512) return launch_f32<3, 4, WK, 2, VEC, FORM, NORM>(p, stream);
+            if (one_round(4, 4) && blocks(2, 2) > 800) return launch_f32<4, 4, WK, 2, VEC, FORM, NORM>(p, stream);
         }
         if constexpr (WK == 16) {
-            if (p.M <= 256 && wide > 400 && blocks(4, 2) <= wide) return launch_f32<4, 2, WK, 2, VEC, FORM>(p, stream);
-            return wide <= 400 ? launch_f32<2, 2, WK, 4, VEC, FORM>(p, stream) : launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+            if (p.M <= 256 && wide > 400 && blocks(4, 2) <= wide) return launch_f32<4, 2, WK, 2, VEC, FORM, NORM>(p, stream);
+            return wide <= 400 ? launch_f32<2, 2, WK, 4, VEC, FORM, NORM>(p, stream) : launch_f32<2, 4, WK, 2, VEC, FORM, NORM>(p, stream);
         }
         const int over = (int)(wide % 512), most = p.K >= 512 && p.K <= 960 ? 256 : 128;
-        if (wide >= 1200 || (wide >= 512 && (over == 0 || over > most))) return launch_f32<2, 4, WK, 2, VEC, FORM>(p, stream);
+        if (wide >= 1200 || (wide >= 512 && (over == 0 || over > most))) return launch_f32<2, 4, WK, 2, VEC, FORM, NORM>(p, stream);
     }
-    return launch_f32<2, 2, WK, 2, VEC, FORM>(p, stream);
+    return launch_f32<2, 2, WK, 2, VEC, FORM, NORM>(p, stream);
 }
 
 // Waves a tile: sixteen from an inner size of 1,024 on, else eight (so that a wave has at least two sixteens at the small
-// models' 576).
+// models' 576).  A fused norm takes eight waves and rows in 16-byte words only.
+#define GF_SIXTEEN_WAVES 1024
+static_assert(GF_SIXTEEN_WAVES / 8 + 16 <= GF_RUN, "a wave's run of the norm's weights");
 template <int FORM>
 static int launch_f32_form(const GemmF32Args& p, hipStream_t stream) {
     const bool vec = p.K % 4 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0 && (uintptr_t)p.A % 16 == 0 && (uintptr_t)p.W % 16 == 0;
-    if (p.K >= 1024) return vec ? launch_f32_tile<16, true, FORM>(p, stream) : launch_f32_tile<16, false, FORM>(p, stream);
-    return vec ? launch_f32_tile<8, true, FORM>(p, stream) : launch_f32_tile<8, false, FORM>(p, stream);
+    if (p.norm_w) {
+        if (!vec || (uintptr_t)p.norm_w % 16 || p.K >= GF_SIXTEEN_WAVES) return (int)hipErrorInvalidValue;
+        return launch_f32_tile<8, true, FORM, true>(p, stream);
+    }
+    if (p.K >= GF_SIXTEEN_WAVES) return vec ? launch_f32_tile<16, true, FORM, false>(p, stream) : launch_f32_tile<16, false, FORM, false>(p, stream);
+    return vec ? launch_f32_tile<8, true, FORM, false>(p, stream) : launch_f32_tile<8, false, FORM, false>(p, stream);
 }
 
+// The entry points with `norm_w`: A is float rows x, and the product's rows are RMSNorm(x[rows]) (rows null: of x's rows in order).
+
 // C[M, N] = silu(A . Wg^T) * (A . Wu^T) with W = [Wg; Wu], 2 N rows
-extern "C" int cisr_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, hipStream_t stream) {
+extern "C" int cisr_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K,
+                                    const float* norm_w, float eps, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return (int)hipErrorInvalidValue;
     GemmF32Args p{A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, 0};
+    p.norm_w = norm_w;
+    p.eps = eps;
+    p.inv_k = 1.0f / (float)K;
     return launch_f32_form<F32_GATED>(p, stream);
 }
 
@@ -324,19 +392,23 @@ extern "C" int cisr_gemm_f32_swiglu(const float* A, int lda, const float* W, int
 // and values to the pages at `slots`
 extern "C" int cisr_gemm_f32_rope(const float* A, int lda, const float* W, int ldw, float* q_out, int ldq, int M, int K, const int* positions,
                                   const int* slots, const float* cos_tab, const float* sin_tab, float* kcache, float* vcache, int heads,
-                                  int kv_heads, int dim, int page_size, int max_pos, hipStream_t stream) {
+                                  int kv_heads, int dim, int page_size, int max_pos, const float* norm_w, float eps, hipStream_t stream) {
     if (M <= 0 || heads <= 0) return 0;
     if (K <= 0 || dim <= 0 || dim % 2 || kv_heads < 0 || page_size <= 0 || max_pos <= 0 || !positions || (kv_heads && (!slots || !kcache || !vcache)))
         return (int)hipErrorInvalidValue;
     GemmF32Args p{A, lda, W, ldw, q_out, ldq, nullptr, 0, M, (heads + 2 * kv_heads) * dim / 2, K, 0,
-                  positions, slots, cos_tab, sin_tab, kcache, vcache, heads, kv_heads, dim, page_size, max_pos};
+                  positions, slots, cos_tab, sin_tab, kcache, vcache, heads, kv_heads, dim, page_size, max_pos, norm_w, eps, 1.0f / (float)K};
     return launch_f32_form<F32_ROTARY>(p, stream);
 }
 
-extern "C" int cisr_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
-                             const float* R, int ldr, int M, int N, int K, hipStream_t stream) {
+extern "C" int cisr_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc, const float* R, int ldr, int M, int N, int K,
+                             const float* norm_w, float eps, const int* rows, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K <= 0) return (int)hipErrorInvalidValue;
-    const GemmF32Args p{A, lda, W, ldw, C, ldc, R, ldr, M, N, K, 0};
+    if (K <= 0 || (rows && !norm_w)) return (int)hipErrorInvalidValue;
+    GemmF32Args p{A, lda, W, ldw, C, ldc, R, ldr, M, N, K, 0};
+    p.norm_w = norm_w;
+    p.eps = eps;
+    p.inv_k = 1.0f / (float)K;
+    p.rows = rows;
     return launch_f32_form<F32_PLAIN>(p, stream);
 }

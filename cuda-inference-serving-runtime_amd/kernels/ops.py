@@ -49,9 +49,9 @@ def _declare(h):
         "cisr_f32_to_bf16": [p, p, ll, p],
         "cisr_bias_add": [p, p, ll, i, i, i, p],
         "cisr_attn_rowwise": [p, i, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f, i, i, p, p, i, p],
-        "cisr_gemm_f32": [p, i, p, i, p, i, p, i, i, i, i, p],
-        "cisr_gemm_f32_swiglu": [p, i, p, i, p, i, i, i, i, p],
-        "cisr_gemm_f32_rope": [p, i, p, i, p, i, i, i, p, p, p, p, p, p, i, i, i, i, i, p],
+        "cisr_gemm_f32": [p, i, p, i, p, i, p, i, i, i, i, p, f, p, p],
+        "cisr_gemm_f32_swiglu": [p, i, p, i, p, i, i, i, i, p, f, p],
+        "cisr_gemm_f32_rope": [p, i, p, i, p, i, i, i, p, p, p, p, p, p, i, i, i, i, i, p, f, p],
         "cisr_gemm_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_bf16_swiglu": [p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_bf16_tile": [p, i, p, i, p, i, p, i, i, i, i, i, i, p],
@@ -819,7 +819,7 @@ def gemm(a, w, out, residual=None, after_norm=False, scratch=None):
         if out.dtype != torch.float32:
             raise KernelError("gemm: float operands need a float output")
         code = lib().cisr_gemm_f32(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
-                                   rp, ldr, m, n, k, _stream())
+                                   rp, ldr, m, n, k, None, 0.0, None, _stream())
     elif (a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w, fused=residual is not None, floats=out.dtype == torch.float32, cut=residual is not None)
           and (at := _ring_operands(a, w, out)) is not None and (residual is None or (ldr % 4 == 0 and rp % 16 == 0))):
         if residual is not None and residual is out and partials_ok(out):
@@ -1000,21 +1000,33 @@ def _skinny_ok(a, w):
             and w.data_ptr() % 16 == 0)
 
 
-def _norm_args(x, norm, k):
-    """(weight pointer, eps, rows pointer, number of output rows) for a fused RMSNorm prologue."""
+def _norm_args(x, norm, k, words=8):
+    """(weight pointer, eps, rows pointer, number of output rows) for a fused RMSNorm prologue that reads `words` floats of a row at a
+    time."""
     weight, eps, rows = norm
     if not isinstance(x, torch.Tensor) or not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1:
         raise KernelError("fused norm: expected float GPU rows with unit column stride (a view of wider rows will do)")
-    if x.shape[1] != k or x.stride(0) % 8 or x.data_ptr() % 16:
-        raise KernelError("fused norm: the residual rows must be 32-byte aligned floats of the product's inner size")
+    if x.shape[1] != k or x.stride(0) % words or x.data_ptr() % 16:
+        raise KernelError(f"fused norm: the residual rows must be {4 * words}-byte aligned floats of the product's inner size")
     wp = _dev(weight, "norm weight", torch.float32, (k,))
     rp = None if rows is None else _dev(rows, "rows", torch.int32)
     return wp, float(eps), rp, (x.shape[0] if rows is None else rows.shape[0])
 
 
-def fused_norm_ok(x, w, rows_out):
+def _f32_norm_ok(x, w, weight=None):
+    """Whether the 32-bit product takes RMSNorm(x) . w^T with the norm (of `weight`) fused: 16-byte aligned float rows, an inner size of a
+    multiple of four below 1,024.  Any number of rows, so that a row's bits do not depend on the others of its step (csrc/gemm_f32.hip has
+    the figures)."""
+    return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.is_cuda and w.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.stride(1) == 1
+            and w.stride(1) == 1 and x.shape[1] % 4 == 0 and x.shape[1] < 1024 and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
+            and (x.data_ptr() | w.data_ptr() | (0 if weight is None else weight.data_ptr())) % 16 == 0)
+
+
+def fused_norm_ok(x, w, rows_out, weight=None):
     """Whether the weight-streaming kernel can take RMSNorm(x) . w^T with the norm fused (and large weights
-    do not make the norm as a kernel of its own and the wide kernel the better choice)."""
+    do not make the norm as a kernel of its own and the wide kernel the better choice), or in 32 bits the product (`weight`: the norm's)."""
+    if w.dtype == torch.float32:
+        return rows_out > 0 and _f32_norm_ok(x, w, weight)
     return (not wide_ok(rows_out, w, after_norm=True, fused=True) and w.dtype == torch.bfloat16 and rows_out <= SKINNY_ROWS and x.dtype == torch.float32 and x.shape[1] % 8 == 0
             and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0)
 
@@ -1027,11 +1039,16 @@ def swiglu_fused_ok(a, w_gate_up):
 
 def gemm_normed(x, norm, w, out):
     """out[R, N] = RMSNorm(x[rows]) . w^T with the norm applied inside the product's kernel.
-    x float [T, K]; norm = (weight float [K], eps, rows int32 [R] or None); w bf16 [N, K]; out float or bf16."""
+    x float [T, K]; norm = (weight float [K], eps, rows int32 [R] or None); w bf16 [N, K], out float or bf16; or w and out float."""
     n, k = w.shape
-    wp, eps, rp, m = _norm_args(x, norm, k)
-    if not fused_norm_ok(x, w, m) or tuple(out.shape) != (m, n) or out.stride(1) != 1:
+    floats = w.dtype == torch.float32
+    wp, eps, rp, m = _norm_args(x, norm, k, 4 if floats else 8)
+    if not fused_norm_ok(x, w, m) or tuple(out.shape) != (m, n) or out.stride(1) != 1 or (floats and (out.dtype != torch.float32 or wp % 16)):
         raise KernelError("gemm_normed: shape not supported by the fused kernel")
+    if floats:
+        _check(lib().cisr_gemm_f32(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), None, 0, m, n, k, wp, eps,
+                                   rp, _stream()), "gemm_normed")
+        return out
     _check(lib().cisr_gemm_skinny_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
                                        None, 0, m, n, k, _storage(out, "out"), 0, wp, eps, rp, _stream()), "gemm_normed")
     return out
@@ -1055,7 +1072,15 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
     if norm is not None:
         if law is not None:
             raise KernelError("gemm_swiglu: the fused norm comes with the silu law only")
-        wp, eps, rp, _ = _norm_args(a, norm, k)
+        floats = w_gate_up.dtype == torch.float32
+        wp, eps, rp, _ = _norm_args(a, norm, k, 4 if floats else 8)
+        if floats:
+            if (not fused_norm_ok(a, w_gate_up, m) or out.dtype != torch.float32 or wp % 16 or rp is not None
+                    or a.untyped_storage().data_ptr() == out.untyped_storage().data_ptr()):
+                raise KernelError("gemm_swiglu: shape not supported by the 32-bit product with the norm fused")
+            _check(lib().cisr_gemm_f32_swiglu(a.data_ptr(), a.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), _dev(out, "out"), out.stride(0),
+                                              m, inter, k, wp, eps, _stream()), "gemm_swiglu")
+            return out
         if not fused_norm_ok(a, w_gate_up, m) or out.dtype != torch.bfloat16:
             raise KernelError("gemm_swiglu: shape not supported by the fused kernel")
         _check(lib().cisr_gemm_skinny_bf16(a.data_ptr(), a.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0),
@@ -1108,16 +1133,18 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         if tuple(gate_up.shape) != (m, two_i) or gate_up.dtype != torch.float32 or not gate_up.is_cuda or gate_up.stride(1) != 1:
             raise KernelError("gemm_swiglu: gate_up is float rows [M, 2I] on the GPU")
         _check(lib().cisr_gemm_f32_swiglu(a.data_ptr(), a.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), _dev(out, "out"), out.stride(0),
-                                          m, inter, k, _stream()), "gemm_swiglu")
+                                          m, inter, k, None, 0.0, _stream()), "gemm_swiglu")
         return out
     gemm(a, w_gate_up, gate_up, scratch=scratch)
     return activate(gate_up, out)
 
 
-def qkv_rope_fused_ok(a, w, head_dim, cos, normed, scratch=None, sin=None):
+def qkv_rope_fused_ok(a, w, head_dim, cos, normed, scratch=None, sin=None, weight=None):
     """Whether the fused projection + rotary + scatter kernel takes this shape and, where `sin` is at hand, these tables (`scratch`: the pool that
-    qkv_rope is given)."""
+    qkv_rope is given; `weight`: that of the norm to be fused)."""
     m, k = a.shape
+    if normed and w.dtype == torch.float32:
+        return _f32_norm_ok(a, w, weight) and qkv_rope_f32_ok(a, w, head_dim, cos)
     if normed and wide_ok(m, w, after_norm=True, fused=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
         return False
     if not normed and _ring_open(scratch) and ring_rope_ok(a, w, head_dim, cos, sin):
@@ -1139,8 +1166,13 @@ def qkv_rope_f32_ok(a, w, head_dim, cos):
             and w.stride(1) == 1 and head_dim % 2 == 0 and 2 * cos.shape[1] == head_dim and 0 < a.shape[0])
 
 
-def _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size):
+def _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm=None):
     m, k = a.shape
+    wp, eps = None, 0.0
+    if norm is not None:
+        wp, eps = _dev(norm[0], "norm weight", torch.float32, (k,)), float(norm[1])
+        if not _f32_norm_ok(a, w) or wp % 16:
+            raise KernelError("qkv_rope: shape not supported by the 32-bit product with the norm fused")
     kp = vp = sp = None
     if kcache is not None:
         pages = kcache.shape[0]
@@ -1153,17 +1185,17 @@ def _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads
     _check(lib().cisr_gemm_f32_rope(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), _dev(q_out, "q_out", torch.float32, (m, heads * dim)),
                                     heads * dim, m, k, _dev(positions, "positions", torch.int32, (m,)), sp, _dev(cos, "cos", torch.float32),
                                     _dev(sin, "sin", torch.float32, (max_pos, dim // 2)), kp, vp, heads, n_kv, dim, page_size, max_pos,
-                                    _stream()), "qkv_rope")
+                                    wp, eps, _stream()), "qkv_rope")
     return q_out
 
 
 def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm=None, scratch=None):
-    """One kernel for a step's projections (few rows, or the ring product): (RMSNorm of the float residual `a` if `norm` = (weight, eps),
+    """One kernel for a step's projections (few rows, the ring product, or 32 bits): (RMSNorm of the float residual `a` if `norm` = (weight, eps),
     else `a` is bf16 and normed), product with w = [Wq; Wk; Wv], rotary embedding of q and k, q into
     q_out [M, heads*dim], k and v into the cache at `slots`.  kcache None: w = Wq only (a layer reading
     another layer's cache)."""
-    if norm is None and qkv_rope_f32_ok(a, w, dim, cos):
-        return _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size)
+    if qkv_rope_f32_ok(a, w, dim, cos):
+        return _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm)
     m, k = a.shape
     has_kv = kcache is not None
     n_kv = kv_heads if has_kv else 0

@@ -81,15 +81,15 @@ class PagedAttention(Mixer):
     def _interleaved(self):
         return getattr(self.position, "pairing", "split_half") == "interleaved"
 
-    def _fused_projection_ok(self, a, normed, scratch):
+    def _fused_projection_ok(self, a, normed, scratch, weight=None):
         cos, sin = self.position.tables()
         # (the fused kernels turn split-half pairs only; another pairing takes the general rotary kernel)
         if self._interleaved or self.bias:
             return False
-        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed, scratch, sin) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
+        return ops.qkv_rope_fused_ok(a, self.w_in, self.head_dim, cos, normed, scratch, sin, weight) or (not normed and ops.qkv_rope_f32_ok(a, self.w_in, self.head_dim, cos))
 
     def fuses_norm(self, norm, residual, ctx):
-        return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True, ctx.scratch)
+        return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True, ctx.scratch, norm.weight)
 
     def forward(self, h, residual, ctx, site, norm=None):
         T = residual.shape[0]
@@ -102,7 +102,7 @@ class PagedAttention(Mixer):
         else:
             kcache_w, vcache_w, slots = kcache, vcache, view.slots
         if norm is not None or self._fused_projection_ok(h, False, ctx.scratch):
-            # few rows (in 32 bits any): norm, projections, rotary embedding and the cache write are one kernel
+            # few rows (in 32 bits any number): norm, projections, rotary embedding and the cache write are one kernel
             q, q_stride = ctx.buffer("attn.q", (T, nh * D), ctx.dtype), nh * D
             ops.qkv_rope(residual if norm is not None else h, self.w_in, q, ctx.positions, slots, cos, sin,
                          kcache_w, vcache_w, nh, nkv, D, view.page_size,
@@ -391,7 +391,7 @@ class LatentAttention(Mixer):
         if self.q_rank is not None:
             first = self.q_size
         q = ctx.buffer("lat.q", (T, nh * (D + R)), ctx.dtype)
-        if self.q_rank is not None and ops.fused_norm_ok(small[:, :first], self.w_q, T):
+        if self.q_rank is not None and ops.fused_norm_ok(small[:, :first], self.w_q, T, self.q_weight):
             # few rows: the query latent's norm rides in the product that reads it
             ops.gemm_normed(small[:, :first], (self.q_weight, self.eps, None), self.w_q, q)
         else:

@@ -44,7 +44,7 @@ class GatedMLP(FeedForward):
             self.b_down = tensors[f"{self.name}.down_proj.bias"].contiguous()
 
     def fuses_norm(self, norm, residual, ctx):
-        return not self.bias and self.law is None and getattr(norm, "fusable_as", None) == "rms" and ops.fused_norm_ok(residual, self.w_gate_up, residual.shape[0])
+        return not self.bias and self.law is None and getattr(norm, "fusable_as", None) == "rms" and ops.fused_norm_ok(residual, self.w_gate_up, residual.shape[0], norm.weight)
 
     def forward(self, h, residual, ctx, norm=None):
         T = residual.shape[0]
