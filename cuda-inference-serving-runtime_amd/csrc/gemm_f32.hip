@@ -259,9 +259,7 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
         float all = 0.f;
 #pragma unroll
         for (int w = 0; w < WK; ++w) all += ssq[(w * TM + i) * 16 + r];
-        const float mean = fmaf(all, p.inv_k, p.eps), half = 0.5f * mean;
-        float f = __builtin_amdgcn_rsqf(mean);
-        if (mean < INFINITY) f = fmaf(f, fmaf(-half * f, f, 0.5f), f);
+        const float f = row_factor(all, p.inv_k, p.eps);
 #pragma unroll
         for (int e = 0; e < 4; ++e) factor[e] = __shfl(f, 4 * g + e, WAVE);
     }

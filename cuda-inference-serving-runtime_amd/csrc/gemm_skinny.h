@@ -16,7 +16,7 @@ struct SkinnyArgs {
     GateLaw law;                       // EPI_SWIGLU: the activation's law (zeros: silu(g) u)
     int act;                           // EPI_STORE without a residual: an ungated activation before the store (ACT_*)
     // NORM
-    const float* norm_w; float eps; const int* rows;
+    const float* norm_w; float eps, inv_k; const int* rows;   // (inv_k: 1 / K)
     // EPI_ROPE
     const int* positions; const int* slots; const float* cos_tab; const float* sin_tab;
     bf16_t* kcache; bf16_t* vcache; int heads, kv_heads, head_dim, page_size, max_pos;

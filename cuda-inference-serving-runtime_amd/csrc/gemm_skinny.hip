@@ -106,7 +106,7 @@ static int skinny_entry(const void* A, int lda, const void* W, int ldw, void* C,
         return (int)hipErrorInvalidValue;
     SkinnyArgs a = {};
     a.A = A; a.lda = lda; a.W = (const bf16_t*)W; a.ldw = ldw; a.C = C; a.ldc = ldc; a.R = R; a.ldr = ldr;
-    a.M = M; a.N = N; a.K = K; a.dual_off = dual_off; a.norm_w = norm_w; a.eps = eps; a.rows = rows; a.law = law; a.act = act;
+    a.M = M; a.N = N; a.K = K; a.dual_off = dual_off; a.norm_w = norm_w; a.eps = eps; a.inv_k = 1.0f / (float)K; a.rows = rows; a.law = law; a.act = act;
     const int epi = dual_off > 0 ? EPI_SWIGLU : EPI_STORE;
     if (cisr_gemv_ahead(M, dual_off > 0 ? 2 * N : N, K, norm_w != nullptr, dual_off > 0)) return cisr_gemv_launch(a, N, norm_w != nullptr, epi, out_dtype, 0, stream);
     if (narrow_wanted(M, dual_off > 0 ? 2 * N : N, K, norm_w != nullptr)) return launch_narrow(a, (N + 3) / 4, norm_w != nullptr, epi, out_dtype, stream);
@@ -127,7 +127,7 @@ extern "C" int cisr_qkv_rope_skinny(const void* A, int lda, const void* W, int l
         return (int)hipErrorInvalidValue;
     SkinnyArgs a = {};
     a.A = A; a.lda = lda; a.W = (const bf16_t*)W; a.ldw = ldw; a.C = q_out; a.ldc = ldq;
-    a.M = M; a.N = (heads + 2 * kv_heads) * head_dim; a.K = K; a.norm_w = norm_w; a.eps = eps;
+    a.M = M; a.N = (heads + 2 * kv_heads) * head_dim; a.K = K; a.norm_w = norm_w; a.eps = eps; a.inv_k = 1.0f / (float)K;
     a.positions = positions; a.slots = slots; a.cos_tab = cos_tab; a.sin_tab = sin_tab;
     a.kcache = (bf16_t*)kcache; a.vcache = (bf16_t*)vcache; a.heads = heads; a.kv_heads = kv_heads;
     a.head_dim = head_dim; a.page_size = page_size; a.max_pos = max_pos;

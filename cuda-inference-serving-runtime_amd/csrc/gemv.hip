@@ -236,7 +236,7 @@ gemv_kernel(SkinnyArgs p, int units, int per_wave) {
     }
     const bool finisher = (lane & ((64 / M) - 1)) == 0 && my_m < p.M;      // one lane for every activation row
     float scale = 1.f;
-    if (NORM) scale = 1.0f / sqrtf((((ssq_s[my_m][0] + ssq_s[my_m][1]) + ssq_s[my_m][2]) + ssq_s[my_m][3]) / (float)K + p.eps);
+    if (NORM) scale = row_factor(((ssq_s[my_m][0] + ssq_s[my_m][1]) + ssq_s[my_m][2]) + ssq_s[my_m][3], p.inv_k, p.eps);
     int pos = 0, slot = -1;
     if (EPI == EPI_ROPE && finisher) {
         pos = p.positions[my_m];
