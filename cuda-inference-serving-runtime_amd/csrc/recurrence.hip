@@ -59,37 +59,82 @@ extern "C" int cisr_linear_scan(const float* q, int ldq, const float* k, int ldk
 // out[t * channels + ch] = silu(bias[ch] + sum_j w[ch * taps + j] * input(t - (taps - 1) + j)).
 // Index channels + h, h < heads (if heads > 0): step[t * heads + h] = softplus(in[t * ld + dt_first + h] + dt_bias[h]),
 // decay[t * heads + h] = exp(-exp(a_log[h]) * step).
+// UNIT (unit.channels > 0): the first `unit.channels` results are heads of unit.dim (a power of two from 16 to 256) channels, each of which
+// becomes x / sqrt(sum(x^2) + eps): the queries and keys of a delta rule, otherwise a kernel of their own (recurrence_delta.hip) that
+// reads and writes them once more.  A head's squares are added neighbour by neighbour, pair by pair, in either kernel.  Of 8,192 channels
+// 4,096 in heads of 128, us of the convolution / with the kernel behind it / so: 1,999 rows 40.6 / 58.7 / 40.6, 300 rows 17.5 / 23.7 / 17.0, 8 single
+// rows 3.4 / 5.8 / 3.7, 64 6.2 / 9.0 / 6.2.
 // SINGLE: every segment has one row (a step of single tokens), so the thread of a (row, channel) is the only one that
 // reads that channel of its request's state, and it moves the state on itself: no second launch.
+struct ConvUnit { int channels, dim; float eps; };
+
+template <int CTRL>
+__device__ __forceinline__ float conv_moved(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false)); }
+
+// the sum over the aligned group of `lanes` (1, 2, 4, ... 64) neighbours, in all of them, without a trip through LDS
+__device__ __forceinline__ float conv_neighbours(float x, int lanes) {
+    if (lanes >= 2) x += conv_moved<0xb1>(x);                  // quad_perm [1, 0, 3, 2]
+    if (lanes >= 4) x += conv_moved<0x4e>(x);                  // quad_perm [2, 3, 0, 1]
+    if (lanes >= 8) x += conv_moved<0x141>(x);                 // row_half_mirror (the quads' sums are the same in all four)
+    if (lanes >= 16) x += conv_moved<0x140>(x);                // row_mirror
+    if (lanes >= 32) {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    if (lanes >= 64) {
+        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    return x;
+}
+
 template <bool SINGLE>
 __global__ void __launch_bounds__(256)
 conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* __restrict__ w, const float* __restrict__ bias,
                  float* conv_state, long long slot_stride, float* __restrict__ out,
                  const int* __restrict__ seg_of_row, const int* __restrict__ seg_start, const int* __restrict__ state_slots,
                  int channels, int taps, int heads, int dt_first, const float* __restrict__ dt_bias,
-                 const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay) {
+                 const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay, ConvUnit unit) {
+    __shared__ float red[4];
     const int t = blockIdx.x;
     const int idx = blockIdx.y * 256 + threadIdx.x;
     const int seg = seg_of_row[t];
-    if (seg < 0 || idx >= channels + heads) return;
-    if (idx >= channels) {
+    if (seg < 0) return;
+    const bool units = (int)blockIdx.y * 256 < unit.channels;       // (uniform: a block that meets in the end, and all of its threads come)
+    if (idx >= channels + heads && !units) return;
+    if (idx >= channels && idx < channels + heads) {
         const int h = idx - channels;
         const float z = in[(size_t)t * ld + dt_first + h] + dt_bias[h];
         const float dt = z > 20.f ? z : log1pf(expf(z));
         step[(size_t)t * heads + h] = dt;
         decay[(size_t)t * heads + h] = expf(-expf(a_log[h]) * dt);
-        return;
+        if (!units) return;
     }
-    const int rel = t - seg_start[seg];
-    float* st = conv_state + (long long)state_slots[seg] * slot_stride;
-    float y = bias ? bias[idx] : 0.f;
-    for (int j = 0; j < taps; ++j) {
-        const int src = rel - (taps - 1) + j;
-        const float x = src >= 0 ? in[(size_t)(t - rel + src) * ld + first + idx] : st[(size_t)(taps - 1 + src) * channels + idx];
-        y += w[(size_t)idx * taps + j] * x;
-        if (SINGLE && j > 0) st[(size_t)(j - 1) * channels + idx] = x;     // (input j of this row is input j - 1 of the next)
+    float y = 0.f;
+    if (idx < channels) {
+        const int rel = t - seg_start[seg];
+        float* st = conv_state + (long long)state_slots[seg] * slot_stride;
+        y = bias ? bias[idx] : 0.f;
+        for (int j = 0; j < taps; ++j) {
+            const int src = rel - (taps - 1) + j;
+            const float x = src >= 0 ? in[(size_t)(t - rel + src) * ld + first + idx] : st[(size_t)(taps - 1 + src) * channels + idx];
+            y += w[(size_t)idx * taps + j] * x;
+            if (SINGLE && j > 0) st[(size_t)(j - 1) * channels + idx] = x;     // (input j of this row is input j - 1 of the next)
+        }
+        y = y / (1.0f + expf(-y));
     }
-    out[(size_t)t * channels + idx] = y / (1.0f + expf(-y));
+    if (units) {
+        float sum = conv_neighbours(y * y, min(unit.dim, WAVE));
+        if (unit.dim > WAVE) {
+            const int wave = threadIdx.x / WAVE;
+            if (threadIdx.x % WAVE == 0) red[wave] = sum;
+            __syncthreads();
+            sum = red[wave & ~1] + red[wave | 1];
+            if (unit.dim > 2 * WAVE) sum = (red[0] + red[1]) + (red[2] + red[3]);
+        }
+        if (idx < unit.channels) y *= rsqrtf(sum + unit.eps);
+    }
+    if (idx < channels) out[(size_t)t * channels + idx] = y;
 }
 
 // The same for portions, four channels a thread and CONV_ROWS rows of the step a block: an input is read once (the taps - 1
@@ -109,13 +154,13 @@ conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* _
 #define CONV_WORDS (3ll << 19)               // inputs of a step of one portion
 #define CONV_WORDS_A_PORTION 170000ll        // and for each of up to sixteen more
 typedef __attribute__((ext_vector_type(4))) float conv_f32x4;
-template <int TAPS>
+template <int TAPS, bool UNIT>
 __global__ void __launch_bounds__(256)
 conv_silu_rows_kernel(const float* __restrict__ in, int ld, int first, const float* __restrict__ w, const float* __restrict__ bias,
                       const float* __restrict__ conv_state, long long slot_stride, float* __restrict__ out,
                       const int* __restrict__ seg_of_row, const int* __restrict__ seg_start, const int* __restrict__ state_slots,
                       int rows, int channels, int heads, int dt_first, const float* __restrict__ dt_bias,
-                      const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay) {
+                      const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay, ConvUnit unit) {
     const int t0 = blockIdx.x * CONV_ROWS, t1 = min(t0 + CONV_ROWS, rows);
     const int channel_blocks = (channels / 4 + 255) / 256;
     if ((int)blockIdx.y >= channel_blocks) {
@@ -132,6 +177,7 @@ conv_silu_rows_kernel(const float* __restrict__ in, int ld, int first, const flo
     }
     const int c = ((int)blockIdx.y * 256 + threadIdx.x) * 4;
     if (c >= channels) return;
+    const int wave_first = __builtin_amdgcn_readfirstlane(c);
     const float* x0 = in + first + c;
     float taps[4][TAPS];
 #pragma unroll
@@ -148,6 +194,12 @@ conv_silu_rows_kernel(const float* __restrict__ in, int ld, int first, const flo
             for (int k = 0; k < 4; ++k) y[k] += taps[k][j] * use[j][k];
 #pragma unroll
         for (int k = 0; k < 4; ++k) y[k] = y[k] / (1.0f + expf(-y[k]));
+        if constexpr (UNIT) {                            // (whole waves beyond the heads pass by)
+            if (wave_first < unit.channels) {
+                const float f = rsqrtf(conv_neighbours((y[0] * y[0] + y[1] * y[1]) + (y[2] * y[2] + y[3] * y[3]), unit.dim / 4) + unit.eps);
+                if (c < unit.channels) y *= f;
+            }
+        }
         *(conv_f32x4*)(out + (size_t)t * channels + c) = y;
     };
     const int whose = seg_of_row[t0];
@@ -230,28 +282,34 @@ extern "C" int cisr_conv_silu(const float* in, int ld, int first, const float* w
                               long long slot_stride, float* out, const int* seg_of_row, const int* seg_start,
                               const int* state_slots, int rows, int segments, int channels, int taps, int heads,
                               int dt_first, const float* dt_bias, const float* a_log, float* step, float* decay,
-                              int single_rows, hipStream_t stream) {
+                              int single_rows, int unit_channels, int unit_dim, float unit_eps, hipStream_t stream) {
     if (rows <= 0 || segments <= 0) return 0;
+    const ConvUnit unit{unit_channels, unit_dim, unit_eps};
+    if (unit_channels < 0 || unit_channels > channels ||
+        (unit_channels && (unit_dim < 16 || unit_dim > 256 || (unit_dim & (unit_dim - 1)) || unit_channels % unit_dim)))
+        return (int)hipErrorInvalidValue;
     if (channels <= 0 || taps < 1 || taps > MAX_TAPS || heads < 0 || segments > 65535) return (int)hipErrorInvalidValue;
     const dim3 grid(rows, (channels + heads + 255) / 256);
     if (single_rows) {       // `single_rows`: the caller knows that no segment has more than one row
         conv_silu_kernel<true><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride,
-            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay);
+            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay, unit);
         return CISR_LAUNCH_CHECK();
     }
     const bool enough = (long long)rows * channels >= CONV_WORDS + CONV_WORDS_A_PORTION * min(segments - 1, 16);
     if (enough && taps >= 2 && taps <= 4 && channels % 4 == 0 && ld % 4 == 0 && first % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0 &&
         (!bias || (uintptr_t)bias % 16 == 0)) {
         const dim3 blocks((rows + CONV_ROWS - 1) / CONV_ROWS, (channels / 4 + 255) / 256 + (heads + 255) / 256);
-#define CONV_ROWS_OF(TAPS) conv_silu_rows_kernel<TAPS><<<blocks, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride, \
-            out, seg_of_row, seg_start, state_slots, rows, channels, heads, dt_first, dt_bias, a_log, step, decay)
+#define CONV_ROWS_AS(TAPS, UNIT) conv_silu_rows_kernel<TAPS, UNIT><<<blocks, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride, \
+            out, seg_of_row, seg_start, state_slots, rows, channels, heads, dt_first, dt_bias, a_log, step, decay, unit)
+#define CONV_ROWS_OF(TAPS) do { if (unit_channels) CONV_ROWS_AS(TAPS, true); else CONV_ROWS_AS(TAPS, false); } while (0)
         if (taps == 2) CONV_ROWS_OF(2);
         else if (taps == 3) CONV_ROWS_OF(3);
         else CONV_ROWS_OF(4);
 #undef CONV_ROWS_OF
+#undef CONV_ROWS_AS
     } else {
         conv_silu_kernel<false><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride,
-            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay);
+            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay, unit);
     }
     int err = CISR_LAUNCH_CHECK();
     if (err || taps == 1) return err;

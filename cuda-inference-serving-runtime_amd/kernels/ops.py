@@ -1790,7 +1790,7 @@ def _rec():
             "cisr_linear_scan": [p, i, p, i, p, i, p, i, i, p, i, p, i, p, ll, p, p, i, i, i, i, i, f, i, i, i, i, p, p, p],
             "cisr_lightning_step": [p, i, p, i, p, i, p, p, i, p, ll, p, p, i, i, i, i, p],
             "cisr_lightning_chunks": [p, i, p, i, p, i, p, p, i, p, ll, p, p, i, i, i, i, i, p, p],
-            "cisr_conv_silu": [p, i, i, p, p, p, ll, p, p, p, p, i, i, i, i, i, i, p, p, p, p, i, p],
+            "cisr_conv_silu": [p, i, i, p, p, p, ll, p, p, p, p, i, i, i, i, i, i, p, p, p, p, i, i, i, f, p],
             "cisr_decay_gate": [p, i, p, p, i, i, f, p],
             "cisr_decay_gate_low_rank": [p, i, i, p, p, p, i, i, f, p],
             "cisr_group_norm_gate": [p, p, i, p, i, p, i, p, i, p, i, i, i, f, i, i, i, p],
@@ -1946,16 +1946,25 @@ def lightning(form, q, k, v, decay, out, state, seg_start, state_slots, heads, r
     return out
 
 
-def conv_silu(x, taps_weight, bias, conv_state, out, seg_of_row, seg_start, state_slots, gates=None, single_rows=False):
+def conv_unit_ok(dim):
+    """Whether conv_silu makes unit vectors of heads of `dim` channels on its way."""
+    return 16 <= dim <= 256 and dim & (dim - 1) == 0
+
+
+def conv_silu(x, taps_weight, bias, conv_state, out, seg_of_row, seg_start, state_slots, gates=None, single_rows=False, unit=None):
     """out[t, c] = silu(bias[c] + sum_j w[c, j] input(t - (K - 1) + j)[c]) over the rows of each segment, the K - 1 inputs
     before a segment's first row taken from its state slot, which then moves on to the last K - 1 inputs.
     x float view [T, channels]; taps_weight float [channels, K]; conv_state float view [slots, >= (K - 1) * channels].
     `gates` = (dt view [T, heads], dt_bias [heads], a_log [heads], step out [T, heads], decay out [T, heads]):
     step = softplus(dt + dt_bias), decay = exp(-exp(a_log) step), made by the same launch.
     `single_rows`: the caller vouches that no segment has more than one row (a step of single tokens); the state then
-    moves on in the same launch instead of a second one."""
+    moves on in the same launch instead of a second one.
+    `unit` = (heads, dim, eps): of the first heads * dim channels every head becomes x / sqrt(sum(x^2) + eps) (conv_unit_ok(dim))."""
     T, channels = x.shape
     K = taps_weight.shape[1]
+    units, unit_dim, unit_eps = unit or (0, 0, 0.0)
+    if units and not conv_unit_ok(unit_dim):
+        raise KernelError("conv_silu: unit vectors of a power of two from 16 to 256 channels")
     segments = state_slots.shape[0]
     xp, ld = _rows_of(x, "x")
     if conv_state.dtype != torch.float32 or conv_state.stride(1) != 1 or conv_state.shape[1] < (K - 1) * channels:
@@ -1976,7 +1985,8 @@ def conv_silu(x, taps_weight, bias, conv_state, out, seg_of_row, seg_start, stat
                                  _dev(seg_of_row, "seg_of_row", torch.int32, (T,)),
                                  _dev(seg_start, "seg_start", torch.int32, (segments + 1,)),
                                  _dev(state_slots, "state_slots", torch.int32, (segments,)), T, segments, channels, K, heads,
-                                 dt_first, bp2, alp, stp, dcp, int(bool(single_rows)), _stream()), "conv_silu")
+                                 dt_first, bp2, alp, stp, dcp, int(bool(single_rows)), units * unit_dim, unit_dim, float(unit_eps), _stream()),
+           "conv_silu")
     return out
 
 

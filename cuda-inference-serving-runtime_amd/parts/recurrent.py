@@ -403,9 +403,12 @@ class GatedDeltaRule(Mixer):
         heads_state = nh * self.dim * self.vdim
         qkv = ctx.buffer("delta.qkv", (T, ch), torch.float32)
         step, decay = ctx.buffer("delta.step", (T, nh), torch.float32), ctx.buffer("delta.decay", (T, nh), torch.float32)
+        fused = ops.conv_unit_ok(self.dim)       # (queries and keys become unit vectors where they are made)
         ops.conv_silu(proj[:, :ch], self.conv, None, state[:, heads_state:], qkv, ctx.seg_of_row, ctx.seg_start, ctx.state_slots,
-                      gates=(proj[:, ch:ch + nh], self.dt_bias, self.a_log, step, decay), single_rows=ctx.decode_only)
-        ops.unit_heads(qkv[:, :2 * qk], 2 * self.kv_heads, self.dim, eps=self.unit_eps)
+                      gates=(proj[:, ch:ch + nh], self.dt_bias, self.a_log, step, decay), single_rows=ctx.decode_only,
+                      unit=(2 * self.kv_heads, self.dim, self.unit_eps) if fused else None)
+        if not fused:
+            ops.unit_heads(qkv[:, :2 * qk], 2 * self.kv_heads, self.dim, eps=self.unit_eps)
         o = ctx.buffer("delta.o", (T, inner), torch.float32)
         operands = (qkv[:, :qk], qkv[:, qk:2 * qk], qkv[:, 2 * qk:], decay, proj[:, ch + nh:ch + 2 * nh], o, state,
                     ctx.seg_start, ctx.state_slots, nh, self.dim, self.vdim)

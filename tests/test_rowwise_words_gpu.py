@@ -165,3 +165,33 @@ def test_layernorm_of_a_block_a_row_is_as_close_to_64_bits_as_of_a_wave_a_row(di
     error = lambda out: ((out.double() - want).norm() / want.norm()).item()
     few = torch.cat([ops.layernorm(part, w, torch.empty_like(part), 1e-5) for part in x.split(64)])
     assert error(few) <= 1.01 * error(ops.layernorm(x, w, torch.empty_like(x), 1e-5))
+
+
+@pytest.mark.parametrize("dim, heads, others", [(16, 3, 20), (32, 2, 0), (64, 5, 8), (128, 4, 260), (256, 3, 4), (128, 120, 10240), (64, 201, 13000)])
+def test_short_convolution_with_unit_heads(dim, heads, others):
+    """Heads whose results become unit vectors, beside channels that stay, in the kernels of few and of many inputs: against the unit vectors as a
+    kernel of their own.  A step of single rows gives the same."""
+    from runtime.kernels import ops
+    units, taps, gates_of = dim * heads, 4, 5
+    channels = units + others
+    for counts, single in (([1] * 7, True), ([40, 1, 90], False)):
+        T, n = sum(counts) + 2, len(counts)
+        seg, starts, slots = np.concatenate([np.repeat(np.arange(n), counts), [-1] * 2]), np.concatenate(([0], np.cumsum(counts))), list(range(n))[::-1]
+        wide = torch.randn(T, channels + 8, device=DEV)
+        x, dt = wide[:, :channels], wide[:, channels:channels + gates_of]
+        w, made = torch.randn(channels, taps, device=DEV), []
+        state = torch.randn(n, (taps - 1) * channels, device=DEV)
+        gate = torch.randn(gates_of, device=DEV)
+        for unit in ((heads, dim, 1e-6), None):
+            out, kept = torch.full((T, channels), 9.0, device=DEV), state.clone()
+            step, decay = (torch.full((T, gates_of), 9.0, device=DEV) for _ in range(2))
+            ops.conv_silu(x, w, None, kept, out, ints(seg), ints(starts), ints(slots), gates=(dt, gate, gate, step, decay), single_rows=single, unit=unit)
+            assert (out[-2:] == 9.0).all()               # (rows of no segment stay)
+            if unit is None:
+                ops.unit_heads(out[:, :units], heads, dim, eps=1e-6)
+            made.append((out[:-2], kept, step, decay))
+        # `dim` squares are added in another order, and a root taken: a few roundings
+        close(made[0][0][:, :units], made[1][0][:, :units].double(), 2e-6)
+        assert torch.equal(made[0][0][:, units:], made[1][0][:, units:]) and all(torch.equal(a, b) for a, b in zip(made[0][1:], made[1][1:]))
+    for bad in (8, 24, 512):
+        assert not ops.conv_unit_ok(bad)
