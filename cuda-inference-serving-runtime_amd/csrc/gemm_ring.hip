@@ -18,7 +18,7 @@ constexpr Tile TILES[] = {
     {128, 256, 7.9f, 0.859f, 0.780f},  {160, 256, 8.6f, 1.029f, 0.855f},  {192, 256, 9.1f, 1.228f, 1.228f},  {224, 256, 10.2f, 1.389f, 1.308f},
     {256, 256, 11.4f, 1.505f, 1.347f}, {288, 256, 12.3f, 1.665f, 1.395f},
 };
-constexpr int UNITS = 256, MOST_SLICES = 8, LEAST_STEPS = 4;
+constexpr int UNITS = 256, MOST_SLICES = 8, LEAST_STEPS = 4, NORMED_COLS = 1024;
 
 struct Plan { int tile, slices; float us; };
 
@@ -61,8 +61,16 @@ bool fits(const RingArgs& a, int out_bytes) {
            (!a.R || (a.ldr % 4 == 0 && (uintptr_t)a.R % 16 == 0)) && (long long)a.lda * 2 * 512 < 0x7fffffffll && reach < 0x7fffffffll;
 }
 
+// The rows A are what cisr_gemm_ring_normed leaves (sums null: they are normed).
+void finish_norm(RingArgs& a, const float* sums, int parts, float eps) {
+    a.sums = const_cast<float*>(sums); a.parts = parts; a.inv_k = 1.f / a.K; a.eps = eps;
+}
+
 int launch(const RingArgs& a, int tile, int mode, hipStream_t stream) {
     const int rows = tile / 1000, cols = tile % 1000;
+    if (a.sums && mode == RING_GATED) mode = RING_GATED_NORMED;
+    if (a.sums && mode == RING_ROPE) mode = RING_ROPE_NORMED;
+    if (a.sums && (mode == RING_FLOAT ? a.parts != (a.N + cols - 1) / cols : a.parts <= 0)) return (int)hipErrorInvalidValue;
     if (cols == 256 && rows >= 224) return cisr_ring_launch_a(a, tile, mode, stream);
     if (cols == 256 && rows >= 96) return cisr_ring_launch_b(a, tile, mode, stream);
     if (cols == 256 || (cols == 128 && rows >= 192)) return cisr_ring_launch_c(a, tile, mode, stream);
@@ -77,6 +85,27 @@ extern "C" int cisr_gemm_ring_slices(int M, int N, int K) {
     return plan_of(M, N, K, false, 0).slices;
 }
 
+// Sums a row that cisr_gemm_ring_normed leaves, or 0 where the product is better followed by the norm as a kernel of its own: where it is
+// best cut along its inner size, as the kernel that adds the slices makes the norm on the way, and in rows of more than NORMED_COLS.  The norm
+// of 1,000 to 2,000 rows is 5 us at any width below 2,048; without it the product before takes 1.3 us more at a width of 576 and
+// 2.7 at 2,048 (it stores the rows a second time), the one behind 1.1 and 4.5 (at 2,048 columns 288 x 256 tiles have 16 sums a row).
+extern "C" int cisr_gemm_ring_normed_parts(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % 4) return 0;
+    const Plan plan = plan_of(M, N, K, false, 0);
+    return plan.slices > 1 || N > NORMED_COLS ? 0 : (N + plan.tile % 1000 - 1) / (plan.tile % 1000);
+}
+
+// C += A . W^T (float), and what a product that finishes the RMSNorm of C's rows reads: `scaled` = bf16(C norm_w) and the sums of squares.
+extern "C" int cisr_gemm_ring_normed(const void* A, int lda, const void* W, int ldw, float* C, int ldc, const float* norm_w, void* scaled, int ldy,
+                                     float* sums, int parts, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, C, ldc, C, ldc, M, N, K, 0, GateLaw{}, 0, 1};
+    if (!fits(a, 4) || !norm_w || (uintptr_t)norm_w % 16 || !scaled || (uintptr_t)scaled % 8 || ldy < N || ldy % 4 || !sums)
+        return (int)hipErrorInvalidValue;
+    a.scaled = (bf16_t*)scaled; a.ldy = ldy; a.norm_w = norm_w; a.sums = sums; a.parts = parts;
+    return launch(a, plan_of(M, N, K, false, 1).tile, RING_FLOAT, stream);
+}
+
 // C = A . W^T, bf16 or float; R (float C only) is added, and may be C; `act` (bf16 C only): an ungated activation.  `tile` 0: the model's.
 extern "C" int cisr_gemm_ring_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* R, int ldr, int M, int N,
                                    int K, int out_dtype, int act, int tile, hipStream_t stream) {
@@ -87,12 +116,14 @@ extern "C" int cisr_gemm_ring_bf16(const void* A, int lda, const void* W, int ld
     return launch(a, tile ? tile : plan_of(M, N, K, false, 1).tile, wide ? RING_FLOAT : RING_STORE, stream);
 }
 
-// C = act(A . Wg^T, A . Wu^T), W = [Wg; Wu] with `dual_off` rows between the blocks; the law as GateLaw.
+// C = act(A . Wg^T, A . Wu^T), W = [Wg; Wu] with `dual_off` rows between the blocks; the law as GateLaw.  `sums` (else null): A's rows are
+// those of cisr_gemm_ring_normed, `parts` sums each, here and below.
 extern "C" int cisr_gemm_ring_bf16_gated(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N, int K, int dual_off,
-                                         float limit, float slope, float shift, int tile, hipStream_t stream) {
+                                         float limit, float slope, float shift, const float* sums, int parts, float eps, int tile, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    const RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, GateLaw{limit, slope, shift}, 0, 1};
+    RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, C, ldc, nullptr, 0, M, N, K, dual_off, GateLaw{limit, slope, shift}, 0, 1};
     if (!fits(a, 2) || dual_off < N) return (int)hipErrorInvalidValue;
+    finish_norm(a, sums, parts, eps);
     return launch(a, tile ? tile : plan_of(M, N, K, true, 1).tile, RING_GATED, stream);
 }
 
@@ -109,7 +140,8 @@ extern "C" int cisr_gemm_ring_partials_bf16(const void* A, int lda, const void* 
 // q into q_out (rows of ldq), k and v into the pages at `slots` (a negative one: nowhere); kv_heads 0: W = Wq only.
 extern "C" int cisr_gemm_ring_rope(const void* A, int lda, const void* W, int ldw, void* q_out, int ldq, int M, int K, const int* positions,
                                    const int* slots, const float* cos_tab, const float* sin_tab, void* kcache, void* vcache, int heads,
-                                   int kv_heads, int dim, int page_size, int max_pos, int tile, hipStream_t stream) {
+                                   int kv_heads, int dim, int page_size, int max_pos, const float* sums, int parts, float eps, int tile,
+                                   hipStream_t stream) {
     if (M <= 0 || heads <= 0) return 0;
     if (dim <= 0 || dim % 32 || kv_heads < 0 || max_pos <= 0 || !positions || !cos_tab || !sin_tab || (uintptr_t)cos_tab % 16 || (uintptr_t)sin_tab % 16 ||
         (kv_heads && (!slots || !kcache || !vcache || page_size <= 0 || (uintptr_t)kcache % 8)) || ldq < heads * dim)
@@ -117,6 +149,7 @@ extern "C" int cisr_gemm_ring_rope(const void* A, int lda, const void* W, int ld
     RingArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, q_out, ldq, nullptr, 0, M, heads * dim, K, 0, GateLaw{}, 0, 1,
                positions, slots, cos_tab, sin_tab, (bf16_t*)kcache, (bf16_t*)vcache, heads, kv_heads, dim, std::max(page_size, 1), max_pos};
     if (!fits(a, 2)) return (int)hipErrorInvalidValue;
+    finish_norm(a, sums, parts, eps);
     a.N = (heads + 2 * kv_heads) * dim;
     if (((long long)a.N + 512) * ldw * 2 >= 0x7fffffffll) return (int)hipErrorInvalidValue;
     return launch(a, tile ? tile : plan_of(M, a.N, K, false, 1).tile, RING_ROPE, stream);

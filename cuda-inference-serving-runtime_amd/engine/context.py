@@ -99,7 +99,19 @@ class StepContext:
 
     def add_product(self, a, w, residual):
         """residual += a . w^T, in place.  Where the product is cut along its inner size and the norm that reads the
-        residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer."""
+        residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer.  Where the part behind
+        that norm can finish it (`read_by`), only its weight is applied here."""
+        reader = getattr(self.next_norm, "read_by", None)
+        if reader:
+            parts = ops.ring_normed_parts(a, w, residual, self.next_norm.weight)
+            if parts:
+                rows = self.buffer("scaled.rows", residual.shape, torch.bfloat16)
+                if reader.takes_scaled(rows, self):
+                    # the norm rides in this product's epilogue and in its reader's: no kernel of its own
+                    sums = self.buffer("scaled.sums", (parts, rows.shape[0]), torch.float32)
+                    ops.gemm_ring_normed(a, w, residual, self.next_norm.weight, rows, sums)
+                    self.leave_normed(self.next_norm, residual, ops.ScaledRows(rows, sums, self.next_norm.eps))
+                    return residual
         if getattr(self.next_norm, "adds_partials", False):
             partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch, finish=True)
             if partials is ops.ADDED:

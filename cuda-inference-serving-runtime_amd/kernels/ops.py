@@ -61,8 +61,10 @@ def _declare(h):
         "cisr_gemm_ring_slices": [i, i, i],
         "cisr_add_rmsnorm_sums": [p, p, i, p, p, i, i, f, i, p],
         "cisr_gemm_ring_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, i, p],
-        "cisr_gemm_ring_bf16_gated": [p, i, p, i, p, i, i, i, i, i, f, f, f, i, p],
-        "cisr_gemm_ring_rope": [p, i, p, i, p, i, i, i, p, p, p, p, p, p, i, i, i, i, i, i, p],
+        "cisr_gemm_ring_bf16_gated": [p, i, p, i, p, i, i, i, i, i, f, f, f, p, i, f, i, p],
+        "cisr_gemm_ring_rope": [p, i, p, i, p, i, i, i, p, p, p, p, p, p, i, i, i, i, i, p, i, f, i, p],
+        "cisr_gemm_ring_normed_parts": [i, i, i],
+        "cisr_gemm_ring_normed": [p, i, p, i, p, i, p, p, i, p, i, i, i, i, p],
         "cisr_gemm_ring_partials_bf16": [p, i, p, i, p, i, i, i, i, i, p],
         "cisr_gemm_skinny_bf16": [p, i, p, i, p, i, p, i, i, i, i, i, i, p, f, p, p],
         "cisr_qkv_rope_skinny": [p, i, p, i, p, i, i, i, p, f, p, p, p, p, p, p, i, i, i, i, i, p],
@@ -755,6 +757,46 @@ def _ring_sums(at, m, n, k, make_buffer):
     return RingSums(parts, slices, m, n)
 
 
+class ScaledRows:
+    """Rows whose RMSNorm is left to the ring product that reads them (gemm_swiglu, qkv_rope): `rows` bf16 [M, K] = x times the norm's
+    weight, `sums` float [parts, M] the squares of x summed by tiles of columns."""
+
+    def __init__(self, rows, sums, eps):
+        self.rows, self.sums, self.eps = rows, sums, float(eps)
+
+    def args(self, m):
+        if self.rows.shape[0] != m or self.sums.dim() != 2 or self.sums.shape[1] != m:
+            raise KernelError("the sums belong to other rows")
+        return _dev(self.sums, "sums", torch.float32), self.sums.shape[0], self.eps
+
+
+def ring_normed_parts(a, w, residual, weight):
+    """How many sums a row gemm_ring_normed leaves, or 0 where it does not take these operands or the norm is better a kernel of its own:
+    a product that is best cut along its inner size, whose slices the norm's kernel adds, and rows of more than 1,024.  us of product,
+    norm and product behind it / of the two products: 1,777 x 576, K 576 then gate and up of 1,536 24.4 / 20.9, K 1,536 then 960 columns
+    with the rotation 22.5 / 20.2, 4,096 rows 36.9 / 35.0 and 33.5 / 31.9; 1,061 x 1,024, K 1,024 then gate and up of 4,096 38.0 / 35.9,
+    4,096 rows 91.3 / 90.6; 1,061 x 2,048, K 2,048 then gate and up of 8,192 86.3 / 86.4; cut ones 640 x 1,024, K 4,096 then 1,536 columns
+    25.2 / 25.3, 1,061 rows 33.4 / 35.0."""
+    (m, k), n = a.shape, w.shape[0]
+    if (w.dtype != torch.bfloat16 or m < RING_MIN_ROWS or m <= SKINNY_ROWS or tuple(residual.shape) != (m, n) or residual.dtype != torch.float32
+            or weight.dtype != torch.float32 or weight.data_ptr() % 16 or not ring_ahead(m, w, fused=True, cut=True)):
+        return 0
+    parts = int(lib().cisr_gemm_ring_normed_parts(m, n, k))
+    return parts if parts and _ring_operands(a, w, residual) is not None else 0
+
+
+def gemm_ring_normed(a, w, residual, weight, rows, sums):
+    """residual (float [M, N], in place) += a . w^T, rows (bf16 [M, N]) = residual weight, sums (float [ring_normed_parts, M]) = its squares
+    summed by tiles of columns: what the product behind an RMSNorm of that weight reads."""
+    (m, k), n = a.shape, w.shape[0]
+    at = _ring_operands(a, w, residual) if tuple(residual.shape) == (m, n) and w.shape[1] == k and residual.dtype == torch.float32 else None
+    if at is None or sums.dim() != 2 or sums.shape[1] != m:
+        raise KernelError("gemm_ring_normed: shape not supported")
+    _check(lib().cisr_gemm_ring_normed(*at, _dev(weight, "norm weight", torch.float32, (n,)), _dev(rows, "rows", torch.bfloat16, (m, n)), n,
+                                       _dev(sums, "sums", torch.float32), sums.shape[0], m, n, k, _stream()), "gemm_ring_normed")
+    return residual
+
+
 def gemm_ring(a, w, out, residual=None, act=0, tile=0):
     """out = a . w^T (+ residual, float rows that may be `out`) by the ring product; `act` (bf16 results): an ungated activation.
     `tile`: rows * 1000 + columns of a block (0: the fastest by the kernel's model of itself)."""
@@ -795,9 +837,9 @@ def gemm_ring_gated(a, w, out, law=None, tile=0):
     return _ring_gated(at, m, inter, k, out, law, tile)
 
 
-def _ring_gated(at, m, inter, k, out, law, tile=0):
+def _ring_gated(at, m, inter, k, out, law, tile=0, sums=(None, 0, 0.0)):
     lim, slope, shift = law or (0.0, 0.0, 0.0)
-    _check(lib().cisr_gemm_ring_bf16_gated(*at, m, inter, k, inter, float(lim), float(slope), float(shift), int(tile), _stream()),
+    _check(lib().cisr_gemm_ring_bf16_gated(*at, m, inter, k, inter, float(lim), float(slope), float(shift), *sums, int(tile), _stream()),
            "gemm_ring_gated")
     return out
 
@@ -1079,20 +1121,31 @@ def gemm_normed(x, norm, w, out):
 GELU_TANH_LAW = (-1.0, 0.0, 0.0)      # the law of gemm_swiglu and glu_clamped that gates by the tanh form of gelu
 
 
+def ring_gated_ok(a, w_gate_up, scratch=None):
+    """Whether gemm_swiglu takes the rows a, contiguous ones, to the ring product (into rows of its own)."""
+    return (a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and w_gate_up.shape[0] % 8 == 0 and _ring_open(scratch)
+            and ring_ahead(a.shape[0], w_gate_up, gated=True, library_rows=a.is_contiguous())
+            and w_gate_up.is_contiguous() and w_gate_up.data_ptr() % 16 == 0 and a.data_ptr() % 16 == 0 and a.is_contiguous()
+            and a.shape[1] % 64 == 0 and a.shape[1] * 1024 < 1 << 31 and (w_gate_up.shape[0] + 512) * a.shape[1] * 2 < 1 << 31)
+
+
 def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=None):
     """out[M, I] = silu(a . Wg^T) * (a . Wu^T) with w_gate_up = [Wg; Wu] ([2I, K]); with `law` = (limit, slope, shift)
     the activation is g sigmoid(slope g) (u + shift), g = min(gate, limit), u = clamp(up, -limit, limit) instead, or with
     GELU_TANH_LAW gelu(gate) u, the gelu's tanh form.
     Few rows of bf16 run one fused weight-streaming kernel (with `norm` = (weight, eps, None), `a` is the float
     residual and RMSNorm is fused too); otherwise the product goes to `gate_up` [M, 2I] and the activation is
-    a second kernel.  `scratch`: the ScratchPool of the caller's steps."""
+    a second kernel.  `a` a ScaledRows (where ring_gated_ok): the product finishes their norm.  `scratch`: the ScratchPool of the caller's steps."""
+    sums = None
+    if isinstance(a, ScaledRows):
+        a, sums = a.rows, a.args(a.rows.shape[0])
     m, k = a.shape
     two_i, k2 = w_gate_up.shape
     inter = two_i // 2
     if k != k2 or two_i % 2 or tuple(out.shape) != (m, inter) or not out.is_contiguous():
         raise KernelError("gemm_swiglu: shapes do not fit")
     if norm is not None:
-        if law is not None:
+        if law is not None or sums is not None:
             raise KernelError("gemm_swiglu: the fused norm comes with the silu law only")
         floats = w_gate_up.dtype == torch.float32
         wp, eps, rp, _ = _norm_args(a, norm, k, 4 if floats else 8)
@@ -1112,7 +1165,9 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
     if out.dtype != a.dtype or a.dtype != w_gate_up.dtype:
         raise KernelError("gemm_swiglu: dtypes differ")
     if a.dtype == torch.bfloat16 and _ring_open(scratch) and ring_ahead(m, w_gate_up, gated=True, library_rows=a.is_contiguous()) and (at := _ring_operands(a, w_gate_up, out)) is not None:
-        return _ring_gated(at, m, inter, k, out, law)
+        return _ring_gated(at, m, inter, k, out, law, sums=sums or (None, 0, 0.0))
+    if sums is not None:
+        raise KernelError("gemm_swiglu: rows without their norm's factor go to the ring product only")
     activate = swiglu if law is None else (lambda gu, o: glu_clamped(gu, o, *law))
     if a.dtype == torch.bfloat16 and library_ok(m, w_gate_up, gated=True) and a.is_contiguous():
         product = _scratch_bf16(scratch, a.device, m, two_i)
@@ -1215,7 +1270,10 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     """One kernel for a step's projections (few rows, the ring product, or 32 bits): (RMSNorm of the float residual `a` if `norm` = (weight, eps),
     else `a` is bf16 and normed), product with w = [Wq; Wk; Wv], rotary embedding of q and k, q into
     q_out [M, heads*dim], k and v into the cache at `slots`.  kcache None: w = Wq only (a layer reading
-    another layer's cache)."""
+    another layer's cache).  `a` a ScaledRows (where ring_rope_ok): the product finishes their norm."""
+    sums = None
+    if isinstance(a, ScaledRows):
+        a, sums = a.rows, a.args(a.rows.shape[0])
     if qkv_rope_f32_ok(a, w, dim, cos):
         return _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm)
     m, k = a.shape
@@ -1224,6 +1282,8 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     # (queries and key pages that are not on 8 bytes, or other tables: up to 64 rows the kernels of few rows)
     ring = (norm is None and _ring_open(scratch) and ring_rope_ok(a, w, dim, cos, sin) and q_out.data_ptr() % 8 == 0
             and (not has_kv or kcache.data_ptr() % 8 == 0))
+    if sums is not None and not ring:
+        raise KernelError("qkv_rope: rows without their norm's factor go to the ring product only")
     if (not (ring or (_few_rope_ok(a, w, dim, cos, False) if norm is None else qkv_rope_fused_ok(a, w, dim, cos, True)))
             or tuple(w.shape) != ((heads + 2 * n_kv) * dim, k)):
         raise KernelError("qkv_rope: shape not supported by the fused kernel")
@@ -1240,8 +1300,8 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     if ring:
         _check(lib().cisr_gemm_ring_rope(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), _dev(q_out, "q_out", torch.bfloat16, (m, heads * dim)),
                                          heads * dim, m, k, _dev(positions, "positions", torch.int32, (m,)), sp, _dev(cos, "cos", torch.float32),
-                                         _dev(sin, "sin", torch.float32, (max_pos, dim // 2)), kp, vp, heads, n_kv, dim, page_size, max_pos, 0,
-                                         _stream()), "qkv_rope")
+                                         _dev(sin, "sin", torch.float32, (max_pos, dim // 2)), kp, vp, heads, n_kv, dim, page_size, max_pos,
+                                         *(sums or (None, 0, 0.0)), 0, _stream()), "qkv_rope")
         return q_out
     if norm is None and wide_ok(m, w, after_norm=True):
         need = _wide_plan(m, w.shape[0], k, False)

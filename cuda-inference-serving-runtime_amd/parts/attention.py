@@ -91,6 +91,11 @@ class PagedAttention(Mixer):
     def fuses_norm(self, norm, residual, ctx):
         return getattr(norm, "fusable_as", None) == "rms" and self._fused_projection_ok(residual, True, ctx.scratch, norm.weight)
 
+    def takes_scaled(self, rows, ctx):
+        """Whether this step's projection of the rows `rows` can finish their norm (ops.ScaledRows)."""
+        cos, sin = self.position.tables()
+        return not (self._interleaved or self.bias) and ops._ring_open(ctx.scratch) and ops.ring_rope_ok(rows, self.w_in, self.head_dim, cos, sin)
+
     def forward(self, h, residual, ctx, site, norm=None):
         T = residual.shape[0]
         D, nh, nkv = self.head_dim, self.heads, self.kv_heads
@@ -101,7 +106,7 @@ class PagedAttention(Mixer):
             kcache_w = vcache_w = slots = None
         else:
             kcache_w, vcache_w, slots = kcache, vcache, view.slots
-        if norm is not None or self._fused_projection_ok(h, False, ctx.scratch):
+        if norm is not None or isinstance(h, ops.ScaledRows) or self._fused_projection_ok(h, False, ctx.scratch):
             # few rows (in 32 bits any number): norm, projections, rotary embedding and the cache write are one kernel
             q, q_stride = ctx.buffer("attn.q", (T, nh * D), ctx.dtype), nh * D
             ops.qkv_rope(residual if norm is not None else h, self.w_in, q, ctx.positions, slots, cos, sin,

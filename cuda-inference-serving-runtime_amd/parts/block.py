@@ -19,6 +19,9 @@ class PreNormBlock(Part):
         if (ffn is None) != (ffn_norm is None):
             raise ValueError("a feed-forward comes with the norm before it, or not at all")
         self.mixer_norm, self.mixer, self.ffn_norm, self.ffn = mixer_norm, mixer, ffn_norm, ffn
+        for norm, reader in ((mixer_norm, mixer), (ffn_norm, ffn)):
+            if getattr(norm, "fusable_as", None) == "rms" and hasattr(reader, "takes_scaled"):
+                norm.read_by = reader if getattr(norm, "read_by", None) in (None, reader) else False
 
     def parts(self):
         return [p for p in (self.mixer_norm, self.mixer, self.ffn_norm, self.ffn) if p is not None]
@@ -67,17 +70,23 @@ class PreNormBlock(Part):
             ctx.settle(residual)
             residual = self.mixer.forward(None, residual, ctx, site, norm=self.mixer_norm)
         else:
-            residual = self.mixer.forward(self.mixer_norm.forward(residual, ctx), residual, ctx, site)
+            residual = self.mixer.forward(self._normed(self.mixer_norm, residual, ctx), residual, ctx, site)
         if self.ffn is None:
             return residual
         if ffn_fuses:
             ctx.settle(residual)
             ctx.next_norm = after
             return self.ffn.forward(None, residual, ctx, norm=self.ffn_norm)
-        h = self.ffn_norm.forward(residual, ctx)
+        h = self._normed(self.ffn_norm, residual, ctx)
         ctx.settle(residual)       # (a norm that adds no partial sums)
         ctx.next_norm = after
         return self.ffn.forward(h, residual, ctx)
+
+    @staticmethod
+    def _normed(norm, residual, ctx):
+        """norm(residual), or the rows that the product before left for the part behind it to finish (ctx.add_product)."""
+        left = ctx.take_normed(norm, residual)
+        return left if isinstance(left, ops.ScaledRows) else norm.forward(residual, ctx)
 
 
 class NormedMean:

@@ -46,6 +46,10 @@ class GatedMLP(FeedForward):
     def fuses_norm(self, norm, residual, ctx):
         return not self.bias and self.law is None and getattr(norm, "fusable_as", None) == "rms" and ops.fused_norm_ok(residual, self.w_gate_up, residual.shape[0], norm.weight)
 
+    def takes_scaled(self, rows, ctx):
+        """Whether this step's product of the rows `rows` can finish their norm (ops.ScaledRows)."""
+        return not self.bias and ops.ring_gated_ok(rows, self.w_gate_up, ctx.scratch)
+
     def forward(self, h, residual, ctx, norm=None):
         T = residual.shape[0]
         act = ctx.buffer("ffn.act", (T, self.intermediate), ctx.dtype)
@@ -55,7 +59,7 @@ class GatedMLP(FeedForward):
             return ops.bias_add(ctx.add_product(act, self.w_down, residual), self.b_down)
         if norm is not None:
             ops.gemm_swiglu(residual, self.w_gate_up, act, norm=(norm.weight, norm.eps, None), scratch=ctx.scratch)
-        elif ops.swiglu_fused_ok(h, self.w_gate_up):
+        elif isinstance(h, ops.ScaledRows) or ops.swiglu_fused_ok(h, self.w_gate_up):
             ops.gemm_swiglu(h, self.w_gate_up, act, scratch=ctx.scratch, law=self.law)   # one kernel: product and activation
         else:
             ops.gemm_swiglu(h, self.w_gate_up, act, gate_up=ctx.buffer("ffn.gate_up", (T, 2 * self.intermediate), ctx.dtype),
