@@ -41,6 +41,33 @@ __device__ __forceinline__ float load_f32(const bf16_t* p) { return bf16_to_f32(
 __device__ __forceinline__ void store_f32(float* p, float v) { *p = v; }
 __device__ __forceinline__ void store_f32(bf16_t* p, float v) { *p = f32_to_bf16(v); }
 
+// V neighbouring elements as floats, by one load or store where V is 4 (16 bytes of floats, 8 of bf16, which the address is a multiple of)
+template <int V>
+__device__ __forceinline__ void load_run(const float* p, float (&v)[V]) {
+    if constexpr (V == 4) { const float4 w = *(const float4*)p; v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w; }
+    else for (int i = 0; i < V; ++i) v[i] = p[i];
+}
+template <int V>
+__device__ __forceinline__ void load_run(const bf16_t* p, float (&v)[V]) {
+    if constexpr (V == 4) {
+        const uint2 w = *(const uint2*)p;
+        v[0] = __uint_as_float(w.x << 16); v[1] = __uint_as_float(w.x & 0xffff0000u);
+        v[2] = __uint_as_float(w.y << 16); v[3] = __uint_as_float(w.y & 0xffff0000u);
+    } else {
+        for (int i = 0; i < V; ++i) v[i] = load_f32(p + i);
+    }
+}
+template <int V>
+__device__ __forceinline__ void store_run(float* p, const float (&v)[V]) {
+    if constexpr (V == 4) *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    else for (int i = 0; i < V; ++i) p[i] = v[i];
+}
+template <int V>
+__device__ __forceinline__ void store_run(bf16_t* p, const float (&v)[V]) {
+    if constexpr (V == 4) *(uint2*)p = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    else for (int i = 0; i < V; ++i) store_f32(p + i, v[i]);
+}
+
 // 1 / sqrt(total inv_k + eps), a row's factor in an RMSNorm that a product finishes: the approximate reciprocal root and one step of
 // Newton's (within 1 unit in the last place; the library's quotient, root and quotient round three times, and as the last thing that a
 // short kernel does are 0.07 us: one row x 3,072 gated, K 576 4.15 -> 4.07 us, x 960 with the rotation 3.38 -> 3.31).

@@ -7,24 +7,30 @@
 
 // ---------------------------------------------------------------- embedding
 // out[r, :] = table[ids[r], :]  (reference: kernels/execution.cu:2-5)
-template <typename T>
-__global__ void embedding_kernel(const int* __restrict__ ids, const T* __restrict__ table,
-                                 float* __restrict__ out, int dim, int vocab) {
-    const int row = blockIdx.x;
+// Bound by two trips to memory, the id's and the row's: a thread a word of V elements (four, or one where the rows are not aligned for that),
+// so that no thread goes round.  Eight rows of 2,048 bf16 in a captured step 5.8 -> 4.1 us (256 threads a row
+// that went round), one of 576 2.9 -> 2.3, 2,345 of 2,048 14.5 -> 11.8.
+template <typename T, int V>
+__global__ void __launch_bounds__(256)
+embedding_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int dim, int vocab) {
+    const int row = blockIdx.x, at = (blockIdx.y * 256 + threadIdx.x) * V;
+    if (at >= dim) return;
     int id = ids[row];
     if (id < 0 || id >= vocab) id = 0;  // padding rows; real ids are checked on the host
-    const T* src = table + (size_t)id * dim;
-    float* dst = out + (size_t)row * dim;
-    for (int d = threadIdx.x; d < dim; d += blockDim.x) dst[d] = load_f32(src + d);
+    float v[V];
+    load_run<V>(table + (size_t)id * dim + at, v);
+    store_run<V>(out + (size_t)row * dim + at, v);
 }
 
 extern "C" int cisr_embedding(const int* ids, const void* table, float* out, int rows, int dim,
                               int vocab, int dtype, hipStream_t stream) {
     if (rows <= 0) return 0;
-    if (dtype == DT_F32)
-        embedding_kernel<float><<<rows, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
-    else
-        embedding_kernel<bf16_t><<<rows, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
+    const bool wide = dim % 4 == 0 && (uintptr_t)table % (dtype == DT_F32 ? 16 : 8) == 0 && (uintptr_t)out % 16 == 0;
+    const dim3 grid(rows, (wide ? dim / 4 + 255 : dim + 255) / 256);
+    if (dtype == DT_F32 && wide) embedding_kernel<float, 4><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
+    else if (dtype == DT_F32) embedding_kernel<float, 1><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
+    else if (wide) embedding_kernel<bf16_t, 4><<<grid, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
+    else embedding_kernel<bf16_t, 1><<<grid, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
     return CISR_LAUNCH_CHECK();
 }
 

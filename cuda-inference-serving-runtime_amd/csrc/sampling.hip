@@ -66,22 +66,31 @@ argmax_partial_kernel(const float* __restrict__ logits, float* __restrict__ pval
     }
 }
 
+// A lane a slice.  (A row that begins with NaN is that place's: nothing compares greater, as in a walk from the first slice on.)  One
+// lane walking the slices: 4.0 us in a captured step of 8 rows, 2.8 so.
+#define ARGMAX_CHUNKS 32
 __global__ void __launch_bounds__(64)
 argmax_final_kernel(const float* __restrict__ pval, const int* __restrict__ pidx, int* __restrict__ out,
-                    const int* __restrict__ index, int out_n, int chunks) {
-    const int row = blockIdx.x;
-    if (threadIdx.x != 0) return;
+                    const int* __restrict__ index, int out_n) {
+    const int row = blockIdx.x, lane = threadIdx.x, at = row * ARGMAX_CHUNKS + lane % ARGMAX_CHUNKS;
     const int dst = index ? index[row] : row;
-    if (dst < 0 || dst >= out_n) return;
-    float bv = -INFINITY; int bi = 0x7fffffff;
-    for (int c = 0; c < chunks; ++c) {
-        const float v = pval[row * chunks + c]; const int i = pidx[row * chunks + c];
-        if (i != 0x7fffffff && (bi == 0x7fffffff || v > bv)) { bv = v; bi = i; }
+    float v = pval[at];
+    int i = lane < ARGMAX_CHUNKS ? pidx[at] : 0x7fffffff;
+    const unsigned long long some = __ballot(i != 0x7fffffff);
+    const int first = some ? __ffsll((long long)some) - 1 : 0;
+    const float at_first = __shfl(v, first, WAVE);
+    const int i_first = __shfl(i, first, WAVE);
+    if (v != v) i = 0x7fffffff;
+#pragma unroll
+    for (int off = 1; off < ARGMAX_CHUNKS; off *= 2) {
+        const float ov = __shfl_xor(v, off, WAVE);
+        const int oi = __shfl_xor(i, off, WAVE);
+        if (oi != 0x7fffffff && (i == 0x7fffffff || ov > v || (ov == v && oi < i))) { v = ov; i = oi; }
     }
-    out[dst] = bi == 0x7fffffff ? 0 : bi;
+    if (at_first != at_first) i = i_first;
+    if (lane == 0 && dst >= 0 && dst < out_n) out[dst] = i == 0x7fffffff ? 0 : i;
 }
 
-#define ARGMAX_CHUNKS 32
 
 // scratch: float [rows * 32] and int [rows * 32].  With `index`, row r's token goes to out[index[r]]
 // (nowhere if that is outside 0..out_n-1) instead of out[r]; without, out_n is rows.
@@ -91,7 +100,7 @@ extern "C" int cisr_argmax(const float* logits, int* out, const int* index, int 
     argmax_partial_kernel<<<dim3(rows, ARGMAX_CHUNKS), 256, 0, stream>>>(logits, scratch_val, scratch_idx, vocab, ARGMAX_CHUNKS);
     int err = CISR_LAUNCH_CHECK();
     if (err) return err;
-    argmax_final_kernel<<<rows, 64, 0, stream>>>(scratch_val, scratch_idx, out, index, index ? out_n : rows, ARGMAX_CHUNKS);
+    argmax_final_kernel<<<rows, 64, 0, stream>>>(scratch_val, scratch_idx, out, index, index ? out_n : rows);
     return CISR_LAUNCH_CHECK();
 }
 
@@ -143,7 +152,7 @@ extern "C" int cisr_argmax_noalloc(const float* logits, int* out, int rows, int 
     argmax_partial_kernel<<<dim3(rows, ARGMAX_CHUNKS), 256, 0, stream>>>(logits, pval, pidx, vocab, ARGMAX_CHUNKS);
     err = CISR_LAUNCH_CHECK();
     if (err) return err;
-    argmax_final_kernel<<<rows, 64, 0, stream>>>(pval, pidx, out, nullptr, rows, ARGMAX_CHUNKS);
+    argmax_final_kernel<<<rows, 64, 0, stream>>>(pval, pidx, out, nullptr, rows);
     return CISR_LAUNCH_CHECK();
 }
 

@@ -65,6 +65,22 @@ def test_embedding(ops, dtype):
     np.testing.assert_array_equal(f64(out), f64(table)[ids.cpu().numpy()])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim, offset", [(1, 0), (4, 0), (576, 0), (576, 1), (1023, 0), (1028, 0), (2048, 2), (4100, 0)])
+def test_embedding_by_words_and_by_elements(ops, dtype, dim, offset):
+    """Rows of one word and more than a block's; tables between words (and their pairs, with the copy in the activations' type)."""
+    table, pairs = (rnd(9 * dim + offset, dtype=dtype, seed=s)[offset:].view(9, dim) for s in (1, 2))
+    ids = torch.tensor([0, 8, 5, 5, -1], dtype=torch.int32, device=DEV)
+    rows = ids.clamp(min=0).long()
+    assert torch.equal(ops.embedding(ids, table, torch.empty(5, dim, device=DEV)), table[rows].float())
+    zeros, starts = torch.zeros(5, dtype=torch.int32, device=DEV), torch.arange(6, dtype=torch.int32, device=DEV)
+    cast, kept = torch.empty(5, dim, dtype=dtype, device=DEV), torch.zeros(5, dtype=torch.int32, device=DEV)
+    out = ops.embedding_pairs(ids, zeros, starts[:5], starts, starts[:5], table, torch.empty(5, dim, device=DEV), scale=2.0, pairs=pairs,
+                              last_token=kept, buckets=8, mul_prev=3, mul_cur=5, cast=cast, single_rows=True)
+    want = table[rows].float() * 2.0 + pairs[8].float()          # (a doubled value is exact, so the sum is rounded once either way)
+    assert torch.equal(out, want) and torch.equal(cast, want.to(dtype)) and torch.equal(kept, rows.int())
+
+
 @pytest.mark.parametrize("dim", [10, 64, 130, 576, 2048, 4100, 8200])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_rmsnorm(ops, dim, out_dtype):
@@ -1252,6 +1268,20 @@ def test_argmax_lowest_index_wins(ops):
     want = f64(logits).argmax(-1)
     np.testing.assert_array_equal(out, want)
     assert out[1] == 17 and out[2] == 0 and out[3] == 1002
+
+
+@pytest.mark.parametrize("vocab", [1, 5, 31, 33, 49152])
+def test_argmax_over_slices_with_ties_and_without_a_number(ops, vocab):
+    """Fewer logits than slices, ties between slices, rows of -inf; a row that begins with NaN is that place's."""
+    z = rnd(6, vocab, seed=vocab)
+    z[0] = -float("inf")
+    z[1, vocab // 2:] = 7.0
+    z[2, 0] = float("nan")
+    z[3, -1] = float("inf")
+    z[4] = 0.0
+    z[4, vocab // 3:] = -0.0
+    got = ops.argmax(z, torch.empty(6, dtype=torch.int32, device=DEV)).tolist()
+    assert got == [0, vocab // 2, 0, vocab - 1, 0, int(f64(z)[5].argmax())]
 
 
 def test_token_choices_scattered_by_index_and_taken_back(ops):
