@@ -72,6 +72,7 @@ class StepContext:
         # part that was told it may (`next_norm`), taken by the norm that reads the rows next (or settled)
         self.unfinished = None
         self.next_norm = None     # the norm that reads the residual stream after the block that runs now, if known
+        self.running = None       # the part that a block runs now, if the block and who runs it add nothing to the stream behind that part
         self.normed = None        # (norm part, residual rows, normed rows): a block made its follower's first norm on the way
         self.layer_tap = getattr(runner, "layer_tap", None)   # callable(schedule index, residual rows) after every layer run, or None
         self.capturing = False    # the step is being recorded into a graph: launches only
@@ -97,11 +98,13 @@ class StepContext:
             self.runner.carry(array)
         return got
 
-    def add_product(self, a, w, residual):
+    def add_product(self, a, w, residual, last=None):
         """residual += a . w^T, in place.  Where the product is cut along its inner size and the norm that reads the
-        residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer.  Where the part behind
-        that norm can finish it (`read_by`), only its weight is applied here."""
-        reader = getattr(self.next_norm, "read_by", None)
+        residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer.  A caller may add more to the
+        residual afterwards, as sums commute; one that does not names itself (`last`: the part whose last addition this is), and if the
+        block that runs it adds nothing either (`running`) and the part behind the norm can finish it (`read_by`), the norm is taken of the
+        rows as they are now: only its weight is applied here."""
+        reader = getattr(self.next_norm, "read_by", None) if last is not None and last is self.running else None
         if reader:
             parts = ops.ring_normed_parts(a, w, residual, self.next_norm.weight)
             if parts:

@@ -91,6 +91,12 @@ class FeedForward(Part):
         raise NotImplementedError
 
 
+def runs_own(part, cls):
+    """Whether `part.forward` is what `cls` defines.  A subclass's or a wrapper's may read its rows otherwise, or add to the residual
+    stream behind what it takes from `cls`."""
+    return getattr(part.forward, "__func__", None) is cls.forward
+
+
 class _Cast:
     """Stands where a norm would in StepContext.leave_normed / take_normed for "the rows themselves in the activations'
     type": whoever writes the residual stream (an embedding, a block that norms after the sum) may leave that copy for

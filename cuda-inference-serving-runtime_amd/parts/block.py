@@ -10,7 +10,7 @@ with weights that read, mix and write them around every sublayer."""
 import torch
 
 from ..kernels import ops
-from .base import CAST, Part, TensorSpec, matrix_operand, register_part
+from .base import CAST, Part, TensorSpec, matrix_operand, register_part, runs_own
 
 
 class PreNormBlock(Part):
@@ -66,21 +66,24 @@ class PreNormBlock(Part):
         after = ctx.next_norm
         ffn_fuses = self.ffn is not None and self.ffn.fuses_norm(self.ffn_norm, residual, ctx)
         ctx.next_norm = after if self.ffn is None else None if ffn_fuses else self.ffn_norm
+        # (behind the block's last part an arrangement made of this one may add to the stream, and whoever looks at it may change it)
+        untouched = runs_own(self, PreNormBlock) and ctx.layer_tap is None
+        ctx.running = self.mixer if self.ffn is not None or untouched else None
         if self.mixer.fuses_norm(self.mixer_norm, residual, ctx):
             ctx.settle(residual)
             residual = self.mixer.forward(None, residual, ctx, site, norm=self.mixer_norm)
         else:
             residual = self.mixer.forward(self._normed(self.mixer_norm, residual, ctx), residual, ctx, site)
+        ctx.running = None
         if self.ffn is None:
             return residual
-        if ffn_fuses:
-            ctx.settle(residual)
-            ctx.next_norm = after
-            return self.ffn.forward(None, residual, ctx, norm=self.ffn_norm)
-        h = self._normed(self.ffn_norm, residual, ctx)
+        h = None if ffn_fuses else self._normed(self.ffn_norm, residual, ctx)
         ctx.settle(residual)       # (a norm that adds no partial sums)
         ctx.next_norm = after
-        return self.ffn.forward(h, residual, ctx)
+        ctx.running = self.ffn if untouched else None
+        residual = self.ffn.forward(h, residual, ctx, norm=self.ffn_norm) if ffn_fuses else self.ffn.forward(h, residual, ctx)
+        ctx.running = None
+        return residual
 
     @staticmethod
     def _normed(norm, residual, ctx):

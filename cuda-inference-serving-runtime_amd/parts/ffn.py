@@ -5,7 +5,7 @@ the products run as they are and a small kernel adds the bias (no fused activati
 import torch
 
 from ..kernels import ops
-from .base import FeedForward, TensorSpec, matrix_operand, register_part
+from .base import FeedForward, TensorSpec, matrix_operand, register_part, runs_own
 
 
 class GatedMLP(FeedForward):
@@ -56,7 +56,7 @@ class GatedMLP(FeedForward):
         if self.bias:
             gate_up = ops.gemm(h, self.w_gate_up, ctx.buffer("ffn.gate_up", (T, 2 * self.intermediate), ctx.dtype), scratch=ctx.scratch)
             ops.swiglu(ops.bias_add(gate_up, self.b_gate_up), act)
-            return ops.bias_add(ctx.add_product(act, self.w_down, residual), self.b_down)
+            return ops.bias_add(ctx.add_product(act, self.w_down, residual), self.b_down)      # (more follows the product: no `last`)
         if norm is not None:
             ops.gemm_swiglu(residual, self.w_gate_up, act, norm=(norm.weight, norm.eps, None), scratch=ctx.scratch)
         elif isinstance(h, ops.ScaledRows) or ops.swiglu_fused_ok(h, self.w_gate_up):
@@ -64,7 +64,7 @@ class GatedMLP(FeedForward):
         else:
             ops.gemm_swiglu(h, self.w_gate_up, act, gate_up=ctx.buffer("ffn.gate_up", (T, 2 * self.intermediate), ctx.dtype),
                             scratch=ctx.scratch, law=self.law)
-        return ctx.add_product(act, self.w_down, residual)
+        return ctx.add_product(act, self.w_down, residual, last=self if runs_own(self, GatedMLP) else None)
 
     def output(self, h, ctx, tag="ffn", unfinished=False):
         """The feed-forward's result, float [T, hidden], without the residual sum (no biases); `unfinished`: it may be
@@ -172,7 +172,7 @@ class DenseMLP(FeedForward):
         if self.bias:
             from .block import add_sublayer
             return add_sublayer(residual, self.output(h, ctx), None, 1.0)
-        return ctx.add_product(self._activations(h, ctx), self.w_down, residual)
+        return ctx.add_product(self._activations(h, ctx), self.w_down, residual, last=self if runs_own(self, DenseMLP) else None)
 
 
 class RoutedExperts(FeedForward):

@@ -1,0 +1,170 @@
+"""Who may finish whose norm: the rules by which a block leaves the norm between two products to the products themselves, with the
+kernels' places taken by torch on the CPU."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+ROWS, WIDTH = 6, 8
+
+
+@pytest.fixture
+def ctx(monkeypatch):
+    """A step context whose products always may leave the next norm."""
+    from runtime.engine.context import StepContext, Workspace
+    from runtime.kernels import ops
+
+    def gemm(a, w, out, residual=None, scratch=None):
+        return out.copy_(a.float() @ w.float().T + (0.0 if residual is None else residual))
+
+    def normed_product(a, w, residual, weight, rows, sums):
+        gemm(a, w, residual, residual)
+        rows.copy_(residual * weight)
+        sums.copy_((residual * residual).sum(1)[None])
+        return residual
+
+    def rmsnorm(x, weight, out, eps, rows=None):
+        return out.copy_(x * torch.rsqrt((x * x).mean(1, keepdim=True) + eps) * weight)
+    for name, fake in (("gemm", gemm), ("gemm_ring_normed", normed_product), ("rmsnorm", rmsnorm), ("ring_normed_parts", lambda *a: 1),
+                       ("gemm_unfinished", lambda *a, **k: None), ("swiglu_fused_ok", lambda *a: True), ("gemm_swiglu", lambda h, w, out, **k: out.zero_())):
+        monkeypatch.setattr(ops, name, fake)
+    runner = SimpleNamespace(cache=None, model=SimpleNamespace(dtype=torch.bfloat16), device="cpu", scratch=None, workspace=Workspace("cpu"))
+    return StepContext(runner)
+
+
+def weights(seed):
+    return torch.randn(WIDTH, WIDTH, generator=torch.Generator().manual_seed(seed)).bfloat16()
+
+
+def rms(seed):
+    from runtime.parts import RMSNorm
+    norm = RMSNorm("n", WIDTH, 1e-5)
+    norm.weight = 1.0 + 0.3 * torch.randn(WIDTH, generator=torch.Generator().manual_seed(seed))
+    return norm
+
+
+def read(part, h):
+    """What a toy part does with the rows that it is given: their normed form, kept in `got`, and what they were, in `kinds`."""
+    from runtime.kernels import ops
+    part.kinds.append(type(h).__name__)
+    if isinstance(h, ops.ScaledRows):
+        h = h.rows.float() * torch.rsqrt(h.sums.sum(0)[:, None] / WIDTH + h.eps)
+    part.got.append(h.float().clone())
+    return h.bfloat16()
+
+
+def toys():
+    """A mixer and a feed-forward that end with a product and can finish the norm of their rows; with `after` they add that behind the product
+    and do not say that it is the last."""
+    from runtime.parts.base import FeedForward, Mixer
+
+    class Toy:
+        def __init__(self, seed, after=0.0):
+            self.w, self.after, self.got, self.kinds = weights(seed), after, [], []
+
+        def takes_scaled(self, rows, ctx):
+            return True
+
+        def forward(self, h, residual, ctx, *site, norm=None):
+            residual = ctx.add_product(read(self, h), self.w, residual, **({} if self.after else {"last": self}))
+            return residual.add_(self.after) if self.after else residual
+    return type("ToyMixer", (Toy, Mixer), {}), type("ToyFFN", (Toy, FeedForward), {})
+
+
+def run(ctx, layers, tap=None):
+    """Runs the layers as a model does; returns the rows after them and the normed rows that every sublayer should have read."""
+    from runtime.models import Model
+    torch.manual_seed(0)
+    x = torch.randn(ROWS, WIDTH)
+    ctx.layer_tap = tap
+    ctx.logit_rows = torch.empty(0)
+    model = Model(None, SimpleNamespace(forward=lambda c: x), layers, None, None, max_positions=1, vocab_size=1)
+    model.forward(ctx)
+    return x
+
+
+def close(part, want):
+    # (bf16 rows, rounded before the factor or after it)
+    return len(part.got) == 1 and ((part.got[0] - want).abs() <= 0.01 * want.abs() + 1e-6).all()
+
+
+def norm_of(norm, x):
+    return x * torch.rsqrt((x * x).mean(1, keepdim=True) + norm.eps) * norm.weight
+
+
+def layers_of(n, block=None, mixer=None, ffn=None, after={}):
+    from runtime.parts import PreNormBlock
+    ToyMixer, ToyFFN = toys()
+    return [(block or PreNormBlock)(rms(i), (mixer or ToyMixer)(10 + i, after.get("mixer", 0.0)), rms(20 + i), (ffn or ToyFFN)(30 + i, after.get("ffn", 0.0)))
+            for i in range(n)]
+
+
+def watch(blocks):
+    """What every sublayer should read, found when it runs: [(part, normed rows)]."""
+    seen = []
+    for block in blocks:
+        for part, norm in ((block.mixer, block.mixer_norm), (block.ffn, block.ffn_norm)):
+            def spy(h, residual, *rest, part=part, norm=norm, real=part.forward, **kw):
+                seen.append((part, norm_of(norm, residual)))
+                return real(h, residual, *rest, **kw)
+            part.forward = spy
+    return seen
+
+
+def right(seen, count):
+    return len(seen) == count and all(close(part, want) for part, want in seen)
+
+
+def kinds(blocks):
+    return [part.kinds for block in blocks for part in (block.mixer, block.ffn)]
+
+
+def test_parts_that_end_with_their_product_leave_the_next_norm(ctx):
+    blocks = layers_of(2)
+    seen = watch(blocks)
+    run(ctx, blocks)
+    assert right(seen, 4) and kinds(blocks) == [["Tensor"], ["ScaledRows"], ["ScaledRows"], ["ScaledRows"]]
+
+
+@pytest.mark.parametrize("which", ["mixer", "ffn"])
+def test_what_a_part_adds_behind_its_product_is_in_the_next_norm(ctx, which):
+    """A part that adds to the rows after its last product: sums commute with a product left unfinished, not with a norm taken already."""
+    blocks = layers_of(2, after={which: 0.7})
+    seen = watch(blocks)
+    run(ctx, blocks)
+    assert right(seen, 4)
+
+
+def test_what_others_add_behind_a_part_is_in_the_next_norm(ctx):
+    """A mixer around another one, an arrangement made of the pre-norm one, and a caller that looks at the rows between two layers."""
+    from runtime.parts import GatedMLP, PreNormBlock
+    ToyMixer, ToyFFN = toys()
+
+    class Around(ToyMixer):
+        def __init__(self, seed, after):
+            super().__init__(seed, after)
+            self.inner, self.kinds = ToyMixer(seed), []
+            self.got = self.inner.got
+
+        def forward(self, h, residual, ctx, *site, norm=None):
+            return self.inner.forward(h, residual, ctx, *site).add_(0.7)
+
+    class More(PreNormBlock):
+        def forward(self, residual, ctx, site):
+            return super().forward(residual, ctx, site).mul_(0.5)
+    for blocks, tap in ((layers_of(2, mixer=Around), None), (layers_of(2, block=More), None), (layers_of(2), lambda index, x: x.mul_(0.5))):
+        seen = watch(blocks)
+        run(ctx, blocks, tap)
+        assert right(seen, 4)
+
+    class Halved(GatedMLP):
+        def forward(self, h, residual, ctx, norm=None):
+            return super().forward(h, residual, ctx, norm=norm).mul_(0.5)
+    asked = []
+    ctx.add_product = lambda a, w, residual, last=None: (asked.append(last), residual)[1]
+    for cls in (GatedMLP, Halved):
+        part = cls("m", WIDTH, WIDTH)
+        part.w_gate_up, part.w_down = torch.cat([weights(1), weights(2)]), weights(3)
+        part.forward(torch.zeros(ROWS, WIDTH).bfloat16(), torch.zeros(ROWS, WIDTH), ctx)
+        asked[-1] = asked[-1] is part
+    assert asked == [True, False]
