@@ -72,7 +72,10 @@ class StepContext:
         # part that was told it may (`next_norm`), taken by the norm that reads the rows next (or settled)
         self.unfinished = None
         self.next_norm = None     # the norm that reads the residual stream after the block that runs now, if known
-        self.running = None       # the part that a block runs now, if the block and who runs it add nothing to the stream behind that part
+        # (part, norm, reader): `part` runs now, nothing is added to the stream behind it, and `reader`, which may finish norms (`takes_scaled`),
+        # reads norm(stream) next.  Set by a block around its parts; the model sets `following` = (layer that runs now, (norm, reader) of the next)
+        self.hand_over = self.following = None
+        self.scaled = None        # (norm, reader, residual rows, ops.ScaledRows): what add_product left for `reader` to finish
         self.normed = None        # (norm part, residual rows, normed rows): a block made its follower's first norm on the way
         self.layer_tap = getattr(runner, "layer_tap", None)   # callable(schedule index, residual rows) after every layer run, or None
         self.capturing = False    # the step is being recorded into a graph: launches only
@@ -102,18 +105,19 @@ class StepContext:
         """residual += a . w^T, in place.  Where the product is cut along its inner size and the norm that reads the
         residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer.  A caller may add more to the
         residual afterwards, as sums commute; one that does not names itself (`last`: the part whose last addition this is), and if the
-        block that runs it adds nothing either (`running`) and the part behind the norm can finish it (`read_by`), the norm is taken of the
+        block that runs it adds nothing either and knows a reader that can finish the norm behind it (`hand_over`), the norm is taken of the
         rows as they are now: only its weight is applied here."""
-        reader = getattr(self.next_norm, "read_by", None) if last is not None and last is self.running else None
-        if reader:
-            parts = ops.ring_normed_parts(a, w, residual, self.next_norm.weight)
+        self.scaled = None
+        if last is not None and self.hand_over is not None and self.hand_over[0] is last:
+            _, norm, reader = self.hand_over
+            parts = ops.ring_normed_parts(a, w, residual, norm.weight)
             if parts:
                 rows = self.buffer("scaled.rows", residual.shape, torch.bfloat16)
                 if reader.takes_scaled(rows, self):
                     # the norm rides in this product's epilogue and in its reader's: no kernel of its own
                     sums = self.buffer("scaled.sums", (parts, rows.shape[0]), torch.float32)
-                    ops.gemm_ring_normed(a, w, residual, self.next_norm.weight, rows, sums)
-                    self.leave_normed(self.next_norm, residual, ops.ScaledRows(rows, sums, self.next_norm.eps))
+                    ops.gemm_ring_normed(a, w, residual, norm.weight, rows, sums)
+                    self.scaled = (norm, reader, residual, ops.ScaledRows(rows, sums, norm.eps))
                     return residual
         if getattr(self.next_norm, "adds_partials", False):
             partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch, finish=True)
@@ -156,6 +160,14 @@ class StepContext:
         got, self.normed = self.normed, None
         if got is not None and got[0] is norm and got[1].data_ptr() == rows.data_ptr():
             return got[2]
+        return None
+
+    def take_scaled(self, norm, reader, rows):
+        """The rows whose norm the product before left to `reader` (ops.ScaledRows), for the block that gives norm(rows) to it; else None (the
+        residual rows themselves are whole either way)."""
+        got, self.scaled = self.scaled, None
+        if got is not None and got[0] is norm and got[1] is reader and got[2].data_ptr() == rows.data_ptr():
+            return got[3]
         return None
 
     def settle(self, rows):

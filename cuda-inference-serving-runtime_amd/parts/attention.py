@@ -94,7 +94,7 @@ class PagedAttention(Mixer):
     def takes_scaled(self, rows, ctx):
         """Whether this step's projection of the rows `rows` can finish their norm (ops.ScaledRows)."""
         cos, sin = self.position.tables()
-        return not (self._interleaved or self.bias) and ops._ring_open(ctx.scratch) and ops.ring_rope_ok(rows, self.w_in, self.head_dim, cos, sin)
+        return runs_own(self, PagedAttention) and not (self._interleaved or self.bias) and ops._ring_open(ctx.scratch) and ops.ring_rope_ok(rows, self.w_in, self.head_dim, cos, sin)
 
     def forward(self, h, residual, ctx, site, norm=None):
         T = residual.shape[0]

@@ -19,9 +19,6 @@ class PreNormBlock(Part):
         if (ffn is None) != (ffn_norm is None):
             raise ValueError("a feed-forward comes with the norm before it, or not at all")
         self.mixer_norm, self.mixer, self.ffn_norm, self.ffn = mixer_norm, mixer, ffn_norm, ffn
-        for norm, reader in ((mixer_norm, mixer), (ffn_norm, ffn)):
-            if getattr(norm, "fusable_as", None) == "rms" and hasattr(reader, "takes_scaled"):
-                norm.read_by = reader if getattr(norm, "read_by", None) in (None, reader) else False
 
     def parts(self):
         return [p for p in (self.mixer_norm, self.mixer, self.ffn_norm, self.ffn) if p is not None]
@@ -60,36 +57,47 @@ class PreNormBlock(Part):
         """The norm that reads the residual stream first: the block before may leave its last product to it."""
         return self.mixer_norm
 
+    def first_reader(self):
+        """(That norm, the part that reads its rows): the block before may leave the norm to that part."""
+        return self.mixer_norm, self.mixer
+
     def forward(self, residual, ctx, site):
         # ctx.next_norm names the norm that reads the residual stream after the part that runs: a part's last
         # product may be left to it (ctx.add_product); on entry it is the norm after this block
-        after = ctx.next_norm
+        after, following = ctx.next_norm, None
+        # behind this block's last part someone else may add to the stream: an arrangement made of it or around it, a caller that looks at the rows
+        if ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock) and ctx.layer_tap is None:
+            following = ctx.following[1]
         ffn_fuses = self.ffn is not None and self.ffn.fuses_norm(self.ffn_norm, residual, ctx)
+        inside = (self.ffn_norm, self.ffn) if self.ffn is not None and not ffn_fuses else None
         ctx.next_norm = after if self.ffn is None else None if ffn_fuses else self.ffn_norm
-        # (behind the block's last part an arrangement made of this one may add to the stream, and whoever looks at it may change it)
-        untouched = runs_own(self, PreNormBlock) and ctx.layer_tap is None
-        ctx.running = self.mixer if self.ffn is not None or untouched else None
-        if self.mixer.fuses_norm(self.mixer_norm, residual, ctx):
+        h = ctx.take_scaled(self.mixer_norm, self.mixer, residual)
+        ctx.hand_over = self._hand_over(self.mixer, following if self.ffn is None else inside)
+        if h is None and self.mixer.fuses_norm(self.mixer_norm, residual, ctx):
             ctx.settle(residual)
             residual = self.mixer.forward(None, residual, ctx, site, norm=self.mixer_norm)
         else:
-            residual = self.mixer.forward(self._normed(self.mixer_norm, residual, ctx), residual, ctx, site)
-        ctx.running = None
+            residual = self.mixer.forward(h if h is not None else self.mixer_norm.forward(residual, ctx), residual, ctx, site)
+        ctx.hand_over = None
         if self.ffn is None:
             return residual
-        h = None if ffn_fuses else self._normed(self.ffn_norm, residual, ctx)
+        h = None
+        if not ffn_fuses:
+            h = ctx.take_scaled(self.ffn_norm, self.ffn, residual)
+            h = h if h is not None else self.ffn_norm.forward(residual, ctx)
         ctx.settle(residual)       # (a norm that adds no partial sums)
         ctx.next_norm = after
-        ctx.running = self.ffn if untouched else None
+        ctx.hand_over = self._hand_over(self.ffn, following)
         residual = self.ffn.forward(h, residual, ctx, norm=self.ffn_norm) if ffn_fuses else self.ffn.forward(h, residual, ctx)
-        ctx.running = None
+        ctx.hand_over = None
         return residual
 
     @staticmethod
-    def _normed(norm, residual, ctx):
-        """norm(residual), or the rows that the product before left for the part behind it to finish (ctx.add_product)."""
-        left = ctx.take_normed(norm, residual)
-        return left if isinstance(left, ops.ScaledRows) else norm.forward(residual, ctx)
+    def _hand_over(part, reader):
+        """What `ctx.hand_over` says while `part` runs; `reader` = (norm, the part that reads its rows), or None."""
+        if reader is None or getattr(reader[0], "fusable_as", None) != "rms" or not hasattr(reader[1], "takes_scaled"):
+            return None
+        return part, *reader
 
 
 class NormedMean:

@@ -48,7 +48,7 @@ class GatedMLP(FeedForward):
 
     def takes_scaled(self, rows, ctx):
         """Whether this step's product of the rows `rows` can finish their norm (ops.ScaledRows)."""
-        return not self.bias and ops.ring_gated_ok(rows, self.w_gate_up, ctx.scratch)
+        return runs_own(self, GatedMLP) and not self.bias and ops.ring_gated_ok(rows, self.w_gate_up, ctx.scratch)
 
     def forward(self, h, residual, ctx, norm=None):
         T = residual.shape[0]

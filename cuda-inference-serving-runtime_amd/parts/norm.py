@@ -13,7 +13,6 @@ class RMSNorm(Part):
     # attributes `weight` (float [dim]) and `eps`.  A mixer, feed-forward or head fuses any norm that says so.
     fusable_as = "rms"
     adds_partials = True    # forward adds the partial sums of a product left unfinished before it (ctx.add_product)
-    read_by = None          # the part that reads this norm's rows and may finish the norm itself (takes_scaled); False: there are several
 
     def __init__(self, name, dim, eps, tensor=None, around_zero=False):
         """`tensor`: the weight's full name where it is not `<name>.weight`.  `around_zero`: the stored weight is the
