@@ -24,7 +24,7 @@ embedding_kernel(const int* __restrict__ ids, const T* __restrict__ table, float
 
 extern "C" int cisr_embedding(const int* ids, const void* table, float* out, int rows, int dim,
                               int vocab, int dtype, hipStream_t stream) {
-    if (rows <= 0) return 0;
+    if (rows <= 0 || dim <= 0) return 0;
     const bool wide = dim % 4 == 0 && (uintptr_t)table % (dtype == DT_F32 ? 16 : 8) == 0 && (uintptr_t)out % 16 == 0;
     const dim3 grid(rows, (wide ? dim / 4 + 255 : dim + 255) / 256);
     if (dtype == DT_F32 && wide) embedding_kernel<float, 4><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);

@@ -81,6 +81,13 @@ def test_embedding_by_words_and_by_elements(ops, dtype, dim, offset):
     assert torch.equal(out, want) and torch.equal(cast, want.to(dtype)) and torch.equal(kept, rows.int())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_embedding_of_no_columns(ops, dtype):
+    """Rows of nothing are nothing to do, not an error."""
+    ids = torch.zeros(3, dtype=torch.int32, device=DEV)
+    assert ops.embedding(ids, torch.empty(9, 0, dtype=dtype, device=DEV), torch.empty(3, 0, device=DEV)).shape == (3, 0)
+
+
 @pytest.mark.parametrize("dim", [10, 64, 130, 576, 2048, 4100, 8200])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_rmsnorm(ops, dim, out_dtype):
