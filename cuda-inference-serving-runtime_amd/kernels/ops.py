@@ -385,7 +385,7 @@ def move_states(storages, source, target):
         return
     n = len(storages)
     bases = (C.c_void_p * n)(*[t.data_ptr() for t in storages])
-    sizes = (C.c_longlong * n)(*[t.stride(0) * t.element_size() for t in storages])
+    sizes = (C.c_longlong * n)(*[t.numel() // t.shape[0] * t.element_size() for t in storages])      # (of one slot the stride says nothing)
     with contextlib.nullcontext() if torch.cuda.current_device() == device.index else torch.cuda.device(device):
         _check(lib().cisr_state_move(bases, sizes, n, -1 if source is None else source, target, _stream()), "move_states")
 

@@ -1412,6 +1412,15 @@ def test_states_of_all_layers_in_one_call(ops, sites):
             ops.move_states(states, source, target)
 
 
+def test_states_of_one_slot_that_lie_in_a_wider_tensor(ops):
+    """A tensor of one slot is contiguous whatever its first stride is: what lies behind the slot is not its own."""
+    wide = torch.ones(3, 2, 50, device=DEV)
+    one = wide[:, 0][1:2]
+    assert one.is_contiguous() and one.stride(0) == 100
+    ops.move_states([one], None, 0)
+    assert (one == 0).all() and wide.sum() == 250
+
+
 def test_page_numbers_are_whole(ops):
     pool = torch.zeros(2, 4, 8, dtype=torch.int32, device=DEV)
     one, two = (torch.tensor([n], dtype=torch.int32, device=DEV) for n in (1, 2))
