@@ -3,7 +3,7 @@
 #pragma once
 #include "common.h"
 
-enum { RING_STORE = 0, RING_GATED = 1, RING_FLOAT = 2, RING_ROPE = 3, RING_GATED_NORMED = 4, RING_ROPE_NORMED = 5 };
+enum { RING_STORE = 0, RING_GATED = 1, RING_FLOAT = 2, RING_ROPE = 3, RING_GATED_NORMED = 4, RING_ROPE_NORMED = 5, RING_FLOAT_NORMED = 6 };
 
 struct RingArgs {
     const bf16_t* A; int lda;
@@ -17,12 +17,11 @@ struct RingArgs {
     // RING_ROPE: W = [Wq; Wk; Wv] (or Wq alone, kv_heads 0); C: q, rows of ldc; k and v go into the pages at `slots`
     const int* positions; const int* slots; const float* cos_tab; const float* sin_tab;
     bf16_t* kcache; bf16_t* vcache; int heads, kv_heads, dim, page_size, max_pos;
-    // An RMSNorm between two ring products, of which no kernel is made.  RING_FLOAT with one slice: rows `scaled` (of ldy) = bf16(C norm_w),
+    // An RMSNorm between two ring products, of which no kernel is made.  RING_FLOAT_NORMED (R given, one slice): rows `scaled` (of ldy) = bf16(C norm_w),
     // sums[i * M + m] = the squares of C's row m summed over the columns of the i-th tile (`parts` of them).  RING_GATED_NORMED and
     // RING_ROPE_NORMED: as the modes without, A is such rows and the factor that the sums give finishes the results
     bf16_t* scaled; int ldy; const float* norm_w; float* sums; int parts; float inv_k, eps;
 };
-
 
 // one function per unit: 0 or a HIP error; hipErrorInvalidValue: the unit does not hold this tile (nothing is launched)
 int cisr_ring_launch_a(const RingArgs& a, int tile, int mode, hipStream_t stream);

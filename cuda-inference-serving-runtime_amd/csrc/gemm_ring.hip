@@ -70,7 +70,8 @@ int launch(const RingArgs& a, int tile, int mode, hipStream_t stream) {
     const int rows = tile / 1000, cols = tile % 1000;
     if (a.sums && mode == RING_GATED) mode = RING_GATED_NORMED;
     if (a.sums && mode == RING_ROPE) mode = RING_ROPE_NORMED;
-    if (a.sums && (mode == RING_FLOAT ? a.parts != (a.N + cols - 1) / cols : a.parts <= 0)) return (int)hipErrorInvalidValue;
+    if (a.sums && mode == RING_FLOAT) mode = RING_FLOAT_NORMED;
+    if (a.sums && (mode == RING_FLOAT_NORMED ? a.parts != (a.N + cols - 1) / cols : a.parts <= 0)) return (int)hipErrorInvalidValue;
     if (cols == 256 && rows >= 224) return cisr_ring_launch_a(a, tile, mode, stream);
     if (cols == 256 && rows >= 96) return cisr_ring_launch_b(a, tile, mode, stream);
     if (cols == 256 || (cols == 128 && rows >= 192)) return cisr_ring_launch_c(a, tile, mode, stream);
