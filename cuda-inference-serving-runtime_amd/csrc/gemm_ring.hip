@@ -91,9 +91,9 @@ extern "C" int cisr_gemm_ring_slices(int M, int N, int K) {
 // of 1,000 to 2,000 rows is 5 us at any width below 2,048; without it the product before takes 1.3 us more at a width of 576 and
 // 2.7 at 2,048 (it stores the rows a second time), the one behind 1.1 and 4.5 (at 2,048 columns 288 x 256 tiles have 16 sums a row).
 extern "C" int cisr_gemm_ring_normed_parts(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % 4) return 0;
+    if (M <= 0 || N <= 0 || N > NORMED_COLS || K <= 0 || K % 64 || N % 4) return 0;
     const Plan plan = plan_of(M, N, K, false, 0);
-    return plan.slices > 1 || N > NORMED_COLS ? 0 : (N + plan.tile % 1000 - 1) / (plan.tile % 1000);
+    return plan.slices > 1 ? 0 : (N + plan.tile % 1000 - 1) / (plan.tile % 1000);
 }
 
 // C += A . W^T (float), and what a product that finishes the RMSNorm of C's rows reads: `scaled` = bf16(C norm_w) and the sums of squares.

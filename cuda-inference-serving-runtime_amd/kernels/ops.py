@@ -646,6 +646,7 @@ def library_ok(m, w, gated=False, plain=False, floats=False):
 
 # bf16 products of many rows whose operands go from memory straight into a ring in LDS (csrc/gemm_ring.inc): from this many rows on.
 RING_MIN_ROWS = 65
+RING_NORMED_COLS = 1024             # the widest rows whose norm two ring products make between them (as csrc/gemm_ring.hip)
 RING_MIN_OUTPUTS, RING_MIN_OUTPUTS_K = 500_000, 40
 RING_MIN_OUTPUTS_SHORT, RING_SHORT_K = 250_000, 1024
 RING_PLAIN_FLOPS, RING_PLAIN_COLS = 15e9, 2048
@@ -778,7 +779,9 @@ def ring_normed_parts(a, w, residual, weight):
     4,096 rows 91.3 / 90.6; 1,061 x 2,048, K 2,048 then gate and up of 8,192 86.3 / 86.4; cut ones 640 x 1,024, K 4,096 then 1,536 columns
     25.2 / 25.3, 1,061 rows 33.4 / 35.0."""
     (m, k), n = a.shape, w.shape[0]
-    if (w.dtype != torch.bfloat16 or m < RING_MIN_ROWS or m <= SKINNY_ROWS or tuple(residual.shape) != (m, n) or residual.dtype != torch.float32
+    if m < RING_MIN_ROWS or m <= SKINNY_ROWS or n > RING_NORMED_COLS:        # (asked by every product of a pre-norm layer: most are told by this)
+        return 0
+    if (w.dtype != torch.bfloat16 or tuple(residual.shape) != (m, n) or residual.dtype != torch.float32
             or weight.dtype != torch.float32 or weight.data_ptr() % 16 or not ring_ahead(m, w, fused=True, cut=True)):
         return 0
     parts = int(lib().cisr_gemm_ring_normed_parts(m, n, k))
@@ -1239,7 +1242,7 @@ def _few_rope_ok(a, w, head_dim, cos, normed):
 
 def qkv_rope_f32_ok(a, w, head_dim, cos):
     """Whether qkv_rope takes these operands as the 32-bit product with the rotation as its epilogue."""
-    return (a.is_cuda and w.is_cuda and a.dtype == torch.float32 and w.dtype == torch.float32 and a.dim() == 2 and a.stride(1) == 1
+    return (w.dtype == torch.float32 and a.dtype == torch.float32 and a.is_cuda and w.is_cuda and a.dim() == 2 and a.stride(1) == 1
             and w.stride(1) == 1 and head_dim % 2 == 0 and 2 * cos.shape[1] == head_dim and 0 < a.shape[0])
 
 

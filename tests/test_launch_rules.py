@@ -135,3 +135,12 @@ def test_ring_product_of_few_rows_at_measured_points(rows, columns, k, floats, r
     from runtime.kernels import ops
     w = torch.empty(columns, k, dtype=torch.bfloat16, device="meta")
     assert ops.ring_ahead(rows, w, floats=floats) is ring
+
+
+def test_products_that_never_leave_a_norm_are_told_by_their_sizes(monkeypatch):
+    """The host asks every product of a pre-norm layer whether it leaves the norm behind it: few rows and wide ones are not planned for."""
+    from runtime.kernels import ops
+    monkeypatch.setattr(ops, "ring_ahead", lambda *a, **k: pytest.fail("asked further"))
+    for rows, cols in ((1, 576), (64, 576), (1061, 1028), (65, 4096)):
+        a, w = torch.empty(rows, 64, dtype=torch.bfloat16), torch.empty(cols, 64, dtype=torch.bfloat16)
+        assert ops.ring_normed_parts(a, w, torch.empty(rows, cols), torch.empty(cols)) == 0
