@@ -108,19 +108,21 @@ class StepContext:
         block that runs it adds nothing either and knows a reader that can finish the norm behind it (`hand_over`), the norm is taken of the
         rows as they are now: only its weight is applied here."""
         self.scaled = None
-        if last is not None and self.hand_over is not None and self.hand_over[0] is last:
-            _, norm, reader = self.hand_over
-            parts = ops.ring_normed_parts(a, w, residual, norm.weight)
-            if parts:
-                rows = self.buffer("scaled.rows", residual.shape, torch.bfloat16)
-                if reader.takes_scaled(rows, self):
-                    # the norm rides in this product's epilogue and in its reader's: no kernel of its own
-                    sums = self.buffer("scaled.sums", (parts, rows.shape[0]), torch.float32)
-                    ops.gemm_ring_normed(a, w, residual, norm.weight, rows, sums)
-                    self.scaled = (norm, reader, residual, ops.ScaledRows(rows, sums, norm.eps))
-                    return residual
         if getattr(self.next_norm, "adds_partials", False):
-            partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch, finish=True)
+            leave = None
+            if last is not None and self.hand_over is not None and self.hand_over[0] is last:
+                _, norm, reader = self.hand_over
+
+                def take(parts):
+                    rows = self.buffer("scaled.rows", residual.shape, torch.bfloat16)
+                    if not reader.takes_scaled(rows, self):
+                        return None
+                    sums = self.buffer("scaled.sums", (parts, rows.shape[0]), torch.float32)
+                    self.scaled = (norm, reader, residual, ops.ScaledRows(rows, sums, norm.eps))
+                    return rows, sums
+                leave = norm.weight, take
+            # (where the norm is left, it rides in this product's epilogue and in its reader's: no kernel of its own)
+            partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch, finish=True, leave=leave)
             if partials is ops.ADDED:
                 return residual
             if partials is not None:

@@ -771,28 +771,28 @@ class ScaledRows:
         return _dev(self.sums, "sums", torch.float32), self.sums.shape[0], self.eps
 
 
-def ring_normed_parts(a, w, residual, weight):
+def ring_normed_parts(a, w, residual, weight, at=None):
     """How many sums a row gemm_ring_normed leaves, or 0 where it does not take these operands or the norm is better a kernel of its own:
     a product that is best cut along its inner size, whose slices the norm's kernel adds, and rows of more than 1,024.  us of product,
     norm and product behind it / of the two products: 1,777 x 576, K 576 then gate and up of 1,536 24.4 / 20.9, K 1,536 then 960 columns
     with the rotation 22.5 / 20.2, 4,096 rows 36.9 / 35.0 and 33.5 / 31.9; 1,061 x 1,024, K 1,024 then gate and up of 4,096 38.0 / 35.9,
     4,096 rows 91.3 / 90.6; 1,061 x 2,048, K 2,048 then gate and up of 8,192 86.3 / 86.4; cut ones 640 x 1,024, K 4,096 then 1,536 columns
-    25.2 / 25.3, 1,061 rows 33.4 / 35.0."""
+    25.2 / 25.3, 1,061 rows 33.4 / 35.0.  `at`: the product's operands (_ring_operands) from a caller that has found the ring product ahead."""
     (m, k), n = a.shape, w.shape[0]
-    if m < RING_MIN_ROWS or m <= SKINNY_ROWS or n > RING_NORMED_COLS:        # (asked by every product of a pre-norm layer: most are told by this)
+    if m < RING_MIN_ROWS or m <= SKINNY_ROWS or n > RING_NORMED_COLS or weight.dtype != torch.float32 or weight.data_ptr() % 16:
         return 0
-    if (w.dtype != torch.bfloat16 or tuple(residual.shape) != (m, n) or residual.dtype != torch.float32
-            or weight.dtype != torch.float32 or weight.data_ptr() % 16 or not ring_ahead(m, w, fused=True, cut=True)):
+    if at is None and (tuple(residual.shape) != (m, n) or residual.dtype != torch.float32 or not ring_ahead(m, w, fused=True, cut=True)
+                       or _ring_operands(a, w, residual) is None):
         return 0
-    parts = int(lib().cisr_gemm_ring_normed_parts(m, n, k))
-    return parts if parts and _ring_operands(a, w, residual) is not None else 0
+    return int(lib().cisr_gemm_ring_normed_parts(m, n, k))
 
 
-def gemm_ring_normed(a, w, residual, weight, rows, sums):
+def gemm_ring_normed(a, w, residual, weight, rows, sums, at=None):
     """residual (float [M, N], in place) += a . w^T, rows (bf16 [M, N]) = residual weight, sums (float [ring_normed_parts, M]) = its squares
-    summed by tiles of columns: what the product behind an RMSNorm of that weight reads."""
+    summed by tiles of columns: what the product behind an RMSNorm of that weight reads.  `at`: the operands, from a caller that has looked at them."""
     (m, k), n = a.shape, w.shape[0]
-    at = _ring_operands(a, w, residual) if tuple(residual.shape) == (m, n) and w.shape[1] == k and residual.dtype == torch.float32 else None
+    if at is None and tuple(residual.shape) == (m, n) and w.shape[1] == k and residual.dtype == torch.float32:
+        at = _ring_operands(a, w, residual)
     if at is None or sums.dim() != 2 or sums.shape[1] != m:
         raise KernelError("gemm_ring_normed: shape not supported")
     _check(lib().cisr_gemm_ring_normed(*at, _dev(weight, "norm weight", torch.float32, (n,)), _dev(rows, "rows", torch.bfloat16, (m, n)), n,
@@ -1025,18 +1025,23 @@ def _gemm_wide(a, w, out, residual, swiglu, what, scratch=None):
 ADDED = (None, -1)      # gemm_unfinished: the product is added already
 
 
-def gemm_unfinished(a, w, residual, scratch=None, finish=False):
+def gemm_unfinished(a, w, residual, scratch=None, finish=False, leave=None):
     """The product a . w^T that is to be added to the float rows `residual`, left unfinished where adding it takes a
     kernel of its own: the wide kernel's partial sums of a product cut into slices, (partial sums [slices, M, N],
     slices), the ring product's, (a RingSums, 0), or the library's bf16 product, (product [M, N], 0); rmsnorm_partials or
     add_partials then are that kernel.  None (nothing done) for every other product: call gemm.  `finish`: a ring product that is
-    best not cut is added to `residual` at once (ADDED), so that gemm need not ask the same again."""
+    best not cut is added to `residual` at once (ADDED), so that gemm need not ask the same again.  `leave` = (norm weight, take), with
+    `finish`: where the norm of the new rows may be left to the product that reads them, take(sums a row) gives (rows, sums) to leave it in
+    (gemm_ring_normed), or None."""
     m, k = a.shape
     n = w.shape[0]
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape[1] != k or tuple(residual.shape) != (m, n)
             or not partials_ok(residual)):
         return None
     if _ring_open(scratch) and ring_ahead(m, w, fused=True, cut=True) and (at := _ring_operands(a, w, residual)) is not None:
+        if leave is not None and (parts := ring_normed_parts(a, w, residual, leave[0], at)) and (to := leave[1](parts)) is not None:
+            gemm_ring_normed(a, w, residual, leave[0], *to, at=at)
+            return ADDED
         sums = _ring_sums(at, m, n, k, lambda floats: _ring_workspace(scratch, a.device, floats))
         if sums is None:                    # (not cut: added in the product's epilogue)
             if not finish:

@@ -77,7 +77,7 @@ def handed(monkeypatch):
     """How many norms have been left to products so far."""
     from runtime.kernels import ops
     seen, real = [], ops.gemm_ring_normed
-    monkeypatch.setattr(ops, "gemm_ring_normed", lambda a, w, *rest: (seen.append(tuple(a.shape)), real(a, w, *rest))[1])
+    monkeypatch.setattr(ops, "gemm_ring_normed", lambda a, w, *rest, **at: (seen.append(tuple(a.shape)), real(a, w, *rest, **at))[1])
     return seen
 
 
@@ -114,7 +114,7 @@ def test_norms_that_products_make_through_a_model(width, heads, kv, ff, rows, ha
     assert np.array_equal(made[1], made[0]) and np.array_equal(made[2], made[0])
     assert_close(made[0], want, "bfloat16")
     assert len(handed) % (2 * len(order) - 1) == 0
-    monkeypatch.setattr(ops, "ring_normed_parts", lambda *a: 0)
+    monkeypatch.setattr(ops, "ring_normed_parts", lambda *a, **at: 0)
     count = len(handed)
     (apart,) = logits_of(model, tokens, "eager")
     assert len(handed) == count
