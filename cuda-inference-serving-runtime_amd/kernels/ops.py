@@ -1086,19 +1086,39 @@ def _norm_args(x, norm, k, words=8):
 
 
 def _f32_norm_ok(x, w, weight=None):
-    """Whether the 32-bit product takes RMSNorm(x) . w^T with the norm (of `weight`) fused: 16-byte aligned float rows, an inner size of a
-    multiple of four below 1,024.  Any number of rows, so that a row's bits do not depend on the others of its step (csrc/gemm_f32.hip has
-    the figures)."""
+    """Whether the 32-bit product can take RMSNorm(x) . w^T with the norm (of `weight`) fused: 16-byte aligned float rows, an inner size of a
+    multiple of four below 1,024.  Any number of rows; f32_norm_ahead says of which it is the faster."""
     return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.is_cuda and w.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.stride(1) == 1
             and w.stride(1) == 1 and x.shape[1] % 4 == 0 and x.shape[1] < 1024 and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
             and (x.data_ptr() | w.data_ptr() | (0 if weight is None else weight.data_ptr())) % 16 == 0)
 
 
+# Results (rows rounded up to their tile's 16 or 32, times columns) up to which a 32-bit product makes its rows' norm: see f32_norm_ahead
+F32_NORM_OUTPUTS, F32_NORM_OUTPUTS_LONG, F32_NORM_LONG_K, F32_NORM_ROPE_OUTPUTS = 1_600_000, 2_400_000, 768, 4_000_000
+F32_NORM_COLS, F32_NORM_COLS_K = 32768, 512
+
+
+def f32_norm_ahead(m, n, k, rope=False):
+    """Whether m rows against float weights [n, k] are faster with the RMSNorm of the rows inside the product (`rope`: with the rotation and
+    the cache write as its epilogue) than as a kernel of its own: that costs a launch, but inside every block of columns makes the norm of its
+    rows again.  us apart / inside, gated products of 3,072 weight rows, K 576: 1 row 6.0 / 4.3, 130 rows 14.7 / 12.0, 256 19.7 / 20.6, 512 31.9 / 29.5,
+    1,024 52.1 / 54.5, 4,096 175 / 198; 8,192 weight rows 130 rows 28.3 / 28.3, 512 66 / 73, 4,096 438 / 522, K 768 512 rows 80 / 84; plain ones of 49,152
+    columns 1 row 21.2 / 20.5, 17 30.1 / 27.9, 32 31.1 / 30.1, 40 (tiles of 64) 54 / 63, 130 122 / 148, K 768 32 rows 38.8 / 35.3, K 256 1 row
+    12.3 / 13.0; 128,256 columns 1 row K 256 24.2 / 28.9, K 768 86.4 / 81.6; 640 x 3,072 K 576 37.0 / 39.0, K 768 44.9 / 44.0; 960 columns with the
+    rotation, K 576 512 rows 14.6 / 12.7, 2,048 40.9 / 38.4, 4,096 75.5 / 73.1, 3,072 columns 512 rows 35.1 / 31.3, 1,024 58.8 / 58.8."""
+    results = n * (-(-m // 16) * 16 if m <= 16 else -(-m // 32) * 32)
+    if rope:
+        return results <= F32_NORM_ROPE_OUTPUTS
+    return (results <= (F32_NORM_OUTPUTS if k < F32_NORM_LONG_K else F32_NORM_OUTPUTS_LONG)
+            and (n <= F32_NORM_COLS or k >= F32_NORM_COLS_K))
+
+
 def fused_norm_ok(x, w, rows_out, weight=None):
     """Whether the weight-streaming kernel can take RMSNorm(x) . w^T with the norm fused (and large weights
-    do not make the norm as a kernel of its own and the wide kernel the better choice), or in 32 bits the product (`weight`: the norm's)."""
+    do not make the norm as a kernel of its own and the wide kernel the better choice), or in 32 bits the product (`weight`: the norm's) and it
+    is the faster so."""
     if w.dtype == torch.float32:
-        return rows_out > 0 and _f32_norm_ok(x, w, weight)
+        return rows_out > 0 and f32_norm_ahead(rows_out, *w.shape) and _f32_norm_ok(x, w, weight)
     return (not wide_ok(rows_out, w, after_norm=True, fused=True) and w.dtype == torch.bfloat16 and rows_out <= SKINNY_ROWS and x.dtype == torch.float32 and x.shape[1] % 8 == 0
             and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0)
 
@@ -1115,7 +1135,8 @@ def gemm_normed(x, norm, w, out):
     n, k = w.shape
     floats = w.dtype == torch.float32
     wp, eps, rp, m = _norm_args(x, norm, k, 4 if floats else 8)
-    if not fused_norm_ok(x, w, m) or tuple(out.shape) != (m, n) or out.stride(1) != 1 or (floats and (out.dtype != torch.float32 or wp % 16)):
+    taken = m > 0 and _f32_norm_ok(x, w) and out.dtype == torch.float32 and wp % 16 == 0 if floats else fused_norm_ok(x, w, m)
+    if not taken or tuple(out.shape) != (m, n) or out.stride(1) != 1:
         raise KernelError("gemm_normed: shape not supported by the fused kernel")
     if floats:
         _check(lib().cisr_gemm_f32(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), None, 0, m, n, k, wp, eps,
@@ -1158,7 +1179,7 @@ def gemm_swiglu(a, w_gate_up, out, gate_up=None, norm=None, scratch=None, law=No
         floats = w_gate_up.dtype == torch.float32
         wp, eps, rp, _ = _norm_args(a, norm, k, 4 if floats else 8)
         if floats:
-            if (not fused_norm_ok(a, w_gate_up, m) or out.dtype != torch.float32 or wp % 16 or rp is not None
+            if (not _f32_norm_ok(a, w_gate_up) or out.dtype != torch.float32 or wp % 16 or rp is not None
                     or a.untyped_storage().data_ptr() == out.untyped_storage().data_ptr()):
                 raise KernelError("gemm_swiglu: shape not supported by the 32-bit product with the norm fused")
             _check(lib().cisr_gemm_f32_swiglu(a.data_ptr(), a.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), _dev(out, "out"), out.stride(0),
@@ -1229,7 +1250,7 @@ def qkv_rope_fused_ok(a, w, head_dim, cos, normed, scratch=None, sin=None, weigh
     qkv_rope is given; `weight`: that of the norm to be fused)."""
     m, k = a.shape
     if normed and w.dtype == torch.float32:
-        return _f32_norm_ok(a, w, weight) and qkv_rope_f32_ok(a, w, head_dim, cos)
+        return f32_norm_ahead(m, w.shape[0], k, rope=True) and _f32_norm_ok(a, w, weight) and qkv_rope_f32_ok(a, w, head_dim, cos)
     if normed and wide_ok(m, w, after_norm=True, fused=True):      # large weights: the norm is a kernel of its own, the projection the wide kernel
         return False
     if not normed and _ring_open(scratch) and ring_rope_ok(a, w, head_dim, cos, sin):

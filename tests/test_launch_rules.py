@@ -144,3 +144,19 @@ def test_products_that_never_leave_a_norm_are_told_by_their_sizes(monkeypatch):
     for rows, cols in ((1, 576), (64, 576), (1061, 1028), (65, 4096)):
         a, w = torch.empty(rows, 64, dtype=torch.bfloat16), torch.empty(cols, 64, dtype=torch.bfloat16)
         assert ops.ring_normed_parts(a, w, torch.empty(rows, cols), torch.empty(cols)) == 0
+
+
+@pytest.mark.parametrize("rows, weight_rows, k, rope, inside", [
+    (1, 3072, 576, False, True), (512, 3072, 576, False, True),            # 31.9 us apart, 29.5 inside
+    (640, 3072, 576, False, False), (640, 3072, 768, False, True),         # 37.0 / 39.0, 44.9 / 44.0
+    (1024, 3072, 768, False, False), (4096, 8192, 576, False, False),      # 63.0 / 64.5, 438 / 522
+    (8, 49152, 576, False, True), (32, 49152, 576, False, True),           # a head: 31.1 / 30.1
+    (33, 49152, 576, False, False), (130, 49152, 576, False, False),       # 54 / 63 (40 rows), 122 / 148
+    (1, 49152, 256, False, False), (1, 32768, 256, False, True),           # 12.3 / 13.0, 9.6 / 9.2
+    (1, 128256, 576, False, False), (1, 128256, 768, False, True),         # 58.3 / 58.5, 86.4 / 81.6
+    (2048, 960, 576, True, True), (4096, 960, 576, True, True),            # the rotation behind it: 40.9 / 38.4, 75.5 / 73.1
+    (1024, 3072, 576, True, True), (2048, 3072, 576, True, False),         # 58.8 / 58.8
+])
+def test_where_a_32_bit_product_makes_its_rows_norm(rows, weight_rows, k, rope, inside):
+    from runtime.kernels.ops import f32_norm_ahead
+    assert f32_norm_ahead(rows, weight_rows, k, rope) is inside
