@@ -7,30 +7,41 @@
 
 // ---------------------------------------------------------------- embedding
 // out[r, :] = table[ids[r], :]  (reference: kernels/execution.cu:2-5)
-// Bound by two trips to memory, the id's and the row's: a thread a word of V elements (four, or one where the rows are not aligned for that),
-// so that no thread goes round.  Eight rows of 2,048 bf16 in a captured step 5.8 -> 4.1 us (256 threads a row
+// Bound by two trips to memory, the id's and the row's: a thread has a word of four elements, so that no thread goes round, or four elements
+// a block apart where the rows are not aligned for words (one each were four times the blocks: 8,192 rows of 1,023 bf16 10.8 us going round,
+// 13.7 with one each, 9.5 so).  Eight rows of 2,048 bf16 in a captured step 5.8 -> 4.1 us (256 threads a row
 // that went round), one of 576 2.9 -> 2.3, 2,345 of 2,048 14.5 -> 11.8.
-template <typename T, int V>
+template <typename T, bool WORDS>
 __global__ void __launch_bounds__(256)
 embedding_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int dim, int vocab) {
-    const int row = blockIdx.x, at = (blockIdx.y * 256 + threadIdx.x) * V;
+    const int row = blockIdx.x, at = blockIdx.y * 1024 + threadIdx.x * (WORDS ? 4 : 1);
     if (at >= dim) return;
     int id = ids[row];
     if (id < 0 || id >= vocab) id = 0;  // padding rows; real ids are checked on the host
-    float v[V];
-    load_run<V>(table + (size_t)id * dim + at, v);
-    store_run<V>(out + (size_t)row * dim + at, v);
+    const T* from = table + (size_t)id * dim;
+    float* to = out + (size_t)row * dim;
+    float v[4];
+    if constexpr (WORDS) {
+        load_run<4>(from + at, v);
+        store_run<4>(to + at, v);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = load_f32(from + min(at + 256 * i, dim - 1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (at + 256 * i < dim) to[at + 256 * i] = v[i];
+    }
 }
 
 extern "C" int cisr_embedding(const int* ids, const void* table, float* out, int rows, int dim,
                               int vocab, int dtype, hipStream_t stream) {
     if (rows <= 0 || dim <= 0) return 0;
     const bool wide = dim % 4 == 0 && (uintptr_t)table % (dtype == DT_F32 ? 16 : 8) == 0 && (uintptr_t)out % 16 == 0;
-    const dim3 grid(rows, (wide ? dim / 4 + 255 : dim + 255) / 256);
-    if (dtype == DT_F32 && wide) embedding_kernel<float, 4><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
-    else if (dtype == DT_F32) embedding_kernel<float, 1><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
-    else if (wide) embedding_kernel<bf16_t, 4><<<grid, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
-    else embedding_kernel<bf16_t, 1><<<grid, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
+    const dim3 grid(rows, (dim + 1023) / 1024);
+    if (dtype == DT_F32 && wide) embedding_kernel<float, true><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
+    else if (dtype == DT_F32) embedding_kernel<float, false><<<grid, 256, 0, stream>>>(ids, (const float*)table, out, dim, vocab);
+    else if (wide) embedding_kernel<bf16_t, true><<<grid, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
+    else embedding_kernel<bf16_t, false><<<grid, 256, 0, stream>>>(ids, (const bf16_t*)table, out, dim, vocab);
     return CISR_LAUNCH_CHECK();
 }
 

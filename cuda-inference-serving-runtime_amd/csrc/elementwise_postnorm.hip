@@ -79,7 +79,10 @@ extern "C" int cisr_embedding_pairs(const int* tokens, const int* positions, con
     if (dim <= 0 || vocab <= 0 || (pairs && (buckets <= 0 || mul_prev < 0 || mul_cur < 0 || !last_token))) return (int)hipErrorInvalidValue;
     const size_t run = table_dtype == DT_F32 ? 16 : 8, cast_run = cast_dtype == DT_F32 ? 16 : 8;
     const bool wide = dim % 4 == 0 && (uintptr_t)table % run == 0 && (uintptr_t)pairs % run == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)cast % cast_run == 0;
-    const int words = wide ? dim / 4 : dim, threads = words >= 1024 ? 1024 : (words + 63) / 64 * 64;
+    // Rows that are not aligned for words: a thread an element as long as all blocks of 1,024 threads are resident, beyond that 256 threads that go
+    // round (8,192 rows of 1,023 bf16 28.2 us with a thread an element, 17.9 so; 300 rows 3.2, going round 3.5).  Of words likewise: 2,048 rows of 8,192 floats
+    // in portions 42.2 / 41.4, 64 rows 5.8, 11.5 going round.
+    const int words = wide ? dim / 4 : dim, most = rows <= 512 ? 1024 : wide ? 512 : 256, threads = words >= most ? most : (words + 63) / 64 * 64;
 #define EMB_V(TE, TH, S, V) embedding_pairs_kernel<TE, TH, S, V><<<rows, threads, 0, stream>>>(tokens, positions, seg_of_row, seg_start, state_slots, \
         last_token, (const TE*)table, (const TE*)pairs, out, (TH*)cast, dim, vocab, scale, buckets, (unsigned long long)mul_prev, (unsigned long long)mul_cur)
 #define EMB(TE, TH, S) do { if (wide) EMB_V(TE, TH, S, 4); else EMB_V(TE, TH, S, 1); } while (0)
