@@ -88,20 +88,18 @@ __device__ __forceinline__ float conv_neighbours(float x, int lanes) {
     return x;
 }
 
-template <bool SINGLE>
+template <bool SINGLE, bool UNIT>
 __global__ void __launch_bounds__(256)
 conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* __restrict__ w, const float* __restrict__ bias,
                  float* conv_state, long long slot_stride, float* __restrict__ out,
                  const int* __restrict__ seg_of_row, const int* __restrict__ seg_start, const int* __restrict__ state_slots,
                  int channels, int taps, int heads, int dt_first, const float* __restrict__ dt_bias,
                  const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay, ConvUnit unit) {
-    __shared__ float red[4];
     const int t = blockIdx.x;
     const int idx = blockIdx.y * 256 + threadIdx.x;
     const int seg = seg_of_row[t];
-    if (seg < 0) return;
-    const bool units = (int)blockIdx.y * 256 < unit.channels;       // (uniform: a block that meets in the end, and all of its threads come)
-    if (idx >= channels + heads && !units) return;
+    const bool units = UNIT && (int)blockIdx.y * 256 < unit.channels;       // (uniform: a block that meets in the end, and all of its threads come)
+    if (seg < 0 || (idx >= channels + heads && !units)) return;
     if (idx >= channels && idx < channels + heads) {
         const int h = idx - channels;
         const float z = in[(size_t)t * ld + dt_first + h] + dt_bias[h];
@@ -124,6 +122,7 @@ conv_silu_kernel(const float* __restrict__ in, int ld, int first, const float* _
         y = y / (1.0f + expf(-y));
     }
     if (units) {
+        __shared__ float red[4];
         float sum = conv_neighbours(y * y, min(unit.dim, WAVE));
         if (unit.dim > WAVE) {
             const int wave = threadIdx.x / WAVE;
@@ -290,9 +289,11 @@ extern "C" int cisr_conv_silu(const float* in, int ld, int first, const float* w
         return (int)hipErrorInvalidValue;
     if (channels <= 0 || taps < 1 || taps > MAX_TAPS || heads < 0 || segments > 65535) return (int)hipErrorInvalidValue;
     const dim3 grid(rows, (channels + heads + 255) / 256);
+#define CONV_FEW_AS(SINGLE, UNIT) conv_silu_kernel<SINGLE, UNIT><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride, \
+        out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay, unit)
+#define CONV_FEW(SINGLE) do { if (unit_channels) CONV_FEW_AS(SINGLE, true); else CONV_FEW_AS(SINGLE, false); } while (0)
     if (single_rows) {       // `single_rows`: the caller knows that no segment has more than one row
-        conv_silu_kernel<true><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride,
-            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay, unit);
+        CONV_FEW(true);
         return CISR_LAUNCH_CHECK();
     }
     const bool enough = (long long)rows * channels >= CONV_WORDS + CONV_WORDS_A_PORTION * min(segments - 1, 16);
@@ -308,9 +309,10 @@ extern "C" int cisr_conv_silu(const float* in, int ld, int first, const float* w
 #undef CONV_ROWS_OF
 #undef CONV_ROWS_AS
     } else {
-        conv_silu_kernel<false><<<grid, 256, 0, stream>>>(in, ld, first, w, bias, conv_state, slot_stride,
-            out, seg_of_row, seg_start, state_slots, channels, taps, heads, dt_first, dt_bias, a_log, step, decay, unit);
+        CONV_FEW(false);
     }
+#undef CONV_FEW
+#undef CONV_FEW_AS
     int err = CISR_LAUNCH_CHECK();
     if (err || taps == 1) return err;
     conv_state_kernel<<<dim3(segments, (channels + 255) / 256), 256, 0, stream>>>(in, ld, first, conv_state, slot_stride, seg_start,
