@@ -372,7 +372,7 @@ def page_copy(pool, src, dst, slabs, pages_per_slab):
 
 def move_states(storages, source, target):
     """t[target] := t[source] (None: zeros) in each of the contiguous tensors `storages`, one launch for all of them on the
-    current stream of their device."""
+    current stream of their device.  (One tensor alone is torch's to clear or copy: 5.5 and 6.8 us of host time, 7.4 and 7.2 with the list; two tensors 7.6 and 7.9, 9.4 and 11.5 one by one.)"""
     storages = [t for t in storages if t.numel()]
     if not storages:
         return
@@ -382,6 +382,10 @@ def move_states(storages, source, target):
         if t.device != device or not 0 <= target < t.shape[0] or (source is not None and not 0 <= source < t.shape[0]):
             raise KernelError("move_states: slots of tensors on one device")
     if source == target:
+        return
+    if len(storages) == 1:
+        own = storages[0][target]
+        own.zero_() if source is None else own.copy_(storages[0][source])
         return
     n = len(storages)
     bases = (C.c_void_p * n)(*[t.data_ptr() for t in storages])
