@@ -3,7 +3,7 @@
 It owns the groups of pages (pages.py), the state slots (state.py), the length
 of every request, and, when given an allocator, the device tensors behind them.
 The host logic runs without a GPU; device work (page copies for copy-on-write,
-zeroing of a fresh state slot) goes through two callbacks.
+clearing and copying of state slots) goes through callbacks.
 
 Per step the step function calls `append_many([(request, n_tokens), ...])`,
 which is atomic: either every request gets its slots in every group, or
@@ -36,8 +36,8 @@ class CacheManager:
                  move_states=None):
         """site_needs: {site id: need (KVNeed or another class with its methods)}; state_needs: {site id: StateNeed}.
         n_pages: pages per group (an int, or {need: int}).  `allocate_pages(shape)` makes a group's device storage,
-        of the shape its need states.  `move_states(storages, source, slot)`, in the place of the two callbacks that take one
-        site's tensor, copies a slot of every site's (source None: clears it)."""
+        of the shape its need states.  `move_states(storages, source, slot)` copies a slot of every site's tensor (source None: clears
+        it); `zero_state(storage, slot)` and `copy_state(storage, source, slot)` say the same of one tensor at a time."""
         self.page_size = page_size
         self.groups = []
         self.group_of_site = {}
@@ -59,7 +59,15 @@ class CacheManager:
         if allocate_state is not None:
             for site, need in self.state_needs.items():
                 self.state_storage[site] = allocate_state(max_requests, need.shape, need.dtype)
-        self._copy_pages, self._zero_state, self._copy_state, self._move_states = copy_pages, zero_state, copy_state, move_states
+        self._copy_pages, self._move_states = copy_pages, move_states
+        if move_states is None:
+            def one_by_one(storages, source, slot):
+                for storage in storages:
+                    if source is None and zero_state is not None:
+                        zero_state(storage, slot)
+                    elif source is not None and copy_state is not None:
+                        copy_state(storage, source, slot)
+            self._move_states = one_by_one
 
     # -- requests ---------------------------------------------------------
     def create(self, request):
@@ -69,11 +77,7 @@ class CacheManager:
         self.lengths[request] = 0
         for group in self.groups:
             group.create(request)
-        if self._move_states is not None:
-            self._move_states(self.state_storage.values(), None, slot)
-        elif self._zero_state is not None:
-            for site in self.state_needs:
-                self._zero_state(self.state_storage[site], slot)
+        self._move_states(self.state_storage.values(), None, slot)
         return slot
 
     def fork(self, source, target):
@@ -84,11 +88,7 @@ class CacheManager:
         self.lengths[target] = self.lengths[source]
         for group in self.groups:
             group.fork(source, target)
-        if self._move_states is not None:
-            self._move_states(self.state_storage.values(), self.slots.slot_of(source), slot)
-        elif self._copy_state is not None:
-            for site in self.state_needs:
-                self._copy_state(self.state_storage[site], self.slots.slot_of(source), slot)
+        self._move_states(self.state_storage.values(), self.slots.slot_of(source), slot)
         return slot
 
     def release(self, request):

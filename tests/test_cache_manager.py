@@ -214,6 +214,16 @@ def test_state_is_zeroed_on_create_and_copied_on_fork():
     assert d.state_slot == 1
 
 
+def test_states_of_all_sites_move_in_one_call():
+    """What the runner gives: one callback for the tensors of all sites, the source's slot and the new request's."""
+    log = []
+    m = CacheManager({0: KVNeed(1, 8)}, 4, 4, 3, state_needs={1: StateNeed((5,), "float32"), 4: StateNeed((2, 3), "int32")},
+                     allocate_state=lambda n, shape, dt: (n, shape, dt), move_states=lambda storages, source, slot: log.append((list(storages), source, slot)))
+    m.create("a"); m.create("b"); m.fork("b", "c"); m.release("a"); m.fork("c", "d")
+    both = [(3, (5,), "float32"), (3, (2, 3), "int32")]
+    assert log == [(both, None, 0), (both, None, 1), (both, 1, 2), (both, 2, 0)]
+
+
 @pytest.mark.parametrize("seed", range(6))
 def test_random_orders_keep_every_page_accounted_for(seed):
     rng = random.Random(seed)
