@@ -94,7 +94,7 @@ __device__ __forceinline__ void finish_pair(const GemmF32Args& p, int m, int n, 
     }
 }
 
-#define GF_RUN 256                       // NORM: most of K that a wave may take (a word a lane)
+#define GF_RUN 256                       // NORM: floats of LDS for a wave's run of the norm's weights (a word a lane stores them; it reads at most 144)
 
 // 16-byte words of LDS: the waves' operands on their way, and then their tiles
 constexpr int gf_lds_items(int tm, int tn, int wk) { return wk * (tm * tn > tm + tn ? tm * tn : tm + tn) * WAVE; }
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(WK * WAVE) gemm_f32_kernel(GemmF32Args p) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) fa[d][i] = gf_load<VEC>(a_row[i], k, K);
     };
-    // NORM: the wave's run of the norm's weights waits in LDS (in registers beside the operands they made tiles of sixteen waves spill)
+    // NORM: the wave's run of the norm's weights waits in LDS and is read a sixteen ahead of its use, beside operands that take the registers
     float* const ssq = (float*)((gf_f32x4*)gf_lds + gf_lds_items(TM, TN, WK));      // [WK][TM * 16] sums of squares
     float* const run = ssq + WK * TM * 16 + wave * GF_RUN - first * 16;              // [WK][GF_RUN], from its first sixteen on
     gf_f32x4 next = {0.f, 0.f, 0.f, 0.f};
@@ -358,7 +358,8 @@ static int launch_f32_tile(const GemmF32Args& p, hipStream_t stream) {
 }
 
 // Waves a tile: sixteen from an inner size of 1,024 on, else eight (so that a wave has at least two sixteens at the small
-// models' 576).  A fused norm takes eight waves and rows in 16-byte words only.
+// models' 576).  A fused norm takes eight waves and rows in 16-byte words only; up to how many results it is the faster, with both sides'
+// times, stands at f32_norm_ahead (kernels/ops.py).
 #define GF_SIXTEEN_WAVES 1024
 static_assert(GF_SIXTEEN_WAVES / 8 + 16 <= GF_RUN, "a wave's run of the norm's weights");
 template <int FORM>
