@@ -58,20 +58,23 @@ class PreNormBlock(Part):
         return self.mixer_norm
 
     def first_reader(self):
-        """(That norm, the part that reads its rows): the block before may leave the norm to that part."""
-        return self.mixer_norm, self.mixer
+        """(That norm, the part that reads its rows): the block before may leave the norm to that part.  None: an arrangement made of this one
+        may add to the stream before it."""
+        return (self.mixer_norm, self.mixer) if runs_own(self, PreNormBlock) else None
 
     def forward(self, residual, ctx, site):
         # ctx.next_norm names the norm that reads the residual stream after the part that runs: a part's last
         # product may be left to it (ctx.add_product); on entry it is the norm after this block
         after, following = ctx.next_norm, None
-        # behind this block's last part someone else may add to the stream: an arrangement made of it or around it, a caller that looks at the rows
-        if ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock) and ctx.layer_tap is None:
+        # before this block's first part and behind its last one someone else may add to the stream: an arrangement made of it or around it, a
+        # caller that looks at the rows
+        own = ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock)
+        if own and ctx.layer_tap is None:
             following = ctx.following[1]
         ffn_fuses = self.ffn is not None and self.ffn.fuses_norm(self.ffn_norm, residual, ctx)
         inside = (self.ffn_norm, self.ffn) if self.ffn is not None and not ffn_fuses else None
         ctx.next_norm = after if self.ffn is None else None if ffn_fuses else self.ffn_norm
-        h = ctx.take_scaled(self.mixer_norm, self.mixer, residual)
+        h = ctx.take_scaled(self.mixer_norm, self.mixer, residual) if own else None
         ctx.hand_over = self._hand_over(self.mixer, following if self.ffn is None else inside)
         if h is None and self.mixer.fuses_norm(self.mixer_norm, residual, ctx):
             ctx.settle(residual)

@@ -129,6 +129,31 @@ def test_parts_that_end_with_their_product_leave_the_next_norm(ctx):
     assert right(seen, 4) and kinds(blocks) == [["Tensor"], ["ScaledRows"], ["ScaledRows"], ["ScaledRows"]]
 
 
+def test_what_others_add_before_a_block_is_in_its_first_norm(ctx):
+    """An arrangement made of the pre-norm one, or around it, that adds to the rows before the block reads them: the norm that the block
+    before left was of the rows as they were."""
+    from runtime.parts import PreNormBlock
+
+    class Before(PreNormBlock):
+        def forward(self, residual, ctx, site):
+            return super().forward(residual.add_(0.7), ctx, site)
+
+    class Around:
+        def __init__(self, inner):
+            self.inner = inner
+
+        def __getattr__(self, name):
+            return getattr(self.inner, name)
+
+        def forward(self, residual, ctx, site):
+            return self.inner.forward(residual.add_(0.7), ctx, site)
+    for block, outer in ((Before, None), (None, Around)):
+        first, last = layers_of(1) + layers_of(1, block=block)
+        seen = watch([first, last])
+        run(ctx, [first, outer(last) if outer else last])
+        assert right(seen, 4)
+
+
 @pytest.mark.parametrize("which", ["mixer", "ffn"])
 def test_what_a_part_adds_behind_its_product_is_in_the_next_norm(ctx, which):
     """A part that adds to the rows after its last product: sums commute with a product left unfinished, not with a norm taken already."""
