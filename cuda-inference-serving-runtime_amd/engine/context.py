@@ -73,7 +73,7 @@ class StepContext:
         self.unfinished = None
         self.next_norm = None     # the norm that reads the residual stream after the block that runs now, if known
         # (part, norm, reader): `part` runs now, nothing is added to the stream behind it, and `reader`, which may finish norms (`takes_scaled`),
-        # reads norm(stream) next.  Set by a block around its parts; the model sets `following` = (layer that runs now, (norm, reader) of the next or None)
+        # reads norm(stream) next.  Set by a block around its parts; the model sets `following` = (layer that runs now, the next one or None)
         self.hand_over = self.following = None
         self.scaled = None        # (norm, reader, residual rows, ops.ScaledRows): what add_product left for `reader` to finish
         self.normed = None        # (norm part, residual rows, normed rows): a block made its follower's first norm on the way

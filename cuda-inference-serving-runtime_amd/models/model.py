@@ -148,7 +148,7 @@ class Model:
             # a block may leave its last product to the norm that reads the residual stream next, if that block names one
             following = self.layers[self.schedule[index + 1].layer] if index < last else None
             ctx.next_norm = following.first_norm() if hasattr(following, "first_norm") else None
-            ctx.following = self.layers[entry.layer], following.first_reader() if hasattr(following, "first_reader") else None
+            ctx.following = self.layers[entry.layer], following
             x = self.layers[entry.layer].forward(x, ctx, self.site_of(index))
             if ctx.layer_tap is not None:      # (a caller that looks at the residual stream after every layer run; eager steps only)
                 ctx.settle(x)

@@ -65,17 +65,19 @@ class PreNormBlock(Part):
     def forward(self, residual, ctx, site):
         # ctx.next_norm names the norm that reads the residual stream after the part that runs: a part's last
         # product may be left to it (ctx.add_product); on entry it is the norm after this block
-        after, following = ctx.next_norm, None
+        after, following, own = ctx.next_norm, None, False
+        many = residual.shape[0] >= ops.RING_MIN_ROWS      # (products of fewer rows leave no norm: nothing is asked, 2 us a layer of host time)
         # before this block's first part and behind its last one someone else may add to the stream: an arrangement made of it or around it, a
         # caller that looks at the rows
-        own = ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock)
-        if own and ctx.layer_tap is None:
-            following = ctx.following[1]
+        if many:
+            own = ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock)
+            if own and ctx.layer_tap is None and hasattr(ctx.following[1], "first_reader"):
+                following = ctx.following[1].first_reader()
         ffn_fuses = self.ffn is not None and self.ffn.fuses_norm(self.ffn_norm, residual, ctx)
-        inside = (self.ffn_norm, self.ffn) if self.ffn is not None and not ffn_fuses else None
         ctx.next_norm = after if self.ffn is None else None if ffn_fuses else self.ffn_norm
         h = ctx.take_scaled(self.mixer_norm, self.mixer, residual) if own else None
-        ctx.hand_over = self._hand_over(self.mixer, following if self.ffn is None else inside)
+        if many:
+            ctx.hand_over = self._hand_over(self.mixer, following if self.ffn is None else None if ffn_fuses else (self.ffn_norm, self.ffn))
         if h is None and self.mixer.fuses_norm(self.mixer_norm, residual, ctx):
             ctx.settle(residual)
             residual = self.mixer.forward(None, residual, ctx, site, norm=self.mixer_norm)
@@ -86,11 +88,12 @@ class PreNormBlock(Part):
             return residual
         h = None
         if not ffn_fuses:
-            h = ctx.take_scaled(self.ffn_norm, self.ffn, residual)
+            h = ctx.take_scaled(self.ffn_norm, self.ffn, residual) if many else None
             h = h if h is not None else self.ffn_norm.forward(residual, ctx)
         ctx.settle(residual)       # (a norm that adds no partial sums)
         ctx.next_norm = after
-        ctx.hand_over = self._hand_over(self.ffn, following)
+        if many:
+            ctx.hand_over = self._hand_over(self.ffn, following)
         residual = self.ffn.forward(h, residual, ctx, norm=self.ffn_norm) if ffn_fuses else self.ffn.forward(h, residual, ctx)
         ctx.hand_over = None
         return residual

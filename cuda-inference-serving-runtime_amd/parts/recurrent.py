@@ -426,7 +426,7 @@ class GatedDeltaRule(Mixer):
         return ctx.product_for_norm(self._normed_result(h, ctx, site), self.w_out, "delta.y")
 
     def forward(self, h, residual, ctx, site, norm=None):
-        return ctx.add_product(self._normed_result(h, ctx, site), self.w_out, residual, last=self if runs_own(self, GatedDeltaRule) else None)
+        return ctx.add_product(self._normed_result(h, ctx, site), self.w_out, residual, last=self if ctx.hand_over is not None and runs_own(self, GatedDeltaRule) else None)
 
 
 class ChannelDeltaRule(GatedDeltaRule):

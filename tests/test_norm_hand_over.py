@@ -5,7 +5,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-ROWS, WIDTH = 6, 8
+ROWS, WIDTH = 65, 8
 
 
 @pytest.fixture
@@ -72,11 +72,11 @@ def toys():
     return type("ToyMixer", (Toy, Mixer), {}), type("ToyFFN", (Toy, FeedForward), {})
 
 
-def run(ctx, layers, tap=None):
+def run(ctx, layers, tap=None, rows=ROWS):
     """Runs the layers as a model does; returns the rows after them and the normed rows that every sublayer should have read."""
     from runtime.models import Model
     torch.manual_seed(0)
-    x = torch.randn(ROWS, WIDTH)
+    x = torch.randn(rows, WIDTH)
     ctx.layer_tap = tap
     ctx.logit_rows = torch.empty(0)
     model = Model(None, SimpleNamespace(forward=lambda c: x), layers, None, None, max_positions=1, vocab_size=1)
@@ -154,6 +154,16 @@ def test_what_others_add_before_a_block_is_in_its_first_norm(ctx):
         assert right(seen, 4)
 
 
+def test_few_rows_are_asked_nothing(ctx):
+    """No product of so few rows leaves a norm: a step of them, made kernel by kernel, pays nothing for the question."""
+    blocks = layers_of(2)
+    seen, named = watch(blocks), []
+    real = ctx.add_product
+    ctx.add_product = lambda *a, last=None: (named.append(ctx.hand_over), real(*a, last=last))[1]
+    run(ctx, blocks, rows=64)
+    assert right(seen, 4) and named == [None] * 4
+
+
 @pytest.mark.parametrize("which", ["mixer", "ffn"])
 def test_what_a_part_adds_behind_its_product_is_in_the_next_norm(ctx, which):
     """A part that adds to the rows after its last product: sums commute with a product left unfinished, not with a norm taken already."""
@@ -201,6 +211,7 @@ def test_what_others_add_behind_a_part_is_in_the_next_norm(ctx):
     for cls in (GatedMLP, Halved):
         part = cls("m", WIDTH, WIDTH)
         part.w_gate_up, part.w_down = torch.cat([weights(1), weights(2)]), weights(3)
+        ctx.hand_over = part, rms(1), part
         part.forward(torch.zeros(ROWS, WIDTH).bfloat16(), torch.zeros(ROWS, WIDTH), ctx)
         asked[-1] = asked[-1] is part
     assert asked == [True, False]
