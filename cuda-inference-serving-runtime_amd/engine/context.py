@@ -72,9 +72,9 @@ class StepContext:
         # part that was told it may (`next_norm`), taken by the norm that reads the rows next (or settled)
         self.unfinished = None
         self.next_norm = None     # the norm that reads the residual stream after the block that runs now, if known
-        # (part, norm, reader): `part` runs now, nothing is added to the stream behind it, and `reader`, which may finish norms (`takes_scaled`),
-        # reads norm(stream) next.  Set by a block around its parts; the model sets `following` = (layer that runs now, the next one or None)
-        self.hand_over = self.following = None
+        # (part, block): `part` runs now, the block adds nothing to the stream behind it and knows who reads the stream next (`reads_next`).
+        # Set by a block around its parts; the model sets `following` = (layer that runs now, the next one or None)
+        self.hand_over = self.following = self.last_of = None
         self.scaled = None        # (norm, reader, residual rows, ops.ScaledRows): what add_product left for `reader` to finish
         self.normed = None        # (norm part, residual rows, normed rows): a block made its follower's first norm on the way
         self.layer_tap = getattr(runner, "layer_tap", None)   # callable(schedule index, residual rows) after every layer run, or None
@@ -101,26 +101,17 @@ class StepContext:
             self.runner.carry(array)
         return got
 
-    def add_product(self, a, w, residual, last=None):
+    def add_product(self, a, w, residual, last=None, of=None):
         """residual += a . w^T, in place.  Where the product is cut along its inner size and the norm that reads the
         residual next can add the slices itself (`next_norm`), they are left to it: one kernel fewer.  A caller may add more to the
-        residual afterwards, as sums commute; one that does not names itself (`last`: the part whose last addition this is), and if the
-        block that runs it adds nothing either and knows a reader that can finish the norm behind it (`hand_over`), the norm is taken of the
-        rows as they are now: only its weight is applied here."""
+        residual afterwards, as sums commute; one that does not names itself (`last`: the part whose last addition this is, as long as its forward
+        is that of the class `of`), and if the block that runs it adds nothing either and knows a reader that can finish the norm behind it
+        (`hand_over`), the norm is taken of the rows as they are now: only its weight is applied here."""
         self.scaled = None
         if getattr(self.next_norm, "adds_partials", False):
             leave = None
             if last is not None and self.hand_over is not None and self.hand_over[0] is last:
-                _, norm, reader = self.hand_over
-
-                def take(parts):
-                    rows = self.buffer("scaled.rows", residual.shape, torch.bfloat16)
-                    if not reader.takes_scaled(rows, self):
-                        return None
-                    sums = self.buffer("scaled.sums", (parts, rows.shape[0]), torch.float32)
-                    self.scaled = (norm, reader, residual, ops.ScaledRows(rows, sums, norm.eps))
-                    return rows, sums
-                leave = norm.weight, take
+                leave, self.last_of = self._leave_norm, of
             # (where the norm is left, it rides in this product's epilogue and in its reader's: no kernel of its own)
             partials = ops.gemm_unfinished(a, w, residual, scratch=self.scratch, finish=True, leave=leave)
             if partials is ops.ADDED:
@@ -129,6 +120,24 @@ class StepContext:
                 self.leave_unfinished(residual, partials)
                 return residual
         return ops.gemm(a, w, residual, residual=residual, scratch=self.scratch)
+
+    def _leave_norm(self, a, w, residual, at):
+        """What a product that may leave the norm of its rows leaves it in, (norm weight, rows, sums), or None.  Asked of few products (a ring product
+        of narrow rows), so that the others do not pay for the answer: 3 to 4 us a layer of a step that runs kernel by kernel."""
+        part, block = self.hand_over
+        found = block.reads_next(part, self.last_of, self)
+        if found is None:
+            return None
+        norm, reader = found
+        parts = ops.ring_normed_parts(a, w, residual, norm.weight, at)
+        if not parts:
+            return None
+        rows = self.buffer("scaled.rows", residual.shape, torch.bfloat16)
+        if not reader.takes_scaled(rows, self):
+            return None
+        sums = self.buffer("scaled.sums", (parts, rows.shape[0]), torch.float32)
+        self.scaled = (norm, reader, residual, ops.ScaledRows(rows, sums, norm.eps))
+        return norm.weight, rows, sums
 
     def product_for_norm(self, a, w, tag):
         """a . w^T as float rows [T, N] in the buffer `tag`, for a part whose result is read next by the kernel that adds

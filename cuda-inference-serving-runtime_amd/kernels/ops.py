@@ -1034,17 +1034,17 @@ def gemm_unfinished(a, w, residual, scratch=None, finish=False, leave=None):
     kernel of its own: the wide kernel's partial sums of a product cut into slices, (partial sums [slices, M, N],
     slices), the ring product's, (a RingSums, 0), or the library's bf16 product, (product [M, N], 0); rmsnorm_partials or
     add_partials then are that kernel.  None (nothing done) for every other product: call gemm.  `finish`: a ring product that is
-    best not cut is added to `residual` at once (ADDED), so that gemm need not ask the same again.  `leave` = (norm weight, take), with
-    `finish`: where the norm of the new rows may be left to the product that reads them, take(sums a row) gives (rows, sums) to leave it in
-    (gemm_ring_normed), or None."""
+    best not cut is added to `residual` at once (ADDED), so that gemm need not ask the same again.  `leave`, with `finish`:
+    leave(a, w, residual, operands) of a ring product of rows whose norm may be left to the product that reads them gives (norm weight, rows, sums) to leave it
+    in (gemm_ring_normed), or None."""
     m, k = a.shape
     n = w.shape[0]
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape[1] != k or tuple(residual.shape) != (m, n)
             or not partials_ok(residual)):
         return None
     if _ring_open(scratch) and ring_ahead(m, w, fused=True, cut=True) and (at := _ring_operands(a, w, residual)) is not None:
-        if leave is not None and (parts := ring_normed_parts(a, w, residual, leave[0], at)) and (to := leave[1](parts)) is not None:
-            gemm_ring_normed(a, w, residual, leave[0], *to, at=at)
+        if leave is not None and n <= RING_NORMED_COLS and m >= RING_MIN_ROWS and (to := leave(a, w, residual, at)) is not None:
+            gemm_ring_normed(a, w, residual, *to, at=at)
             return ADDED
         sums = _ring_sums(at, m, n, k, lambda floats: _ring_workspace(scratch, a.device, floats))
         if sums is None:                    # (not cut: added in the product's epilogue)
@@ -1307,7 +1307,7 @@ def qkv_rope(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_
     sums = None
     if isinstance(a, ScaledRows):
         a, sums = a.rows, a.args(a.rows.shape[0])
-    if qkv_rope_f32_ok(a, w, dim, cos):
+    if w.dtype == torch.float32 and qkv_rope_f32_ok(a, w, dim, cos):
         return _qkv_rope_f32(a, w, q_out, positions, slots, cos, sin, kcache, vcache, heads, kv_heads, dim, page_size, norm)
     m, k = a.shape
     has_kv = kcache is not None

@@ -128,7 +128,7 @@ class PagedAttention(Mixer):
         if unmerged is not None:
             residual = ops.gemm_merged(unmerged, nh, D, self.w_out, residual, residual)
         else:
-            residual = ctx.add_product(out, self.w_out, residual, last=self if ctx.hand_over is not None and self.b_out is None and runs_own(self, PagedAttention) else None)
+            residual = ctx.add_product(out, self.w_out, residual, last=self if self.b_out is None else None, of=PagedAttention)
         if self.b_out is not None:
             ops.bias_add(residual, self.b_out)   # (sums commute: slices of the product that a later norm adds may still be out; its norm is not taken yet)
         return residual
@@ -417,7 +417,7 @@ class LatentAttention(Mixer):
         return ctx.product_for_norm(self._heads_result(h, ctx, site), self.w_out, "lat.y")
 
     def forward(self, h, residual, ctx, site, norm=None):
-        return ctx.add_product(self._heads_result(h, ctx, site), self.w_out, residual, last=self if ctx.hand_over is not None and runs_own(self, LatentAttention) else None)
+        return ctx.add_product(self._heads_result(h, ctx, site), self.w_out, residual, last=self, of=LatentAttention)
 
 
 class SigmoidAttention(Mixer):

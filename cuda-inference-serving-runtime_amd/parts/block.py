@@ -62,22 +62,33 @@ class PreNormBlock(Part):
         may add to the stream before it."""
         return (self.mixer_norm, self.mixer) if runs_own(self, PreNormBlock) else None
 
+    def reads_next(self, part, of, ctx):
+        """(norm, reader) that read the residual stream as `part` leaves it, if the reader may finish the norm (`takes_scaled`); else None.  `of`:
+        the class whose forward says that it adds nothing more, if the part may have another (ctx.add_product)."""
+        if of is not None and not runs_own(part, of):
+            return None
+        if part is self.mixer and self.ffn is not None:
+            found = self.ffn_norm, self.ffn
+        elif self._alone(ctx) and ctx.layer_tap is None and hasattr(ctx.following[1], "first_reader"):
+            found = ctx.following[1].first_reader()
+        else:
+            found = None
+        if found is None or getattr(found[0], "fusable_as", None) != "rms" or not hasattr(found[1], "takes_scaled"):
+            return None
+        return found
+
+    def _alone(self, ctx):
+        """Whether nobody adds to the stream before this block's first part and behind its last one: an arrangement made of it or around it may."""
+        return ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock)
+
     def forward(self, residual, ctx, site):
         # ctx.next_norm names the norm that reads the residual stream after the part that runs: a part's last
         # product may be left to it (ctx.add_product); on entry it is the norm after this block
-        after, following, own = ctx.next_norm, None, False
-        many = residual.shape[0] >= ops.RING_MIN_ROWS      # (products of fewer rows leave no norm: nothing is asked, 2 us a layer of host time)
-        # before this block's first part and behind its last one someone else may add to the stream: an arrangement made of it or around it, a
-        # caller that looks at the rows
-        if many:
-            own = ctx.following is not None and ctx.following[0] is self and runs_own(self, PreNormBlock)
-            if own and ctx.layer_tap is None and hasattr(ctx.following[1], "first_reader"):
-                following = ctx.following[1].first_reader()
+        after = ctx.next_norm
         ffn_fuses = self.ffn is not None and self.ffn.fuses_norm(self.ffn_norm, residual, ctx)
         ctx.next_norm = after if self.ffn is None else None if ffn_fuses else self.ffn_norm
-        h = ctx.take_scaled(self.mixer_norm, self.mixer, residual) if own else None
-        if many:
-            ctx.hand_over = self._hand_over(self.mixer, following if self.ffn is None else None if ffn_fuses else (self.ffn_norm, self.ffn))
+        h = ctx.take_scaled(self.mixer_norm, self.mixer, residual) if ctx.scaled is not None and self._alone(ctx) else None
+        ctx.hand_over = self.mixer, self
         if h is None and self.mixer.fuses_norm(self.mixer_norm, residual, ctx):
             ctx.settle(residual)
             residual = self.mixer.forward(None, residual, ctx, site, norm=self.mixer_norm)
@@ -88,22 +99,14 @@ class PreNormBlock(Part):
             return residual
         h = None
         if not ffn_fuses:
-            h = ctx.take_scaled(self.ffn_norm, self.ffn, residual) if many else None
+            h = ctx.take_scaled(self.ffn_norm, self.ffn, residual) if ctx.scaled is not None else None
             h = h if h is not None else self.ffn_norm.forward(residual, ctx)
         ctx.settle(residual)       # (a norm that adds no partial sums)
         ctx.next_norm = after
-        if many:
-            ctx.hand_over = self._hand_over(self.ffn, following)
+        ctx.hand_over = self.ffn, self
         residual = self.ffn.forward(h, residual, ctx, norm=self.ffn_norm) if ffn_fuses else self.ffn.forward(h, residual, ctx)
         ctx.hand_over = None
         return residual
-
-    @staticmethod
-    def _hand_over(part, reader):
-        """What `ctx.hand_over` says while `part` runs; `reader` = (norm, the part that reads its rows), or None."""
-        if reader is None or getattr(reader[0], "fusable_as", None) != "rms" or not hasattr(reader[1], "takes_scaled"):
-            return None
-        return part, *reader
 
 
 class NormedMean:

@@ -64,7 +64,7 @@ class GatedMLP(FeedForward):
         else:
             ops.gemm_swiglu(h, self.w_gate_up, act, gate_up=ctx.buffer("ffn.gate_up", (T, 2 * self.intermediate), ctx.dtype),
                             scratch=ctx.scratch, law=self.law)
-        return ctx.add_product(act, self.w_down, residual, last=self if ctx.hand_over is not None and runs_own(self, GatedMLP) else None)
+        return ctx.add_product(act, self.w_down, residual, last=self, of=GatedMLP)
 
     def output(self, h, ctx, tag="ffn", unfinished=False):
         """The feed-forward's result, float [T, hidden], without the residual sum (no biases); `unfinished`: it may be
@@ -172,7 +172,7 @@ class DenseMLP(FeedForward):
         if self.bias:
             from .block import add_sublayer
             return add_sublayer(residual, self.output(h, ctx), None, 1.0)
-        return ctx.add_product(self._activations(h, ctx), self.w_down, residual, last=self if ctx.hand_over is not None and runs_own(self, DenseMLP) else None)
+        return ctx.add_product(self._activations(h, ctx), self.w_down, residual, last=self, of=DenseMLP)
 
 
 class RoutedExperts(FeedForward):

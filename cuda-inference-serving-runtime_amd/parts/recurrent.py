@@ -39,7 +39,7 @@ import torch
 from ..cache.pages import StateNeed
 from ..kernels import library, ops
 from ..weights.loader import AnySize
-from .base import Mixer, TensorSpec, matrix_operand, register_part, runs_own
+from .base import Mixer, TensorSpec, matrix_operand, register_part
 
 
 def _float(t):
@@ -426,7 +426,7 @@ class GatedDeltaRule(Mixer):
         return ctx.product_for_norm(self._normed_result(h, ctx, site), self.w_out, "delta.y")
 
     def forward(self, h, residual, ctx, site, norm=None):
-        return ctx.add_product(self._normed_result(h, ctx, site), self.w_out, residual, last=self if ctx.hand_over is not None and runs_own(self, GatedDeltaRule) else None)
+        return ctx.add_product(self._normed_result(h, ctx, site), self.w_out, residual, last=self, of=GatedDeltaRule)
 
 
 class ChannelDeltaRule(GatedDeltaRule):

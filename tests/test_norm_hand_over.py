@@ -18,16 +18,16 @@ def ctx(monkeypatch):
         return out.copy_(a.float() @ w.float().T + (0.0 if residual is None else residual))
 
     def unfinished(a, w, residual, scratch=None, finish=False, leave=None):
-        to = None if leave is None else leave[1](1)
+        to = None if leave is None or a.shape[0] < ROWS else leave(a, w, residual, ())
         if to is not None:
             gemm(a, w, residual, residual)
-            to[0].copy_(residual * leave[0])
-            to[1].copy_((residual * residual).sum(1)[None])
+            to[1].copy_(residual * to[0])
+            to[2].copy_((residual * residual).sum(1)[None])
             return ops.ADDED
 
     def rmsnorm(x, weight, out, eps, rows=None):
         return out.copy_(x * torch.rsqrt((x * x).mean(1, keepdim=True) + eps) * weight)
-    for name, fake in (("gemm", gemm), ("gemm_unfinished", unfinished), ("rmsnorm", rmsnorm), ("swiglu_fused_ok", lambda *a: True), ("gemm_swiglu", lambda h, w, out, **k: out.zero_())):
+    for name, fake in (("gemm", gemm), ("gemm_unfinished", unfinished), ("ring_normed_parts", lambda *a: 1), ("rmsnorm", rmsnorm), ("swiglu_fused_ok", lambda *a: True), ("gemm_swiglu", lambda h, w, out, **k: out.zero_())):
         monkeypatch.setattr(ops, name, fake)
     runner = SimpleNamespace(cache=None, model=SimpleNamespace(dtype=torch.bfloat16), device="cpu", scratch=None, workspace=Workspace("cpu"))
     return StepContext(runner)
@@ -154,14 +154,16 @@ def test_what_others_add_before_a_block_is_in_its_first_norm(ctx):
         assert right(seen, 4)
 
 
-def test_few_rows_are_asked_nothing(ctx):
-    """No product of so few rows leaves a norm: a step of them, made kernel by kernel, pays nothing for the question."""
-    blocks = layers_of(2)
-    seen, named = watch(blocks), []
-    real = ctx.add_product
-    ctx.add_product = lambda *a, last=None: (named.append(ctx.hand_over), real(*a, last=last))[1]
-    run(ctx, blocks, rows=64)
-    assert right(seen, 4) and named == [None] * 4
+def test_products_that_leave_no_norm_are_not_asked_who_reads_it(ctx, monkeypatch):
+    """Finding the reader costs host time where a step runs kernel by kernel: only a product that may leave its norm pays for it."""
+    from runtime.parts import PreNormBlock
+    blocks, asked = layers_of(2), []
+    seen, real = watch(blocks), PreNormBlock.reads_next
+    monkeypatch.setattr(PreNormBlock, "reads_next", lambda self, *a: (asked.append(self), real(self, *a))[1])
+    run(ctx, blocks, rows=ROWS - 1)
+    assert right(seen, 4) and not asked
+    run(ctx, blocks)
+    assert right(seen, 8) and len(asked) == 3         # (the last product has no norm behind it that adds)
 
 
 @pytest.mark.parametrize("which", ["mixer", "ffn"])
@@ -206,15 +208,15 @@ def test_what_others_add_behind_a_part_is_in_the_next_norm(ctx):
     class Halved(GatedMLP):
         def forward(self, h, residual, ctx, norm=None):
             return super().forward(h, residual, ctx, norm=norm).mul_(0.5)
-    asked = []
-    ctx.add_product = lambda a, w, residual, last=None: (asked.append(last), residual)[1]
+    named = []
+    ctx.add_product = lambda a, w, residual, last=None, of=None: (named.append((last, of)), residual)[1]
     for cls in (GatedMLP, Halved):
         part = cls("m", WIDTH, WIDTH)
         part.w_gate_up, part.w_down = torch.cat([weights(1), weights(2)]), weights(3)
-        ctx.hand_over = part, rms(1), part
         part.forward(torch.zeros(ROWS, WIDTH).bfloat16(), torch.zeros(ROWS, WIDTH), ctx)
-        asked[-1] = asked[-1] is part
-    assert asked == [True, False]
+        block = PreNormBlock(rms(1), part, rms(2), ToyFFN(3))
+        assert named.pop() == (part, GatedMLP)
+        assert block.reads_next(part, GatedMLP, ctx) == ((block.ffn_norm, block.ffn) if cls is GatedMLP else None)
 
 
 def test_a_norm_is_left_to_the_part_that_reads_it_in_this_step_only(ctx, monkeypatch):
