@@ -73,9 +73,10 @@ class PreNormBlock(Part):
             found = ctx.following[1].first_reader()
         else:
             found = None
-        if found is None or getattr(found[0], "fusable_as", None) != "rms" or not hasattr(found[1], "takes_scaled"):
+        if found is None or getattr(found[0], "fusable_as", None) != "rms":
             return None
-        return found
+        # (a part around another one may pass the other's answers on: it is not the one that they are about)
+        return found if getattr(getattr(found[1], "takes_scaled", None), "__self__", None) is found[1] else None
 
     def _alone(self, ctx):
         """Whether nobody adds to the stream before this block's first part and behind its last one: an arrangement made of it or around it may."""

@@ -129,6 +129,25 @@ def test_parts_that_end_with_their_product_leave_the_next_norm(ctx):
     assert right(seen, 4) and kinds(blocks) == [["Tensor"], ["ScaledRows"], ["ScaledRows"], ["ScaledRows"]]
 
 
+def test_a_part_around_another_is_given_normed_rows(ctx):
+    """A feed-forward that answers for another one in all but its forward: what the inner one can finish is not said for the outer one."""
+    class Around:
+        def __init__(self, inner):
+            self.inner = inner
+
+        def __getattr__(self, name):
+            return getattr(self.inner, name)
+
+        def forward(self, h, residual, ctx, norm=None):
+            return self.inner.forward(h * 1.0, residual, ctx)
+    blocks = layers_of(2)
+    seen = watch(blocks)
+    for block in blocks:
+        block.ffn = Around(block.ffn)
+    run(ctx, blocks)
+    assert right(seen, 4) and kinds(blocks) == [["Tensor"]] * 4
+
+
 def test_what_others_add_before_a_block_is_in_its_first_norm(ctx):
     """An arrangement made of the pre-norm one, or around it, that adds to the rows before the block reads them: the norm that the block
     before left was of the rows as they were."""
